@@ -1,0 +1,92 @@
+// What the two files of the windowed attention with a sink share: the arguments of its kernels and how a score is
+// shaped on its way to the softmax.
+#pragma once
+
+#include "common.h"
+
+struct ScoreShape {
+  float cap;                       // 0: no cap
+  const float *temp, *r1, *r2;     // a number a query head each, or null (r1 and r2 together)
+  const float* dist;               // [nh][dist_n], or null
+  int dist_n;
+};
+
+struct SinkArgs {
+  int ldq, ldo, ldg, rows, rows_per_tile, heads_per_tile, nh, nkv, KD, VD;
+  const int *row_pos, *row_seq, *seq_slot, *block_table;
+  int bt_stride, BS;
+  float scale;
+  int window, keep_first, sink;
+  // single tokens of a bfloat16 run may share a tile's keys out over `ksplit` workgroups (blockIdx.z): each takes
+  // the rounds of SPLIT chunks whose number is its own modulo ksplit and leaves its partial result in `part`,
+  // which a second launch merges in the order of the workgroups
+  int ksplit;
+  float* part;
+  int maps, out_f32;
+  const float* sinks;  // null: the sink's score is 0
+  ScoreShape shape;
+  const float* wide_gate;
+  int ldwg;
+  int chunk;  // 0: no chunks
+};
+
+// the first key of the window (or of the chunk) of a row at position p
+__device__ inline int first_key(const SinkArgs& a, int p) {
+  const int lo = (a.window > 0 && p >= a.window) ? p - a.window + 1 : 0;
+  return a.chunk > 0 ? max(lo, p / a.chunk * a.chunk) : lo;
+}
+
+// What a lane needs of its query head to shape a score.
+struct HeadShape {
+  float mul, cap, inv_cap, r1, r2;
+  const float* dist;
+  int last;
+  bool log_bias;
+};
+
+__device__ inline HeadShape head_shape(const SinkArgs& a, int h) {
+  HeadShape s;
+  s.mul = a.shape.temp != nullptr ? a.scale * a.shape.temp[h] : a.scale;
+  s.cap = a.shape.cap, s.inv_cap = a.shape.cap > 0.f ? 1.f / a.shape.cap : 0.f;
+  s.r1 = a.shape.r1 != nullptr ? a.shape.r1[h] : 0.f, s.r2 = a.shape.r1 != nullptr ? a.shape.r2[h] : 0.f;
+  s.log_bias = a.shape.r1 != nullptr;
+  s.last = a.shape.dist_n - 1;
+  s.dist = a.shape.dist != nullptr ? a.shape.dist + (long long)h * a.shape.dist_n : nullptr;
+  return s;
+}
+
+// The score of a key `d` positions back (d >= 0).  EXACT: the library's tanh and logarithm (32-bit runs); else the
+// hardware's exponential and logarithm, whose absolute error is that of a 32-bit rounding of 1.
+template <bool EXACT>
+__device__ inline float shaped(float dot, int d, const HeadShape& s) {
+  float v = dot * s.mul;
+  if (s.cap > 0.f) {
+    const float y = v * s.inv_cap;
+    if constexpr (EXACT) {
+      v = s.cap * tanhf(y);
+    } else {
+      const float e = __expf(-2.f * fabsf(y));
+      v = copysignf(s.cap * (1.f - e) * __builtin_amdgcn_rcpf(1.f + e), y);
+    }
+  }
+  if (s.log_bias) {
+    if constexpr (EXACT) v -= s.r1 * log1pf(s.r2 * (float)d);
+    else v -= s.r1 * __logf(fmaf(s.r2, (float)d, 1.f));
+  }
+  if (s.dist != nullptr) v += s.dist[min(d, s.last)];
+  return v;
+}
+
+template <typename T>
+__device__ inline void put_out(T* out, long long at, float v, int out_f32) {
+  if (out_f32) ((float*)out)[at] = v;
+  else out[at] = from_f32<T>(v);
+}
+
+inline bool scores_shaped(const ScoreShape& s) {
+  return s.cap > 0.f || s.temp != nullptr || s.r1 != nullptr || s.dist != nullptr;
+}
+
+// Prompts of a bfloat16 run (attention_sink_rows.hip).  -> 1 launched, 0 not a launch that it takes, -2 an error.
+int lq_sink_rows32(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache,
+                   const int* cu_rows, const SinkArgs& a, int batch, hipStream_t stream);

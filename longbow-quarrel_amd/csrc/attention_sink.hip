@@ -26,7 +26,7 @@
 //   s += dist[h][min(p - t, dist_n - 1)]   (a bias looked up by distance, the last entry for all that is farther).
 // The sink's score is not shaped.  `wide_gate`: a logit for every entry of the result, [rows, nh * value size] in
 // 32-bit, whose sigmoid multiplies it.
-#include "common.h"
+#include "attention_sink.h"
 
 namespace {
 
@@ -41,85 +41,6 @@ __device__ inline f32x4 ld4(const bf16_t* p) {
   r.z = __uint_as_float(v.y << 16);
   r.w = __uint_as_float(v.y & 0xffff0000u);
   return r;
-}
-
-struct ScoreShape {
-  float cap;                       // 0: no cap
-  const float *temp, *r1, *r2;     // a number a query head each, or null (r1 and r2 together)
-  const float* dist;               // [nh][dist_n], or null
-  int dist_n;
-};
-
-struct SinkArgs {
-  int ldq, ldo, ldg, rows, rows_per_tile, heads_per_tile, nh, nkv, KD, VD;
-  const int *row_pos, *row_seq, *seq_slot, *block_table;
-  int bt_stride, BS;
-  float scale;
-  int window, keep_first, sink;
-  // single tokens of a bfloat16 run may share a tile's keys out over `ksplit` workgroups (blockIdx.z): each takes
-  // the rounds of SPLIT chunks whose number is its own modulo ksplit and leaves its partial result in `part`,
-  // which a second launch merges in the order of the workgroups
-  int ksplit;
-  float* part;
-  int maps, out_f32;
-  const float* sinks;  // null: the sink's score is 0
-  ScoreShape shape;
-  const float* wide_gate;
-  int ldwg;
-  int chunk;  // 0: no chunks
-};
-
-// the first key of the window (or of the chunk) of a row at position p
-__device__ inline int first_key(const SinkArgs& a, int p) {
-  const int lo = (a.window > 0 && p >= a.window) ? p - a.window + 1 : 0;
-  return a.chunk > 0 ? max(lo, p / a.chunk * a.chunk) : lo;
-}
-
-// What a lane needs of its query head to shape a score.
-struct HeadShape {
-  float mul, cap, inv_cap, r1, r2;
-  const float* dist;
-  int last;
-  bool log_bias;
-};
-
-__device__ inline HeadShape head_shape(const SinkArgs& a, int h) {
-  HeadShape s;
-  s.mul = a.shape.temp != nullptr ? a.scale * a.shape.temp[h] : a.scale;
-  s.cap = a.shape.cap, s.inv_cap = a.shape.cap > 0.f ? 1.f / a.shape.cap : 0.f;
-  s.r1 = a.shape.r1 != nullptr ? a.shape.r1[h] : 0.f, s.r2 = a.shape.r1 != nullptr ? a.shape.r2[h] : 0.f;
-  s.log_bias = a.shape.r1 != nullptr;
-  s.last = a.shape.dist_n - 1;
-  s.dist = a.shape.dist != nullptr ? a.shape.dist + (long long)h * a.shape.dist_n : nullptr;
-  return s;
-}
-
-// The score of a key `d` positions back (d >= 0).  EXACT: the library's tanh and logarithm (32-bit runs); else the
-// hardware's exponential and logarithm, whose absolute error is that of a 32-bit rounding of 1.
-template <bool EXACT>
-__device__ inline float shaped(float dot, int d, const HeadShape& s) {
-  float v = dot * s.mul;
-  if (s.cap > 0.f) {
-    const float y = v * s.inv_cap;
-    if constexpr (EXACT) {
-      v = s.cap * tanhf(y);
-    } else {
-      const float e = __expf(-2.f * fabsf(y));
-      v = copysignf(s.cap * (1.f - e) * __builtin_amdgcn_rcpf(1.f + e), y);
-    }
-  }
-  if (s.log_bias) {
-    if constexpr (EXACT) v -= s.r1 * log1pf(s.r2 * (float)d);
-    else v -= s.r1 * __logf(fmaf(s.r2, (float)d, 1.f));
-  }
-  if (s.dist != nullptr) v += s.dist[min(d, s.last)];
-  return v;
-}
-
-template <typename T>
-__device__ inline void put_out(T* out, long long at, float v, int out_f32) {
-  if (out_f32) ((float*)out)[at] = v;
-  else out[at] = from_f32<T>(v);
 }
 
 constexpr int MAX_KD = 256;
@@ -531,10 +452,6 @@ TileShape tile_shape(int el, int rows, int batch, int nh, int nkv, int KD, int V
   return t;
 }
 
-bool scores_shaped(const ScoreShape& s) {
-  return s.cap > 0.f || s.temp != nullptr || s.r1 != nullptr || s.dist != nullptr;
-}
-
 template <typename T>
 bool launch_tiles(const void* q, void* out, const void* gate, const void* kcache, const void* vcache, const SinkArgs& a,
                   int batch, int max_len, float* part, long long part_floats, hipStream_t stream) {
@@ -610,7 +527,7 @@ extern "C" int lq_sink_attention(const void* q, int ldq, void* out, int ldo, con
                                  int force_rows, int max_len, float* part, long long part_floats, const float* sinks,
                                  int maps, int out_f32, float cap, const float* temp, const float* r1, const float* r2,
                                  const float* dist, int dist_n, const float* wide_gate, int ldwg, int chunk,
-                                 hipStream_t stream) {
+                                 const int* cu_rows, hipStream_t stream) {
   LQ_REQUIRE(chunk >= 0 && (chunk == 0 || keep_first == 0), "sink_attention: chunks of %d with %d kept first tokens", chunk, keep_first);
   LQ_REQUIRE(cap >= 0.f && (r1 == nullptr) == (r2 == nullptr) && (dist == nullptr || dist_n > 0),
              "sink_attention: a cap of %g, a table by distance of %d entries", (double)cap, dist_n);
@@ -632,6 +549,12 @@ extern "C" int lq_sink_attention(const void* q, int ldq, void* out, int ldo, con
   a.maps = maps, a.out_f32 = out_f32 || dtype == LQ_F32, a.sinks = sinks;
   a.shape = {cap, temp, r1, r2, dist, dist_n};
   a.wide_gate = wide_gate, a.ldwg = ldwg, a.chunk = chunk;
+  if (!force_rows && dtype == LQ_BF16 && rows > batch && cu_rows != nullptr) {
+    const int taken = lq_sink_rows32((const bf16_t*)q, out, (const bf16_t*)gate, (const bf16_t*)kcache,
+                                     (const bf16_t*)vcache, cu_rows, a, batch, stream);
+    if (taken < 0) return taken;
+    if (taken) return 0;
+  }
   if (!force_rows) {
     const bool done = dtype == LQ_F32
                           ? launch_tiles<float>(q, out, gate, kcache, vcache, a, batch, max_len, part, part_floats, stream)

@@ -20,7 +20,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 12  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 13  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -759,7 +759,8 @@ class HipKernels:
                        workspace: Optional[torch.Tensor] = None, sink_values: Optional[torch.Tensor] = None,
                        maps: int = 1, softcap: float = 0.0, temp: Optional[torch.Tensor] = None,
                        log_bias: Optional[tuple] = None, distance_bias: Optional[torch.Tensor] = None,
-                       wide_gate: Optional[torch.Tensor] = None, chunk: int = 0) -> None:
+                       wide_gate: Optional[torch.Tensor] = None, chunk: int = 0,
+                       cu_rows: Optional[torch.Tensor] = None) -> None:
         """Attention of the step's rows over their slots' cached keys: row at position p sees t <= p with
         p - t < window (0: all) or t < keep_first, and with `chunk` > 0 only t of its own run of `chunk` positions
         (p // chunk == t // chunk); with `sink` the softmax's denominator has one more term e^0;
@@ -776,9 +777,10 @@ class HipKernels:
         (float32 [heads]); softcap * tanh(score / softcap); minus r1 ln(1 + r2 n) with `log_bias` = (r1, r2) (float32
         [heads] each), n the distance p - t; plus `distance_bias` [heads, entries] at column min(n, entries - 1).  The
         sink's score is not shaped.  `wide_gate` float32 [rows, heads * value_dim]: every entry of the result times the
-        sigmoid of its own."""
+        sigmoid of its own.  `cu_rows` (int32 [batch + 1], where each sequence's rows start): prompts of a bfloat16 run
+        then go by tiles of 32 rows of one sequence."""
         self._dev(q, out, gate, row_pos, row_seq, seq_slot, block_table, kcache, vcache, sink_values, temp, distance_bias,
-                  wide_gate)
+                  wide_gate, cu_rows)
         rows, batch = q.shape[0], seq_slot.numel()
         self._i32(row_pos, "row_pos", rows)
         self._i32(row_seq, "row_seq", rows)
@@ -811,6 +813,8 @@ class HipKernels:
             raise KernelLibraryError("sink_attention: the wide gate is float32 [rows, heads * value_dim]")
         if workspace is not None:
             self._f32(workspace, "sink_attention: workspace", workspace.numel())
+        if cu_rows is not None:
+            self._i32(cu_rows, "cu_rows", batch + 1)
         self._check(self.lib.lq_sink_attention(
             _ptr(q), c_int(self._rows2d(q, "q")), _ptr(out), c_int(self._rows2d(out, "out")), _ptr(gate),
             c_int(0 if gate is None else self._rows2d(gate, "gate")), c_int(_code(q)), c_int(rows), c_int(batch),
@@ -821,7 +825,7 @@ class HipKernels:
             c_longlong(0 if workspace is None else workspace.numel()), _ptr(sink_values), c_int(maps),
             c_int(1 if out.dtype == torch.float32 else 0), c_float(softcap), _ptr(temp), _ptr(r1), _ptr(r2),
             _ptr(distance_bias), c_int(0 if distance_bias is None else int(distance_bias.shape[1])), _ptr(wide_gate),
-            c_int(0 if wide_gate is None else self._rows2d(wide_gate, "wide_gate")), c_int(chunk), self.stream))
+            c_int(0 if wide_gate is None else self._rows2d(wide_gate, "wide_gate")), c_int(chunk), _ptr(cu_rows), self.stream))
 
     def diff_combine(self, both: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int, value_dim: int, lam: float,
                      eps: float, gain: float) -> None:

@@ -60,10 +60,13 @@ from .rope import rotary_frequencies, rotary_magnitude, step_angles
 def split_scratch(ctx: StepContext, dtype, heads: int, kv_heads: int, key_dim: int, value_dim: int, block_size: int,
                   window: int, keep_first: int, chunk: int = 0) -> Dict[str, object]:
     """The keywords with which `sink_attention` may share a decoding step's keys out over several workgroups a tile:
-    the step's bound of the lengths and the scratch that the kernel object asks for (nothing where it asks for none)."""
+    the step's bound of the lengths and the scratch that the kernel object asks for (nothing where it asks for none);
+    for other steps where each sequence's rows start, by which it may cut them into tiles."""
     ask = getattr(ctx.kernels, "sink_attention_workspace", None)
-    if ask is None or not ctx.decode:
+    if ask is None:
         return {}
+    if not ctx.decode:
+        return {"cu_rows": ctx.cu_rows}
     need = ask(dtype, ctx.rows, ctx.batch, heads, kv_heads, key_dim, value_dim, block_size, window, keep_first, ctx.max_len,
                **({"chunk": chunk} if chunk else {}))
     return dict(max_len=ctx.max_len, workspace=ctx.ws.alloc((need,), torch.float32)) if need else {}

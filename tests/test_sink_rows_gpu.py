@@ -1,0 +1,81 @@
+"""Prompts through the 32 x 32 score tiles of the windowed attention (`cu_rows` given) against the general kernel, one
+wavefront a row and head, at the sizes where tiles, blocks and halves end."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+PLAIN = dict(sink=False)
+CASES = [  # heads, key heads, key size, value size, (new, held) of every sequence, options
+    (16, 4, 128, 128, [(1, 0), (32, 0), (33, 63), (2, 64)], dict(window=1024, keep_first=4)),
+    (16, 4, 128, 128, [(200, 0), (31, 1000)], dict(window=100, keep_first=70)),
+    (8, 2, 128, 128, [(129, 30)], dict(PLAIN, chunk=48)),
+    (8, 2, 128, 128, [(70, 90)], dict(PLAIN, window=33)),
+    (4, 4, 64, 64, [(127, 0), (130, 1)], PLAIN),
+    (6, 3, 64, 48, [(65, 0), (63, 0), (1, 200)], dict(sinks=True)),
+    (3, 1, 40, 24, [(97, 31)], PLAIN),
+    (8, 2, 112, 80, [(40, 61)], dict(window=64, gate=True)),
+    (8, 4, 128, 256, [(77, 51), (3, 0)], dict(PLAIN, maps=2, window=90)),
+    (4, 1, 96, 136, [(65, 0)], dict(PLAIN, wide=True)),
+    (16, 1, 256, 192, [(33, 31), (64, 0)], PLAIN),
+    (4, 1, 200, 104, [(50, 15)], PLAIN),
+    (8, 2, 128, 128, [(90, 300)], dict(sinks=True, cap=30.0, log=True, window=200)),
+    (8, 2, 64, 64, [(90, 300)], dict(PLAIN, cap=5.0, dist=100, temp=True, wide=True)),
+]
+
+
+@pytest.mark.parametrize("H,G,D,P,seqs,options", CASES)
+def test_tiles_of_32_rows(H, G, D, P, seqs, options):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(H * 1000 + D + P)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    o = dict(options)
+    maps = o.pop("maps", 1)
+    blocks = [-(-(n + held) // 64) for n, held in seqs]
+    order = torch.randperm(sum(blocks), generator=gen).int()
+    table = torch.zeros(len(seqs), max(blocks), dtype=torch.int32)
+    at = 0
+    for b, n in enumerate(blocks):
+        table[b, :n] = order[at : at + n]
+        at += n
+    k = rand(sum(blocks), G // maps, 64, maps * D).bfloat16()
+    v = rand(sum(blocks), G // maps, P, 64).bfloat16()
+    for b, (n, held) in enumerate(seqs):  # what was never written may be anything
+        if (n + held) % 64:
+            v[table[b, blocks[b] - 1].long(), :, :, (n + held) % 64 :] = float("nan")
+            k[table[b, blocks[b] - 1].long(), :, (n + held) % 64 :] = float("inf")
+    rows = sum(n for n, _ in seqs)
+    q = rand(rows, H * D).bfloat16()
+    more = dict(window=o.get("window", 0), keep_first=o.get("keep_first", 0), sink=o.get("sink", True), maps=maps,
+                chunk=o.get("chunk", 0), softcap=o.get("cap", 0.0))
+    if "sinks" in o:
+        more["sink_values"] = rand(H)
+    if "gate" in o:
+        more["gate"] = rand(rows, H).bfloat16()
+    if "wide" in o:
+        more["wide_gate"] = rand(rows, H * P)
+    if "temp" in o:
+        more["temp"] = 1 + 0.1 * rand(H)
+    if "log" in o:
+        more["log_bias"] = (rand(H).abs(), rand(H).abs())
+    if "dist" in o:
+        more["distance_bias"] = rand(H, o["dist"])
+    pos = i32(held + i for n, held in seqs for i in range(n))
+    seq = i32(b for b, (n, _) in enumerate(seqs) for _ in range(n))
+    starts = i32([sum(n for n, _ in seqs[:b]) for b in range(len(seqs) + 1)])
+    kn = HipKernels()
+    for dtype in (torch.float32, torch.bfloat16):
+        got, want = (torch.full((rows, H * P), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+        args = (H, G, D, P, pos, seq, i32(range(len(seqs))), table.cuda(), k, v, 64, D ** -0.5)
+        kn.sink_attention(q, got, *args, cu_rows=starts, **more)
+        kn.force_generic = True
+        kn.sink_attention(q, want, *args, **more)
+        kn.force_generic = False
+        # Sums of N terms in another order differ by at most 2 N 2^-24 of sum p |v| <= max |v|, the exponentials'
+        # arguments (up to 30 with the log bias) by 2^-22 of themselves: 1.4e-4 + 1e-5 of 4.7 at N = 1 031, and what
+        # is seen is a hundredth of that.  In bfloat16 the two may round to neighbours: 2^-8 of the value.
+        assert torch.isfinite(want).all()
+        far = (got.float() - want.float()).abs()
+        assert (far <= 7e-5 + (want.float().abs() * 2 ** -7 if dtype == torch.bfloat16 else 0)).all(), far.max()
