@@ -1,0 +1,478 @@
+// The gated delta rule over long portions of a sequence, in chunks of 64 tokens on the matrix cores.
+//
+// Token by token (recurrent.hip):  S <- diag(g_t) S;  u_t = beta_t (v_t - S^T k_t);  S <- S + k_t u_t^T;  o_t = S^T q_t,
+// a chain of two exchanges over a column's lanes a token, 0.31 to 0.42 microseconds of it and 1.2 where the chip is
+// full.  Over a chunk that starts from the state S, with p_t the product of the decays g_1 .. g_t of a key channel and
+// f_st that of g_(s+1) .. g_t (all of them products of numbers up to 1, never quotients):
+//   A[t][s] = sum_n k_t k_s f_st (s < t),  B[t][s] = sum_n q_t k_s f_st (s <= t)
+//   U = T (V - K~ S),  T = (I + diag(beta) A)^-1 diag(beta),  K~_t = p_t k_t
+//   O = Q~ S + B U,  Q~_t = p_t q_t;      S <- diag(p_64) S + sum_s (f_s,64 k_s) u_s^T
+// T, B, K~, Q~ and the last factor do not depend on the state: a first launch makes them for all chunks and heads side by
+// side (`delta_prepare_kernel`), in the order in which the second reads its operands.  The second (`delta_walk_kernel`)
+// walks a sequence's chunks in order, a workgroup a head and 16 columns of the values.
+//
+// Everything is 32-bit (v_mfma_f32_16x16x4_f32: lane l gives A[l % 16][k = l / 16] and B[k = l / 16][l % 16] and
+// receives D[4 (l / 16) + e][l % 16]).  Which entry stands for which k is free as long as both operands agree: step s of
+// a run of 16 k takes k = 4 (l / 16) + s, so that a result's four registers are the next product's B operands as they
+// are, and an A operand is four neighbouring entries of a row.  "Fragments" below: 16 rows by 16 k, lane l's four
+// entries (row l % 16, k = 4 (l / 16) .. + 3) at 4 l.
+//
+// Chunks count from a sequence's first row of the step; a last chunk's missing tokens take part as zeros.
+#include <type_traits>
+
+#include "device_math.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr int CHUNK = 64, SUB = 16, NMAX = 128;  // tokens a chunk and a block of it; key channels (fewer: zeros)
+constexpr int KT = CHUNK / SUB, NT = NMAX / 16;
+constexpr int FRAG = 256;                        // floats a fragment
+// a (chunk, head)'s part of the scratch, in floats
+constexpr int AT_KEYS = 0, AT_QUERIES = AT_KEYS + KT * NT * FRAG, AT_UPDATE = AT_QUERIES + KT * NT * FRAG,
+              AT_T = AT_UPDATE + NT * KT * FRAG, AT_B = AT_T + KT * KT * FRAG, AT_DECAY = AT_B + KT * KT * FRAG,
+              PART = AT_DECAY + NMAX;
+
+struct DeltaArgs {
+  const float *q, *k, *v, *beta, *a, *dt_bias, *a_log;
+  int ldq, ldk, ldv, ldbeta, lda, ldo;
+  float *state, *out, *scratch;
+  int heads, kv_heads, N, P, batch, channel_decay;
+  const int *seq_slot, *cu_rows;
+};
+
+__device__ inline f32x4 step4(const f32x4& a, const f32x4& b, f32x4 c) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
+  return c;
+}
+
+template <int CTRL>
+__device__ inline float add_from(float keep, float give) {  // the partner's `give` on top of this lane's `keep`
+  return keep + dpp_swap<CTRL>(give);
+}
+
+// The sums over a wavefront of up to COUNT (8 or 16) values: lane s (modulo 16) ends up with that of v[s] (modulo COUNT).
+// Every exchange halves the values a lane still carries: its partner takes the other half.
+template <int COUNT>
+__device__ inline float sums_by_lane(float (&v)[SUB]) {
+  const int lane = threadIdx.x;
+  if constexpr (COUNT == 16) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = add_from<0x140>(lane & 8 ? v[i + 8] : v[i], lane & 8 ? v[i] : v[i + 8]);  // 15 - lane
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = add_from<0x140>(v[i], v[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = add_from<0x141>(lane & 4 ? v[i + 4] : v[i], lane & 4 ? v[i] : v[i + 4]);  // 7 - lane
+#pragma unroll
+  for (int i = 0; i < 2; ++i) v[i] = add_from<0x4E>(lane & 2 ? v[i + 2] : v[i], lane & 2 ? v[i] : v[i + 2]);
+  float x = add_from<0xB1>(lane & 1 ? v[1] : v[0], lane & 1 ? v[0] : v[1]);
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+
+// exp(rate ln(1 + e^z)).  ln(1 + x) of x = e^-|z| <= 1 as 2 atanh(x / (2 + x)), whose series in s^2 <= 1 / 9 ends below
+// 2^-25 of it with s^15: a third of the library function's instructions, which were 4 microseconds of a chunk's 26.
+__device__ inline float decay_of(float z, float rate) {
+  const float x = expf(-fabsf(z)), d = 2.f + x;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.f), r, r);
+  const float s = x * r, y = s * s;
+  float p = 2.f / 15.f;
+  p = fmaf(p, y, 2.f / 13.f), p = fmaf(p, y, 2.f / 11.f), p = fmaf(p, y, 2.f / 9.f), p = fmaf(p, y, 2.f / 7.f);
+  p = fmaf(p, y, 2.f / 5.f), p = fmaf(p, y, 2.f / 3.f);
+  return expf(rate * (fmaxf(z, 0.f) + fmaf(s * y, p, 2.f * s)));
+}
+
+// The chunks of all sequences are numbered through.  -> the sequence of chunk number t and its number within it (-1:
+// past the last).  Lane i holds sequence i of a run of 64; every wavefront works out the same.
+__device__ inline int2 find_chunk(const int* __restrict__ cu_rows, int batch, int t) {
+  const int lane = threadIdx.x & 63;
+  for (int b0 = 0; b0 < batch; b0 += 64) {
+    const int b = min(b0 + lane, batch - 1);
+    const int mine = b0 + lane < batch ? (cu_rows[b + 1] - cu_rows[b] + CHUNK - 1) / CHUNK : 0;
+    int upto = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int before = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += before;
+    }
+    const unsigned long long past = __ballot(upto > t);
+    if (past) {
+      const int at = __ffsll(past) - 1;
+      return make_int2(__builtin_amdgcn_readfirstlane(b0 + at),
+                       __builtin_amdgcn_readfirstlane(t - __shfl(upto - mine, at, 64)));
+    }
+    t -= __shfl(upto, 63, 64);
+  }
+  return make_int2(-1, -1);
+}
+
+// the number of sequence b's first chunk
+__device__ inline int first_chunk(const int* __restrict__ cu_rows, int b) {
+  int n = 0;
+  for (int i = threadIdx.x & 63; i < b; i += 64) n += (cu_rows[i + 1] - cu_rows[i] + CHUNK - 1) / CHUNK;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
+constexpr int LD = NMAX + 4;   // floats a row of LDS: neighbouring rows start 4 banks apart
+constexpr int LDT = CHUNK + 4;
+
+struct Prepared {
+  float k[CHUNK][LD], q[CHUNK][LD], g[CHUNK][LD];  // after the blocks: k and q by the decays from their block's start, k by those to its end
+  float block[KT][NMAX];                           // the product of a block's decays
+  float m[CHUNK][LDT];                             // A, then T
+  float b[CHUNK][LDT];
+  float inv[KT][SUB][SUB + 4];                     // the inverses of the blocks on the diagonal
+  float beta[CHUNK];
+};
+
+// One workgroup of eight wavefronts a (chunk, head).  Wavefronts w and w + 4 first make A and B within block w, channel
+// by channel (a lane holds two, and for every earlier token of the block the product of the decays since): no
+// factoring of f_st into a row's and a column's part is safe where decays are strong.  Between blocks it is: from the
+// row's block's start on, and up to the column's block's end.
+template <bool QUADS>
+__global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  Prepared& L = *(Prepared*)smem;
+  const int2 at = find_chunk(a.cu_rows, a.batch, blockIdx.x);
+  if (at.x < 0) return;
+  const int h = blockIdx.y, j = h / (a.heads / a.kv_heads), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const long long r0 = a.cu_rows[at.x] + (long long)at.y * CHUNK;
+  const int nt = min(CHUNK, (int)(a.cu_rows[at.x + 1] - r0)), N = a.N;
+  float* to = a.scratch + ((long long)blockIdx.x * a.heads + h) * PART;
+  const float rate = -expf(a.a_log[h]);
+
+  // every load of a thread is asked for before the first is waited for
+  if constexpr (QUADS) {
+    constexpr int PER = CHUNK * NMAX / 4 / 512;
+    f32x4 k[PER], q[PER], z[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = tid + 512 * i, t = e / (NMAX / 4), n = e % (NMAX / 4) * 4;
+      k[i] = q[i] = z[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (t < nt && n < N) {
+        const long long r = r0 + t;
+        k[i] = *(const f32x4*)(a.k + r * a.ldk + j * N + n), q[i] = *(const f32x4*)(a.q + r * a.ldq + j * N + n);
+        if (a.channel_decay) z[i] = *(const f32x4*)(a.a + r * a.lda + h * N + n) + *(const f32x4*)(a.dt_bias + h * N + n);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = tid + 512 * i, t = e / (NMAX / 4), n = e % (NMAX / 4) * 4;
+      *(f32x4*)&L.k[t][n] = k[i], *(f32x4*)&L.q[t][n] = q[i];
+      if (a.channel_decay) {
+        f32x4 g = {1.f, 1.f, 1.f, 1.f};
+        if (t < nt && n < N)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) g[x] = decay_of(z[i][x], rate);
+        *(f32x4*)&L.g[t][n] = g;
+      }
+    }
+  } else {
+    for (int e = tid; e < CHUNK * NMAX; e += 512) {
+      const int t = e / NMAX, n = e % NMAX;
+      const bool there = t < nt && n < N;
+      const long long r = r0 + t;
+      L.k[t][n] = there ? a.k[r * a.ldk + j * N + n] : 0.f;
+      L.q[t][n] = there ? a.q[r * a.ldq + j * N + n] : 0.f;
+      if (a.channel_decay)
+        L.g[t][n] = there ? decay_of(a.a[r * a.lda + h * N + n] + a.dt_bias[h * N + n], rate) : 1.f;
+    }
+  }
+  if (!a.channel_decay) {  // one decay a head: a thread makes that of its row
+    const int t = tid >> 3;
+    const float g = t < nt ? decay_of(a.a[(r0 + t) * a.lda + h] + a.dt_bias[h], rate) : 1.f;
+    for (int n = tid & 7; n < NMAX; n += 8) L.g[t][n] = g;
+  }
+  if (tid < CHUNK) L.beta[tid] = tid < nt ? sigmoid_f(a.beta[(r0 + tid) * a.ldbeta + h]) : 0.f;
+  for (int e = tid; e < CHUNK * LDT; e += 512) (&L.m[0][0])[e] = 0.f, (&L.b[0][0])[e] = 0.f;
+  __syncthreads();
+
+  {  // within a block of 16 tokens
+    const int blk = w & 3;
+    const bool of_b = w >= KT;
+    float faded[SUB][2], from_start[SUB][2], run[2] = {1.f, 1.f};  // faded: a token's k by the decays since
+    auto row_of = [&](auto full, int t) {
+      constexpr int COUNT = decltype(full)::value;
+      const int row = SUB * blk + t;
+      float with[2], sums[SUB];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int n = lane + 64 * c;
+        const float g = L.g[row][n];
+#pragma unroll
+        for (int s = 0; s < COUNT; ++s)
+          if (s < t) faded[s][c] *= g;
+        faded[t][c] = L.k[row][n];
+        with[c] = of_b ? L.q[row][n] : faded[t][c];
+        run[c] *= g;
+        from_start[t][c] = with[c] * run[c];
+      }
+#pragma unroll
+      for (int s = 0; s < COUNT; ++s) sums[s] = s <= t ? fmaf(faded[s][1], with[1], faded[s][0] * with[0]) : 0.f;
+      const float sum = sums_by_lane<COUNT>(sums);
+      // (stored here: else the rows' loads and sums run into one another and out of registers)
+      if (lane < (of_b ? t + 1 : t)) (of_b ? L.b : L.m)[row][SUB * blk + lane] = sum;
+      asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int t = 0; t < 8; ++t) row_of(std::integral_constant<int, 8>{}, t);
+#pragma unroll
+    for (int t = 8; t < SUB; ++t) row_of(std::integral_constant<int, 16>{}, t);
+    __syncthreads();  // (the plain rows have been read)
+#pragma unroll
+    for (int t = 0; t < SUB; ++t)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int row = SUB * blk + t, n = lane + 64 * c;
+        (of_b ? L.q : L.k)[row][n] = from_start[t][c];
+        if (!of_b) L.g[row][n] = faded[t][c];
+      }
+    if (!of_b) L.block[blk][lane] = run[0], L.block[blk][lane + 64] = run[1];
+  }
+  __syncthreads();
+
+  // K~ and Q~ as fragments, rows tokens
+#pragma unroll
+  for (int e = tid; e < KT * NT * 64; e += 512) {
+    const int mt = e / (NT * 64), row = SUB * mt + (e & 15), n = e / 64 % NT * 16 + (e >> 4 & 3) * 4;
+    f32x4 f = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+    for (int i = 0; i < KT - 1; ++i)
+      if (i < mt) f *= *(const f32x4*)&L.block[i][n];
+    *(f32x4*)(to + AT_KEYS + e * 4) = *(const f32x4*)&L.k[row][n] * f;
+    *(f32x4*)(to + AT_QUERIES + e * 4) = *(const f32x4*)&L.q[row][n] * f;
+  }
+  // what the state is updated with, rows key channels
+#pragma unroll
+  for (int e = tid; e < NT * KT * 64; e += 512) {
+    const int kb = e / 64 % KT, n = e / (KT * 64) * 16 + (e & 15), t = SUB * kb + (e >> 4 & 3) * 4;
+    float f = 1.f;
+#pragma unroll
+    for (int i = 1; i < KT; ++i)
+      if (i > kb) f *= L.block[i][n];
+    *(f32x4*)(to + AT_UPDATE + e * 4) = (f32x4){L.g[t][n] * f, L.g[t + 1][n] * f, L.g[t + 2][n] * f, L.g[t + 3][n] * f};
+  }
+  if (tid < NMAX) {
+    float f = 1.f;
+    for (int i = 0; i < KT; ++i) f *= L.block[i][tid];
+    to[AT_DECAY + tid] = f;
+  }
+  // between blocks: six pairs of A and of B
+  const int c = lane & 15, g = lane >> 4;
+  for (int u = w; u < 12; u += 8) {
+    const int pair = u >> 1, i = pair < 1 ? 1 : pair < 3 ? 2 : 3, jb = pair - i * (i - 1) / 2;
+    const float(*rows)[LD] = (u & 1) ? L.q : L.k;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int nb = 0; nb < NT; ++nb) {
+      const int n = 16 * nb + 4 * g;
+      f32x4 col = *(const f32x4*)&L.g[SUB * jb + c][n];
+      for (int x = jb + 1; x < i; ++x) col *= *(const f32x4*)&L.block[x][n];
+      acc[nb & 1] = step4(*(const f32x4*)&rows[SUB * i + c][n], col, acc[nb & 1]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ((u & 1) ? L.b : L.m)[SUB * i + 4 * g + e][SUB * jb + c] = acc[0][e] + acc[1][e];
+  }
+  // the inverse of I + diag(beta) A: the blocks on the diagonal by substitution, a lane a column
+  if (w < KT && lane < SUB) {
+    float x[SUB];
+#pragma unroll
+    for (int t = 0; t < SUB; ++t) {
+      float sum = 0.f;
+#pragma unroll
+      for (int s = 0; s < t; ++s) sum = fmaf(L.m[SUB * w + t][SUB * w + s], x[s], sum);
+      x[t] = (t == lane ? 1.f : 0.f) - L.beta[SUB * w + t] * sum;
+      L.inv[w][t][lane] = x[t];
+    }
+  }
+  __syncthreads();
+  // ... and wavefront w the column of blocks w: X_ww is that inverse, X_iw = -X_ii sum_m (beta A)_im X_mw
+  f32x4 X[KT];
+#pragma unroll
+  for (int i = 0; i < KT; ++i) X[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < KT; ++i) {
+    if (w < KT && i == w) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) X[i][e] = L.inv[i][4 * g + e][c];
+    } else if (i > w) {
+      f32x4 Z = {0.f, 0.f, 0.f, 0.f};
+      const float bi = L.beta[SUB * i + c];
+#pragma unroll
+      for (int x = 0; x < i; ++x)
+        if (x >= w) Z = step4(*(const f32x4*)&L.m[SUB * i + c][SUB * x + 4 * g] * bi, X[x], Z);
+      X[i] = step4(*(const f32x4*)&L.inv[i][c][4 * g] * -1.f, Z, X[i]);
+    }
+  }
+  __syncthreads();  // (A has been read)
+  if (w < KT) {
+#pragma unroll
+    for (int i = 0; i < KT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) L.m[SUB * i + 4 * g + e][SUB * w + c] = X[i][e] * L.beta[SUB * w + c];
+  }
+  __syncthreads();
+  for (int e = tid; e < KT * KT * 64; e += 512) {
+    const int row = SUB * (e / (KT * 64)) + (e & 15), s = e / 64 % KT * SUB + (e >> 4 & 3) * 4;
+    *(f32x4*)(to + AT_T + e * 4) = *(const f32x4*)&L.m[row][s];
+    *(f32x4*)(to + AT_B + e * 4) = *(const f32x4*)&L.b[row][s];
+  }
+}
+
+__device__ inline void lds_barrier() {  // this wavefront's LDS accesses are done, its loads from memory need not be
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// One workgroup of eight wavefronts a (sequence, head, 16 columns of the values); wavefront w holds channels 16 w .. + 15
+// of the state.  A chunk: wavefronts 0 to 3 make 16 tokens of V - K~ S each and 4 to 7 of Q~ S; then 0 to 3 of U; then
+// all update the state and 4 to 7 add B U.  Tiles cross between wavefronts through LDS in lane order.  A chunk's
+// operands are asked for as soon as the chunk before has used theirs.
+__global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
+  __shared__ f32x4 Ss[NT][64], Ws[KT][64], Us[KT][64];
+  const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int c = lane & 15, g = lane >> 4, p = blockIdx.y * 16 + c, mt = w & 3;
+  const bool second = w >= KT;  // Q~, B and the results
+  const long long r0 = a.cu_rows[b], r1 = a.cu_rows[b + 1];
+  const int chunks = (int)((r1 - r0 + CHUNK - 1) / CHUNK);
+  if (chunks <= 0) return;
+  const float* part = a.scratch + ((long long)first_chunk(a.cu_rows, b) * a.heads + h) * PART;
+  const long long step = (long long)a.heads * PART;
+  float* sp = a.state + (((long long)a.seq_slot[b] * a.heads + h) * a.P + min(p, a.P - 1)) * a.N;
+  const bool live = p < a.P;
+  f32x4 S;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int n = 16 * w + 4 * g + e;
+    S[e] = live && n < a.N ? sp[n] : 0.f;
+  }
+  Ss[w][lane] = S;
+
+  f32x4 rows[NT], tri[KT], upd[KT], V = {0.f, 0.f, 0.f, 0.f}, decay;
+  auto ask_rows = [&](const float* from) {
+#pragma unroll
+    for (int nb = 0; nb < NT; ++nb)
+      rows[nb] = *(const f32x4*)(from + (second ? AT_QUERIES : AT_KEYS) + ((mt * NT + nb) * 64 + lane) * 4);
+  };
+  auto ask_tri = [&](const float* from) {
+#pragma unroll
+    for (int kb = 0; kb < KT; ++kb)
+      if (kb <= mt) tri[kb] = *(const f32x4*)(from + (second ? AT_B : AT_T) + ((mt * KT + kb) * 64 + lane) * 4);
+  };
+  auto ask_upd = [&](const float* from) {
+#pragma unroll
+    for (int kb = 0; kb < KT; ++kb) upd[kb] = *(const f32x4*)(from + AT_UPDATE + ((w * KT + kb) * 64 + lane) * 4);
+    decay = *(const f32x4*)(from + AT_DECAY + 16 * w + 4 * g);
+  };
+  auto ask_v = [&](long long c0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const long long r = c0 + SUB * mt + 4 * g + e;
+      V[e] = live && r < r1 ? a.v[r * a.ldv + (long long)h * a.P + p] : 0.f;
+    }
+  };
+  ask_rows(part), ask_tri(part), ask_upd(part);
+  if (!second) ask_v(r0);
+  lds_barrier();
+  for (int i = 0; i < chunks; ++i, part += step) {
+    const bool more = i + 1 < chunks;
+    const long long c0 = r0 + (long long)i * CHUNK;
+    f32x4 acc[4];  // (four chains of products: their roundings are smaller, and none waits for the one before it)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) acc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int nb = 0; nb < NT; ++nb) acc[nb & 3] = step4(rows[nb], Ss[nb][lane], acc[nb & 3]);
+    f32x4 Y = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    if (more) ask_rows(part + step);
+    if (!second) {
+      Ws[mt][lane] = V - Y;
+      if (more) ask_v(c0 + CHUNK);
+    }
+    lds_barrier();
+    if (!second) {
+      f32x4 U = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < KT; ++kb)
+        if (kb <= mt) U = step4(tri[kb], Ws[kb][lane], U);
+      Us[mt][lane] = U;
+      if (more) ask_tri(part + step);
+    }
+    lds_barrier();
+    // (what the chunk adds is summed by itself: one rounding at the state's size a chunk, not one a product)
+    f32x4 add[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int kb = 0; kb < KT; ++kb) add[kb & 1] = step4(upd[kb], Us[kb][lane], add[kb & 1]);
+    S = S * decay + (add[0] + add[1]);
+    Ss[w][lane] = S;
+    if (more) ask_upd(part + step);
+    if (second) {
+      f32x4 own = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < KT; ++kb)
+        if (kb <= mt) own = step4(tri[kb], Us[kb][lane], own);
+      Y += own;
+      if (more) ask_tri(part + step);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const long long r = c0 + SUB * mt + 4 * g + e;
+        if (live && r < r1) a.out[r * a.ldo + (long long)h * a.P + p] = Y[e];
+      }
+    }
+    lds_barrier();
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int n = 16 * w + 4 * g + e;
+    if (live && n < a.N) sp[n] = S[e];
+  }
+}
+
+}  // namespace
+
+// Float32 scratch with which a launch runs in chunks (0: token by token).  Microseconds a launch, token by token and in
+// chunks, 16 heads of 128 x 128 over 8 q/k heads, a decay every channel (the unit vectors' launch in both): 48 tokens
+// 32 / 34, 64 tokens 40 / 35, 256 tokens 124 / 49, 2 048 tokens 900 / 172 (one decay a head 651 / 169), 8 192 tokens
+// 3 560 / 715, three sequences of 257, 878 and 1 500 tokens 769 / 208, eight of 60 92 / 60, eight of 512 584 / 242.  Of
+// 2 048 tokens' 172 the preparation is 50 (21 for a workgroup by itself, a compute unit's LDS holds one), the walk 110
+// (3.3 a chunk, of which the matrix instructions of a SIMD are 1.5: half the chip is idle with 128 workgroups).
+// Relative error against 64 bits at 2 048 tokens: 3.3e-7 both ways with a decay every channel, 4.9e-7 and 5.1e-7
+// with one a head; of the state at their end 3.4e-7 and 3.3e-7, 4.5e-7 both.
+constexpr int LQ_DELTA_MIN = 56;
+extern "C" long long lq_delta_scan_workspace(int rows, int batch, int heads, int Dk, int P, int max_rows) {
+  if (rows <= 0 || batch <= 0 || heads <= 0 || P <= 0 || Dk <= 0 || Dk > NMAX || max_rows < LQ_DELTA_MIN) return 0;
+  return (long long)(rows / CHUNK + batch) * heads * PART;
+}
+
+// q and k hold unit vectors already.  -> 0, or -2
+int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* beta,
+                    int ldbeta, const float* a, int lda, const float* dt_bias, const float* a_log, float* state, float* out,
+                    int ldo, int heads, int kv_heads, int Dk, int P, const int* seq_slot, const int* cu_rows, int batch,
+                    int rows, int channel_decay, float* scratch, hipStream_t stream) {
+  DeltaArgs d = {q, k, v, beta, a, dt_bias, a_log, ldq, ldk, ldv, ldbeta, lda, ldo, state, out, scratch,
+                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows};
+  const bool quads = Dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && (!channel_decay || lda % 4 == 0) &&
+                     (((uintptr_t)q | (uintptr_t)k | (channel_decay ? (uintptr_t)a | (uintptr_t)dt_bias : 0)) & 15) == 0;
+  const auto prepare = quads ? delta_prepare_kernel<true> : delta_prepare_kernel<false>;
+  static bool configured[2] = {false, false};
+  if (!configured[quads]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)prepare, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(Prepared));
+    if (e != hipSuccess) {
+      lq_set_error("delta_scan: cannot reserve %d bytes of LDS: %s", (int)sizeof(Prepared), hipGetErrorString(e));
+      return -2;
+    }
+    configured[quads] = true;
+  }
+  prepare<<<dim3(rows / CHUNK + batch, heads), 512, sizeof(Prepared), stream>>>(d);
+  LQ_CHECK_LAUNCH("delta_scan(chunks)");
+  delta_walk_kernel<<<dim3((unsigned)batch * heads, lq_ceil_div(P, 16)), 512, 0, stream>>>(d);
+  LQ_CHECK_LAUNCH("delta_scan(walk over chunks)");
+  return 0;
+}

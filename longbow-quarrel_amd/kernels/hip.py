@@ -20,7 +20,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 13  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 14  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -1075,16 +1075,26 @@ class HipKernels:
                                            c_float(den_eps), c_float(eps), _ptr(out), c_int(_code(out)), c_int(ldo),
                                            c_int(rows), c_int(heads), c_int(nz // heads), self.stream))
 
+    @query
+    def delta_scan_workspace(self, rows: int, batch: int, heads: int, key_dim: int, value_dim: int, max_rows: int) -> int:
+        """Float32 entries of scratch with which `delta_scan` runs in chunks of tokens (0: token by token)."""
+        self.lib.lq_delta_scan_workspace.restype = c_longlong
+        return int(self.lib.lq_delta_scan_workspace(c_int(rows), c_int(batch), c_int(heads), c_int(key_dim),
+                                                    c_int(value_dim), c_int(max_rows)))
+
     def delta_scan(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, a: torch.Tensor,
                    dt_bias: torch.Tensor, a_log: torch.Tensor, state: torch.Tensor, out: torch.Tensor, heads: int,
                    kv_heads: int, key_dim: int, value_dim: int, q_scale: float, unit_eps: float,
-                   seq_slot: torch.Tensor, cu_rows: torch.Tensor, batch: int, channel_decay: bool = False) -> None:
+                   seq_slot: torch.Tensor, cu_rows: torch.Tensor, batch: int, channel_decay: bool = False,
+                   max_rows: int = 0, workspace: Optional[torch.Tensor] = None) -> None:
         """The gated delta rule along every sequence of the step, token by token: q and k made unit vectors per
         head (x / sqrt(sum x^2 + unit_eps)), q times q_scale, beta = sigmoid(beta), g = exp(-exp(a_log)
         softplus(a + dt_bias)); S <- g S, u = beta (v - S^T k), S <- S + k u^T, out = S^T q.  state [slots, heads,
         value_dim, key_dim].  All float32.  q and k are overwritten with their unit vectors.  The decay is one number
         a head (a [rows, heads], dt_bias [heads]) or, with `channel_decay`, one for every key channel of every head
-        (a [rows, heads * key_dim], dt_bias [heads * key_dim]), multiplying the state's rows of that channel."""
+        (a [rows, heads * key_dim], dt_bias [heads * key_dim]), multiplying the state's rows of that channel.
+        `max_rows` (the most rows a sequence brings) and `workspace` (`delta_scan_workspace(...)` floats) let long
+        portions run in chunks of tokens, whose sums are in another order."""
         rows = q.shape[0]
         n_decay = heads * key_dim if channel_decay else heads
         for t, what, cols in ((q, "q", kv_heads * key_dim), (k, "k", kv_heads * key_dim), (v, "v", heads * value_dim),
@@ -1097,6 +1107,8 @@ class HipKernels:
         self._f32(state, "delta_scan: state")
         if state.dim() != 4 or tuple(state.shape[1:]) != (heads, value_dim, key_dim) or not state.is_contiguous():
             raise KernelLibraryError("delta_scan: state must be dense [slots, heads, value_dim, key_dim]")
+        if workspace is not None:
+            self._f32(workspace, "delta_scan: workspace", workspace.numel())
         self._i32(seq_slot, "seq_slot", batch)
         self._i32(cu_rows, "cu_rows", batch + 1)
         ld = self._rows2d
@@ -1106,7 +1118,8 @@ class HipKernels:
                                            c_int(ld(out, "out")), c_int(heads), c_int(kv_heads), c_int(key_dim),
                                            c_int(value_dim), c_float(q_scale), c_float(unit_eps), _ptr(seq_slot),
                                            _ptr(cu_rows), c_int(batch), c_int(rows), c_int(1 if channel_decay else 0),
-                                           self.stream))
+                                           c_int(max_rows), _ptr(workspace),
+                                           c_longlong(0 if workspace is None else workspace.numel()), self.stream))
 
     def gated_rmsnorm(self, y: torch.Tensor, z: torch.Tensor, weight: Optional[torch.Tensor], eps: float, group: int,
                       out: torch.Tensor, gate_first: bool = True, gate: str = "silu") -> None:

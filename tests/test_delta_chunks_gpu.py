@@ -1,0 +1,41 @@
+"""The gated delta rule in chunks of 64 tokens against the walk token by token (no scratch given), at the sizes where
+chunks, blocks of 16 tokens, value slices and rows of key channels end."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lens,H,G,N,P,channel,shift", [
+    ([64], 2, 1, 128, 128, True, 0.0), ([1, 65, 16], 4, 2, 128, 128, False, 0.0), ([129, 63], 3, 3, 128, 128, True, 0.0),
+    ([200], 2, 2, 48, 40, True, 0.0), ([80, 17, 128], 2, 1, 64, 256, False, 0.0), ([70], 2, 1, 30, 17, True, 0.0),
+    ([66], 1, 1, 16, 16, False, 0.0), ([130], 2, 1, 128, 32, True, 8.0), ([130], 2, 1, 128, 32, False, 8.0),
+    ([130], 2, 1, 128, 32, True, -8.0), ([57] + [1] * 70, 2, 1, 64, 32, True, 0.0)])
+def test_chunks_of_the_delta_rule(lens, H, G, N, P, channel, shift):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(N * P + len(lens))
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, batch = sum(lens), len(lens)
+    q, k, v, beta = rand(rows, G * N), rand(rows, G * N), rand(rows, H * P), rand(rows, H)
+    k[1::3] = 0.9 * k[0::3][: k[1::3].shape[0]] + 0.1 * k[1::3]  # keys that overwrite one another
+    n_decay = H * N if channel else H
+    a, dt_bias, a_log = 0.3 * rand(rows, n_decay), rand(n_decay) - 3.0 + shift, 0.5 * rand(H) + 1.0
+    state = rand(batch, H, P, N)
+    cu = i32(sum(lens[:b]) for b in range(batch + 1))
+    kn = HipKernels()
+    need = kn.delta_scan_workspace(rows, batch, H, N, P, max(lens))
+    assert need > 0 and kn.delta_scan_workspace(batch, batch, H, N, P, 1) == 0
+    got = {}
+    for scratch in (None, torch.full((need,), float("nan"), device="cuda")):
+        out, end, qq, kk = torch.full((rows, H * P), float("nan"), device="cuda"), state.clone(), q.clone(), k.clone()
+        more = {} if scratch is None else dict(max_rows=max(lens), workspace=scratch)
+        kn.delta_scan(qq, kk, v, beta, a, dt_bias, a_log, end, out, H, G, N, P, N ** -0.5, 1e-6,
+                      i32(reversed(range(batch))), cu, batch, channel_decay=channel, **more)
+        got[scratch is not None] = out, end
+    for walked, chunked in zip(got[False], got[True]):
+        # Every step is a contraction, so an error made at a token is not enlarged by the later ones: at most some 4
+        # roundings of 2^-24 a token at the result's size, 200 tokens.
+        assert torch.isfinite(walked).all()
+        assert (walked - chunked).abs().max() <= 200 * 4 * 2.0 ** -24 * walked.abs().max()
