@@ -51,6 +51,27 @@ extern "C" int lq_linear(const void* x, const void* w, void* out, int in_dtype, 
   return lq_gemm_generic(x, w, out, in_dtype, out_dtype, M, N, K, lda, ldw, ldc, stream);
 }
 
+int lq_gemm_grouped(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc,
+                    const int* counts, int groups, long long w_step, int packed, hipStream_t stream);
+
+// Whether lq_linear_grouped takes weights [N, K] of a mixture of `groups` experts (else: a product an expert).
+extern "C" int lq_linear_grouped_supported(int in_dtype, int groups, int N, int K, int force_generic) {
+  return !force_generic && in_dtype == LQ_BF16 && groups >= 1 && groups <= 64 && K % 64 == 0 && K >= 512 && N > 0;
+}
+
+// out (32-bit) = x . W_i^T for x's rows in runs, counts[i] rows (on the device) for expert i, whose weight lies i * w_step
+// entries behind the first's.  Rows of x beyond the counts' sum are not read, and their rows of out not written.
+extern "C" int lq_linear_grouped(const void* x, const void* w, void* out, int in_dtype, int M, int N, int K, int lda, int ldw,
+                                 int ldc, const int* counts, int groups, long long w_step, int w_packed, hipStream_t stream) {
+  LQ_REQUIRE(M > 0 && lda >= K && ldw >= K && ldc >= N && w_step >= 0, "linear_grouped: bad sizes or strides");
+  LQ_REQUIRE(x && w && out && counts, "linear_grouped: null pointer");
+  LQ_REQUIRE(lq_linear_grouped_supported(in_dtype, groups, N, K, 0) && lq_gemm_mfma_accepts(x, w, in_dtype, K, lda, ldw) &&
+                 w_step % 8 == 0,
+             "linear_grouped: %d experts of [%d, %d] are not taken", groups, N, K);
+  LQ_REQUIRE(!w_packed || (ldw == K && N % 8 == 0 && w_step % (8ll * K) == 0), "linear_grouped: these weights are not packed rows in eights");
+  return lq_gemm_grouped(x, w, out, M, N, K, lda, ldw, ldc, counts, groups, w_step, w_packed, stream);
+}
+
 // Whether lq_linear_swiglu takes this problem (else: lq_linear into [M, 2I] and lq_swiglu).
 extern "C" int lq_linear_swiglu_supported(int in_dtype, int N, int K) {
   return in_dtype == LQ_BF16 && N % 16 == 0 && K % 8 == 0;

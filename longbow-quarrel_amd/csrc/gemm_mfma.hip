@@ -320,10 +320,19 @@ struct PipeShape {
   __device__ static int swizzle(int row) { return (row / (256 / ROW_BYTES)) & (CPR - 1); }
 };
 
-template <int GM, int GN, int WM, int WN, int BK, int STAGES, int EPI, typename TO, bool ALTERNATE = false>
+// A's rows in groups that lie one behind the other, counts[i] rows of group i, each with a weight of its own
+// (group i's begins i * w_step entries behind the first's): the mixture of experts' products in one launch.  The host does
+// not know the counts: the grid holds as many row tiles as they can come to, and a workgroup finds its own.
+struct Groups {
+  const int* counts;
+  int n;  // at most 64
+  long long w_step;
+};
+
+template <int GM, int GN, int WM, int WN, int BK, int STAGES, int EPI, typename TO, bool ALTERNATE = false, bool GROUPED = false>
 __global__ __launch_bounds__(GM * GN * 64, 2) void gemm_bf16_pipelined_kernel(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw, TO* __restrict__ C, int ldc, int M,
-    int N, int K, int tiles_m, int tiles_n, int k_share, long long split_stride, int packed) {
+    int N, int K, int tiles_m, int tiles_n, int k_share, long long split_stride, int packed, Groups groups) {
   using S = PipeShape<GM, GN, WM, WN, BK, STAGES>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char plds[];
 
@@ -331,7 +340,24 @@ __global__ __launch_bounds__(GM * GN * 64, 2) void gemm_bf16_pipelined_kernel(
   int pid = blockIdx.x;
   if (total % 8 == 0) pid = (pid % 8) * (total / 8) + pid / 8;  // one XCD walks a contiguous run of tiles
   int tm = pid % tiles_m, tn = pid / tiles_m;
-  if (total % 8 == 0 && tiles_m > 8 && (total / 8) % tiles_m == 0) {
+  if constexpr (GROUPED) {
+    const int lane = threadIdx.x & 63, rows = lane < groups.n ? groups.counts[lane] : 0;
+    const int mine = (rows + S::BM - 1) / S::BM;
+    int upto = mine, rows_upto = rows;  // tiles and rows of the groups up to this lane's
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int t = __shfl_up(upto, off, 64), r = __shfl_up(rows_upto, off, 64);
+      if (lane >= off) upto += t, rows_upto += r;
+    }
+    const unsigned long long past = __ballot(upto > tm);
+    if (past == 0) return;  // (the whole workgroup: fewer tiles than there could have been)
+    const int at = __ffsll(past) - 1;
+    tm = __builtin_amdgcn_readfirstlane(tm - __shfl(upto - mine, at, 64));
+    M = __builtin_amdgcn_readfirstlane(__shfl(rows, at, 64));
+    const int first = __builtin_amdgcn_readfirstlane(__shfl(rows_upto - rows, at, 64));
+    A += (long long)first * lda, C += (long long)first * ldc;
+    W += __builtin_amdgcn_readfirstlane(at) * groups.w_step;
+  } else if (total % 8 == 0 && tiles_m > 8 && (total / 8) % tiles_m == 0) {
     // The 32 tiles that an XCD works on together should share operands both ways: 8 row tiles by 4 column
     // tiles ask for 12 tiles' worth of operand rows, 32 row tiles of one column tile for 33.  The XCD's run
     // is whole columns of tiles: walk them four columns at a time, and each such band in windows of 8 row
@@ -577,13 +603,14 @@ __global__ __launch_bounds__(GM * GN * 64, 2) void gemm_bf16_pipelined_kernel(
   }
 }
 
-template <int GM, int GN, int WM, int WN, int BK, int STAGES, int EPI, typename TO, bool ALTERNATE = false>
+template <int GM, int GN, int WM, int WN, int BK, int STAGES, int EPI, typename TO, bool ALTERNATE = false, bool GROUPED = false>
 int launch_pipelined(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc,
-                     int splits, long long split_stride, hipStream_t stream, int packed = 0) {
+                     int splits, long long split_stride, hipStream_t stream, int packed = 0, Groups groups = Groups()) {
   using S = PipeShape<GM, GN, WM, WN, BK, STAGES>;
   LQ_REQUIRE(!packed || (BK == 64 && N % 8 == 0), "linear: a packed weight needs slabs of 64 k and rows in eights");
-  const int tiles_m = lq_ceil_div(M, S::BM), tiles_n = lq_ceil_div(N, S::BN);
-  auto kernel = gemm_bf16_pipelined_kernel<GM, GN, WM, WN, BK, STAGES, EPI, TO, ALTERNATE>;
+  // (in groups: each may end with a tile that is part empty)
+  const int tiles_m = GROUPED ? M / S::BM + groups.n : lq_ceil_div(M, S::BM), tiles_n = lq_ceil_div(N, S::BN);
+  auto kernel = gemm_bf16_pipelined_kernel<GM, GN, WM, WN, BK, STAGES, EPI, TO, ALTERNATE, GROUPED>;
   static bool configured = false;
   if (!configured && S::LDS_BYTES > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -603,7 +630,7 @@ int launch_pipelined(const void* A, const void* W, void* C, int M, int N, int K,
              "linear: rows too far apart for the tile's 32-bit offsets");
   kernel<<<dim3((int)blocks, splits), S::NW * 64, S::LDS_BYTES, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, (TO*)C, ldc, M, N, K, tiles_m, tiles_n, K / splits, split_stride,
-      packed);
+      packed, groups);
   LQ_CHECK_LAUNCH("linear(mfma pipelined)");
   return 0;
 }
@@ -1237,6 +1264,20 @@ bool lq_gemm_mfma_accepts(const void* x, const void* w, int in_dtype, int K, int
 }
 
 bool lq_gemm_packable(int N, int K) { return gemm_packable(N, K); }
+
+// x [M, K] bfloat16, its rows in `groups` runs of counts[i] (on the device; together at most M), times group i's weight
+// [N, K] at w + i * w_step, into 32-bit out [M, N].
+int lq_gemm_grouped(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc,
+                    const int* counts, int groups, long long w_step, int packed, hipStream_t stream) {
+  const Groups g = {counts, groups, w_step};
+  // 256-row tiles from 256 rows an expert on; fewer leave most of such a tile empty.  Microseconds, 8 experts, a launch an
+  // expert / 128 x 128 tiles / 256 x 256 tiles: 1 024 rows of 3 584 x 2 048 108 / 42 / 42, of 2 048 x 3 584 166 / 36 / 61;
+  // 2 048 rows 142 / 65 / 46 and 219 / 67 / 65; 8 002 rows 186 / 190 / 151 and 242 / 178 / 151; 8 192 rows of
+  // 14 336 x 4 096 1 023 / 1 294 / 886.
+  if (M / groups >= 256)
+    return launch_pipelined<4, 2, 2, 4, 64, 2, EPI_NONE, float, true, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+  return launch_pipelined<4, 2, 1, 2, 64, 4, EPI_NONE, float, false, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+}
 
 int lq_gemm_mfma(const void* x, const void* w, void* out, int out_dtype, int M, int N, int K, int lda,
                  int ldw, int ldc, int epilogue, int splits, long long split_stride, int packed, hipStream_t stream) {

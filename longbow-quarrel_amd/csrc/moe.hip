@@ -141,35 +141,61 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(const T* __restrict__
   for (int c = threadIdx.x; c < width; c += 256) out[(long long)r * ldo + c] += w * to_f32(h[(long long)r * ldh + c]);
 }
 
+// VEC (1 or 4) neighbouring entries
+template <typename T, int VEC>
+__device__ inline void store_run(T* o, const float (&v)[VEC]) {
+  if constexpr (VEC == 4 && sizeof(T) == 2) {
+    uint2 packed;
+    packed.x = (uint32_t)f32_to_bf16(v[0]).bits | ((uint32_t)f32_to_bf16(v[1]).bits << 16);
+    packed.y = (uint32_t)f32_to_bf16(v[2]).bits | ((uint32_t)f32_to_bf16(v[3]).bits << 16);
+    *(uint2*)o = packed;
+  } else if constexpr (VEC == 4) {
+    *(float4*)o = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+    *o = from_f32<T>(v[0]);
+  }
+}
+
 // gu [rows, E, 2, ff] (gate then up of every expert), route [rows, E]; out [rows, E, ff]:
 // g = min(w gate, limit), u = clamp(w up, -limit, limit), y = g sigmoid(1.702 g) (u + 1) for a chosen expert (its
 // weight w on what it read: `on_input`; otherwise w multiplies y), 0 for the others.  `plain_silu`: the expert is
 // y = silu(gate) up without clamps.
-template <typename T>
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void moe_glu_kernel(const float* __restrict__ gu, long long ldg,
                                                       const float* __restrict__ route, T* __restrict__ out,
                                                       long long ldo, int E, int ff, float limit, int on_input,
                                                       int plain_silu) {
   const int r = blockIdx.y;
-  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int i = (blockIdx.x * 256 + threadIdx.x) * VEC;  // VEC entries a thread, all of one expert
   if (i >= E * ff) return;
   const int e = i / ff, c = i - e * ff;
   const float w = route[(long long)r * E + e];
-  float y = 0.f;
+  float y[VEC], gate[VEC], up[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) y[j] = 0.f;
   if (w >= 0.f) {
-    const float* p = gu + r * ldg + (long long)e * 2 * ff;
-    const float s = on_input ? w : 1.f;
-    if (plain_silu) {
-      const float g = p[c] * s;
-      y = g / (1.f + expf(-g)) * (p[ff + c] * s);
+    const float* p = gu + r * ldg + (long long)e * 2 * ff + c;
+    if constexpr (VEC == 4) {
+      const float4 a = *(const float4*)p, b = *(const float4*)(p + ff);
+      gate[0] = a.x, gate[1] = a.y, gate[2] = a.z, gate[3] = a.w, up[0] = b.x, up[1] = b.y, up[2] = b.z, up[3] = b.w;
     } else {
-      const float g = fminf(p[c] * s, limit);
-      const float u = fminf(fmaxf(p[ff + c] * s, -limit), limit);
-      y = g / (1.f + expf(-1.702f * g)) * (u + 1.f);
+      gate[0] = p[0], up[0] = p[ff];
     }
-    if (!on_input) y *= w;
+    const float s = on_input ? w : 1.f;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      if (plain_silu) {
+        const float g = gate[j] * s;
+        y[j] = g / (1.f + expf(-g)) * (up[j] * s);
+      } else {
+        const float g = fminf(gate[j] * s, limit);
+        const float u = fminf(fmaxf(up[j] * s, -limit), limit);
+        y[j] = g / (1.f + expf(-1.702f * g)) * (u + 1.f);
+      }
+      if (!on_input) y[j] *= w;
+    }
   }
-  out[r * ldo + i] = from_f32<T>(y);
+  store_run<T, VEC>(out + r * ldo + i, y);
 }
 
 // The same for experts without a gate: u [rows, E ff + shared], out likewise: out = act(u) w for a chosen expert's entries,
@@ -195,27 +221,18 @@ __global__ __launch_bounds__(256) void moe_act_kernel(const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < VEC; ++j) v[j] = activate(v[j], act) * w;
   }
-  T* o = out + r * ldo + i;
-  if constexpr (VEC == 4 && sizeof(T) == 2) {
-    uint2 packed;
-    packed.x = (uint32_t)f32_to_bf16(v[0]).bits | ((uint32_t)f32_to_bf16(v[1]).bits << 16);
-    packed.y = (uint32_t)f32_to_bf16(v[2]).bits | ((uint32_t)f32_to_bf16(v[3]).bits << 16);
-    *(uint2*)o = packed;
-  } else if constexpr (VEC == 4) {
-    *(float4*)o = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    *o = from_f32<T>(v[0]);
-  }
+  store_run<T, VEC>(out + r * ldo + i, v);
 }
 
 // ---- a step's rows sorted by expert ----------------------------------------------------------------------------------
+constexpr int SORT_THREADS = 1024;  // (the walk over the rows is a chain of barriers)
 // counts[e] = rows that chose expert e; one workgroup an expert.
-__global__ __launch_bounds__(256) void moe_count_kernel(const float* __restrict__ route, int rows, int E,
+__global__ __launch_bounds__(SORT_THREADS) void moe_count_kernel(const float* __restrict__ route, int rows, int E,
                                                         int* __restrict__ counts) {
   __shared__ float red[16];
   const int e = blockIdx.x;
   float n = 0.f;  // (counts of up to 2^24 rows are whole numbers in 32-bit floats)
-  for (int r = threadIdx.x; r < rows; r += 256) n += route[(long long)r * E + e] >= 0.f ? 1.f : 0.f;
+  for (int r = threadIdx.x; r < rows; r += SORT_THREADS) n += route[(long long)r * E + e] >= 0.f ? 1.f : 0.f;
   n = block_sum(n, red);
   if (threadIdx.x == 0) counts[e] = (int)n;
 }
@@ -223,11 +240,11 @@ __global__ __launch_bounds__(256) void moe_count_kernel(const float* __restrict_
 // Expert e's rows, in ascending order, take the places offset(e) .. offset(e) + counts[e] - 1 of the sorted list
 // (offset: the counts of the experts before it): order[place] = row, weight[place] = the row's weight for the expert,
 // place_of[row, e] = place (-1 for an expert the row did not choose).  One workgroup an expert walks the rows in
-// chunks of 256 with a running count, so the order does not depend on timing.
-__global__ __launch_bounds__(256) void moe_place_kernel(const float* __restrict__ route, int rows, int E,
+// chunks of SORT_THREADS with a running count, so the order does not depend on timing.
+__global__ __launch_bounds__(SORT_THREADS) void moe_place_kernel(const float* __restrict__ route, int rows, int E,
                                                         const int* __restrict__ counts, int* __restrict__ order,
-                                                        float* __restrict__ weight, int* __restrict__ place_of) {
-  __shared__ int wave_n[4];
+                                                        float* __restrict__ weight, int* __restrict__ place_of, int places) {
+  __shared__ int wave_n[SORT_THREADS / 64];
   __shared__ int base;
   const int e = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (threadIdx.x == 0) {
@@ -236,7 +253,7 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const float* __restrict_
     base = off;
   }
   __syncthreads();
-  for (int r0 = 0; r0 < rows; r0 += 256) {
+  for (int r0 = 0; r0 < rows; r0 += SORT_THREADS) {
     const int r = r0 + threadIdx.x;
     const float w = r < rows ? route[(long long)r * E + e] : -1.f;
     const bool chosen = w >= 0.f;
@@ -249,32 +266,44 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const float* __restrict_
     if (chosen) order[at] = r, weight[at] = w;
     if (r < rows) place_of[(long long)r * E + e] = chosen ? at : -1;
     __syncthreads();
-    if (threadIdx.x == 0) base += wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
+    if (threadIdx.x == 0) for (int i = 0; i < SORT_THREADS / 64; ++i) base += wave_n[i];
     __syncthreads();
   }
+  if (e == E - 1)  // places that nobody takes name a row that there is, with no weight
+    for (int at = base + threadIdx.x; at < places; at += SORT_THREADS) order[at] = 0, weight[at] = -1.f;
 }
 
-// dst[i, :] = src[order[i], :] (16-bit or 32-bit rows)
-template <typename T>
-__global__ __launch_bounds__(256) void moe_gather_kernel(const T* __restrict__ src, int lds_, const int* __restrict__ order,
-                                                         T* __restrict__ dst, int width) {
-  const T* s = src + (long long)order[blockIdx.x] * lds_;
-  T* d = dst + (long long)blockIdx.x * width;
+// dst[i, :] = src[order[i], :], rows of `width` units
+template <typename U>
+__global__ __launch_bounds__(256) void moe_gather_kernel(const U* __restrict__ src, long long ld, const int* __restrict__ order,
+                                                         U* __restrict__ dst, int width) {
+  const U* s = src + (long long)order[blockIdx.x] * ld;
+  U* d = dst + (long long)blockIdx.x * width;
   for (int i = threadIdx.x; i < width; i += 256) d[i] = s[i];
 }
 
 // out[r, :] = the sum, over the experts that row r chose in ascending order, of ys[place_of[r, e], :]
+template <int VEC>
 __global__ __launch_bounds__(256) void moe_scatter_kernel(const float* __restrict__ ys, const int* __restrict__ place_of, int E,
                                                           float* __restrict__ out, int ldo, int width) {
   const int r = blockIdx.x;
   const int* places = place_of + (long long)r * E;
-  for (int i = threadIdx.x; i < width; i += 256) {
-    float acc = 0.f;
+  for (int i = threadIdx.x * VEC; i < width; i += 256 * VEC) {
+    float acc[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) acc[j] = 0.f;
     for (int e = 0; e < E; ++e) {
       const int at = places[e];
-      if (at >= 0) acc += ys[(long long)at * width + i];
+      if (at < 0) continue;
+      const float* y = ys + (long long)at * width + i;
+      if constexpr (VEC == 4) {
+        const float4 q = *(const float4*)y;
+        acc[0] += q.x, acc[1] += q.y, acc[2] += q.z, acc[3] += q.w;
+      } else {
+        acc[0] += y[0];
+      }
     }
-    out[(long long)r * ldo + i] = acc;
+    store_run<float, VEC>(out + (long long)r * ldo + i, acc);
   }
 }
 
@@ -326,16 +355,24 @@ extern "C" int lq_moe_glu(const float* gu, long long ldg, const float* route, vo
              rows, experts, ff);
   LQ_REQUIRE(ldg >= 2ll * experts * ff && ldo >= (long long)experts * ff, "moe_glu: a row stride is smaller than its row");
   LQ_REQUIRE(gu && route && out, "moe_glu: null pointer");
+  LQ_REQUIRE(out_dtype == LQ_F32 || out_dtype == LQ_BF16, "moe_glu: unknown dtype %d", out_dtype);
+  // four entries a thread where they lie in whole vectors
+  const bool quads = ff % 4 == 0 && ldg % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)gu & 15) == 0 &&
+                     ((uintptr_t)out & (out_dtype == LQ_BF16 ? 7 : 15)) == 0;
   for (int r0 = 0; r0 < rows; r0 += 65535) {
     const int nr = rows - r0 < 65535 ? rows - r0 : 65535;
-    dim3 grid(lq_ceil_div(experts * ff, 256), nr);
-    if (out_dtype == LQ_F32)
-      moe_glu_kernel<float><<<grid, 256, 0, stream>>>(gu + r0 * ldg, ldg, route + (long long)r0 * experts,
-                                                      (float*)out + r0 * ldo, ldo, experts, ff, limit, on_input, plain_silu);
-    else if (out_dtype == LQ_BF16)
-      moe_glu_kernel<bf16_t><<<grid, 256, 0, stream>>>(gu + r0 * ldg, ldg, route + (long long)r0 * experts,
-                                                       (bf16_t*)out + r0 * ldo, ldo, experts, ff, limit, on_input, plain_silu);
-    else LQ_REQUIRE(false, "moe_glu: unknown dtype %d", out_dtype);
+    dim3 grid((unsigned)lq_ceil_div64((long long)experts * ff, quads ? 1024 : 256), nr);
+#define LQ_MOE_GLU(T, VEC)                                                                                        \
+  moe_glu_kernel<T, VEC><<<grid, 256, 0, stream>>>(gu + r0 * ldg, ldg, route + (long long)r0 * experts,           \
+                                                   (T*)out + r0 * ldo, ldo, experts, ff, limit, on_input, plain_silu)
+    if (out_dtype == LQ_F32) {
+      if (quads) LQ_MOE_GLU(float, 4);
+      else LQ_MOE_GLU(float, 1);
+    } else {
+      if (quads) LQ_MOE_GLU(bf16_t, 4);
+      else LQ_MOE_GLU(bf16_t, 1);
+    }
+#undef LQ_MOE_GLU
   }
   LQ_CHECK_LAUNCH("moe_glu");
   return 0;
@@ -373,12 +410,13 @@ extern "C" int lq_moe_act(const float* u, long long ldu, const float* route, voi
 // route [rows, experts] (a weight, or -1): counts [experts], order and weight [pairs] (pairs: the chosen
 // (row, expert) couples, expert by expert, rows ascending), place_of [rows, experts]
 extern "C" int lq_moe_sort(const float* route, int rows, int experts, int* counts, int* order, float* weight, int* place_of,
-                           hipStream_t stream) {
+                           int places, hipStream_t stream) {
+  LQ_REQUIRE(places >= 0, "moe_sort: %d places", places);
   LQ_REQUIRE(rows > 0 && rows < (1 << 24) && experts > 0 && experts <= 65535, "moe_sort: rows %d, experts %d", rows, experts);
   LQ_REQUIRE(route && counts && order && weight && place_of, "moe_sort: null pointer");
-  moe_count_kernel<<<experts, 256, 0, stream>>>(route, rows, experts, counts);
+  moe_count_kernel<<<experts, SORT_THREADS, 0, stream>>>(route, rows, experts, counts);
   LQ_CHECK_LAUNCH("moe_sort(count)");
-  moe_place_kernel<<<experts, 256, 0, stream>>>(route, rows, experts, counts, order, weight, place_of);
+  moe_place_kernel<<<experts, SORT_THREADS, 0, stream>>>(route, rows, experts, counts, order, weight, place_of, places);
   LQ_CHECK_LAUNCH("moe_sort(place)");
   return 0;
 }
@@ -387,9 +425,12 @@ extern "C" int lq_moe_gather(const void* src, int dtype, int ld, const int* orde
                              hipStream_t stream) {
   LQ_REQUIRE(n > 0 && width > 0 && ld >= width, "moe_gather: %d rows of %d (stride %d)", n, width, ld);
   LQ_REQUIRE(src && order && dst, "moe_gather: null pointer");
-  if (dtype == LQ_F32) moe_gather_kernel<float><<<n, 256, 0, stream>>>((const float*)src, ld, order, (float*)dst, width);
-  else if (dtype == LQ_BF16) moe_gather_kernel<bf16_t><<<n, 256, 0, stream>>>((const bf16_t*)src, ld, order, (bf16_t*)dst, width);
-  else LQ_REQUIRE(false, "moe_gather: unknown dtype %d", dtype);
+  LQ_REQUIRE(dtype == LQ_F32 || dtype == LQ_BF16, "moe_gather: unknown dtype %d", dtype);
+  const int per = dtype == LQ_F32 ? 4 : 8;  // entries in 16 bytes
+  if (width % per == 0 && ld % per == 0 && (((uintptr_t)src | (uintptr_t)dst) & 15) == 0)
+    moe_gather_kernel<uint4><<<n, 256, 0, stream>>>((const uint4*)src, ld / per, order, (uint4*)dst, width / per);
+  else if (dtype == LQ_F32) moe_gather_kernel<float><<<n, 256, 0, stream>>>((const float*)src, ld, order, (float*)dst, width);
+  else moe_gather_kernel<bf16_t><<<n, 256, 0, stream>>>((const bf16_t*)src, ld, order, (bf16_t*)dst, width);
   LQ_CHECK_LAUNCH("moe_gather");
   return 0;
 }
@@ -398,7 +439,10 @@ extern "C" int lq_moe_scatter(const float* ys, const int* place_of, int experts,
                               hipStream_t stream) {
   LQ_REQUIRE(rows > 0 && width > 0 && experts > 0 && ldo >= width, "moe_scatter: rows %d, width %d, experts %d", rows, width, experts);
   LQ_REQUIRE(ys && place_of && out, "moe_scatter: null pointer");
-  moe_scatter_kernel<<<rows, 256, 0, stream>>>(ys, place_of, experts, out, ldo, width);
+  if (width % 4 == 0 && ldo % 4 == 0 && (((uintptr_t)ys | (uintptr_t)out) & 15) == 0)
+    moe_scatter_kernel<4><<<rows, 256, 0, stream>>>(ys, place_of, experts, out, ldo, width);
+  else
+    moe_scatter_kernel<1><<<rows, 256, 0, stream>>>(ys, place_of, experts, out, ldo, width);
   LQ_CHECK_LAUNCH("moe_scatter");
   return 0;
 }

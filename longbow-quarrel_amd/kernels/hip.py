@@ -20,7 +20,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 14  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 15  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -346,6 +346,34 @@ class HipKernels:
                                 ldc, pieces, stride, 1 if self.force_generic else 0, _packed(w), self.stream)
         if rc:
             self._check(rc)
+
+    @query
+    def linear_grouped_supported(self, dtype: torch.dtype, groups: int, n: int, k: int) -> bool:
+        """Whether `linear_grouped` takes a mixture of `groups` experts with weights [n, k]."""
+        if dtype not in _DTYPE_CODE:
+            return False
+        return bool(self.lib.lq_linear_grouped_supported(c_int(_DTYPE_CODE[dtype]), c_int(groups), c_int(n), c_int(k),
+                                                         c_int(1 if self.force_generic else 0)))
+
+    def linear_grouped(self, x: torch.Tensor, ws, out: torch.Tensor, counts: torch.Tensor) -> None:
+        """out (float32) = x . ws[i]^T for x's rows in runs, one behind the other: counts[i] rows (int32, on the device)
+        for weight i.  The weights are views of one matrix, equally far apart (an expert's rows, dense or packed, or its
+        columns).  Rows beyond the counts' sum are neither read nor written."""
+        self._dev(x, out, counts)
+        m, k, ldx = self._mat(x, "linear_grouped: x")
+        n, kw, ldw = self._mat(ws[0], "linear_grouped: w")
+        mo, no, ldc = self._mat(out, "linear_grouped: out")
+        self._i32(counts, "counts", len(ws))
+        at = [w.data_ptr() for w in ws]
+        step = (at[1] - at[0]) // ws[0].element_size() if len(ws) > 1 else 0
+        if (kw, mo, no) != (k, m, n) or out.dtype != torch.float32 or x.dtype != ws[0].dtype \
+                or any(tuple(w.shape) != (n, k) or w.dtype != x.dtype or self._mat(w, "w")[2] != ldw
+                       or _packed(w) != _packed(ws[0]) for w in ws) \
+                or any(a != at[0] + i * step * ws[0].element_size() for i, a in enumerate(at)):
+            raise KernelLibraryError("linear_grouped: x [M, K], equal weights [N, K] equally far apart, out float32 [M, N]")
+        self._check(self.lib.lq_linear_grouped(_ptr(x), c_void_p(at[0]), _ptr(out), c_int(_code(x)), c_int(m), c_int(n),
+                                               c_int(k), c_int(ldx), c_int(ldw), c_int(ldc), _ptr(counts), c_int(len(ws)),
+                                               c_longlong(step), c_int(_packed(ws[0])), self.stream))
 
     # -- the two products around a norm, for a few rows (decoding): x += act . w^T leaves every row's
     # sum of squares in parts, and the product after the norm normalises its input from them itself
@@ -1614,10 +1642,10 @@ class HipKernels:
         return PackedWeight(w.data.view(-1)[start * k : (start + n) * k].view(n, k), n, k)
 
     def moe_sort(self, route: torch.Tensor, counts: torch.Tensor, order: torch.Tensor, weight: torch.Tensor,
-                 place_of: torch.Tensor) -> None:
+                 place_of: torch.Tensor, fill: bool = False) -> None:
         """The chosen (row, expert) couples of route [rows, experts] (a weight, or -1), expert by expert with rows
         ascending: counts[e] rows of expert e, order[place] = row, weight[place] = its weight, place_of[row, e] =
-        place or -1."""
+        place or -1.  With `fill` the places behind them get row 0 and weight -1."""
         rows, experts = route.shape
         self._f32(route, "moe_sort: route", rows * experts)
         self._f32(weight, "moe_sort: weight")
@@ -1628,7 +1656,7 @@ class HipKernels:
             raise KernelLibraryError("moe_sort: order (int32) and weight (float32) hold a place for every chosen couple")
         self._dev(route, counts, order, weight, place_of)
         self._check(self.lib.lq_moe_sort(_ptr(route), c_int(rows), c_int(experts), _ptr(counts), _ptr(order), _ptr(weight),
-                                         _ptr(place_of), self.stream))
+                                         _ptr(place_of), c_int(order.numel() if fill else 0), self.stream))
 
     def moe_gather(self, src: torch.Tensor, order: torch.Tensor, dst: torch.Tensor, n: int) -> None:
         """dst[i] = src[order[i]] for the first n places."""

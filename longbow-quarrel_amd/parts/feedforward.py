@@ -226,8 +226,10 @@ class MixtureOfExperts(FeedForward):
     experts' columns: a batch of more than a few tokens reads nearly all experts anyway.  A prompt step of
     `sort_from_rows` rows or more is sorted by expert first (`moe_sort`: the chosen (row, expert) couples expert by
     expert, rows ascending), the rows gathered in that order, and every expert's two products run over its own rows
-    only; the results go back to their rows and are added in the order of the experts.  The host reads the experts'
-    row counts for that (one wait a layer), which a captured step never does: it takes the first way."""
+    only, all experts' in one launch that finds the row counts on the device; the results go back to their rows and are
+    added in the order of the experts.  Where the kernels have no such launch for the weights, the products are
+    launched expert by expert and the host reads the row counts (one wait a layer), which a captured step never does:
+    it takes the first way."""
 
     graph_safe = True
     takes_out = True
@@ -453,6 +455,21 @@ class MixtureOfExperts(FeedForward):
         self._pass_on(h, out, ctx)
         return out
 
+    def _expert_unit(self, gu, weight, act, ctx: StepContext) -> None:
+        """The activations of sorted rows, each with one expert and its weight."""
+        if self.gated:
+            more = {"activation": self.activation} if self.activation != "clamped_swish" else {}
+            ctx.kernels.moe_glu(gu, weight, act, 1, self.inner, self.limit, self.weight_input, **more)
+        else:
+            ctx.kernels.moe_act(gu, weight, act, 1, self.inner, self.activation)
+
+    def _grouped(self, h, ctx: StepContext) -> bool:
+        """Whether one launch takes all experts' products, whatever their numbers of rows."""
+        ask = getattr(ctx.kernels, "linear_grouped_supported", None)
+        w = self.gate_up_of[0]
+        return ask is not None and h.dtype == w.dtype == self.w_down.dtype == ctx.dtype and self.down_of[0].stride(0) % 8 == 0 \
+            and ask(h.dtype, self.experts, self.n_in * self.inner, self.width) and ask(h.dtype, self.experts, self.width, self.inner)
+
     def _sorted(self, h, route, out, ctx: StepContext) -> None:
         """The step's rows sorted by expert: every expert's products over its own rows only."""
         kn = ctx.kernels
@@ -462,7 +479,19 @@ class MixtureOfExperts(FeedForward):
         order = ctx.ws.alloc((pairs,), torch.int32)       # sorted place -> row
         weight = ctx.ws.alloc((pairs, 1), torch.float32)  # sorted place -> the row's weight for its expert
         place_of = ctx.ws.alloc((rows, E), torch.int32)   # (row, expert) -> sorted place, or -1
-        kn.moe_sort(route, counts, order, weight, place_of)
+        grouped = self._grouped(h, ctx)
+        kn.moe_sort(route, counts, order, weight, place_of, **({"fill": True} if grouped else {}))
+        if grouped:
+            hs = ctx.ws.alloc((pairs, self.width), h.dtype)
+            kn.moe_gather(h, order, hs, pairs)  # (places that no couple takes: row 0, which nobody reads)
+            gu = ctx.ws.alloc((pairs, self.n_in * ff), torch.float32)
+            kn.linear_grouped(hs, self.gate_up_of[:E], gu, counts)
+            act = ctx.ws.alloc((pairs, ff), ctx.dtype)
+            self._expert_unit(gu, weight, act, ctx)
+            ys = ctx.ws.alloc((pairs, self.width), torch.float32)
+            kn.linear_grouped(act, self.down_of[:E], ys, counts)
+            kn.moe_scatter(ys, place_of, out)
+            return
         n_of = counts.tolist()  # the one wait: the products below are launched with every expert's number of rows
         total = sum(n_of)
         if total == 0:
@@ -477,11 +506,7 @@ class MixtureOfExperts(FeedForward):
                 project(kn, ctx, hs[at : at + n], self.gate_up_of[e], gu[at : at + n])
                 at += n
         act = ctx.ws.alloc((pairs, ff), ctx.dtype)
-        if self.gated:
-            more = {"activation": self.activation} if self.activation != "clamped_swish" else {}
-            kn.moe_glu(gu[:total], weight[:total], act[:total], 1, ff, self.limit, self.weight_input, **more)
-        else:
-            kn.moe_act(gu[:total], weight[:total], act[:total], 1, ff, self.activation)
+        self._expert_unit(gu[:total], weight[:total], act[:total], ctx)
         ys = ctx.ws.alloc((pairs, self.width), torch.float32)
         at = 0
         for e, n in enumerate(n_of):
