@@ -17,11 +17,6 @@ struct SinkArgs {
   int bt_stride, BS;
   float scale;
   int window, keep_first, sink;
-  // single tokens of a bfloat16 run may share a tile's keys out over `ksplit` workgroups (blockIdx.z): each takes
-  // the rounds of SPLIT chunks whose number is its own modulo ksplit and leaves its partial result in `part`,
-  // which a second launch merges in the order of the workgroups
-  int ksplit;
-  float* part;
   int maps, out_f32;
   const float* sinks;  // null: the sink's score is 0
   ScoreShape shape;
@@ -90,3 +85,10 @@ inline bool scores_shaped(const ScoreShape& s) {
 // Prompts of a bfloat16 run (attention_sink_rows.hip).  -> 1 launched, 0 not a launch that it takes, -2 an error.
 int lq_sink_rows32(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache,
                    const int* cu_rows, const SinkArgs& a, int batch, hipStream_t stream);
+
+// Single tokens of a bfloat16 run (attention_sink_decode.hip); the same answers.
+int lq_sink_decode(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache,
+                   const SinkArgs& a, int max_len, float* part, long long part_floats, int* tickets, long long tickets_n,
+                   hipStream_t stream);
+long long lq_sink_decode_workspace(int rows, int nh, int nkv, int KD, int VD, int block_size, int window, int keep_first,
+                                   int chunk, int max_len);

@@ -1,0 +1,338 @@
+// Steps of single tokens of a bfloat16 run through the windowed attention of attention_sink.hip (the same masks, sinks,
+// shaped scores, maps and gates).
+//
+// A workgroup of four wavefronts takes one row of the step, up to 16 query heads of one key head and one of `splits`
+// shares of the keys: the blocks of 64 positions that the row sees, numbered from the kept first ones on, go to the
+// wavefronts of all shares in turn, so that at a few thousand keys every wavefront has one.  It asks for all of a block's
+// keys and values before it waits for any: what bounds such a step is the chain of round trips to memory, not the bytes
+// (tiles that asked for a few bytes of a key row at a time, a product between, and a second launch that merged the
+// shares: microseconds before and now, 8 rows, 16 heads: 4 key heads of 128 at 512 keys 20 -> 12, at 1 500 keys under a
+// window of 1 024 31 -> 13, with values of 256 and two maps 28 -> 16; one key head of 256 with values of 192 28 -> 21;
+// 64 rows at 500 keys 34 -> 19; 2 rows with capped scores and a table of biases 30 -> 15).  The shares of a row meet in its last workgroup to finish
+// (a ticket a row and key head; partial results pass the dies' caches as device-scope atomics), which adds them up in
+// their order.
+//
+//   S^T[key][head] = K . Q^T by v_mfma_f32_16x16x32_bf16: lane (c = l % 16, g = l / 16) gives A[c][8 g .. + 8] and B[c][the
+//   same] and receives D[4 g + e][c].  Row i of tile j (of a run of 32 keys) is key 8 (i / 4) + 4 j + i % 4: a lane's scores
+//   of both tiles are then keys 8 g .. + 7 of its head, which O^T[d][head] += V^T . P^T takes as they are.
+// The probabilities stay 32-bit, multiplied in three bfloat16 parts that add up to them exactly (attention_sink_rows.hip).
+// Values of positions that were never written count as zero.
+#include "attention_sink.h"
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+namespace {
+
+constexpr int BLOCK = 64, NW = 4, MAX_SPLITS = 64;
+constexpr float LOG2E = 1.44269504088896340736f;
+constexpr float NONE = -3.0e38f;  // the running maximum of a row that has seen no key
+
+__device__ inline bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+__device__ inline unsigned upper2(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ inline float below_upper(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+
+// over the four lanes that share l % 16
+__device__ inline float across_max(float x) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ inline float across_sum(float x) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+__device__ inline void publish(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ inline float published(const float* p) {
+  return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct Shares {
+  int splits;
+  float* part;   // [row][key head's tile][split]: cols x VD results, then cols maxima and cols sums
+  int* tickets;  // [row][key head's tile], zero between launches
+};
+
+// KD and VD up to 32 KS and 16 VT: sizes in between run with zeros behind their keys and values.
+template <int KS, int VT, bool SHAPED>
+__global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink_decode_kernel(
+    const bf16_t* __restrict__ q, void* __restrict__ out, const bf16_t* __restrict__ gate,
+    const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache, SinkArgs a, Shares sh) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];  // [NW][16][VD + 4]
+  __shared__ float lds_m[NW][16], lds_l[NW][16];
+  __shared__ int last;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int r = blockIdx.x, split = blockIdx.z, group = a.nh / a.nkv, tiles = (group + 15) / 16;
+  const int kvh = blockIdx.y / tiles, hbase = kvh * group + blockIdx.y % tiles * 16, cols = min(16, (kvh + 1) * group - hbase);
+  const int h = hbase + min(c, cols - 1);
+  const int nvh = a.nkv / a.maps, vh = kvh / a.maps, KD = a.KD, VD = a.VD, row_floats = VD + 4;
+  const long long krow = (long long)a.maps * KD;
+
+  const int pos = a.row_pos[r], lo = first_key(a, pos);
+  const int* table = a.block_table + (long long)a.seq_slot[a.row_seq[r]] * a.bt_stride;
+  const int wstart = lo / BLOCK * BLOCK;                                         // first block of the window
+  const int kept = (min(a.keep_first, wstart) + BLOCK - 1) / BLOCK;              // blocks of kept keys below it
+  const int blocks = kept + pos / BLOCK - wstart / BLOCK + 1;
+  const int live = min(sh.splits, (blocks + NW - 1) / NW);                       // shares with a block for some wavefront
+  if (split >= live) return;                                                     // the whole workgroup
+
+  u32x4 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d = 32 * ks + 8 * g;
+    qf[ks] = d < KD ? *(const u32x4*)(q + (long long)r * a.ldq + h * KD + d) : (u32x4){0u, 0u, 0u, 0u};
+  }
+  HeadShape hs;
+  if constexpr (SHAPED) hs = head_shape(a, h);
+  const float c2 = a.scale * LOG2E;
+  float m = NONE, l = 0.f;  // the head's running maximum (in powers of two); this lane's share of its sum
+  if (a.sink && split == 0 && w == 0) m = a.sinks != nullptr ? a.sinks[h] * LOG2E : 0.f, l = g == 0 ? 1.f : 0.f;
+  f32x4 o[VT];  // o[dt][e]: value entry 16 dt + 4 g + e of head c
+#pragma unroll
+  for (int dt = 0; dt < VT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  for (int i = split * NW + w; i < blocks; i += live * NW) {
+    const int t0 = i < kept ? i * BLOCK : wstart + (i - kept) * BLOCK;
+    const long long blk = table[t0 / BLOCK];
+    const bf16_t* kb = kcache + (blk * nvh + vh) * BLOCK * krow + (kvh % a.maps) * KD + 8 * g;
+    const bf16_t* vb = vcache + (blk * nvh + vh) * (long long)VD * BLOCK + 8 * g;
+    u32x4 kf[4][KS], vf[VT][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = 32 * (j >> 1) + (c >> 2) * 8 + (j & 1) * 4 + (c & 3);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        kf[j][ks] = 32 * ks + 8 * g < KD ? *(const u32x4*)(kb + key * krow + 32 * ks) : (u32x4){0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int dt = 0; dt < VT; ++dt)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        vf[dt][j] = 16 * dt + c < VD ? *(const u32x4*)(vb + (16 * dt + c) * BLOCK + 32 * j) : (u32x4){0u, 0u, 0u, 0u};
+    __builtin_amdgcn_sched_barrier(0);  // (all of them before the first product)
+    f32x4 st[4];  // st[j][e]: key t0 + 32 (j / 2) + 8 g + 4 (j % 2) + e
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      st[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        st[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[j][ks]), as_bf16x8(qf[ks]), st[j], 0, 0, 0);
+    }
+    float top = NONE;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = t0 + 32 * (j >> 1) + 8 * g + 4 * (j & 1) + e;
+        float s;
+        if constexpr (SHAPED) s = shaped<false>(st[j][e], max(pos - t, 0), hs) * LOG2E;
+        else s = st[j][e] * c2;
+        st[j][e] = t <= pos && (t >= lo || t < a.keep_first) ? s : -INFINITY;
+        top = fmaxf(top, st[j][e]);
+      }
+    const float m_new = fmaxf(m, across_max(top)), alpha = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        st[j][e] = __builtin_amdgcn_exp2f(st[j][e] - m);
+        sum += st[j][e];
+      }
+    l = l * alpha + sum;
+#pragma unroll
+    for (int dt = 0; dt < VT; ++dt) o[dt] *= alpha;
+    if (t0 + BLOCK - 1 > pos) {  // (0 times what lies in unwritten memory may be NaN)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int t = t0 + 32 * j + 8 * g + 2 * x;
+          const unsigned keep = t + 1 <= pos ? 0xffffffffu : t <= pos ? 0x0000ffffu : 0u;
+#pragma unroll
+          for (int dt = 0; dt < VT; ++dt) vf[dt][j][x] &= keep;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      u32x4 part[3];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float p0 = st[2 * j + (x >> 1)][2 * (x & 1)], p1 = st[2 * j + (x >> 1)][2 * (x & 1) + 1];
+        const float q0 = below_upper(p0), q1 = below_upper(p1);
+        part[0][x] = upper2(p0, p1), part[1][x] = upper2(q0, q1), part[2][x] = upper2(below_upper(q0), below_upper(q1));
+      }
+#pragma unroll
+      for (int i3 = 2; i3 >= 0; --i3)
+#pragma unroll
+        for (int dt = 0; dt < VT; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf[dt][j]), as_bf16x8(part[i3]), o[dt], 0, 0, 0);
+    }
+  }
+  // the wavefronts' results meet
+  l = across_sum(l);
+#pragma unroll
+  for (int dt = 0; dt < VT; ++dt)
+    if (16 * dt + 4 * g < VD && c < cols) *(f32x4*)(lds + (w * 16 + c) * row_floats + 16 * dt + 4 * g) = o[dt];
+  if (g == 0) lds_m[w][c] = m, lds_l[w][c] = l;
+  __syncthreads();
+  const long long at = (long long)r * gridDim.y + blockIdx.y;
+  const int share_floats = min(16, group) * (VD + 2), first = hbase * VD;
+  float* mine = sh.part + (at * sh.splits + split) * share_floats;
+  // a head's entry from its sum over the keys
+  auto finish = [&](int idx, float sum, float L) {
+    float f = 1.0f / L;
+    const int hh = hbase + idx / VD;
+    if (gate != nullptr) f /= 1.f + expf(-to_f32(gate[(long long)r * a.ldg + hh]));
+    float v = sum * f;
+    if (a.wide_gate != nullptr) v /= 1.f + expf(-a.wide_gate[(long long)r * a.ldwg + first + idx]);
+    put_out((bf16_t*)out, (long long)r * a.ldo + first + idx, v, a.out_f32);
+  };
+  for (int idx = tid; idx < cols * VD; idx += NW * 64) {
+    const int cc = idx / VD, d = idx - cc * VD;
+    float M = lds_m[0][cc];
+#pragma unroll
+    for (int j = 1; j < NW; ++j) M = fmaxf(M, lds_m[j][cc]);
+    float sum = 0.f, L = 0.f;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      const float f = __builtin_amdgcn_exp2f(lds_m[j][cc] - M);
+      sum = fmaf(f, lds[(j * 16 + cc) * row_floats + d], sum), L = fmaf(f, lds_l[j][cc], L);
+    }
+    if (live == 1) {
+      finish(idx, sum, L);
+    } else {
+      publish(mine + idx, sum);
+      if (d == 0) publish(mine + cols * VD + cc, M), publish(mine + cols * VD + cols + cc, L);
+    }
+  }
+  if (live == 1) return;
+  // Once every thread's stores have completed the workgroup takes a ticket; the last one adds the shares up.
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  if (tid == 0)
+    last = __hip_atomic_fetch_add(sh.tickets + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == live - 1;
+  __syncthreads();
+  if (!last) return;
+  const float* shares = sh.part + at * sh.splits * share_floats;
+  // every share's factor for every head, and the heads' sums ...
+  __shared__ float factor[MAX_SPLITS][16], sums[MAX_SPLITS][16], whole[16];
+  for (int x = tid; x < live * cols; x += NW * 64) {
+    const int s = x / cols, cc = x - s * cols;
+    const float* p = shares + s * share_floats + cols * VD + cc;
+    factor[s][cc] = published(p), sums[s][cc] = published(p + cols);
+  }
+  __syncthreads();
+  if (tid < cols) {
+    float M = NONE, L = 0.f;
+    for (int s = 0; s < live; ++s) M = fmaxf(M, factor[s][tid]);
+    for (int s = 0; s < live; ++s) {
+      const float f = __builtin_amdgcn_exp2f(factor[s][tid] - M);
+      factor[s][tid] = f, L = fmaf(f, sums[s][tid], L);
+    }
+    whole[tid] = L;
+  }
+  __syncthreads();
+  // ... then their results, four entries of four shares asked for together
+  for (int i0 = tid; i0 < cols * VD; i0 += 4 * NW * 64) {
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < live; s0 += 4) {
+      float v[4][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          v[j][x] = published(shares + min(s0 + j, live - 1) * share_floats + min(i0 + x * NW * 64, cols * VD - 1));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          if (s0 + j < live) sum[x] = fmaf(factor[s0 + j][min(i0 + x * NW * 64, cols * VD - 1) / VD], v[j][x], sum[x]);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int idx = i0 + x * NW * 64;
+      if (idx < cols * VD) finish(idx, sum[x], whole[idx / VD]);
+    }
+  }
+  if (tid == 0) __hip_atomic_store(sh.tickets + at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+}
+
+template <int KS, int VT>
+int launch(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache, const SinkArgs& a,
+           const Shares& sh, dim3 grid, hipStream_t stream) {
+  const int bytes = NW * 16 * (a.VD + 4) * (int)sizeof(float);
+  const bool with_shape = scores_shaped(a.shape);
+  const auto kernel = with_shape ? sink_decode_kernel<KS, VT, true> : sink_decode_kernel<KS, VT, false>;
+  static bool configured[2] = {false, false};
+  if (!configured[with_shape]) {
+    const int most = NW * 16 * (16 * VT + 4) * (int)sizeof(float);
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    if (e != hipSuccess) {
+      lq_set_error("sink_attention: cannot reserve %d bytes of LDS: %s", most, hipGetErrorString(e));
+      return -2;
+    }
+    configured[with_shape] = true;
+  }
+  kernel<<<grid, NW * 64, bytes, stream>>>(q, out, gate, kcache, vcache, a, sh);
+  LQ_CHECK_LAUNCH("sink_attention(single tokens)");
+  return 1;
+}
+
+// Shares of a row's keys: as many as give every wavefront one block of the `max_len` bound, within two rounds of
+// workgroups.
+int splits_for(int rows, int nh, int nkv, int window, int keep_first, int chunk, int max_len) {
+  if (max_len <= 0) return 1;
+  const long long seen = window > 0 ? (long long)window + keep_first + 2 * BLOCK : max_len;
+  int keys = seen < max_len ? (int)seen : max_len;
+  if (chunk > 0 && chunk + BLOCK < keys) keys = chunk + BLOCK;
+  const int tiles = rows * nkv * lq_ceil_div(nh / nkv, 16), wanted = lq_ceil_div(lq_ceil_div(keys, BLOCK) + 1, NW);
+  int room = 2 * lq_compute_units() / tiles;
+  if (room > MAX_SPLITS) room = MAX_SPLITS;
+  return wanted < room ? wanted : room > 1 ? room : 1;
+}
+
+bool takes(int KD, int VD, int block_size, int nh, int nkv, int rows) {
+  return block_size == BLOCK && KD % 8 == 0 && VD % 4 == 0 && KD <= 256 && VD <= 256 &&
+         (long long)nkv * lq_ceil_div(nh / nkv, 16) <= 65535 && rows < (1 << 22);
+}
+
+}  // namespace
+
+long long lq_sink_decode_workspace(int rows, int nh, int nkv, int KD, int VD, int block_size, int window, int keep_first,
+                                   int chunk, int max_len) {
+  if (!takes(KD, VD, block_size, nh, nkv, rows)) return 0;
+  const int splits = splits_for(rows, nh, nkv, window, keep_first, chunk, max_len), group = nh / nkv;
+  if (splits == 1) return 0;
+  return (long long)rows * nkv * lq_ceil_div(group, 16) * splits * (group < 16 ? group : 16) * (VD + 2);
+}
+
+int lq_sink_decode(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache,
+                   const SinkArgs& a, int max_len, float* part, long long part_floats, int* tickets, long long tickets_n,
+                   hipStream_t stream) {
+  if (a.ldq % 8 != 0 || ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) % 16 != 0 ||
+      !takes(a.KD, a.VD, a.BS, a.nh, a.nkv, a.rows))
+    return 0;
+  const int tiles = a.nkv * lq_ceil_div(a.nh / a.nkv, 16);
+  Shares sh = {1, part, tickets};
+  if (part != nullptr && tickets != nullptr && (long long)a.rows * tiles <= tickets_n) {
+    const long long need = lq_sink_decode_workspace(a.rows, a.nh, a.nkv, a.KD, a.VD, a.BS, a.window, a.keep_first, a.chunk, max_len);
+    if (need > 0 && need <= part_floats) sh.splits = splits_for(a.rows, a.nh, a.nkv, a.window, a.keep_first, a.chunk, max_len);
+  }
+  const dim3 grid(a.rows, tiles, sh.splits);
+#define LQ_DECODE(KS, VT) launch<KS, VT>(q, out, gate, kcache, vcache, a, sh, grid, stream)
+  if (a.KD <= 64 && a.VD <= 64) return LQ_DECODE(2, 4);
+  if (a.KD <= 128 && a.VD <= 128) return LQ_DECODE(4, 8);
+  if (a.KD <= 128) return LQ_DECODE(4, 16);
+  if (a.VD <= 192) return LQ_DECODE(8, 12);
+  return LQ_DECODE(8, 16);
+#undef LQ_DECODE
+}

@@ -20,7 +20,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 15  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 16  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -843,7 +843,10 @@ class HipKernels:
             self._f32(workspace, "sink_attention: workspace", workspace.numel())
         if cu_rows is not None:
             self._i32(cu_rows, "cu_rows", batch + 1)
-        self._check(self.lib.lq_sink_attention(
+        # (shares of the keys meet by the tickets that the causal attention's decoding uses: launches of one object do
+        # not overlap)
+        tickets = self.tickets(q.device) if workspace is not None else None
+        rc = self.lib.lq_sink_attention(
             _ptr(q), c_int(self._rows2d(q, "q")), _ptr(out), c_int(self._rows2d(out, "out")), _ptr(gate),
             c_int(0 if gate is None else self._rows2d(gate, "gate")), c_int(_code(q)), c_int(rows), c_int(batch),
             c_int(heads), c_int(kv_heads), c_int(key_dim), c_int(value_dim), _ptr(row_pos), _ptr(row_seq),
@@ -853,7 +856,15 @@ class HipKernels:
             c_longlong(0 if workspace is None else workspace.numel()), _ptr(sink_values), c_int(maps),
             c_int(1 if out.dtype == torch.float32 else 0), c_float(softcap), _ptr(temp), _ptr(r1), _ptr(r2),
             _ptr(distance_bias), c_int(0 if distance_bias is None else int(distance_bias.shape[1])), _ptr(wide_gate),
-            c_int(0 if wide_gate is None else self._rows2d(wide_gate, "wide_gate")), c_int(chunk), _ptr(cu_rows), self.stream))
+            c_int(0 if wide_gate is None else self._rows2d(wide_gate, "wide_gate")), c_int(chunk), _ptr(cu_rows), _ptr(tickets),
+            c_longlong(0 if tickets is None else tickets.numel()), self.stream)
+        if rc != 0:
+            message = self.lib.lq_last_error().decode("utf-8", "replace")
+            try:
+                if tickets is not None:
+                    tickets.zero_()  # (a launch that did not run whole may have left some)
+            finally:
+                raise KernelLibraryError(message)
 
     def diff_combine(self, both: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int, value_dim: int, lam: float,
                      eps: float, gain: float) -> None:

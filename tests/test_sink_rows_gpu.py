@@ -1,5 +1,6 @@
-"""Prompts through the 32 x 32 score tiles of the windowed attention (`cu_rows` given) against the general kernel, one
-wavefront a row and head, at the sizes where tiles, blocks and halves end."""
+"""Prompts through the 32 x 32 score tiles of the windowed attention (`cu_rows` given), and steps of single tokens through
+their own kernel, against the general kernel, one wavefront a row and head, at the sizes where tiles, blocks, halves and
+shares of the keys end."""
 import pytest
 import torch
 
@@ -24,8 +25,27 @@ CASES = [  # heads, key heads, key size, value size, (new, held) of every sequen
 ]
 
 
+LENGTHS = [1, 63, 64, 65, 255, 256, 257, 300, 700, 1030]
+SINGLE = [  # heads, key heads, key size, value size, options
+    (16, 4, 128, 128, dict(window=256, keep_first=70)), (16, 4, 128, 128, dict(PLAIN, chunk=100)),
+    (16, 1, 256, 192, PLAIN), (40, 2, 64, 40, dict(sinks=True, gate=True)), (4, 1, 256, 256, PLAIN),
+    (8, 4, 128, 256, dict(PLAIN, maps=2, window=600)), (3, 3, 40, 24, dict(window=1, wide=True)),
+    (8, 2, 128, 128, dict(sinks=True, cap=30.0, log=True, window=200)),
+    (8, 2, 64, 64, dict(PLAIN, cap=5.0, dist=100, temp=True, wide=True))]
+
+
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("H,G,D,P,options", SINGLE)
+def test_single_tokens(H, G, D, P, options, shared):
+    check(H, G, D, P, [(1, n - 1) for n in LENGTHS], options, shared)
+
+
 @pytest.mark.parametrize("H,G,D,P,seqs,options", CASES)
 def test_tiles_of_32_rows(H, G, D, P, seqs, options):
+    check(H, G, D, P, seqs, options, False)
+
+
+def check(H, G, D, P, seqs, options, shared):
     from longbow_quarrel_amd.kernels.hip import HipKernels
 
     gen = torch.Generator().manual_seed(H * 1000 + D + P)
@@ -69,7 +89,17 @@ def test_tiles_of_32_rows(H, G, D, P, seqs, options):
     for dtype in (torch.float32, torch.bfloat16):
         got, want = (torch.full((rows, H * P), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
         args = (H, G, D, P, pos, seq, i32(range(len(seqs))), table.cuda(), k, v, 64, D ** -0.5)
-        kn.sink_attention(q, got, *args, cu_rows=starts, **more)
+        how = dict(cu_rows=starts)
+        if rows == len(seqs):
+            how = dict(decode=True)
+            longest = max(n + held for n, held in seqs)
+            need = kn.sink_attention_workspace(torch.bfloat16, rows, rows, H, G, D, P, 64, more["window"], more["keep_first"],
+                                               longest, chunk=more["chunk"])
+            if shared and need:
+                how.update(max_len=longest, workspace=torch.full((need,), float("nan"), device="cuda"))
+        for _ in range(2):  # (a launch leaves the tickets as it found them)
+            got.fill_(float("nan"))
+            kn.sink_attention(q, got, *args, **how, **more)
         kn.force_generic = True
         kn.sink_attention(q, want, *args, **more)
         kn.force_generic = False
