@@ -20,7 +20,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 16  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 17  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -981,21 +981,23 @@ class HipKernels:
                                             c_int(self._ACTIVATIONS[activation]), c_int(_code(x)), self.stream))
 
     @query
-    def ssd_scan_workspace(self, batch: int, heads: int, head_dim: int, n_state: int, max_rows: int) -> int:
-        """Float32 entries of scratch with which `ssd_scan` runs this launch in segments (0: it does not)."""
+    def ssd_scan_workspace(self, batch: int, heads: int, head_dim: int, n_state: int, max_rows: int, rows: int = 0) -> int:
+        """Float32 entries of scratch with which `ssd_scan` runs this launch in segments, or with `rows` (the step's) in
+        chunks where it can (0: it does neither)."""
         self.lib.lq_ssd_scan_workspace.restype = c_longlong
         return int(self.lib.lq_ssd_scan_workspace(c_int(batch), c_int(heads), c_int(head_dim), c_int(n_state),
-                                                  c_int(max_rows)))
+                                                  c_int(max_rows), c_int(rows)))
 
     def ssd_scan(self, x: torch.Tensor, b_in: torch.Tensor, c_in: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor,
                  a_log: torch.Tensor, d_skip: torch.Tensor, state: torch.Tensor, y: torch.Tensor, heads: int,
                  head_dim: int, n_state: int, groups: int, seq_slot: torch.Tensor, cu_rows: torch.Tensor,
                  batch: int, max_rows: int = 0, workspace: Optional[torch.Tensor] = None,
-                 decay: Optional[torch.Tensor] = None, ones: bool = False) -> None:
+                 decay: Optional[torch.Tensor] = None, ones: bool = False, chunks: bool = False) -> None:
         """The Mamba-2 recurrence along every sequence of the step, token by token: with dt = softplus(dt + dt_bias),
         S <- exp(-exp(a_log) dt) S + dt B x^T and y = S^T C + d_skip x per head; state [slots, heads, head_dim,
         n_state] is read and left at the step's end.  All float32.  `max_rows` (the most rows a sequence brings)
-        and `workspace` (`ssd_scan_workspace(...)` floats) let a launch of few long sequences run in segments.
+        and `workspace` (`ssd_scan_workspace(...)` floats) let a launch of few long sequences run in segments;
+        with `chunks` (and scratch asked for with the step's rows) long portions run in chunks of tokens.
         `decay` [rows, heads]: a token's decay and step (`dt` as it is) are given, S <- decay S + dt B x^T, y = S^T C;
         dt_bias, a_log and d_skip are then None.  `ones`: head_dim counts one column more than x has for a head, the
         last, whose input is one (its result is the sum of the steps' B under the same decays, times C)."""
@@ -1027,7 +1029,7 @@ class HipKernels:
                                          c_int(batch), c_int(max_rows if workspace is not None else 0), _ptr(workspace),
                                          c_longlong(0 if workspace is None else workspace.numel()), _ptr(decay),
                                          c_int(0 if decay is None else ld(decay, "decay")), c_int(1 if ones else 0),
-                                         self.stream))
+                                         c_int(rows if chunks else 0), self.stream))
 
     @query
     def selective_scan_workspace(self, batch: int, channels: int, n_state: int, max_rows: int) -> int:

@@ -20,6 +20,18 @@ def _round4(n: int) -> int:
     return (n + 3) // 4 * 4
 
 
+def _scan_scratch(ctx: StepContext, heads: int, head_dim: int, state: int) -> dict:
+    """The keywords with which `ssd_scan` may cut long prompts into parts that run side by side: into chunks of tokens
+    in a bfloat16 run, else (a few very long ones) into segments; nothing where the kernel object asks for no scratch."""
+    ask = getattr(ctx.kernels, "ssd_scan_workspace", None)
+    if ask is None:
+        return {}
+    chunks = ctx.dtype == torch.bfloat16
+    need = ask(ctx.batch, heads, head_dim, state, ctx.max_new, *((ctx.rows,) if chunks else ()))
+    return dict(max_rows=ctx.max_new, workspace=ctx.ws.alloc((need,), torch.float32),
+                **({"chunks": True} if chunks else {})) if need else {}
+
+
 class _Recurrent(Mixer):
     graph_safe = True
     takes_out = True
@@ -107,10 +119,7 @@ class Mamba2(_Recurrent):
                        ctx.row_pos, ctx.row_seq, ctx.seq_slot, ctx.seq_start, ctx.seq_len, ctx.cu_rows, ctx.batch,
                        activation="silu")
         y = ctx.ws.alloc((rows, self.inner), torch.float32)
-        # a few long prompts: the kernel may cut them into segments that run side by side, given scratch
-        ask = getattr(kn, "ssd_scan_workspace", None)
-        need = ask(ctx.batch, self.heads, self.head_dim, self.state, ctx.max_new) if ask is not None else 0
-        more = dict(max_rows=ctx.max_new, workspace=ctx.ws.alloc((need,), torch.float32)) if need else {}
+        more = _scan_scratch(ctx, self.heads, self.head_dim, self.state)
         kn.ssd_scan(xbc[:, : self.inner], xbc[:, self.inner : self.inner + gn], xbc[:, self.inner + gn :], dt,
                     self.dt_bias, self.a_log, self.d, state, y, self.heads, self.head_dim, self.state, self.groups,
                     ctx.seq_slot, ctx.cu_rows, ctx.batch, **more)
@@ -274,9 +283,7 @@ class MatrixMemory(_Recurrent):
                         ctx.seq_slot, ctx.cu_rows, ctx.batch)
         cols = self.value_dim + 1
         y = ctx.ws.alloc((rows, nh * cols), torch.float32)
-        ask = getattr(kn, "ssd_scan_workspace", None)
-        need = ask(ctx.batch, nh, cols, self.key_dim, ctx.max_new) if ask is not None else 0
-        more = dict(max_rows=ctx.max_new, workspace=ctx.ws.alloc((need,), torch.float32)) if need else {}
+        more = _scan_scratch(ctx, nh, cols, self.key_dim)
         kn.ssd_scan(u[:, 2 * qk : 2 * qk + vw], u[:, qk : 2 * qk], u[:, :qk], take, None, None, None, state, y, nh, cols,
                     self.key_dim, nh, ctx.seq_slot, ctx.cu_rows, ctx.batch, decay=decay, ones=True, **more)
         normed = ctx.ws.alloc((rows, vw), ctx.dtype)

@@ -1,0 +1,43 @@
+"""The state-space scan in chunks of 64 tokens against the walk token by token (no scratch given), at the sizes where
+chunks, blocks of 16 tokens, slices of columns and halves of channels end."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lens,H,G,N,P,given,shift", [
+    ([128], 4, 2, 128, 64, False, 0.0), ([1, 129, 63, 64, 65], 4, 1, 128, 64, False, 0.0), ([150], 2, 2, 30, 17, False, 0.0),
+    ([140, 16], 3, 3, 48, 40, False, 0.0), ([130], 2, 1, 256, 100, False, 0.0), ([200], 2, 2, 132, 64, False, 0.0),
+    ([130, 70], 2, 2, 256, 129, True, 0.0), ([128], 1, 1, 64, 65, True, 0.0), ([129], 2, 2, 30, 18, True, 0.0),
+    ([131], 2, 1, 128, 64, False, 8.0), ([131], 2, 1, 128, 64, False, -8.0), ([128] + [1] * 70, 2, 1, 64, 32, False, 0.0)])
+def test_chunks_of_the_state_space_scan(lens, H, G, N, P, given, shift):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(N * P + len(lens))
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, batch = sum(lens), len(lens)
+    x, b, c, dt = rand(rows, H * (P - given)), 0.3 * rand(rows, G * N), 0.3 * rand(rows, G * N), rand(rows, H)
+    made = (rand(H) - 3.0 + shift, 0.5 * rand(H) + 1.0, rand(H))
+    more = {}
+    if given:  # a matrix memory's: decays and steps as they are, and a column of ones
+        made, dt, more = (None, None, None), dt.abs(), dict(decay=torch.sigmoid(rand(rows, H) + 3.0), ones=True)
+    state = rand(batch, H, P, N)
+    cu = i32(sum(lens[:i]) for i in range(batch + 1))
+    kn = HipKernels()
+    need = kn.ssd_scan_workspace(batch, H, P, N, max(lens), rows)
+    assert need > 0 and kn.ssd_scan_workspace(batch, H, P, N, 1, batch) == 0
+    got = {}
+    for scratch in (None, torch.full((need,), float("nan"), device="cuda")):
+        y, end = torch.full((rows, H * P), float("nan"), device="cuda"), state.clone()
+        how = {} if scratch is None else dict(max_rows=max(lens), workspace=scratch, chunks=True)
+        kn.ssd_scan(x, b, c, dt, *made, end, y, H, P, N, G, i32(reversed(range(batch))), cu, batch, **how, **more)
+        got[scratch is not None] = y, end
+    # Sums of up to 200 tokens' terms and then N channels' in another order: at most (3 x 200 + N) roundings of 2^-24 at
+    # the size of the terms' absolute sum, which the largest state entry times sum_n |C_n| bounds.
+    (walked, end0), (chunked, end1) = got[False], got[True]
+    assert torch.isfinite(walked).all() and torch.isfinite(end0).all()
+    unit = (3 * 200 + N) * 2.0 ** -24 * end0.abs().max().clamp(min=float(state.abs().max()))
+    assert (end0 - end1).abs().max() <= unit
+    assert (walked - chunked).abs().max() <= unit * c.abs().view(rows, G, N).sum(-1).max() + 1e-6 * walked.abs().max()
