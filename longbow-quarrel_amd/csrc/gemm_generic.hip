@@ -17,9 +17,10 @@
 // k past K count as zeros, which change no sum.  The rounding error of a long row grows with
 // K / 256 + 64 additions instead of K.
 //
-// Two kernels: an LDS-tiled one (block tiles of 64 x 64 or 128 x 128, any size and alignment), and one for
-// up to 16 rows that streams the weights straight from memory, a block of waves a tile of 16 columns, its
-// waves taking chunks in turn and adding their sums up in order through LDS.
+// Three kernels: an LDS-tiled one (block tiles of 64 x 64 or 128 x 128, any size and alignment); a pipelined one of
+// 128 x 128 tiles for float32 operands in whole pieces with K in 32s; and one for up to 16 rows that streams the weights
+// straight from memory, a block of waves a tile of 16 columns, its waves taking chunks in turn and adding their sums up
+// in order through LDS.
 #include "common.h"
 
 namespace {
@@ -127,6 +128,97 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const T* __restrict
     }
 }
 
+// ---- pipelined: the same tiles, operands in whole pieces ---------------------------------------------------
+// 128 x 128 a block, 4 waves of 64 x 64.  Stages of 32 k (two slabs) go from memory straight into LDS (16 bytes a lane, no
+// registers), two stages taking turns: the next one's transfers fly while this one is multiplied, 128 matrix instructions
+// a wave, behind one barrier a stage.  A lane's four k of a slab are one 16-byte read.  An LDS row is 32 k, 128 bytes; its
+// piece u lies at u ^ (row / 2 % 8), so that the 16 rows of a fragment lie in different banks.  Two blocks a compute
+// unit, so that one multiplies while the other waits at its barrier.  The tiles go to the dies in runs, row tiles first:
+// a die's blocks share their weights.
+// What bounded the kernel above: its LDS accesses, four bytes at a time, two barriers a slab.  Microseconds, above and here
+// (the same bits): 865 x 28 672 x 4 096 3 181 / 1 783 (64 / 114 of 157 TFLOP/s), 865 x 4 096 x 14 336 2 214 / 948,
+// 2 048 x 28 672 x 4 096 6 438 / 3 623 (133 TFLOP/s: what is left is the half-filled last round and the barriers).
+constexpr int STAGE_K = 32, TILE = 128;
+
+template <typename TO, int TM>  // 32 TM rows a block
+__global__ __launch_bounds__(256, 2) void gemm_f32_pipelined_kernel(const float* __restrict__ A, int lda,
+                                                                    const float* __restrict__ W, int ldw,
+                                                                    TO* __restrict__ C, int ldc, int M, int N, int K,
+                                                                    int tiles_m, int tiles_n) {
+  constexpr int BM = 32 * TM, PER = (BM + TILE) / 32;  // transfers of 8 rows that a wave asks for a stage
+  __shared__ __attribute__((aligned(1024))) unsigned char stage[2][(BM + TILE) * STAGE_K * 4];  // A's rows, then W's
+  const int run = ((int)gridDim.x + 7) / 8, tile = (int)blockIdx.x % 8 * run + (int)blockIdx.x / 8;
+  if (tile >= tiles_m * tiles_n) return;  // (the whole block: the grid is eight runs)
+  const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * TILE;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
+
+  // a wave's transfers of a stage: 8 rows each, lane l the piece at place l % 8 of row l / 8
+  const float* from[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int row = (wave * PER + j) * 8 + (lane >> 3), piece = (lane & 7) ^ (row >> 1 & 7);
+    from[j] = row < BM ? A + (long long)min(m0 + row, M - 1) * lda + piece * 4
+                       : W + (long long)min(n0 + row - BM, N - 1) * ldw + piece * 4;
+  }
+  auto ask = [&](int s, int k0) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from[j] + k0),
+                                       (__attribute__((address_space(3))) void*)(stage[s] + (wave * PER + j) * 1024), 16, 0, 0);
+  };
+  f32x4 total[TM][4], chunk[TM][4];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) total[i][j] = chunk[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const int swizzle = r16 >> 1;  // (tiles of 16 rows start at whole periods of it)
+
+  ask(0, 0);
+  for (int k0 = 0, s = 0; k0 < K; k0 += STAGE_K, s ^= 1) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's transfers of the stage have landed,
+    asm volatile("s_barrier" ::: "memory");  // and everyone's; and everyone is done reading the other stage
+    if (k0 + STAGE_K < K) ask(s ^ 1, k0 + STAGE_K);
+    const unsigned char* as = stage[s] + (wm * 16 * TM + r16) * 128;
+    const unsigned char* ws = stage[s] + (BM + wn * 64 + r16) * 128;
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+      const int at = ((sl * 4 + g) ^ swizzle) * 16;
+      f32x4 a[TM], b[4];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = *(const f32x4*)(as + i * 2048 + at);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = *(const f32x4*)(ws + j * 2048 + at);
+#pragma unroll
+      for (int j4 = 0; j4 < 4; ++j4)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) chunk[i][j] = mfma4(a[i][j4], b[j][j4], chunk[i][j]);
+    }
+    if ((k0 + STAGE_K) % CHUNK == 0 || k0 + STAGE_K >= K) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          total[i][j] += chunk[i][j];
+          chunk[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + (wn * 4 + j) * 16 + r16;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + (wm * TM + i) * 16 + 4 * g + e;
+        if (m < M && n < N) C[(long long)m * ldc + n] = from_f32<TO>(total[i][j][e]);
+      }
+    }
+}
+
 // ---- at most 16 rows: the weights streamed from memory ---------------------------------------------------
 // Four k of a row as float32: 16 bytes of float32 or 8 bytes of bfloat16.
 __device__ inline f32x4 load4(const float* p) { return *(const f32x4*)p; }
@@ -140,59 +232,75 @@ __device__ inline f32x4 load4(const bf16_t* p) {
   return r;
 }
 
-constexpr int ROWS_WAVES = 8;  // waves a block; each takes every eighth chunk
-
-template <typename T, typename TO>
-__global__ __launch_bounds__(ROWS_WAVES * 64) void gemm_f32_rows_kernel(const T* __restrict__ X, int ldx,
-                                                                        const T* __restrict__ W, int ldw,
-                                                                        TO* __restrict__ C, int ldc, int M, int N, int K) {
-  __shared__ float sums[2][ROWS_WAVES][256];
+// Up to 16 MT rows: MT row tiles share a wave's weights.  NW waves a block take chunks in turn.  The weights of a whole
+// chunk are asked for together (16 loads of 1 KiB a wave), x four slabs at a time: within 128 registers a compute unit
+// holds 16 waves, as two blocks of 8, of which one streams while the other's meet, or as one of 16 where there are no
+// more blocks than compute units.
+template <typename T, typename TO, int MT, int ROWS_WAVES>
+__global__ __launch_bounds__(ROWS_WAVES * 64, MT <= 2 ? 4 : 2) void gemm_f32_rows_kernel(const T* __restrict__ X, int ldx,
+                                                                                        const T* __restrict__ W, int ldw,
+                                                                                        TO* __restrict__ C, int ldc, int M, int N,
+                                                                                        int K) {
+  __shared__ float sums[2][ROWS_WAVES][MT * 256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c16 = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * 16;
   const T* wp = W + (long long)min(n0 + c16, N - 1) * ldw + 4 * g;
-  const T* xp = X + (long long)min(c16, M - 1) * ldx + 4 * g;
+  const T* xp[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xp[i] = X + (long long)min(16 * i + c16, M - 1) * ldx + 4 * g;
   const int chunks = (K + CHUNK - 1) / CHUNK;
-  f32x4 total = {0.f, 0.f, 0.f, 0.f};
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 total = zero;  // of row tile `wave`
   for (int round = 0; round * ROWS_WAVES < chunks; ++round) {
     const int ch = round * ROWS_WAVES + wave;
-    f32x4 sum = zero;
+    f32x4 sum[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) sum[i] = zero;
     if (ch < chunks) {
       const int k_begin = ch * CHUNK;
-      // all of the chunk's weights are asked for together (16 loads of 1 KiB a wave), then its x
-      f32x4 wv[CHUNK / SLAB], xv[CHUNK / SLAB];
+      f32x4 wv[CHUNK / SLAB];
 #pragma unroll
       for (int s = 0; s < CHUNK / SLAB; ++s) {
         const int k = k_begin + s * SLAB;  // this lane's four k: k + 4 g .. k + 4 g + 3 (K is a multiple of 4)
         wv[s] = k + 4 * g < K ? load4(wp + k) : zero;
       }
 #pragma unroll
-      for (int s = 0; s < CHUNK / SLAB; ++s) {
-        const int k = k_begin + s * SLAB;
-        xv[s] = k + 4 * g < K ? load4(xp + k) : zero;
-      }
+      for (int s0 = 0; s0 < CHUNK / SLAB; s0 += 4) {
+        f32x4 xv[MT][4];
 #pragma unroll
-      for (int s = 0; s < CHUNK / SLAB; ++s) {
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j4 = 0; j4 < 4; ++j4) sum = mfma4(xv[s][j4], wv[s][j4], sum);
+          for (int s = 0; s < 4; ++s) {
+            const int k = k_begin + (s0 + s) * SLAB;
+            xv[i][s] = k + 4 * g < K ? load4(xp[i] + k) : zero;
+          }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int j4 = 0; j4 < 4; ++j4)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) sum[i] = mfma4(xv[i][s][j4], wv[s0 + s][j4], sum[i]);
       }
     }
-    // the round's chunks join the running sum in ascending order (every wave adds the same, wave 0 stores)
-    float(*buf)[256] = sums[round & 1];
+    // the round's chunks join the running sum in ascending order (wave i adds row tile i)
+    float(*buf)[MT * 256] = sums[round & 1];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) buf[wave][e * 64 + lane] = sum[e];
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) buf[wave][i * 256 + e * 64 + lane] = sum[i][e];
     __syncthreads();  // (two buffers: the one written two rounds ago has been read by then)
     const int n_round = min(ROWS_WAVES, chunks - round * ROWS_WAVES);
-    for (int w = 0; w < n_round; ++w)
+    if (wave < MT)
+      for (int w = 0; w < n_round; ++w)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) total[e] += buf[w][e * 64 + lane];
+        for (int e = 0; e < 4; ++e) total[e] += buf[w][wave * 256 + e * 64 + lane];
   }
-  if (wave == 0) {
+  if (wave < MT) {
     const int n = n0 + c16;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int m = 4 * g + e;
+      const int m = 16 * wave + 4 * g + e;
       if (m < M && n < N) C[(long long)m * ldc + n] = from_f32<TO>(total[e]);
     }
   }
@@ -204,11 +312,36 @@ int launch(const void* x, const void* w, void* out, int M, int N, int K, int lda
   // rows of four k each, fetched as one piece: K, the strides and the addresses must allow it
   const bool pieces = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)x % (4 * el)) == 0 &&
                       ((uintptr_t)w % (4 * el)) == 0;
-  if (M <= 16 && pieces) {
-    gemm_f32_rows_kernel<T, TO><<<lq_ceil_div(N, 16), ROWS_WAVES * 64, 0, stream>>>((const T*)x, lda, (const T*)w, ldw,
-                                                                                   (TO*)out, ldc, M, N, K);
+  // 33 to 64 rows of a weight whose 128-column tiles fill half of the chip or more: pipelined tiles of 64 rows (64 rows of
+  // 28 672 x 4 096 tiled 453, by the rows' kernel 325, here 166 us)
+  const bool wide = sizeof(T) == 4 && pieces && K % STAGE_K == 0 && M > 32 && 2 * lq_ceil_div(N, TILE) >= lq_compute_units();
+  if (M <= 64 && pieces && !wide) {
+    // Microseconds before (up to 16 rows: 8 waves, all of x at once; beyond: the tiled kernel) and now, float32: 4 rows of
+    // 28 672 x 4 096 124 -> 109, of 128 256 x 4 096 507 -> 431, of 4 096 x 14 336 55 -> 50, of 4 096 x 4 096 23 -> 19; 17 rows of
+    // 28 672 x 4 096 300 -> 160, 40 rows of 4 096 x 4 096 239 -> 46.
+    const bool sixteen = M <= 32 && lq_ceil_div(N, 16) <= lq_compute_units() && K > 8 * CHUNK;
+    const auto kernel = M > 32 ? gemm_f32_rows_kernel<T, TO, 4, 8>
+                        : M > 16 ? (sixteen ? gemm_f32_rows_kernel<T, TO, 2, 16> : gemm_f32_rows_kernel<T, TO, 2, 8>)
+                                 : (sixteen ? gemm_f32_rows_kernel<T, TO, 1, 16> : gemm_f32_rows_kernel<T, TO, 1, 8>);
+    kernel<<<lq_ceil_div(N, 16), sixteen ? 1024 : 512, 0, stream>>>((const T*)x, lda, (const T*)w, ldw, (TO*)out, ldc, M, N, K);
     LQ_CHECK_LAUNCH("linear(float32 rows)");
     return 0;
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (wide || (pieces && M > 64 && N > 64 && K % STAGE_K == 0)) {
+      const int tiles_n = lq_ceil_div(N, TILE), cus = lq_compute_units();
+      const long long whole = (long long)lq_ceil_div(M, TILE) * tiles_n, halves = (long long)lq_ceil_div(M, TILE / 2) * tiles_n;
+      LQ_REQUIRE(halves < (1ll << 30), "linear: too many tiles");
+      // tiles of 64 rows where the fullest compute unit then has less to do (865 x 6 144 x 4 096 546 -> 448 us, 300 x 6 144 x
+      // 4 096 282 -> 166; where both come to the same the whole tile is a little faster: 3 623 against 3 841 at 2 048 rows)
+      const bool half = lq_ceil_div64(halves, cus) < 2 * lq_ceil_div64(whole, cus);
+      const long long tiles = half ? halves : whole;
+      const auto kernel = half ? gemm_f32_pipelined_kernel<TO, 2> : gemm_f32_pipelined_kernel<TO, 4>;
+      kernel<<<(int)((tiles + 7) / 8 * 8), 256, 0, stream>>>((const float*)x, lda, (const float*)w, ldw, (TO*)out, ldc, M, N, K,
+                                                            (int)(tiles / tiles_n), tiles_n);
+      LQ_CHECK_LAUNCH("linear(float32 pipelined)");
+      return 0;
+    }
   }
   if (M > 64 && N > 64) {
     dim3 grid(lq_ceil_div(N, 128), lq_ceil_div(M, 128));
