@@ -181,6 +181,9 @@ class _Arena:
         nbytes = (int(nbytes) + self.ALIGN - 1) // self.ALIGN * self.ALIGN
         self.buf = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         self._typed = {}  # dtype -> the whole buffer seen as that dtype: a piece of it is one view away
+        # (place, shape, dtype) -> the view given out for it before: the layers of a step ask for the same pieces again,
+        # and making a view costs the host more than looking one up (a step of 17 rows asks 131 times).  Bounded.
+        self._views = {}
 
     def rewind(self) -> None:
         self.off = 0
@@ -193,30 +196,41 @@ class _Arena:
         self.high = 0
         self._spill = []
 
+    MAX_VIEWS = 1024
+
     def alloc(self, shape, dtype: torch.dtype, frozen: bool) -> torch.Tensor:
+        start = (self.off + self.ALIGN - 1) // self.ALIGN * self.ALIGN
+        shape = tuple(shape)
+        seen = self._views.get((start, shape, dtype))
+        if seen is not None:
+            view, self.off = seen
+            if self.off > self.high:
+                self.high = self.off
+            return view
         n = 1
         for s in shape:
             n *= int(s)
-        nbytes = n * dtype.itemsize
-        start = (self.off + self.ALIGN - 1) // self.ALIGN * self.ALIGN
-        end = start + nbytes
+        end = start + n * dtype.itemsize
         self.off = end
         self.high = max(self.high, end)
         if end > self.buf.numel():
             if frozen:
                 raise RuntimeError("workspace of a captured graph is too small for this step")
-            t = torch.empty(tuple(shape), dtype=dtype, device=self.device)  # this step only; reset() grows
+            t = torch.empty(shape, dtype=dtype, device=self.device)  # this step only; reset() grows
             self._spill.append(t)
             return t
         base = self._typed.get(dtype)
         if base is None:
             base = self._typed[dtype] = self.buf.view(dtype)
-        shape = tuple(shape)
         strides, step = [], 1
         for d in reversed(shape):
             strides.append(step)
             step *= int(d)
-        return base.as_strided(shape, strides[::-1], start // dtype.itemsize)
+        view = base.as_strided(shape, strides[::-1], start // dtype.itemsize)
+        if len(self._views) >= self.MAX_VIEWS:
+            self._views.clear()
+        self._views[start, shape, dtype] = (view, end)
+        return view
 
 
 class Workspace:
