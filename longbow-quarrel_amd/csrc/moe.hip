@@ -78,10 +78,141 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
       if (out(e) >= 0.f) out(e) /= total;
 }
 
+constexpr int ROUTE_PER = 16;  // outputs a lane at most in the kernels below
+
+// The same choice with a wavefront a row, for up to 64 PER experts: lane l has the outputs l, l + 64, ...  A thread a row
+// reads its logits one behind the other and works out every score again in each of its `top` searches: at 8 rows a chain
+// of latencies on one wavefront, whatever the rest of the chip does.  Here the scores are made once, a search is a maximum
+// over the lanes, and a group's mark is one lane's search in LDS.  Sums are added up in the order of the kernel above, so
+// the weights are the same to the bit.
+// A thread a row -> a wavefront a row, the same bits: 8 rows, 2 of 8 experts 8.1 -> 2.9 us; 8 rows, 4 of 16 in groups
+// with a softmax 29 -> 5.6; 8 rows, 8 of 64 in groups 220 -> 7.1; 2635 rows of 16 35.7 -> 6.3; 17 rows of 1024 1414 -> 45.
+template <int PER>
+__global__ __launch_bounds__(256) void moe_route_lanes_kernel(const float* __restrict__ z, int ldz, float* __restrict__ route,
+                                                              int rows, int E, int top, int renorm,
+                                                              const float* __restrict__ correction, int groups, int keep,
+                                                              int softmax, int mark_max, float renorm_eps,
+                                                              float* __restrict__ ident, int n_ident) {
+  extern __shared__ float lds[];  // [4][E]: a row's choice scores, where groups are marked
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (r >= rows) return;  // (a wavefront shares nothing with the others: no barrier below)
+  float s[PER], v[PER];   // scores; what the choice goes by
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int e = lane + 64 * j;
+    s[j] = e < E ? z[(long long)r * ldz + e] : -INFINITY;
+  }
+  if (softmax) {
+    float zmax = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) zmax = fmaxf(zmax, s[j]);
+    zmax = wave_max(zmax);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      s[j] = expf(s[j] - zmax);
+      const int n = E - 64 * j < 64 ? E - 64 * j : 64;
+      for (int i = 0; i < n; ++i) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[j]), i));
+    }
+    const float inv_sum = 1.f / sum;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) s[j] *= inv_sum;
+  } else {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) s[j] = 1.f / (1.f + expf(-s[j]));
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int e = lane + 64 * j;
+    v[j] = correction != nullptr && e < E ? s[j] + correction[e] : s[j];
+  }
+  // Of the lanes' values the largest, the lowest index among equals; a value that is no number counts only where it is
+  // the first of the candidates (which bit j of `from` marks), and then wins.  -> its index, or -1
+  auto pick = [&](const float* val, unsigned from, int n) {
+    int first = -1;
+    float most = -INFINITY;
+#pragma unroll
+    for (int j = PER - 1; j >= 0; --j) {
+      if (j >= n) continue;
+      const unsigned long long some = __ballot((from >> j) & 1u);
+      if (some != 0ull) first = 64 * j + (int)__builtin_ctzll(some);
+      if (((from >> j) & 1u) && val[j] > most) most = val[j];
+    }
+    if (first < 0) return -1;
+    most = wave_max(most);
+    int best = first;
+    bool odd = false;
+#pragma unroll
+    for (int j = PER - 1; j >= 0; --j) {
+      if (j >= n) continue;
+      const unsigned long long same = __ballot(((from >> j) & 1u) && val[j] == most);
+      if (same != 0ull) best = 64 * j + (int)__builtin_ctzll(same);
+      odd = odd || __ballot(64 * j + lane == first && val[j] != val[j]) != 0ull;
+    }
+    return odd ? first : best;
+  };
+  unsigned from = 0;  // bit j: output lane + 64 j may still be chosen
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (lane + 64 * j < E) from |= 1u << j;
+  if (groups > 1 && keep < groups) {
+    float* mine = lds + (threadIdx.x >> 6) * E;
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (lane + 64 * j < E) mine[lane + 64 * j] = v[j];
+    __builtin_amdgcn_wave_barrier();
+    __threadfence_block();
+    const int per = E / groups;
+    float a = -INFINITY, b = -INFINITY;  // the two largest choice scores of group `lane`
+    if (lane < groups)
+      for (int i = 0; i < per; ++i) {
+        const float x = mine[lane * per + i];
+        if (x > a) b = a, a = x;
+        else if (x > b) b = x;
+      }
+    float mark[PER];
+    mark[0] = per > 1 && !mark_max ? a + b : a;
+    unsigned left = lane < groups ? 1u : 0u;
+    unsigned long long kept = 0ull;  // bit g: group g may be chosen from
+    for (int n = 0; n < keep; ++n) {
+      const int g = pick(mark, left, 1);
+      if (g < 0) break;
+      kept |= 1ull << g;
+      if (lane == g) left = 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (lane + 64 * j < E && !((kept >> ((lane + 64 * j) / per)) & 1ull)) from &= ~(1u << j);
+  }
+  float total = 0.f;
+  unsigned chosen = 0;
+  for (int k = 0; k < top; ++k) {
+    const int best = pick(v, from, PER);
+    if (best < 0) break;
+    float w = 0.f;
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (best / 64 == j) w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[j]), best % 64));
+    total += w == w ? w : 0.f;
+    if (lane == best % 64) from &= ~(1u << (best / 64)), chosen |= 1u << (best / 64);
+  }
+  total += renorm_eps;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int e = lane + 64 * j;
+    if (e >= E) continue;
+    float w = -1.f;
+    if ((chosen >> j) & 1u) {
+      w = s[j] == s[j] ? s[j] : 0.f;
+      if (renorm && total > 0.f) w /= total;
+    }
+    const int R = E - n_ident;
+    if (e < R) route[(long long)r * R + e] = w;
+    else ident[(long long)r * n_ident + e - R] = w;
+  }
+}
+
 // The `top` largest logits win (the lower index on a tie) and the weights are the softmax over these alone.  A wavefront a
 // row: lane l has the logits l, l + 64, ...; every round finds the largest that is left.
-constexpr int ROUTE_PER = 16;  // logits a lane at most
-
 __global__ __launch_bounds__(256) void moe_route_chosen_kernel(const float* __restrict__ z, int ldz, float* __restrict__ route,
                                                                int rows, int E, int top) {
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -329,8 +460,19 @@ extern "C" int lq_moe_route(const float* z, int ldz, float* route, int rows, int
     LQ_CHECK_LAUNCH("moe_route(softmax over the chosen)");
     return 0;
   }
-  moe_route_kernel<<<lq_ceil_div(rows, 64), 64, 0, stream>>>(z, ldz, route, rows, experts, top, renormalize, correction,
-                                                             groups, keep, softmax, mark_max, renorm_eps, ident, n_ident);
+  // (up to 16 outputs a lane, as above; more would not stay in registers)
+  const size_t lds = groups > 1 ? 4 * (size_t)experts * sizeof(float) : 0;
+#define LQ_ROUTE(PER)                                                                                                \
+  moe_route_lanes_kernel<PER><<<lq_ceil_div(rows, 4), 256, lds, stream>>>(z, ldz, route, rows, experts, top, renormalize, \
+                                                                          correction, groups, keep, softmax, mark_max,  \
+                                                                          renorm_eps, ident, n_ident)
+  if (experts <= 64) LQ_ROUTE(1);
+  else if (experts <= 256) LQ_ROUTE(4);
+  else if (experts <= 64 * ROUTE_PER) LQ_ROUTE(ROUTE_PER);
+  else
+    moe_route_kernel<<<lq_ceil_div(rows, 64), 64, 0, stream>>>(z, ldz, route, rows, experts, top, renormalize, correction,
+                                                               groups, keep, softmax, mark_max, renorm_eps, ident, n_ident);
+#undef LQ_ROUTE
   LQ_CHECK_LAUNCH("moe_route");
   return 0;
 }
