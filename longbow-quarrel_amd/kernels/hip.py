@@ -436,9 +436,11 @@ class HipKernels:
             return False
         return bool(self.lib.lq_linear_swiglu_supported(c_int(_DTYPE_CODE[dtype]), c_int(rows_out), c_int(k)))
 
+    _GLU_FORMS = {"silu": 0, "gelu_tanh": 1, "relu": 2}
+
     def linear_swiglu(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, activation: str = "silu") -> None:
         """out[M, I] = silu(gate) * up with [gate | up] = x . w^T, in one kernel; `activation` "gelu_tanh": the tanh form
-        of gelu in silu's place (bfloat16 out).  w [2 I, K] holds the
+        of gelu, "relu": relu in silu's place (bfloat16 out).  w [2 I, K] holds the
         gate and up rows interleaved in groups of 8: rows 16j..16j+7 gate 8j..8j+7, rows 16j+8..16j+15
         up 8j..8j+7 (see `interleave_gate_up`)."""
         m, k, ldx = self._mat(x, "linear_swiglu: x")
@@ -447,10 +449,10 @@ class HipKernels:
         if kw != k or mo != m or no != n // 2 or n % 16 != 0 or x.dtype != w.dtype:
             raise KernelLibraryError(
                 f"linear_swiglu: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)} do not fit")
-        if activation not in ("silu", "gelu_tanh"):
+        if activation not in self._GLU_FORMS:
             raise KernelLibraryError(f"linear_swiglu: activation {activation!r}")
         rc = self.lib.lq_linear_swiglu(x.data_ptr(), w.data_ptr(), out.data_ptr(), _code(x), _code(out), m, n, k,
-                                       ldx, ldw, ldc, _packed(w), 1 if activation == "gelu_tanh" else 0, self.stream)
+                                       ldx, ldw, ldc, _packed(w), self._GLU_FORMS[activation], self.stream)
         if rc:
             self._check(rc)
 

@@ -72,8 +72,8 @@ class SwiGLU(FeedForward):
 @FEED_FORWARDS.register("glu")
 class GatedLinearUnit(FeedForward):
     """down(act(gate(h)) * up(h)) with a choice of `activation` ("relu", "silu", "gelu_tanh").  gate and up are one
-    matrix product whose 32-bit result the activation kernel reads; with "gelu_tanh" and no bias, in a bfloat16 run, the
-    product's epilogue applies it (gate and up rows interleaved when weights are bound).  With `bias` every projection has one
+    matrix product whose 32-bit result the activation kernel reads; with "gelu_tanh" or "relu" and no bias, in a bfloat16
+    run, the product's epilogue applies it to its 32-bit sums (gate and up rows interleaved when weights are bound).  With `bias` every projection has one
     (`<name>.b`): the activation kernel adds gate's and up's; down's is one more column of its weight, which meets a
     column of ones that the activation kernel leaves behind its result."""
 
@@ -112,7 +112,7 @@ class GatedLinearUnit(FeedForward):
         if gate.dtype != up.dtype:
             raise ValueError(f"{self.names['gate']}: gate and up projections are stored in different dtypes")
         kn = env.kernels
-        self.fused = self.activation == "gelu_tanh" and not self.bias and gate.dtype == env.dtype == torch.bfloat16 and \
+        self.fused = self.activation in ("gelu_tanh", "relu") and not self.bias and gate.dtype == env.dtype == torch.bfloat16 and \
             self.inner % 8 == 0 and getattr(kn, "linear_swiglu_supported", lambda *a: False)(gate.dtype, 2 * self.inner, self.width)
         if self.fused:
             self.w_gate_up = product_weight(env, kn.interleave_gate_up(gate, up))
