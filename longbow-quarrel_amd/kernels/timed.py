@@ -49,6 +49,8 @@ class TimedKernels:
         if name.startswith("linear"):
             x = args[0]
             w = args[3] if name == "linear_scaled" else args[1]
+            if isinstance(w, (list, tuple)):  # a run of equal weights (`linear_grouped`)
+                return f"{name} {x.shape[0]} x {w[0].shape[0]} x {w[0].shape[1]} of {len(w)}"
             return f"{name} {x.shape[0]} x {w.shape[0]} x {w.shape[1]}"
         return name
 
