@@ -170,7 +170,12 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
   const int kept_end = min(a.keep_first, wstart);  // kept keys that lie below that block
 
   float m = NONE, l = 0.f;  // the row's running maximum (in powers of two); this lane's share of its sum
-  if (a.sink && ks == 0) m = a.sinks != nullptr ? a.sinks[h] * LOG2E : 0.f, l = hf == 0 ? 1.f : 0.f;
+  if (a.sink && ks == 0) {
+    // (a sink of -inf, or so low that it is in powers of two, adds nothing: the maximum itself stays finite, since -inf
+    // less -inf is no number in a row that sees none of its first keys)
+    const float s = a.sinks != nullptr ? a.sinks[h] * LOG2E : 0.f;
+    m = fmaxf(s, NONE), l = hf == 0 ? __builtin_amdgcn_exp2f(s - m) : 0.f;
+  }
   f32x16 o[VT];
 #pragma unroll
   for (int dt = 0; dt < VT; ++dt)

@@ -22,6 +22,9 @@ CASES = [  # heads, key heads, key size, value size, (new, held) of every sequen
     (4, 1, 200, 104, [(50, 15)], PLAIN),
     (8, 2, 128, 128, [(90, 300)], dict(sinks=True, cap=30.0, log=True, window=200)),
     (8, 2, 64, 64, [(90, 300)], dict(PLAIN, cap=5.0, dist=100, temp=True, wide=True)),
+    (8, 2, 128, 128, [(130, 300), (40, 0)], dict(sinks="lowest", window=100)),
+    (4, 1, 64, 64, [(200, 30)], dict(sinks="none", chunk=50)), (8, 4, 200, 104, [(100, 90)], dict(sinks="lowest", window=40)),
+    (6, 3, 128, 256, [(140, 64)], dict(sinks="none", window=33, keep_first=3)),
 ]
 
 
@@ -31,7 +34,8 @@ SINGLE = [  # heads, key heads, key size, value size, options
     (16, 1, 256, 192, PLAIN), (40, 2, 64, 40, dict(sinks=True, gate=True)), (4, 1, 256, 256, PLAIN),
     (8, 4, 128, 256, dict(PLAIN, maps=2, window=600)), (3, 3, 40, 24, dict(window=1, wide=True)),
     (8, 2, 128, 128, dict(sinks=True, cap=30.0, log=True, window=200)),
-    (8, 2, 64, 64, dict(PLAIN, cap=5.0, dist=100, temp=True, wide=True))]
+    (8, 2, 64, 64, dict(PLAIN, cap=5.0, dist=100, temp=True, wide=True)),
+    (8, 2, 128, 128, dict(sinks="lowest", window=100)), (4, 1, 64, 64, dict(sinks="none", chunk=50))]
 
 
 @pytest.mark.parametrize("shared", [False, True])
@@ -72,6 +76,10 @@ def check(H, G, D, P, seqs, options, shared):
                 chunk=o.get("chunk", 0), softcap=o.get("cap", 0.0))
     if "sinks" in o:
         more["sink_values"] = rand(H)
+        lowest = {"none": [float("-inf")], "lowest": [torch.finfo(torch.float32).min, -2.4e38, -2.0e38, float("-inf")]}.get(o["sinks"], [])
+        for i in range(H if lowest else 0):  # (a sink that says no more than an absent one, beside ordinary ones)
+            if i % 3 < 2:
+                more["sink_values"][i] = lowest[i % len(lowest)]
     if "gate" in o:
         more["gate"] = rand(rows, H).bfloat16()
     if "wide" in o:
