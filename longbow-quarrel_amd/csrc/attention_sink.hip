@@ -8,11 +8,16 @@
 // there is a sink (a key of score 0 without a value; with `sinks`, a learned score a query head that is not scaled:
 // the maximum starts there), at -inf and 0 otherwise.  out = sum p_t v_t, times
 // sigmoid(gate[r, h]) where a gate is given.  Scores, probabilities and sums are 32-bit for either dtype of
-// q and the cache; the products run on the matrix cores in their 32-bit mode (v_mfma_f32_16x16x4_f32).
+// q and the cache.
 //
-// Keys are walked in chunks of 64 aligned to absolute positions, the kept first chunks before the window's, so
-// the order of every sum depends on the row's position only: not on how the tokens were cut into steps nor on
-// what else is in the batch.
+// Of a bfloat16 run, prompts take the tiles of attention_sink_rows.hip and single tokens those of
+// attention_sink_decode.hip, where sizes, strides and alignment allow it (the rules stand there); everything else runs
+// here, the products on the matrix cores in their 32-bit mode (v_mfma_f32_16x16x4_f32).
+//
+// Keys are walked in blocks of 64 aligned to absolute positions, the kept first blocks before the window's.  Here and
+// for prompts the order of every sum depends on the row's position only: not on how the tokens were cut into steps nor
+// on what else is in the batch.  The shares of a single token's keys in a bfloat16 run depend on the step's number of
+// rows and its bound of the lengths, and so does the order in which they are added up.
 //
 // Cache layout: K[block][kv head][offset][key size], V[block][kv head][value size][offset].
 //

@@ -268,7 +268,8 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
       for (int e = 1; e < 16; ++e) top = fmaxf(top, sc[e]);
       top = halves_max(top);
       if (__any(top > m + SLACK)) {
-        const float m_new = fmaxf(m, top), alpha = __builtin_amdgcn_exp2f(m - m_new);
+        // (each row by its own scores: its roundings do not depend on which rows share the tile)
+        const float m_new = top > m + SLACK ? top : m, alpha = __builtin_amdgcn_exp2f(m - m_new);
         l *= alpha;
         m = m_new;
 #pragma unroll

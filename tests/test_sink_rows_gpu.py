@@ -117,3 +117,31 @@ def check(H, G, D, P, seqs, options, shared):
         assert torch.isfinite(want).all()
         far = (got.float() - want.float()).abs()
         assert (far <= 7e-5 + (want.float().abs() * 2 ** -7 if dtype == torch.bfloat16 else 0)).all(), far.max()
+
+
+@pytest.mark.parametrize("H,G,D,P,options", [(8, 2, 128, 128, PLAIN), (4, 1, 64, 64, dict(PLAIN, window=70)), (2, 2, 200, 104, PLAIN)])
+def test_a_row_has_the_same_bits_whatever_its_neighbours(H, G, D, P, options):
+    """A prompt's row beside rows of ordinary scores, beside rows of scores 60 times as large (whose maximum moves in every
+    block), and in a portion of its own length."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(D)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    held, rows = 150, 100
+    k, v, q = rand(4, G, 64, D).bfloat16(), rand(4, G, P, 64).bfloat16(), 3 * rand(rows, H * D)
+    kn = HipKernels()
+
+    def run(first, q):
+        n = q.shape[0]
+        out = torch.full((n, H * P), float("nan"), device="cuda")
+        kn.sink_attention(q.bfloat16(), out, H, G, D, P, i32(range(held + first, held + first + n)), i32([0] * n), i32([0]),
+                          i32([2, 0, 3, 1]).view(1, 4), k, v, 64, D ** -0.5, cu_rows=i32([0, n]), **options)
+        return out
+
+    want = run(0, q)
+    pushed = q.clone()
+    pushed[1::2] *= 60
+    assert torch.equal(run(0, pushed)[::2], want[::2])
+    for first, n in ((0, 2), (31, 40), (57, 43)):
+        assert torch.equal(run(first, q[first : first + n]), want[first : first + n]), (first, n)
