@@ -78,6 +78,12 @@ __device__ inline void put_out(T* out, long long at, float v, int out_f32) {
   else out[at] = from_f32<T>(v);
 }
 
+// Eight neighbouring entries of a row of q, which starts on 8 bytes.
+__device__ inline uint4 load_q8(const bf16_t* p) {
+  const uint2 lo = *(const uint2*)p, hi = *(const uint2*)(p + 4);
+  return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+
 inline bool scores_shaped(const ScoreShape& s) {
   return s.cap > 0.f || s.temp != nullptr || s.r1 != nullptr || s.dist != nullptr;
 }

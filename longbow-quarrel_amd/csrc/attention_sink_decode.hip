@@ -87,7 +87,7 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int d = 32 * ks + 8 * g;
-    qf[ks] = d < KD ? *(const u32x4*)(q + (long long)r * a.ldq + h * KD + d) : (u32x4){0u, 0u, 0u, 0u};
+    qf[ks] = d < KD ? __builtin_bit_cast(u32x4, load_q8(q + (long long)r * a.ldq + h * KD + d)) : (u32x4){0u, 0u, 0u, 0u};
   }
   HeadShape hs;
   if constexpr (SHAPED) hs = head_shape(a, h);
@@ -318,7 +318,7 @@ long long lq_sink_decode_workspace(int rows, int nh, int nkv, int KD, int VD, in
 int lq_sink_decode(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache,
                    const SinkArgs& a, int max_len, float* part, long long part_floats, int* tickets, long long tickets_n,
                    hipStream_t stream) {
-  if (a.ldq % 8 != 0 || ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) % 16 != 0 ||
+  if (a.ldq % 4 != 0 || (uintptr_t)q % 8 != 0 || ((uintptr_t)kcache | (uintptr_t)vcache) % 16 != 0 ||
       !takes(a.KD, a.VD, a.BS, a.nh, a.nkv, a.rows))
     return 0;
   const int tiles = a.nkv * lq_ceil_div(a.nh / a.nkv, 16);

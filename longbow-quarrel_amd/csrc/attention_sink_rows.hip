@@ -151,7 +151,8 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
 #pragma unroll
   for (int kk = 0; kk < KS16; ++kk) {
     const int unit = 2 * kk + hf;
-    qf[kk] = unit < k_units ? *(const u32x4*)(q + (long long)my_row * a.ldq + h * KD + unit * 8) : (u32x4){0u, 0u, 0u, 0u};
+    qf[kk] = unit < k_units ? __builtin_bit_cast(u32x4, load_q8(q + (long long)my_row * a.ldq + h * KD + unit * 8))
+                            : (u32x4){0u, 0u, 0u, 0u};
   }
   // (lane i reads the operand row of key i with bits 2 and 3 exchanged)
   const int key_of_lane = (c & ~12) | ((c & 4) << 1) | ((c & 8) >> 1);
@@ -404,7 +405,9 @@ int lq_sink_rows32(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t*
   // Values of more than 128 or keys of more than 128 entries have no registers for two wavefronts a SIMD: a wavefront
   // there takes both halves of a block (two wavefronts, spilling: 126 and 146 microseconds for the two cases above).
   // 32-bit results against 64 bits: relative error 1.9e-7 (2.2e-7 before) at 2 048 rows.
-  const bool aligned = a.ldq % 8 == 0 && ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 &&
+  // Rows of q lie any multiple of 4 entries apart: they may be part of a product's wider rows (a gate a head behind 12
+  // heads: 2 316 entries).
+  const bool aligned = a.ldq % 4 == 0 && (uintptr_t)q % 8 == 0 && ((uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 &&
                        a.ldo % 4 == 0 && (uintptr_t)out % (a.out_f32 ? 16 : 8) == 0;
   if (!aligned || a.BS != BLOCK || a.KD % 8 != 0 || a.VD % 8 != 0 || a.KD > 256 || a.VD > 256 ||
       (a.KD > 128 && a.VD > 192))

@@ -108,6 +108,12 @@ def check(H, G, D, P, seqs, options, shared):
         for _ in range(2):  # (a launch leaves the tickets as it found them)
             got.fill_(float("nan"))
             kn.sink_attention(q, got, *args, **how, **more)
+        # rows of q 4 entries more than a multiple of 8 apart, and starting on 8 bytes: the same kernel, the same bits
+        wide = torch.zeros(rows, H * D + (4 if H * D % 8 == 0 else 0) + 8, dtype=q.dtype, device="cuda")
+        wide[:, 4 : 4 + H * D] = q
+        apart = torch.full_like(got, float("nan"))
+        kn.sink_attention(wide[:, 4 : 4 + H * D], apart, *args, **how, **more)
+        assert torch.equal(apart, got)
         kn.force_generic = True
         kn.sink_attention(q, want, *args, **more)
         kn.force_generic = False
