@@ -8,9 +8,9 @@
 // (tiles that asked for a few bytes of a key row at a time, a product between, and a second launch that merged the
 // shares: microseconds before and now, 8 rows, 16 heads: 4 key heads of 128 at 512 keys 20 -> 12, at 1 500 keys under a
 // window of 1 024 31 -> 13, with values of 256 and two maps 28 -> 16; one key head of 256 with values of 192 28 -> 21;
-// 64 rows at 500 keys 34 -> 19; 2 rows with capped scores and a table of biases 30 -> 15).  The shares of a row meet in its last workgroup to finish
-// (a ticket a row and key head; partial results pass the dies' caches as device-scope atomics), which adds them up in
-// their order.
+// 64 rows at 500 keys 34 -> 19; 2 rows with capped scores and a table of biases 30 -> 15).  The shares of a row meet in its
+// last workgroup to finish (a ticket a row and key head; partial results pass the dies' caches as device-scope atomics),
+// which adds them up in their order; a caller who gives no tickets gets a second launch that does the same.
 //
 //   S^T[key][head] = K . Q^T by v_mfma_f32_16x16x32_bf16: lane (c = l % 16, g = l / 16) gives A[c][8 g .. + 8] and B[c][the
 //   same] and receives D[4 g + e][c].  Row i of tile j (of a run of 32 keys) is key 8 (i / 4) + 4 j + i % 4: a lane's scores
@@ -57,8 +57,96 @@ __device__ inline float published(const float* p) {
 struct Shares {
   int splits;
   float* part;   // [row][key head's tile][split]: cols x VD results, then cols maxima and cols sums
-  int* tickets;  // [row][key head's tile], zero between launches
+  int* tickets;  // [row][key head's tile], zero between launches; or null: a second launch adds the shares up
 };
+
+// Which keys a row sees, in blocks of 64 positions, the kept first ones below the window's.
+struct Blocks {
+  int lo, wstart, kept, n;
+};
+__device__ inline Blocks blocks_of(const SinkArgs& a, int pos) {
+  Blocks b;
+  b.lo = first_key(a, pos);
+  b.wstart = b.lo / BLOCK * BLOCK;                                // first block of the window
+  b.kept = (min(a.keep_first, b.wstart) + BLOCK - 1) / BLOCK;     // blocks of kept keys below it
+  b.n = b.kept + pos / BLOCK - b.wstart / BLOCK + 1;
+  return b;
+}
+__device__ inline int live_shares(const Shares& sh, const Blocks& b) {  // shares with a block for some wavefront
+  return min(sh.splits, (b.n + NW - 1) / NW);
+}
+
+// A workgroup's row and key head's tile: its query heads hbase .. hbase + cols - 1.
+struct Heads {
+  int kvh, hbase, cols, share_floats;
+};
+__device__ inline Heads heads_of(const SinkArgs& a) {
+  const int group = a.nh / a.nkv, tiles = (group + 15) / 16, kvh = blockIdx.y / tiles;
+  const int hbase = kvh * group + blockIdx.y % tiles * 16;
+  return {kvh, hbase, min(16, (kvh + 1) * group - hbase), min(16, group) * (a.VD + 2)};
+}
+
+// A head's entry (idx: of the tile's cols x VD) from its sum over the keys and that of the probabilities.
+__device__ inline void finish(void* out, const bf16_t* gate, const SinkArgs& a, int r, int hbase, int idx, float sum, float L) {
+  float f = 1.0f / L;
+  const int hh = hbase + idx / a.VD, first = hbase * a.VD;
+  if (gate != nullptr) f /= 1.f + expf(-to_f32(gate[(long long)r * a.ldg + hh]));
+  float v = sum * f;
+  if (a.wide_gate != nullptr) v /= 1.f + expf(-a.wide_gate[(long long)r * a.ldwg + first + idx]);
+  put_out((bf16_t*)out, (long long)r * a.ldo + first + idx, v, a.out_f32);
+}
+
+// The shares of a row and tile added up in their order, by a whole workgroup.
+__device__ inline void add_shares(void* out, const bf16_t* gate, const SinkArgs& a, const Shares& sh, const Heads& hd, int live) {
+  __shared__ float factor[MAX_SPLITS][16], sums[MAX_SPLITS][16], whole[16];
+  const int tid = threadIdx.x, r = blockIdx.x, cols = hd.cols, VD = a.VD;
+  const float* shares = sh.part + ((long long)r * gridDim.y + blockIdx.y) * sh.splits * hd.share_floats;
+  // every share's factor for every head, and the heads' sums ...
+  for (int x = tid; x < live * cols; x += NW * 64) {
+    const int s = x / cols, cc = x - s * cols;
+    const float* p = shares + s * hd.share_floats + cols * VD + cc;
+    factor[s][cc] = published(p), sums[s][cc] = published(p + cols);
+  }
+  __syncthreads();
+  if (tid < cols) {
+    float M = NONE, L = 0.f;
+    for (int s = 0; s < live; ++s) M = fmaxf(M, factor[s][tid]);
+    for (int s = 0; s < live; ++s) {
+      const float f = __builtin_amdgcn_exp2f(factor[s][tid] - M);
+      factor[s][tid] = f, L = fmaf(f, sums[s][tid], L);
+    }
+    whole[tid] = L;
+  }
+  __syncthreads();
+  // ... then their results, four entries of four shares asked for together
+  for (int i0 = tid; i0 < cols * VD; i0 += 4 * NW * 64) {
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < live; s0 += 4) {
+      float v[4][4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          v[j][x] = published(shares + min(s0 + j, live - 1) * hd.share_floats + min(i0 + x * NW * 64, cols * VD - 1));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          if (s0 + j < live) sum[x] = fmaf(factor[s0 + j][min(i0 + x * NW * 64, cols * VD - 1) / VD], v[j][x], sum[x]);
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int idx = i0 + x * NW * 64;
+      if (idx < cols * VD) finish(out, gate, a, r, hd.hbase, idx, sum[x], whole[idx / VD]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(NW * 64) void sink_add_shares_kernel(void* __restrict__ out, const bf16_t* __restrict__ gate,
+                                                                  SinkArgs a, Shares sh) {
+  const int live = live_shares(sh, blocks_of(a, a.row_pos[blockIdx.x]));
+  if (live > 1) add_shares(out, gate, a, sh, heads_of(a), live);  // (else the row is finished)
+}
 
 // KD and VD up to 32 KS and 16 VT: sizes in between run with zeros behind their keys and values.
 template <int KS, int VT, bool SHAPED>
@@ -69,19 +157,17 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
   __shared__ float lds_m[NW][16], lds_l[NW][16];
   __shared__ int last;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
-  const int r = blockIdx.x, split = blockIdx.z, group = a.nh / a.nkv, tiles = (group + 15) / 16;
-  const int kvh = blockIdx.y / tiles, hbase = kvh * group + blockIdx.y % tiles * 16, cols = min(16, (kvh + 1) * group - hbase);
-  const int h = hbase + min(c, cols - 1);
+  const int r = blockIdx.x, split = blockIdx.z;
+  const Heads hd = heads_of(a);
+  const int kvh = hd.kvh, hbase = hd.hbase, cols = hd.cols, h = hbase + min(c, cols - 1);
   const int nvh = a.nkv / a.maps, vh = kvh / a.maps, KD = a.KD, VD = a.VD, row_floats = VD + 4;
   const long long krow = (long long)a.maps * KD;
 
-  const int pos = a.row_pos[r], lo = first_key(a, pos);
+  const int pos = a.row_pos[r];
   const int* table = a.block_table + (long long)a.seq_slot[a.row_seq[r]] * a.bt_stride;
-  const int wstart = lo / BLOCK * BLOCK;                                         // first block of the window
-  const int kept = (min(a.keep_first, wstart) + BLOCK - 1) / BLOCK;              // blocks of kept keys below it
-  const int blocks = kept + pos / BLOCK - wstart / BLOCK + 1;
-  const int live = min(sh.splits, (blocks + NW - 1) / NW);                       // shares with a block for some wavefront
-  if (split >= live) return;                                                     // the whole workgroup
+  const Blocks seen = blocks_of(a, pos);
+  const int lo = seen.lo, wstart = seen.wstart, kept = seen.kept, blocks = seen.n, live = live_shares(sh, seen);
+  if (split >= live) return;  // the whole workgroup
 
   u32x4 qf[KS];
 #pragma unroll
@@ -185,17 +271,7 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
   if (g == 0) lds_m[w][c] = m, lds_l[w][c] = l;
   __syncthreads();
   const long long at = (long long)r * gridDim.y + blockIdx.y;
-  const int share_floats = min(16, group) * (VD + 2), first = hbase * VD;
-  float* mine = sh.part + (at * sh.splits + split) * share_floats;
-  // a head's entry from its sum over the keys
-  auto finish = [&](int idx, float sum, float L) {
-    float f = 1.0f / L;
-    const int hh = hbase + idx / VD;
-    if (gate != nullptr) f /= 1.f + expf(-to_f32(gate[(long long)r * a.ldg + hh]));
-    float v = sum * f;
-    if (a.wide_gate != nullptr) v /= 1.f + expf(-a.wide_gate[(long long)r * a.ldwg + first + idx]);
-    put_out((bf16_t*)out, (long long)r * a.ldo + first + idx, v, a.out_f32);
-  };
+  float* mine = sh.part + (at * sh.splits + split) * hd.share_floats;
   for (int idx = tid; idx < cols * VD; idx += NW * 64) {
     const int cc = idx / VD, d = idx - cc * VD;
     float M = lds_m[0][cc];
@@ -208,13 +284,13 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
       sum = fmaf(f, lds[(j * 16 + cc) * row_floats + d], sum), L = fmaf(f, lds_l[j][cc], L);
     }
     if (live == 1) {
-      finish(idx, sum, L);
+      finish(out, gate, a, r, hbase, idx, sum, L);
     } else {
       publish(mine + idx, sum);
       if (d == 0) publish(mine + cols * VD + cc, M), publish(mine + cols * VD + cols + cc, L);
     }
   }
-  if (live == 1) return;
+  if (live == 1 || sh.tickets == nullptr) return;
   // Once every thread's stores have completed the workgroup takes a ticket; the last one adds the shares up.
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
@@ -222,47 +298,7 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
     last = __hip_atomic_fetch_add(sh.tickets + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == live - 1;
   __syncthreads();
   if (!last) return;
-  const float* shares = sh.part + at * sh.splits * share_floats;
-  // every share's factor for every head, and the heads' sums ...
-  __shared__ float factor[MAX_SPLITS][16], sums[MAX_SPLITS][16], whole[16];
-  for (int x = tid; x < live * cols; x += NW * 64) {
-    const int s = x / cols, cc = x - s * cols;
-    const float* p = shares + s * share_floats + cols * VD + cc;
-    factor[s][cc] = published(p), sums[s][cc] = published(p + cols);
-  }
-  __syncthreads();
-  if (tid < cols) {
-    float M = NONE, L = 0.f;
-    for (int s = 0; s < live; ++s) M = fmaxf(M, factor[s][tid]);
-    for (int s = 0; s < live; ++s) {
-      const float f = __builtin_amdgcn_exp2f(factor[s][tid] - M);
-      factor[s][tid] = f, L = fmaf(f, sums[s][tid], L);
-    }
-    whole[tid] = L;
-  }
-  __syncthreads();
-  // ... then their results, four entries of four shares asked for together
-  for (int i0 = tid; i0 < cols * VD; i0 += 4 * NW * 64) {
-    float sum[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < live; s0 += 4) {
-      float v[4][4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int x = 0; x < 4; ++x)
-          v[j][x] = published(shares + min(s0 + j, live - 1) * share_floats + min(i0 + x * NW * 64, cols * VD - 1));
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int x = 0; x < 4; ++x)
-          if (s0 + j < live) sum[x] = fmaf(factor[s0 + j][min(i0 + x * NW * 64, cols * VD - 1) / VD], v[j][x], sum[x]);
-    }
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int idx = i0 + x * NW * 64;
-      if (idx < cols * VD) finish(idx, sum[x], whole[idx / VD]);
-    }
-  }
+  add_shares(out, gate, a, sh, hd, live);
   if (tid == 0) __hip_atomic_store(sh.tickets + at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
 }
 
@@ -284,6 +320,10 @@ int launch(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache,
   }
   kernel<<<grid, NW * 64, bytes, stream>>>(q, out, gate, kcache, vcache, a, sh);
   LQ_CHECK_LAUNCH("sink_attention(single tokens)");
+  if (sh.splits > 1 && sh.tickets == nullptr) {
+    sink_add_shares_kernel<<<dim3(grid.x, grid.y), NW * 64, 0, stream>>>(out, gate, a, sh);
+    LQ_CHECK_LAUNCH("sink_attention(shares of single tokens)");
+  }
   return 1;
 }
 
@@ -322,8 +362,8 @@ int lq_sink_decode(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t*
       !takes(a.KD, a.VD, a.BS, a.nh, a.nkv, a.rows))
     return 0;
   const int tiles = a.nkv * lq_ceil_div(a.nh / a.nkv, 16);
-  Shares sh = {1, part, tickets};
-  if (part != nullptr && tickets != nullptr && (long long)a.rows * tiles <= tickets_n) {
+  Shares sh = {1, part, (long long)a.rows * tiles <= tickets_n ? tickets : nullptr};
+  if (part != nullptr) {
     const long long need = lq_sink_decode_workspace(a.rows, a.nh, a.nkv, a.KD, a.VD, a.BS, a.window, a.keep_first, a.chunk, max_len);
     if (need > 0 && need <= part_floats) sh.splits = splits_for(a.rows, a.nh, a.nkv, a.window, a.keep_first, a.chunk, max_len);
   }

@@ -790,7 +790,7 @@ class HipKernels:
                        maps: int = 1, softcap: float = 0.0, temp: Optional[torch.Tensor] = None,
                        log_bias: Optional[tuple] = None, distance_bias: Optional[torch.Tensor] = None,
                        wide_gate: Optional[torch.Tensor] = None, chunk: int = 0,
-                       cu_rows: Optional[torch.Tensor] = None) -> None:
+                       cu_rows: Optional[torch.Tensor] = None, tickets: Optional[torch.Tensor] = None) -> None:
         """Attention of the step's rows over their slots' cached keys: row at position p sees t <= p with
         p - t < window (0: all) or t < keep_first, and with `chunk` > 0 only t of its own run of `chunk` positions
         (p // chunk == t // chunk); with `sink` the softmax's denominator has one more term e^0;
@@ -808,9 +808,11 @@ class HipKernels:
         [heads] each), n the distance p - t; plus `distance_bias` [heads, entries] at column min(n, entries - 1).  The
         sink's score is not shaped.  `wide_gate` float32 [rows, heads * value_dim]: every entry of the result times the
         sigmoid of its own.  `cu_rows` (int32 [batch + 1], where each sequence's rows start): prompts of a bfloat16 run
-        then go by tiles of 32 rows of one sequence."""
+        then go by tiles of 32 rows of one sequence.  `tickets` (int32, zero, and left zero): counters by which the last
+        workgroup of a row adds the shares of its keys up; launches that may overlap have counters (and a workspace) of
+        their own.  Without them a second launch does it."""
         self._dev(q, out, gate, row_pos, row_seq, seq_slot, block_table, kcache, vcache, sink_values, temp, distance_bias,
-                  wide_gate, cu_rows)
+                  wide_gate, cu_rows, tickets)
         rows, batch = q.shape[0], seq_slot.numel()
         self._i32(row_pos, "row_pos", rows)
         self._i32(row_seq, "row_seq", rows)
@@ -845,9 +847,8 @@ class HipKernels:
             self._f32(workspace, "sink_attention: workspace", workspace.numel())
         if cu_rows is not None:
             self._i32(cu_rows, "cu_rows", batch + 1)
-        # (shares of the keys meet by the tickets that the causal attention's decoding uses: launches of one object do
-        # not overlap)
-        tickets = self.tickets(q.device) if workspace is not None else None
+        if tickets is not None:
+            self._i32(tickets, "tickets", tickets.numel())
         rc = self.lib.lq_sink_attention(
             _ptr(q), c_int(self._rows2d(q, "q")), _ptr(out), c_int(self._rows2d(out, "out")), _ptr(gate),
             c_int(0 if gate is None else self._rows2d(gate, "gate")), c_int(_code(q)), c_int(rows), c_int(batch),

@@ -250,6 +250,9 @@ class Workspace:
         self.device = device
         self.step = _Arena(device, nbytes)
         self.runs = [_Arena(device, nbytes), _Arena(device, nbytes)]
+        # counters that a launch finds zero and leaves zero (the steps that use this workspace follow one another): one
+        # for each of a launch's rows of work that are shared out, which are no more than the chip has compute units
+        self.tickets = torch.zeros(1024, dtype=torch.int32, device=device)
         self.cur = 0
         self.frozen = False  # set while a graph that uses these buffers is alive
 

@@ -69,7 +69,7 @@ def split_scratch(ctx: StepContext, dtype, heads: int, kv_heads: int, key_dim: i
         return {"cu_rows": ctx.cu_rows}
     need = ask(dtype, ctx.rows, ctx.batch, heads, kv_heads, key_dim, value_dim, block_size, window, keep_first, ctx.max_len,
                **({"chunk": chunk} if chunk else {}))
-    return dict(max_len=ctx.max_len, workspace=ctx.ws.alloc((need,), torch.float32)) if need else {}
+    return dict(max_len=ctx.max_len, workspace=ctx.ws.alloc((need,), torch.float32), tickets=ctx.ws.tickets) if need else {}
 
 
 def distance_rows(rows: int, most: float, window: int = 0) -> List[int]:

@@ -114,6 +114,13 @@ def check(H, G, D, P, seqs, options, shared):
         apart = torch.full_like(got, float("nan"))
         kn.sink_attention(wide[:, 4 : 4 + H * D], apart, *args, **how, **more)
         assert torch.equal(apart, got)
+        if "workspace" in how:  # the shares added up by their last workgroup, or by a second launch: the same bits
+            counters = torch.zeros(1024, dtype=torch.int32, device="cuda")
+            for _ in range(2):  # (a launch leaves the counters as it found them)
+                apart.fill_(float("nan"))
+                kn.sink_attention(q, apart, *args, **how, **more, tickets=counters)
+                assert torch.equal(apart, got) and not counters.any()
+            assert not kn.tickets(q.device).any()  # (the object's own are for the causal attention)
         kn.force_generic = True
         kn.sink_attention(q, want, *args, **more)
         kn.force_generic = False
