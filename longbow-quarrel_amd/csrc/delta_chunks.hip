@@ -20,9 +20,7 @@
 // Chunks count from a sequence's first row of the step; a last chunk's missing tokens take part as zeros.
 #include <type_traits>
 
-#include "device_math.h"
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+#include "scan_chunks.h"
 
 namespace {
 
@@ -41,12 +39,6 @@ struct DeltaArgs {
   int heads, kv_heads, N, P, batch, channel_decay;
   const int *seq_slot, *cu_rows;
 };
-
-__device__ inline f32x4 step4(const f32x4& a, const f32x4& b, f32x4 c) {
-#pragma unroll
-  for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
-  return c;
-}
 
 template <int CTRL>
 __device__ inline float add_from(float keep, float give) {  // the partner's `give` on top of this lane's `keep`
@@ -310,7 +302,11 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
 #pragma unroll
       for (int x = 0; x < i; ++x)
         if (x >= w) Z = step4(*(const f32x4*)&L.m[SUB * i + c][SUB * x + 4 * g] * bi, X[x], Z);
-      X[i] = step4(*(const f32x4*)&L.inv[i][c][4 * g] * -1.f, Z, X[i]);
+      {
+        const float odd = not_finite(Z, 0.f);
+        const f32x4 inv = *(const f32x4*)&L.inv[i][c][4 * g] * -1.f;
+        X[i] = __any(odd != odd) ? step4_lower(inv, Z, X[i]) : step4(inv, Z, X[i]);
+      }
     }
   }
   __syncthreads();  // (A has been read)
@@ -318,7 +314,10 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
 #pragma unroll
     for (int i = 0; i < KT; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) L.m[SUB * i + 4 * g + e][SUB * w + c] = X[i][e] * L.beta[SUB * w + c];
+      for (int e = 0; e < 4; ++e) {  // (a token's beta multiplies none of the zeros above the diagonal: it may be NaN)
+        const int row = SUB * i + 4 * g + e, col = SUB * w + c;
+        L.m[row][col] = row >= col ? X[i][e] * L.beta[col] : 0.f;
+      }
   }
   __syncthreads();
   for (int e = tid; e < KT * KT * 64; e += 512) {
@@ -338,6 +337,7 @@ __device__ inline void lds_barrier() {  // this wavefront's LDS accesses are don
 // operands are asked for as soon as the chunk before has used theirs.
 __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   __shared__ f32x4 Ss[NT][64], Ws[KT][64], Us[KT][64];
+  __shared__ int again;
   const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, p = blockIdx.y * 16 + c, mt = w & 3;
   const bool second = w >= KT;  // Q~, B and the results
@@ -348,15 +348,7 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   const long long step = (long long)a.heads * PART;
   float* sp = a.state + (((long long)a.seq_slot[b] * a.heads + h) * a.P + min(p, a.P - 1)) * a.N;
   const bool live = p < a.P;
-  f32x4 S;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int n = 16 * w + 4 * g + e;
-    S[e] = live && n < a.N ? sp[n] : 0.f;
-  }
-  Ss[w][lane] = S;
-
-  f32x4 rows[NT], tri[KT], upd[KT], V = {0.f, 0.f, 0.f, 0.f}, decay;
+  f32x4 S, rows[NT], tri[KT - 1], diag, upd[KT], V, decay;
   auto ask_rows = [&](const float* from) {
 #pragma unroll
     for (int nb = 0; nb < NT; ++nb)
@@ -364,8 +356,9 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   };
   auto ask_tri = [&](const float* from) {
 #pragma unroll
-    for (int kb = 0; kb < KT; ++kb)
-      if (kb <= mt) tri[kb] = *(const f32x4*)(from + (second ? AT_B : AT_T) + ((mt * KT + kb) * 64 + lane) * 4);
+    for (int kb = 0; kb < KT - 1; ++kb)
+      if (kb < mt) tri[kb] = *(const f32x4*)(from + (second ? AT_B : AT_T) + ((mt * KT + kb) * 64 + lane) * 4);
+    diag = *(const f32x4*)(from + (second ? AT_B : AT_T) + ((mt * KT + mt) * 64 + lane) * 4);
   };
   auto ask_upd = [&](const float* from) {
 #pragma unroll
@@ -379,54 +372,81 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
       V[e] = live && r < r1 ? a.v[r * a.ldv + (long long)h * a.P + p] : 0.f;
     }
   };
-  ask_rows(part), ask_tri(part), ask_upd(part);
-  if (!second) ask_v(r0);
-  lds_barrier();
-  for (int i = 0; i < chunks; ++i, part += step) {
-    const bool more = i + 1 < chunks;
-    const long long c0 = r0 + (long long)i * CHUNK;
-    f32x4 acc[4];  // (four chains of products: their roundings are smaller, and none waits for the one before it)
+  // The triangular products' zeros are no matter until a token brings a NaN or an infinity (V - K~ S or U has one): then
+  // all is walked again, and none of them reaches an earlier token.  (A test of every chunk's operands ahead of those
+  // products lay in the chain and took 0.5 of its 3.3 microseconds; this takes 171 for 168.6 microseconds of a whole launch
+  // of 2 048 tokens.)
+  if (tid == 0) again = 0;  // (barriers follow)
+  int careful = 0;
+  while (true) {
+    const float* from = part;
+    float odd = 0.f;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) acc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int nb = 0; nb < NT; ++nb) acc[nb & 3] = step4(rows[nb], Ss[nb][lane], acc[nb & 3]);
-    f32x4 Y = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    if (more) ask_rows(part + step);
-    if (!second) {
-      Ws[mt][lane] = V - Y;
-      if (more) ask_v(c0 + CHUNK);
+    for (int e = 0; e < 4; ++e) {
+      const int n = 16 * w + 4 * g + e;
+      S[e] = live && n < a.N ? sp[n] : 0.f;
     }
-    lds_barrier();
-    if (!second) {
-      f32x4 U = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kb = 0; kb < KT; ++kb)
-        if (kb <= mt) U = step4(tri[kb], Ws[kb][lane], U);
-      Us[mt][lane] = U;
-      if (more) ask_tri(part + step);
-    }
-    lds_barrier();
-    // (what the chunk adds is summed by itself: one rounding at the state's size a chunk, not one a product)
-    f32x4 add[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int kb = 0; kb < KT; ++kb) add[kb & 1] = step4(upd[kb], Us[kb][lane], add[kb & 1]);
-    S = S * decay + (add[0] + add[1]);
     Ss[w][lane] = S;
-    if (more) ask_upd(part + step);
-    if (second) {
-      f32x4 own = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kb = 0; kb < KT; ++kb)
-        if (kb <= mt) own = step4(tri[kb], Us[kb][lane], own);
-      Y += own;
-      if (more) ask_tri(part + step);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const long long r = c0 + SUB * mt + 4 * g + e;
-        if (live && r < r1) a.out[r * a.ldo + (long long)h * a.P + p] = Y[e];
-      }
-    }
+    V = (f32x4){0.f, 0.f, 0.f, 0.f};
+    ask_rows(from), ask_tri(from), ask_upd(from);
+    if (!second) ask_v(r0);
     lds_barrier();
+    for (int i = 0; i < chunks; ++i, from += step) {
+      const bool more = i + 1 < chunks;
+      const long long c0 = r0 + (long long)i * CHUNK;
+      f32x4 acc[4];  // (four chains of products: their roundings are smaller, and none waits for the one before it)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) acc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int nb = 0; nb < NT; ++nb) acc[nb & 3] = step4(rows[nb], Ss[nb][lane], acc[nb & 3]);
+      f32x4 Y = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      if (more) ask_rows(from + step);
+      if (!second) {
+        const f32x4 W = V - Y;
+        Ws[mt][lane] = W;
+        odd = not_finite(W, odd);
+        if (more) ask_v(c0 + CHUNK);
+      }
+      lds_barrier();
+      if (!second) {
+        f32x4 U = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < KT - 1; ++kb)
+          if (kb < mt) U = step4(tri[kb], Ws[kb][lane], U);
+        U = careful ? step4_lower(diag, Ws[mt][lane], U) : step4(diag, Ws[mt][lane], U);
+        Us[mt][lane] = U;
+        odd = not_finite(U, odd);
+        if (more) ask_tri(from + step);
+      }
+      lds_barrier();
+      // (what the chunk adds is summed by itself: one rounding at the state's size a chunk, not one a product)
+      f32x4 add[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int kb = 0; kb < KT; ++kb) add[kb & 1] = step4(upd[kb], Us[kb][lane], add[kb & 1]);
+      S = S * decay + (add[0] + add[1]);
+      Ss[w][lane] = S;
+      if (more) ask_upd(from + step);
+      if (second) {
+        f32x4 own = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < KT - 1; ++kb)
+          if (kb < mt) own = step4(tri[kb], Us[kb][lane], own);
+        own = careful ? step4_lower(diag, Us[mt][lane], own) : step4(diag, Us[mt][lane], own);
+        Y += own;
+        if (more) ask_tri(from + step);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const long long r = c0 + SUB * mt + 4 * g + e;
+          if (live && r < r1) a.out[r * a.ldo + (long long)h * a.P + p] = Y[e];
+        }
+      }
+      lds_barrier();
+    }
+    if (careful) break;
+    if (odd != odd) again = 1;
+    lds_barrier();  // (no wait for the results' stores)
+    careful = __builtin_amdgcn_readfirstlane(again);
+    if (!careful) break;
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {

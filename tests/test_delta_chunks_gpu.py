@@ -39,3 +39,38 @@ def test_chunks_of_the_delta_rule(lens, H, G, N, P, channel, shift):
         # roundings of 2^-24 a token at the result's size, 200 tokens.
         assert torch.isfinite(walked).all()
         assert (walked - chunked).abs().max() <= 200 * 4 * 2.0 ** -24 * walked.abs().max()
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("what", ["q", "k", "v", "beta", "a"])
+@pytest.mark.parametrize("at", [0, 21, 47, 63, 64, 90])
+def test_what_is_no_number_reaches_later_tokens_only(what, at, channel):
+    """A NaN or an infinity at a token: the results before it stay what they are without it, in chunks as token by token,
+    and from it on the same ones are no numbers."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(at)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, H, G, N, P = 100, 2, 1, 64, 48
+    given = dict(q=rand(rows, G * N), k=rand(rows, G * N), v=rand(rows, H * P), beta=rand(rows, H),
+                 a=0.3 * rand(rows, H * N if channel else H))
+    dt_bias, a_log, state = rand(given["a"].shape[1]) - 3.0, 0.5 * rand(H) + 1.0, rand(1, H, P, N)
+    kn = HipKernels()
+    need = kn.delta_scan_workspace(rows, 1, H, N, P, rows)
+    got = {}
+    for case, bad in (("plain", None), ("nan", float("nan")), ("inf", float("inf"))):
+        t = {name: x.clone() for name, x in given.items()}
+        if bad is not None:
+            t[what][at, :1] = bad
+        for scratch in (None, torch.full((need,), float("nan"), device="cuda")):
+            out, end = torch.full((rows, H * P), float("nan"), device="cuda"), state.clone()
+            more = {} if scratch is None else dict(max_rows=rows, workspace=scratch)
+            kn.delta_scan(t["q"].clone(), t["k"].clone(), t["v"], t["beta"], t["a"], dt_bias, a_log, end, out, H, G, N, P,
+                          N ** -0.5, 1e-6, i32([0]), i32([0, rows]), 1, channel_decay=channel, **more)
+            got[case, scratch is not None] = out, end
+    for bad in ("nan", "inf"):
+        (walked, end0), (chunked, end1) = got[bad, False], got[bad, True]
+        assert torch.equal(chunked[:at], got["plain", True][0][:at])
+        assert torch.equal(torch.isfinite(walked), torch.isfinite(chunked))
+        assert torch.equal(torch.isfinite(end0), torch.isfinite(end1))
