@@ -13,9 +13,9 @@
 // scratch lies in tiles of 16 channels n by 16 columns p in a result's order, lane l's four entries (n = 4 (l / 16) .. + 3,
 // p = l % 16) at 4 l, which is also the order in which the third launch takes it as an operand.
 // Chunks count from a sequence's first row of the step; a last chunk's missing tokens take part as zeros.
-#include "device_math.h"
+#include <type_traits>
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+#include "scan_chunks.h"
 
 namespace {
 
@@ -35,12 +35,6 @@ struct SsdArgs {
 __host__ __device__ inline int n_tiles(int N) { return (N + HALF - 1) / HALF * NT; }
 __host__ __device__ inline int p_tiles(int P) { return (P + 15) / 16; }
 __host__ __device__ inline long long part_floats(int N, int P) { return (long long)n_tiles(N) * p_tiles(P) * FRAG; }
-
-__device__ inline f32x4 step4(const f32x4& a, const f32x4& b, f32x4 c) {
-#pragma unroll
-  for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], c, 0, 0, 0);
-  return c;
-}
 
 // The chunks of all sequences are numbered through.  -> the sequence of chunk number t and its number within it (-1:
 // past the last).  Lane i holds sequence i of a run of 64; every wavefront works out the same.
@@ -237,6 +231,7 @@ struct OutLds {
   float C[CHUNK][LDN], B[CHUNK][LDN], x[CHUNK][LDX];
   float G[CHUNK][LDX];  // first f_st s_s, then that times C_t . B_s
   float decay[CHUNK], step[CHUNK], from_start[CHUNK];
+  int odd;  // x or B has an entry that is no finite number
 };
 
 // A chunk's results.  One workgroup of eight wavefronts a (chunk, head, 64 columns): wavefronts w and w + 4 take 16
@@ -265,8 +260,12 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   };
   ask(0);
   xs.fetch(a.x + r0 * a.ldx + (long long)h * Px + p0, a.ldx, nt, Px - p0);
+  if (tid == 0) L.odd = 0;
   if (tid < CHUNK) token_scalars(a, r0 + tid, tid < nt, h, L.decay[tid], L.step[tid]);
   xs.stash(&L.x[0][0], LDX);
+  float nan_if = 0.f;
+#pragma unroll
+  for (int i = 0; i < xs.PER; ++i) nan_if = not_finite(xs.v[i], nan_if);
   __syncthreads();
   if (a.ones && tid < nt && Px >= p0 && Px < p0 + COLS) L.x[tid][Px - p0] = 1.f;
   if (w == 7) {  // lane s: f_st s_s for every t
@@ -295,6 +294,9 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   auto tile_of = [](int u, int& mt, int& st) { mt = u < 1 ? 0 : u < 3 ? 1 : u < 6 ? 2 : 3, st = u - mt * (mt + 1) / 2; };
   for (int n0 = 0; n0 < a.N; n0 += HALF) {
     cs.stash(&L.C[0][0], LDN), bs.stash(&L.B[0][0], LDN);
+#pragma unroll
+    for (int i = 0; i < bs.PER; ++i) nan_if = not_finite(bs.v[i], nan_if);
+    if (nan_if != nan_if) L.odd = 1;  // (read behind the barriers below)
     f32x4 now[NT];
 #pragma unroll
     for (int nb = 0; nb < NT; ++nb) now[nb] = S[nb];
@@ -323,30 +325,41 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
         inter[i][nb & 3] = step4(*(const f32x4*)&L.C[SUB * (m0 + i) + c][16 * nb + 4 * g], now[nb], inter[i][nb & 3]);
     __syncthreads();
   }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int u = w + 8 * i;
-    if (u < 10) {
-      int mt, st;
-      tile_of(u, mt, st);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) L.G[SUB * mt + 4 * g + e][SUB * st + c] *= G[i][e];
-    }
-  }
-  __syncthreads();
   f32x4 own[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) own[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  // `careful`: what is no finite number reaches no earlier token
+  auto scaled = [&](auto careful) {
 #pragma unroll
-  for (int kb = 0; kb < KT; ++kb) {
-    if (kb > m0 + 1) continue;
-    f32x4 x_;
+    for (int i = 0; i < 2; ++i) {
+      const int u = w + 8 * i;
+      if (u < 10) {
+        int mt, st;
+        tile_of(u, mt, st);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) x_[s] = L.x[SUB * kb + 4 * g + s][16 * pt + c];
+        for (int e = 0; e < 4; ++e)  // (above the diagonal zeros, which a NaN in a later token's B must leave as they are)
+          if (!careful || mt > st || 4 * g + e >= c) L.G[SUB * mt + 4 * g + e][SUB * st + c] *= G[i][e];
+      }
+    }
+    __syncthreads();
+  };
+  auto own_tokens = [&](auto careful) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (kb <= m0 + i) own[i] = step4(*(const f32x4*)&L.G[SUB * (m0 + i) + c][SUB * kb + 4 * g], x_, own[i]);
-  }
+    for (int kb = 0; kb < KT; ++kb) {
+      if (kb > m0 + 1) continue;
+      f32x4 x_;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x_[s] = L.x[SUB * kb + 4 * g + s][16 * pt + c];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (kb <= m0 + i) {
+          const f32x4 G_ = *(const f32x4*)&L.G[SUB * (m0 + i) + c][SUB * kb + 4 * g];
+          own[i] = careful && kb == m0 + i ? step4_lower(G_, x_, own[i]) : step4(G_, x_, own[i]);
+        }
+    }
+  };
+  if (__builtin_amdgcn_readfirstlane(L.odd)) scaled(std::true_type{}), own_tokens(std::true_type{});
+  else scaled(std::false_type{}), own_tokens(std::false_type{});
   const int p = p0 + 16 * pt + c;
   const float D = a.decay == nullptr ? a.d_skip[h] : 0.f;
   if (p >= a.P) return;

@@ -41,3 +41,40 @@ def test_chunks_of_the_state_space_scan(lens, H, G, N, P, given, shift):
     unit = (3 * 200 + N) * 2.0 ** -24 * end0.abs().max().clamp(min=float(state.abs().max()))
     assert (end0 - end1).abs().max() <= unit
     assert (walked - chunked).abs().max() <= unit * c.abs().view(rows, G, N).sum(-1).max() + 1e-6 * walked.abs().max()
+
+
+@pytest.mark.parametrize("given", [False, True])
+@pytest.mark.parametrize("what", ["x", "b", "c", "dt"])
+@pytest.mark.parametrize("at", [0, 21, 47, 63, 64, 110])
+def test_what_is_no_number_reaches_later_tokens_only(what, at, given):
+    """A NaN or an infinity at a token: the results before it stay what they are without it, in chunks as token by token,
+    and from it on the same ones are no numbers."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(at)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, H, G, N, P = 140, 2, 1, 64, 48
+    plain = dict(x=rand(rows, H * (P - given)), b=0.3 * rand(rows, G * N), c=0.3 * rand(rows, G * N), dt=rand(rows, H).abs())
+    made = (rand(H) - 3.0, 0.5 * rand(H) + 1.0, rand(H))
+    more = {}
+    if given:
+        made, more = (None, None, None), dict(decay=torch.sigmoid(rand(rows, H) + 3.0), ones=True)
+    state = rand(1, H, P, N)
+    kn = HipKernels()
+    need = kn.ssd_scan_workspace(1, H, P, N, rows, rows)
+    got = {}
+    for case, bad in (("plain", None), ("nan", float("nan")), ("inf", float("inf"))):
+        t = {name: x.clone() for name, x in plain.items()}
+        if bad is not None:
+            t[what][at, :1] = bad
+        for scratch in (None, torch.full((need,), float("nan"), device="cuda")):
+            y, end = torch.full((rows, H * P), float("nan"), device="cuda"), state.clone()
+            how = {} if scratch is None else dict(max_rows=rows, workspace=scratch, chunks=True)
+            kn.ssd_scan(t["x"], t["b"], t["c"], t["dt"], *made, end, y, H, P, N, G, i32([0]), i32([0, rows]), 1, **how, **more)
+            got[case, scratch is not None] = y, end
+    for bad in ("nan", "inf"):
+        (walked, end0), (chunked, end1) = got[bad, False], got[bad, True]
+        assert torch.equal(chunked[:at], got["plain", True][0][:at])
+        assert torch.equal(torch.isfinite(walked), torch.isfinite(chunked))
+        assert torch.equal(torch.isfinite(end0), torch.isfinite(end1))
