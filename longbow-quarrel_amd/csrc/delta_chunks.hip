@@ -38,6 +38,7 @@ struct DeltaArgs {
   float *state, *out, *scratch;
   int heads, kv_heads, N, P, batch, channel_decay;
   const int *seq_slot, *cu_rows;
+  int first, last;  // the chunks of this pair of launches: numbers first .. last - 1, the scratch of `first` at its start
 };
 
 template <int CTRL>
@@ -134,7 +135,7 @@ template <bool QUADS>
 __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   Prepared& L = *(Prepared*)smem;
-  const int2 at = find_chunk(a.cu_rows, a.batch, blockIdx.x);
+  const int2 at = find_chunk(a.cu_rows, a.batch, a.first + blockIdx.x);
   if (at.x < 0) return;
   const int h = blockIdx.y, j = h / (a.heads / a.kv_heads), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const long long r0 = a.cu_rows[at.x] + (long long)at.y * CHUNK;
@@ -341,10 +342,12 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, p = blockIdx.y * 16 + c, mt = w & 3;
   const bool second = w >= KT;  // Q~, B and the results
-  const long long r0 = a.cu_rows[b], r1 = a.cu_rows[b + 1];
-  const int chunks = (int)((r1 - r0 + CHUNK - 1) / CHUNK);
+  const long long r1 = a.cu_rows[b + 1];
+  const int base = first_chunk(a.cu_rows, b), i0 = max(a.first - base, 0);
+  const int chunks = min((int)((r1 - a.cu_rows[b] + CHUNK - 1) / CHUNK), a.last - base) - i0;  // from the sequence's i0th on
   if (chunks <= 0) return;
-  const float* part = a.scratch + ((long long)first_chunk(a.cu_rows, b) * a.heads + h) * PART;
+  const long long r0 = a.cu_rows[b] + (long long)i0 * CHUNK;
+  const float* part = a.scratch + ((long long)(base + i0 - a.first) * a.heads + h) * PART;
   const long long step = (long long)a.heads * PART;
   float* sp = a.state + (((long long)a.seq_slot[b] * a.heads + h) * a.P + min(p, a.P - 1)) * a.N;
   const bool live = p < a.P;
@@ -466,18 +469,27 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
 // Relative error against 64 bits at 2 048 tokens: 3.3e-7 both ways with a decay every channel, 4.9e-7 and 5.1e-7
 // with one a head; of the state at their end 3.4e-7 and 3.3e-7, 4.5e-7 both.
 constexpr int LQ_DELTA_MIN = 56;
+// A launch of more chunks than the scratch holds goes in rounds of equal numbers of them, each from the state that the
+// last one left: a prompt's scratch is bounded (131.6 KB a chunk and head: 4.3 GB for 65 536 rows of 16 heads).  Rounds
+// cost where the sequences of one leave the chip idle: 32 heads, four of 2 048 tokens 1 007 us in one round (556 MB), 1 002
+// with 256 MB, 1 065 with 128, 1 093 with 64; 8 192 tokens of one sequence 928, 982, 965, 999; 16 heads, eight of 512 240
+// in one round (152 MB), 279 with 128 MB, 287 with 64.
+constexpr long long LQ_DELTA_SCRATCH = 64ll << 20;  // floats
 extern "C" long long lq_delta_scan_workspace(int rows, int batch, int heads, int Dk, int P, int max_rows) {
   if (rows <= 0 || batch <= 0 || heads <= 0 || P <= 0 || Dk <= 0 || Dk > NMAX || max_rows < LQ_DELTA_MIN) return 0;
-  return (long long)(rows / CHUNK + batch) * heads * PART;
+  if (heads > 65535 || lq_ceil_div(P, 16) > 65535) return 0;
+  const long long a_chunk = (long long)heads * PART, most = LQ_DELTA_SCRATCH / a_chunk, all = rows / CHUNK + (long long)batch;
+  return a_chunk * (all <= most ? all : most > 1 ? most : 1);
 }
+extern "C" long long lq_delta_scan_least(int heads) { return (long long)heads * PART; }  // of one chunk
 
-// q and k hold unit vectors already.  -> 0, or -2
+// q and k hold unit vectors already.  `scratch`: at least a chunk's floats for every head.  -> 0, or -2
 int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* beta,
                     int ldbeta, const float* a, int lda, const float* dt_bias, const float* a_log, float* state, float* out,
                     int ldo, int heads, int kv_heads, int Dk, int P, const int* seq_slot, const int* cu_rows, int batch,
-                    int rows, int channel_decay, float* scratch, hipStream_t stream) {
+                    int rows, int channel_decay, float* scratch, long long scratch_floats, hipStream_t stream) {
   DeltaArgs d = {q, k, v, beta, a, dt_bias, a_log, ldq, ldk, ldv, ldbeta, lda, ldo, state, out, scratch,
-                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows};
+                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows, 0, 0};
   const bool quads = Dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && (!channel_decay || lda % 4 == 0) &&
                      (((uintptr_t)q | (uintptr_t)k | (channel_decay ? (uintptr_t)a | (uintptr_t)dt_bias : 0)) & 15) == 0;
   const auto prepare = quads ? delta_prepare_kernel<true> : delta_prepare_kernel<false>;
@@ -490,9 +502,14 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
     }
     configured[quads] = true;
   }
-  prepare<<<dim3(rows / CHUNK + batch, heads), 512, sizeof(Prepared), stream>>>(d);
-  LQ_CHECK_LAUNCH("delta_scan(chunks)");
-  delta_walk_kernel<<<dim3((unsigned)batch * heads, lq_ceil_div(P, 16)), 512, 0, stream>>>(d);
-  LQ_CHECK_LAUNCH("delta_scan(walk over chunks)");
+  const long long all = rows / CHUNK + (long long)batch, fit = scratch_floats / ((long long)heads * PART);
+  const long long rounds = (all + fit - 1) / fit, room = (all + rounds - 1) / rounds;
+  for (long long first = 0; first < all; first += room) {
+    d.first = (int)first, d.last = (int)(first + room < all ? first + room : all);
+    prepare<<<dim3(d.last - d.first, heads), 512, sizeof(Prepared), stream>>>(d);
+    LQ_CHECK_LAUNCH("delta_scan(chunks)");
+    delta_walk_kernel<<<dim3((unsigned)batch * heads, lq_ceil_div(P, 16)), 512, 0, stream>>>(d);
+    LQ_CHECK_LAUNCH("delta_scan(walk over chunks)");
+  }
   return 0;
 }

@@ -1316,11 +1316,13 @@ extern "C" long long lq_delta_scan_workspace(int rows, int batch, int heads, int
 int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* beta,
                     int ldbeta, const float* a, int lda, const float* dt_bias, const float* a_log, float* state, float* out,
                     int ldo, int heads, int kv_heads, int Dk, int P, const int* seq_slot, const int* cu_rows, int batch,
-                    int rows, int channel_decay, float* scratch, hipStream_t stream);
+                    int rows, int channel_decay, float* scratch, long long scratch_floats, hipStream_t stream);
+extern "C" long long lq_delta_scan_least(int heads);
 
 // q and k [rows, kv_heads * Dk], v [rows, heads * P], beta and a [rows, heads] (raw), state [slots, heads, P, Dk],
 // out [rows, heads * P]; `max_rows`: the most rows a sequence brings (0: unknown); `scratch`:
-// lq_delta_scan_workspace(...) floats for a launch in chunks, or null
+// lq_delta_scan_workspace(...) floats for a launch in chunks, or null (fewer make more rounds, down to
+// lq_delta_scan_least(heads))
 // (q and k are made unit vectors in place)
 // `channel_decay`: a [rows, heads * Dk] and dt_bias [heads * Dk], a decay for every key channel of every head
 extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* v, int ldv, const float* beta,
@@ -1339,11 +1341,11 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
   LQ_CHECK_LAUNCH("delta_scan(unit vectors)");
   const long long need = scratch != nullptr ? lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) : 0;
   if (need > 0) {
-    LQ_REQUIRE(need <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
-               "delta_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", need, scratch_floats);
-    LQ_REQUIRE(heads <= 65535 && lq_ceil_div(P, 16) <= 65535, "delta_scan: %d heads of %d values", heads, P);
+    LQ_REQUIRE(lq_delta_scan_least(heads) <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
+               "delta_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", lq_delta_scan_least(heads),
+               scratch_floats);
     return lq_delta_chunks(q, ldq, k, ldk, v, ldv, beta, ldbeta, a, lda, dt_bias, a_log, state, out, ldo, heads, kv_heads,
-                           Dk, P, seq_slot, cu_rows, batch, rows, channel_decay, scratch, stream);
+                           Dk, P, seq_slot, cu_rows, batch, rows, channel_decay, scratch, scratch_floats, stream);
   }
   dim3 grid((unsigned)(batch * heads), lq_ceil_div(P, cfg.cols));
   ScanShape sh = {heads, kv_heads, P, Dk, seq_slot, cu_rows};

@@ -1121,7 +1121,8 @@ class HipKernels:
 
     @query
     def delta_scan_workspace(self, rows: int, batch: int, heads: int, key_dim: int, value_dim: int, max_rows: int) -> int:
-        """Float32 entries of scratch with which `delta_scan` runs in chunks of tokens (0: token by token)."""
+        """Float32 entries of scratch with which `delta_scan` runs in chunks of tokens (0: token by token), at most some
+        256 MB: with less it takes them in more rounds, down to a chunk a round."""
         self.lib.lq_delta_scan_workspace.restype = c_longlong
         return int(self.lib.lq_delta_scan_workspace(c_int(rows), c_int(batch), c_int(heads), c_int(key_dim),
                                                     c_int(value_dim), c_int(max_rows)))

@@ -74,3 +74,36 @@ def test_what_is_no_number_reaches_later_tokens_only(what, at, channel):
         assert torch.equal(chunked[:at], got["plain", True][0][:at])
         assert torch.equal(torch.isfinite(walked), torch.isfinite(chunked))
         assert torch.equal(torch.isfinite(end0), torch.isfinite(end1))
+
+
+@pytest.mark.parametrize("lens", [[300], [65, 1, 130, 64, 70]])
+@pytest.mark.parametrize("chunks", [1, 2, 3])
+def test_rounds_of_chunks_make_the_same_bits(lens, chunks):
+    """A workspace of fewer chunks than the step has: the chunks go in rounds, from state to state."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(chunks)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, batch, H, G, N, P = sum(lens), len(lens), 4, 2, 64, 80
+    q, k, v, beta, a = rand(rows, G * N), rand(rows, G * N), rand(rows, H * P), rand(rows, H), rand(rows, H * N)
+    dt_bias, a_log, state = rand(H * N) - 3.0, 0.5 * rand(H) + 1.0, rand(batch, H, P, N)
+    kn = HipKernels()
+    need = kn.delta_scan_workspace(rows, batch, H, N, P, max(lens))
+    a_chunk = need // (rows // 64 + batch)
+    got = []
+    for floats in (need, chunks * a_chunk):
+        out, end = torch.full((rows, H * P), float("nan"), device="cuda"), state.clone()
+        kn.delta_scan(q.clone(), k.clone(), v, beta, a, dt_bias, a_log, end, out, H, G, N, P, N ** -0.5, 1e-6, i32(range(batch)),
+                      i32(sum(lens[:b]) for b in range(batch + 1)), batch, channel_decay=True, max_rows=max(lens),
+                      workspace=torch.full((floats,), float("nan"), device="cuda"))
+        got.append((out, end))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+def test_scratch_is_bounded():
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    for rows, batch, heads in ((65536, 1, 16), (8192, 64, 32), (1 << 20, 4, 128)):
+        assert 0 < kn.delta_scan_workspace(rows, batch, heads, 128, 128, rows // batch) <= 64 << 20
