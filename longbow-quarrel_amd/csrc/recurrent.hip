@@ -1248,7 +1248,8 @@ long long lq_ssd_chunks_floats(int rows, int batch, int heads, int P, int N, int
 int lq_ssd_chunks(const float* x, int ldx, const float* B, int ldb, const float* C, int ldc, const float* dt, int lddt,
                   const float* dt_bias, const float* a_log, const float* d_skip, float* state, float* y, int ldy, int heads,
                   int P, int N, int groups, const int* seq_slot, const int* cu_rows, int batch, int rows, float* scratch,
-                  const float* decay, int lddecay, int ones, hipStream_t stream);
+                  long long scratch_floats, const float* decay, int lddecay, int ones, hipStream_t stream);
+long long lq_ssd_chunks_least(int heads, int P, int N);
 
 // `rows` > 0: of a launch in chunks, where it can be one; else of a launch in segments.
 extern "C" long long lq_ssd_scan_workspace(int batch, int heads, int P, int N, int max_rows, int rows) {
@@ -1259,7 +1260,8 @@ extern "C" long long lq_ssd_scan_workspace(int batch, int heads, int P, int N, i
 
 // x [rows, heads * P], B and C [rows, groups * N], dt [rows, heads] (before its softplus), state
 // [slots, heads, P, N], y [rows, heads * P]; rows lie sequence by sequence (cu_rows).  `max_rows`: the most rows a
-// sequence brings (0: unknown); `scratch`: lq_ssd_scan_workspace(...) floats, or null (then no segments).
+// sequence brings (0: unknown); `scratch`: lq_ssd_scan_workspace(...) floats, or null (then no segments; a launch in chunks
+// takes fewer too, down to lq_ssd_chunks_least(...), in more rounds).
 // `decay` [rows, heads] (or null): a token's decay and step are given, S <- decay S + dt B x^T, y = S^T C; dt_bias, a_log
 // and d_skip are then null.  `rows` > 0: the step's rows, and the launch may run in chunks.  `ones`: x is [rows, heads * (P - 1)], and a head's last column has the input one.
 extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, const float* Cm, int ldc, const float* dt,
@@ -1276,10 +1278,11 @@ extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, co
   LQ_REQUIRE(decay != nullptr || (dt_bias && a_log && d_skip), "ssd_scan: neither decays nor what makes them");
   const long long chunks = scratch != nullptr ? lq_ssd_chunks_floats(rows, batch, heads, P, N, max_rows) : 0;
   if (chunks > 0) {
-    LQ_REQUIRE(chunks <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
-               "ssd_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", chunks, scratch_floats);
+    const long long least = lq_ssd_chunks_least(heads, P, N);
+    LQ_REQUIRE(least <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
+               "ssd_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", least, scratch_floats);
     return lq_ssd_chunks(x, ldx, Bm, ldb, Cm, ldc, dt, lddt, dt_bias, a_log, d_skip, state, y, ldy, heads, P, N, groups,
-                         seq_slot, cu_rows, batch, rows, scratch, decay, lddecay, ones, stream);
+                         seq_slot, cu_rows, batch, rows, scratch, scratch_floats, decay, lddecay, ones, stream);
   }
   const long long need = scratch != nullptr ? ssd_segment_floats(batch, heads, P, N, max_rows) : 0;
   ScanLaunch cfg;

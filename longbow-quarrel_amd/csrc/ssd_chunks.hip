@@ -30,6 +30,7 @@ struct SsdArgs {
   float *state, *y, *scratch, *ends;  // scratch: [chunk][head][state]; ends: [chunk][head], p_64
   int heads, groups, N, P, ones, batch;
   const int *seq_slot, *cu_rows;
+  int first, last;  // the chunks of these three launches: numbers first .. last - 1, the scratch of `first` at its start
 };
 
 __host__ __device__ inline int n_tiles(int N) { return (N + HALF - 1) / HALF * NT; }
@@ -121,7 +122,7 @@ template <bool QUADS>
 __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(SsdArgs a) {
   __shared__ __attribute__((aligned(16))) float Bs[CHUNK][LDN], Xs[CHUNK][LDX];
   __shared__ float weight[CHUNK];
-  const int2 at = find_chunk(a.cu_rows, a.batch, blockIdx.x);
+  const int2 at = find_chunk(a.cu_rows, a.batch, a.first + blockIdx.x);
   if (at.x < 0) return;
   const int h = blockIdx.y, grp = h / (a.heads / a.groups), p0 = blockIdx.z * COLS, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, Px = a.P - a.ones;
@@ -194,8 +195,9 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(SsdArgs a) {
 // a (sequence, head)'s state; four chunks' loads are asked for together.
 __global__ __launch_bounds__(256) void ssd_chunk_chain_kernel(SsdArgs a) {
   const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads, tiles_p = p_tiles(a.P);
-  const int chunks = (a.cu_rows[b + 1] - a.cu_rows[b] + CHUNK - 1) / CHUNK;
-  const long long part = part_floats(a.N, a.P), place = (long long)first_chunk(a.cu_rows, b) * a.heads + h;
+  const int base = first_chunk(a.cu_rows, b), i0 = max(a.first - base, 0);
+  const int chunks = min((a.cu_rows[b + 1] - a.cu_rows[b] + CHUNK - 1) / CHUNK, a.last - base) - i0;  // from the sequence's i0th on
+  const long long part = part_floats(a.N, a.P), place = (long long)(base + i0 - a.first) * a.heads + h;
   const long long quad = (long long)blockIdx.y * 256 + threadIdx.x;
   if (chunks <= 0 || quad * 4 >= part) return;
   const int tile = (int)(quad / 64), lane = (int)(quad % 64);
@@ -207,18 +209,18 @@ __global__ __launch_bounds__(256) void ssd_chunk_chain_kernel(SsdArgs a) {
   const long long step = (long long)a.heads * part;
   float* at = a.scratch + place * part + quad * 4;
   const float* ends = a.ends + place;
-  for (int i0 = 0; i0 < chunks; i0 += 4) {
+  for (int done = 0; done < chunks; done += 4) {
     f32x4 add[4];
     float d[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int i = min(i0 + j, chunks - 1);
+      const int i = min(done + j, chunks - 1);
       add[j] = *(const f32x4*)(at + i * step), d[j] = ends[(long long)i * a.heads];
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (i0 + j < chunks) {
-        *(f32x4*)(at + (i0 + j) * step) = S;
+      if (done + j < chunks) {
+        *(f32x4*)(at + (done + j) * step) = S;
         S = S * d[j] + add[j];
       }
   }
@@ -240,7 +242,7 @@ template <bool QUADS>
 __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   OutLds& L = *(OutLds*)smem;
-  const int2 at = find_chunk(a.cu_rows, a.batch, blockIdx.x);
+  const int2 at = find_chunk(a.cu_rows, a.batch, a.first + blockIdx.x);
   if (at.x < 0) return;
   const int h = blockIdx.y, grp = h / (a.heads / a.groups), p0 = blockIdx.z * COLS, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, Px = a.P - a.ones, pt = w & 3, m0 = w >> 2 << 1;  // token tiles m0 and m0 + 1
@@ -384,19 +386,29 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
 // results (of its state 1.2e-7 and 1.1e-7).
 constexpr int LQ_SSD_MIN = 128;
 
+// A launch of more chunks than the scratch holds goes in rounds of equal numbers of them, each from the state that the
+// last one left: a prompt's scratch is bounded (a matrix memory of 4 heads of 256 x 513 takes 2.2 MB a chunk).
+// Microseconds in one round and with 256, 128 and 64 MB: 32 heads of 128 x 64, 32 768 tokens (538 MB) 1 476, 1 577,
+// 1 537, 1 690; the memory, 8 192 tokens (279 MB) 610, 615, 643, 675, sixteen sequences of 512 (311 MB) 626, 664, 671, 811.
+constexpr long long LQ_SSD_SCRATCH = 64ll << 20;  // floats
+
+long long lq_ssd_chunks_least(int heads, int P, int N) { return heads * (part_floats(N, P) + 1); }  // of one chunk
+
 long long lq_ssd_chunks_floats(int rows, int batch, int heads, int P, int N, int max_rows) {
   if (rows <= 0 || N > 2 * HALF || max_rows < LQ_SSD_MIN || heads > 65535 || lq_ceil_div(P, COLS) > 65535) return 0;
-  return (long long)(rows / CHUNK + batch) * heads * (part_floats(N, P) + 1);
+  const long long a_chunk = lq_ssd_chunks_least(heads, P, N), most = LQ_SSD_SCRATCH / a_chunk, all = rows / CHUNK + (long long)batch;
+  return a_chunk * (all <= most ? all : most > 1 ? most : 1);
 }
 
-// -> 0, or -2.  `scratch`: lq_ssd_chunks_floats(...) floats
+// -> 0, or -2.  `scratch`: lq_ssd_chunks_floats(...) floats, or fewer, down to lq_ssd_chunks_least(...)
 int lq_ssd_chunks(const float* x, int ldx, const float* B, int ldb, const float* C, int ldc, const float* dt, int lddt,
                   const float* dt_bias, const float* a_log, const float* d_skip, float* state, float* y, int ldy, int heads,
                   int P, int N, int groups, const int* seq_slot, const int* cu_rows, int batch, int rows, float* scratch,
-                  const float* decay, int lddecay, int ones, hipStream_t stream) {
-  const int chunks = rows / CHUNK + batch;
+                  long long scratch_floats, const float* decay, int lddecay, int ones, hipStream_t stream) {
+  const long long all = rows / CHUNK + (long long)batch, fit = scratch_floats / lq_ssd_chunks_least(heads, P, N);
+  const long long rounds = (all + fit - 1) / fit, room = (all + rounds - 1) / rounds;
   SsdArgs a = {x, B, C, dt, dt_bias, a_log, d_skip, decay, ldx, ldb, ldc, lddt, lddecay, ldy, state, y, scratch,
-               scratch + (long long)chunks * heads * part_floats(N, P), heads, groups, N, P, ones, batch, seq_slot, cu_rows};
+               scratch + room * heads * part_floats(N, P), heads, groups, N, P, ones, batch, seq_slot, cu_rows, 0, 0};
   const bool quads = N % 4 == 0 && (P - ones) % 4 == 0 && ldx % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
                      (((uintptr_t)x | (uintptr_t)B | (uintptr_t)C) & 15) == 0;
   const auto state_kernel = quads ? ssd_chunk_state_kernel<true> : ssd_chunk_state_kernel<false>;
@@ -410,12 +422,15 @@ int lq_ssd_chunks(const float* x, int ldx, const float* B, int ldb, const float*
     }
     configured[quads] = true;
   }
-  const dim3 grid(chunks, heads, lq_ceil_div(P, COLS));
-  state_kernel<<<grid, 256, 0, stream>>>(a);
-  LQ_CHECK_LAUNCH("ssd_scan(chunks' states)");
-  ssd_chunk_chain_kernel<<<dim3((unsigned)batch * heads, (unsigned)lq_ceil_div64(part_floats(N, P), 1024)), 256, 0, stream>>>(a);
-  LQ_CHECK_LAUNCH("ssd_scan(chunks in a chain)");
-  out_kernel<<<grid, 512, sizeof(OutLds), stream>>>(a);
-  LQ_CHECK_LAUNCH("ssd_scan(chunks' results)");
+  for (long long first = 0; first < all; first += room) {
+    a.first = (int)first, a.last = (int)(first + room < all ? first + room : all);
+    const dim3 grid(a.last - a.first, heads, lq_ceil_div(P, COLS));
+    state_kernel<<<grid, 256, 0, stream>>>(a);
+    LQ_CHECK_LAUNCH("ssd_scan(chunks' states)");
+    ssd_chunk_chain_kernel<<<dim3((unsigned)batch * heads, (unsigned)lq_ceil_div64(part_floats(N, P), 1024)), 256, 0, stream>>>(a);
+    LQ_CHECK_LAUNCH("ssd_scan(chunks in a chain)");
+    out_kernel<<<grid, 512, sizeof(OutLds), stream>>>(a);
+    LQ_CHECK_LAUNCH("ssd_scan(chunks' results)");
+  }
   return 0;
 }

@@ -986,7 +986,8 @@ class HipKernels:
     @query
     def ssd_scan_workspace(self, batch: int, heads: int, head_dim: int, n_state: int, max_rows: int, rows: int = 0) -> int:
         """Float32 entries of scratch with which `ssd_scan` runs this launch in segments, or with `rows` (the step's) in
-        chunks where it can (0: it does neither)."""
+        chunks where it can (0: it does neither); of chunks at most some 256 MB: with less it takes them in more rounds,
+        down to a chunk a round."""
         self.lib.lq_ssd_scan_workspace.restype = c_longlong
         return int(self.lib.lq_ssd_scan_workspace(c_int(batch), c_int(heads), c_int(head_dim), c_int(n_state),
                                                   c_int(max_rows), c_int(rows)))

@@ -78,3 +78,35 @@ def test_what_is_no_number_reaches_later_tokens_only(what, at, given):
         assert torch.equal(chunked[:at], got["plain", True][0][:at])
         assert torch.equal(torch.isfinite(walked), torch.isfinite(chunked))
         assert torch.equal(torch.isfinite(end0), torch.isfinite(end1))
+
+
+@pytest.mark.parametrize("lens", [[300], [65, 1, 130, 64, 70]])
+@pytest.mark.parametrize("chunks", [1, 2, 3])
+def test_rounds_of_chunks_make_the_same_bits(lens, chunks):
+    """A workspace of fewer chunks than the step has: the chunks go in rounds, from state to state."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(chunks)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, batch, H, G, N, P = sum(lens), len(lens), 4, 2, 64, 80
+    x, b, c, dt = rand(rows, H * P), 0.3 * rand(rows, G * N), 0.3 * rand(rows, G * N), rand(rows, H)
+    made, state = (rand(H) - 3.0, 0.5 * rand(H) + 1.0, rand(H)), rand(batch, H, P, N)
+    kn = HipKernels()
+    need = kn.ssd_scan_workspace(batch, H, P, N, max(lens), rows)
+    a_chunk = need // (rows // 64 + batch)
+    got = []
+    for floats in (need, chunks * a_chunk):
+        y, end = torch.full((rows, H * P), float("nan"), device="cuda"), state.clone()
+        kn.ssd_scan(x, b, c, dt, *made, end, y, H, P, N, G, i32(range(batch)), i32(sum(lens[:i]) for i in range(batch + 1)),
+                    batch, max_rows=max(lens), workspace=torch.full((floats,), float("nan"), device="cuda"), chunks=True)
+        got.append((y, end))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+def test_scratch_is_bounded():
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    for rows, batch, heads, P, N in ((65536, 1, 32, 64, 128), (16384, 8, 4, 513, 256), (1 << 20, 4, 128, 64, 128)):
+        assert 0 < kn.ssd_scan_workspace(batch, heads, P, N, rows // batch, rows) <= 64 << 20
