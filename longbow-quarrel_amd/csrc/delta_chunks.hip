@@ -18,15 +18,14 @@
 // entries (row l % 16, k = 4 (l / 16) .. + 3) at 4 l.
 //
 // Chunks count from a sequence's first row of the step; a last chunk's missing tokens take part as zeros.
+#include <cmath>
 #include <type_traits>
 
 #include "scan_chunks.h"
 
 namespace {
 
-constexpr int CHUNK = 64, SUB = 16, NMAX = 128;  // tokens a chunk and a block of it; key channels (fewer: zeros)
-constexpr int KT = CHUNK / SUB, NT = NMAX / 16;
-constexpr int FRAG = 256;                        // floats a fragment
+constexpr int NMAX = 128, NT = NMAX / 16;  // key channels (fewer: zeros)
 // a (chunk, head)'s part of the scratch, in floats
 constexpr int AT_KEYS = 0, AT_QUERIES = AT_KEYS + KT * NT * FRAG, AT_UPDATE = AT_QUERIES + KT * NT * FRAG,
               AT_T = AT_UPDATE + NT * KT * FRAG, AT_B = AT_T + KT * KT * FRAG, AT_DECAY = AT_B + KT * KT * FRAG,
@@ -38,6 +37,7 @@ struct DeltaArgs {
   float *state, *out, *scratch;
   int heads, kv_heads, N, P, batch, channel_decay;
   const int *seq_slot, *cu_rows;
+  int least;        // sequences of fewer tokens are not taken
   int first, last;  // the chunks of this pair of launches: numbers first .. last - 1, the scratch of `first` at its start
 };
 
@@ -82,39 +82,6 @@ __device__ inline float decay_of(float z, float rate) {
   return expf(rate * (fmaxf(z, 0.f) + fmaf(s * y, p, 2.f * s)));
 }
 
-// The chunks of all sequences are numbered through.  -> the sequence of chunk number t and its number within it (-1:
-// past the last).  Lane i holds sequence i of a run of 64; every wavefront works out the same.
-__device__ inline int2 find_chunk(const int* __restrict__ cu_rows, int batch, int t) {
-  const int lane = threadIdx.x & 63;
-  for (int b0 = 0; b0 < batch; b0 += 64) {
-    const int b = min(b0 + lane, batch - 1);
-    const int mine = b0 + lane < batch ? (cu_rows[b + 1] - cu_rows[b] + CHUNK - 1) / CHUNK : 0;
-    int upto = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int before = __shfl_up(upto, off, 64);
-      if (lane >= off) upto += before;
-    }
-    const unsigned long long past = __ballot(upto > t);
-    if (past) {
-      const int at = __ffsll(past) - 1;
-      return make_int2(__builtin_amdgcn_readfirstlane(b0 + at),
-                       __builtin_amdgcn_readfirstlane(t - __shfl(upto - mine, at, 64)));
-    }
-    t -= __shfl(upto, 63, 64);
-  }
-  return make_int2(-1, -1);
-}
-
-// the number of sequence b's first chunk
-__device__ inline int first_chunk(const int* __restrict__ cu_rows, int b) {
-  int n = 0;
-  for (int i = threadIdx.x & 63; i < b; i += 64) n += (cu_rows[i + 1] - cu_rows[i] + CHUNK - 1) / CHUNK;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-  return __builtin_amdgcn_readfirstlane(n);
-}
-
 constexpr int LD = NMAX + 4;   // floats a row of LDS: neighbouring rows start 4 banks apart
 constexpr int LDT = CHUNK + 4;
 
@@ -135,7 +102,7 @@ template <bool QUADS>
 __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   Prepared& L = *(Prepared*)smem;
-  const int2 at = find_chunk(a.cu_rows, a.batch, a.first + blockIdx.x);
+  const int2 at = find_chunk(a.cu_rows, a.batch, a.least, a.first + blockIdx.x);
   if (at.x < 0) return;
   const int h = blockIdx.y, j = h / (a.heads / a.kv_heads), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const long long r0 = a.cu_rows[at.x] + (long long)at.y * CHUNK;
@@ -343,8 +310,8 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   const int c = lane & 15, g = lane >> 4, p = blockIdx.y * 16 + c, mt = w & 3;
   const bool second = w >= KT;  // Q~, B and the results
   const long long r1 = a.cu_rows[b + 1];
-  const int base = first_chunk(a.cu_rows, b), i0 = max(a.first - base, 0);
-  const int chunks = min((int)((r1 - a.cu_rows[b] + CHUNK - 1) / CHUNK), a.last - base) - i0;  // from the sequence's i0th on
+  const int base = first_chunk(a.cu_rows, b, a.least), i0 = max(a.first - base, 0);
+  const int chunks = min(chunks_of((int)(r1 - a.cu_rows[b]), a.least), a.last - base) - i0;  // from the sequence's i0th on
   if (chunks <= 0) return;
   const long long r0 = a.cu_rows[b] + (long long)i0 * CHUNK;
   const float* part = a.scratch + ((long long)(base + i0 - a.first) * a.heads + h) * PART;
@@ -469,6 +436,14 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
 // Relative error against 64 bits at 2 048 tokens: 3.3e-7 both ways with a decay every channel, 4.9e-7 and 5.1e-7
 // with one a head; of the state at their end 3.4e-7 and 3.3e-7, 4.5e-7 both.
 constexpr int LQ_DELTA_MIN = 56;
+// A step's sequences of fewer tokens than this walk, beside the longer ones in chunks: a chunk of one token costs as much
+// as one of 64 wherever all chunks together are more than the chip takes at once.  Microseconds, 16 heads of 128 x 128, a
+// decay a channel, token by token / all in chunks / the long ones only: 512 tokens beside 16 of 1 308 / 131 / 106, 2 000
+// beside 70 of 1 1 225 / 460 / 358; a decay a head, 2 000 beside eight of 20 632 / 209 / 187.
+int lq_delta_least_rows(int rows, int batch, int heads, int channel_decay) {
+  return most_chunks(rows, batch, 1) * heads <= lq_compute_units() ? 1 : channel_decay ? 24 : 48;
+}
+extern "C" long long lq_delta_scan_least(int heads);
 // A launch of more chunks than the scratch holds goes in rounds of equal numbers of them, each from the state that the
 // last one left: a prompt's scratch is bounded (131.6 KB a chunk and head: 4.3 GB for 65 536 rows of 16 heads).  Rounds
 // cost where the sequences of one leave the chip idle: 32 heads, four of 2 048 tokens 1 007 us in one round (556 MB), 1 002
@@ -478,10 +453,33 @@ constexpr long long LQ_DELTA_SCRATCH = 64ll << 20;  // floats
 extern "C" long long lq_delta_scan_workspace(int rows, int batch, int heads, int Dk, int P, int max_rows) {
   if (rows <= 0 || batch <= 0 || heads <= 0 || P <= 0 || Dk <= 0 || Dk > NMAX || max_rows < LQ_DELTA_MIN) return 0;
   if (heads > 65535 || lq_ceil_div(P, 16) > 65535) return 0;
-  const long long a_chunk = (long long)heads * PART, most = LQ_DELTA_SCRATCH / a_chunk, all = rows / CHUNK + (long long)batch;
-  return a_chunk * (all <= most ? all : most > 1 ? most : 1);
+  return chunks_scratch(most_chunks(rows, batch, lq_delta_least_rows(rows, batch, heads, 1)), lq_delta_scan_least(heads), LQ_DELTA_SCRATCH);
 }
 extern "C" long long lq_delta_scan_least(int heads) { return (long long)heads * PART; }  // of one chunk
+
+// Whether a launch is faster in chunks (given scratch) than token by token, by what both take.  A chunk costs the same
+// whatever the sizes (their zeros are multiplied too) and however few tokens it has; a walk's token costs little where
+// states are small or one decay serves a head, as soon as there are workgroups for the whole chip.  Microseconds, walk /
+// chunks, 16 heads of 128 x 128: a decay a head, 70 sequences of 64 tokens 306 / 418, of 200 845 / 1 163, 16 of 100
+// 126 / 151, eight of 512 267 / 215, one of 256 89 / 44; a decay a channel, 16 of 64 171 / 112, 70 of 200 2 037 / 1 249;
+// of 64 x 64, 16 of 128 74 / 107.
+extern "C" int lq_delta_scan_in_chunks(int rows, int batch, int heads, int Dk, int P, int max_rows, int channel_decay) {
+  if (lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) == 0) return 0;
+  const double size = P / 128.0 * (Dk > 64 ? Dk / 128.0 : 0.4), cols = (P + 15) / 16;
+  const double latency = channel_decay ? 0.42 : 0.31, token = (channel_decay ? 8.5e-3 : 3.7e-3) * size * heads;
+  const double state = (channel_decay ? 0.12 : 0.045) * size * heads;  // a sequence's state, read and written
+  auto walk = [&](double n, double longest, double sequences) {
+    return 10 + sqrt(token * n * token * n + latency * longest * latency * longest) + state * sequences;
+  };
+  // the sequences beside the longest, by their mean, go in chunks as it does or all token by token
+  const double rest = rows - max_rows, least = lq_delta_least_rows(rows, batch, heads, channel_decay);
+  const bool alike = batch == 1 || rest >= least * (batch - 1);
+  const double in_chunks = alike ? batch : 1, of_chunks = (alike ? rows : max_rows) / 64.0 + in_chunks / 2;
+  const double products = 0.0145 * cols * heads * of_chunks, chain = 3.3 * (max_rows / 64 + 1);
+  double chunks = 25 + 0.085 * heads * of_chunks + (products > chain ? products : chain) + 0.15 * P / 128 * heads * in_chunks;
+  if (!alike) chunks += 20 + walk(rest, least, batch - 1);
+  return 0.9 * chunks < walk(rows, max_rows, batch);
+}
 
 // q and k hold unit vectors already.  `scratch`: at least a chunk's floats for every head.  -> 0, or -2
 int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* beta,
@@ -489,7 +487,7 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
                     int ldo, int heads, int kv_heads, int Dk, int P, const int* seq_slot, const int* cu_rows, int batch,
                     int rows, int channel_decay, float* scratch, long long scratch_floats, hipStream_t stream) {
   DeltaArgs d = {q, k, v, beta, a, dt_bias, a_log, ldq, ldk, ldv, ldbeta, lda, ldo, state, out, scratch,
-                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows, 0, 0};
+                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows, lq_delta_least_rows(rows, batch, heads, channel_decay), 0, 0};
   const bool quads = Dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && (!channel_decay || lda % 4 == 0) &&
                      (((uintptr_t)q | (uintptr_t)k | (channel_decay ? (uintptr_t)a | (uintptr_t)dt_bias : 0)) & 15) == 0;
   const auto prepare = quads ? delta_prepare_kernel<true> : delta_prepare_kernel<false>;
@@ -502,8 +500,7 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
     }
     configured[quads] = true;
   }
-  const long long all = rows / CHUNK + (long long)batch, fit = scratch_floats / ((long long)heads * PART);
-  const long long rounds = (all + fit - 1) / fit, room = (all + rounds - 1) / rounds;
+  const long long all = most_chunks(rows, batch, d.least), room = chunks_a_round(all, scratch_floats, lq_delta_scan_least(heads));
   for (long long first = 0; first < all; first += room) {
     d.first = (int)first, d.last = (int)(first + room < all ? first + room : all);
     prepare<<<dim3(d.last - d.first, heads), 512, sizeof(Prepared), stream>>>(d);

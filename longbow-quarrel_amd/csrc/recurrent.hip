@@ -240,6 +240,7 @@ struct ScanShape {
   // made of a logit; `ones`: the head's last column is not in x ([rows, heads * (P - 1)]), its input is one
   const float* decay = nullptr;
   int lddecay = 0, ones = 0;
+  int below = 0x7fffffff;  // sequences of so many tokens or more are left out: they go in chunks
 };
 
 // The chunk-wise staging that both scans share.  `a`, `b`: the two shared rows of a token ([rows, groups * N] each),
@@ -475,6 +476,7 @@ __global__ __launch_bounds__(TH) void delta_scan_kernel(const float* __restrict_
   const bool live = p < P;
   const int slab = (N + LN - 1) / LN;
   const long long r0 = sh.cu_rows[b], r1 = sh.cu_rows[b + 1];
+  if (r1 - r0 >= sh.below) return;
   float* sp = state + (((long long)sh.seq_slot[b] * heads + h) * P + (live ? p : 0)) * N;
   constexpr int NP = LN * SLAB;  // a shared row in LDS, padded with zeros: entries past N take part as zeros
   const int buf_floats = TT * (2 * NP + 2 * cols + 2);  // shared rows, inputs, decay and step, outputs
@@ -834,6 +836,7 @@ __global__ __launch_bounds__(TH) void delta_channel_scan_kernel(const float* __r
   const int tid = threadIdx.x, l = tid % LN, col = tid / LN, p0 = blockIdx.y * cols, p = p0 + col;
   const bool live = p < P;
   const long long r0 = sh.cu_rows[b], r1 = sh.cu_rows[b + 1];
+  if (r1 - r0 >= sh.below) return;
   float* sp = state + (((long long)sh.seq_slot[b] * heads + h) * P + (live ? p : 0)) * N;
   float S[SLAB];
 #pragma unroll
@@ -1321,9 +1324,10 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
                     int ldo, int heads, int kv_heads, int Dk, int P, const int* seq_slot, const int* cu_rows, int batch,
                     int rows, int channel_decay, float* scratch, long long scratch_floats, hipStream_t stream);
 extern "C" long long lq_delta_scan_least(int heads);
+int lq_delta_least_rows(int rows, int batch, int heads, int channel_decay);
 
 // q and k [rows, kv_heads * Dk], v [rows, heads * P], beta and a [rows, heads] (raw), state [slots, heads, P, Dk],
-// out [rows, heads * P]; `max_rows`: the most rows a sequence brings (0: unknown); `scratch`:
+// out [rows, heads * P]; `max_rows`: the most rows that a sequence brings (0: unknown); `scratch`:
 // lq_delta_scan_workspace(...) floats for a launch in chunks, or null (fewer make more rounds, down to
 // lq_delta_scan_least(heads))
 // (q and k are made unit vectors in place)
@@ -1342,16 +1346,20 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
   LQ_REQUIRE(rows > 0 && rows <= 0x7fffffff && kv_heads <= 65535, "delta_scan: %d rows, %d q/k heads", rows, kv_heads);
   unit_heads_kernel<<<dim3((unsigned)rows, kv_heads), 64, 0, stream>>>(q, ldq, k, ldk, Dk, q_scale, unit_eps);
   LQ_CHECK_LAUNCH("delta_scan(unit vectors)");
+  int below = 0x7fffffff;  // what is walked token by token
   const long long need = scratch != nullptr ? lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) : 0;
   if (need > 0) {
     LQ_REQUIRE(lq_delta_scan_least(heads) <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
                "delta_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", lq_delta_scan_least(heads),
                scratch_floats);
-    return lq_delta_chunks(q, ldq, k, ldk, v, ldv, beta, ldbeta, a, lda, dt_bias, a_log, state, out, ldo, heads, kv_heads,
-                           Dk, P, seq_slot, cu_rows, batch, rows, channel_decay, scratch, scratch_floats, stream);
+    const int rc = lq_delta_chunks(q, ldq, k, ldk, v, ldv, beta, ldbeta, a, lda, dt_bias, a_log, state, out, ldo, heads, kv_heads,
+                                   Dk, P, seq_slot, cu_rows, batch, rows, channel_decay, scratch, scratch_floats, stream);
+    below = lq_delta_least_rows(rows, batch, heads, channel_decay);
+    if (rc != 0 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
   }
   dim3 grid((unsigned)(batch * heads), lq_ceil_div(P, cfg.cols));
   ScanShape sh = {heads, kv_heads, P, Dk, seq_slot, cu_rows};
+  sh.below = below;
   if (channel_decay) {
     const int np = cfg.ln * cfg.slab;
     const bool single = rows == batch;  // every sequence brings one token

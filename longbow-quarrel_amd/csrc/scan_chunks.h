@@ -1,4 +1,5 @@
-// What the scans in chunks of 64 tokens share (delta_chunks.hip, ssd_chunks.hip): products of tiles of 16 x 16 in 32 bits.
+// What the scans in chunks of 64 tokens share (delta_chunks.hip, ssd_chunks.hip): how chunks are numbered, and products of
+// tiles of 16 x 16 in 32 bits.
 #pragma once
 
 #include "device_math.h"
@@ -6,6 +7,45 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
+
+constexpr int CHUNK = 64, SUB = 16, KT = CHUNK / SUB;  // tokens a chunk and a block of it; blocks a chunk
+constexpr int FRAG = 256;                              // floats a tile of 16 x 16
+
+// The chunks of a sequence of n tokens: none for one shorter than `least`, which is walked token by token instead.
+__device__ inline int chunks_of(int n, int least) { return n >= least ? (n + CHUNK - 1) / CHUNK : 0; }
+
+// The chunks of all sequences are numbered through.  -> the sequence of chunk number t and its number within it (-1:
+// past the last).  Lane i holds sequence i of a run of 64; every wavefront works out the same.
+__device__ inline int2 find_chunk(const int* __restrict__ cu_rows, int batch, int least, int t) {
+  const int lane = threadIdx.x & 63;
+  for (int b0 = 0; b0 < batch; b0 += 64) {
+    const int b = min(b0 + lane, batch - 1);
+    const int mine = b0 + lane < batch ? chunks_of(cu_rows[b + 1] - cu_rows[b], least) : 0;
+    int upto = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int before = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += before;
+    }
+    const unsigned long long past = __ballot(upto > t);
+    if (past) {
+      const int at = __ffsll(past) - 1;
+      return make_int2(__builtin_amdgcn_readfirstlane(b0 + at),
+                       __builtin_amdgcn_readfirstlane(t - __shfl(upto - mine, at, 64)));
+    }
+    t -= __shfl(upto, 63, 64);
+  }
+  return make_int2(-1, -1);
+}
+
+// the number of sequence b's first chunk
+__device__ inline int first_chunk(const int* __restrict__ cu_rows, int b, int least) {
+  int n = 0;
+  for (int i = threadIdx.x & 63; i < b; i += 64) n += chunks_of(cu_rows[i + 1] - cu_rows[i], least);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
 
 // c + A . B by v_mfma_f32_16x16x4_f32: lane l gives A[l % 16][4 (l / 16) .. + 3] and B[4 (l / 16) .. + 3][l % 16] and
 // receives D[4 (l / 16) + e][l % 16].
@@ -41,6 +81,23 @@ __device__ inline f32x4 step4_lower(const f32x4& a, const f32x4& b, f32x4 c) {
 // NaN once a tile has had an entry that is no finite number (from 0 on).
 __device__ inline float not_finite(const f32x4& b, float so_far) {
   return fmaf(b[0], 0.f, fmaf(b[1], 0.f, fmaf(b[2], 0.f, fmaf(b[3], 0.f, so_far))));
+}
+
+// The most chunks that `rows` tokens of `batch` sequences can have.
+inline long long most_chunks(int rows, int batch, int least) {
+  return rows / CHUNK + (long long)(rows / least < batch ? rows / least : batch);
+}
+
+// A launch's chunks in rounds of equal numbers, each within the scratch.
+inline long long chunks_a_round(long long all, long long scratch_floats, long long a_chunk) {
+  const long long fit = scratch_floats / a_chunk, rounds = (all + fit - 1) / fit;
+  return (all + rounds - 1) / rounds;
+}
+
+// The floats that a launch asks for: its chunks', or as many as `bound` floats hold, or one chunk's.
+inline long long chunks_scratch(long long all, long long a_chunk, long long bound) {
+  const long long most = bound / a_chunk > 1 ? bound / a_chunk : 1;
+  return a_chunk * (all < most ? all : most);
 }
 
 }  // namespace

@@ -19,10 +19,8 @@
 
 namespace {
 
-constexpr int CHUNK = 64, SUB = 16, KT = CHUNK / SUB;
 constexpr int HALF = 128, NT = HALF / 16;  // channels that a workgroup holds in LDS at a time
 constexpr int COLS = 64;                   // columns of the values a workgroup
-constexpr int FRAG = 256;                  // floats a tile
 
 struct SsdArgs {
   const float *x, *B, *C, *dt, *dt_bias, *a_log, *d_skip, *decay;
@@ -30,44 +28,13 @@ struct SsdArgs {
   float *state, *y, *scratch, *ends;  // scratch: [chunk][head][state]; ends: [chunk][head], p_64
   int heads, groups, N, P, ones, batch;
   const int *seq_slot, *cu_rows;
+  int least;        // sequences of fewer tokens are not taken
   int first, last;  // the chunks of these three launches: numbers first .. last - 1, the scratch of `first` at its start
 };
 
 __host__ __device__ inline int n_tiles(int N) { return (N + HALF - 1) / HALF * NT; }
 __host__ __device__ inline int p_tiles(int P) { return (P + 15) / 16; }
 __host__ __device__ inline long long part_floats(int N, int P) { return (long long)n_tiles(N) * p_tiles(P) * FRAG; }
-
-// The chunks of all sequences are numbered through.  -> the sequence of chunk number t and its number within it (-1:
-// past the last).  Lane i holds sequence i of a run of 64; every wavefront works out the same.
-__device__ inline int2 find_chunk(const int* __restrict__ cu_rows, int batch, int t) {
-  const int lane = threadIdx.x & 63;
-  for (int b0 = 0; b0 < batch; b0 += 64) {
-    const int b = min(b0 + lane, batch - 1);
-    const int mine = b0 + lane < batch ? (cu_rows[b + 1] - cu_rows[b] + CHUNK - 1) / CHUNK : 0;
-    int upto = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int before = __shfl_up(upto, off, 64);
-      if (lane >= off) upto += before;
-    }
-    const unsigned long long past = __ballot(upto > t);
-    if (past) {
-      const int at = __ffsll(past) - 1;
-      return make_int2(__builtin_amdgcn_readfirstlane(b0 + at),
-                       __builtin_amdgcn_readfirstlane(t - __shfl(upto - mine, at, 64)));
-    }
-    t -= __shfl(upto, 63, 64);
-  }
-  return make_int2(-1, -1);
-}
-
-__device__ inline int first_chunk(const int* __restrict__ cu_rows, int b) {
-  int n = 0;
-  for (int i = threadIdx.x & 63; i < b; i += 64) n += (cu_rows[i + 1] - cu_rows[i] + CHUNK - 1) / CHUNK;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-  return __builtin_amdgcn_readfirstlane(n);
-}
 
 // A token's decay and step (one thread a token; past the portion's end: nothing decays and nothing is added).
 __device__ inline void token_scalars(const SsdArgs& a, long long row, bool there, int h, float& decay, float& step) {
@@ -122,7 +89,7 @@ template <bool QUADS>
 __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(SsdArgs a) {
   __shared__ __attribute__((aligned(16))) float Bs[CHUNK][LDN], Xs[CHUNK][LDX];
   __shared__ float weight[CHUNK];
-  const int2 at = find_chunk(a.cu_rows, a.batch, a.first + blockIdx.x);
+  const int2 at = find_chunk(a.cu_rows, a.batch, a.least, a.first + blockIdx.x);
   if (at.x < 0) return;
   const int h = blockIdx.y, grp = h / (a.heads / a.groups), p0 = blockIdx.z * COLS, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, Px = a.P - a.ones;
@@ -195,8 +162,8 @@ __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(SsdArgs a) {
 // a (sequence, head)'s state; four chunks' loads are asked for together.
 __global__ __launch_bounds__(256) void ssd_chunk_chain_kernel(SsdArgs a) {
   const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads, tiles_p = p_tiles(a.P);
-  const int base = first_chunk(a.cu_rows, b), i0 = max(a.first - base, 0);
-  const int chunks = min((a.cu_rows[b + 1] - a.cu_rows[b] + CHUNK - 1) / CHUNK, a.last - base) - i0;  // from the sequence's i0th on
+  const int base = first_chunk(a.cu_rows, b, a.least), i0 = max(a.first - base, 0);
+  const int chunks = min(chunks_of(a.cu_rows[b + 1] - a.cu_rows[b], a.least), a.last - base) - i0;  // from the sequence's i0th on
   const long long part = part_floats(a.N, a.P), place = (long long)(base + i0 - a.first) * a.heads + h;
   const long long quad = (long long)blockIdx.y * 256 + threadIdx.x;
   if (chunks <= 0 || quad * 4 >= part) return;
@@ -242,7 +209,7 @@ template <bool QUADS>
 __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   OutLds& L = *(OutLds*)smem;
-  const int2 at = find_chunk(a.cu_rows, a.batch, a.first + blockIdx.x);
+  const int2 at = find_chunk(a.cu_rows, a.batch, a.least, a.first + blockIdx.x);
   if (at.x < 0) return;
   const int h = blockIdx.y, grp = h / (a.heads / a.groups), p0 = blockIdx.z * COLS, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, Px = a.P - a.ones, pt = w & 3, m0 = w >> 2 << 1;  // token tiles m0 and m0 + 1
@@ -385,6 +352,7 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
 // against 64 bits: 5.9e-8 and 4.7e-8 at 2 048 tokens (of the state 4.8e-7 and 4.4e-7), 1.4e-7 and 1.7e-7 of the memory's
 // results (of its state 1.2e-7 and 1.1e-7).
 constexpr int LQ_SSD_MIN = 128;
+constexpr int LQ_SSD_LEAST = 1;
 
 // A launch of more chunks than the scratch holds goes in rounds of equal numbers of them, each from the state that the
 // last one left: a prompt's scratch is bounded (a matrix memory of 4 heads of 256 x 513 takes 2.2 MB a chunk).
@@ -396,8 +364,7 @@ long long lq_ssd_chunks_least(int heads, int P, int N) { return heads * (part_fl
 
 long long lq_ssd_chunks_floats(int rows, int batch, int heads, int P, int N, int max_rows) {
   if (rows <= 0 || N > 2 * HALF || max_rows < LQ_SSD_MIN || heads > 65535 || lq_ceil_div(P, COLS) > 65535) return 0;
-  const long long a_chunk = lq_ssd_chunks_least(heads, P, N), most = LQ_SSD_SCRATCH / a_chunk, all = rows / CHUNK + (long long)batch;
-  return a_chunk * (all <= most ? all : most > 1 ? most : 1);
+  return chunks_scratch(most_chunks(rows, batch, LQ_SSD_LEAST), lq_ssd_chunks_least(heads, P, N), LQ_SSD_SCRATCH);
 }
 
 // -> 0, or -2.  `scratch`: lq_ssd_chunks_floats(...) floats, or fewer, down to lq_ssd_chunks_least(...)
@@ -405,10 +372,10 @@ int lq_ssd_chunks(const float* x, int ldx, const float* B, int ldb, const float*
                   const float* dt_bias, const float* a_log, const float* d_skip, float* state, float* y, int ldy, int heads,
                   int P, int N, int groups, const int* seq_slot, const int* cu_rows, int batch, int rows, float* scratch,
                   long long scratch_floats, const float* decay, int lddecay, int ones, hipStream_t stream) {
-  const long long all = rows / CHUNK + (long long)batch, fit = scratch_floats / lq_ssd_chunks_least(heads, P, N);
-  const long long rounds = (all + fit - 1) / fit, room = (all + rounds - 1) / rounds;
+  const long long all = most_chunks(rows, batch, LQ_SSD_LEAST);
+  const long long room = chunks_a_round(all, scratch_floats, lq_ssd_chunks_least(heads, P, N));
   SsdArgs a = {x, B, C, dt, dt_bias, a_log, d_skip, decay, ldx, ldb, ldc, lddt, lddecay, ldy, state, y, scratch,
-               scratch + room * heads * part_floats(N, P), heads, groups, N, P, ones, batch, seq_slot, cu_rows, 0, 0};
+               scratch + room * heads * part_floats(N, P), heads, groups, N, P, ones, batch, seq_slot, cu_rows, LQ_SSD_LEAST, 0, 0};
   const bool quads = N % 4 == 0 && (P - ones) % 4 == 0 && ldx % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
                      (((uintptr_t)x | (uintptr_t)B | (uintptr_t)C) & 15) == 0;
   const auto state_kernel = quads ? ssd_chunk_state_kernel<true> : ssd_chunk_state_kernel<false>;

@@ -1128,6 +1128,13 @@ class HipKernels:
         return int(self.lib.lq_delta_scan_workspace(c_int(rows), c_int(batch), c_int(heads), c_int(key_dim),
                                                     c_int(value_dim), c_int(max_rows)))
 
+    @query
+    def delta_scan_in_chunks(self, rows: int, batch: int, heads: int, key_dim: int, value_dim: int, max_rows: int,
+                             channel_decay: bool) -> bool:
+        """Whether `delta_scan` is faster in chunks of tokens than token by token, for these sizes."""
+        return bool(self.lib.lq_delta_scan_in_chunks(c_int(rows), c_int(batch), c_int(heads), c_int(key_dim), c_int(value_dim),
+                                                     c_int(max_rows), c_int(1 if channel_decay else 0)))
+
     def delta_scan(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, a: torch.Tensor,
                    dt_bias: torch.Tensor, a_log: torch.Tensor, state: torch.Tensor, out: torch.Tensor, heads: int,
                    kv_heads: int, key_dim: int, value_dim: int, q_scale: float, unit_eps: float,
@@ -1139,8 +1146,8 @@ class HipKernels:
         value_dim, key_dim].  All float32.  q and k are overwritten with their unit vectors.  The decay is one number
         a head (a [rows, heads], dt_bias [heads]) or, with `channel_decay`, one for every key channel of every head
         (a [rows, heads * key_dim], dt_bias [heads * key_dim]), multiplying the state's rows of that channel.
-        `max_rows` (the most rows a sequence brings) and `workspace` (`delta_scan_workspace(...)` floats) let long
-        portions run in chunks of tokens, whose sums are in another order."""
+        `max_rows` (the most rows that a sequence brings) and `workspace` (`delta_scan_workspace(...)` floats) let the
+        step's long portions run in chunks of tokens, whose sums are in another order."""
         rows = q.shape[0]
         n_decay = heads * key_dim if channel_decay else heads
         for t, what, cols in ((q, "q", kv_heads * key_dim), (k, "k", kv_heads * key_dim), (v, "v", heads * value_dim),

@@ -423,10 +423,10 @@ class GatedDelta(_Recurrent):
         o = ctx.ws.alloc((rows, self.v_width), torch.float32)
         more = {"channel_decay": True} if self.channel_decay else {}
         # long portions of a bfloat16 run go in chunks, given scratch (a 32-bit run's sums keep their one order)
-        ask = getattr(kn, "delta_scan_workspace", None) if ctx.dtype == torch.bfloat16 else None
-        need = ask(rows, ctx.batch, nh, self.key_dim, self.value_dim, ctx.max_new) if ask is not None else 0
-        if need:
-            more.update(max_rows=ctx.max_new, workspace=ctx.ws.alloc((need,), torch.float32))
+        ask = getattr(kn, "delta_scan_in_chunks", None) if ctx.dtype == torch.bfloat16 else None
+        sizes = (rows, ctx.batch, nh, self.key_dim, self.value_dim, ctx.max_new)
+        if ask is not None and ask(*sizes, self.channel_decay):
+            more.update(max_rows=ctx.max_new, workspace=ctx.ws.alloc((kn.delta_scan_workspace(*sizes),), torch.float32))
         kn.delta_scan(qkv[:, : self.qk_width], qkv[:, self.qk_width : 2 * self.qk_width], qkv[:, 2 * self.qk_width :],
                       u[:, cc : cc + nh], decay, self.dt_bias, self.a_log, state, o, self.heads,
                       self.kv_heads, self.key_dim, self.value_dim, self.key_dim ** -0.5, self.UNIT_EPS,

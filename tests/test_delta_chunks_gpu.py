@@ -107,3 +107,55 @@ def test_scratch_is_bounded():
     kn = HipKernels()
     for rows, batch, heads in ((65536, 1, 16), (8192, 64, 32), (1 << 20, 4, 128)):
         assert 0 < kn.delta_scan_workspace(rows, batch, heads, 128, 128, rows // batch) <= 64 << 20
+
+
+@pytest.mark.parametrize("channel,least", [(True, 24), (False, 48)])
+def test_short_sequences_beside_a_long_one_are_walked(channel, least):
+    """More chunks than the chip takes at once: sequences of fewer than `least` tokens have the bits of the walk token by
+    token, the others those of a launch of their own in chunks."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(least)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    lens = [1, least - 1, 100, least, 64] + [2] * 40 + [least + 1]
+    rows, batch, H, G, N, P = sum(lens), len(lens), 8, 4, 64, 48
+    q, k, v, beta, a = rand(rows, G * N), rand(rows, G * N), rand(rows, H * P), rand(rows, H), rand(rows, H * N if channel else H)
+    dt_bias, a_log, state = rand(a.shape[1]) - 3.0, 0.5 * rand(H) + 1.0, rand(batch, H, P, N)
+    kn = HipKernels()
+
+    all_lens = lens
+
+    def run(first, lens, floats):
+        n, at, B = sum(lens), sum(all_lens[:first]), len(lens)
+        out, end = torch.full((n, H * P), float("nan"), device="cuda"), state[first : first + B].clone()
+        part = lambda x: x[at : at + n].clone()
+        more = dict(max_rows=max(lens), workspace=torch.full((floats,), float("nan"), device="cuda")) if floats else {}
+        kn.delta_scan(part(q), part(k), part(v), part(beta), part(a), dt_bias, a_log, end, out, H, G, N, P, N ** -0.5, 1e-6,
+                      i32(range(B)), i32(sum(lens[:b]) for b in range(B + 1)), B, channel_decay=channel, **more)
+        return out, end
+
+    need = lambda lens: kn.delta_scan_workspace(sum(lens), len(lens), H, N, P, max(lens))
+    (got, got_end), (walked, walked_end) = run(0, lens, need(lens)), run(0, lens, 0)
+    for b, n in enumerate(lens):
+        at = sum(lens[:b])
+        if n < least:
+            assert torch.equal(got[at : at + n], walked[at : at + n]) and torch.equal(got_end[b], walked_end[b])
+        else:
+            far = 64 * 4 * 2.0 ** -24  # (as above: at most some 4 roundings a token, here up to 100 tokens)
+            assert (got[at : at + n] - walked[at : at + n]).abs().max() <= 2 * far * walked.abs().max()
+            if need([n]):  # (a launch of its own is in chunks too)
+                alone, end = run(b, [n], need([n]))
+                assert torch.equal(got[at : at + n], alone) and torch.equal(got_end[b], end[0])
+
+
+def test_which_launches_are_faster_in_chunks():
+    """Sizes far from where both ways take as long: few long sequences in chunks, very many or short ones token by token."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    ask = HipKernels().delta_scan_in_chunks
+    for channel in (False, True):
+        assert ask(256, 1, 16, 128, 128, 256, channel) and ask(8192, 1, 16, 128, 128, 8192, channel) and ask(3990, 70, 16, 128, 128, 2000, channel)
+        assert not ask(16, 1, 16, 128, 128, 16, channel) and not ask(256, 256, 16, 128, 128, 1, channel)
+        assert not ask(70 * 57, 70, 16, 64, 64, 57, channel)
+    assert not ask(70 * 200, 70, 16, 128, 128, 200, False) and ask(70 * 200, 70, 16, 128, 128, 200, True)
