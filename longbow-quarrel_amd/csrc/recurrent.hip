@@ -274,6 +274,7 @@ __global__ __launch_bounds__(TH) void ssd_scan_kernel(const float* __restrict__ 
   const bool live = p < P;
   const int slab = (N + LN - 1) / LN;
   long long r0 = sh.cu_rows[b], r1 = sh.cu_rows[b + 1];
+  if (r1 - r0 >= sh.below) return;
   // A long sequence of a launch in segments (see SegArgs): this workgroup's segment, where it starts from and
   // where it leaves its state.
   const int seg = blockIdx.z;
@@ -1253,12 +1254,19 @@ int lq_ssd_chunks(const float* x, int ldx, const float* B, int ldb, const float*
                   int P, int N, int groups, const int* seq_slot, const int* cu_rows, int batch, int rows, float* scratch,
                   long long scratch_floats, const float* decay, int lddecay, int ones, hipStream_t stream);
 long long lq_ssd_chunks_least(int heads, int P, int N);
+int lq_ssd_least_rows(int rows, int batch, int heads);
+bool lq_ssd_chunks_faster(int batch, int heads, int P, int N, int max_rows, int rows, bool segments);
 
 // `rows` > 0: of a launch in chunks, where it can be one; else of a launch in segments.
 extern "C" long long lq_ssd_scan_workspace(int batch, int heads, int P, int N, int max_rows, int rows) {
   if (batch <= 0 || heads <= 0 || P <= 0 || N <= 0) return 0;
   const long long chunks = lq_ssd_chunks_floats(rows, batch, heads, P, N, max_rows);
   return chunks > 0 ? chunks : ssd_segment_floats(batch, heads, P, N, max_rows);
+}
+
+extern "C" int lq_ssd_scan_in_chunks(int batch, int heads, int P, int N, int max_rows, int rows) {
+  if (batch <= 0 || heads <= 0 || P <= 0 || N <= 0) return 0;
+  return lq_ssd_chunks_faster(batch, heads, P, N, max_rows, rows, ssd_segment_floats(batch, heads, P, N, max_rows) > 0);
 }
 
 // x [rows, heads * P], B and C [rows, groups * N], dt [rows, heads] (before its softplus), state
@@ -1279,15 +1287,18 @@ extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, co
              "ssd_scan: a row stride is smaller than its row");
   LQ_REQUIRE(x && Bm && Cm && dt && state && y && seq_slot && cu_rows, "ssd_scan: null pointer");
   LQ_REQUIRE(decay != nullptr || (dt_bias && a_log && d_skip), "ssd_scan: neither decays nor what makes them");
+  int below = 0x7fffffff;  // what is walked token by token
   const long long chunks = scratch != nullptr ? lq_ssd_chunks_floats(rows, batch, heads, P, N, max_rows) : 0;
   if (chunks > 0) {
     const long long least = lq_ssd_chunks_least(heads, P, N);
     LQ_REQUIRE(least <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
                "ssd_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", least, scratch_floats);
-    return lq_ssd_chunks(x, ldx, Bm, ldb, Cm, ldc, dt, lddt, dt_bias, a_log, d_skip, state, y, ldy, heads, P, N, groups,
+    const int rc = lq_ssd_chunks(x, ldx, Bm, ldb, Cm, ldc, dt, lddt, dt_bias, a_log, d_skip, state, y, ldy, heads, P, N, groups,
                          seq_slot, cu_rows, batch, rows, scratch, scratch_floats, decay, lddecay, ones, stream);
+    below = lq_ssd_least_rows(rows, batch, heads);
+    if (rc != 0 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
   }
-  const long long need = scratch != nullptr ? ssd_segment_floats(batch, heads, P, N, max_rows) : 0;
+  const long long need = scratch != nullptr && chunks == 0 ? ssd_segment_floats(batch, heads, P, N, max_rows) : 0;
   ScanLaunch cfg;
   LQ_REQUIRE(scan_launch(N, P, (long long)batch * heads * (need > 0 ? SEG_COUNT : 1), cfg),
              "ssd_scan: state size %d is too large", N);
@@ -1299,6 +1310,7 @@ extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, co
     sg.decay = scratch + (long long)batch * heads * SEG_COUNT * P * N;
   }
   ScanShape sh = {heads, groups, P, N, seq_slot, cu_rows, decay, lddecay, ones};
+  sh.below = below;
 #define LQ_SSD(LN, SL, TH)                                                                                              \
   ssd_scan_kernel<LN, SL, TH><<<grid, cfg.threads, cfg.lds, stream>>>(x, ldx, Bm, ldb, Cm, ldc, dt, lddt, dt_bias, a_log, \
                                                                   d_skip, state, y, ldy, sh, sg)

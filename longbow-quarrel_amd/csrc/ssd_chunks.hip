@@ -13,6 +13,7 @@
 // scratch lies in tiles of 16 channels n by 16 columns p in a result's order, lane l's four entries (n = 4 (l / 16) .. + 3,
 // p = l % 16) at 4 l, which is also the order in which the third launch takes it as an operand.
 // Chunks count from a sequence's first row of the step; a last chunk's missing tokens take part as zeros.
+#include <cmath>
 #include <type_traits>
 
 #include "scan_chunks.h"
@@ -352,7 +353,11 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
 // against 64 bits: 5.9e-8 and 4.7e-8 at 2 048 tokens (of the state 4.8e-7 and 4.4e-7), 1.4e-7 and 1.7e-7 of the memory's
 // results (of its state 1.2e-7 and 1.1e-7).
 constexpr int LQ_SSD_MIN = 128;
-constexpr int LQ_SSD_LEAST = 1;
+// A step's sequences of fewer tokens than this walk, beside the longer ones in chunks: a chunk of one token costs as much
+// as one of 64 wherever all chunks together are more than the chip takes at once.  Microseconds, 32 heads of 128 x 64, token by token / all in
+// chunks / the long ones only: 512 tokens beside 16 of 1 164 / 94 / 69, 2 000 beside eight of 20 544 / 134 / 129, a memory
+// of 256 x 513, 2 000 beside eight of 1 925 / 207 / 195.
+int lq_ssd_least_rows(int rows, int batch, int heads) { return most_chunks(rows, batch, 1) * heads <= lq_compute_units() ? 1 : 48; }
 
 // A launch of more chunks than the scratch holds goes in rounds of equal numbers of them, each from the state that the
 // last one left: a prompt's scratch is bounded (a matrix memory of 4 heads of 256 x 513 takes 2.2 MB a chunk).
@@ -364,7 +369,29 @@ long long lq_ssd_chunks_least(int heads, int P, int N) { return heads * (part_fl
 
 long long lq_ssd_chunks_floats(int rows, int batch, int heads, int P, int N, int max_rows) {
   if (rows <= 0 || N > 2 * HALF || max_rows < LQ_SSD_MIN || heads > 65535 || lq_ceil_div(P, COLS) > 65535) return 0;
-  return chunks_scratch(most_chunks(rows, batch, LQ_SSD_LEAST), lq_ssd_chunks_least(heads, P, N), LQ_SSD_SCRATCH);
+  return chunks_scratch(most_chunks(rows, batch, lq_ssd_least_rows(rows, batch, heads)), lq_ssd_chunks_least(heads, P, N), LQ_SSD_SCRATCH);
+}
+
+// Whether a launch is faster in chunks (given scratch) than token by token (`segments`: in segments), by what both take.
+// A chunk of up to 128 channels costs the same however few they are and however few tokens it has; a walk's token costs little
+// where states are small, as soon as there are workgroups for the whole chip.  Microseconds, walk / chunks, 32 heads: of
+// 128 x 64, one sequence of 130 tokens 43 / 30, eight of 512 234 / 183, 32 of 256 451 / 389; of 64 x 64, eight of 256 93 / 101,
+// 32 of 256 231 / 353, one of 2 048 181 / 102; of 16 x 64, four of 1 000 139 / 178, eight of 512 144 / 178; of 64 x 16, eight
+// of 1 000 159 / 302.
+bool lq_ssd_chunks_faster(int batch, int heads, int P, int N, int max_rows, int rows, bool segments) {
+  if (lq_ssd_chunks_floats(rows, batch, heads, P, N, max_rows) == 0) return false;
+  const double token = 1.75e-3 * P / 64 * (N > 128 ? N / 80.0 : N > 32 ? N / 128.0 : 0.25) * heads, state = 0.02 * P / 64 * N / 128 * heads;
+  auto walk = [&](double n, double longest, double sequences, bool segments) {
+    const double chain = segments ? 20 + 0.12 * longest : (N > 32 ? 0.3 : 0.45) * longest, all = (segments ? 2 : 1) * token * n;
+    return 5 + (segments ? fmax(chain, all) : sqrt(chain * chain + all * all)) + state * sequences;
+  };
+  // the sequences beside the longest, by their mean, go in chunks as it does or all token by token
+  const double rest = rows - max_rows, least = lq_ssd_least_rows(rows, batch, heads);
+  const bool alike = batch == 1 || rest >= least * (batch - 1);
+  const double of_chunks = alike ? rows / 64.0 + batch / 2.0 : max_rows / 64.0 + 0.5;
+  double chunks = 24 + (N > HALF ? 0.125 : 0.082) * lq_ceil_div(P, COLS) * heads * of_chunks;
+  if (!alike) chunks += 10 + walk(rest, least, batch - 1, false);
+  return 0.9 * chunks < walk(rows, max_rows, batch, segments);
 }
 
 // -> 0, or -2.  `scratch`: lq_ssd_chunks_floats(...) floats, or fewer, down to lq_ssd_chunks_least(...)
@@ -372,10 +399,11 @@ int lq_ssd_chunks(const float* x, int ldx, const float* B, int ldb, const float*
                   const float* dt_bias, const float* a_log, const float* d_skip, float* state, float* y, int ldy, int heads,
                   int P, int N, int groups, const int* seq_slot, const int* cu_rows, int batch, int rows, float* scratch,
                   long long scratch_floats, const float* decay, int lddecay, int ones, hipStream_t stream) {
-  const long long all = most_chunks(rows, batch, LQ_SSD_LEAST);
+  const int least = lq_ssd_least_rows(rows, batch, heads);
+  const long long all = most_chunks(rows, batch, least);
   const long long room = chunks_a_round(all, scratch_floats, lq_ssd_chunks_least(heads, P, N));
   SsdArgs a = {x, B, C, dt, dt_bias, a_log, d_skip, decay, ldx, ldb, ldc, lddt, lddecay, ldy, state, y, scratch,
-               scratch + room * heads * part_floats(N, P), heads, groups, N, P, ones, batch, seq_slot, cu_rows, LQ_SSD_LEAST, 0, 0};
+               scratch + room * heads * part_floats(N, P), heads, groups, N, P, ones, batch, seq_slot, cu_rows, least, 0, 0};
   const bool quads = N % 4 == 0 && (P - ones) % 4 == 0 && ldx % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
                      (((uintptr_t)x | (uintptr_t)B | (uintptr_t)C) & 15) == 0;
   const auto state_kernel = quads ? ssd_chunk_state_kernel<true> : ssd_chunk_state_kernel<false>;

@@ -992,6 +992,12 @@ class HipKernels:
         return int(self.lib.lq_ssd_scan_workspace(c_int(batch), c_int(heads), c_int(head_dim), c_int(n_state),
                                                   c_int(max_rows), c_int(rows)))
 
+    @query
+    def ssd_scan_in_chunks(self, batch: int, heads: int, head_dim: int, n_state: int, max_rows: int, rows: int) -> bool:
+        """Whether `ssd_scan` is faster in chunks of tokens than token by token or in segments, for these sizes."""
+        return bool(self.lib.lq_ssd_scan_in_chunks(c_int(batch), c_int(heads), c_int(head_dim), c_int(n_state), c_int(max_rows),
+                                                   c_int(rows)))
+
     def ssd_scan(self, x: torch.Tensor, b_in: torch.Tensor, c_in: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor,
                  a_log: torch.Tensor, d_skip: torch.Tensor, state: torch.Tensor, y: torch.Tensor, heads: int,
                  head_dim: int, n_state: int, groups: int, seq_slot: torch.Tensor, cu_rows: torch.Tensor,

@@ -26,8 +26,9 @@ def _scan_scratch(ctx: StepContext, heads: int, head_dim: int, state: int) -> di
     ask = getattr(ctx.kernels, "ssd_scan_workspace", None)
     if ask is None:
         return {}
-    chunks = ctx.dtype == torch.bfloat16
-    need = ask(ctx.batch, heads, head_dim, state, ctx.max_new, *((ctx.rows,) if chunks else ()))
+    sizes = (ctx.batch, heads, head_dim, state, ctx.max_new)
+    chunks = ctx.dtype == torch.bfloat16 and ctx.kernels.ssd_scan_in_chunks(*sizes, ctx.rows)
+    need = ask(*sizes, *((ctx.rows,) if chunks else ()))
     return dict(max_rows=ctx.max_new, workspace=ctx.ws.alloc((need,), torch.float32),
                 **({"chunks": True} if chunks else {})) if need else {}
 

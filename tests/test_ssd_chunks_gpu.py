@@ -110,3 +110,52 @@ def test_scratch_is_bounded():
     kn = HipKernels()
     for rows, batch, heads, P, N in ((65536, 1, 32, 64, 128), (16384, 8, 4, 513, 256), (1 << 20, 4, 128, 64, 128)):
         assert 0 < kn.ssd_scan_workspace(batch, heads, P, N, rows // batch, rows) <= 64 << 20
+
+
+def test_short_sequences_beside_a_long_one_are_walked():
+    """More chunks than the chip takes at once: sequences of fewer than 48 tokens have the bits of the walk token by token,
+    the others those of a launch of their own in chunks."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(48)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    lens = [1, 47, 200, 48, 64, 130] + [2] * 40 + [49]
+    rows, batch, H, G, N, P = sum(lens), len(lens), 8, 4, 64, 48
+    x, b, c, dt = rand(rows, H * P), 0.3 * rand(rows, G * N), 0.3 * rand(rows, G * N), rand(rows, H)
+    made, state = (rand(H) - 3.0, 0.5 * rand(H) + 1.0, rand(H)), rand(batch, H, P, N)
+    kn = HipKernels()
+    need = lambda mine: kn.ssd_scan_workspace(len(mine), H, P, N, max(mine), sum(mine)) if max(mine) >= 128 else 0
+
+    def run(first, mine, floats):
+        n, at, B = sum(mine), sum(lens[:first]), len(mine)
+        y, end = torch.full((n, H * P), float("nan"), device="cuda"), state[first : first + B].clone()
+        part = lambda t: t[at : at + n]
+        how = dict(max_rows=max(mine), workspace=torch.full((floats,), float("nan"), device="cuda"), chunks=True) if floats else {}
+        kn.ssd_scan(part(x), part(b), part(c), part(dt), *made, end, y, H, P, N, G, i32(range(B)),
+                    i32(sum(mine[:i]) for i in range(B + 1)), B, **how)
+        return y, end
+
+    (got, got_end), (walked, walked_end) = run(0, lens, need(lens)), run(0, lens, 0)
+    unit = (3 * 200 + N) * 2.0 ** -24 * walked_end.abs().max().clamp(min=float(state.abs().max()))  # (as above)
+    for s, n in enumerate(lens):
+        at = sum(lens[:s])
+        if n < 48:
+            assert torch.equal(got[at : at + n], walked[at : at + n]) and torch.equal(got_end[s], walked_end[s])
+        else:
+            assert (got[at : at + n] - walked[at : at + n]).abs().max() <= unit * c.abs().view(rows, G, N).sum(-1).max() + 1e-6 * walked.abs().max()
+            if need([n]):  # (a launch of its own is in chunks too)
+                alone, end = run(s, [n], need([n]))
+                assert torch.equal(got[at : at + n], alone) and torch.equal(got_end[s], end[0])
+
+
+def test_which_launches_are_faster_in_chunks():
+    """Sizes far from where both ways take as long: few long sequences in chunks, very many or short ones of small states
+    token by token."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    ask = HipKernels().ssd_scan_in_chunks
+    assert ask(1, 32, 64, 128, 2048, 2048) and ask(8, 32, 64, 128, 512, 4096) and ask(1, 4, 513, 256, 2048, 2048)
+    assert ask(71, 32, 64, 128, 2000, 2070)
+    assert not ask(1, 32, 64, 128, 100, 100) and not ask(64, 32, 64, 128, 1, 64) and not ask(8, 32, 16, 64, 1000, 8000)
+    assert not ask(32, 32, 64, 16, 256, 32 * 256) and not ask(1, 32, 64, 300, 2048, 2048)
