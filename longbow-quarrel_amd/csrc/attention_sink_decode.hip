@@ -334,10 +334,10 @@ int splits_for(int rows, int nh, int nkv, int window, int keep_first, int chunk,
   const long long seen = window > 0 ? (long long)window + keep_first + 2 * BLOCK : max_len;
   int keys = seen < max_len ? (int)seen : max_len;
   if (chunk > 0 && chunk + BLOCK < keys) keys = chunk + BLOCK;
-  const int tiles = rows * nkv * lq_ceil_div(nh / nkv, 16), wanted = lq_ceil_div(lq_ceil_div(keys, BLOCK) + 1, NW);
-  int room = 2 * lq_compute_units() / tiles;
-  if (room > MAX_SPLITS) room = MAX_SPLITS;
-  return wanted < room ? wanted : room > 1 ? room : 1;
+  const long long tiles = (long long)rows * nkv * lq_ceil_div(nh / nkv, 16);
+  const int wanted = lq_ceil_div(lq_ceil_div(keys, BLOCK) + 1, NW), room = (int)(2 * lq_compute_units() / tiles);
+  const int most = room > MAX_SPLITS ? MAX_SPLITS : room;
+  return wanted < most ? wanted : most > 1 ? most : 1;
 }
 
 bool takes(int KD, int VD, int block_size, int nh, int nkv, int rows) {

@@ -132,6 +132,15 @@ def check(H, G, D, P, seqs, options, shared):
         assert (far <= 7e-5 + (want.float().abs() * 2 ** -7 if dtype == torch.bfloat16 else 0)).all(), far.max()
 
 
+def test_scratch_of_very_many_rows_and_heads():
+    """2^32 rows and key heads together are no number of 32 bits; so many share nothing out and ask for no scratch."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    ask = HipKernels().sink_attention_workspace
+    assert ask(torch.bfloat16, 1 << 17, 1 << 17, 1 << 15, 1 << 15, 64, 64, 64, 0, 0, 4096) == 0
+    assert ask(torch.bfloat16, 2, 2, 16, 4, 64, 64, 64, 0, 0, 4096) > 0
+
+
 @pytest.mark.parametrize("H,G,D,P,options", [(8, 2, 128, 128, PLAIN), (4, 1, 64, 64, dict(PLAIN, window=70)), (2, 2, 200, 104, PLAIN)])
 def test_a_row_has_the_same_bits_whatever_its_neighbours(H, G, D, P, options):
     """A prompt's row beside rows of ordinary scores, beside rows of scores 60 times as large (whose maximum moves in every
