@@ -209,8 +209,9 @@ def test_router_and_experts_activation(kn):
         assert uc.err(out.cpu(), want) < TOL_F32
 
 
-def test_rows_sorted_by_expert_and_back(kn):
-    rows, E, width = 300, 5, 40
+@pytest.mark.parametrize("rows,width", [(300, 40), (1023, 40), (1024, 37), (1025, 40), (2500, 37)])
+def test_rows_sorted_by_expert_and_back(kn, rows, width):
+    E = 5  # (the sort walks 1 024 rows at a time; rows of 37 are no whole vectors)
     route = torch.where(rnd(rows, E, seed=1) > 0.3, rnd(rows, E, seed=2).abs(), torch.full((rows, E), -1.0))
     route[7] = -1.0  # a row that chose nothing
     pairs = int((route >= 0).sum())
@@ -222,14 +223,18 @@ def test_rows_sorted_by_expert_and_back(kn):
     assert order[:pairs].tolist() == want_order and bool((order[pairs:] == -7).all())
     want_w = [float(route[r, e]) for e in range(E) for r in range(rows) if route[r, e] >= 0]
     assert weight[:pairs, 0].tolist() == want_w
-    at = 0
+    filled, weights = torch.full_like(order, -7), torch.zeros_like(weight)
+    kn.moe_sort(dev(route), counts, filled, weights, place_of, fill=True)
+    assert torch.equal(filled[:pairs], order[:pairs]) and torch.equal(weights[:pairs], weight[:pairs])
+    assert not filled[pairs:].any() and bool((weights[pairs:] == -1).all())
+    at, places = 0, place_of.cpu()
     for e in range(E):
         for r in range(rows):
             if route[r, e] >= 0:
-                assert int(place_of[r, e]) == at
+                assert int(places[r, e]) == at
                 at += 1
             else:
-                assert int(place_of[r, e]) == -1
+                assert int(places[r, e]) == -1
     for dtype in (torch.float32, torch.bfloat16):
         src = rnd(rows, width + 8, seed=3).to(dtype)
         dst = torch.zeros(rows * E, width, dtype=dtype, device=DEV)
