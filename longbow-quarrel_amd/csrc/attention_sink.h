@@ -2,7 +2,12 @@
 // shaped on its way to the softmax.
 #pragma once
 
+#include <cfloat>
+
 #include "common.h"
+
+constexpr float LOG2E = 1.44269504088896340736f;
+constexpr float NONE = -3.0e38f;  // the running maximum of a row that has seen no key (finite: no inf - inf)
 
 struct ScoreShape {
   float cap;                       // 0: no cap
@@ -29,6 +34,18 @@ struct SinkArgs {
 __device__ inline int first_key(const SinkArgs& a, int p) {
   const int lo = (a.window > 0 && p >= a.window) ? p - a.window + 1 : 0;
   return a.chunk > 0 ? max(lo, p / a.chunk * a.chunk) : lo;
+}
+
+// Where a query head's softmax starts from its sink: the running maximum in powers of two, finite whatever the sink, and
+// the sink's part of the sum.  A sink of -inf, or so low that it is in powers of two, adds nothing; one so high that it is
+// infinite in powers of two outweighs every key; NaN and +inf make NaN of the sum.
+struct SinkStart {
+  float m, l;
+};
+__device__ inline SinkStart sink_start(const SinkArgs& a, int h) {
+  if (a.sinks == nullptr) return {0.f, 1.f};
+  const float s = a.sinks[h], m = s * LOG2E;
+  return {fminf(fmaxf(m, NONE), FLT_MAX), m < NONE ? 0.f : fmaf(s, 0.f, 1.f)};
 }
 
 // What a lane needs of its query head to shape a score.

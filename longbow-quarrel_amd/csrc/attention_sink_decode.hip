@@ -26,8 +26,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int BLOCK = 64, NW = 4, MAX_SPLITS = 64;
-constexpr float LOG2E = 1.44269504088896340736f;
-constexpr float NONE = -3.0e38f;  // the running maximum of a row that has seen no key
 
 __device__ inline bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 __device__ inline unsigned upper2(float lo, float hi) {
@@ -179,7 +177,10 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
   if constexpr (SHAPED) hs = head_shape(a, h);
   const float c2 = a.scale * LOG2E;
   float m = NONE, l = 0.f;  // the head's running maximum (in powers of two); this lane's share of its sum
-  if (a.sink && split == 0 && w == 0) m = a.sinks != nullptr ? a.sinks[h] * LOG2E : 0.f, l = g == 0 ? 1.f : 0.f;
+  if (a.sink && split == 0 && w == 0) {
+    const SinkStart start = sink_start(a, h);
+    m = start.m, l = g == 0 ? start.l : 0.f;
+  }
   f32x4 o[VT];  // o[dt][e]: value entry 16 dt + 4 g + e of head c
 #pragma unroll
   for (int dt = 0; dt < VT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};

@@ -43,8 +43,6 @@ namespace {
 
 constexpr int BLOCK = 64;                    // positions a cache block
 constexpr int SLOTS = 4;                     // tiles of 32 rows a workgroup
-constexpr float LOG2E = 1.44269504088896340736f;
-constexpr float NONE = -3.0e38f;             // the running maximum of a row that has seen no key (finite: no inf - inf)
 constexpr float SLACK = 8.0f;                // the maximum moves when a score lies this far (in powers of two) above it
 
 __device__ inline bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -172,10 +170,8 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
 
   float m = NONE, l = 0.f;  // the row's running maximum (in powers of two); this lane's share of its sum
   if (a.sink && ks == 0) {
-    // (a sink of -inf, or so low that it is in powers of two, adds nothing: the maximum itself stays finite, since -inf
-    // less -inf is no number in a row that sees none of its first keys)
-    const float s = a.sinks != nullptr ? a.sinks[h] * LOG2E : 0.f;
-    m = fmaxf(s, NONE), l = hf == 0 ? __builtin_amdgcn_exp2f(s - m) : 0.f;
+    const SinkStart start = sink_start(a, h);
+    m = start.m, l = hf == 0 ? start.l : 0.f;
   }
   f32x16 o[VT];
 #pragma unroll

@@ -25,6 +25,7 @@ CASES = [  # heads, key heads, key size, value size, (new, held) of every sequen
     (8, 2, 128, 128, [(130, 300), (40, 0)], dict(sinks="lowest", window=100)),
     (4, 1, 64, 64, [(200, 30)], dict(sinks="none", chunk=50)), (8, 4, 200, 104, [(100, 90)], dict(sinks="lowest", window=40)),
     (6, 3, 128, 256, [(140, 64)], dict(sinks="none", window=33, keep_first=3)),
+    (8, 2, 128, 128, [(130, 300), (40, 0)], dict(sinks="highest", window=100)), (8, 4, 200, 104, [(100, 90)], dict(sinks="highest", window=40)),
 ]
 
 
@@ -35,6 +36,7 @@ SINGLE = [  # heads, key heads, key size, value size, options
     (8, 4, 128, 256, dict(PLAIN, maps=2, window=600)), (3, 3, 40, 24, dict(window=1, wide=True)),
     (8, 2, 128, 128, dict(sinks=True, cap=30.0, log=True, window=200)),
     (8, 2, 64, 64, dict(PLAIN, cap=5.0, dist=100, temp=True, wide=True)),
+    (8, 2, 128, 128, dict(sinks="highest", window=300)),
     (8, 2, 128, 128, dict(sinks="lowest", window=100)), (4, 1, 64, 64, dict(sinks="none", chunk=50))]
 
 
@@ -76,10 +78,11 @@ def check(H, G, D, P, seqs, options, shared):
                 chunk=o.get("chunk", 0), softcap=o.get("cap", 0.0))
     if "sinks" in o:
         more["sink_values"] = rand(H)
-        lowest = {"none": [float("-inf")], "lowest": [torch.finfo(torch.float32).min, -2.4e38, -2.0e38, float("-inf")]}.get(o["sinks"], [])
-        for i in range(H if lowest else 0):  # (a sink that says no more than an absent one, beside ordinary ones)
+        most = torch.finfo(torch.float32).max
+        odd = {"none": [float("-inf")], "lowest": [-most, -2.4e38, -2.0e38, float("-inf")], "highest": [most, 2.4e38, 2.0e38]}.get(o["sinks"], [])
+        for i in range(H if odd else 0):  # (a sink that says no more than an absent one, or all there is, beside ordinary ones)
             if i % 3 < 2:
-                more["sink_values"][i] = lowest[i % len(lowest)]
+                more["sink_values"][i] = odd[i % len(odd)]
     if "gate" in o:
         more["gate"] = rand(rows, H).bfloat16()
     if "wide" in o:
