@@ -1287,7 +1287,7 @@ extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, co
              "ssd_scan: a row stride is smaller than its row");
   LQ_REQUIRE(x && Bm && Cm && dt && state && y && seq_slot && cu_rows, "ssd_scan: null pointer");
   LQ_REQUIRE(decay != nullptr || (dt_bias && a_log && d_skip), "ssd_scan: neither decays nor what makes them");
-  int below = 0x7fffffff;  // what is walked token by token
+  int below = 0x7fffffff;  // sequences of fewer rows are walked token by token
   const long long chunks = scratch != nullptr ? lq_ssd_chunks_floats(rows, batch, heads, P, N, max_rows) : 0;
   if (chunks > 0) {
     const long long least = lq_ssd_chunks_least(heads, P, N);
@@ -1296,7 +1296,7 @@ extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, co
     const int rc = lq_ssd_chunks(x, ldx, Bm, ldb, Cm, ldc, dt, lddt, dt_bias, a_log, d_skip, state, y, ldy, heads, P, N, groups,
                          seq_slot, cu_rows, batch, rows, scratch, scratch_floats, decay, lddecay, ones, stream);
     below = lq_ssd_least_rows(rows, batch, heads);
-    if (rc != 0 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
+    if (rc != 0 || below <= 1 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
   }
   const long long need = scratch != nullptr && chunks == 0 ? ssd_segment_floats(batch, heads, P, N, max_rows) : 0;
   ScanLaunch cfg;
@@ -1358,7 +1358,7 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
   LQ_REQUIRE(rows > 0 && rows <= 0x7fffffff && kv_heads <= 65535, "delta_scan: %d rows, %d q/k heads", rows, kv_heads);
   unit_heads_kernel<<<dim3((unsigned)rows, kv_heads), 64, 0, stream>>>(q, ldq, k, ldk, Dk, q_scale, unit_eps);
   LQ_CHECK_LAUNCH("delta_scan(unit vectors)");
-  int below = 0x7fffffff;  // what is walked token by token
+  int below = 0x7fffffff;  // sequences of fewer rows are walked token by token
   const long long need = scratch != nullptr ? lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) : 0;
   if (need > 0) {
     LQ_REQUIRE(lq_delta_scan_least(heads) <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
@@ -1367,7 +1367,7 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
     const int rc = lq_delta_chunks(q, ldq, k, ldk, v, ldv, beta, ldbeta, a, lda, dt_bias, a_log, state, out, ldo, heads, kv_heads,
                                    Dk, P, seq_slot, cu_rows, batch, rows, channel_decay, scratch, scratch_floats, stream);
     below = lq_delta_least_rows(rows, batch, heads, channel_decay);
-    if (rc != 0 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
+    if (rc != 0 || below <= 1 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
   }
   dim3 grid((unsigned)(batch * heads), lq_ceil_div(P, cfg.cols));
   ScanShape sh = {heads, kv_heads, P, Dk, seq_slot, cu_rows};
