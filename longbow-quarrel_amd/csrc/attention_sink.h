@@ -1,5 +1,5 @@
-// What the two files of the windowed attention with a sink share: the arguments of its kernels and how a score is
-// shaped on its way to the softmax.
+// What the three files of the windowed attention with a sink share: the arguments of its kernels, how a score is shaped on
+// its way to the softmax, and how a 32-bit probability is cut into bfloat16 operands.
 #pragma once
 
 #include <cfloat>
@@ -100,6 +100,18 @@ __device__ inline uint4 load_q8(const bf16_t* p) {
   const uint2 lo = *(const uint2*)p, hi = *(const uint2*)(p + 4);
   return make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ inline bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+// A 32-bit number as the exact sum of three bfloat16 numbers: its upper half, the upper half of what is below that, and the
+// rest.  The upper halves of two words, side by side, are two entries of an operand.
+__device__ inline unsigned upper2(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ inline float below_upper(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 
 inline bool scores_shaped(const ScoreShape& s) {
   return s.cap > 0.f || s.temp != nullptr || s.r1 != nullptr || s.dist != nullptr;

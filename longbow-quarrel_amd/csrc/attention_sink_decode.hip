@@ -19,19 +19,11 @@
 // Values of positions that were never written count as zero.
 #include "attention_sink.h"
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
 constexpr int BLOCK = 64, NW = 4, MAX_SPLITS = 64;
-
-__device__ inline bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-__device__ inline unsigned upper2(float lo, float hi) {
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ inline float below_upper(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 
 // over the four lanes that share l % 16
 __device__ inline float across_max(float x) {

@@ -30,14 +30,13 @@
 // wavefronts are 0.85: the softmax, the cutting of the probabilities and the round trips through LDS between the
 // products bound it.
 #include "attention_sink.h"
+#include "sequence_parts.h"
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
@@ -45,17 +44,9 @@ constexpr int BLOCK = 64;                    // positions a cache block
 constexpr int SLOTS = 4;                     // tiles of 32 rows a workgroup
 constexpr float SLACK = 8.0f;                // the maximum moves when a score lies this far (in powers of two) above it
 
-__device__ inline bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-
 __device__ inline unsigned pack2(float lo, float hi) {  // round to nearest even
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
 }
-
-// the upper halves of two 32-bit words, side by side
-__device__ inline unsigned upper2(float lo, float hi) {
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ inline float below_upper(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 
 __device__ inline float halves_max(float x) {
   auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -72,34 +63,6 @@ __device__ inline int wave_least(int v) {
   return __builtin_amdgcn_readfirstlane(v);
 }
 __device__ inline int wave_most(int v) { return -wave_least(-v); }
-
-// Which tile of `block_rows` rows of which sequence a workgroup takes: tiles are numbered through the sequences, the
-// last part-filled.  Lane i holds sequence i of a run of 64; every wavefront works out the same.
-struct Tile {
-  int seq, row, rows;  // rows 0: past the last tile
-};
-__device__ inline Tile find_tile(const int* __restrict__ cu_rows, int batch, int block_rows, int t) {
-  const int lane = threadIdx.x & 63;
-  for (int b0 = 0; b0 < batch; b0 += 64) {
-    const int b = min(b0 + lane, batch - 1), begin = cu_rows[b], n = b0 + lane < batch ? cu_rows[b + 1] - begin : 0;
-    const int mine = (n + block_rows - 1) / block_rows;
-    int upto = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int before = __shfl_up(upto, off, 64);
-      if (lane >= off) upto += before;
-    }
-    const unsigned long long past = __ballot(upto > t);
-    if (past) {
-      const int at = __ffsll(past) - 1;
-      const int k = t - __shfl(upto - mine, at, 64), first = __shfl(begin, at, 64), count = __shfl(n, at, 64);
-      return {__builtin_amdgcn_readfirstlane(b0 + at), __builtin_amdgcn_readfirstlane(first + k * block_rows),
-              __builtin_amdgcn_readfirstlane(min(block_rows, count - k * block_rows))};
-    }
-    t -= __shfl(upto, 63, 64);
-  }
-  return {0, 0, 0};
-}
 
 // KD and VD up to 16 KS16 and 32 VT: sizes in between run with zeros behind their keys and values.
 template <int KS16, int VT>
@@ -130,7 +93,7 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
   // late tiles, which see the most keys, come first; neighbouring workgroups are different heads, so that a die's L2
   // holds few heads' keys
   const int per_tile = gridDim.x / tiles;
-  const Tile tile = find_tile(cu_rows, batch, 32 * (SLOTS / heads), tiles - 1 - (int)blockIdx.x / per_tile);
+  const Part tile = find_part(cu_rows, batch, 32 * (SLOTS / heads), 1, tiles - 1 - (int)blockIdx.x / per_tile);
   if (tile.rows <= 0) return;  // the whole workgroup
   const int hbase = (int)(blockIdx.x % per_tile) * heads, kvh = hbase / (a.nh / a.nkv);
   const int h = hbase + slot % heads;
@@ -139,7 +102,7 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
   const long long krow = (long long)a.maps * KD;
   const int my_at = slot / heads * 32 + c;  // this lane's row within the workgroup's: maybe past its last
   const bool mine = my_at < tile.rows;
-  const int my_row = tile.row + min(my_at, tile.rows - 1);
+  const int my_row = tile.first + min(my_at, tile.rows - 1);
   const int my_pos = a.row_pos[my_row], my_lo = first_key(a, my_pos);
   HeadShape hs;
   if constexpr (SHAPED) hs = head_shape(a, h);
@@ -158,7 +121,7 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
   // what the workgroup's rows see together, and what this tile's do
   int lo_min = 0x7fffffff, pos_max = -1;
   for (int i = lane; i < tile.rows; i += 64) {
-    const int p = a.row_pos[tile.row + i];
+    const int p = a.row_pos[tile.first + i];
     lo_min = min(lo_min, first_key(a, p)), pos_max = max(pos_max, p);
   }
   lo_min = wave_least(lo_min), pos_max = wave_most(pos_max);
@@ -230,78 +193,78 @@ __global__ __launch_bounds__(SLOTS * KS * 64, KS) void sink_rows32_kernel(const 
     const unsigned char* cur = smem + turn * L::STAGE;
 #pragma unroll
     for (int half = KS == 2 ? ks : 0; half < (KS == 2 ? ks + 1 : 2); ++half) {
-    const int tw = t0 + 32 * half;  // this wavefront's 32 keys
-    if (tw <= t_pos_max && (tw + 31 >= t_lo_min || tw < a.keep_first)) {
-      f32x16 sc;
+      const int tw = t0 + 32 * half;  // this wavefront's 32 keys
+      if (tw <= t_pos_max && (tw + 31 >= t_lo_min || tw < a.keep_first)) {
+        f32x16 sc;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) sc[e] = 0.f;
-      u32x4 kf[KS16];
+        for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+        u32x4 kf[KS16];
 #pragma unroll
-      for (int kk = 0; kk < KS16; ++kk) kf[kk] = *(const u32x4*)(cur + L::k_at(32 * half + key_of_lane, 2 * kk + hf));
+        for (int kk = 0; kk < KS16; ++kk) kf[kk] = *(const u32x4*)(cur + L::k_at(32 * half + key_of_lane, 2 * kk + hf));
 #pragma unroll
-      for (int kk = 0; kk < KS16; ++kk)
-        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[kk]), as_bf16x8(qf[kk]), sc, 0, 0, 0);
-      // sc[e] is the score of key tw + 16 (e / 8) + 8 hf + e % 8
-      const bool masked = !(tw + 31 <= t_pos_min && (tw >= t_lo_max || tw + 31 < a.keep_first));
-      if constexpr (SHAPED) {
+        for (int kk = 0; kk < KS16; ++kk)
+          sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[kk]), as_bf16x8(qf[kk]), sc, 0, 0, 0);
+        // sc[e] is the score of key tw + 16 (e / 8) + 8 hf + e % 8
+        const bool masked = !(tw + 31 <= t_pos_min && (tw >= t_lo_max || tw + 31 < a.keep_first));
+        if constexpr (SHAPED) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int t = tw + 16 * (e / 8) + 8 * hf + e % 8;
-          sc[e] = shaped<false>(sc[e], max(my_pos - t, 0), hs) * LOG2E;
+          for (int e = 0; e < 16; ++e) {
+            const int t = tw + 16 * (e / 8) + 8 * hf + e % 8;
+            sc[e] = shaped<false>(sc[e], max(my_pos - t, 0), hs) * LOG2E;
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sc[e] *= c2;
         }
-      } else {
+        if (masked) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) sc[e] *= c2;
-      }
-      if (masked) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int t = tw + 16 * (e / 8) + 8 * hf + e % 8;
-          if (!(mine && t <= my_pos && (t >= my_lo || t < a.keep_first))) sc[e] = -INFINITY;
+          for (int e = 0; e < 16; ++e) {
+            const int t = tw + 16 * (e / 8) + 8 * hf + e % 8;
+            if (!(mine && t <= my_pos && (t >= my_lo || t < a.keep_first))) sc[e] = -INFINITY;
+          }
         }
-      }
-      float top = sc[0];
+        float top = sc[0];
 #pragma unroll
-      for (int e = 1; e < 16; ++e) top = fmaxf(top, sc[e]);
-      top = halves_max(top);
-      if (__any(top > m + SLACK)) {
-        // (each row by its own scores: its roundings do not depend on which rows share the tile)
-        const float m_new = top > m + SLACK ? top : m, alpha = __builtin_amdgcn_exp2f(m - m_new);
-        l *= alpha;
-        m = m_new;
-#pragma unroll
-        for (int dt = 0; dt < VT; ++dt)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
-      }
-      float sum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        sc[e] = __builtin_amdgcn_exp2f(sc[e] - m);
-        sum += sc[e];
-      }
-      l += sum;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        u32x4 vf[VT];
-#pragma unroll
-        for (int dt = 0; dt < VT; ++dt) vf[dt] = *(const u32x4*)(cur + L::v_at(32 * dt + c, 4 * half + 2 * s + hf));
-        u32x4 part[3];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float p0 = sc[8 * s + 2 * j], p1 = sc[8 * s + 2 * j + 1];
-          const float q0 = below_upper(p0), q1 = below_upper(p1);
-          part[0][j] = upper2(p0, p1);
-          part[1][j] = upper2(q0, q1);
-          part[2][j] = upper2(below_upper(q0), below_upper(q1));
-        }
-#pragma unroll
-        for (int i = 2; i >= 0; --i)
+        for (int e = 1; e < 16; ++e) top = fmaxf(top, sc[e]);
+        top = halves_max(top);
+        if (__any(top > m + SLACK)) {
+          // (each row by its own scores: its roundings do not depend on which rows share the tile)
+          const float m_new = top > m + SLACK ? top : m, alpha = __builtin_amdgcn_exp2f(m - m_new);
+          l *= alpha;
+          m = m_new;
 #pragma unroll
           for (int dt = 0; dt < VT; ++dt)
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vf[dt]), as_bf16x8(part[i]), o[dt], 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          sc[e] = __builtin_amdgcn_exp2f(sc[e] - m);
+          sum += sc[e];
+        }
+        l += sum;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          u32x4 vf[VT];
+#pragma unroll
+          for (int dt = 0; dt < VT; ++dt) vf[dt] = *(const u32x4*)(cur + L::v_at(32 * dt + c, 4 * half + 2 * s + hf));
+          u32x4 part[3];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float p0 = sc[8 * s + 2 * j], p1 = sc[8 * s + 2 * j + 1];
+            const float q0 = below_upper(p0), q1 = below_upper(p1);
+            part[0][j] = upper2(p0, p1);
+            part[1][j] = upper2(q0, q1);
+            part[2][j] = upper2(below_upper(q0), below_upper(q1));
+          }
+#pragma unroll
+          for (int i = 2; i >= 0; --i)
+#pragma unroll
+            for (int dt = 0; dt < VT; ++dt)
+              o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vf[dt]), as_bf16x8(part[i]), o[dt], 0, 0, 0);
+        }
       }
-    }
     }
     // Nobody reads the other stage: its last readers passed the barrier below a block ago.
     if (more) stash(next, smem + (turn ^ 1) * L::STAGE);

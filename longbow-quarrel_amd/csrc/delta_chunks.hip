@@ -102,11 +102,11 @@ template <bool QUADS>
 __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   Prepared& L = *(Prepared*)smem;
-  const int2 at = find_chunk(a.cu_rows, a.batch, a.least, a.first + blockIdx.x);
-  if (at.x < 0) return;
+  const Part at = find_part(a.cu_rows, a.batch, CHUNK, a.least, a.first + blockIdx.x);
+  if (at.seq < 0) return;
   const int h = blockIdx.y, j = h / (a.heads / a.kv_heads), tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const long long r0 = a.cu_rows[at.x] + (long long)at.y * CHUNK;
-  const int nt = min(CHUNK, (int)(a.cu_rows[at.x + 1] - r0)), N = a.N;
+  const long long r0 = at.first;
+  const int nt = at.rows, N = a.N;
   float* to = a.scratch + ((long long)blockIdx.x * a.heads + h) * PART;
   const float rate = -expf(a.a_log[h]);
 

@@ -18,9 +18,9 @@
 // K / 256 + 64 additions instead of K.
 //
 // Three kernels: an LDS-tiled one (block tiles of 64 x 64 or 128 x 128, any size and alignment); a pipelined one of
-// 128 x 128 tiles for float32 operands in whole pieces with K in 32s; and one for up to 16 rows that streams the weights
-// straight from memory, a block of waves a tile of 16 columns, its waves taking chunks in turn and adding their sums up
-// in order through LDS.
+// 128 x 128 or 64 x 128 tiles for float32 operands in whole pieces with K in 32s, from 33 rows on; and one for up to 64 rows
+// that streams the weights straight from memory, a block of waves a tile of 16 columns, its waves taking chunks in turn and
+// adding their sums up in order through LDS.
 #include "common.h"
 
 namespace {
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const T* __restrict
 }
 
 // ---- pipelined: the same tiles, operands in whole pieces ---------------------------------------------------
-// 128 x 128 a block, 4 waves of 64 x 64.  Stages of 32 k (two slabs) go from memory straight into LDS (16 bytes a lane, no
+// 128 x 128 a block, 4 waves of 64 x 64; or 64 x 128, waves of 32 x 64.  Stages of 32 k (two slabs) go from memory straight into LDS (16 bytes a lane, no
 // registers), two stages taking turns: the next one's transfers fly while this one is multiplied, 128 matrix instructions
 // a wave, behind one barrier a stage.  A lane's four k of a slab are one 16-byte read.  An LDS row is 32 k, 128 bytes; its
 // piece u lies at u ^ (row / 2 % 8), so that the 16 rows of a fragment lie in different banks.  Two blocks a compute
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pipelined_kernel(const float*
     }
 }
 
-// ---- at most 16 rows: the weights streamed from memory ---------------------------------------------------
+// ---- at most 64 rows: the weights streamed from memory ---------------------------------------------------
 // Four k of a row as float32: 16 bytes of float32 or 8 bytes of bfloat16.
 __device__ inline f32x4 load4(const float* p) { return *(const f32x4*)p; }
 __device__ inline f32x4 load4(const bf16_t* p) {

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "device_math.h"
+#include "sequence_parts.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -12,31 +13,7 @@ constexpr int CHUNK = 64, SUB = 16, KT = CHUNK / SUB;  // tokens a chunk and a b
 constexpr int FRAG = 256;                              // floats a tile of 16 x 16
 
 // The chunks of a sequence of n tokens: none for one shorter than `least`, which is walked token by token instead.
-__device__ inline int chunks_of(int n, int least) { return n >= least ? (n + CHUNK - 1) / CHUNK : 0; }
-
-// The chunks of all sequences are numbered through.  -> the sequence of chunk number t and its number within it (-1:
-// past the last).  Lane i holds sequence i of a run of 64; every wavefront works out the same.
-__device__ inline int2 find_chunk(const int* __restrict__ cu_rows, int batch, int least, int t) {
-  const int lane = threadIdx.x & 63;
-  for (int b0 = 0; b0 < batch; b0 += 64) {
-    const int b = min(b0 + lane, batch - 1);
-    const int mine = b0 + lane < batch ? chunks_of(cu_rows[b + 1] - cu_rows[b], least) : 0;
-    int upto = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int before = __shfl_up(upto, off, 64);
-      if (lane >= off) upto += before;
-    }
-    const unsigned long long past = __ballot(upto > t);
-    if (past) {
-      const int at = __ffsll(past) - 1;
-      return make_int2(__builtin_amdgcn_readfirstlane(b0 + at),
-                       __builtin_amdgcn_readfirstlane(t - __shfl(upto - mine, at, 64)));
-    }
-    t -= __shfl(upto, 63, 64);
-  }
-  return make_int2(-1, -1);
-}
+__device__ inline int chunks_of(int n, int least) { return parts_of(n, CHUNK, least); }
 
 // the number of sequence b's first chunk
 __device__ inline int first_chunk(const int* __restrict__ cu_rows, int b, int least) {

@@ -90,12 +90,12 @@ template <bool QUADS>
 __global__ __launch_bounds__(256) void ssd_chunk_state_kernel(SsdArgs a) {
   __shared__ __attribute__((aligned(16))) float Bs[CHUNK][LDN], Xs[CHUNK][LDX];
   __shared__ float weight[CHUNK];
-  const int2 at = find_chunk(a.cu_rows, a.batch, a.least, a.first + blockIdx.x);
-  if (at.x < 0) return;
+  const Part at = find_part(a.cu_rows, a.batch, CHUNK, a.least, a.first + blockIdx.x);
+  if (at.seq < 0) return;
   const int h = blockIdx.y, grp = h / (a.heads / a.groups), p0 = blockIdx.z * COLS, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, Px = a.P - a.ones;
-  const long long r0 = a.cu_rows[at.x] + (long long)at.y * CHUNK, place = (long long)blockIdx.x * a.heads + h;
-  const int nt = min(CHUNK, (int)(a.cu_rows[at.x + 1] - r0));
+  const long long r0 = at.first, place = (long long)blockIdx.x * a.heads + h;
+  const int nt = at.rows;
   Slab<COLS, 256, QUADS> xs;
   Slab<HALF, 256, QUADS> bs;
   xs.fetch(a.x + r0 * a.ldx + (long long)h * Px + p0, a.ldx, nt, Px - p0);
@@ -210,12 +210,12 @@ template <bool QUADS>
 __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   OutLds& L = *(OutLds*)smem;
-  const int2 at = find_chunk(a.cu_rows, a.batch, a.least, a.first + blockIdx.x);
-  if (at.x < 0) return;
+  const Part at = find_part(a.cu_rows, a.batch, CHUNK, a.least, a.first + blockIdx.x);
+  if (at.seq < 0) return;
   const int h = blockIdx.y, grp = h / (a.heads / a.groups), p0 = blockIdx.z * COLS, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane & 15, g = lane >> 4, Px = a.P - a.ones, pt = w & 3, m0 = w >> 2 << 1;  // token tiles m0 and m0 + 1
-  const long long r0 = a.cu_rows[at.x] + (long long)at.y * CHUNK, place = (long long)blockIdx.x * a.heads + h;
-  const int nt = min(CHUNK, (int)(a.cu_rows[at.x + 1] - r0)), tiles_p = p_tiles(a.P);
+  const long long r0 = at.first, place = (long long)blockIdx.x * a.heads + h;
+  const int nt = at.rows, tiles_p = p_tiles(a.P);
   const float* start = a.scratch + place * part_floats(a.N, a.P);
   const int my_pt = min(p0 / 16 + pt, tiles_p - 1);
   Slab<COLS, 512, QUADS> xs;
