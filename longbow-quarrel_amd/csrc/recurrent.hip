@@ -1270,16 +1270,16 @@ extern "C" int lq_ssd_scan_in_chunks(int batch, int heads, int P, int N, int max
 }
 
 // x [rows, heads * P], B and C [rows, groups * N], dt [rows, heads] (before its softplus), state
-// [slots, heads, P, N], y [rows, heads * P]; rows lie sequence by sequence (cu_rows).  `max_rows`: the most rows a
-// sequence brings (0: unknown); `scratch`: lq_ssd_scan_workspace(...) floats, or null (then no segments; a launch in chunks
+// [slots, heads, P, N], y [rows, heads * P]; rows lie sequence by sequence (cu_rows).  `max_rows`, `min_rows`: the most and
+// the fewest rows a sequence brings (0: unknown); `scratch`: lq_ssd_scan_workspace(...) floats, or null (then no segments; a launch in chunks
 // takes fewer too, down to lq_ssd_chunks_least(...), in more rounds).
 // `decay` [rows, heads] (or null): a token's decay and step are given, S <- decay S + dt B x^T, y = S^T C; dt_bias, a_log
 // and d_skip are then null.  `rows` > 0: the step's rows, and the launch may run in chunks.  `ones`: x is [rows, heads * (P - 1)], and a head's last column has the input one.
 extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, const float* Cm, int ldc, const float* dt,
                            int lddt, const float* dt_bias, const float* a_log, const float* d_skip, float* state, float* y,
                            int ldy, int heads, int P, int N, int groups, const int* seq_slot, const int* cu_rows, int batch,
-                           int max_rows, float* scratch, long long scratch_floats, const float* decay, int lddecay, int ones,
-                           int rows, hipStream_t stream) {
+                           int max_rows, int min_rows, float* scratch, long long scratch_floats, const float* decay, int lddecay,
+                           int ones, int rows, hipStream_t stream) {
   LQ_REQUIRE(heads > 0 && P > 0 && N > 0 && groups > 0 && heads % groups == 0 && batch > 0, "ssd_scan: bad sizes");
   LQ_REQUIRE(ones == 0 || (ones == 1 && P > 1), "ssd_scan: a column of ones beside %d columns", P - 1);
   LQ_REQUIRE(ldx >= heads * (P - ones) && ldy >= heads * P && ldb >= groups * N && ldc >= groups * N && lddt >= heads &&
@@ -1296,7 +1296,7 @@ extern "C" int lq_ssd_scan(const float* x, int ldx, const float* Bm, int ldb, co
     const int rc = lq_ssd_chunks(x, ldx, Bm, ldb, Cm, ldc, dt, lddt, dt_bias, a_log, d_skip, state, y, ldy, heads, P, N, groups,
                          seq_slot, cu_rows, batch, rows, scratch, scratch_floats, decay, lddecay, ones, stream);
     below = lq_ssd_least_rows(rows, batch, heads);
-    if (rc != 0 || below <= 1 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
+    if (rc != 0 || below <= 1 || min_rows >= below || rows - (batch - 1ll) * max_rows >= below) return rc;  // (none is shorter)
   }
   const long long need = scratch != nullptr && chunks == 0 ? ssd_segment_floats(batch, heads, P, N, max_rows) : 0;
   ScanLaunch cfg;
@@ -1339,7 +1339,7 @@ extern "C" long long lq_delta_scan_least(int heads);
 int lq_delta_least_rows(int rows, int batch, int heads, int channel_decay);
 
 // q and k [rows, kv_heads * Dk], v [rows, heads * P], beta and a [rows, heads] (raw), state [slots, heads, P, Dk],
-// out [rows, heads * P]; `max_rows`: the most rows that a sequence brings (0: unknown); `scratch`:
+// out [rows, heads * P]; `max_rows`, `min_rows`: the most and the fewest rows that a sequence brings (0: unknown); `scratch`:
 // lq_delta_scan_workspace(...) floats for a launch in chunks, or null (fewer make more rounds, down to
 // lq_delta_scan_least(heads))
 // (q and k are made unit vectors in place)
@@ -1348,7 +1348,7 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
                              int ldbeta, const float* a, int lda, const float* dt_bias, const float* a_log, float* state,
                              float* out, int ldo, int heads, int kv_heads, int Dk, int P, float q_scale, float unit_eps,
                              const int* seq_slot, const int* cu_rows, int batch, int rows, int channel_decay,
-                             int max_rows, float* scratch, long long scratch_floats, hipStream_t stream) {
+                             int max_rows, int min_rows, float* scratch, long long scratch_floats, hipStream_t stream) {
   LQ_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && Dk > 0 && P > 0 && batch > 0, "delta_scan: bad sizes");
   LQ_REQUIRE(ldq >= kv_heads * Dk && ldk >= kv_heads * Dk && ldv >= heads * P && ldo >= heads * P && ldbeta >= heads &&
                  lda >= (channel_decay ? heads * Dk : heads), "delta_scan: a row stride is smaller than its row");
@@ -1367,7 +1367,7 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
     const int rc = lq_delta_chunks(q, ldq, k, ldk, v, ldv, beta, ldbeta, a, lda, dt_bias, a_log, state, out, ldo, heads, kv_heads,
                                    Dk, P, seq_slot, cu_rows, batch, rows, channel_decay, scratch, scratch_floats, stream);
     below = lq_delta_least_rows(rows, batch, heads, channel_decay);
-    if (rc != 0 || below <= 1 || rows - (batch - 1ll) * max_rows >= below) return rc;  // (no sequence can be shorter)
+    if (rc != 0 || below <= 1 || min_rows >= below || rows - (batch - 1ll) * max_rows >= below) return rc;  // (none is shorter)
   }
   dim3 grid((unsigned)(batch * heads), lq_ceil_div(P, cfg.cols));
   ScanShape sh = {heads, kv_heads, P, Dk, seq_slot, cu_rows};

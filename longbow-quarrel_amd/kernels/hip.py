@@ -20,7 +20,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 17  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 18  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -1002,12 +1002,13 @@ class HipKernels:
                  a_log: torch.Tensor, d_skip: torch.Tensor, state: torch.Tensor, y: torch.Tensor, heads: int,
                  head_dim: int, n_state: int, groups: int, seq_slot: torch.Tensor, cu_rows: torch.Tensor,
                  batch: int, max_rows: int = 0, workspace: Optional[torch.Tensor] = None,
-                 decay: Optional[torch.Tensor] = None, ones: bool = False, chunks: bool = False) -> None:
+                 decay: Optional[torch.Tensor] = None, ones: bool = False, chunks: bool = False, min_rows: int = 0) -> None:
         """The Mamba-2 recurrence along every sequence of the step, token by token: with dt = softplus(dt + dt_bias),
         S <- exp(-exp(a_log) dt) S + dt B x^T and y = S^T C + d_skip x per head; state [slots, heads, head_dim,
         n_state] is read and left at the step's end.  All float32.  `max_rows` (the most rows a sequence brings)
         and `workspace` (`ssd_scan_workspace(...)` floats) let a launch of few long sequences run in segments;
-        with `chunks` (and scratch asked for with the step's rows) long portions run in chunks of tokens.
+        with `chunks` (and scratch asked for with the step's rows) long portions run in chunks of tokens; `min_rows` (the
+        fewest rows a sequence brings, 0: unknown) spares the launch for short ones where there are none.
         `decay` [rows, heads]: a token's decay and step (`dt` as it is) are given, S <- decay S + dt B x^T, y = S^T C;
         dt_bias, a_log and d_skip are then None.  `ones`: head_dim counts one column more than x has for a head, the
         last, whose input is one (its result is the sum of the steps' B under the same decays, times C)."""
@@ -1036,7 +1037,7 @@ class HipKernels:
                                          c_int(ld(c_in, "C")), _ptr(dt), c_int(ld(dt, "dt")), _ptr(dt_bias), _ptr(a_log),
                                          _ptr(d_skip), _ptr(state), _ptr(y), c_int(ld(y, "y")), c_int(heads),
                                          c_int(head_dim), c_int(n_state), c_int(groups), _ptr(seq_slot), _ptr(cu_rows),
-                                         c_int(batch), c_int(max_rows if workspace is not None else 0), _ptr(workspace),
+                                         c_int(batch), c_int(max_rows if workspace is not None else 0), c_int(min_rows), _ptr(workspace),
                                          c_longlong(0 if workspace is None else workspace.numel()), _ptr(decay),
                                          c_int(0 if decay is None else ld(decay, "decay")), c_int(1 if ones else 0),
                                          c_int(rows if chunks else 0), self.stream))
@@ -1145,7 +1146,7 @@ class HipKernels:
                    dt_bias: torch.Tensor, a_log: torch.Tensor, state: torch.Tensor, out: torch.Tensor, heads: int,
                    kv_heads: int, key_dim: int, value_dim: int, q_scale: float, unit_eps: float,
                    seq_slot: torch.Tensor, cu_rows: torch.Tensor, batch: int, channel_decay: bool = False,
-                   max_rows: int = 0, workspace: Optional[torch.Tensor] = None) -> None:
+                   max_rows: int = 0, workspace: Optional[torch.Tensor] = None, min_rows: int = 0) -> None:
         """The gated delta rule along every sequence of the step, token by token: q and k made unit vectors per
         head (x / sqrt(sum x^2 + unit_eps)), q times q_scale, beta = sigmoid(beta), g = exp(-exp(a_log)
         softplus(a + dt_bias)); S <- g S, u = beta (v - S^T k), S <- S + k u^T, out = S^T q.  state [slots, heads,
@@ -1153,7 +1154,8 @@ class HipKernels:
         a head (a [rows, heads], dt_bias [heads]) or, with `channel_decay`, one for every key channel of every head
         (a [rows, heads * key_dim], dt_bias [heads * key_dim]), multiplying the state's rows of that channel.
         `max_rows` (the most rows that a sequence brings) and `workspace` (`delta_scan_workspace(...)` floats) let the
-        step's long portions run in chunks of tokens, whose sums are in another order."""
+        step's long portions run in chunks of tokens, whose sums are in another order; `min_rows` (the fewest, 0: unknown)
+        spares the launch for short ones where there are none."""
         rows = q.shape[0]
         n_decay = heads * key_dim if channel_decay else heads
         for t, what, cols in ((q, "q", kv_heads * key_dim), (k, "k", kv_heads * key_dim), (v, "v", heads * value_dim),
@@ -1177,7 +1179,7 @@ class HipKernels:
                                            c_int(ld(out, "out")), c_int(heads), c_int(kv_heads), c_int(key_dim),
                                            c_int(value_dim), c_float(q_scale), c_float(unit_eps), _ptr(seq_slot),
                                            _ptr(cu_rows), c_int(batch), c_int(rows), c_int(1 if channel_decay else 0),
-                                           c_int(max_rows), _ptr(workspace),
+                                           c_int(max_rows), c_int(min_rows), _ptr(workspace),
                                            c_longlong(0 if workspace is None else workspace.numel()), self.stream))
 
     def gated_rmsnorm(self, y: torch.Tensor, z: torch.Tensor, weight: Optional[torch.Tensor], eps: float, group: int,

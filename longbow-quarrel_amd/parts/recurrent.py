@@ -30,7 +30,7 @@ def _scan_scratch(ctx: StepContext, heads: int, head_dim: int, state: int) -> di
     chunks = ctx.dtype == torch.bfloat16 and ctx.kernels.ssd_scan_in_chunks(*sizes, ctx.rows)
     need = ask(*sizes, *((ctx.rows,) if chunks else ()))
     return dict(max_rows=ctx.max_new, workspace=ctx.ws.alloc((need,), torch.float32),
-                **({"chunks": True} if chunks else {})) if need else {}
+                **({"chunks": True, "min_rows": min(ctx.host_new, default=0)} if chunks else {})) if need else {}
 
 
 class _Recurrent(Mixer):
@@ -427,7 +427,8 @@ class GatedDelta(_Recurrent):
         ask = getattr(kn, "delta_scan_in_chunks", None) if ctx.dtype == torch.bfloat16 else None
         sizes = (rows, ctx.batch, nh, self.key_dim, self.value_dim, ctx.max_new)
         if ask is not None and ask(*sizes, self.channel_decay):
-            more.update(max_rows=ctx.max_new, workspace=ctx.ws.alloc((kn.delta_scan_workspace(*sizes),), torch.float32))
+            more.update(max_rows=ctx.max_new, min_rows=min(ctx.host_new, default=0),
+                        workspace=ctx.ws.alloc((kn.delta_scan_workspace(*sizes),), torch.float32))
         kn.delta_scan(qkv[:, : self.qk_width], qkv[:, self.qk_width : 2 * self.qk_width], qkv[:, 2 * self.qk_width :],
                       u[:, cc : cc + nh], decay, self.dt_bias, self.a_log, state, o, self.heads,
                       self.kv_heads, self.key_dim, self.value_dim, self.key_dim ** -0.5, self.UNIT_EPS,

@@ -130,7 +130,7 @@ def test_short_sequences_beside_a_long_one_are_walked(channel, least):
         n, at, B = sum(lens), sum(all_lens[:first]), len(lens)
         out, end = torch.full((n, H * P), float("nan"), device="cuda"), state[first : first + B].clone()
         part = lambda x: x[at : at + n].clone()
-        more = dict(max_rows=max(lens), workspace=torch.full((floats,), float("nan"), device="cuda")) if floats else {}
+        more = dict(max_rows=max(lens), min_rows=min(lens), workspace=torch.full((floats,), float("nan"), device="cuda")) if floats else {}
         kn.delta_scan(part(q), part(k), part(v), part(beta), part(a), dt_bias, a_log, end, out, H, G, N, P, N ** -0.5, 1e-6,
                       i32(range(B)), i32(sum(lens[:b]) for b in range(B + 1)), B, channel_decay=channel, **more)
         return out, end

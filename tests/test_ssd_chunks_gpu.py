@@ -131,7 +131,7 @@ def test_short_sequences_beside_a_long_one_are_walked():
         n, at, B = sum(mine), sum(lens[:first]), len(mine)
         y, end = torch.full((n, H * P), float("nan"), device="cuda"), state[first : first + B].clone()
         part = lambda t: t[at : at + n]
-        how = dict(max_rows=max(mine), workspace=torch.full((floats,), float("nan"), device="cuda"), chunks=True) if floats else {}
+        how = dict(max_rows=max(mine), min_rows=min(mine), workspace=torch.full((floats,), float("nan"), device="cuda"), chunks=True) if floats else {}
         kn.ssd_scan(part(x), part(b), part(c), part(dt), *made, end, y, H, P, N, G, i32(range(B)),
                     i32(sum(mine[:i]) for i in range(B + 1)), B, **how)
         return y, end
