@@ -338,38 +338,44 @@ __global__ __launch_bounds__(GM * GN * 64, 2) void gemm_bf16_pipelined_kernel(
   using S = PipeShape<GM, GN, WM, WN, BK, STAGES>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char plds[];
 
-  const int total = tiles_m * tiles_n;
-  int pid = blockIdx.x;
-  if (total % 8 == 0) pid = (pid % 8) * (total / 8) + pid / 8;  // one XCD walks a contiguous run of tiles
-  int tm = pid % tiles_m, tn = pid / tiles_m;
+  // A row tile of a group: `mine` tiles and `rows` rows are this lane's group's, `upto` and `rows_upto` those of the groups
+  // up to it.  The host does not know how many there are: the grid holds as many as there can be.
+  int rows = 0, mine = 0, upto = 0, rows_upto = 0;
   if constexpr (GROUPED) {
-    const int lane = threadIdx.x & 63, rows = lane < groups.n ? groups.counts[lane] : 0;
-    const int mine = (rows + S::BM - 1) / S::BM;
-    int upto = mine, rows_upto = rows;  // tiles and rows of the groups up to this lane's
+    const int lane = threadIdx.x & 63;
+    rows = rows_upto = lane < groups.n ? groups.counts[lane] : 0;
+    mine = upto = (rows + S::BM - 1) / S::BM;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const int t = __shfl_up(upto, off, 64), r = __shfl_up(rows_upto, off, 64);
       if (lane >= off) upto += t, rows_upto += r;
     }
-    const unsigned long long past = __ballot(upto > tm);
-    if (past == 0) return;  // (the whole workgroup: fewer tiles than there could have been)
-    const int at = __ffsll(past) - 1;
+    tiles_m = __builtin_amdgcn_readfirstlane(__shfl(upto, 63, 64));
+    if (blockIdx.x >= (unsigned)(tiles_m * tiles_n)) return;  // (the whole workgroup)
+  }
+  // Consecutive workgroups go to the 8 XCDs in turn, so that an XCD takes every eighth: it is given a contiguous run of the
+  // tiles' order (the first total % 8 XCDs one tile more).  The 32 tiles that an XCD works on together should share operands
+  // both ways (8 row tiles by 4 column tiles ask for 12 tiles' worth of operand rows, 32 row tiles of one column for
+  // 33): the order is bands of four columns, each band in windows of 8 row tiles (the last of a band has what is left).
+  // Where the tiles were no multiple of 8, neighbours used to land on different XCDs, each of which read the same weights:
+  // 128 x 64 tiles of 4 112 columns of K 2 048, 4 096 rows 165 -> 105 us; 64 x 64, 300 rows 19.2 -> 13.6.
+  const int total = tiles_m * tiles_n, xcd = blockIdx.x % 8;
+  const int pid = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+  int tm = pid % tiles_m, tn = pid / tiles_m;
+  if (tiles_m > 8) {
+    const int band = pid / (4 * tiles_m), in_band = pid % (4 * tiles_m), width = min(4, tiles_n - 4 * band);
+    const int whole = tiles_m / 8, window = min(in_band / (8 * width), whole);
+    const int in_window = in_band - window * 8 * width, height = window < whole ? 8 : tiles_m - 8 * whole;
+    tm = window * 8 + in_window % height;
+    tn = 4 * band + in_window / height;
+  }
+  if constexpr (GROUPED) {
+    const int at = __ffsll((unsigned long long)__ballot(upto > tm)) - 1;  // (the first group that reaches this tile)
     tm = __builtin_amdgcn_readfirstlane(tm - __shfl(upto - mine, at, 64));
     M = __builtin_amdgcn_readfirstlane(__shfl(rows, at, 64));
     const int first = __builtin_amdgcn_readfirstlane(__shfl(rows_upto - rows, at, 64));
     A += (long long)first * lda, C += (long long)first * ldc;
     W += __builtin_amdgcn_readfirstlane(at) * groups.w_step;
-  } else if (total % 8 == 0 && tiles_m > 8 && (total / 8) % tiles_m == 0) {
-    // The 32 tiles that an XCD works on together should share operands both ways: 8 row tiles by 4 column
-    // tiles ask for 12 tiles' worth of operand rows, 32 row tiles of one column tile for 33.  The XCD's run
-    // is whole columns of tiles: walk them four columns at a time, and each such band in windows of 8 row
-    // tiles (the last window of a band has what is left).
-    const int run = total / 8, cols = run / tiles_m, r = pid % run, first_col = (pid / run) * cols;
-    const int band = r / (4 * tiles_m), in_band = r % (4 * tiles_m), width = min(4, cols - 4 * band);
-    const int whole = tiles_m / 8, window = min(in_band / (8 * width), whole);
-    const int in_window = in_band - window * 8 * width, height = window < whole ? 8 : tiles_m - 8 * whole;
-    tm = window * 8 + in_window % height;
-    tn = first_col + 4 * band + in_window / height;
   }
   const int m0 = tm * S::BM, n0 = tn * S::BN;
   const int k_begin = blockIdx.y * k_share;
@@ -1029,25 +1035,11 @@ inline bool gemm_packable(int N, int K) {
   return N >= 8 * lq_compute_units() && N % 8 == 0 && K >= 512 && K % 64 == 0;
 }
 
-// The large pipelined tile pays once its tiles (times the shares of K) fill three quarters of the chip.
-inline bool fills_chip(long long blocks) { return blocks * 4 >= 3ll * lq_compute_units(); }
-
-// Shares of K for more than 64 rows: few tiles of 256 x 256 (a narrow weight matrix, a short prompt)
-// leave compute units idle; sharing K out over blocks fills them.
-int tiled_splits(int M, int N, int K) {
-  if (K % 64 != 0) return 1;
-  const long long t256 = (long long)lq_ceil_div(M, 256) * lq_ceil_div(N, 256);
-  int splits = 1;
-  while (splits < 8 && !fills_chip(t256 * splits) && K % (128 * splits) == 0 && K / (splits * 2) >= 1024) splits *= 2;
-  return splits;
-}
-
-// ---- 13 to 256 rows of a wide matrix: the weights are what is read, once, at the speed of the memory.
-// The pipelined kernel streams them best (transfers of three or four slabs in flight, no registers in
-// between) when its tile covers all rows, so that a weight is read once, and is narrow enough, with K shared
-// out over blocks, for about one block a compute unit: 64 x 128 (8 waves), 128 x 128 (8 waves) or 256 x 128
-// tiles (8 waves) of 4, 4 and 3 stages.  A product that must come out whole (16-bit out: its consumer adds no
-// pieces) and has few columns takes the 64- or 32-column sibling instead.
+// ---- 13 to 64 rows of a wide matrix: the weights are what is read, once, at the speed of the memory.
+// The pipelined kernel streams them best (transfers of four slabs in flight, no registers in between) when its
+// tile covers all rows, so that a weight is read once, and is narrow enough, with K shared out over blocks, for about one
+// block a compute unit: 64 x 128 (8 waves) or 64 x 64 tiles.  A product that must come out whole (16-bit out: its
+// consumer adds no pieces) and has few columns takes 64 x 64 or 64 x 32 tiles.
 // (from 13 rows: with packed weights the tiles stream as fast as the matrix-vector kernels, whose time grows
 // with every row beyond 8; 8B shape, a decoding step at batch 12 4.10 ms either way, at batch 16 4.30 -> 4.13, at
 // batch 24 4.55 -> 4.10, at batch 32 4.74 -> 4.25)
@@ -1058,7 +1050,7 @@ inline bool mid_rows(int M, int N, int K) {
   // (a head over a large vocabulary, a thousand tiles and more, stays with the matrix-vector kernel while one row
   // tile takes the rows: 1B shape at 16 rows 105 against 124 us)
   if (M <= 16 && N >= 128 * lq_compute_units()) return false;
-  return M > LQ_MID_ROWS_FROM && M <= 256 && K % 64 == 0 && K >= 512 && N >= 8 * lq_compute_units();
+  return M > LQ_MID_ROWS_FROM && M <= 64 && K % 64 == 0 && K >= 512 && N >= 8 * lq_compute_units();
 }
 
 inline int mid_splits_for(int tiles, int K) {
@@ -1074,8 +1066,7 @@ inline int mid_splits_for(int tiles, int K) {
 // what is left to gain: 8B shape at 64 rows, the norm after o and down 7.8 -> 6.9 us); where blocks are fewer
 // than compute units a block's bytes in flight bound it, and the wide tile has twice as many (q, k and v at 64
 // rows: 13.2 against 16.0 us).
-inline bool mid_narrow(int M, int N, int K) {
-  if (M > 64) return false;
+inline bool mid_narrow(int N, int K) {
   const int cus = lq_compute_units();
   const int wide = lq_ceil_div(N, 128) * mid_splits_for(lq_ceil_div(N, 128), K);
   const int narrow = lq_ceil_div(N, 64) * mid_splits_for(lq_ceil_div(N, 64), K);
@@ -1083,37 +1074,113 @@ inline bool mid_narrow(int M, int N, int K) {
   return (narrow < cus ? narrow : cus) > (wide < cus ? wide : cus) || (narrow >= cus && wide >= cus);
 }
 
-int mid_splits(int M, int N, int K) {
-  return mid_splits_for(lq_ceil_div(N, mid_narrow(M, N, K) ? 64 : 128), K);
+int mid_splits(int N, int K) {
+  return mid_splits_for(lq_ceil_div(N, mid_narrow(N, K) ? 64 : 128), K);
 }
 
 template <int EPI, typename TO>
 int launch_mid(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc, int splits,
                long long split_stride, hipStream_t stream, int packed) {
   // Whole and with few columns: 64- or 32-column tiles (a gated epilogue's pairs lie within 16 columns).
-  // Gated with 2 x 8192 columns of K 2048, 128-column tiles -> these: 17 rows 15.2 -> 13.7 us, 128 rows 22.2 -> 18.5, 200
-  // rows 34.8 -> 25.7; 2 x 4096 of K 1536: 17 rows 11.5 -> 9.1, 200 rows 28.4 -> 14.5.
+  // Gated with 2 x 8192 columns of K 2048, 128-column tiles -> these: 17 rows 15.2 -> 13.7 us; 2 x 4096 of K 1536: 11.5 -> 9.1.
   if constexpr (EPI != EPI_RESIDUAL) {
     const int want = 3 * lq_compute_units() / 4;
-    if (splits == 1 && lq_ceil_div(N, 64) < want) {
-      if (M <= 64) return launch_pipelined<2, 1, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-      if (M <= 128) return launch_pipelined<4, 1, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-      return launch_pipelined<8, 1, 1, 1, 64, 3, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-    }
-    if (splits == 1 && lq_ceil_div(N, 128) < want) {
-      if (M <= 64) return launch_pipelined<2, 2, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-      if (M <= 128) return launch_pipelined<2, 2, 2, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-      return launch_pipelined<4, 2, 2, 1, 64, 3, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-    }
+    if (splits == 1 && lq_ceil_div(N, 64) < want)
+      return launch_pipelined<2, 1, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
+    if (splits == 1 && lq_ceil_div(N, 128) < want)
+      return launch_pipelined<2, 2, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
   }
   if constexpr (EPI == EPI_NONE)
-    if (splits > 1 && mid_narrow(M, N, K))
+    if (splits > 1 && mid_narrow(N, K))
       return launch_pipelined<2, 2, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-  if (M <= 64)
-    return launch_pipelined<2, 4, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-  if (M <= 128)
-    return launch_pipelined<4, 2, 1, 2, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-  return launch_pipelined<4, 2, 2, 2, 64, 3, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+  return launch_pipelined<2, 4, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+}
+
+// ---- more rows, K in 64s: which tile, and in how many shares of K
+// Tiles run in rounds of one (or two, where two fit a compute unit's LDS) on every compute unit, and whether the last round
+// is full matters as much as how fast a tile is: 1 024 rows of 2 048 x 2 048 are 32 tiles of 256 x 256 (36 us), 128 of
+// 128 x 128 (20) or 256 of 128 x 64 (14), 2 048 rows of 4 112 columns are 200 of 256 x 192 (40 us) or 528 of 128 x 128 (63).
+// So a product asks what each tile would take: microseconds are
+//   fixed + slabs (per_round * rounds + per_layer * layers + per_fill * fill) + out_fill * fill,
+// slabs of 64 k, fill the tiles (times shares) a compute unit, rounds and layers how often all units are filled with as many as fit
+// and with one each.  The constants are least-squares fits to 19 sizes (1 024 to 14 336 columns of K 1 024 to 14 336) at 64 to
+// 4 096 rows and 1 to 8 shares, weights from memory; the fits are off by 6 to 9 % (r.m.s.), and the tile that they name takes
+// 0.2 % more than the best of the six on average, 17 % at most.  Against one rule for each range of rows (256 x 256, 256 x 192,
+// 128 x 128 and one covering tile up to 256 rows) the products take 0.79 of the time on average over these sizes whole, 0.72 in pieces
+// with their addition: 512 rows of 2 048 x 3 584 30.3 -> 15.9 us, 2 635 of 4 112 x 2 048 74 -> 45, 4 096 x 2 048 x 2 048 46 -> 36.
+struct TileTime {
+  int rows, cols, on_unit;  // on_unit: how many workgroups a compute unit holds (their LDS)
+  float fixed, per_round, per_layer, per_fill, out_fill;
+};
+enum { T256x256, T256x192, T256x128, T128x128, T128x64, T64x64, TILES };
+constexpr TileTime tile_times[TILES] = {
+    {256, 256, 1, 4.30f, 0.985f, 0.f, 0.325f, 10.59f}, {256, 192, 1, 3.19f, 0.800f, 0.f, 0.243f, 8.45f},
+    {256, 128, 1, 2.66f, 0.655f, 0.f, 0.221f, 5.73f},  {128, 128, 1, 2.64f, 0.468f, 0.f, 0.101f, 3.23f},
+    {128, 64, 2, 2.33f, 0.123f, 0.172f, 0.082f, 1.34f}, {64, 64, 2, 2.48f, 0.108f, 0.099f, 0.042f, 0.88f}};
+
+float tile_us(int tile, long long tiles, int K, int splits) {
+  const TileTime& t = tile_times[tile];
+  const int cus = lq_compute_units();
+  const long long n = tiles * splits;
+  const float fill = (float)n / cus, slabs = K / 64 / splits;
+  return t.fixed + slabs * (t.per_round * lq_ceil_div64(n, (long long)cus * t.on_unit) + t.per_layer * lq_ceil_div64(n, cus) + t.per_fill * fill) +
+         t.out_fill * fill;
+}
+
+float product_us(int tile, int M, int N, int K, int splits) {
+  return tile_us(tile, (long long)lq_ceil_div(M, tile_times[tile].rows) * lq_ceil_div(N, tile_times[tile].cols), K, splits);
+}
+
+int best_tile(int M, int N, int K, int splits) {
+  int best = 0;
+  for (int t = 1; t < TILES; ++t)
+    if (product_us(t, M, N, K, splits) < product_us(best, M, N, K, splits)) best = t;
+  return best;
+}
+
+// From 65 rows, or 17 of a weight too narrow for the kernels that stream a wide one (40 rows of 1 536 x 1 536 8.8 -> 7.7 us, in four
+// pieces 4.2; of 1 024 x 3 584 15.6 -> 14.2 and 5.8).
+inline bool takes_rows(int M, int N, int K) {
+  return K % 64 == 0 && K >= 512 && (M > 64 || (M > 16 && N < 8 * lq_compute_units()));
+}
+
+// Shares of K: as many as make the product (whose time has the writing of its pieces) and the reading of the further pieces, 4
+// bytes an entry at the 6 TB/s at which a norm reads, fastest.
+int tiled_splits(int M, int N, int K) {
+  int best = 1;
+  float least = 0.f;
+  for (int s = 1; s <= 8 && K % (64 * s) == 0 && K / s >= 256; s *= 2) {
+    const float us = product_us(best_tile(M, N, K, s), M, N, K, s) + (s - 1) * (0.3f + 4.f * M * N / 6e6f);
+    if (s == 1 || us < 0.97f * least) best = s, least = us;  // (a tie goes to fewer pieces)
+  }
+  return best;
+}
+
+template <int EPI, typename TO>
+int launch_rows(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc, int splits,
+                long long split_stride, hipStream_t stream, int packed, bool whole_rounds = true) {
+  const int tile = best_tile(M, N, K, splits);
+  // Whole rounds of 256-column tiles, and the columns that are left in a launch of their own with the tile that suits them, where
+  // that wins by more than the estimate is off (2 048 x 28 672: three rounds and 256 tiles of 256 x 128 instead of 3.5 rounds).
+  const int tm = lq_ceil_div(M, 256), n1 = lq_ceil_div(N, 256) * tm / lq_compute_units() * lq_compute_units() / tm * 256;
+  if (whole_rounds && splits == 1 && n1 > 0 && n1 < N) {
+    const float two = product_us(T256x256, M, n1, K, 1) + product_us(best_tile(M, N - n1, K, 1), M, N - n1, K, 1);
+    if (two < 0.95f * product_us(tile, M, N, K, 1)) {
+      const int col2 = is_glu(EPI) ? n1 / 2 : n1;  // where the second launch's columns start in out
+      int rc = launch_pipelined<4, 2, 2, 4, 64, 2, EPI, TO, true>(x, w, out, M, n1, K, lda, ldw, ldc, 1, 0, stream, packed);
+      if (rc != 0) return rc;
+      return launch_rows<EPI, TO>(x, (const bf16_t*)w + (long long)n1 * ldw, (TO*)out + col2, M, N - n1, K, lda, ldw, ldc, 1, 0,
+                                  stream, packed, false);
+    }
+  }
+  switch (tile) {
+    case T256x256: return launch_pipelined<4, 2, 2, 4, 64, 2, EPI, TO, true>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+    case T256x192: return launch_pipelined<4, 2, 2, 3, 64, 2, EPI, TO, true>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+    case T256x128: return launch_pipelined<4, 2, 2, 2, 64, 2, EPI, TO, true>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+    case T128x128: return launch_pipelined<4, 2, 1, 2, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+    case T128x64: return launch_pipelined<4, 2, 1, 1, 64, 3, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+    default: return launch_pipelined<2, 2, 1, 1, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+  }
 }
 
 // Shares of K for up to 16 rows of a weight with so few columns that its tiles of 16 leave most of the chip idle and
@@ -1128,8 +1195,8 @@ int narrow_splits(int M, int N, int K) {
 }
 
 int mfma_splits(int M, int N, int K) {
-  if (mid_rows(M, N, K)) return mid_splits(M, N, K);
-  return M <= 64 ? v3_splits(M, N, K) : tiled_splits(M, N, K);
+  if (mid_rows(M, N, K)) return mid_splits(N, K);
+  return takes_rows(M, N, K) ? tiled_splits(M, N, K) : v3_splits(M, N, K);
 }
 
 template <int EPI, typename TO>
@@ -1149,11 +1216,10 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
     }
   }
   if (mid_rows(M, N, K)) return launch_mid<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+  if (takes_rows(M, N, K)) return launch_rows<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   if (splits > 1) {
     if (M <= 32) return launch_skinny_v3<2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-    if (M <= 64) return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-    return launch_pipelined<4, 2, 2, 4, 64, 2, EPI, TO, true>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride,
-                                                              stream, packed);
+    return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   }
   // wide enough to give every compute unit a run of columns: the balanced kernel; else the simple one
   const bool wide = N >= 8 * lq_compute_units() && K >= 512;
@@ -1169,43 +1235,10 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
     if (wide) return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
     return pick_skinny<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, stream);
   }
-  // the largest tile that still fills the chip: 256 rows by 256, 224 or 192 columns (8 waves), 128 x 256
-  // (4 waves, pipelined), then the register-staged kernels, which also take a K that is no multiple of 32
-  const long long t256 = (long long)lq_ceil_div(M, 256) * lq_ceil_div(N, 256);
+  // a K that is no multiple of 64, or a short one: slabs of 32 k, then the register-staged kernels, which take any K
   const long long t128 = (long long)lq_ceil_div(M, 128) * lq_ceil_div(N, 256);
-  if (K % 64 == 0 && fills_chip(t256)) {
-    // Tiles run in rounds of one a compute unit; a narrower tile can save a round or fill a round that
-    // a wider one leaves part empty.  Cost of a round relative to the 256-column tile, as measured.
-    const int cus = lq_compute_units(), tm = lq_ceil_div(M, 256);
-    // (A last round that is part empty costs less than a whole one, which the rounding up does not know: a
-    // narrower tile has to win by a margin.)
-    const double c256 = 0.95 * lq_ceil_div(tm * lq_ceil_div(N, 256), cus);
-    const double c224 = 1.13 * lq_ceil_div(tm * lq_ceil_div(N, 224), cus);
-    const double c192 = 0.78 * lq_ceil_div(tm * lq_ceil_div(N, 192), cus);
-    if (c256 <= c224 && c256 <= c192) {
-      // Whole rounds of 256-column tiles, and where what is left would fill half a round or less, that rest
-      // as 128-column tiles in a launch of its own: a round of half-size tiles instead of a round of whole
-      // tiles on half the chip (2 048 x 28 672: three rounds and 256 half tiles instead of 3.5 rounds).
-      const int tn = lq_ceil_div(N, 256), rest = (tm * tn) % cus;
-      if (N % 256 == 0 && tm * tn > cus && 4 * rest >= cus && rest % tm == 0 && 2 * rest <= cus + cus / 8) {
-        const int n1 = (tn - rest / tm) * 256, n2 = N - n1;
-        const int col2 = is_glu(EPI) ? n1 / 2 : n1;  // where the second launch's columns start in out
-        int rc = launch_pipelined<4, 2, 2, 4, 64, 2, EPI, TO, true>(x, w, out, M, n1, K, lda, ldw, ldc, 1, 0, stream, packed);
-        if (rc != 0) return rc;
-        return launch_pipelined<4, 2, 2, 2, 64, 2, EPI, TO, true>(x, (const bf16_t*)w + (long long)n1 * ldw,
-                                                                  (TO*)out + col2, M, n2, K, lda, ldw, ldc, 1, 0, stream, packed);
-      }
-      return launch_pipelined<4, 2, 2, 4, 64, 2, EPI, TO, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-    }
-    if (c224 <= c192)
-      return launch_pipelined<8, 1, 1, 7, 64, 2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-    return launch_pipelined<4, 2, 2, 3, 64, 2, EPI, TO, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-  }
-  if (!packed && K % 32 == 0 && t128 >= lq_compute_units())
+  if (K % 32 == 0 && t128 >= lq_compute_units())
     return launch_pipelined<2, 2, 2, 4, 32, 3, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
-  // few tiles even of 128 x 256 (some hundred rows of a narrow matrix): 128 x 128 tiles, four stages deep
-  if (K % 64 == 0 && K >= 512)
-    return launch_pipelined<4, 2, 1, 2, 64, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
   if (t128 >= 2 * lq_compute_units()) return launch_tiled<2, 4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, stream);
   return launch_tiled<2, 2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, stream);
 }
@@ -1274,13 +1307,21 @@ bool lq_gemm_packable(int N, int K) { return gemm_packable(N, K); }
 int lq_gemm_grouped(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc,
                     const int* counts, int groups, long long w_step, int packed, hipStream_t stream) {
   const Groups g = {counts, groups, w_step};
-  // 256-row tiles from 256 rows an expert on; fewer leave most of such a tile empty.  Microseconds, 8 experts, a launch an
-  // expert / 128 x 128 tiles / 256 x 256 tiles: 1 024 rows of 3 584 x 2 048 108 / 42 / 42, of 2 048 x 3 584 166 / 36 / 61;
-  // 2 048 rows 142 / 65 / 46 and 219 / 67 / 65; 8 002 rows 186 / 190 / 151 and 242 / 178 / 151; 8 192 rows of
-  // 14 336 x 4 096 1 023 / 1 294 / 886.
-  if (M / groups >= 256)
-    return launch_pipelined<4, 2, 2, 4, 64, 2, EPI_NONE, float, true, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
-  return launch_pipelined<4, 2, 1, 2, 64, 4, EPI_NONE, float, false, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+  // The tile by what it would take with half a tile a group more than the rows come to.  Microseconds, 8 groups,
+  // one rule by rows a group (256 x 256 or 128 x 128) -> this: 500 rows of 3 584 x 2 048 44 -> 29, 4 000 rows 98 -> 90, 8 002 rows
+  // 151 -> 116, 4 000 rows of 2 048 x 3 584 85 -> 73; 5 272 rows of 5 120 x 2 048 116 either way, 1 024 of 2 048 x 3 584 42 -> 44.
+  int best = T256x256;
+  float least = 0.f;
+  for (int t = T256x256; t <= T128x128; ++t) {
+    const float us = tile_us(t, ((long long)M / tile_times[t].rows + (groups + 1) / 2) * lq_ceil_div(N, tile_times[t].cols), K, 1);
+    if (t == T256x256 || us < least) best = t, least = us;
+  }
+  switch (best) {
+    case T256x256: return launch_pipelined<4, 2, 2, 4, 64, 2, EPI_NONE, float, true, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+    case T256x192: return launch_pipelined<4, 2, 2, 3, 64, 2, EPI_NONE, float, true, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+    case T256x128: return launch_pipelined<4, 2, 2, 2, 64, 2, EPI_NONE, float, true, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+    default: return launch_pipelined<4, 2, 1, 2, 64, 4, EPI_NONE, float, false, true>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed, g);
+  }
 }
 
 int lq_gemm_mfma(const void* x, const void* w, void* out, int out_dtype, int M, int N, int K, int lda,
