@@ -998,6 +998,8 @@ struct Branches {
   const float* y[4];
   const float* w[4];  // (null: one branch, taken as it is)
   const float* b[4];  // null: no bias
+  int pieces;         // of a branch taken as it is: as many rows x width pieces behind y[0], `apart` entries each, are its sum
+  long long apart;
 };
 
 template <typename T, int PER>
@@ -1007,10 +1009,11 @@ __global__ __launch_bounds__(256) void branches_residual_kernel(float* __restric
   __shared__ float red[16];
   const long long base = (long long)blockIdx.x * width;
   const int quads = width / 4;
-  embed_f32x4 xv[PER], y[PER], one[PER];
+  embed_f32x4 xv[PER], y[PER], one[PER], gain[PER];  // (all asked for ahead of the sums, whose barriers no load passes)
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int q = threadIdx.x + i * 256;
+    gain[i] = q < quads ? ((const embed_f32x4*)w)[q] : (embed_f32x4){0.f, 0.f, 0.f, 0.f};
     one[i] = q < quads ? ((const embed_f32x4*)(in.y[0] + base))[q] : (embed_f32x4){0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
@@ -1042,6 +1045,12 @@ __global__ __launch_bounds__(256) void branches_residual_kernel(float* __restric
       }
     }
   }
+  for (int p = 1; p < in.pieces; ++p)  // in their order
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int q = threadIdx.x + i * 256;
+      if (q < quads) y[i] += ((const embed_f32x4*)(in.y[0] + p * in.apart + base))[q];
+    }
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < PER; ++i)
@@ -1052,7 +1061,7 @@ __global__ __launch_bounds__(256) void branches_residual_kernel(float* __restric
   for (int i = 0; i < PER; ++i) {
     const int q = threadIdx.x + i * 256;
     if (q >= quads) continue;
-    const embed_f32x4 v = xv[i] + y[i] * inv * ((const embed_f32x4*)w)[q];
+    const embed_f32x4 v = xv[i] + y[i] * inv * gain[i];
     ((embed_f32x4*)(x + base))[q] = v;
     if (rounded != nullptr) {
       if constexpr (sizeof(T) == 2) {
@@ -1270,7 +1279,7 @@ extern "C" int lq_mean_residual(float* x, const float* stack, int n_in, const fl
   LQ_REQUIRE(x && stack && w, "mean_residual: null pointer");
   const float* ws[4] = {w0, w1, w2, w3};
   const float* bs[4] = {b0, b1, b2, b3};
-  Branches in;
+  Branches in = {};
   for (int i = 0; i < 4; ++i) {
     in.y[i] = i < n_in ? stack + (long long)i * rows * width : nullptr;
     in.w[i] = i < n_in ? ws[i] : nullptr, in.b[i] = i < n_in ? bs[i] : nullptr;
@@ -1282,15 +1291,17 @@ extern "C" int lq_mean_residual(float* x, const float* stack, int n_in, const fl
   return launch_branches(x, in, n_in, branch_eps, w, eps, rounded, rounded_dtype, rows, width, stream);
 }
 
-extern "C" int lq_rmsnorm_residual(float* x, const float* y, const float* w, float eps, void* rounded, int rounded_dtype,
+// y [pieces, rows, width]: their sum is meant; more than one where lq_mean_residual_accepts the width.
+extern "C" int lq_rmsnorm_residual(float* x, const float* y, int pieces, const float* w, float eps, void* rounded, int rounded_dtype,
                                    int rows, int width, hipStream_t stream) {
-  LQ_REQUIRE(rows > 0 && width > 0, "rmsnorm_residual: rows %d and width %d must be positive", rows, width);
+  LQ_REQUIRE(rows > 0 && width > 0 && pieces >= 1, "rmsnorm_residual: rows %d, width %d and %d pieces must be positive", rows, width, pieces);
   LQ_REQUIRE(x && y && w, "rmsnorm_residual: null pointer");
   if (branches_fit(x, rounded, rounded_dtype, width) && (uintptr_t)y % 16 == 0 && (uintptr_t)w % 16 == 0) {
     Branches in = {};
-    in.y[0] = y;
+    in.y[0] = y, in.pieces = pieces, in.apart = (long long)rows * width;
     return launch_branches(x, in, 1, 0.f, w, eps, rounded, rounded_dtype, rows, width, stream);
   }
+  LQ_REQUIRE(pieces == 1, "rmsnorm_residual: pieces have columns in fours on 16 bytes, at most 8192 of them");
   if (rounded == nullptr || rounded_dtype == LQ_F32)
     rmsnorm_residual_kernel<float><<<rows, 256, 0, stream>>>(x, y, w, eps, (float*)rounded, width);
   else if (rounded_dtype == LQ_BF16)

@@ -33,7 +33,7 @@ extern "C" int lq_linear_narrow_splits(int in_dtype, int M, int N, int K, int fo
 }
 
 // Whether a bfloat16 weight [N, K] may be handed to the products packed (lq_pack_weight): only where every
-// kernel that can meet it reads that layout.  `w_packed` below says that w is; its ldw is then K.
+// kernel that can meet it reads that layout.  `w_packed` below says that w is; its ldw is then the whole matrix's K.
 extern "C" int lq_weight_packable(int dtype, int N, int K) { return dtype == LQ_BF16 && lq_gemm_packable(N, K); }
 
 extern "C" int lq_linear(const void* x, const void* w, void* out, int in_dtype, int out_dtype,
@@ -43,7 +43,8 @@ extern "C" int lq_linear(const void* x, const void* w, void* out, int in_dtype, 
   LQ_REQUIRE(lda >= K && ldw >= K && ldc >= N, "linear: a row stride is smaller than its row");
   LQ_REQUIRE(x && w && out, "linear: null pointer");
   LQ_REQUIRE(splits >= 1 && (splits == 1 || split_stride >= (long long)M * ldc), "linear: bad split arguments");
-  LQ_REQUIRE(!w_packed || (ldw == K && lq_weight_packable(in_dtype, N, K)), "linear: this weight cannot be packed");
+  // (a packed weight's ldw is the whole matrix's K, a multiple of 64, where w is a run of its columns)
+  LQ_REQUIRE(!w_packed || (ldw % 64 == 0 && lq_weight_packable(in_dtype, N, K)), "linear: this weight cannot be packed");
   if (!force_generic && lq_gemm_mfma_accepts(x, w, in_dtype, K, lda, ldw))
     return lq_gemm_mfma(x, w, out, out_dtype, M, N, K, lda, ldw, ldc, 0, splits, split_stride, w_packed, stream);
   LQ_REQUIRE(splits == 1, "linear: only the matrix-core kernels split K");
@@ -68,7 +69,9 @@ extern "C" int lq_linear_grouped(const void* x, const void* w, void* out, int in
   LQ_REQUIRE(lq_linear_grouped_supported(in_dtype, groups, N, K, 0) && lq_gemm_mfma_accepts(x, w, in_dtype, K, lda, ldw) &&
                  w_step % 8 == 0,
              "linear_grouped: %d experts of [%d, %d] are not taken", groups, N, K);
-  LQ_REQUIRE(!w_packed || (ldw == K && N % 8 == 0 && w_step % (8ll * K) == 0), "linear_grouped: these weights are not packed rows in eights");
+  // (packed rows of one matrix, or packed columns: runs of 64 of them lie 512 entries apart)
+  LQ_REQUIRE(!w_packed || (N % 8 == 0 && ldw % 64 == 0 && (ldw == K ? w_step % (8ll * K) == 0 : w_step % 512 == 0)),
+             "linear_grouped: these weights are not packed rows in eights or columns in 64s");
   return lq_gemm_grouped(x, w, out, M, N, K, lda, ldw, ldc, counts, groups, w_step, w_packed, stream);
 }
 

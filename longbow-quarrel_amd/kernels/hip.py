@@ -86,9 +86,11 @@ class PackedWeight:
 
     packed = True
 
-    def __init__(self, data: torch.Tensor, rows: int, cols: int) -> None:
+    def __init__(self, data: torch.Tensor, rows: int, cols: int, whole: Optional[int] = None) -> None:
+        """`data` begins at the weight's first entry; `whole`: the columns of the matrix that it is a run of columns of."""
         self.data, self.shape, self.dtype, self.device = data, torch.Size((rows, cols)), data.dtype, data.device
         self.is_cuda = data.is_cuda
+        self.whole = cols if whole is None else whole
 
     def data_ptr(self) -> int:
         return self.data.data_ptr()
@@ -97,17 +99,17 @@ class PackedWeight:
         return 2
 
     def stride(self, i: Optional[int] = None):
-        st = (self.shape[1], 1)
+        st = (self.whole, 1)
         return st if i is None else st[i]
 
     def is_contiguous(self) -> bool:
-        return True
+        return self.whole == self.shape[1]
 
     def contiguous(self) -> "PackedWeight":
         return self
 
     def numel(self) -> int:
-        return self.data.numel()
+        return self.shape.numel()
 
     def element_size(self) -> int:
         return self.data.element_size()
@@ -1282,16 +1284,18 @@ class HipKernels:
     def rmsnorm_residual(self, x: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float,
                          rounded: Optional[torch.Tensor] = None) -> None:
         """x += y / sqrt(mean(y^2) + eps) * weight, row by row (x and y float32); `rounded`, where given, takes the
-        new x in its own dtype."""
+        new x in its own dtype.  y may hold several pieces [pieces, rows, width] whose sum is meant, where
+        `mean_residual_takes` the width."""
         self._dev(x, y, weight, rounded)
         rows, width = x.shape
-        if x.dtype != torch.float32 or y.dtype != torch.float32 or tuple(y.shape) != (rows, width) \
+        pieces = y.shape[0] if y.dim() == 3 else 1
+        if x.dtype != torch.float32 or y.dtype != torch.float32 or tuple(y.shape[-2:]) != (rows, width) \
                 or not x.is_contiguous() or not y.is_contiguous():
-            raise KernelLibraryError("rmsnorm_residual: x and y must be dense float32 of one shape")
+            raise KernelLibraryError("rmsnorm_residual: x and y must be dense float32 of one shape (y may come in pieces)")
         self._f32(weight, "rmsnorm_residual: weight", width)
         if rounded is not None and (tuple(rounded.shape) != (rows, width) or not rounded.is_contiguous()):
             raise KernelLibraryError("rmsnorm_residual: rounded must be dense and shaped like x")
-        self._check(self.lib.lq_rmsnorm_residual(_ptr(x), _ptr(y), _ptr(weight), c_float(eps), _ptr(rounded),
+        self._check(self.lib.lq_rmsnorm_residual(_ptr(x), _ptr(y), c_int(pieces), _ptr(weight), c_float(eps), _ptr(rounded),
                                                  c_int(_code(rounded) if rounded is not None else 0), c_int(rows),
                                                  c_int(width), self.stream))
 
@@ -1662,6 +1666,62 @@ class HipKernels:
                                         c_int(rows), c_int(experts), c_int(ff), c_int(shared),
                                         c_int(self._ACTIVATIONS[activation]), self.stream))
 
+    @query
+    def moe_few_supported(self, dtype: torch.dtype, rows: int, experts: int, ff: int, shared: int, width: int) -> bool:
+        """Whether `moe_few` takes a mixture of `experts` of `ff` columns (and one of `shared`) over so few rows."""
+        if self.force_generic or dtype not in _DTYPE_CODE:
+            return False
+        return bool(self.lib.lq_moe_few_supported(c_int(_DTYPE_CODE[dtype]), c_int(rows), c_int(experts), c_int(ff),
+                                                  c_int(shared), c_int(width)))
+
+    @query
+    def moe_few_pieces(self, width: int) -> int:
+        """In how many pieces `moe_few` likes to leave its result (1, 2 or 4)."""
+        return int(self.lib.lq_moe_few_pieces(c_int(width)))
+
+    _FEW_UNITS = {"clamped_swish": 0, "silu": 1, "relu2": 2}
+
+    def moe_few(self, h: torch.Tensor, w_in, w_out: torch.Tensor, route: torch.Tensor, act: torch.Tensor, out: torch.Tensor,
+                ff: int, shared: int, activation: str, limit: float = 0.0, on_input: bool = False,
+                shared_gate: Optional[torch.Tensor] = None, passed: Optional[torch.Tensor] = None) -> None:
+        """out (float32 [rows, width], or [pieces, rows, width] that sum to it) = the mixture over the rows of h, whose experts' weights (or -1) are in route [rows, experts], reading the
+        chosen experts' matrices alone.  w_in: the rows of every expert's gate and up matrices one behind the other (up alone
+        for "relu2"), the shared expert's last; w_out [width, experts * ff + shared]; act: scratch [rows, that many]
+        in the dtype of h.  `on_input`: the weight multiplies what an expert reads; `shared_gate` [rows, 1]: the logit of
+        a gate on the shared expert; `passed` [rows, n]: identity experts' weights, which multiply h itself."""
+        rows, width, ldh = self._mat(h, "moe_few: h")
+        nin, kin, ldi = self._mat(w_in, "moe_few: w_in")
+        nout, kout, ldw = self._mat(w_out, "moe_few: w_out")
+        ra, na, lda = self._mat(act, "moe_few: act")
+        pieces = out.shape[0] if out.dim() == 3 else 1
+        ro, no, ldo = self._mat(out[0] if out.dim() == 3 else out, "moe_few: out")
+        experts = route.shape[1]
+        inner = experts * ff + shared
+        self._f32(route, "moe_few: route", rows * experts)
+        if activation not in self._FEW_UNITS or nin != inner * (1 if activation == "relu2" else 2) or (kin, nout, kout) != (width, width, inner) \
+                or (ra, na, ro, no) != (rows, inner, rows, width) or out.dtype != torch.float32 \
+                or not h.dtype == w_in.dtype == w_out.dtype == act.dtype == torch.bfloat16 or tuple(route.shape) != (rows, experts):
+            raise KernelLibraryError("moe_few: h [rows, width], w_in, w_out [width, experts * ff + shared], route [rows, experts], "
+                                     "act [rows, experts * ff + shared] (bfloat16), out float32 [rows, width]")
+        ldg = 0
+        if shared_gate is not None:
+            ldg = self._mat(shared_gate, "moe_few: shared_gate")[2]
+            if tuple(shared_gate.shape) != (rows, 1) or shared_gate.dtype != torch.float32:
+                raise KernelLibraryError("moe_few: the shared expert's gate is float32 [rows, 1]")
+        if passed is not None:
+            self._f32(passed, "moe_few: passed")
+            if passed.dim() != 2 or passed.shape[0] != rows or not passed.is_contiguous():
+                raise KernelLibraryError("moe_few: identity experts' weights are dense [rows, n]")
+        self._check(self.lib.lq_moe_few_first(_ptr(h), c_int(ldh), _ptr(w_in), c_int(ldi), c_int(_packed(w_in)), _ptr(route), _ptr(act),
+                                              c_int(lda), c_int(rows), c_int(experts), c_int(ff), c_int(shared), c_int(width),
+                                              c_int(self._FEW_UNITS[activation]), c_float(limit), c_int(1 if on_input else 0),
+                                              _ptr(shared_gate), c_int(ldg), self.stream))
+        self._check(self.lib.lq_moe_few_second(_ptr(act), c_int(lda), _ptr(w_out), c_int(ldw), c_int(_packed(w_out)), _ptr(route),
+                                               _ptr(out), c_int(ldo), c_int(pieces),
+                                               c_longlong(out.stride(0) if pieces > 1 else 0), c_int(rows), c_int(experts), c_int(ff), c_int(shared), c_int(width), _ptr(h),
+                                               c_int(ldh), _ptr(passed), c_int(passed.shape[1] if passed is not None else 0),
+                                               self.stream))
+
     def weight_rows(self, w, start: int, n: int):
         """Rows start .. start + n of a product weight as a weight of its own: a view of a dense one; of a packed
         one the same run of its memory, where the rows are whole groups of eight and a matrix of that size is
@@ -1673,6 +1733,18 @@ class HipKernels:
                 not self.lib.lq_weight_packable(c_int(_DTYPE_CODE[w.dtype]), c_int(n), c_int(k)):
             return None
         return PackedWeight(w.data.view(-1)[start * k : (start + n) * k].view(n, k), n, k)
+
+    def weight_columns(self, w, start: int, n: int):
+        """Columns start .. start + n of a product weight as a weight of its own: a view of a dense one; of a packed one
+        the same runs of its memory, where they are whole runs of 64 and a matrix of that size is packed at all (else
+        None)."""
+        if not getattr(w, "packed", False):
+            return w[:, start : start + n]
+        rows, k = w.shape
+        if start % 64 or n % 64 or start + n > k or w.whole != k or \
+                not self.lib.lq_weight_packable(c_int(_DTYPE_CODE[w.dtype]), c_int(rows), c_int(n)):
+            return None
+        return PackedWeight(w.data.view(-1)[start * 8 :], rows, n, whole=k)
 
     def moe_sort(self, route: torch.Tensor, counts: torch.Tensor, order: torch.Tensor, weight: torch.Tensor,
                  place_of: torch.Tensor, fill: bool = False) -> None:

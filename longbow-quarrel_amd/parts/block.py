@@ -212,8 +212,15 @@ class OutputNormBlock(Block):
 
     @staticmethod
     def _run(part, args, ctx: StepContext, width: int) -> torch.Tensor:
-        """A sublayer's result, whole [rows, width] in 32-bit."""
+        """A sublayer's result in 32-bit: whole [rows, width], or in pieces that the norm adds up."""
         rows = args[0].shape[0]
+        in_pieces, takes = getattr(part, "forward_pieces", None), getattr(ctx.kernels, "mean_residual_takes", None)
+        if in_pieces is not None and takes is not None and takes(width):
+            got, scales = in_pieces(*args)
+            for piece, scale in zip(got if got.dim() == 3 else got[None], scales):
+                if scale != 1.0:
+                    ctx.kernels.scale(piece, scale)
+            return got[0] if got.dim() == 3 and got.shape[0] == 1 else got
         if part.takes_out:
             out = ctx.ws.alloc((rows, width), torch.float32)
             part.forward(*args, out=out)

@@ -222,8 +222,9 @@ class MixtureOfExperts(FeedForward):
 
     How it runs.  The experts' gate and up matrices are one matrix [experts * 2 ff, width] and their down matrices
     one [width, experts * ff]: with the activations of the experts that a token did not choose set to zero, the down
-    product adds the chosen experts' results by itself.  A step of few rows (decoding) runs every row through all
-    experts' columns: a batch of more than a few tokens reads nearly all experts anyway.  A prompt step of
+    product adds the chosen experts' results by itself.  Up to 16 rows (decoding)
+    go through two launches that read the matrices of the chosen experts alone (`moe_few`); where the kernels do not take
+    the sizes, and up to `sort_from_rows`, every row runs through all experts' columns.  A prompt step of
     `sort_from_rows` rows or more is sorted by expert first (`moe_sort`: the chosen (row, expert) couples expert by
     expert, rows ascending), the rows gathered in that order, and every expert's two products run over its own rows
     only, all experts' in one launch that finds the row counts on the device; the results go back to their rows and are
@@ -329,11 +330,16 @@ class MixtureOfExperts(FeedForward):
             if any(w is None for w in self.gate_up_of):
                 self.w_gate_up = whole
                 self.gate_up_of = [whole[at : at + n] for at, n in runs]
-        # the second matrix stays dense: an expert is a run of its columns, which only the dense order can give
-        self.w_down = torch.cat(down, dim=1).contiguous()  # [width, E * ff (+ ffs)]
-        self.down_of = [self.w_down[:, e * ff : (e + 1) * ff] for e in range(E)]
-        if ffs:
-            self.down_of.append(self.w_down[:, E * ff :])
+        # an expert is a run of the second matrix's columns, which must be a weight in the matrix's order too
+        whole = torch.cat(down, dim=1).contiguous()  # [width, E * ff (+ ffs)]
+        runs = [(e * ff, ff) for e in range(E)] + ([(E * ff, ffs)] if ffs else [])
+        self.w_down = product_weight(env, whole)
+        columns_of = getattr(env.kernels, "weight_columns", None)
+        if self.w_down is not whole:
+            self.down_of = [columns_of(self.w_down, at, n) if columns_of else None for at, n in runs]
+        if self.w_down is whole or any(w is None for w in self.down_of):
+            self.w_down = whole
+            self.down_of = [whole[:, at : at + n] for at, n in runs]
         if self.correction:
             self.w_correction = tensors[f"{self.prefix}.{self.n['correction']}"].contiguous()
         # the router's product as it is stored: bfloat16 operands multiply exactly into 32-bit sums, and its result
@@ -372,6 +378,13 @@ class MixtureOfExperts(FeedForward):
         self._step = (passed, z[:, N:] if self.shared_gate else None)
         return route
 
+    def _few(self, h, ctx: StepContext) -> bool:
+        """Whether the kernels take the step's rows through the chosen experts' weights alone."""
+        ask = getattr(ctx.kernels, "moe_few_supported", None)
+        return ask is not None and h.dtype == self.w_gate_up.dtype == self.w_down.dtype == ctx.dtype \
+            and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 \
+            and ask(h.dtype, h.shape[0], self.experts, self.inner, self.shared_inner, self.width)
+
     def _pass_on(self, h, out, ctx: StepContext) -> None:
         """The identity experts' share: out += h * (the sum of the chosen identity experts' weights)."""
         passed = self._step[0]
@@ -396,7 +409,7 @@ class MixtureOfExperts(FeedForward):
         """The result in pieces [n, rows, width] that the caller adds: the routed experts' sum, and the shared
         expert's result where a step's rows were sorted by expert (otherwise one product adds both)."""
         rows = h.shape[0]
-        if not self._sorts(rows, ctx) and not self.gated:
+        if not self._sorts(rows, ctx) and (not self.gated or self._few(h, ctx)):
             out = self.forward(h, ctx)  # (whole, or in the pieces that its last product leaves)
             return out, (1.0,) * (out.shape[0] if out.dim() == 3 else 1)
         if not (self.shared_inner and self._sorts(rows, ctx)):
@@ -422,6 +435,15 @@ class MixtureOfExperts(FeedForward):
         rows, E, ff, ffs = h.shape[0], self.experts, self.inner, self.shared_inner
         route = self._route(h, ctx)
         sorts = self._sorts(rows, ctx)
+        if not sorts and self._few(h, ctx):
+            if out is None:
+                pieces = kn.moe_few_pieces(self.width)
+                out = ctx.ws.alloc((pieces, rows, self.width) if pieces > 1 else (rows, self.width), torch.float32)
+            act = ctx.ws.alloc((rows, E * ff + ffs), ctx.dtype)
+            passed, gate = self._step
+            kn.moe_few(h, self.w_gate_up, self.w_down, route, act, out, ff, ffs, self.activation, limit=self.limit,
+                       on_input=self.weight_input, shared_gate=gate, passed=passed)
+            return out
         in_pieces = out is None and not self.gated and not sorts  # what the last product likes to leave
         if out is None and not in_pieces:
             out = ctx.ws.alloc((rows, self.width), torch.float32)
