@@ -79,13 +79,17 @@ class GatedLinearUnit(FeedForward):
 
     graph_safe = True
     ACTIVATIONS = ("silu", "relu", "gelu_tanh")
-    BIAS_TAIL = 8  # columns behind the activations: a one and zeros (a product's K stays a multiple of eight)
+    #: columns behind the activations, a one and zeros: a product's K stays a multiple of 64, without which neither the packed
+    #: weights nor the pipelined tiles take it (2 048 x 7 168: 100 rows 106 us with 8 columns, 27 with 64; 2 635 rows 146 and 97;
+    #: a few rows 9.0 and 10.7), or of eight
+    BIAS_TAIL = {True: 64, False: 8}
 
     def __init__(self, width: int, inner: int, prefix: str, activation: str = "silu", bias: bool = False,
                  names: Optional[Mapping[str, str]] = None) -> None:
         if activation not in self.ACTIVATIONS:
             raise ValueError(f"unknown activation {activation!r}; known: {', '.join(self.ACTIVATIONS)}")
         self.width, self.inner, self.activation, self.bias = int(width), int(inner), activation, bool(bias)
+        self.tail = self.BIAS_TAIL[self.inner % 64 == 0]
         n = {"gate": "gate", "up": "up", "down": "down"}
         n.update(names or {})
         self.names: Dict[str, str] = {key: f"{prefix}.{val}" for key, val in n.items()}
@@ -122,7 +126,7 @@ class GatedLinearUnit(FeedForward):
         if self.bias:
             self.b_gate_up = torch.cat([tensors[self.names["gate"] + ".b"], tensors[self.names["up"] + ".b"]]).contiguous()
             b = tensors[self.names["down"] + ".b"].to(down.dtype)
-            down = torch.cat([down, b[:, None], down.new_zeros((self.width, self.BIAS_TAIL - 1))], dim=1)
+            down = torch.cat([down, b[:, None], down.new_zeros((self.width, self.tail - 1))], dim=1)
         self.w_down = product_weight(env, down)
 
     takes_out = True
@@ -140,8 +144,8 @@ class GatedLinearUnit(FeedForward):
         gu = ctx.ws.alloc((rows, 2 * self.inner), torch.float32)
         project(kn, ctx, h, self.w_gate_up, gu)
         if self.bias:
-            act = ctx.ws.alloc((rows, self.inner + self.BIAS_TAIL), self.w_down.dtype)
-            kn.glu(gu, act, self.activation, bias=self.b_gate_up, tail=self.BIAS_TAIL)
+            act = ctx.ws.alloc((rows, self.inner + self.tail), self.w_down.dtype)
+            kn.glu(gu, act, self.activation, bias=self.b_gate_up, tail=self.tail)
         else:
             act = ctx.ws.alloc((rows, self.inner), ctx.dtype)
             kn.glu(gu, act, self.activation)
