@@ -312,37 +312,67 @@ __global__ __launch_bounds__(256) void qkv_norm_store4_kernel(const float* __res
 }
 
 // A product a head: out[r, h ohs + n] = sum_k x[r, h K + k] w[h, n, k], bfloat16 operands on
-// v_mfma_f32_16x16x16_bf16 (exact products, 32-bit sums).  A workgroup of four wavefronts takes 64 rows by 64
+// v_mfma_f32_16x16x16_bf16 or 16x16x32 (exact products, 32-bit sums).  A workgroup of four wavefronts takes 64 rows by 64
 // columns of one head; a wavefront 16 rows by the 64 columns, its operands straight from memory (a head's weight
-// is small and stays in the caches; the four wavefronts read the same columns).  K in steps of 16, ascending: a
+// is small and stays in the caches; the four wavefronts read the same columns).  K in ascending steps: a
 // row's sums do not depend on what else is in the launch.
 typedef short bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-template <typename TO>
-__global__ __launch_bounds__(256) void linear_heads_kernel(const bf16_t* __restrict__ x, int ldx,
-                                                           const bf16_t* __restrict__ w, TO* __restrict__ out, int ldo,
-                                                           int rows, int N, int K, int ohs) {
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+// A run of STEP / 4 neighbouring k of one row, the operand of a matrix instruction; 32-bit numbers rounded to nearest even.
+template <int STEP>
+__device__ inline auto run_of_k(const bf16_t* p) {
+  if constexpr (STEP == 32) return __builtin_bit_cast(bf16x8_t, *(const uint4*)p);
+  else return __builtin_bit_cast(bf16x4_t, *(const uint2*)p);
+}
+__device__ inline uint32_t rounded2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, bf16x2_t));
+}
+template <int STEP>
+__device__ inline auto run_of_k(const float* p) {
+  const float4 a = *(const float4*)p;
+  if constexpr (STEP == 32) {
+    const float4 b = *(const float4*)(p + 4);
+    return __builtin_bit_cast(bf16x8_t, make_uint4(rounded2(a.x, a.y), rounded2(a.z, a.w), rounded2(b.x, b.y), rounded2(b.z, b.w)));
+  } else {
+    return __builtin_bit_cast(bf16x4_t, make_uint2(rounded2(a.x, a.y), rounded2(a.z, a.w)));
+  }
+}
+
+// FEW: at most 16 rows, and the four wavefronts take 16 of the 64 columns each (else 16 of 64 rows): single tokens are bound by
+// one wavefront's chain of loads and products.  STEP: k an instruction, 32 where K is a multiple of it and operands lie on 16
+// bytes.  16 heads of 128 x 192, from 16 k and 64 columns a wavefront: 8 rows 5.05 -> 2.85 us,
+// 2 000 rows 29.9 -> 17.6.
+template <bool FEW, int STEP, typename TI, typename TO>
+__device__ inline void linear_heads_tile(const TI* __restrict__ x, int ldx, const bf16_t* __restrict__ w, TO* __restrict__ out,
+                                         int ldo, int rows, int N, int K, int ohs) {
+  constexpr int COLS = FEW ? 1 : 4, RUN = STEP / 4;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const int h = blockIdx.z, r0 = blockIdx.x * 64 + 16 * wave, n0 = blockIdx.y * 64;
-  if (r0 >= rows) return;
-  const bf16_t* xa = x + (long long)min(r0 + c, rows - 1) * ldx + (long long)h * K + 4 * g;
-  const bf16_t* wb[4];
+  const int h = blockIdx.z, r0 = blockIdx.x * 64 + (FEW ? 0 : 16 * wave), n0 = blockIdx.y * 64 + (FEW ? 16 * wave : 0);
+  if (r0 >= rows || n0 >= N) return;
+  const TI* xa = x + (long long)min(r0 + c, rows - 1) * ldx + (long long)h * K + RUN * g;
+  const bf16_t* wb[COLS];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) wb[j] = w + ((long long)h * N + min(n0 + 16 * j + c, N - 1)) * K + 4 * g;
-  f32x4_t acc[4];
+  for (int j = 0; j < COLS; ++j) wb[j] = w + ((long long)h * N + min(n0 + 16 * j + c, N - 1)) * K + RUN * g;
+  f32x4_t acc[COLS];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  for (int ks = 0; ks < K; ks += 16) {
-    const bf16x4_t a = __builtin_bit_cast(bf16x4_t, *(const uint2*)(xa + ks));
+  for (int j = 0; j < COLS; ++j) acc[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int ks = 0; ks < K; ks += STEP) {
+    const auto a = run_of_k<STEP>(xa + ks);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bf16x4_t bv = __builtin_bit_cast(bf16x4_t, *(const uint2*)(wb[j] + ks));
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bv, acc[j], 0, 0, 0);
+    for (int j = 0; j < COLS; ++j) {
+      const auto b = run_of_k<STEP>(wb[j] + ks);
+      if constexpr (STEP == 32) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[j], 0, 0, 0);
+      else acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
     }
   }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < COLS; ++j) {
     const int n = n0 + 16 * j + c;
     if (n >= N) continue;
 #pragma unroll
@@ -350,6 +380,102 @@ __global__ __launch_bounds__(256) void linear_heads_kernel(const bf16_t* __restr
       const int r = r0 + 4 * g + e;
       if (r < rows) out[(long long)r * ldo + (long long)h * ohs + n] = from_f32<TO>(acc[j][e]);
     }
+  }
+}
+
+template <bool FEW, int STEP, typename TO>
+__global__ __launch_bounds__(256) void linear_heads_kernel(const bf16_t* __restrict__ x, int ldx,
+                                                           const bf16_t* __restrict__ w, TO* __restrict__ out, int ldo,
+                                                           int rows, int N, int K, int ohs) {
+  linear_heads_tile<FEW, STEP, bf16_t, TO>(x, ldx, w, out, ldo, rows, N, K, ohs);
+}
+
+// ---- a latent layer's rows in two launches: what its first product leaves, and what its second does ----------------------
+// Single tokens pay a launch's three to four microseconds for every step between two products: the two norms, the two
+// rotations, the store into the cache and the fold of the key's lift into the query were six launches and two products (31 us of
+// a layer at 8 rows of width 2 048, of which the arithmetic is a few), and are two around one product (12).
+struct Turn {  // cos and sin of a row's angles [rows][dims / 2][2], before `mag`
+  const float* cs;
+  int dims, interleaved;
+  float mag;
+};
+
+// Entry i of a rotated vector v (dims of its entries turn, the rest pass).
+__device__ inline float turned_at(const float* v, int i, const Turn& t, const float* cs) {
+  if (i >= t.dims) return v[i];
+  const int half = t.dims >> 1;
+  int j, mate;
+  bool first;
+  if (t.interleaved) j = i >> 1, first = !(i & 1), mate = i ^ 1;
+  else first = i < half, j = first ? i : i - half, mate = first ? i + half : i - half;
+  const float c = cs[2 * j] * t.mag, s = cs[2 * j + 1] * t.mag;
+  return first ? v[i] * c - v[mate] * s : v[i] * c + v[mate] * s;
+}
+
+struct LatentRows {
+  int lds, q_rank, kv_rank, rot_dim, ldcq;
+  float eps;
+  const float *wq, *wkv;
+  Turn turn;
+  const int *row_pos, *row_seq, *seq_slot, *block_table;
+  int bt_stride, BS;
+};
+constexpr int LATENT_PER = 8;  // entries of a normed run that a thread holds
+
+// src [rows, q_rank (+ kv_rank + rot_dim)].  Workgroup (r, 0): cq = the RMS norm of the row's first q_rank entries.  (r, 1): the
+// norm of the next kv_rank, and the rest rotated, as the row's key in the cache (K [block][BS][kv_rank + rot_dim]); the
+// former also as its value (V [block][kv_rank][BS]).
+template <typename T>
+__global__ __launch_bounds__(256) void latent_rows_kernel(const float* __restrict__ src, T* __restrict__ cq, T* __restrict__ kcache,
+                                                          T* __restrict__ vcache, LatentRows a) {
+  __shared__ float red[16];
+  const int r = blockIdx.x;
+  const bool own = blockIdx.y == 1;
+  const int n = own ? a.kv_rank : a.q_rank;
+  const float* s = src + (long long)r * a.lds + (own ? a.q_rank : 0);
+  const float* w = own ? a.wkv : a.wq;
+  float v[LATENT_PER], gain[LATENT_PER], acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < LATENT_PER; ++i) {
+    const int e = threadIdx.x + 256 * i;
+    v[i] = e < n ? s[e] : 0.f, gain[i] = e < n ? w[e] : 0.f;
+    acc = fmaf(v[i], v[i], acc);
+  }
+  T *k = nullptr, *val = nullptr;
+  if (own) {
+    const int p = a.row_pos[r], kd = a.kv_rank + a.rot_dim, off = p % a.BS;
+    const long long blk = a.block_table[(long long)a.seq_slot[a.row_seq[r]] * a.bt_stride + p / a.BS];
+    k = kcache + (blk * a.BS + off) * kd, val = vcache + blk * a.kv_rank * a.BS + off;
+    const float* cs = a.turn.cs + (long long)r * a.turn.dims;
+    for (int i = threadIdx.x; i < a.rot_dim; i += 256) k[a.kv_rank + i] = from_f32<T>(turned_at(s + n, i, a.turn, cs));
+  }
+  const float inv = 1.f / sqrtf(block_sum(acc, red) / (float)n + a.eps);
+#pragma unroll
+  for (int i = 0; i < LATENT_PER; ++i) {
+    const int e = threadIdx.x + 256 * i;
+    if (e >= n) continue;
+    const T o = from_f32<T>(v[i] * inv * gain[i]);
+    if (own) k[e] = o, val[(long long)e * a.BS] = o;
+    else cq[(long long)r * a.ldcq + e] = o;
+  }
+}
+
+// x [rows, heads K + heads rot_dim] (32-bit: every head's unrotated entries, then every head's rotated ones): out's head h gets
+// w[h] (N x K) times its unrotated entries, rounded to bfloat16, and behind them its rotated ones.  The last of gridDim.y
+// workgroups rotates.
+template <bool FEW, int STEP>
+__global__ __launch_bounds__(256) void latent_query_kernel(const float* __restrict__ x, int ldx, const bf16_t* __restrict__ w,
+                                                           bf16_t* __restrict__ out, int ldo, int rows, int N, int K, int rot_dim,
+                                                           Turn turn) {
+  if (blockIdx.y + 1 < gridDim.y) {
+    linear_heads_tile<FEW, STEP, float, bf16_t>(x, ldx, w, out, ldo, rows, N, K, N + rot_dim);
+    return;
+  }
+  const int h = blockIdx.z, heads = gridDim.z, lane = threadIdx.x & 63;
+  for (int r = blockIdx.x * 64 + (threadIdx.x >> 6); r < min(rows, (int)blockIdx.x * 64 + 64); r += 4) {  // a wavefront a row
+    const float *v = x + (long long)r * ldx + heads * K + h * rot_dim, *cs = turn.cs + (long long)r * turn.dims;
+    bf16_t* o = out + (long long)r * ldo + h * (N + rot_dim) + N;
+    for (int i = lane; i < rot_dim; i += 64) o[i] = f32_to_bf16(turned_at(v, i, turn, cs));
   }
 }
 
@@ -493,13 +619,60 @@ extern "C" int lq_linear_heads(const void* x, int ldx, const void* w, void* out,
   LQ_REQUIRE(lq_linear_heads_accepts(x, w, in_dtype, K, ldx), "linear_heads: bfloat16 operands, K in 16s, rows on 8 bytes");
   LQ_REQUIRE(lq_ceil_div(N, 64) <= 65535, "linear_heads: too many columns");
   dim3 grid(lq_ceil_div(rows, 64), lq_ceil_div(N, 64), heads);
-  if (out_dtype == LQ_F32)
-    linear_heads_kernel<float><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, (float*)out, ldo, rows, N, K,
-                                                         out_head_stride);
-  else if (out_dtype == LQ_BF16)
-    linear_heads_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, (bf16_t*)out, ldo, rows, N,
-                                                          K, out_head_stride);
+  const bool wide = K % 32 == 0 && ldx % 8 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0, few = rows <= 16;
+#define LQ_HEADS(FEW, STEP, T)                                                                                                        \
+  linear_heads_kernel<FEW, STEP, T><<<grid, 256, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, (T*)out, ldo, rows, N, K, \
+                                                              out_head_stride)
+#define LQ_HEADS_T(T) (wide ? (few ? LQ_HEADS(true, 32, T) : LQ_HEADS(false, 32, T)) : (few ? LQ_HEADS(true, 16, T) : LQ_HEADS(false, 16, T)))
+  if (out_dtype == LQ_F32) LQ_HEADS_T(float);
+  else if (out_dtype == LQ_BF16) LQ_HEADS_T(bf16_t);
   else LQ_REQUIRE(false, "linear_heads: unknown dtype %d", out_dtype);
+#undef LQ_HEADS_T
+#undef LQ_HEADS
   LQ_CHECK_LAUNCH("linear_heads");
+  return 0;
+}
+
+// Whether lq_latent_rows and lq_latent_query take a latent layer's sizes (in a bfloat16 run).
+extern "C" int lq_latent_accepts(int dtype, int heads, int dim, int rot_dim, int kv_rank, int q_rank) {
+  return dtype == LQ_BF16 && heads >= 1 && heads <= 65535 && dim >= 16 && dim % 16 == 0 && rot_dim >= 2 && rot_dim <= 1024 &&
+         kv_rank >= 1 && kv_rank <= 256 * LATENT_PER && q_rank >= 1 && q_rank <= 256 * LATENT_PER &&
+         (long long)heads * (dim + rot_dim) <= 0x3fffffff && (long long)heads * (kv_rank + rot_dim) <= 0x3fffffff;
+}
+
+// src float32 [rows, q_rank (+ kv_rank + rot_dim)], cos_sin float32 [rows, dims / 2, 2]; kcache null: no key or value of its own.
+extern "C" int lq_latent_rows(const float* src, int lds_, int rows, int q_rank, int kv_rank, int rot_dim, const float* wq, const float* wkv,
+                              float eps, const float* cos_sin, int dims, int interleaved, float magnitude, void* cq, int ldcq,
+                              const int* row_pos, const int* row_seq, const int* seq_slot, const int* block_table, int bt_stride,
+                              void* kcache, void* vcache, int block_size, hipStream_t stream) {
+  const bool own = kcache != nullptr;
+  LQ_REQUIRE(rows > 0 && lq_latent_accepts(LQ_BF16, 1, 16, rot_dim, kv_rank, q_rank), "latent_rows: rows %d, ranks %d and %d, %d rotated", rows,
+             q_rank, kv_rank, rot_dim);
+  LQ_REQUIRE(lds_ >= q_rank + (own ? kv_rank + rot_dim : 0) && ldcq >= q_rank, "latent_rows: a row stride is smaller than its row");
+  LQ_REQUIRE(src && wq && cq && own == (vcache != nullptr), "latent_rows: null pointer");
+  LQ_REQUIRE(!own || (wkv && cos_sin && dims >= 2 && dims % 2 == 0 && dims <= rot_dim && row_pos && row_seq && seq_slot && block_table &&
+                      block_size > 0 && bt_stride > 0), "latent_rows: the cache needs the rows' places and angles");
+  const LatentRows a = {lds_, q_rank, kv_rank, rot_dim, ldcq, eps, wq, wkv, {cos_sin, dims, interleaved, magnitude},
+                        row_pos, row_seq, seq_slot, block_table, bt_stride, block_size};
+  latent_rows_kernel<bf16_t><<<dim3(rows, own ? 2 : 1), 256, 0, stream>>>(src, (bf16_t*)cq, (bf16_t*)kcache, (bf16_t*)vcache, a);
+  LQ_CHECK_LAUNCH("latent_rows");
+  return 0;
+}
+
+// x float32 [rows, heads * dim + heads * rot_dim], w bfloat16 [heads, kv_rank, dim] dense, out bfloat16 [rows, heads * (kv_rank + rot_dim)]
+extern "C" int lq_latent_query(const float* x, int ldx, const void* w, void* out, int ldo, int rows, int heads, int dim, int rot_dim,
+                               int kv_rank, const float* cos_sin, int dims, int interleaved, float magnitude, hipStream_t stream) {
+  LQ_REQUIRE(rows > 0 && lq_latent_accepts(LQ_BF16, heads, dim, rot_dim, kv_rank, 1), "latent_query: rows %d, %d heads of %d and %d, rank %d", rows,
+             heads, dim, rot_dim, kv_rank);
+  LQ_REQUIRE(ldx >= heads * (dim + rot_dim) && ldo >= heads * (kv_rank + rot_dim), "latent_query: a row stride is smaller than its row");
+  LQ_REQUIRE(x && w && out && cos_sin && dims >= 2 && dims % 2 == 0 && dims <= rot_dim, "latent_query: null pointer, or %d rotated of %d", dims, rot_dim);
+  LQ_REQUIRE(ldx % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 8 == 0, "latent_query: operands are not aligned");
+  const dim3 grid(lq_ceil_div(rows, 64), lq_ceil_div(kv_rank, 64) + 1, heads);
+  const bool wide = dim % 32 == 0 && (uintptr_t)w % 16 == 0;
+  const auto kernel = rows <= 16 ? (wide ? latent_query_kernel<true, 32> : latent_query_kernel<true, 16>)
+                                 : (wide ? latent_query_kernel<false, 32> : latent_query_kernel<false, 16>);
+  kernel<<<grid, 256, 0, stream>>>(x, ldx, (const bf16_t*)w, (bf16_t*)out, ldo, rows, kv_rank, dim, rot_dim,
+                                   Turn{cos_sin, dims, interleaved, magnitude});
+  LQ_CHECK_LAUNCH("latent_query");
   return 0;
 }

@@ -1328,6 +1328,71 @@ class HipKernels:
                                        c_int(1 if interleaved else 0), _ptr(freqs), c_float(magnitude), _ptr(row_pos),
                                        self.stream))
 
+    @query
+    def latent_accepts(self, dtype: torch.dtype, heads: int, dim: int, rot_dim: int, kv_rank: int, q_rank: int) -> bool:
+        """Whether `latent_rows` and `latent_query` take a layer with attention through a cached latent of these sizes."""
+        if self.force_generic or dtype not in _DTYPE_CODE:
+            return False
+        return bool(self.lib.lq_latent_accepts(c_int(_DTYPE_CODE[dtype]), c_int(heads), c_int(dim), c_int(rot_dim), c_int(kv_rank),
+                                               c_int(q_rank)))
+
+    def _angles(self, cos_sin: torch.Tensor, rows: int, what: str) -> int:
+        self._f32(cos_sin, what)
+        if cos_sin.dim() != 3 or cos_sin.shape[0] != rows or cos_sin.shape[2] != 2 or not cos_sin.is_contiguous():
+            raise KernelLibraryError(f"{what}: cos_sin float32 [rows, pairs, 2]")
+        return 2 * cos_sin.shape[1]
+
+    def latent_rows(self, src: torch.Tensor, q_weight: torch.Tensor, cq: torch.Tensor, eps: float,
+                    kv_weight: Optional[torch.Tensor] = None, rot_dim: int = 0, cos_sin: Optional[torch.Tensor] = None,
+                    interleaved: bool = False, magnitude: float = 1.0, row_pos: Optional[torch.Tensor] = None,
+                    row_seq: Optional[torch.Tensor] = None, seq_slot: Optional[torch.Tensor] = None,
+                    block_table: Optional[torch.Tensor] = None, kcache: Optional[torch.Tensor] = None,
+                    vcache: Optional[torch.Tensor] = None, block_size: int = 0) -> None:
+        """src float32 [rows, q | latent | rotated part]: cq (bfloat16) = the RMS norm of the q columns times q_weight; with a
+        cache, the latent normed likewise (kv_weight) and the rotated part (angles cos_sin [rows, pairs, 2], pairing and
+        magnitude as `rotary`) are the row's key, the latent its value, at the rows' positions (layout as `kv_store`)."""
+        rows, ns, lds = self._mat(src, "latent_rows: src")
+        rc, nq, ldcq = self._mat(cq, "latent_rows: cq")
+        self._f32(src, "latent_rows: src")
+        self._f32(q_weight, "latent_rows: q_weight", nq)
+        if rc != rows or cq.dtype != torch.bfloat16:
+            raise KernelLibraryError("latent_rows: cq bfloat16 [rows, q]")
+        kv, dims = 1, 0
+        if kcache is not None:
+            kv = kv_weight.numel()
+            self._f32(kv_weight, "latent_rows: kv_weight", kv)
+            self._dev(kcache, vcache, block_table)
+            dims = self._angles(cos_sin, rows, "latent_rows")
+            for t, what in ((row_pos, "row_pos"), (row_seq, "row_seq")):
+                self._i32(t, what, rows)
+            if ns != nq + kv + rot_dim or tuple(kcache.shape[1:]) != (1, block_size, kv + rot_dim) \
+                    or tuple(vcache.shape[1:]) != (1, kv, block_size) or kcache.dtype != cq.dtype or vcache.dtype != cq.dtype \
+                    or not kcache.is_contiguous() or not vcache.is_contiguous() or block_table.dtype != torch.int32:
+                raise KernelLibraryError("latent_rows: src [rows, q | latent | rotated], a cache of latent rows")
+        elif ns != nq:
+            raise KernelLibraryError("latent_rows: without a cache src holds the q columns alone")
+        self._check(self.lib.lq_latent_rows(
+            _ptr(src), c_int(lds), c_int(rows), c_int(nq), c_int(kv), c_int(rot_dim if kcache is not None else 2), _ptr(q_weight),
+            _ptr(kv_weight), c_float(eps), _ptr(cos_sin), c_int(dims), c_int(1 if interleaved else 0), c_float(magnitude), _ptr(cq),
+            c_int(ldcq), _ptr(row_pos), _ptr(row_seq), _ptr(seq_slot), _ptr(block_table),
+            c_int(block_table.stride(0) if block_table is not None else 0), _ptr(kcache), _ptr(vcache), c_int(block_size), self.stream))
+
+    def latent_query(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, rot_dim: int, cos_sin: torch.Tensor,
+                     interleaved: bool, magnitude: float) -> None:
+        """x float32 [rows, heads * dim | heads * rot_dim], w bfloat16 [heads, rank, dim]: out (bfloat16) holds for every head
+        w[h] times its unrotated entries, which are rounded to bfloat16 first, and its rotated ones (as `rotary`)."""
+        rows, nx, ldx = self._mat(x, "latent_query: x")
+        ro, no, ldo = self._mat(out, "latent_query: out")
+        heads, rank, dim = w.shape
+        self._f32(x, "latent_query: x")
+        dims = self._angles(cos_sin, rows, "latent_query")
+        if not w.is_contiguous() or not w.is_cuda or w.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 \
+                or nx != heads * (dim + rot_dim) or (ro, no) != (rows, heads * (rank + rot_dim)):
+            raise KernelLibraryError("latent_query: x [rows, heads * (dim + rot_dim)], out [rows, heads * (rank + rot_dim)]")
+        self._check(self.lib.lq_latent_query(_ptr(x), c_int(ldx), _ptr(w), _ptr(out), c_int(ldo), c_int(rows), c_int(heads), c_int(dim),
+                                             c_int(rot_dim), c_int(rank), _ptr(cos_sin), c_int(dims), c_int(1 if interleaved else 0),
+                                             c_float(magnitude), self.stream))
+
     def rotary_qkv(self, src: torch.Tensor, q_out: torch.Tensor, k_out: torch.Tensor, v_out: torch.Tensor, heads: int,
                    kv_heads: int, key_dim: int, value_dim: int, dims: int, interleaved: bool,
                    freqs: Optional[torch.Tensor], magnitude: float, norm_eps: Optional[float],

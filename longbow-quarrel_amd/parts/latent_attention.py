@@ -28,7 +28,7 @@ import torch
 
 from .base import (MIXERS, VECTOR32, BuildEnv, KVNeed, LayerCache, Mixer, StepContext, TensorSpec, product_weight,
                    project)
-from .rope import rotary_frequencies, rotary_magnitude
+from .rope import rotary_frequencies, rotary_magnitude, step_angles
 from .sink_attention import split_scratch
 
 
@@ -87,9 +87,18 @@ class LatentAttention(Mixer):
         self.q_norm_w = tensors[nm["dq_norm"]].contiguous()
         self.kv_norm_w = tensors[nm["dkv_norm"]].contiguous() if self.own_kv else None
         uq = tensors[nm["uq"]].reshape(H, self.dim + self.rot_dim, self.q_rank)
-        # the heads' unrotated rows first, then their rotated rows: two products, each with the result it feeds
-        self.w_uq_plain = product_weight(env, uq[:, : self.dim].reshape(H * self.dim, self.q_rank).contiguous())
-        self.w_uq_rot = product_weight(env, uq[:, self.dim :].reshape(H * self.rot_dim, self.q_rank).contiguous())
+        # the heads' unrotated rows first, then their rotated rows: one product, whose 32-bit result one launch folds and rotates,
+        # or two, each with the result it feeds
+        plain = uq[:, : self.dim].reshape(H * self.dim, self.q_rank)
+        rot = uq[:, self.dim :].reshape(H * self.rot_dim, self.q_rank)
+        ask = getattr(env.kernels, "latent_accepts", None)
+        self.fused = ask is not None and env.dtype == tensors[nm["uk"]].dtype == uq.dtype and \
+            ask(env.dtype, H, self.dim, self.rot_dim, self.kv_rank, self.q_rank)
+        if self.fused:
+            self.w_uq = product_weight(env, torch.cat([plain, rot], dim=0))
+        else:
+            self.w_uq_plain = product_weight(env, plain.contiguous())
+            self.w_uq_rot = product_weight(env, rot.contiguous())
         # head n's Wuk_n^T [kv_rank, dim]: the weight of the product that folds the key's lift into the query
         self.w_uk_t = tensors[nm["uk"]].reshape(H, self.dim, self.kv_rank).transpose(1, 2).contiguous()
         self.w_uv = tensors[nm["uv"]].reshape(H, self.value_dim, self.kv_rank).contiguous()
@@ -114,6 +123,34 @@ class LatentAttention(Mixer):
         down = ctx.ws.alloc((rows, _round8(n_down)), torch.float32)[:, :n_down]
         project(kn, ctx, h, self.w_down, down)
         cq = ctx.ws.alloc((rows, _round8(qr)), ctx.dtype)[:, :qr]
+        q = ctx.ws.alloc((rows, H * kd), ctx.dtype)  # head n: [Wuk_n^T q_unrot | q_rot rotated]
+        if self.fused:
+            angles = step_angles(ctx, self.freqs, self.freq_table)
+            turn = dict(rot_dim=rd, cos_sin=angles, interleaved=inter, magnitude=self.magnitude)
+            place = dict(turn, kv_weight=self.kv_norm_w, row_pos=ctx.row_pos, row_seq=ctx.row_seq, seq_slot=ctx.seq_slot,
+                         block_table=cache.block_table, kcache=cache.k, vcache=cache.v, block_size=cache.block_size) if self.own_kv else {}
+            kn.latent_rows(down, self.q_norm_w, cq, self.eps, **place)
+            q_all = ctx.ws.alloc((rows, (H * (self.dim + rd) + 3) // 4 * 4), torch.float32)[:, : H * (self.dim + rd)]
+            project(kn, ctx, cq, self.w_uq, q_all)
+            kn.latent_query(q_all, self.w_uk_t, q, **turn)
+        else:
+            self._rows_and_query(down, cq, q, ctx, cache)
+        mean = ctx.ws.alloc((rows, H * r), ctx.dtype)  # every head's weighted mean of latents
+        kn.sink_attention(q, mean, H, 1, kd, r, ctx.row_pos, ctx.row_seq, ctx.seq_slot, cache.block_table, cache.k,
+                          cache.v, cache.block_size, self.scale, window=0, keep_first=0, sink=False, gate=None,
+                          decode=ctx.decode, **split_scratch(ctx, q.dtype, H, 1, kd, r, cache.block_size, 0, 0))
+        att = ctx.ws.alloc((rows, H * self.value_dim), ctx.dtype)
+        kn.linear_heads(mean, self.w_uv, att, H, self.value_dim)
+        if out is None:
+            out = ctx.ws.alloc((rows, self.width), torch.float32)
+        project(kn, ctx, att, self.w_o, out)
+        return out
+
+    def _rows_and_query(self, down, cq, q, ctx: StepContext, cache: LayerCache) -> None:
+        """The norms, rotations, the store into the cache and the heads' queries, a launch each."""
+        kn, rows, H = ctx.kernels, down.shape[0], self.heads
+        qr, r, rd, kd = self.q_rank, self.kv_rank, self.rot_dim, self.key_dim
+        inter = self.pairing == "interleaved"
         kn.rmsnorm_cols(down[:, :qr], self.q_norm_w, self.eps, cq)
         if self.own_kv:
             row = ctx.ws.alloc((rows, _round8(kd)), ctx.dtype)[:, :kd]
@@ -126,16 +163,5 @@ class LatentAttention(Mixer):
         project(kn, ctx, cq, self.w_uq_plain, q_plain)
         q_rot = ctx.ws.alloc((rows, H * rd), torch.float32)
         project(kn, ctx, cq, self.w_uq_rot, q_rot)
-        q = ctx.ws.alloc((rows, H * kd), ctx.dtype)  # head n: [Wuk_n^T q_unrot | q_rot rotated]
         kn.linear_heads(q_plain, self.w_uk_t, q, H, kd)
         kn.rotary(q_rot, q[:, r:], H, rd, kd, self.rot_dims, inter, self.freqs, self.magnitude, ctx.row_pos)
-        mean = ctx.ws.alloc((rows, H * r), ctx.dtype)  # every head's weighted mean of latents
-        kn.sink_attention(q, mean, H, 1, kd, r, ctx.row_pos, ctx.row_seq, ctx.seq_slot, cache.block_table, cache.k,
-                          cache.v, cache.block_size, self.scale, window=0, keep_first=0, sink=False, gate=None,
-                          decode=ctx.decode, **split_scratch(ctx, q.dtype, H, 1, kd, r, cache.block_size, 0, 0))
-        att = ctx.ws.alloc((rows, H * self.value_dim), ctx.dtype)
-        kn.linear_heads(mean, self.w_uv, att, H, self.value_dim)
-        if out is None:
-            out = ctx.ws.alloc((rows, self.width), torch.float32)
-        project(kn, ctx, att, self.w_o, out)
-        return out
