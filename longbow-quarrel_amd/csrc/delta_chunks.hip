@@ -39,6 +39,7 @@ struct DeltaArgs {
   const int *seq_slot, *cu_rows;
   int least;        // sequences of fewer tokens are not taken
   int first, last;  // the chunks of this pair of launches: numbers first .. last - 1, the scratch of `first` at its start
+  float q_scale, inv_tau;  // of gated linear attention
 };
 
 template <int CTRL>
@@ -98,7 +99,13 @@ struct Prepared {
 // by channel (a lane holds two, and for every earlier token of the block the product of the decays since): no
 // factoring of f_st into a row's and a column's part is safe where decays are strong.  Between blocks it is: from the
 // row's block's start on, and up to the column's block's end.
-template <bool QUADS>
+// ERASE: the delta rule.  Without it (gated linear attention) U is V: only B, Q~, the update's factor and the decays are made, and a
+// channel's decay is sigmoid(z + bias)^inv_tau.
+// (What the state is multiplied with from chunk to chunk is there the exponential of a sum of logarithms, rounded once where a
+// product of 64 decays is rounded at each: these errors are what adds up along a sequence.)
+__device__ inline float log_decay(float z, float inv_tau) { return -softplus_f(-z) * inv_tau; }
+
+template <bool QUADS, bool ERASE>
 __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   Prepared& L = *(Prepared*)smem;
@@ -108,7 +115,7 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
   const long long r0 = at.first;
   const int nt = at.rows, N = a.N;
   float* to = a.scratch + ((long long)blockIdx.x * a.heads + h) * PART;
-  const float rate = -expf(a.a_log[h]);
+  const float rate = ERASE ? -expf(a.a_log[h]) : 0.f;
 
   // every load of a thread is asked for before the first is waited for
   if constexpr (QUADS) {
@@ -121,9 +128,11 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
       if (t < nt && n < N) {
         const long long r = r0 + t;
         k[i] = *(const f32x4*)(a.k + r * a.ldk + j * N + n), q[i] = *(const f32x4*)(a.q + r * a.ldq + j * N + n);
+        if constexpr (!ERASE) q[i] *= a.q_scale;
         if (a.channel_decay) z[i] = *(const f32x4*)(a.a + r * a.lda + h * N + n) + *(const f32x4*)(a.dt_bias + h * N + n);
       }
     }
+    f32x4 logs = {0.f, 0.f, 0.f, 0.f};  // (a thread's channels are the same in every turn)
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int e = tid + 512 * i, t = e / (NMAX / 4), n = e % (NMAX / 4) * 4;
@@ -132,28 +141,48 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
         f32x4 g = {1.f, 1.f, 1.f, 1.f};
         if (t < nt && n < N)
 #pragma unroll
-          for (int x = 0; x < 4; ++x) g[x] = decay_of(z[i][x], rate);
+          for (int x = 0; x < 4; ++x) {
+            if constexpr (ERASE) {
+              g[x] = decay_of(z[i][x], rate);
+            } else {
+              const float log = log_decay(z[i][x], a.inv_tau);
+              logs[x] += log, g[x] = expf(log);
+            }
+          }
         *(f32x4*)&L.g[t][n] = g;
       }
     }
+    if constexpr (!ERASE) *(f32x4*)(&L.m[0][0] + (tid / (NMAX / 4)) * NMAX + tid % (NMAX / 4) * 4) = logs;
   } else {
+    float logs = 0.f;
     for (int e = tid; e < CHUNK * NMAX; e += 512) {
       const int t = e / NMAX, n = e % NMAX;
       const bool there = t < nt && n < N;
       const long long r = r0 + t;
       L.k[t][n] = there ? a.k[r * a.ldk + j * N + n] : 0.f;
-      L.q[t][n] = there ? a.q[r * a.ldq + j * N + n] : 0.f;
-      if (a.channel_decay)
-        L.g[t][n] = there ? decay_of(a.a[r * a.lda + h * N + n] + a.dt_bias[h * N + n], rate) : 1.f;
+      L.q[t][n] = there ? a.q[r * a.ldq + j * N + n] * (ERASE ? 1.f : a.q_scale) : 0.f;
+      if (a.channel_decay) {
+        const float z = there ? a.a[r * a.lda + h * N + n] + a.dt_bias[h * N + n] : 0.f;
+        if constexpr (ERASE) {
+          L.g[t][n] = there ? decay_of(z, rate) : 1.f;
+        } else {
+          const float log = there ? log_decay(z, a.inv_tau) : 0.f;
+          logs += log, L.g[t][n] = expf(log);
+        }
+      }
     }
+    if constexpr (!ERASE) (&L.m[0][0])[tid] = logs;
   }
-  if (!a.channel_decay) {  // one decay a head: a thread makes that of its row
+  if (ERASE && !a.channel_decay) {  // one decay a head: a thread makes that of its row
     const int t = tid >> 3;
     const float g = t < nt ? decay_of(a.a[(r0 + t) * a.lda + h] + a.dt_bias[h], rate) : 1.f;
     for (int n = tid & 7; n < NMAX; n += 8) L.g[t][n] = g;
   }
-  if (tid < CHUNK) L.beta[tid] = tid < nt ? sigmoid_f(a.beta[(r0 + tid) * a.ldbeta + h]) : 0.f;
-  for (int e = tid; e < CHUNK * LDT; e += 512) (&L.m[0][0])[e] = 0.f, (&L.b[0][0])[e] = 0.f;
+  if (ERASE && tid < CHUNK) L.beta[tid] = tid < nt ? sigmoid_f(a.beta[(r0 + tid) * a.ldbeta + h]) : 0.f;
+  for (int e = tid; e < CHUNK * LDT; e += 512) {
+    if constexpr (ERASE) (&L.m[0][0])[e] = 0.f;  // (else it holds the threads' sums of logarithms)
+    (&L.b[0][0])[e] = 0.f;
+  }
   __syncthreads();
 
   {  // within a block of 16 tokens
@@ -176,6 +205,7 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
         run[c] *= g;
         from_start[t][c] = with[c] * run[c];
       }
+      if (!ERASE && !of_b) return;  // (no A)
 #pragma unroll
       for (int s = 0; s < COUNT; ++s) sums[s] = s <= t ? fmaf(faded[s][1], with[1], faded[s][0] * with[0]) : 0.f;
       const float sum = sums_by_lane<COUNT>(sums);
@@ -208,7 +238,7 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
 #pragma unroll
     for (int i = 0; i < KT - 1; ++i)
       if (i < mt) f *= *(const f32x4*)&L.block[i][n];
-    *(f32x4*)(to + AT_KEYS + e * 4) = *(const f32x4*)&L.k[row][n] * f;
+    if constexpr (ERASE) *(f32x4*)(to + AT_KEYS + e * 4) = *(const f32x4*)&L.k[row][n] * f;
     *(f32x4*)(to + AT_QUERIES + e * 4) = *(const f32x4*)&L.q[row][n] * f;
   }
   // what the state is updated with, rows key channels
@@ -223,12 +253,18 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
   }
   if (tid < NMAX) {
     float f = 1.f;
-    for (int i = 0; i < KT; ++i) f *= L.block[i][tid];
+    if constexpr (ERASE) {
+      for (int i = 0; i < KT; ++i) f *= L.block[i][tid];
+    } else {
+      f = 0.f;
+      for (int i = 0; i < (QUADS ? 512 / (NMAX / 4) : 512 / NMAX); ++i) f += (&L.m[0][0])[i * NMAX + tid];
+      f = expf(f);
+    }
     to[AT_DECAY + tid] = f;
   }
   // between blocks: six pairs of A and of B
   const int c = lane & 15, g = lane >> 4;
-  for (int u = w; u < 12; u += 8) {
+  for (int u = ERASE ? w : 2 * w + 1; u < 12; u += ERASE ? 8 : 16) {
     const int pair = u >> 1, i = pair < 1 ? 1 : pair < 3 ? 2 : 3, jb = pair - i * (i - 1) / 2;
     const float(*rows)[LD] = (u & 1) ? L.q : L.k;
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -241,6 +277,12 @@ __global__ __launch_bounds__(512, 2) void delta_prepare_kernel(DeltaArgs a) {
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) ((u & 1) ? L.b : L.m)[SUB * i + 4 * g + e][SUB * jb + c] = acc[0][e] + acc[1][e];
+  }
+  if constexpr (!ERASE) {
+    __syncthreads();
+    for (int e = tid; e < KT * KT * 64; e += 512)
+      *(f32x4*)(to + AT_B + e * 4) = *(const f32x4*)&L.b[SUB * (e / (KT * 64)) + (e & 15)][e / 64 % KT * SUB + (e >> 4 & 3) * 4];
+    return;
   }
   // the inverse of I + diag(beta) A: the blocks on the diagonal by substitution, a lane a column
   if (w < KT && lane < SUB) {
@@ -425,6 +467,101 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   }
 }
 
+// The walk of gated linear attention, U = V:  O = Q~ S + B V;  S <- diag(p_64) S + sum_s (f_s,64 k_s) v_s^T.  One workgroup of eight
+// wavefronts a (sequence, head, 16 columns of the values).  Wavefront w holds channels 16 w .. + 15 of the state; for the results
+// it takes 16 tokens (w % 4) and half of the sums (w / 4: channels and blocks of tokens).  The state and the values stand in LDS
+// twice, so that a chunk has one barrier.
+__global__ __launch_bounds__(512, 2) void gla_walk_kernel(DeltaArgs a) {
+  __shared__ f32x4 Ss[2][NT][64], Vs[2][KT][64], Ps[2][KT][64];
+  const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int c = lane & 15, g = lane >> 4, p = blockIdx.y * 16 + c, mt = w & 3, half = w >> 2;
+  const long long r1 = a.cu_rows[b + 1];
+  const int base = first_chunk(a.cu_rows, b, a.least), i0 = max(a.first - base, 0);
+  const int chunks = min(chunks_of((int)(r1 - a.cu_rows[b]), a.least), a.last - base) - i0;  // from the sequence's i0th on
+  if (chunks <= 0) return;
+  const long long r0 = a.cu_rows[b] + (long long)i0 * CHUNK;
+  const float* from = a.scratch + ((long long)(base + i0 - a.first) * a.heads + h) * PART;
+  const long long step = (long long)a.heads * PART;
+  float* sp = a.state + (((long long)a.seq_slot[b] * a.heads + h) * a.P + min(p, a.P - 1)) * a.N;
+  const bool live = p < a.P;
+  f32x4 S, rows[NT / 2], tri[2], upd[KT], V = {0.f, 0.f, 0.f, 0.f}, decay;
+  auto ask = [&](const float* f) {
+#pragma unroll
+    for (int nb = 0; nb < NT / 2; ++nb) rows[nb] = *(const f32x4*)(f + AT_QUERIES + ((mt * NT + half * (NT / 2) + nb) * 64 + lane) * 4);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+      if (2 * half + x <= mt) tri[x] = *(const f32x4*)(f + AT_B + ((mt * KT + 2 * half + x) * 64 + lane) * 4);
+#pragma unroll
+    for (int kb = 0; kb < KT; ++kb) upd[kb] = *(const f32x4*)(f + AT_UPDATE + ((w * KT + kb) * 64 + lane) * 4);
+    decay = *(const f32x4*)(f + AT_DECAY + 16 * w + 4 * g);
+  };
+  auto ask_v = [&](long long c0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const long long r = c0 + SUB * mt + 4 * g + e;
+      V[e] = live && r < r1 ? a.v[r * a.ldv + (long long)h * a.P + p] : 0.f;
+    }
+  };
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int n = 16 * w + 4 * g + e;
+    S[e] = live && n < a.N ? sp[n] : 0.f;
+  }
+  ask(from);
+  if (half == 0) ask_v(r0);
+  Ss[0][w][lane] = S;
+  if (half == 0) {
+    Vs[0][mt][lane] = V;
+    if (chunks > 1) ask_v(r0 + CHUNK);
+  }
+  lds_barrier();
+  for (int i = 0; i < chunks; ++i, from += step) {
+    const int cur = i & 1;
+    const long long c0 = r0 + (long long)i * CHUNK;
+    f32x4 acc[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) acc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int nb = 0; nb < NT / 2; ++nb) acc[nb & 1] = step4(rows[nb], Ss[cur][half * (NT / 2) + nb][lane], acc[nb & 1]);
+    f32x4 own = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int kb = 2 * half + x;
+      if (kb > mt) continue;
+      const f32x4 v = Vs[cur][kb][lane];
+      const float odd = not_finite(v, 0.f);
+      // (B's zeros above the diagonal meet no NaN and no infinity of a later token)
+      own = kb == mt && __any(odd != odd) ? step4_lower(tri[x], v, own) : step4(tri[x], v, own);
+    }
+    // (what the chunk adds is summed by itself: one rounding at the state's size a chunk, not one a product)
+#pragma unroll
+    for (int kb = 0; kb < KT; ++kb) acc[2 + (kb & 1)] = step4(upd[kb], Vs[cur][kb][lane], acc[2 + (kb & 1)]);
+    S = S * decay + (acc[2] + acc[3]);
+    if (i + 1 < chunks) ask(from + step);
+    const f32x4 Y = (acc[0] + acc[1]) + own;
+    if (half == 1) Ps[cur][mt][lane] = Y;
+    Ss[cur ^ 1][w][lane] = S;
+    if (half == 0 && i + 1 < chunks) {
+      Vs[cur ^ 1][mt][lane] = V;
+      if (i + 2 < chunks) ask_v(c0 + 2 * CHUNK);
+    }
+    lds_barrier();
+    if (half == 0) {
+      const f32x4 whole = Y + Ps[cur][mt][lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const long long r = c0 + SUB * mt + 4 * g + e;
+        if (live && r < r1) a.out[r * a.ldo + (long long)h * a.P + p] = whole[e];
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int n = 16 * w + 4 * g + e;
+    if (live && n < a.N) sp[n] = S[e];
+  }
+}
+
 }  // namespace
 
 // Float32 scratch with which a launch runs in chunks (0: token by token).  Microseconds a launch, token by token and in
@@ -487,10 +624,10 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
                     int ldo, int heads, int kv_heads, int Dk, int P, const int* seq_slot, const int* cu_rows, int batch,
                     int rows, int channel_decay, float* scratch, long long scratch_floats, hipStream_t stream) {
   DeltaArgs d = {q, k, v, beta, a, dt_bias, a_log, ldq, ldk, ldv, ldbeta, lda, ldo, state, out, scratch,
-                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows, lq_delta_least_rows(rows, batch, heads, channel_decay), 0, 0};
+                 heads, kv_heads, Dk, P, batch, channel_decay, seq_slot, cu_rows, lq_delta_least_rows(rows, batch, heads, channel_decay), 0, 0, 0.f, 0.f};
   const bool quads = Dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && (!channel_decay || lda % 4 == 0) &&
                      (((uintptr_t)q | (uintptr_t)k | (channel_decay ? (uintptr_t)a | (uintptr_t)dt_bias : 0)) & 15) == 0;
-  const auto prepare = quads ? delta_prepare_kernel<true> : delta_prepare_kernel<false>;
+  const auto prepare = quads ? delta_prepare_kernel<true, true> : delta_prepare_kernel<false, true>;
   static bool configured[2] = {false, false};
   if (!configured[quads]) {
     const hipError_t e = hipFuncSetAttribute((const void*)prepare, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(Prepared));
@@ -507,6 +644,47 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
     LQ_CHECK_LAUNCH("delta_scan(chunks)");
     delta_walk_kernel<<<dim3((unsigned)batch * heads, lq_ceil_div(P, 16)), 512, 0, stream>>>(d);
     LQ_CHECK_LAUNCH("delta_scan(walk over chunks)");
+  }
+  return 0;
+}
+
+// ---- gated linear attention
+// Float32 scratch for a launch in chunks (0: sizes that are not taken, or a launch that is faster token by token: the longest
+// portion below 48 tokens, 96 of states of up to 4 096 entries).  Microseconds, token by token (in segments where it has them) and
+// in chunks, heads of 128 x 256: 8 heads, 48 tokens 27 / 25, 128 tokens 60 / 29, 512 165 / 44, 3 000 781 / 144, eight sequences
+// of 200 to 700 710 / 135, 24 of 120 400 / 119, 300 tokens beside seven of one 189 / 59; 16 heads, 2 048 994 / 119; 4 heads of 64 x
+// 64, 64 tokens 26 / 27, 300 99 / 35.  Error against 64 bits, 2 048 tokens of 128 x 256: 2.8e-6 and 5.0e-7, of the state they leave
+// 4.3e-6 and 3.1e-7; 64 tokens 2.2e-7 and 2.3e-7.
+extern "C" long long lq_gla_chunks_workspace(int rows, int batch, int heads, int Dk, int P, int max_rows) {
+  if (rows <= 0 || batch <= 0 || heads <= 0 || P <= 0 || Dk <= 0 || Dk > NMAX || max_rows < (Dk * P > 4096 ? 48 : 96)) return 0;
+  if (heads > 65535 || lq_ceil_div(P, 16) > 65535) return 0;
+  return chunks_scratch(most_chunks(rows, batch, 1), lq_delta_scan_least(heads), LQ_DELTA_SCRATCH);
+}
+
+int lq_gla_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* z, int ldz, const float* bias,
+                  float* state, float* out, int ldo, int heads, int Dk, int P, float q_scale, float inv_tau, const int* seq_slot,
+                  const int* cu_rows, int batch, int rows, float* scratch, long long scratch_floats, hipStream_t stream) {
+  DeltaArgs d = {q, k, v, nullptr, z, bias, nullptr, ldq, ldk, ldv, 0, ldz, ldo, state, out, scratch, heads, heads, Dk, P, batch, 1,
+                 seq_slot, cu_rows, 1, 0, 0, q_scale, inv_tau};
+  const bool quads = Dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldz % 4 == 0 &&
+                     (((uintptr_t)q | (uintptr_t)k | (uintptr_t)z | (uintptr_t)bias) & 15) == 0;
+  const auto prepare = quads ? delta_prepare_kernel<true, false> : delta_prepare_kernel<false, false>;
+  static bool configured[2] = {false, false};
+  if (!configured[quads]) {
+    const hipError_t e = hipFuncSetAttribute((const void*)prepare, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(Prepared));
+    if (e != hipSuccess) {
+      lq_set_error("gla_scan: cannot reserve %d bytes of LDS: %s", (int)sizeof(Prepared), hipGetErrorString(e));
+      return -2;
+    }
+    configured[quads] = true;
+  }
+  const long long all = most_chunks(rows, batch, 1), room = chunks_a_round(all, scratch_floats, lq_delta_scan_least(heads));
+  for (long long first = 0; first < all; first += room) {
+    d.first = (int)first, d.last = (int)(first + room < all ? first + room : all);
+    prepare<<<dim3(d.last - d.first, heads), 512, sizeof(Prepared), stream>>>(d);
+    LQ_CHECK_LAUNCH("gla_scan(chunks)");
+    gla_walk_kernel<<<dim3((unsigned)batch * heads, lq_ceil_div(P, 16)), 512, 0, stream>>>(d);
+    LQ_CHECK_LAUNCH("gla_scan(walk over chunks)");
   }
   return 0;
 }

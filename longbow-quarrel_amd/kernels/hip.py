@@ -1575,16 +1575,27 @@ class HipKernels:
         return int(self.lib.lq_gla_scan_workspace(c_int(batch), c_int(heads), c_int(value_dim), c_int(key_dim),
                                                   c_int(max_rows)))
 
+    @query
+    def gla_chunks_workspace(self, rows: int, batch: int, heads: int, key_dim: int, value_dim: int, max_rows: int) -> int:
+        """Float32 entries of scratch with which `gla_scan` runs this launch in chunks on the matrix cores (0: it is not to)."""
+        if self.force_generic:
+            return 0
+        self.lib.lq_gla_chunks_workspace.restype = c_longlong
+        return int(self.lib.lq_gla_chunks_workspace(c_int(rows), c_int(batch), c_int(heads), c_int(key_dim), c_int(value_dim),
+                                                    c_int(max_rows)))
+
     def gla_scan(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor, bias: torch.Tensor,
                  state: torch.Tensor, out: torch.Tensor, heads: int, key_dim: int, value_dim: int, q_scale: float,
                  inv_tau: float, seq_slot: torch.Tensor, cu_rows: torch.Tensor, batch: int, max_rows: int = 0,
-                 workspace: Optional[torch.Tensor] = None) -> None:
+                 workspace: Optional[torch.Tensor] = None, chunked: bool = False) -> None:
         """Gated linear attention along every sequence of the step, token by token: with the decay a =
         sigmoid(z + bias)^inv_tau for every key channel, S <- diag(a) S + k v^T and out = S^T (q q_scale) per head;
         state [slots, heads, value_dim, key_dim] is read and left at the step's end.  All float32.  `max_rows` (the
         most rows a sequence brings) and `workspace` (`gla_scan_workspace(...)` floats) let a launch of few long
         sequences run in segments side by side (every segment from zero, the end states chained with the products
-        of the segments' decays, the segments again from their true starts)."""
+        of the segments' decays, the segments again from their true starts); with `chunked` (and
+        `gla_chunks_workspace(...)` floats) the sequences go in chunks of 64 tokens on the matrix cores, in 32 bits, with
+        other orders of the sums."""
         rows = q.shape[0]
         for t, what, cols in ((q, "q", heads * key_dim), (k, "k", heads * key_dim), (z, "z", heads * key_dim),
                               (v, "v", heads * value_dim), (out, "out", heads * value_dim)):
@@ -1604,7 +1615,8 @@ class HipKernels:
                                          c_int(ld(v, "v")), _ptr(z), c_int(ld(z, "z")), _ptr(bias), _ptr(state), _ptr(out),
                                          c_int(ld(out, "out")), c_int(heads), c_int(key_dim), c_int(value_dim),
                                          c_float(q_scale), c_float(inv_tau), _ptr(seq_slot), _ptr(cu_rows), c_int(batch),
-                                         c_int(max_rows if workspace is not None else 0), _ptr(workspace),
+                                         c_int(rows), c_int(max_rows if workspace is not None else 0), c_int(1 if chunked else 0),
+                                         _ptr(workspace),
                                          c_longlong(0 if workspace is None else workspace.numel()), self.stream))
 
     @query
