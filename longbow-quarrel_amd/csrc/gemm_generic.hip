@@ -18,7 +18,7 @@
 // K / 256 + 64 additions instead of K.
 //
 // Three kernels: an LDS-tiled one (block tiles of 64 x 64 or 128 x 128, any size and alignment); a pipelined one of
-// 128 x 128 or 64 x 128 tiles for float32 operands in whole pieces with K in 32s, from 33 rows on; and one for up to 64 rows
+// 32 to 128 x 128 tiles for float32 operands in whole pieces with K in 32s, from 33 rows on; and one for up to 64 rows
 // that streams the weights straight from memory, a block of waves a tile of 16 columns, its waves taking chunks in turn and
 // adding their sums up in order through LDS.
 #include "common.h"
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const T* __restrict
 }
 
 // ---- pipelined: the same tiles, operands in whole pieces ---------------------------------------------------
-// 128 x 128 a block, 4 waves of 64 x 64; or 64 x 128, waves of 32 x 64.  Stages of 32 k (two slabs) go from memory straight into LDS (16 bytes a lane, no
+// 32 TM x 128 a block (TM 1 to 4), 4 waves of 16 TM x 64.  Stages of 32 k (two slabs) go from memory straight into LDS (16 bytes a lane, no
 // registers), two stages taking turns: the next one's transfers fly while this one is multiplied, 128 matrix instructions
 // a wave, behind one barrier a stage.  A lane's four k of a slab are one 16-byte read.  An LDS row is 32 k, 128 bytes; its
 // piece u lies at u ^ (row / 2 % 8), so that the 16 rows of a fragment lie in different banks.  Two blocks a compute
@@ -306,6 +306,18 @@ __global__ __launch_bounds__(ROWS_WAVES * 64, MT <= 2 ? 4 : 2) void gemm_f32_row
   }
 }
 
+// Tiles of 32, 64, 96 or 128 rows by 128 columns: what a product takes goes by the tiles of the fullest compute unit, and a narrow
+// tile fills the chip better while a wide one multiplies faster.  Microseconds for K 4 096: one tile a compute unit, and each of
+// several (measured over 2 048 to 28 672 columns of K 2 048 to 14 336 at 65 to 1 200 rows; the shape that this names is within 3 %
+// of the best of the four there, but for 28 672 columns of 433 rows: 964 for 936).  With 64 and 128 rows alone, by which fills the
+// fullest unit less, -> this: 100 rows of 2 048 x 2 048 77 -> 48 us, of 4 096 x 4 096 150 -> 95, of 4 096 x 14 336 514 -> 344, 333 of
+// 6 144 x 4 096 271 -> 212, 600 of 4 096 x 14 336 931 -> 725, 333 of 28 672 x 4 096 793 -> 739, 865 of 6 144 x 4 096 422 -> 409.
+float pipelined_us(int tm, int M, int tiles_n, int K) {
+  constexpr float one[4] = {95.f, 152.f, 211.f, 270.f}, each[4] = {74.5f, 137.f, 201.f, 262.f}, first[4] = {8.f, 0.f, 2.f, 4.f};
+  const long long n = lq_ceil_div64((long long)lq_ceil_div(M, 32 * tm) * tiles_n, lq_compute_units());
+  return (n <= 1 ? one[tm - 1] : first[tm - 1] + each[tm - 1] * n) * K / 4096.f;
+}
+
 template <typename T, typename TO>
 int launch(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc, hipStream_t stream) {
   const int el = (int)sizeof(T);
@@ -329,14 +341,16 @@ int launch(const void* x, const void* w, void* out, int M, int N, int K, int lda
   }
   if constexpr (sizeof(T) == 4) {
     if (wide || (pieces && M > 64 && N > 64 && K % STAGE_K == 0)) {
-      const int tiles_n = lq_ceil_div(N, TILE), cus = lq_compute_units();
-      const long long whole = (long long)lq_ceil_div(M, TILE) * tiles_n, halves = (long long)lq_ceil_div(M, TILE / 2) * tiles_n;
-      LQ_REQUIRE(halves < (1ll << 30), "linear: too many tiles");
-      // tiles of 64 rows where the fullest compute unit then has less to do (865 x 6 144 x 4 096 546 -> 448 us, 300 x 6 144 x
-      // 4 096 282 -> 166; where both come to the same the whole tile is a little faster: 3 623 against 3 841 at 2 048 rows)
-      const bool half = lq_ceil_div64(halves, cus) < 2 * lq_ceil_div64(whole, cus);
-      const long long tiles = half ? halves : whole;
-      const auto kernel = half ? gemm_f32_pipelined_kernel<TO, 2> : gemm_f32_pipelined_kernel<TO, 4>;
+      const int tiles_n = lq_ceil_div(N, TILE);
+      LQ_REQUIRE((long long)lq_ceil_div(M, 32) * tiles_n < (1ll << 30), "linear: too many tiles");
+      int tm = 4;
+      for (int t = 3; t >= 1; --t)
+        if (pipelined_us(t, M, tiles_n, K) < pipelined_us(tm, M, tiles_n, K)) tm = t;
+      const long long tiles = (long long)lq_ceil_div(M, 32 * tm) * tiles_n;
+      const auto kernel = tm == 1   ? gemm_f32_pipelined_kernel<TO, 1>
+                          : tm == 2 ? gemm_f32_pipelined_kernel<TO, 2>
+                          : tm == 3 ? gemm_f32_pipelined_kernel<TO, 3>
+                                    : gemm_f32_pipelined_kernel<TO, 4>;
       kernel<<<(int)((tiles + 7) / 8 * 8), 256, 0, stream>>>((const float*)x, lda, (const float*)w, ldw, (TO*)out, ldc, M, N, K,
                                                             (int)(tiles / tiles_n), tiles_n);
       LQ_CHECK_LAUNCH("linear(float32 pipelined)");

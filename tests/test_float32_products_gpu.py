@@ -23,3 +23,23 @@ def test_a_row_has_the_same_bits_in_every_launch(n, k):
         out = torch.full((rows, n), float("nan"), device="cuda")
         kn.linear(x[:rows], w, out)
         assert torch.equal(out, one[:rows]), rows
+
+
+@pytest.mark.parametrize("n", [2048, 6144])
+def test_a_row_has_the_same_bits_in_every_tile_of_a_wide_weight(n):
+    """Numbers of rows around the edges of tiles of 32, 64, 96 and 128, each of which some of these launches take."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, k = HipKernels(), 544
+    gen = torch.Generator().manual_seed(n)
+    x, w = torch.randn(1201, k, generator=gen).cuda(), torch.randn(n, k, generator=gen).cuda()
+    some = [0, 1, 31, 32, 63, 64, 95, 96, 97, 127, 128, 129, 191, 288, 330, 575, 863, 1151, 1152, 1199, 1200]
+    one = torch.empty(1201, n, device="cuda")
+    for r in some:
+        kn.linear(x[r : r + 1], w, one[r : r + 1])
+    for rows in (65, 95, 96, 97, 161, 257, 289, 333, 600, 865, 1000, 1153, 1201):
+        out = torch.full((rows, n), float("nan"), device="cuda")
+        kn.linear(x[:rows], w, out)
+        mine = [r for r in some if r < rows]
+        assert torch.equal(out[mine], one[mine]), rows
+        assert bool(out.isfinite().all()), rows
