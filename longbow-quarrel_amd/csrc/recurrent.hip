@@ -1453,6 +1453,9 @@ extern "C" int lq_gated_rmsnorm(const float* y, int ldy, const float* z, int ldz
   return 0;
 }
 
+int lq_branches_mean(const float* const* y, const float* const* w, const float* const* b, int n_in, float eps, float* out, int rows,
+                     int width, hipStream_t stream);
+
 // stack [n_in, rows, width] dense float32; w0..w3 the branches' weights [width], b0..b3 their biases [width] or null
 extern "C" int lq_rmsnorm_mean(const float* stack, int n_in, const float* w0, const float* w1, const float* w2,
                                const float* w3, const float* b0, const float* b1, const float* b2, const float* b3,
@@ -1467,6 +1470,8 @@ extern "C" int lq_rmsnorm_mean(const float* stack, int n_in, const float* w0, co
     LQ_REQUIRE(i >= n_in || ws[i] != nullptr, "rmsnorm_mean: branch %d has no weight", i);
   }
   LQ_REQUIRE(stack && out, "rmsnorm_mean: null pointer");
+  const int taken = lq_branches_mean(in.x, in.w, in.b, n_in, eps, out, rows, width, stream);
+  if (taken != 0) return taken < 0 ? taken : 0;
   rmsnorm_mean_kernel<<<rows, width >= 4096 ? 1024 : width >= 1024 ? 256 : 64, 0, stream>>>(in, n_in, eps, out, width);
   LQ_CHECK_LAUNCH("rmsnorm_mean");
   return 0;
