@@ -311,6 +311,140 @@ __global__ __launch_bounds__(256) void qkv_norm_store4_kernel(const float* __res
   }
 }
 
+// The same for many rows, units of a head of 4 LANES entries: LANES lanes a unit.  Queries and keys: a thread takes four rows of its
+// unit, all asked for together.  Values lie in the cache with the positions of an entry side by side: the first row of every
+// aligned run of eight positions (or of a sequence) takes the run, eight rows at once, and writes 16 bytes an entry where the run is
+// whole, in the place of a 2-byte store an entry and row.  A unit's sum of squares is the kernel's above, bit for bit.
+constexpr int QKV_ROWS = 4, RUN = 8;
+
+__device__ inline void store_run8(bf16_t* o, const float (&v)[RUN]) {
+  uint4 packed;
+  uint32_t* u = &packed.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) u[i] = (uint32_t)f32_to_bf16(v[2 * i]).bits | ((uint32_t)f32_to_bf16(v[2 * i + 1]).bits << 16);
+  *(uint4*)o = packed;
+}
+__device__ inline void store_run8(float* o, const float (&v)[RUN]) {
+  ((float4*)o)[0] = make_float4(v[0], v[1], v[2], v[3]), ((float4*)o)[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+
+template <int LANES>
+__device__ inline float unit_sum(float v) {
+#pragma unroll
+  for (int off = LANES / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+template <typename T, int LANES>
+__global__ __launch_bounds__(256) void qkv_norm_store_rows_kernel(const float* __restrict__ src, T* __restrict__ q_out,
+                                                                  T* __restrict__ kcache, T* __restrict__ vcache, QkvUnits a, int rows,
+                                                                  int qk_blocks) {
+  constexpr int UNITS = 256 / LANES, N = 4 * LANES;
+  const int lane = threadIdx.x % LANES, mine = threadIdx.x / LANES, QW = a.H * N, KW = a.G * N, e0 = 4 * lane;
+  const bool stored = kcache != nullptr;
+  auto fetch = [&](int r, int col) {
+    float4 v = *(const float4*)(src + (long long)r * a.lds + col + e0);
+    if (a.bias != nullptr) {
+      const float4 add = *(const float4*)(a.bias + col + e0);
+      v.x += add.x, v.y += add.y, v.z += add.z, v.w += add.w;
+    }
+    return v;
+  };
+  auto rstd = [&](const float4& v) {
+    return 1.f / sqrtf(unit_sum<LANES>(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, 0.f))))) / (float)N + a.eps);
+  };
+  if ((int)blockIdx.x < qk_blocks) {
+    const int units = a.H + (stored ? a.G : 0), per_rows = (units + UNITS - 1) / UNITS;
+    const int u = (int)blockIdx.x % per_rows * UNITS + mine, r0 = (int)blockIdx.x / per_rows * QKV_ROWS;
+    if (u >= units) return;
+    const bool is_q = u < a.H;
+    const int col = u * N;  // (keys lie behind the queries)
+    float4 v[QKV_ROWS];
+#pragma unroll
+    for (int j = 0; j < QKV_ROWS; ++j) v[j] = fetch(min(r0 + j, rows - 1), col);
+    const float* w = is_q ? a.wq : a.wk;
+    const float4 gain = w != nullptr ? *(const float4*)(w + e0) : make_float4(1.f, 1.f, 1.f, 1.f);
+#pragma unroll
+    for (int j = 0; j < QKV_ROWS; ++j) {
+      const int r = min(r0 + j, rows - 1);
+      float x[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+      if (a.cs != nullptr && e0 < a.dims) {
+        const float* cs = a.cs + (long long)r * a.dims;
+        const float *sf = src + (long long)r * a.lds + col, *bf = a.bias != nullptr ? a.bias + col : nullptr;
+        float mate[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (a.interleaved) {
+            mate[k] = x[k ^ 1];
+          } else {
+            const int m = e0 + k < a.dims ? pair_mate(a, e0 + k) : e0;
+            mate[k] = bf != nullptr ? sf[m] + bf[m] : sf[m];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (e0 + k < a.dims) x[k] = turned_entry(a, cs, e0 + k, x[k], mate[k]);
+      }
+      if (a.norm_qk) {
+        const float inv = rstd(make_float4(x[0], x[1], x[2], x[3]));
+        x[0] *= inv, x[1] *= inv, x[2] *= inv, x[3] *= inv;
+      }
+      if (w != nullptr) x[0] *= gain.x, x[1] *= gain.y, x[2] *= gain.z, x[3] *= gain.w;
+      if (r0 + j >= rows) continue;
+      T* o;
+      if (is_q) {
+        o = q_out + (long long)r * a.ldq + col + e0;
+      } else {
+        const int p = a.row_pos[r];
+        const long long blk = a.block_table[(long long)a.seq_slot[a.row_seq[r]] * a.bt_stride + p / a.BS];
+        o = kcache + ((blk * a.G + u - a.H) * a.BS + p % a.BS) * N + e0;
+      }
+      if constexpr (sizeof(T) == 4) {
+        *(float4*)o = make_float4(x[0], x[1], x[2], x[3]);
+      } else {
+        uint2 packed;
+        packed.x = (uint32_t)f32_to_bf16(x[0]).bits | ((uint32_t)f32_to_bf16(x[1]).bits << 16);
+        packed.y = (uint32_t)f32_to_bf16(x[2]).bits | ((uint32_t)f32_to_bf16(x[3]).bits << 16);
+        *(uint2*)o = packed;
+      }
+    }
+    return;
+  }
+  // values (V = N entries a head)
+  const int per_row = (a.G + UNITS - 1) / UNITS, at = (int)blockIdx.x - qk_blocks, r = at / per_row, u = at % per_row * UNITS + mine;
+  const int p = a.row_pos[r], seq = a.row_seq[r];
+  if (p % RUN != 0 && r > 0 && a.row_seq[r - 1] == seq && a.row_pos[r - 1] == p - 1) return;  // (the whole workgroup: another row takes it)
+  const int i0 = threadIdx.x & 63, ri = min(r + i0, rows - 1);  // (a lane looks at a row of the run: one trip to memory)
+  const bool follows = i0 < RUN - p % RUN && r + i0 < rows && a.row_seq[ri] == seq && a.row_pos[ri] == p + i0;
+  const int n = __ffsll(~(unsigned long long)__ballot(follows)) - 1;  // rows of the run, one at least
+  if (u >= a.G) return;
+  const int col = (a.v_from_k ? QW : QW + KW) + u * N;
+  float4 v[RUN];
+#pragma unroll
+  for (int i = 0; i < RUN; ++i) v[i] = fetch(r + min(i, n - 1), col);
+  if (a.norm_v)
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) {
+      const float inv = rstd(v[i]);
+      v[i].x *= inv, v[i].y *= inv, v[i].z *= inv, v[i].w *= inv;
+    }
+  const long long blk = a.block_table[(long long)a.seq_slot[seq] * a.bt_stride + p / a.BS];
+  T* o = vcache + ((blk * a.G + u) * (long long)N + e0) * a.BS + p % a.BS;
+#pragma unroll
+  for (int k = 0; k < 4; ++k, o += a.BS) {
+    float x[RUN];
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) x[i] = k == 0 ? v[i].x : k == 1 ? v[i].y : k == 2 ? v[i].z : v[i].w;
+    if (n == RUN) {
+      store_run8(o, x);
+    } else {
+#pragma unroll
+      for (int i = 0; i < RUN; ++i)
+        if (i < n) o[i] = from_f32<T>(x[i]);
+    }
+  }
+}
+
 // A product a head: out[r, h ohs + n] = sum_k x[r, h K + k] w[h, n, k], bfloat16 operands on
 // v_mfma_f32_16x16x16_bf16 or 16x16x32 (exact products, 32-bit sums).  A workgroup of four wavefronts takes 64 rows by 64
 // columns of one head; a wavefront 16 rows by the 64 columns, its operands straight from memory (a head's weight
@@ -582,6 +716,26 @@ extern "C" int lq_qkv_norm_store(const float* src, int lds_, const float* bias, 
   const bool fours = key_dim % 4 == 0 && value_dim % 4 == 0 && lds_ % 4 == 0 && ldq % 4 == 0 && (uintptr_t)src % 16 == 0 &&
                      (uintptr_t)bias % 16 == 0 && (uintptr_t)wq % 16 == 0 && (uintptr_t)wk % 16 == 0 &&
                      (uintptr_t)q_out % (4 * el) == 0 && (uintptr_t)kcache % (4 * el) == 0 && most <= 16384;
+  // many rows of heads of 64, 128 or 256, one size for keys and values: the kernel that takes runs of rows.  Microseconds, 16 query
+  // heads of 128 over 4, by units and by runs: 64 rows 4.2 / 7.3, 500 rows 8.3 / 9.3, 800 rows 11.9 / 10.5, 2 000 rows 26.2 / 16.0,
+  // 2 635 rows 33.2 / 21.4, 4 096 rows 48.8 / 31.1
+  const bool runs = fours && rows >= 640 && unit_q == key_dim && unit_k == key_dim && (kcache == nullptr || (unit_v == value_dim && value_dim == key_dim)) &&
+                    (key_dim == 64 || key_dim == 128 || key_dim == 256) && block_size % RUN == 0 && (uintptr_t)vcache % 16 == 0 &&
+                    (long long)rows * (heads + kv_heads) < (1ll << 30);
+  if (runs) {
+    const int in_block = 1024 / key_dim, qk = heads + (kcache != nullptr ? kv_heads : 0);
+    const int qk_blocks = lq_ceil_div(rows, QKV_ROWS) * lq_ceil_div(qk, in_block);
+    const int blocks = qk_blocks + (kcache != nullptr ? rows * lq_ceil_div(kv_heads, in_block) : 0);
+#define LQ_QKV_ROWS(T)                                                                                                          \
+  (key_dim == 64 ? qkv_norm_store_rows_kernel<T, 16> : key_dim == 128 ? qkv_norm_store_rows_kernel<T, 32> : qkv_norm_store_rows_kernel<T, 64>) \
+      <<<blocks, 256, 0, stream>>>(src, (T*)q_out, (T*)kcache, (T*)vcache, a, rows, qk_blocks)
+    if (dtype == LQ_F32) LQ_QKV_ROWS(float);
+    else if (dtype == LQ_BF16) LQ_QKV_ROWS(bf16_t);
+    else LQ_REQUIRE(false, "qkv_norm_store: unknown dtype %d", dtype);
+#undef LQ_QKV_ROWS
+    LQ_CHECK_LAUNCH("qkv_norm_store(rows)");
+    return 0;
+  }
 #define LQ_QKV4(T, WIDE, PER)                                                                                        \
   qkv_norm_store4_kernel<T, WIDE, PER><<<grid, 256, 0, stream>>>(src, (T*)q_out, (T*)kcache, (T*)vcache, a)
 #define LQ_QKV(T)                                                                                                    \

@@ -132,7 +132,7 @@ class SinkWindowAttention(Mixer):
                              "part, `qk_norm_eps` or a gate a head")
         if rotary is not None and qk_norm == "row":
             raise ValueError("a norm over all heads of a row together is not combined with a rotation ahead of it")
-        # without any of those, q, k and v pass the kernel that rotates and norms them (`rotary_qkv`)
+        # a rotation or a norm without a weight alone takes the same kernel
         self.prepared = not self.stored and (rotary is not None or qk_norm_eps is not None)
         if self.values_from_keys and key_dim != value_dim:
             raise ValueError(f"values that are the keys are as wide as they are ({key_dim}, {value_dim})")
@@ -257,8 +257,8 @@ class SinkWindowAttention(Mixer):
         total = sum(n for _, n in self._projections())
         total_padded = (total + 3) // 4 * 4  # rows of the product start on 16 bytes
         wide_gate = None
-        if self.stored:
-            # biases and norms are taken on the product's 32-bit result; keys and values go straight into the cache
+        if self.stored or self.prepared:
+            # biases, rotations and norms are taken on the product's 32-bit result; keys and values go straight into the cache
             proj = ctx.ws.alloc((rows, total_padded), torch.float32)[:, :total]
             project(kn, ctx, h, self.w_in, proj)
             q, k, v, gate = ctx.ws.alloc((rows, self.q_width), ctx.dtype), None, None, None
@@ -268,21 +268,12 @@ class SinkWindowAttention(Mixer):
             if self.rot_dims:
                 place.update(cos_sin=step_angles(ctx, self.freqs, self.freq_table), interleaved=self.rot_interleaved,
                              magnitude=self.rot_magnitude)
-            kn.qkv_norm_store(proj[:, :n_qkv], q, self.heads, self.kv_heads, self.key_dim, self.value_dim, self.norm_eps,
-                              bias=self.in_bias, q_weight=self.q_norm_w, k_weight=self.k_norm_w,
-                              norm_qk="head" if self.qk_norm == "unit" else self.qk_norm,
-                              norm_v=self.value_norm, v_from_k=self.values_from_keys, **place)
+            normed = "head" if self.qk_norm == "unit" or self.qk_norm_eps is not None else self.qk_norm
+            kn.qkv_norm_store(proj[:, :n_qkv], q, self.heads, self.kv_heads, self.key_dim, self.value_dim,
+                              self.norm_eps if self.qk_norm_eps is None else self.qk_norm_eps, bias=self.in_bias,
+                              q_weight=self.q_norm_w, k_weight=self.k_norm_w, norm_qk=normed, norm_v=self.value_norm,
+                              v_from_k=self.values_from_keys, **place)
             wide_gate = proj[:, n_qkv:] if self.entry_gate else None
-        elif self.prepared:
-            # the product's 32-bit result is rotated and normed in 32-bit, then rounded to what the cache holds
-            proj = ctx.ws.alloc((rows, total_padded), torch.float32)[:, :total]
-            project(kn, ctx, h, self.w_in, proj)
-            q = ctx.ws.alloc((rows, self.q_width), ctx.dtype)
-            k = ctx.ws.alloc((rows, self.k_width), ctx.dtype)
-            v = ctx.ws.alloc((rows, self.v_width), ctx.dtype)
-            gate = None
-            kn.rotary_qkv(proj, q, k, v, self.heads, self.kv_heads, self.key_dim, self.value_dim, self.rot_dims,
-                          self.rot_interleaved, self.freqs, self.rot_magnitude, self.qk_norm_eps, ctx.row_pos)
         else:
             # q, k and v in the run's dtype (what the cache holds); the gate's logits ride in the same product
             proj = ctx.ws.alloc((rows, total_padded), ctx.dtype)[:, :total]
