@@ -1,4 +1,4 @@
-"""Compiles csrc/*.hip for gfx950 into one shared library with hipcc.
+"""Compiles csrc/*.hip for gfx950 into one shared library with hipcc, and csrc/host/host_calls.cpp into a Python module beside it.
 
 `ensure_built()` is what the kernel loader calls: it compiles when no library
 matching the sources' hash is there, into `_lib/` beside the package or, if that
@@ -21,6 +21,8 @@ from typing import List, Optional
 PKG_DIR = os.path.dirname(os.path.realpath(__file__))
 SRC_DIR = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "liblqkernels.so"
+HOST_NAME = "lqhost.so"
+HOST_SRC = os.path.join(SRC_DIR, "host", "host_calls.cpp")
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}",
@@ -48,7 +50,7 @@ def _headers() -> List[str]:
 def source_hash() -> str:
     h = hashlib.sha256()
     h.update(" ".join(FLAGS).encode())
-    for path in _sources() + _headers():
+    for path in _sources() + _headers() + [HOST_SRC]:
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
             h.update(f.read())
@@ -88,7 +90,7 @@ def find_built() -> Optional[str]:
     for d in lib_dirs():
         lib = os.path.join(d, LIB_NAME)
         stamp = os.path.join(d, LIB_NAME + ".hash")
-        if os.path.isfile(lib) and os.path.isfile(stamp):
+        if os.path.isfile(lib) and os.path.isfile(stamp) and os.path.isfile(os.path.join(d, HOST_NAME)):
             with open(stamp) as f:
                 if f.read().strip() == want:
                     return lib
@@ -97,6 +99,27 @@ def find_built() -> Optional[str]:
 
 def _log(msg: str) -> None:
     print(f"[longbow-quarrel_amd build] {msg}", file=sys.stderr, flush=True)
+
+
+def build_host(out_dir: str, env) -> None:
+    """The Python module of the launches' host side, against this interpreter's and this torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++") or shutil.which("clang++")
+    if not cxx:
+        raise BuildError("no C++ compiler for the launches' host side (looked at $CXX, g++, c++, clang++)")
+    tmp = os.path.join(out_dir, f".{HOST_NAME}.{os.getpid()}")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for path in include_paths() + [sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", path]
+    cmd += [HOST_SRC, "-o", tmp] + [f"-L{path}" for path in library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+    if proc.returncode != 0:
+        raise BuildError(f"{cxx} failed on {HOST_SRC}:\n{proc.stderr[-4000:]}")
+    os.replace(tmp, os.path.join(out_dir, HOST_NAME))
 
 
 def build(force: bool = False, jobs: Optional[int] = None) -> str:
@@ -129,7 +152,9 @@ def build(force: bool = False, jobs: Optional[int] = None) -> str:
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(build_host, out_dir, env)
         objs = list(pool.map(compile_one, srcs))
+        host.result()
     lib_tmp = os.path.join(out_dir, f".{LIB_NAME}.{os.getpid()}")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", lib_tmp]
     proc = subprocess.run(cmd, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)

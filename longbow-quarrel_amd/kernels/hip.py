@@ -1,4 +1,4 @@
-"""The hand-written gfx950 kernels, bound through ctypes.
+"""The hand-written gfx950 kernels, bound through ctypes (a prompt's most frequent launches through a module of their own).
 
 `HipKernels` is the only compute backend of the library.  Every method checks
 on the host what its kernel and grid assume (dtype, device, contiguity, sizes),
@@ -11,6 +11,9 @@ here.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
+import os
 from ctypes import c_double, c_float, c_int, c_longlong, c_void_p
 from typing import Optional
 
@@ -20,7 +23,7 @@ from .. import build as _build
 from .dry import query
 
 F32, BF16 = 0, 1
-ABI_VERSION = 18  # lq_abi_version() of the library these wrappers were written for
+ABI_VERSION = 19  # lq_abi_version() of the library these wrappers were written for
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -61,8 +64,32 @@ def load_library() -> ctypes.CDLL:
     lib.lq_attention.argtypes = [vp, ci, vp, ci, ci, ci, ci, ci, ci, ci, vp, vp, vp, vp, vp, ci, vp, vp, ci, cf, ci, ci, ci,
                                  vp, cl, vp, cl, vp, vp, ci, ci, vp, ci, ci, cl, ci, vp]
     lib.lq_rope_store_pieces.argtypes = [vp, ci, ci, cl, vp, ci, ci, ci, ci, ci, vp, vp, vp, vp, vp, ci, vp, vp, ci, vp]
+    lib.lq_linear_splits.argtypes = lib.lq_linear_narrow_splits.argtypes = [ci] * 5
+    lib.lq_linear_fused_parts.argtypes = [ci] * 4
     _LIB = lib
     return lib
+
+
+_HOST = None
+
+
+def load_host():
+    """The module that makes a prompt's launches in C++ (csrc/host/host_calls.cpp), told where the library's functions are."""
+    global _HOST
+    if _HOST is None:
+        lib = load_library()
+        path = os.path.join(os.path.dirname(lib._name), _build.HOST_NAME)
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("lqhost", path)
+            host = importlib.util.module_from_spec(importlib.util.spec_from_file_location("lqhost", path, loader=loader))
+            loader.exec_module(host)
+        except (ImportError, OSError) as e:
+            raise KernelLibraryError(f"cannot load {path}: {e}") from e
+        host.use(*(ctypes.cast(fn, c_void_p).value for fn in (
+            lib.lq_linear, lib.lq_linear_splits, lib.lq_linear_narrow_splits, lib.lq_linear_swiglu, lib.lq_rmsnorm, lib.lq_attention,
+            lib.lq_rope_store_pieces)))
+        _HOST = host
+    return _HOST
 
 
 def _ptr(t: Optional[torch.Tensor]) -> c_void_p:
@@ -124,6 +151,7 @@ class HipKernels:
 
     def __init__(self) -> None:
         self.lib = load_library()
+        self.host = load_host()
         if not torch.cuda.is_available():
             raise KernelLibraryError("no HIP device is visible; this library runs on a gfx950 GPU only")
         self._stream: Optional[int] = None
@@ -155,9 +183,16 @@ class HipKernels:
 
     @property
     def stream(self) -> c_void_p:
-        if self._stream is not None:
-            return c_void_p(self._stream)
-        return c_void_p(int(torch.cuda.current_stream().cuda_stream))
+        return c_void_p(self._stream_number())
+
+    def _stream_number(self) -> int:
+        return self._stream if self._stream is not None else int(torch.cuda.current_stream().cuda_stream)
+
+    def _launched(self, rc: int) -> bool:
+        """What a function of the host module says: launched (True), or that the checks here are to find out (False)."""
+        if rc < 0:
+            self._check(rc)
+        return rc > 0
 
     def _check(self, rc: int) -> None:
         if rc != 0:
@@ -261,6 +296,8 @@ class HipKernels:
     def rmsnorm(self, x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor,
                 delta: Optional[torch.Tensor] = None) -> None:
         """(x += delta;) out = x / sqrt(mean(x^2) + eps) * weight, row by row; x is float32."""
+        if self._launched(self.host.rmsnorm(x, weight, eps, out, delta, self._stream_number())):
+            return
         rows, width, ldx = self._mat(x, "rmsnorm: x")
         if delta is not None:
             self._dev(delta)
@@ -312,8 +349,7 @@ class HipKernels:
         [pieces, M, N]; the kernel then splits K over more blocks and each piece is a partial sum."""
         if dtype not in _DTYPE_CODE:
             return 1
-        return int(self.lib.lq_linear_splits(c_int(_DTYPE_CODE[dtype]), c_int(m), c_int(n), c_int(k),
-                                             c_int(1 if self.force_generic else 0)))
+        return self.lib.lq_linear_splits(_DTYPE_CODE[dtype], m, n, k, 1 if self.force_generic else 0)
 
     @query
     def linear_narrow_pieces(self, dtype: torch.dtype, m: int, n: int, k: int) -> int:
@@ -321,12 +357,13 @@ class HipKernels:
         rows of its own and a long K."""
         if dtype not in _DTYPE_CODE:
             return 1
-        return int(self.lib.lq_linear_narrow_splits(c_int(_DTYPE_CODE[dtype]), c_int(m), c_int(n), c_int(k),
-                                                    c_int(1 if self.force_generic else 0)))
+        return self.lib.lq_linear_narrow_splits(_DTYPE_CODE[dtype], m, n, k, 1 if self.force_generic else 0)
 
     def linear(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
         """out[M, N] = x[M, K] . w[N, K]^T with 32-bit accumulation; or out[pieces, M, N] with
         `linear_pieces` pieces that sum to it."""
+        if self._launched(self.host.linear(x, w, out, 1 if self.force_generic else 0, self._stream_number())):
+            return
         m, k, ldx = self._mat(x, "linear: x")
         n, kw, ldw = self._mat(w, "linear: w")
         pieces, stride = 1, 0
@@ -385,7 +422,7 @@ class HipKernels:
         not take the size (use `linear` and `rmsnorm`)."""
         if self.force_generic or dtype not in _DTYPE_CODE:
             return 0
-        return int(self.lib.lq_linear_fused_parts(c_int(_DTYPE_CODE[dtype]), c_int(m), c_int(n), c_int(k)))
+        return self.lib.lq_linear_fused_parts(_DTYPE_CODE[dtype], m, n, k)
 
     def linear_residual(self, act: torch.Tensor, w: torch.Tensor, x: torch.Tensor, sq_parts: torch.Tensor,
                         gain: Optional[torch.Tensor] = None, scaled: Optional[torch.Tensor] = None) -> None:
@@ -445,6 +482,9 @@ class HipKernels:
         of gelu, "relu": relu in silu's place (bfloat16 out).  w [2 I, K] holds the
         gate and up rows interleaved in groups of 8: rows 16j..16j+7 gate 8j..8j+7, rows 16j+8..16j+15
         up 8j..8j+7 (see `interleave_gate_up`)."""
+        if activation in self._GLU_FORMS and self._launched(
+                self.host.linear_swiglu(x, w, out, self._GLU_FORMS[activation], self._stream_number())):
+            return
         m, k, ldx = self._mat(x, "linear_swiglu: x")
         n, kw, ldw = self._mat(w, "linear_swiglu: w")
         mo, no, ldc = self._mat(out, "linear_swiglu: out")
@@ -511,6 +551,9 @@ class HipKernels:
         the projection with q, k and v side by side: adds the pieces in ascending order, rounds the sums to
         bfloat16 as the whole product would have, rotates q (into q_out, bfloat16 [rows, heads * head_dim])
         and k, and writes k and v into the paged cache."""
+        if self._launched(self.host.rope_store_pieces(qkv, q_out, heads, kv_heads, head_dim, freqs, row_pos, row_seq, seq_slot,
+                                                      block_table, kcache, vcache, block_size, self._stream_number())):
+            return
         self._dev(qkv, q_out, freqs, row_pos, row_seq, seq_slot, block_table, kcache, vcache)
         if qkv.dim() != 3 or qkv.dtype != torch.float32 or not qkv.is_contiguous() \
                 or qkv.shape[2] != (heads + 2 * kv_heads) * head_dim:
@@ -681,6 +724,10 @@ class HipKernels:
         the cache itself.  With `pieces` > 1 (such a launch only, where `attention_adds_pieces` says so)
         q, k_new and v_new are float32 views into the first of that many partial sums of the projection,
         `piece_stride` elements apart (what `linear` leaves in a 3-D out): the launch adds them up."""
+        if not decode and workspace is None and cos_sin is None and pieces == 1 and self.host.attention(
+                q, out, heads, kv_heads, head_dim, row_pos, row_seq, seq_slot, cu_rows, block_table, kcache, vcache, block_size, scale,
+                window, max_len, self.tickets(q.device), 1 if self.force_generic else 0, self._stream_number()) > 0:
+            return
         self._dev(q, out, row_pos, row_seq, seq_slot, cu_rows, block_table, kcache, vcache, workspace)
         rows = q.shape[0]
         batch = seq_slot.numel()
