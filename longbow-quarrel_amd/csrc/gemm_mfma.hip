@@ -946,6 +946,96 @@ __global__ __launch_bounds__(KW * 64) void gemm_bf16_skinny_v3_kernel(const bf16
   }
 }
 
+// ------------------------------------------------------------------ at most 8 rows, 8 columns a block
+// A weight of few columns gives the balanced kernel 8 columns a block, half of a matrix instruction's, and its waves wait for 256 k
+// at a time.  Here the 8 rows of x and 8 columns of W of 64 k fill one half of the instruction's rows and columns and those of the
+// next 64 k the other: D's two diagonal quarters are the two sums (the others are of no use), every lane's load is one of its own,
+// and a wave's chunks of 128 k (every sixteenth) are asked for four at a time ahead of the products.
+template <int EPI, typename TO, bool PACKED>
+__global__ __launch_bounds__(1024) void gemm_bf16_pair_kernel(const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int ldw,
+                                                              TO* __restrict__ C, int ldc, int M, int N, int K, ResidualOut res) {
+  constexpr int KW = 16, CHUNK = 128, DEPTH = 4;
+  __shared__ float red[KW][256];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), g = lane >> 4, c16 = lane & 15;
+  const int n0 = blockIdx.x * 8, n = n0 + (c16 & 7), half = c16 >> 3;  // (a dense weight's last columns may be fewer than 8)
+  const bf16_t* wp = PACKED ? W + (long long)n0 * ldw + (c16 & 7) * 64 + half * 512 + g * 8 : W + (long long)min(n, N - 1) * ldw + half * 64 + g * 8;
+  const bf16_t* xp = X + (long long)min(c16 & 7, M - 1) * ldx + half * 64 + g * 8;
+  const int mine = (K / CHUNK - wave + KW - 1) / KW;  // this wave's chunks (none: 0 or less)
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  u32x4 wv[DEPTH][2], xv[DEPTH][2];
+  auto ask = [&](int d, int i) {
+    const int k = (wave + KW * i) * CHUNK;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      wv[d][j] = i < mine ? *(const u32x4*)(wp + (PACKED ? k * 8ll : k) + 32 * j) : zero;
+      xv[d][j] = i < mine ? *(const u32x4*)(xp + k + 32 * j) : zero;
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) ask(d, d);
+  // the row (of D's upper quarter) and column that this lane finishes, four waves' worth of them
+  const int row = 4 * g + wave;
+  const bool ends = wave < 4 && c16 < 8 && row < M && n < N;
+  float old = 0.f, gain = 0.f;
+  if constexpr (EPI == EPI_RESIDUAL) {
+    if (ends) {
+      old = C[(long long)row * ldc + n];
+      if (res.gain != nullptr) gain = res.gain[n];
+    }
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < mine; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xv[d][j]), as_bf16x8(wv[d][j]), acc, 0, 0, 0);
+      if (i + DEPTH < mine) ask(d, i + d + DEPTH);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) red[wave][e * 64 + lane] = acc[e];
+  __syncthreads();
+  if (wave >= 4) return;
+  float s = 0.f;
+  if (ends) {
+#pragma unroll
+    for (int w = 0; w < KW; ++w) s += red[w][wave * 64 + lane] + red[w][wave * 64 + lane + 40];  // (and row + 8, column + 8)
+  }
+  if constexpr (EPI == EPI_RESIDUAL) {
+    const float fresh = ends ? old + s : 0.f;
+    float sq = fresh * fresh;
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);  // the block's 8 columns
+    if (!ends) return;
+    C[(long long)row * ldc + n] = fresh;
+    if (res.scaled != nullptr) res.scaled[(long long)row * res.ld_scaled + n] = f32_to_bf16(fresh * gain);
+    if (c16 == 0) res.sq_out[(long long)row * gridDim.x + blockIdx.x] = sq;
+  } else if (ends) {
+    store_out<TO>(C + (long long)row * ldc + n, s);
+  }
+}
+
+// Up to 8 columns a compute unit, and where that is what the balanced kernel has too (2 048 columns), few rows or a K whose chunks
+// are all in flight at once: beyond, rows of x take as long as the weight, and the balanced kernel reads them in longer runs.
+// Microseconds before (the simple kernel below 2 048 columns, the balanced one) and here, at 1, 4 and 8 rows: 128 x 2 048 4.2 / 3.2,
+// 5.0 / 3.7, 5.3 / 4.1; 1 024 x 3 584 6.6 / 5.0, 7.5 / 5.8, 8.3 / 6.4; 1 536 x 5 376 9.6 / 7.2, 10.6 / 7.9, 11.7 / 8.8; 2 048 x 2 048 5.1 /
+// 4.5, 5.3 / 4.8, 5.5 / 5.1; 2 048 x 4 096 7.4 / 6.2, 7.4 / 7.1, 7.9 / 7.9; 2 048 x 8 192 12.2 / 9.5, 12.4 / 11.5, 12.7 / 13.4; 3 072 x 3 072
+// 7.4 / 7.8, 7.9 / 8.8, 8.0 / 9.8; 4 096 x 14 336 26.7 / 26.6, 27.1 / 31.8, 29.6 / 38.0.
+inline bool takes_pairs(int M, int N, int K) {
+  const int cus = lq_compute_units();
+  return M <= 8 && K % 128 == 0 && K >= 512 && (N < 8 * cus || (N == 8 * cus && (M <= 4 || K <= 4096)));
+}
+
+template <int EPI, typename TO>
+int launch_pairs(const void* X, const void* W, void* C, int M, int N, int K, int ldx, int ldw, int ldc, hipStream_t stream, int packed,
+                 ResidualOut res = ResidualOut()) {
+  const auto kernel = packed ? gemm_bf16_pair_kernel<EPI, TO, true> : gemm_bf16_pair_kernel<EPI, TO, false>;
+  kernel<<<lq_ceil_div(N, 8), 1024, 0, stream>>>((const bf16_t*)X, ldx, (const bf16_t*)W, ldw, (TO*)C, ldc, M, N, K, res);
+  LQ_CHECK_LAUNCH("linear(mfma pairs)");
+  return 0;
+}
+
 // How many blocks should share K for an [M, K] x [N, K]^T product with the balanced kernel (1: no
 // split).  With several row tiles a block wants several column tiles too, so that the x fragments it
 // holds are used more than once; a matrix with few columns gets them by giving each block a wider run
@@ -1186,7 +1276,7 @@ int launch_rows(const void* x, const void* w, void* out, int M, int N, int K, in
 // Shares of K for up to 16 rows of a weight with so few columns that its tiles of 16 leave most of the chip idle and
 // one of them walks a long K: asked for by callers that add the pieces up right away (`lq_linear_narrow_splits`).
 int narrow_splits(int M, int N, int K) {
-  if (M > 16 || N >= 8 * lq_compute_units() || K % 64 != 0) return 1;
+  if (M > 16 || N >= 8 * lq_compute_units() || K % 64 != 0 || takes_pairs(M, N, K)) return 1;
   int splits = 1;
   while (splits < 16 && lq_ceil_div(N, 16) * splits * 2 <= 2 * lq_compute_units() && K % (128 * splits) == 0 &&
          K / (splits * 2) >= 1024)
@@ -1221,6 +1311,8 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
     if (M <= 32) return launch_skinny_v3<2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
     return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   }
+  if constexpr (EPI == EPI_NONE)
+    if (takes_pairs(M, N, K)) return launch_pairs<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, stream, packed);
   // wide enough to give every compute unit a run of columns: the balanced kernel; else the simple one
   const bool wide = N >= 8 * lq_compute_units() && K >= 512;
   if (M <= 16) {
@@ -1268,6 +1360,9 @@ int lq_gemm_residual(const void* act, const void* w, float* x, float* sq_out, co
   res.gain = gain;
   res.scaled = (bf16_t*)scaled;
   res.ld_scaled = ld_scaled;
+  // (a block of 8 columns leaves one part either way: lq_gemm_fused_parts)
+  if (takes_pairs(M, N, K) && N == 8 * lq_compute_units())
+    return launch_pairs<EPI_RESIDUAL, float>(act, w, x, M, N, K, lda, ldw, ldx, stream, packed, res);
   return launch_skinny_v3<1, EPI_RESIDUAL, float>(act, w, x, M, N, K, lda, ldw, ldx, 1, 0, stream, packed, RowScale(), res);
 }
 

@@ -1,0 +1,49 @@
+"""Products of at most 8 rows and 8 columns a compute unit, around the edges of chunks of 128 k and blocks of 8 columns."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 7, 8])
+@pytest.mark.parametrize("n,k", [(1, 512), (8, 640), (9, 2048), (136, 2176), (1000, 4096), (1536, 5376), (2048, 512), (2048, 1920), (2048, 8320)])
+def test_products(rows, n, k):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    gen = torch.Generator().manual_seed(n + k)
+    x, w = torch.randn(rows, k + 8, generator=gen).bfloat16().cuda()[:, :k], torch.randn(n, k, generator=gen).bfloat16().cuda()
+    want = x.double() @ w.double().T
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)  # (products of bfloat16 are exact; a rounding a term)
+    wide = torch.full((rows, n + 5), 7.0, device="cuda")
+    for held in (w, kn.pack_weight(w)):
+        kn.linear(x, held, wide[:, :n])
+        assert ((wide[:, :n] - want).abs() <= bound).all() and bool((wide[:, n:] == 7.0).all())
+    narrow = torch.empty(rows, n, dtype=torch.bfloat16, device="cuda")
+    kn.linear(x, w, narrow)
+    assert ((narrow - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()
+    # an infinity or NaN in one row or column stays there
+    x2, w2 = x.clone(), w.clone()
+    x2[0, k - 1], w2[n - 1, 3] = float("inf"), float("nan")
+    kn.linear(x2, w2, wide[:, :n])
+    assert not bool(wide[0, :n].isfinite().any()) and bool(wide[:, n - 1].isnan().all())
+    if rows > 1 and n > 1:
+        assert ((wide[1:, : n - 1] - want[1:, : n - 1]).abs() <= bound[1:, : n - 1]).all()
+
+
+@pytest.mark.parametrize("rows,k", [(1, 512), (4, 8192), (8, 4096), (8, 8192), (3, 2176)])
+def test_into_the_stream(rows, k):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, n = HipKernels(), 2048
+    gen = torch.Generator().manual_seed(k)
+    act, w = torch.randn(rows, k, generator=gen).bfloat16().cuda(), kn.pack_weight(torch.randn(n, k, generator=gen).bfloat16().cuda() * 0.1)
+    x, gain = torch.randn(rows, n, generator=gen).cuda(), torch.randn(n, generator=gen).cuda()
+    plain = torch.empty(rows, n, device="cuda")
+    kn.linear(act, w, plain)
+    parts = kn.linear_fused_parts(torch.bfloat16, rows, n, k)
+    assert parts > 0
+    sq, scaled, got = torch.full((rows, parts), 7.0, device="cuda"), torch.empty(rows, n, dtype=torch.bfloat16, device="cuda"), x.clone()
+    kn.linear_residual(act, w, got, sq, gain=gain, scaled=scaled)
+    assert torch.equal(got, x + plain) and torch.equal(scaled, (got * gain).bfloat16())
+    assert ((sq.double().sum(1) - (got.double() ** 2).sum(1)).abs() <= 2048 * 2.0 ** -24 * (got.double() ** 2).sum(1)).all()
