@@ -197,17 +197,23 @@ __global__ __launch_bounds__(256) void ssd_chunk_chain_kernel(SsdArgs a) {
     if (p < a.P && n + e < a.N) sp[n + e] = S[e];
 }
 
+// (64 channels at a time: 70 KB of LDS, two workgroups a compute unit, whose loads, decays and products overlap)
+constexpr int RUN = 64, RT = RUN / 16, LDR = RUN + 4;
+
 struct OutLds {
-  float C[CHUNK][LDN], B[CHUNK][LDN], x[CHUNK][LDX];
+  float C[CHUNK][LDR], B[CHUNK][LDR], x[CHUNK][LDX];
   float G[CHUNK][LDX];  // first f_st s_s, then that times C_t . B_s
   float decay[CHUNK], step[CHUNK], from_start[CHUNK];
   int odd;  // x or B has an entry that is no finite number
 };
 
 // A chunk's results.  One workgroup of eight wavefronts a (chunk, head, 64 columns): wavefronts w and w + 4 take 16
-// columns, the first its first 32 tokens and the second its last.
+// columns, the first its first 32 tokens and the second its last.  A workgroup is a chain of trips to memory, the decays' products
+// and 4 microseconds of matrix instructions; one a compute unit (128 channels at a time), with the decays' products of 64 tokens in
+// one wavefront's row, took 17.  32 heads of 128 x 64, 2 048 tokens: 68
+// -> 46 us.
 template <bool QUADS>
-__global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
+__global__ __launch_bounds__(512, 4) void ssd_chunk_out_kernel(SsdArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   OutLds& L = *(OutLds*)smem;
   const Part at = find_part(a.cu_rows, a.batch, CHUNK, a.least, a.first + blockIdx.x);
@@ -219,14 +225,10 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   const float* start = a.scratch + place * part_floats(a.N, a.P);
   const int my_pt = min(p0 / 16 + pt, tiles_p - 1);
   Slab<COLS, 512, QUADS> xs;
-  Slab<HALF, 512, QUADS> cs, bs;
-  f32x4 S[NT];
+  Slab<RUN, 512, QUADS> cs, bs;
   auto ask = [&](int n0) {
     cs.fetch(a.C + r0 * a.ldc + (long long)grp * a.N + n0, a.ldc, nt, a.N - n0);
     bs.fetch(a.B + r0 * a.ldb + (long long)grp * a.N + n0, a.ldb, nt, a.N - n0);
-#pragma unroll
-    for (int nb = 0; nb < NT; ++nb)
-      S[nb] = *(const f32x4*)(start + (((long long)(n0 / 16 + nb) * tiles_p + my_pt) * 64 + lane) * 4);
   };
   ask(0);
   xs.fetch(a.x + r0 * a.ldx + (long long)h * Px + p0, a.ldx, nt, Px - p0);
@@ -238,13 +240,33 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
   for (int i = 0; i < xs.PER; ++i) nan_if = not_finite(xs.v[i], nan_if);
   __syncthreads();
   if (a.ones && tid < nt && Px >= p0 && Px < p0 + COLS) L.x[tid][Px - p0] = 1.f;
-  if (w == 7) {  // lane s: f_st s_s for every t
+  if (w >= KT) {  // f_st s_s, lane s: wavefront KT + j the 16 tokens t of block j
+    const int j = w - KT, blk = lane >> 4;
+    float v = L.decay[lane];  // the products of a block's decays from a token to the block's end
+#pragma unroll
+    for (int off = 1; off < SUB; off <<= 1) {
+      const float later = __shfl_down(v, off, 64);
+      if ((lane & 15) + off < SUB) v *= later;
+    }
+    const float after = __shfl_down(v, 1, 64);
     float f = L.step[lane];
-    for (int t = 0; t < CHUNK; ++t) {
+    if (blk < j) {  // what lies between the token and block j
+      if ((lane & 15) < SUB - 1) f *= after;
+    } else if (blk > j) {
+      f = 0.f;
+    }
+#pragma unroll
+    for (int i = 1; i < KT - 1; ++i) {
+      const float whole = __shfl(v, SUB * i, 64);
+      if (blk < i && i < j) f *= whole;
+    }
+#pragma unroll
+    for (int i = 0; i < SUB; ++i) {
+      const int t = SUB * j + i;
       if (t > lane) f *= L.decay[t];
       L.G[t][lane] = t >= lane ? f : 0.f;
     }
-  } else if (w == 6) {  // p_t
+  } else if (w == 0) {  // p_t
     float p = L.decay[lane];
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -262,16 +284,16 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
     for (int j = 0; j < 4; ++j) inter[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
   auto tile_of = [](int u, int& mt, int& st) { mt = u < 1 ? 0 : u < 3 ? 1 : u < 6 ? 2 : 3, st = u - mt * (mt + 1) / 2; };
-  for (int n0 = 0; n0 < a.N; n0 += HALF) {
-    cs.stash(&L.C[0][0], LDN), bs.stash(&L.B[0][0], LDN);
+  for (int n0 = 0; n0 < a.N; n0 += RUN) {
+    f32x4 S[RT];  // (used last)
+#pragma unroll
+    for (int nb = 0; nb < RT; ++nb) S[nb] = *(const f32x4*)(start + (((long long)(n0 / 16 + nb) * tiles_p + my_pt) * 64 + lane) * 4);
+    cs.stash(&L.C[0][0], LDR), bs.stash(&L.B[0][0], LDR);
 #pragma unroll
     for (int i = 0; i < bs.PER; ++i) nan_if = not_finite(bs.v[i], nan_if);
     if (nan_if != nan_if) L.odd = 1;  // (read behind the barriers below)
-    f32x4 now[NT];
-#pragma unroll
-    for (int nb = 0; nb < NT; ++nb) now[nb] = S[nb];
     __syncthreads();
-    if (n0 + HALF < a.N) ask(n0 + HALF);
+    if (n0 + RUN < a.N) ask(n0 + RUN);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int u = w + 8 * i;
@@ -282,7 +304,7 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
 #pragma unroll
         for (int x = 0; x < 4; ++x) acc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int nb = 0; nb < NT; ++nb)
+        for (int nb = 0; nb < RT; ++nb)
           acc[nb & 3] = step4(*(const f32x4*)&L.C[SUB * mt + c][16 * nb + 4 * g], *(const f32x4*)&L.B[SUB * st + c][16 * nb + 4 * g],
                               acc[nb & 3]);
         G[i] += (acc[0] + acc[1]) + (acc[2] + acc[3]);
@@ -291,8 +313,8 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int nb = 0; nb < NT; ++nb)
-        inter[i][nb & 3] = step4(*(const f32x4*)&L.C[SUB * (m0 + i) + c][16 * nb + 4 * g], now[nb], inter[i][nb & 3]);
+      for (int nb = 0; nb < RT; ++nb)
+        inter[i][nb & 3] = step4(*(const f32x4*)&L.C[SUB * (m0 + i) + c][16 * nb + 4 * g], S[nb], inter[i][nb & 3]);
     __syncthreads();
   }
   f32x4 own[2];
@@ -347,9 +369,9 @@ __global__ __launch_bounds__(512, 2) void ssd_chunk_out_kernel(SsdArgs a) {
 }  // namespace
 
 // From 128 rows of the longest sequence on, states of up to 256 channels (two rounds through LDS).  Microseconds a launch,
-// token by token (long sequences in segments) and in chunks: 32 heads of 128 x 64 over 8 groups, 130 tokens 44 / 31, 512
-// tokens 83 / 51, 2 048 tokens 263 / 110, 8 192 tokens 892 / 377, eight of 130 73 / 74, eight of 512 244 / 184; a matrix
-// memory of 4 heads of 256 x 513, 130 tokens 62 / 42, two sequences of 900 and 1 100 tokens 635 / 170.  Relative error
+// token by token (long sequences in segments) and in chunks: 32 heads of 128 x 64 over 8 groups, 130 tokens 42 / 26, 512
+// tokens 83 / 41, 2 048 tokens 263 / 88, eight of 130 72 / 65, eight of 512 233 / 142; a matrix memory of 4 heads of 256 x
+// 512, two sequences of 1 000 and 1 100 tokens 635 / 134.  Relative error
 // against 64 bits: 5.9e-8 and 4.7e-8 at 2 048 tokens (of the state 4.8e-7 and 4.4e-7), 1.4e-7 and 1.7e-7 of the memory's
 // results (of its state 1.2e-7 and 1.1e-7).
 constexpr int LQ_SSD_MIN = 128;
@@ -375,9 +397,9 @@ long long lq_ssd_chunks_floats(int rows, int batch, int heads, int P, int N, int
 // Whether a launch is faster in chunks (given scratch) than token by token (`segments`: in segments), by what both take.
 // A chunk of up to 128 channels costs the same however few they are and however few tokens it has; a walk's token costs little
 // where states are small, as soon as there are workgroups for the whole chip.  Microseconds, walk / chunks, 32 heads: of
-// 128 x 64, one sequence of 130 tokens 43 / 30, eight of 512 234 / 183, 32 of 256 451 / 389; of 64 x 64, eight of 256 93 / 101,
-// 32 of 256 231 / 353, one of 2 048 181 / 102; of 16 x 64, four of 1 000 139 / 178, eight of 512 144 / 178; of 64 x 16, eight
-// of 1 000 159 / 302.
+// 128 x 64, one sequence of 130 tokens 42 / 26, eight of 512 233 / 142, 32 of 256 461 / 318; of 64 x 64, eight of 256 90 / 76,
+// 32 of 256 227 / 245, one of 2 048 181 / 75; of 16 x 64, four of 1 000 137 / 121, eight of 512 144 / 121; of 64 x 16, eight
+// of 1 000 159 / 192.
 bool lq_ssd_chunks_faster(int batch, int heads, int P, int N, int max_rows, int rows, bool segments) {
   if (lq_ssd_chunks_floats(rows, batch, heads, P, N, max_rows) == 0) return false;
   const double token = 1.75e-3 * P / 64 * (N > 128 ? N / 80.0 : N > 32 ? N / 128.0 : 0.25) * heads, state = 0.02 * P / 64 * N / 128 * heads;
@@ -389,7 +411,7 @@ bool lq_ssd_chunks_faster(int batch, int heads, int P, int N, int max_rows, int 
   const double rest = rows - max_rows, least = lq_ssd_least_rows(rows, batch, heads);
   const bool alike = batch == 1 || rest >= least * (batch - 1);
   const double of_chunks = alike ? rows / 64.0 + batch / 2.0 : max_rows / 64.0 + 0.5;
-  double chunks = 24 + (N > HALF ? 0.125 : 0.082) * lq_ceil_div(P, COLS) * heads * of_chunks;
+  double chunks = 24 + (N > HALF ? 0.1 : 0.061) * lq_ceil_div(P, COLS) * heads * of_chunks;
   if (!alike) chunks += 10 + walk(rest, least, batch - 1, false);
   return 0.9 * chunks < walk(rows, max_rows, batch, segments);
 }
