@@ -9,6 +9,7 @@ int lq_gemm_mfma(const void* x, const void* w, void* out, int out_dtype, int M, 
 bool lq_gemm_packable(int N, int K);
 int lq_gemm_mfma_splits(int M, int N, int K);
 int lq_gemm_narrow_splits(int M, int N, int K);
+bool lq_gemm_pairs(int M, int N, int K);
 int lq_gemm_fused_parts(int M, int N, int K);
 int lq_gemm_residual(const void* act, const void* w, float* x, float* sq_out, const float* gain, void* scaled,
                      int ld_scaled, int M, int N, int K, int lda, int ldw, int ldx, int packed, hipStream_t stream);
@@ -30,6 +31,14 @@ extern "C" int lq_linear_narrow_splits(int in_dtype, int M, int N, int K, int fo
   const int usual = lq_linear_splits(in_dtype, M, N, K, force_generic);
   if (usual > 1 || force_generic || in_dtype != LQ_BF16 || K % 8 != 0) return usual;
   return lq_gemm_narrow_splits(M, N, K);
+}
+
+// Whether that caller is better off without pieces: at most 8 rows, whose kernel takes K in pairs of chunks, up to four pieces.
+// Microseconds in pieces with the launch that adds them up, and whole: 128 x 2 048 in two, 1 row 4.4 and 2.9, 8 rows 5.2 and 3.8; 8
+// rows of 64 x 4 096 in four 5.4 and 5.4; 288 x 8 192 in eight, 1 row 5.9 and 6.2, 8 rows 6.8 and 9.0.
+extern "C" int lq_linear_whole(int in_dtype, int M, int N, int K, int force_generic) {
+  return !force_generic && in_dtype == LQ_BF16 && K % 8 == 0 && lq_gemm_mfma_splits(M, N, K) <= 1 && lq_gemm_pairs(M, N, K) &&
+         lq_gemm_narrow_splits(M, N, K) <= 4;
 }
 
 // Whether a bfloat16 weight [N, K] may be handed to the products packed (lq_pack_weight): only where every

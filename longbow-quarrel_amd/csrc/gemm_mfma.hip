@@ -1276,7 +1276,7 @@ int launch_rows(const void* x, const void* w, void* out, int M, int N, int K, in
 // Shares of K for up to 16 rows of a weight with so few columns that its tiles of 16 leave most of the chip idle and
 // one of them walks a long K: asked for by callers that add the pieces up right away (`lq_linear_narrow_splits`).
 int narrow_splits(int M, int N, int K) {
-  if (M > 16 || N >= 8 * lq_compute_units() || K % 64 != 0 || takes_pairs(M, N, K)) return 1;
+  if (M > 16 || N >= 8 * lq_compute_units() || K % 64 != 0) return 1;
   int splits = 1;
   while (splits < 16 && lq_ceil_div(N, 16) * splits * 2 <= 2 * lq_compute_units() && K % (128 * splits) == 0 &&
          K / (splits * 2) >= 1024)
@@ -1340,6 +1340,8 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
 int lq_gemm_mfma_splits(int M, int N, int K) { return mfma_splits(M, N, K); }
 
 int lq_gemm_narrow_splits(int M, int N, int K) { return narrow_splits(M, N, K); }
+
+bool lq_gemm_pairs(int M, int N, int K) { return takes_pairs(M, N, K); }
 
 // The decode pair around a norm.  `residual`: x[M, N] (float32) += act[M, K] . w[N, K]^T; sq_out[M][parts]
 // takes each row's sum of squares over a block's columns, and, with a gain, scaled[M, N] takes

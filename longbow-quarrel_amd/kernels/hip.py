@@ -64,7 +64,7 @@ def load_library() -> ctypes.CDLL:
     lib.lq_attention.argtypes = [vp, ci, vp, ci, ci, ci, ci, ci, ci, ci, vp, vp, vp, vp, vp, ci, vp, vp, ci, cf, ci, ci, ci,
                                  vp, cl, vp, cl, vp, vp, ci, ci, vp, ci, ci, cl, ci, vp]
     lib.lq_rope_store_pieces.argtypes = [vp, ci, ci, cl, vp, ci, ci, ci, ci, ci, vp, vp, vp, vp, vp, ci, vp, vp, ci, vp]
-    lib.lq_linear_splits.argtypes = lib.lq_linear_narrow_splits.argtypes = [ci] * 5
+    lib.lq_linear_splits.argtypes = lib.lq_linear_narrow_splits.argtypes = lib.lq_linear_whole.argtypes = [ci] * 5
     lib.lq_linear_fused_parts.argtypes = [ci] * 4
     _LIB = lib
     return lib
@@ -358,6 +358,11 @@ class HipKernels:
         if dtype not in _DTYPE_CODE:
             return 1
         return self.lib.lq_linear_narrow_splits(_DTYPE_CODE[dtype], m, n, k, 1 if self.force_generic else 0)
+
+    @query
+    def linear_whole(self, dtype: torch.dtype, m: int, n: int, k: int) -> bool:
+        """Whether that caller gets the product sooner without pieces, from `linear` into its output."""
+        return dtype in _DTYPE_CODE and bool(self.lib.lq_linear_whole(_DTYPE_CODE[dtype], m, n, k, 1 if self.force_generic else 0))
 
     def linear(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
         """out[M, N] = x[M, K] . w[N, K]^T with 32-bit accumulation; or out[pieces, M, N] with

@@ -47,3 +47,22 @@ def test_into_the_stream(rows, k):
     kn.linear_residual(act, w, got, sq, gain=gain, scaled=scaled)
     assert torch.equal(got, x + plain) and torch.equal(scaled, (got * gain).bfloat16())
     assert ((sq.double().sum(1) - (got.double() ** 2).sum(1)).abs() <= 2048 * 2.0 ** -24 * (got.double() ** 2).sum(1)).all()
+
+
+@pytest.mark.parametrize("rows,n,k,whole", [(1, 128, 2048, True), (8, 64, 4096, True), (8, 288, 8192, False), (9, 128, 2048, False),
+                                            (3, 160, 2112, False), (2, 4096, 4096, False)])
+def test_whole_or_in_pieces_added_up(rows, n, k, whole):
+    from types import SimpleNamespace
+
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+    from longbow_quarrel_amd.parts.base import project_narrow
+
+    kn = HipKernels()
+    assert kn.linear_whole(torch.bfloat16, rows, n, k) == whole and not kn.linear_whole(torch.float32, rows, n, k)
+    gen = torch.Generator().manual_seed(n + k)
+    x, w = torch.randn(rows, k, generator=gen).bfloat16().cuda(), torch.randn(n, k, generator=gen).bfloat16().cuda()
+    out = torch.empty(rows, n, device="cuda")
+    ws = SimpleNamespace(alloc=lambda shape, dtype, **_: torch.empty(shape, dtype=dtype, device="cuda"))
+    project_narrow(kn, SimpleNamespace(ws=ws, kernels=kn), x, w, out)
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((out - x.double() @ w.double().T).abs() <= bound).all()
