@@ -102,6 +102,17 @@ bool pieces_of(PyObject* o, const Matrix& x, const void*& at, int& type, int& n,
   return type >= 0;
 }
 
+// Python's lock, given back while a launch is made (it waits where the stream's queue is full).
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+int launch(F f) {
+  Unlocked unlocked;
+  return f() ?: 1;
+}
+
 long long number(PyObject* o) { return PyLong_AsLongLong(o); }
 void* address(PyObject* o) { return (void*)PyLong_AsUnsignedLongLong(o); }
 
@@ -126,8 +137,10 @@ int linear(PyObject* const* a) {
     return 0;
   }
   if (w.cols != x.cols || out.rows != x.rows || out.cols != w.rows || x.type != w.type) return 0;
-  return lq_linear(x.at, w.at, out.at, x.type, out.type, (int)x.rows, (int)w.rows, (int)x.cols, (int)x.ld, (int)w.ld, (int)out.ld, pieces,
-                   apart, generic, w.packed, stream) ?: 1;
+  return launch([&] {
+    return lq_linear(x.at, w.at, out.at, x.type, out.type, (int)x.rows, (int)w.rows, (int)x.cols, (int)x.ld, (int)w.ld, (int)out.ld, pieces,
+                     apart, generic, w.packed, stream);
+  });
 }
 
 // linear_swiglu(x, w, out, form, stream)
@@ -137,8 +150,10 @@ int linear_swiglu(PyObject* const* a) {
   void* stream = address(a[4]);
   if (PyErr_Occurred() || !matrix(a[0], x) || !weight(a[1], w) || !matrix(a[2], out)) return 0;
   if (w.cols != x.cols || out.rows != x.rows || out.cols != w.rows / 2 || w.rows % 16 != 0 || x.type != w.type) return 0;
-  return lq_linear_swiglu(x.at, w.at, out.at, x.type, out.type, (int)x.rows, (int)w.rows, (int)x.cols, (int)x.ld, (int)w.ld, (int)out.ld,
-                          w.packed, form, stream) ?: 1;
+  return launch([&] {
+    return lq_linear_swiglu(x.at, w.at, out.at, x.type, out.type, (int)x.rows, (int)w.rows, (int)x.cols, (int)x.ld, (int)w.ld, (int)out.ld,
+                            w.packed, form, stream);
+  });
 }
 
 // rmsnorm(x, weight, eps, out, delta, stream)
@@ -154,7 +169,9 @@ int rmsnorm(PyObject* const* a) {
   if (x.type != 0 || (x.ld != x.cols && x.rows > 1) || w->scalar_type() != at::kFloat || w->numel() != x.cols || !w->is_contiguous() ||
       out.rows != x.rows || out.cols != x.cols || (out.ld != x.cols && x.rows > 1))
     return 0;
-  return lq_rmsnorm(x.at, delta, type, n, apart, w->data_ptr(), eps, out.at, out.type, (int)x.rows, (int)x.cols, stream) ?: 1;
+  return launch([&, gain = w->data_ptr()] {
+    return lq_rmsnorm(x.at, delta, type, n, apart, gain, eps, out.at, out.type, (int)x.rows, (int)x.cols, stream);
+  });
 }
 
 // Keys and values in the paged layout, [blocks, kv_heads, block, head] and [blocks, kv_heads, head, block].
@@ -188,10 +205,13 @@ int attention(PyObject* const* a) {
       out.cols < heads * head || q.cols < heads * head || q.type != out.type ||
       !paged(a[10], a[11], kv_heads, head, block, out.type ? at::kBFloat16 : at::kFloat, k, v))
     return 0;
-  return lq_attention(q.at, (int)q.ld, out.at, (int)out.ld, out.type, (int)q.rows, (int)batch, (int)heads, (int)kv_heads, (int)head, pos,
-                      seq, slots->data_ptr(), cu, table->data_ptr(), (int)table->stride(0), k, v, (int)block,
-                      scale, (int)window, 0, (int)max_len, nullptr, 0, tickets->data_ptr(), tickets->numel(), nullptr, nullptr, 0, 0, nullptr,
-                      0, 1, 0, (int)generic, stream) ?: 1;
+  void *slot = slots->data_ptr(), *blocks = table->data_ptr(), *counters = tickets->data_ptr();
+  const long long ld = table->stride(0), room = tickets->numel();
+  return launch([&] {
+    return lq_attention(q.at, (int)q.ld, out.at, (int)out.ld, out.type, (int)q.rows, (int)batch, (int)heads, (int)kv_heads, (int)head, pos,
+                        seq, slot, cu, blocks, (int)ld, k, v, (int)block, scale, (int)window, 0, (int)max_len, nullptr, 0, counters, room,
+                        nullptr, nullptr, 0, 0, nullptr, 0, 1, 0, (int)generic, stream);
+  });
 }
 
 // rope_store_pieces(qkv, q_out, heads, kv_heads, head_dim, freqs, row_pos, row_seq, seq_slot, block_table, k, v, block, stream)
@@ -210,9 +230,12 @@ int rope_store_pieces(PyObject* const* a) {
       (slots->dim() > 0 && slots->stride(-1) != 1 && slots->size(-1) != 1) || table->scalar_type() != at::kInt || table->dim() != 2 ||
       (table->stride(1) != 1 && table->size(1) != 1) || !paged(a[10], a[11], kv_heads, head, block, at::kBFloat16, k, v))
     return 0;
-  return lq_rope_store_pieces(qkv->data_ptr(), (int)qkv->size(2), (int)qkv->size(0), qkv->stride(0), q.at, (int)q.ld, (int)q.rows,
-                              (int)heads, (int)kv_heads, (int)head, freqs->data_ptr(), pos, seq, slots->data_ptr(), table->data_ptr(),
-                              (int)table->stride(0), k, v, (int)block, stream) ?: 1;
+  void *in = qkv->data_ptr(), *angles = freqs->data_ptr(), *slot = slots->data_ptr(), *blocks = table->data_ptr();
+  const long long n = qkv->size(2), pieces = qkv->size(0), apart = qkv->stride(0), ld = table->stride(0);
+  return launch([&] {
+    return lq_rope_store_pieces(in, (int)n, (int)pieces, apart, q.at, (int)q.ld, (int)q.rows, (int)heads, (int)kv_heads, (int)head, angles,
+                                pos, seq, slot, blocks, (int)ld, k, v, (int)block, stream);
+  });
 }
 
 // A function of N arguments.  What torch throws means "not as the launch wants it": the caller's own checks meet it again.
