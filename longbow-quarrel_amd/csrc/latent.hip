@@ -121,7 +121,8 @@ __global__ __launch_bounds__(256) void rotary_qkv_kernel(const float* __restrict
 // Queries, keys and values of a step's rows, from the 32-bit result of their one product to what the attention kernel
 // reads and straight into the paged cache.  src [rows, H D + G D (+ G V)]; `bias` (a number a column, or null) is added
 // first.  With `cs` (cos and sin of the row's angles, [rows][dims / 2][2]) the first `dims` entries of every query and key
-// head are then rotated, pairs and magnitude as in `rotary_kernel` (units of a head only).  q and k are normed in units of `unit_q` and `unit_k` entries (a head each, or the whole row of
+// unit are then rotated, pairs and magnitude as in `rotary_kernel` (units of a head, or of an equal part of one: the maps of
+// differential attention, whose keys lie side by side in a head's cache row).  q and k are normed in units of `unit_q` and `unit_k` entries (a head each, or the whole row of
 // all heads; units divided by their root mean square, eps inside the root, times a weight of the unit's size), values in
 // units of a head without a weight (`norm_v`) or not at all; `v_from_k`: there are no value columns, the values are the
 // keys as they are before rotation and norm.  k and v go to the row's position in the cache (K [block][G][BS][D],
@@ -311,7 +312,8 @@ __global__ __launch_bounds__(256) void qkv_norm_store4_kernel(const float* __res
   }
 }
 
-// The same for many rows, units of a head of 4 LANES entries: LANES lanes a unit.  Queries and keys: a thread takes four rows of its
+// The same for many rows, units of 4 LANES entries (a query or key head, or an equal part of one) and value heads of 4 VLANES: LANES
+// lanes a unit.  Queries and keys: a thread takes four rows of its
 // unit, all asked for together.  Values lie in the cache with the positions of an entry side by side: the first row of every
 // aligned run of eight positions (or of a sequence) takes the run, eight rows at once, and writes 16 bytes an entry where the run is
 // whole, in the place of a 2-byte store an entry and row.  A unit's sum of squares is the kernel's above, bit for bit.
@@ -335,33 +337,32 @@ __device__ inline float unit_sum(float v) {
   return v;
 }
 
-template <typename T, int LANES>
+template <typename T, int LANES, int VLANES>
 __global__ __launch_bounds__(256) void qkv_norm_store_rows_kernel(const float* __restrict__ src, T* __restrict__ q_out,
                                                                   T* __restrict__ kcache, T* __restrict__ vcache, QkvUnits a, int rows,
                                                                   int qk_blocks) {
-  constexpr int UNITS = 256 / LANES, N = 4 * LANES;
-  const int lane = threadIdx.x % LANES, mine = threadIdx.x / LANES, QW = a.H * N, KW = a.G * N, e0 = 4 * lane;
+  constexpr int UNITS = 256 / LANES, N = 4 * LANES, VUNITS = 256 / VLANES, VN = 4 * VLANES;
+  const int QW = a.H * a.D, KW = a.G * a.D;
   const bool stored = kcache != nullptr;
   auto fetch = [&](int r, int col) {
-    float4 v = *(const float4*)(src + (long long)r * a.lds + col + e0);
+    float4 v = *(const float4*)(src + (long long)r * a.lds + col);
     if (a.bias != nullptr) {
-      const float4 add = *(const float4*)(a.bias + col + e0);
+      const float4 add = *(const float4*)(a.bias + col);
       v.x += add.x, v.y += add.y, v.z += add.z, v.w += add.w;
     }
     return v;
   };
-  auto rstd = [&](const float4& v) {
-    return 1.f / sqrtf(unit_sum<LANES>(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, 0.f))))) / (float)N + a.eps);
-  };
+  auto squares = [](const float4& v) { return fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, 0.f)))); };
   if ((int)blockIdx.x < qk_blocks) {
-    const int units = a.H + (stored ? a.G : 0), per_rows = (units + UNITS - 1) / UNITS;
+    const int lane = threadIdx.x % LANES, mine = threadIdx.x / LANES, e0 = 4 * lane, parts = a.D / N, queries = a.H * parts;
+    const int units = queries + (stored ? a.G * parts : 0), per_rows = (units + UNITS - 1) / UNITS;
     const int u = (int)blockIdx.x % per_rows * UNITS + mine, r0 = (int)blockIdx.x / per_rows * QKV_ROWS;
     if (u >= units) return;
-    const bool is_q = u < a.H;
+    const bool is_q = u < queries;
     const int col = u * N;  // (keys lie behind the queries)
     float4 v[QKV_ROWS];
 #pragma unroll
-    for (int j = 0; j < QKV_ROWS; ++j) v[j] = fetch(min(r0 + j, rows - 1), col);
+    for (int j = 0; j < QKV_ROWS; ++j) v[j] = fetch(min(r0 + j, rows - 1), col + e0);
     const float* w = is_q ? a.wq : a.wk;
     const float4 gain = w != nullptr ? *(const float4*)(w + e0) : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
@@ -386,7 +387,7 @@ __global__ __launch_bounds__(256) void qkv_norm_store_rows_kernel(const float* _
           if (e0 + k < a.dims) x[k] = turned_entry(a, cs, e0 + k, x[k], mate[k]);
       }
       if (a.norm_qk) {
-        const float inv = rstd(make_float4(x[0], x[1], x[2], x[3]));
+        const float inv = 1.f / sqrtf(unit_sum<LANES>(squares(make_float4(x[0], x[1], x[2], x[3]))) / (float)N + a.eps);
         x[0] *= inv, x[1] *= inv, x[2] *= inv, x[3] *= inv;
       }
       if (w != nullptr) x[0] *= gain.x, x[1] *= gain.y, x[2] *= gain.z, x[3] *= gain.w;
@@ -397,7 +398,8 @@ __global__ __launch_bounds__(256) void qkv_norm_store_rows_kernel(const float* _
       } else {
         const int p = a.row_pos[r];
         const long long blk = a.block_table[(long long)a.seq_slot[a.row_seq[r]] * a.bt_stride + p / a.BS];
-        o = kcache + ((blk * a.G + u - a.H) * a.BS + p % a.BS) * N + e0;
+        const int ku = u - queries, head = ku / parts;
+        o = kcache + ((blk * a.G + head) * a.BS + p % a.BS) * (long long)a.D + (ku - head * parts) * N + e0;
       }
       if constexpr (sizeof(T) == 4) {
         *(float4*)o = make_float4(x[0], x[1], x[2], x[3]);
@@ -410,26 +412,27 @@ __global__ __launch_bounds__(256) void qkv_norm_store_rows_kernel(const float* _
     }
     return;
   }
-  // values (V = N entries a head)
-  const int per_row = (a.G + UNITS - 1) / UNITS, at = (int)blockIdx.x - qk_blocks, r = at / per_row, u = at % per_row * UNITS + mine;
+  // values (V = VN entries a head)
+  const int e0 = 4 * (threadIdx.x % VLANES), per_row = (a.G + VUNITS - 1) / VUNITS, at = (int)blockIdx.x - qk_blocks;
+  const int r = at / per_row, u = at % per_row * VUNITS + (int)threadIdx.x / VLANES;
   const int p = a.row_pos[r], seq = a.row_seq[r];
   if (p % RUN != 0 && r > 0 && a.row_seq[r - 1] == seq && a.row_pos[r - 1] == p - 1) return;  // (the whole workgroup: another row takes it)
   const int i0 = threadIdx.x & 63, ri = min(r + i0, rows - 1);  // (a lane looks at a row of the run: one trip to memory)
   const bool follows = i0 < RUN - p % RUN && r + i0 < rows && a.row_seq[ri] == seq && a.row_pos[ri] == p + i0;
   const int n = __ffsll(~(unsigned long long)__ballot(follows)) - 1;  // rows of the run, one at least
   if (u >= a.G) return;
-  const int col = (a.v_from_k ? QW : QW + KW) + u * N;
+  const int col = (a.v_from_k ? QW : QW + KW) + u * VN + e0;
   float4 v[RUN];
 #pragma unroll
   for (int i = 0; i < RUN; ++i) v[i] = fetch(r + min(i, n - 1), col);
   if (a.norm_v)
 #pragma unroll
     for (int i = 0; i < RUN; ++i) {
-      const float inv = rstd(v[i]);
+      const float inv = 1.f / sqrtf(unit_sum<VLANES>(squares(v[i])) / (float)VN + a.eps);
       v[i].x *= inv, v[i].y *= inv, v[i].z *= inv, v[i].w *= inv;
     }
   const long long blk = a.block_table[(long long)a.seq_slot[seq] * a.bt_stride + p / a.BS];
-  T* o = vcache + ((blk * a.G + u) * (long long)N + e0) * a.BS + p % a.BS;
+  T* o = vcache + ((blk * a.G + u) * (long long)VN + e0) * a.BS + p % a.BS;
 #pragma unroll
   for (int k = 0; k < 4; ++k, o += a.BS) {
     float x[RUN];
@@ -678,7 +681,8 @@ extern "C" int lq_rotary_qkv(const float* src, int lds_, void* q_out, int ldq, v
   return 0;
 }
 
-// bias: null or a number for every column of src; wq, wk: weights of unit_q and unit_k entries, or null (with
+// bias: null or a number for every column of src; wq, wk: weights of unit_q and unit_k entries, or null (a rotation is one of
+// every unit: of a head, or of an equal part of one) (with
 // `norm_qk` off: no norm of q and k); kcache and vcache null: q alone.
 extern "C" int lq_qkv_norm_store(const float* src, int lds_, const float* bias, const float* wq, const float* wk, int unit_q,
                                  int unit_k, int norm_qk, int norm_v, int v_from_k, float eps, void* q_out, int ldq, int dtype,
@@ -686,7 +690,7 @@ extern "C" int lq_qkv_norm_store(const float* src, int lds_, const float* bias, 
                                  const int* row_seq, const int* seq_slot, const int* block_table, int bt_stride, void* kcache,
                                  void* vcache, int block_size, const float* cos_sin, int dims, int interleaved,
                                  float magnitude, hipStream_t stream) {
-  LQ_REQUIRE(cos_sin == nullptr || (dims >= 2 && dims % 2 == 0 && dims <= key_dim && unit_q == key_dim && unit_k == key_dim),
+  LQ_REQUIRE(cos_sin == nullptr || (dims >= 2 && dims % 2 == 0 && dims <= unit_q && unit_q == unit_k && unit_q > 0 && key_dim % unit_q == 0),
              "qkv_norm_store: %d rotated entries in units of %d and %d for heads of %d", dims, unit_q, unit_k, key_dim);
   LQ_REQUIRE(rows > 0 && rows <= 0x7fffffff && heads > 0 && kv_heads > 0 && key_dim > 0 && value_dim > 0,
              "qkv_norm_store: rows %d, heads %d and %d, sizes %d and %d", rows, heads, kv_heads, key_dim, value_dim);
@@ -699,7 +703,7 @@ extern "C" int lq_qkv_norm_store(const float* src, int lds_, const float* bias, 
              "qkv_norm_store: the cache needs the rows' places");
   LQ_REQUIRE(norm_qk || (wq == nullptr && wk == nullptr), "qkv_norm_store: weights without a norm");
   // (values go head by head where queries and keys do; they are only copied there)
-  const int unit_v = norm_v || (unit_q == key_dim && unit_k == key_dim) ? value_dim : VW;
+  const int unit_v = norm_v || (key_dim % unit_q == 0 && key_dim % unit_k == 0) ? value_dim : VW;
   QkvUnits a = {lds_, ldq, heads, kv_heads, key_dim, value_dim, unit_q, unit_k, norm_qk, norm_v, v_from_k,
                 eps, bias, wq, wk, row_pos, row_seq, seq_slot, block_table, bt_stride, block_size,
                 unit_v, cos_sin, cos_sin != nullptr ? dims : 0, interleaved, magnitude};
@@ -713,21 +717,25 @@ extern "C" int lq_qkv_norm_store(const float* src, int lds_, const float* bias, 
   const int el = dtype == LQ_F32 ? 4 : 2;
   int most = unit_q > unit_k ? unit_q : unit_k;
   if (kcache != nullptr && unit_v > most) most = unit_v;
-  const bool fours = key_dim % 4 == 0 && value_dim % 4 == 0 && lds_ % 4 == 0 && ldq % 4 == 0 && (uintptr_t)src % 16 == 0 &&
+  const bool fours = key_dim % 4 == 0 && unit_q % 4 == 0 && unit_k % 4 == 0 && value_dim % 4 == 0 && lds_ % 4 == 0 && ldq % 4 == 0 && (uintptr_t)src % 16 == 0 &&
                      (uintptr_t)bias % 16 == 0 && (uintptr_t)wq % 16 == 0 && (uintptr_t)wk % 16 == 0 &&
                      (uintptr_t)q_out % (4 * el) == 0 && (uintptr_t)kcache % (4 * el) == 0 && most <= 16384;
-  // many rows of heads of 64, 128 or 256, one size for keys and values: the kernel that takes runs of rows.  Microseconds, 16 query
+  // many rows of units of 64, 128 or 256, values of a unit's size or twice it: the kernel that takes runs of rows.  Microseconds, 16 query
   // heads of 128 over 4, by units and by runs: 64 rows 4.2 / 7.3, 500 rows 8.3 / 9.3, 800 rows 11.9 / 10.5, 2 000 rows 26.2 / 16.0,
   // 2 635 rows 33.2 / 21.4, 4 096 rows 48.8 / 31.1
-  const bool runs = fours && rows >= 640 && unit_q == key_dim && unit_k == key_dim && (kcache == nullptr || (unit_v == value_dim && value_dim == key_dim)) &&
-                    (key_dim == 64 || key_dim == 128 || key_dim == 256) && block_size % RUN == 0 && (uintptr_t)vcache % 16 == 0 &&
-                    (long long)rows * (heads + kv_heads) < (1ll << 30);
+  const bool runs = fours && rows >= 640 && unit_q == unit_k && key_dim % unit_q == 0 &&
+                    (kcache == nullptr || (unit_v == value_dim && (value_dim == unit_q || value_dim == 2 * unit_q))) &&
+                    (unit_q == 64 || unit_q == 128 || (unit_q == 256 && (kcache == nullptr || value_dim == 256))) && block_size % RUN == 0 &&
+                    (uintptr_t)vcache % 16 == 0 && (long long)rows * (heads + kv_heads) * (key_dim / unit_q) < (1ll << 30);
   if (runs) {
-    const int in_block = 1024 / key_dim, qk = heads + (kcache != nullptr ? kv_heads : 0);
+    const int in_block = 1024 / unit_q, qk = (heads + (kcache != nullptr ? kv_heads : 0)) * (key_dim / unit_q);
     const int qk_blocks = lq_ceil_div(rows, QKV_ROWS) * lq_ceil_div(qk, in_block);
-    const int blocks = qk_blocks + (kcache != nullptr ? rows * lq_ceil_div(kv_heads, in_block) : 0);
-#define LQ_QKV_ROWS(T)                                                                                                          \
-  (key_dim == 64 ? qkv_norm_store_rows_kernel<T, 16> : key_dim == 128 ? qkv_norm_store_rows_kernel<T, 32> : qkv_norm_store_rows_kernel<T, 64>) \
+    const bool twice = kcache != nullptr && value_dim != unit_q;
+    const int blocks = qk_blocks + (kcache != nullptr ? rows * lq_ceil_div(kv_heads, 1024 / value_dim) : 0);
+#define LQ_QKV_ROWS(T)                                                                                                     \
+  (twice ? unit_q == 64 ? qkv_norm_store_rows_kernel<T, 16, 32> : qkv_norm_store_rows_kernel<T, 32, 64>                   \
+   : unit_q == 64 ? qkv_norm_store_rows_kernel<T, 16, 16>                                                                 \
+   : unit_q == 128 ? qkv_norm_store_rows_kernel<T, 32, 32> : qkv_norm_store_rows_kernel<T, 64, 64>)                       \
       <<<blocks, 256, 0, stream>>>(src, (T*)q_out, (T*)kcache, (T*)vcache, a, rows, qk_blocks)
     if (dtype == LQ_F32) LQ_QKV_ROWS(float);
     else if (dtype == LQ_BF16) LQ_QKV_ROWS(bf16_t);

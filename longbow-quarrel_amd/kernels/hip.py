@@ -148,6 +148,7 @@ def _packed(w) -> int:
 
 class HipKernels:
     name = "hip-gfx950"
+    stores_maps = True  # `qkv_norm_store` takes heads in parts (`maps`)
 
     def __init__(self) -> None:
         self.lib = load_library()
@@ -1481,7 +1482,7 @@ class HipKernels:
                        seq_slot: Optional[torch.Tensor] = None, block_table: Optional[torch.Tensor] = None,
                        kcache: Optional[torch.Tensor] = None, vcache: Optional[torch.Tensor] = None,
                        block_size: int = 0, cos_sin: Optional[torch.Tensor] = None, interleaved: bool = False,
-                       magnitude: float = 1.0) -> None:
+                       magnitude: float = 1.0, maps: int = 1) -> None:
         """src float32 [rows, queries | keys (| values)], `bias` (float32, a number a column) added first.  `norm_qk`:
         None, "head" (every query and key head divided by its root mean square) or "row" (all heads of a row's queries
         together, all of its keys together); q_weight and k_weight (of the normed run's size) multiply the result.
@@ -1489,14 +1490,17 @@ class HipKernels:
         the keys with their bias, before rotation and norm.  `cos_sin` (float32 [rows, pairs, 2], `rope_table`): the first
         2 pairs entries of every query and key head are rotated after the bias and before the norm, in half-split or
         interleaved pairs, cos and sin times `magnitude`.  Queries go to q_out in its dtype; keys and values straight into
-        the paged cache (layout as `kv_store`) at the rows' positions, or nowhere when kcache is None."""
+        the paged cache (layout as `kv_store`) at the rows' positions, or nowhere when kcache is None.  `maps`: a query or
+        key head is so many equal parts, each rotated and normed by itself."""
         rows, ns, lds = self._mat(src, "qkv_norm_store: src")
         rq, nq, ldq = self._mat(q_out, "qkv_norm_store: q")
         kw, vw = kv_heads * key_dim, 0 if v_from_k else kv_heads * value_dim
         if src.dtype != torch.float32 or ns != heads * key_dim + kw + vw or (rq, nq) != (rows, heads * key_dim) \
                 or norm_qk not in (None, "head", "row") or (v_from_k and key_dim != value_dim):
             raise KernelLibraryError("qkv_norm_store: src float32 [rows, q | k | v], q_out [rows, q], norm_qk None, 'head' or 'row'")
-        uq, uk = (heads * key_dim, kw) if norm_qk == "row" else (key_dim, key_dim)
+        if maps < 1 or key_dim % maps or (maps > 1 and norm_qk == "row"):
+            raise KernelLibraryError(f"qkv_norm_store: heads of {key_dim} in {maps} parts")
+        uq, uk = (heads * key_dim, kw) if norm_qk == "row" else (key_dim // maps, key_dim // maps)
         if bias is not None:
             self._f32(bias, "qkv_norm_store: bias", ns)
         for t, what, n in ((q_weight, "q_weight", uq), (k_weight, "k_weight", uk)):
@@ -1506,7 +1510,7 @@ class HipKernels:
         if cos_sin is not None:
             dims = 2 * int(cos_sin.shape[1])
             self._f32(cos_sin, "qkv_norm_store: cos_sin", rows * dims)
-            if norm_qk == "row" or dims > key_dim:
+            if norm_qk == "row" or dims > uq:
                 raise KernelLibraryError("qkv_norm_store: a rotation of at most a head's entries, not with a norm by row")
         if norm_qk is None and (q_weight is not None or k_weight is not None):
             raise KernelLibraryError("qkv_norm_store: weights without a norm")

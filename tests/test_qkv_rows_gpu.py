@@ -68,3 +68,35 @@ def test_mean_of_normed_branches(rows, width, bias):
     size = (y / torch.sqrt((y * y).mean(-1, keepdim=True) + 1e-5) * w.double()[:, None]).abs().mean(0)
     # (an entry: some ten roundings; the sum of squares: 2^-24 for each of a thread's entries at most, halved by the root)
     assert ((out.cpu().double() - want).abs() <= (16 + width / 256) * 2.0 ** -24 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("N,V,H,G,dims,inter", [(64, 64, 3, 2, 64, False), (64, 128, 2, 3, 30, True), (128, 256, 8, 2, 64, False),
+                                                (128, 128, 5, 5, 0, False), (256, 512, 2, 1, 256, True), (30, 44, 3, 1, 14, False)])
+@pytest.mark.parametrize("rows", [1, 639, 645])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_heads_in_two_parts(N, V, H, G, dims, inter, rows, dtype):
+    """Keys of two parts are one row of the cache; otherwise the bits are those of twice as many heads, half as wide."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, M, BS, blocks = HipKernels(), 2, 64, 12
+    gen = torch.Generator().manual_seed(N + V + rows)
+    pos = torch.arange(5, 5 + rows).int().cuda()
+    seq, slot = torch.zeros(rows, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    table = torch.randperm(blocks, generator=gen).int().view(1, blocks).cuda()
+    cols = M * (H + G) * N + G * V
+    src = torch.randn(rows, (cols + 3) // 4 * 4, generator=gen).cuda()[:, :cols]
+    angles = torch.randn(rows, dims // 2, 2, generator=gen).cuda() if dims else None
+    made = lambda *s: torch.full(s, 7.0, dtype=dtype, device="cuda")
+    q, k, v = made(rows, M * H * N), made(blocks, G, BS, M * N), made(blocks, G, V, BS)
+    q2, k2, v2 = made(rows, M * H * N), made(blocks, M * G, BS, N), made(blocks, M * G, V // M, BS)
+
+    def place(lo, hi):
+        turn = {} if angles is None else dict(cos_sin=angles[lo:hi].contiguous(), interleaved=inter, magnitude=1.25)
+        return dict(row_pos=pos[lo:hi].contiguous(), row_seq=seq[lo:hi].contiguous(), seq_slot=slot, block_table=table, block_size=BS, **turn)
+
+    kn.qkv_norm_store(src, q, H, G, M * N, V, 0.0, maps=M, kcache=k, vcache=v, **place(0, rows))
+    for lo in range(0, rows, 100):
+        hi = min(rows, lo + 100)
+        kn.qkv_norm_store(src[lo:hi], q2[lo:hi], M * H, M * G, N, V // M, 0.0, kcache=k2, vcache=v2, **place(lo, hi))
+    assert torch.equal(q, q2) and torch.equal(v, v2.reshape(v.shape))
+    assert torch.equal(k, k2.view(blocks, G, M, BS, N).transpose(2, 3).reshape(k.shape))
