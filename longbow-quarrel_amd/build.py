@@ -3,6 +3,9 @@
 `ensure_built()` is what the kernel loader calls: it compiles when no library
 matching the sources' hash is there, into `_lib/` beside the package or, if that
 place cannot be written, into a per-user folder under the temp directory.
+`ensure_host()` does the same for the module, whose file is named after all that it was compiled against (this
+interpreter, this torch, the sources): another environment's module is never loaded, and several lie side by side.
+Where it cannot be compiled the launches' checks are made in Python.
 `build(force=True)` always compiles.  A progress line goes to stderr for every
 file so that a first call shows that it is alive.
 """
@@ -10,9 +13,11 @@ from __future__ import annotations
 
 import hashlib
 import os
+import shlex
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import time
 from concurrent.futures import ThreadPoolExecutor
@@ -21,7 +26,7 @@ from typing import List, Optional
 PKG_DIR = os.path.dirname(os.path.realpath(__file__))
 SRC_DIR = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "liblqkernels.so"
-HOST_NAME = "lqhost.so"
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared"]
 HOST_SRC = os.path.join(SRC_DIR, "host", "host_calls.cpp")
 ARCH = "gfx950"
 FLAGS = [
@@ -50,11 +55,24 @@ def _headers() -> List[str]:
 def source_hash() -> str:
     h = hashlib.sha256()
     h.update(" ".join(FLAGS).encode())
-    for path in _sources() + _headers() + [HOST_SRC]:
+    for path in _sources() + _headers():
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
+
+
+def host_name() -> str:
+    """The file of the launches' host side that this interpreter and this torch can load.  It reads tensors by their C++
+    layout, so a module that was compiled against others would read wrong addresses and sizes without an error."""
+    import torch
+
+    env = [sysconfig.get_config_var("SOABI") or sys.version, torch.__version__, str(torch.version.git_version),
+           str(int(torch._C._GLIBCXX_USE_CXX11_ABI))] + HOST_FLAGS
+    h = hashlib.sha256("\0".join(env).encode())
+    with open(HOST_SRC, "rb") as f:
+        h.update(f.read())
+    return f"lqhost.{h.hexdigest()[:16]}.so"
 
 
 def _hipcc() -> str:
@@ -90,36 +108,65 @@ def find_built() -> Optional[str]:
     for d in lib_dirs():
         lib = os.path.join(d, LIB_NAME)
         stamp = os.path.join(d, LIB_NAME + ".hash")
-        if os.path.isfile(lib) and os.path.isfile(stamp) and os.path.isfile(os.path.join(d, HOST_NAME)):
+        if os.path.isfile(lib) and os.path.isfile(stamp):
             with open(stamp) as f:
                 if f.read().strip() == want:
                     return lib
     return None
 
 
-def _log(msg: str) -> None:
+def _compiler_env() -> dict:
+    env = dict(os.environ)
+    # an empty or unwritable HOME must not stop the compiler's own caches
+    env.setdefault("TMPDIR", tempfile.gettempdir())
+    return env
+
+
+def log(msg: str) -> None:
     print(f"[longbow-quarrel_amd build] {msg}", file=sys.stderr, flush=True)
 
 
-def build_host(out_dir: str, env) -> None:
-    """The Python module of the launches' host side, against this interpreter's and this torch's headers."""
-    import sysconfig
+def find_host() -> Optional[str]:
+    paths = [os.path.join(d, host_name()) for d in lib_dirs()]
+    return next((p for p in paths if os.path.isfile(p)), None)
 
+
+def build_host(out_dir: str) -> str:
+    """The Python module of the launches' host side, against this interpreter's and this torch's headers."""
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
 
-    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++") or shutil.which("clang++")
+    cxx = shlex.split(os.environ.get("CXX", "")) or [c for c in map(shutil.which, ("g++", "c++", "clang++")) if c][:1]
     if not cxx:
         raise BuildError("no C++ compiler for the launches' host side (looked at $CXX, g++, c++, clang++)")
-    tmp = os.path.join(out_dir, f".{HOST_NAME}.{os.getpid()}")
-    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    tmp = os.path.join(out_dir, f".lqhost.{os.getpid()}")
+    cmd = [*cxx, *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
     for path in include_paths() + [sysconfig.get_paths()["include"]]:
         cmd += ["-isystem", path]
     cmd += [HOST_SRC, "-o", tmp] + [f"-L{path}" for path in library_paths()] + ["-ltorch_python", "-ltorch_cpu", "-lc10"]
-    proc = subprocess.run(cmd, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+    try:
+        proc = subprocess.run(cmd, env=_compiler_env(), stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+    except OSError as e:
+        raise BuildError(f"{cxx[0]}: {e}") from e
     if proc.returncode != 0:
-        raise BuildError(f"{cxx} failed on {HOST_SRC}:\n{proc.stderr[-4000:]}")
-    os.replace(tmp, os.path.join(out_dir, HOST_NAME))
+        raise BuildError(f"{cxx[0]} failed on {HOST_SRC}:\n{proc.stderr[-4000:]}")
+    path = os.path.join(out_dir, host_name())
+    os.replace(tmp, path)
+    return path
+
+
+def ensure_host() -> str:
+    """The module's path; compiled now if this environment has none (BuildError where that cannot be done)."""
+    got = find_host()
+    if got:
+        return got
+    out_dir = next((d for d in lib_dirs() if _writable_dir(d)), None)
+    if out_dir is None:
+        raise BuildError(f"no writable place for the launches' host side among {lib_dirs()}")
+    t = time.time()
+    path = build_host(out_dir)
+    log(f"built {path} in {time.time() - t:.1f}s")
+    return path
 
 
 def build(force: bool = False, jobs: Optional[int] = None) -> str:
@@ -133,13 +180,11 @@ def build(force: bool = False, jobs: Optional[int] = None) -> str:
         raise BuildError(f"no writable place for the kernel library among {lib_dirs()}")
     obj_dir = os.path.join(out_dir, "obj")
     os.makedirs(obj_dir, exist_ok=True)
-    env = dict(os.environ)
-    # an empty or unwritable HOME must not stop the compiler's own caches
-    env.setdefault("TMPDIR", tempfile.gettempdir())
+    env = _compiler_env()
     srcs = _sources()
     jobs = jobs or min(len(srcs), int(os.environ.get("MAX_JOBS", "8")), 16)
     t0 = time.time()
-    _log(f"compiling {len(srcs)} files for {ARCH} with {hipcc} into {out_dir}")
+    log(f"compiling {len(srcs)} files for {ARCH} with {hipcc} into {out_dir}")
 
     def compile_one(src: str) -> str:
         obj = os.path.join(obj_dir, os.path.basename(src)[:-4] + ".o")
@@ -148,13 +193,18 @@ def build(force: bool = False, jobs: Optional[int] = None) -> str:
         proc = subprocess.run(cmd, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
         if proc.returncode != 0:
             raise BuildError(f"hipcc failed on {src}:\n{proc.stderr[-4000:]}")
-        _log(f"  {os.path.basename(src)} done in {time.time() - t:.1f}s")
+        log(f"  {os.path.basename(src)} done in {time.time() - t:.1f}s")
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        host = pool.submit(build_host, out_dir, env)
+        host = pool.submit(build_host, out_dir)
         objs = list(pool.map(compile_one, srcs))
-        host.result()
+        try:
+            host.result()
+        except BuildError as e:  # (the kernels need no module: whoever loads them does without)
+            if force:
+                raise
+            log(str(e))
     lib_tmp = os.path.join(out_dir, f".{LIB_NAME}.{os.getpid()}")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", lib_tmp]
     proc = subprocess.run(cmd, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
@@ -164,7 +214,7 @@ def build(force: bool = False, jobs: Optional[int] = None) -> str:
     os.replace(lib_tmp, lib)
     with open(os.path.join(out_dir, LIB_NAME + ".hash"), "w") as f:
         f.write(source_hash())
-    _log(f"built {lib} in {time.time() - t0:.1f}s")
+    log(f"built {lib} in {time.time() - t0:.1f}s")
     return lib
 
 
