@@ -1422,14 +1422,13 @@ class HipKernels:
         if kcache is not None:
             kv = kv_weight.numel()
             self._f32(kv_weight, "latent_rows: kv_weight", kv)
-            self._dev(kcache, vcache, block_table)
+            self._dev(kcache, vcache, row_pos, row_seq, seq_slot, block_table)
             dims = self._angles(cos_sin, rows, "latent_rows")
-            for t, what in ((row_pos, "row_pos"), (row_seq, "row_seq")):
-                self._i32(t, what, rows)
-            if ns != nq + kv + rot_dim or tuple(kcache.shape[1:]) != (1, block_size, kv + rot_dim) \
-                    or tuple(vcache.shape[1:]) != (1, kv, block_size) or kcache.dtype != cq.dtype or vcache.dtype != cq.dtype \
-                    or not kcache.is_contiguous() or not vcache.is_contiguous() or block_table.dtype != torch.int32:
-                raise KernelLibraryError("latent_rows: src [rows, q | latent | rotated], a cache of latent rows")
+            self._i32(row_pos, "row_pos", rows)
+            self._i32(row_seq, "row_seq", rows)
+            self._check_paged(kcache, vcache, 1, kv + rot_dim, kv, block_size, block_table, seq_slot, "latent_rows")
+            if ns != nq + kv + rot_dim or kcache.dtype != cq.dtype:
+                raise KernelLibraryError("latent_rows: src [rows, q | latent | rotated], a cache of latent rows in cq's dtype")
         elif ns != nq:
             raise KernelLibraryError("latent_rows: without a cache src holds the q columns alone")
         self._check(self.lib.lq_latent_rows(
