@@ -141,6 +141,8 @@ class PackedWeight:
         return self.whole == self.shape[1]
 
     def contiguous(self) -> "PackedWeight":
+        if not self.is_contiguous():
+            raise KernelLibraryError("a run of a packed weight's columns has no copy of its own")
         return self
 
     def numel(self) -> int:
@@ -1872,7 +1874,8 @@ class HipKernels:
         if start % 8 or n % 8 or start + n > rows or \
                 not self.lib.lq_weight_packable(c_int(_DTYPE_CODE[w.dtype]), c_int(n), c_int(k)):
             return None
-        return PackedWeight(w.data.view(-1)[start * k : (start + n) * k].view(n, k), n, k)
+        run = w.data.view(-1)[start * w.whole :]
+        return PackedWeight(run[: n * k].view(n, k), n, k) if w.whole == k else PackedWeight(run, n, k, whole=w.whole)
 
     def weight_columns(self, w, start: int, n: int):
         """Columns start .. start + n of a product weight as a weight of its own: a view of a dense one; of a packed one

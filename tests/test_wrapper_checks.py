@@ -45,3 +45,28 @@ def test_a_latent_layers_rows_and_their_places(kn):
             kn.latent_rows(**{**given, name: wrong})
     with pytest.raises(pytest.fail.Exception):  # (the whole of it comes through)
         kn.latent_rows(**given)
+
+
+def test_runs_of_a_packed_weight():
+    """Rows of a run of columns lie as far apart as the whole matrix's: runs of runs begin where `packed_at` says."""
+    kn = object.__new__(HipKernels)
+    kn.lib = hip.load_library()
+    rows, cols = 4112, 1600
+    whole = hip.PackedWeight(torch.arange(rows * cols).to(torch.int32).view(torch.bfloat16).view(-1)[::2].reshape(rows, cols), rows, cols)
+    packed_at = lambda r, c: (r // 8 * 8) * cols + c // 64 * 512 + r % 8 * 64 + c % 64  # (8 rows' runs of 64 side by side)
+    flat = whole.data.view(-1)
+
+    def begins_at(w, r, c):
+        return w.data_ptr() == flat[packed_at(r, c):].data_ptr()
+
+    columns = kn.weight_columns(whole, 1024, 576)
+    assert tuple(columns.shape) == (rows, 576) and columns.stride() == (cols, 1) and begins_at(columns, 0, 1024)
+    part = kn.weight_rows(columns, 16, 2048)
+    assert tuple(part.shape) == (2048, 576) and part.stride() == (cols, 1) and begins_at(part, 16, 1024)
+    assert not part.is_contiguous() and kn.weight_columns(part, 0, 512) is None
+    with pytest.raises(KernelLibraryError):
+        part.contiguous()
+    part = kn.weight_rows(whole, 2056, 2056)
+    assert part.stride() == (cols, 1) and begins_at(part, 2056, 0) and part.contiguous() is part and part.data.numel() == part.numel()
+    for start, n in ((4, 2048), (0, 2052), (2072, 2048), (0, 1024)):
+        assert kn.weight_rows(columns, start, n) is None
