@@ -1228,10 +1228,12 @@ int best_tile(int M, int N, int K, int splits) {
   return best;
 }
 
-// From 65 rows, or 17 of a weight too narrow for the kernels that stream a wide one (40 rows of 1 536 x 1 536 8.8 -> 7.7 us, in four
-// pieces 4.2; of 1 024 x 3 584 15.6 -> 14.2 and 5.8).
-inline bool takes_rows(int M, int N, int K) {
-  return K % 64 == 0 && K >= 512 && (M > 64 || (M > 16 && N < 8 * lq_compute_units()));
+// From 65 rows, or 17 of a weight too narrow for the kernels that stream a wide one: in pieces (from K 1 024 on up to 32 rows), and whole
+// from 33 rows.  Microseconds, the simple kernel / 64 x 64 tiles whole / in pieces with their addition, 1 536 columns: 17 rows of K 512
+// 4.0 / 4.6 / 4.2, of 2 048 7.1 / 9.4 / 5.7, of 4 096 11.1 / 15.8 / 7.3, of 14 336 34.9 / 57.5 / 14.0; 24 rows 4.3 / 4.7 / 4.2, 8.2 / 9.5 / 5.8, 13.0 / 16.0 /
+// 7.4, 40.7 / 58.3 / 14.1; 40 rows 5.4 / 4.8 / 4.4, 10.8 / 9.6 / 6.0, 17.8 / 16.1 / 7.6, 58.4 / 60.5 / 14.7.
+inline bool takes_rows(int M, int N, int K, bool pieces) {
+  return K % 64 == 0 && K >= 512 && (M > 64 || (N < 8 * lq_compute_units() && (M > 32 || (M > 16 && pieces && K >= 1024))));
 }
 
 // Shares of K: as many as make the product (whose time has the writing of its pieces) and the reading of the further pieces, 4
@@ -1286,7 +1288,7 @@ int narrow_splits(int M, int N, int K) {
 
 int mfma_splits(int M, int N, int K) {
   if (mid_rows(M, N, K)) return mid_splits(N, K);
-  return takes_rows(M, N, K) ? tiled_splits(M, N, K) : v3_splits(M, N, K);
+  return takes_rows(M, N, K, true) ? tiled_splits(M, N, K) : v3_splits(M, N, K);
 }
 
 template <int EPI, typename TO>
@@ -1306,7 +1308,7 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
     }
   }
   if (mid_rows(M, N, K)) return launch_mid<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-  if (takes_rows(M, N, K)) return launch_rows<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+  if (takes_rows(M, N, K, splits > 1)) return launch_rows<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   if (splits > 1) {
     if (M <= 32) return launch_skinny_v3<2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
     return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);

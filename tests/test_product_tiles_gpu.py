@@ -67,3 +67,18 @@ def test_groups_of_rows_on_every_tile(counts, n, k):
         assert within(out[at : at + c], x[at : at + c], ws[e]), e
         at += c
     assert bool((out[at:] == 7).all())
+
+
+@pytest.mark.parametrize("n,k", [(128, 512), (1536, 2048), (1000, 4096)])
+def test_whole_products_of_a_few_rows_more_than_16(n, k):
+    """Up to 32 rows of a narrow weight stay with the kernel of 16 rows: the same sums, bit for bit."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    x, w = torch.randn(32, k, generator=gen, device="cuda").bfloat16(), torch.randn(n, k, generator=gen, device="cuda").bfloat16()
+    few = torch.cat([kn.linear(x[at : at + 16], w, part := torch.empty(16, n, device="cuda")) or part for at in (0, 16)])
+    for rows in (17, 24, 32):
+        got = torch.empty(rows, n, device="cuda")
+        kn.linear(x[:rows], w, got)
+        assert within(got, x[:rows], w) and torch.equal(got, few[:rows])
