@@ -1001,18 +1001,21 @@ struct Branches {
   long long apart;
 };
 
-template <typename T, int PER>
+// EARLY: the last weight is asked for ahead of the sums, whose barriers no load passes.  That is a round trip less for few rows (8 rows
+// of 4 096, one branch 5.61 -> 5.25 us, two 7.59 -> 7.27); many rows hide it and pay for the registers with fewer workgroups a compute
+// unit (1 000 rows of 3 072, one branch 7.7 -> 9.7, three 15.9 -> 20.3; 4 096 rows of 4 096, three 64 -> 72).
+template <typename T, int PER, bool EARLY>
 __global__ __launch_bounds__(256) void branches_residual_kernel(float* __restrict__ x, Branches in, int n_in, float branch_eps,
                                                                 const float* __restrict__ w, float eps,
                                                                 T* __restrict__ rounded, int width) {
   __shared__ float red[16];
   const long long base = (long long)blockIdx.x * width;
   const int quads = width / 4;
-  embed_f32x4 xv[PER], y[PER], one[PER], gain[PER];  // (all asked for ahead of the sums, whose barriers no load passes)
+  embed_f32x4 xv[PER], y[PER], one[PER], gain[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int q = threadIdx.x + i * 256;
-    gain[i] = q < quads ? ((const embed_f32x4*)w)[q] : (embed_f32x4){0.f, 0.f, 0.f, 0.f};
+    if constexpr (EARLY) gain[i] = q < quads ? ((const embed_f32x4*)w)[q] : (embed_f32x4){0.f, 0.f, 0.f, 0.f};
     one[i] = q < quads ? ((const embed_f32x4*)(in.y[0] + base))[q] : (embed_f32x4){0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
@@ -1060,6 +1063,7 @@ __global__ __launch_bounds__(256) void branches_residual_kernel(float* __restric
   for (int i = 0; i < PER; ++i) {
     const int q = threadIdx.x + i * 256;
     if (q >= quads) continue;
+    if constexpr (!EARLY) gain[i] = ((const embed_f32x4*)w)[q];
     const embed_f32x4 v = xv[i] + y[i] * inv * gain[i];
     ((embed_f32x4*)(x + base))[q] = v;
     if (rounded != nullptr) {
@@ -1292,14 +1296,17 @@ static bool branches_fit(const float* x, const void* rounded, int rounded_dtype,
 static int launch_branches(float* x, const Branches& in, int n_in, float branch_eps, const float* w, float eps, void* rounded,
                            int rounded_dtype, int rows, int width, hipStream_t stream) {
   const int per = lq_ceil_div(width / 4, 256);
-#define LQ_BRANCHES(T, PER)                                                                                                \
-  branches_residual_kernel<T, PER><<<rows, 256, 0, stream>>>(x, in, n_in, branch_eps, w, eps, (T*)rounded, width)
-#define LQ_BRANCHES_T(T)                          \
-  do {                                            \
-    if (per <= 1) LQ_BRANCHES(T, 1);              \
-    else if (per <= 2) LQ_BRANCHES(T, 2);         \
-    else if (per <= 4) LQ_BRANCHES(T, 4);         \
-    else LQ_BRANCHES(T, 8);                       \
+  const bool early = rows <= 2 * lq_compute_units();  // (of 1 024 columns and fewer, and of more than 4 096, neither way is faster)
+#define LQ_BRANCHES(T, PER, EARLY)                                                                                         \
+  branches_residual_kernel<T, PER, EARLY><<<rows, 256, 0, stream>>>(x, in, n_in, branch_eps, w, eps, (T*)rounded, width)
+#define LQ_BRANCHES_T(T)                                       \
+  do {                                                         \
+    if (per <= 1) LQ_BRANCHES(T, 1, false);                    \
+    else if (per <= 2 && early) LQ_BRANCHES(T, 2, true);       \
+    else if (per <= 2) LQ_BRANCHES(T, 2, false);               \
+    else if (per <= 4 && early) LQ_BRANCHES(T, 4, true);       \
+    else if (per <= 4) LQ_BRANCHES(T, 4, false);               \
+    else LQ_BRANCHES(T, 8, false);                             \
   } while (0)
   if (rounded == nullptr || rounded_dtype == LQ_F32) LQ_BRANCHES_T(float);
   else if (rounded_dtype == LQ_BF16) LQ_BRANCHES_T(bf16_t);
