@@ -649,16 +649,32 @@ int lq_delta_chunks(const float* q, int ldq, const float* k, int ldk, const floa
 }
 
 // ---- gated linear attention
-// Float32 scratch for a launch in chunks (0: sizes that are not taken, or a launch that is faster token by token: the longest
-// portion below 48 tokens, 96 of states of up to 4 096 entries).  Microseconds, token by token (in segments where it has them) and
-// in chunks, heads of 128 x 256: 8 heads, 48 tokens 27 / 25, 128 tokens 60 / 29, 512 165 / 44, 3 000 781 / 144, eight sequences
-// of 200 to 700 710 / 135, 24 of 120 400 / 119, 300 tokens beside seven of one 189 / 59; 16 heads, 2 048 994 / 119; 4 heads of 64 x
-// 64, 64 tokens 26 / 27, 300 99 / 35.  Error against 64 bits, 2 048 tokens of 128 x 256: 2.8e-6 and 5.0e-7, of the state they leave
+// Float32 scratch for a launch in chunks (0: sizes that are not taken: key heads of more than 128, portions below 48 tokens, 96 of
+// states of up to 4 096 entries).  Microseconds, token by token (in segments where it has them) and
+// in chunks, heads of 128 x 256: 8 heads, 48 tokens 28 / 25, 128 tokens 59 / 30, 512 159 / 44, 3 000 781 / 144, eight sequences
+// of 200 to 700 710 / 135, 24 of 120 400 / 119; 16 heads, 2 048 994 / 119; 4 heads of 64 x
+// 64, 300 tokens 99 / 35.  Error against 64 bits, 2 048 tokens of 128 x 256: 2.8e-6 and 5.0e-7, of the state they leave
 // 4.3e-6 and 3.1e-7; 64 tokens 2.2e-7 and 2.3e-7.
 extern "C" long long lq_gla_chunks_workspace(int rows, int batch, int heads, int Dk, int P, int max_rows) {
   if (rows <= 0 || batch <= 0 || heads <= 0 || P <= 0 || Dk <= 0 || Dk > NMAX || max_rows < (Dk * P > 4096 ? 48 : 96)) return 0;
   if (heads > 65535 || lq_ceil_div(P, 16) > 65535) return 0;
   return chunks_scratch(most_chunks(rows, batch, 1), lq_delta_scan_least(heads), LQ_DELTA_SCRATCH);
+}
+
+// Whether a launch is faster in chunks than token by token, by what both take.  A chunk costs the same however few tokens it has, so
+// that one prompt beside many single tokens, or many short portions, may be sooner walked.  Microseconds, walk / chunks, 16 heads of 64 x
+// 128: 300 tokens alone 99 / 37, beside 31 single ones 127 / 115, beside 128 160 / 405; 48 beside 128 77 / 387; 24 portions of 64 74 / 92, 96
+// of 64 261 / 357; 16 heads of 128 x 256, 64 tokens beside 128 554 / 740, 512 beside 128 818 / 775.  Over 1 116 launches (see lq_gla_walk_us; this
+// estimate is off by 13 %) the way that is named takes 0.5 % more than the better of the two, and in five of them 5 % and more above the walk
+// (64 heads of 64 x 64, two sequences of 1 000 beside 30 of 5: 344 / 567; 16 of 64 x 128, eight of 512 beside 56 of 1: 273 / 340).
+double lq_gla_walk_us(int rows, int batch, int heads, int N, int P, int max_rows);
+extern "C" int lq_gla_scan_in_chunks(int rows, int batch, int heads, int Dk, int P, int max_rows) {
+  if (lq_gla_chunks_workspace(rows, batch, heads, Dk, P, max_rows) == 0) return 0;
+  const double longest = lq_ceil_div(max_rows, CHUNK), others = batch - 1, mean = others > 0 ? (rows - max_rows) / others / CHUNK + 0.5 : 0;
+  const double chunks = heads * (longest + others * (mean > 1 ? mean : 1));
+  const double products = 0.005 * lq_ceil_div(P, 16) * chunks, chain = 2.5 * longest, state = (double)batch * heads * P * Dk / (128 * 128);
+  const double us = 20 + (Dk % 4 == 0 ? 0.09 : 0.1) * chunks + (products > chain ? products : chain) + 0.076 * state;
+  return us < lq_gla_walk_us(rows, batch, heads, Dk, P, max_rows);
 }
 
 int lq_gla_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* z, int ldz, const float* bias,

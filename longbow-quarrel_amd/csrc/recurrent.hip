@@ -1491,6 +1491,20 @@ extern "C" long long lq_gla_scan_workspace(int batch, int heads, int P, int N, i
   return gla_segment_floats(batch, heads, P, N, max_rows);
 }
 
+// Microseconds that a launch takes token by token (in segments where it has them): a workgroup's token, all of them over the chip or
+// the longest sequence's one after the other, and the states read and written.  Fitted to 1 116 launches of eleven sizes (2 to 64 heads of
+// 17 x 40 to 128 x 512, 1 to 129 sequences of 1 to 3 000 tokens), off by 20 % (r.m.s.).
+double lq_gla_walk_us(int rows, int batch, int heads, int N, int P, int max_rows) {
+  ScanLaunch cfg;
+  if (!scan_launch(N, P, (long long)batch * heads, cfg)) return 1e30;
+  const double width = cfg.ln * cfg.slab / 128.0, state = (double)heads * P * width / 128;
+  const double tokens = (0.15 + 0.77 * width) * 1e-3 * rows * heads * lq_ceil_div(P, cfg.cols);
+  if (gla_segment_floats(batch, heads, P, N, max_rows) == 0)
+    return 3 + hypot(tokens, (0.2 + 0.26 * width) * max_rows) + 0.117 * state * batch;
+  const int cut = rows / SEG_MIN_ROWS < batch ? rows / SEG_MIN_ROWS : batch;  // sequences in segments, at most
+  return 10 + hypot(2 * tokens, 0.073 * max_rows) + state * (1.26 * cut + 0.117 * (batch - cut));
+}
+
 int lq_gla_chunks(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* z, int ldz, const float* bias,
                   float* state, float* out, int ldo, int heads, int Dk, int P, float q_scale, float inv_tau, const int* seq_slot,
                   const int* cu_rows, int batch, int rows, float* scratch, long long scratch_floats, hipStream_t stream);

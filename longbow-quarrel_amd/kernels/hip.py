@@ -1642,12 +1642,18 @@ class HipKernels:
 
     @query
     def gla_chunks_workspace(self, rows: int, batch: int, heads: int, key_dim: int, value_dim: int, max_rows: int) -> int:
-        """Float32 entries of scratch with which `gla_scan` runs this launch in chunks on the matrix cores (0: it is not to)."""
+        """Float32 entries of scratch with which `gla_scan` runs this launch in chunks on the matrix cores (0: it does not)."""
         if self.force_generic:
             return 0
         self.lib.lq_gla_chunks_workspace.restype = c_longlong
         return int(self.lib.lq_gla_chunks_workspace(c_int(rows), c_int(batch), c_int(heads), c_int(key_dim), c_int(value_dim),
                                                     c_int(max_rows)))
+
+    @query
+    def gla_scan_in_chunks(self, rows: int, batch: int, heads: int, key_dim: int, value_dim: int, max_rows: int) -> bool:
+        """Whether `gla_scan` is faster in chunks of tokens than token by token, for these sizes."""
+        return not self.force_generic and bool(self.lib.lq_gla_scan_in_chunks(
+            c_int(rows), c_int(batch), c_int(heads), c_int(key_dim), c_int(value_dim), c_int(max_rows)))
 
     def gla_scan(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, z: torch.Tensor, bias: torch.Tensor,
                  state: torch.Tensor, out: torch.Tensor, heads: int, key_dim: int, value_dim: int, q_scale: float,

@@ -614,8 +614,9 @@ class GatedLinearAttention(Mixer):
         o = ctx.ws.alloc((rows, vw), torch.float32)
         # a bfloat16 run's prompts go in chunks where that is faster; else a few long ones may be cut into segments that run
         # side by side, given scratch
-        chunks = getattr(kn, "gla_chunks_workspace", None) if ctx.dtype != torch.float32 and not ctx.decode else None
-        need = chunks(rows, ctx.batch, self.heads, self.key_dim, self.value_dim, ctx.max_new) if chunks is not None else 0
+        sizes = (rows, ctx.batch, self.heads, self.key_dim, self.value_dim, ctx.max_new)
+        faster = getattr(kn, "gla_scan_in_chunks", None) if ctx.dtype != torch.float32 and not ctx.decode else None
+        need = kn.gla_chunks_workspace(*sizes) if faster is not None and faster(*sizes) else 0
         more = {"chunked": True} if need else {}
         if not need:
             ask = getattr(kn, "gla_scan_workspace", None)
