@@ -1143,6 +1143,12 @@ inline bool mid_rows(int M, int N, int K) {
   return M > LQ_MID_ROWS_FROM && M <= 64 && K % 64 == 0 && K >= 512 && N >= 8 * lq_compute_units();
 }
 
+// Whole products of up to 32 rows and 16 columns a compute unit stay with the balanced kernel: the covering tiles, 32 columns each, are then
+// few and walk K alone.  Microseconds, tiles / balanced: 2 048 columns of K 7 296, 13 rows 28.6 / 13.1, 16 28.6 / 13.9, 24 28.4 / 19.2, 32
+// 28.8 / 22.5, 33 28.7 / 23.7, 48 28.7 / 29.8; of K 512, 16 rows 4.7 / 3.8, 32 5.0 / 4.2; 4 096 columns of K 4 096, 16 rows 17.9 / 12.0, 32 17.8 / 16.2, 48
+// 17.7 / 19.8; 6 144 of K 2 048, 16 rows 10.7 / 8.9, 32 10.7 / 11.7.
+inline bool few_whole(int M, int N) { return M <= 32 && N <= 16 * lq_compute_units(); }
+
 inline int mid_splits_for(int tiles, int K) {
   const int want = 3 * lq_compute_units() / 4;
   int splits = 1;
@@ -1307,7 +1313,7 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
       return -1;
     }
   }
-  if (mid_rows(M, N, K)) return launch_mid<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+  if (mid_rows(M, N, K) && !(splits == 1 && few_whole(M, N))) return launch_mid<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   if (takes_rows(M, N, K, splits > 1)) return launch_rows<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   if (splits > 1) {
     if (M <= 32) return launch_skinny_v3<2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);

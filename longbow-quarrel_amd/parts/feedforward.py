@@ -79,17 +79,20 @@ class GatedLinearUnit(FeedForward):
 
     graph_safe = True
     ACTIVATIONS = ("silu", "relu", "gelu_tanh")
-    #: columns behind the activations, a one and zeros: a product's K stays a multiple of 64, without which neither the packed
-    #: weights nor the pipelined tiles take it (2 048 x 7 168: 100 rows 106 us with 8 columns, 27 with 64; 2 635 rows 146 and 97;
-    #: a few rows 9.0 and 10.7), or of eight
-    BIAS_TAIL = {True: 64, False: 8}
+    @staticmethod
+    def bias_tail(inner: int) -> int:
+        """Columns behind the activations, a one and zeros: the second product's K is then a multiple of 128 where that takes no more
+        than 128 of them, else of eight.  The packed weights and the pipelined tiles want K in 64s, the kernel of at most 8 rows in
+        pairs of 64.  Microseconds of 2 048 x 7 168 with 8, 64 and 128 columns: 1 row 10.3, 11.1, 8.9; 4 rows 10.1, 10.7, 9.5; 8 rows 10.8, 11.4, 11.4;
+        16 rows 12.9, 13.8, 13.7; 32 rows 22.0, 22.0, 22.2; 100 rows 139, 31, 31; 2 635 rows 148, 102, 102."""
+        return 128 - inner % 128 if inner % 64 == 0 else 8
 
     def __init__(self, width: int, inner: int, prefix: str, activation: str = "silu", bias: bool = False,
                  names: Optional[Mapping[str, str]] = None) -> None:
         if activation not in self.ACTIVATIONS:
             raise ValueError(f"unknown activation {activation!r}; known: {', '.join(self.ACTIVATIONS)}")
         self.width, self.inner, self.activation, self.bias = int(width), int(inner), activation, bool(bias)
-        self.tail = self.BIAS_TAIL[self.inner % 64 == 0]
+        self.tail = self.bias_tail(self.inner)
         n = {"gate": "gate", "up": "up", "down": "down"}
         n.update(names or {})
         self.names: Dict[str, str] = {key: f"{prefix}.{val}" for key, val in n.items()}

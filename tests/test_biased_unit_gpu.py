@@ -1,0 +1,43 @@
+"""A gated unit with biases, whose second product carries its bias as one more column behind the activations."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from longbow_quarrel_amd.parts.feedforward import GatedLinearUnit
+
+
+def test_columns_behind_the_activations():
+    """K in 128s, which the kernel of at most 8 rows wants, wherever K was in 64s."""
+    for inner in (64, 128, 576, 1024, 4032, 7168):
+        tail = GatedLinearUnit(64, inner, "m", bias=True).tail
+        assert (inner + tail) % 128 == 0 and 0 < tail <= 128
+    assert GatedLinearUnit(64, 40, "m", bias=True).tail == 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,inner", [(512, 576), (512, 512), (2048, 640), (264, 520), (2056, 1024)])
+@pytest.mark.parametrize("rows", [1, 8, 17, 33, 100])
+def test_against_the_formula(width, inner, rows):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+    from longbow_quarrel_amd.parts import BuildEnv
+    from longbow_quarrel_amd.weights import random_tensors
+
+    kn, dev = HipKernels(), torch.device("cuda:0")
+    part = GatedLinearUnit(width, inner, "m", bias=True)
+    tensors = random_tensors(part.tensor_specs(), 3, torch.bfloat16, 0.1, device=dev)
+    tensors = {s.name: tensors[s.name].float() if s.kind == "vector32" else tensors[s.name] for s in part.tensor_specs()}
+    part.bind(dict(tensors), BuildEnv(torch.bfloat16, dev, kn))
+    h = torch.randn(rows, width, generator=torch.Generator().manual_seed(inner)).bfloat16().cuda()
+    ws = SimpleNamespace(alloc=lambda shape, dtype, **_: torch.full(tuple(shape), float("nan"), dtype=dtype, device=dev))
+    got = part.forward(h, SimpleNamespace(kernels=kn, ws=ws, dtype=torch.bfloat16)).double()
+
+    t = {k: v.double() for k, v in tensors.items()}
+    g, u = (h.double() @ t[f"m.{n}"].T + t[f"m.{n}.b"] for n in ("gate", "up"))
+    act = (g * torch.sigmoid(g) * u).bfloat16().double()
+    want = act @ t["m.down"].T + t["m.down.b"]
+    # 32-bit sums of exact products in the second, and in the first so close to 64 bits that an activation rounds to its other
+    # neighbour in bfloat16 (2^-8 of it) about once in a thousand: four of the row's largest allow for that
+    terms = act.abs() @ t["m.down"].abs().T + t["m.down.b"].abs()
+    largest = act.abs().amax(1, keepdim=True) * t["m.down"].abs().amax(1)
+    assert ((got - want).abs() <= (inner + 128) * 2.0 ** -24 * terms + 4 * 2.0 ** -8 * largest).all()

@@ -82,3 +82,29 @@ def test_whole_products_of_a_few_rows_more_than_16(n, k):
         got = torch.empty(rows, n, device="cuda")
         kn.linear(x[:rows], w, got)
         assert within(got, x[:rows], w) and torch.equal(got, few[:rows])
+
+
+@pytest.mark.parametrize("n,k", [(2048, 512), (2056, 7296), (4096, 2048), (4104, 1088)])
+def test_whole_products_of_13_to_32_rows(n, k):
+    """Up to 4 096 columns they stay with the kernel of fewer rows: up to 16 the same sums, bit for bit."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, bf = HipKernels(), torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    x, w = torch.randn(33, k, generator=gen, device="cuda").to(bf), torch.randn(n, k, generator=gen, device="cuda").to(bf)
+    few = torch.empty(12, n, device="cuda")
+    kn.linear(x[:12], w, few)
+    for held in (w, kn.pack_weight(w)):
+        for rows in (13, 16, 17, 32, 33):
+            got = torch.full((rows + 1, n), 7.0, device="cuda")
+            kn.linear(x[:rows], held, got[:rows])
+            assert within(got[:rows], x[:rows], w) and bool((got[rows:] == 7).all())
+            assert rows > 16 or n > 4096 or torch.equal(got[:12], few)
+            out = torch.full((rows, n), float("nan"), dtype=bf, device="cuda")
+            kn.linear(x[:rows], held, out)
+            assert torch.equal(out, got[:rows].to(bf))
+            if n % 16 == 0:
+                gated = torch.full((rows, n // 2), float("nan"), dtype=bf, device="cuda")
+                kn.linear_swiglu(x[:rows], held, gated, activation="relu")
+                gate, up = got[:rows].view(rows, n // 16, 2, 8).unbind(2)
+                assert torch.equal(gated, (gate.clamp(min=0) * up).reshape(rows, n // 2).to(bf))
