@@ -720,10 +720,14 @@ extern "C" int lq_qkv_norm_store(const float* src, int lds_, const float* bias, 
   const bool fours = key_dim % 4 == 0 && unit_q % 4 == 0 && unit_k % 4 == 0 && value_dim % 4 == 0 && lds_ % 4 == 0 && ldq % 4 == 0 && (uintptr_t)src % 16 == 0 &&
                      (uintptr_t)bias % 16 == 0 && (uintptr_t)wq % 16 == 0 && (uintptr_t)wk % 16 == 0 &&
                      (uintptr_t)q_out % (4 * el) == 0 && (uintptr_t)kcache % (4 * el) == 0 && most <= 16384;
-  // many rows of units of 64, 128 or 256, values of a unit's size or twice it: the kernel that takes runs of rows.  Microseconds, 16 query
-  // heads of 128 over 4, by units and by runs: 64 rows 4.2 / 7.3, 500 rows 8.3 / 9.3, 800 rows 11.9 / 10.5, 2 000 rows 26.2 / 16.0,
-  // 2 635 rows 33.2 / 21.4, 4 096 rows 48.8 / 31.1
-  const bool runs = fours && rows >= 640 && unit_q == unit_k && key_dim % unit_q == 0 &&
+  // many rows of units of 64, 128 or 256, values of a unit's size or twice it: the kernel that takes runs of rows.  It gains where rows
+  // are wide: a workgroup has lanes for 1 024 entries of the values, which few heads leave idle.  Microseconds by units and by runs, one
+  // sequence (and a row a sequence): 32 query heads of 64 over 8, 640 rows 17.4 / 10.9 (21.9 / 14.2); 64 of 128 over 8, 640 rows 29.3 / 19.7 (32.2 / 22.9);
+  // 16 of 128 over 4, 640 rows 11.1 / 11.0 (13.0 / 14.3), 900 14.5 / 13.4 (17.5 / 16.9), 2 000 26.2 / 16.0, 4 096 48.8 / 31.1; 16 of 256 over 4, 640 rows 15.5 /
+  // 16.3 (18.9 / 20.2), 900 20.5 / 19.9 (25.0 / 24.5); 8 of 256 over 2, 640 rows 9.3 / 11.0 (10.8 / 14.5), 1 300 15.8 / 17.0; 4 of 256 over 1, 640 rows 6.7 / 9.3,
+  // 4 096 21.5 / 23.7
+  const int least = unit_q == 64 || (unit_q == 128 && kv_heads >= 8) ? 640 : unit_q == 128 || kv_heads >= 4 ? 1024 : 2048;
+  const bool runs = fours && rows >= least && (unit_q != 256 || kv_heads >= 2) && unit_q == unit_k && key_dim % unit_q == 0 &&
                     (kcache == nullptr || (unit_v == value_dim && (value_dim == unit_q || value_dim == 2 * unit_q))) &&
                     (unit_q == 64 || unit_q == 128 || (unit_q == 256 && (kcache == nullptr || value_dim == 256))) && block_size % RUN == 0 &&
                     (uintptr_t)vcache % 16 == 0 && (long long)rows * (heads + kv_heads) * (key_dim / unit_q) < (1ll << 30);
