@@ -1199,11 +1199,14 @@ int launch_mid(const void* x, const void* w, void* out, int M, int N, int K, int
 // So a product asks what each tile would take: microseconds are
 //   fixed + slabs (per_round * rounds + per_layer * layers + per_fill * fill) + out_fill * fill,
 // slabs of 64 k, fill the tiles (times shares) a compute unit, rounds and layers how often all units are filled with as many as fit
-// and with one each.  The constants are least-squares fits to 19 sizes (1 024 to 14 336 columns of K 1 024 to 14 336) at 64 to
-// 4 096 rows and 1 to 8 shares, weights from memory; the fits are off by 6 to 9 % (r.m.s.), and the tile that they name takes
-// 0.2 % more than the best of the six on average, 17 % at most.  Against one rule for each range of rows (256 x 256, 256 x 192,
-// 128 x 128 and one covering tile up to 256 rows) the products take 0.79 of the time on average over these sizes whole, 0.72 in pieces
-// with their addition: 512 rows of 2 048 x 3 584 30.3 -> 15.9 us, 2 635 of 4 112 x 2 048 74 -> 45, 4 096 x 2 048 x 2 048 46 -> 36.
+// and with one each.  The constants are least-squares fits at 64 to 4 096 rows and 1 to 8 shares, weights from memory.  Measured again over
+// 4 406 products (15 row counts of 65 to 4 096, 1 024 to 28 672 columns, K 512 to 14 336), each on all six tiles: times of 32-bit results
+// lie 6 to 8 % above the estimate and scatter by 7 to 9 %, gated ones 10 to 22 % above, and the tile that is named takes 0.6 % more than the best of
+// the six on average, 28 % at most.  Against one rule for each range of rows (256 x 256, 256 x 192, 128 x 128 and one covering tile up to 256 rows)
+// over 6 283 products of 17 rows and more: 0.78 of the time on average, 54 of them more than 5 % slower, 16 % at most (300 rows of 4 096 x 14 336 in
+// pieces 59 -> 66, 65 rows of 14 336 x 4 096 28.0 -> 30.6); 512 rows of 2 048 x 3 584 30.3 -> 15.9 us, 2 635 of 4 112 x 2 048 74 -> 45.  Of a short K, 65
+// rows and more: 2 814 products of K 128 to 448 0.67 of the time, 469 of K 64 (of which gated ones come here) 0.90, 48 of them all more than
+// 5 % slower, 26 % at most (1 000 rows of 8 192 x 256 12.7 -> 15.9).
 struct TileTime {
   int rows, cols, on_unit;  // on_unit: how many workgroups a compute unit holds (their LDS)
   float fixed, per_round, per_layer, per_fill, out_fill;
@@ -1227,19 +1230,24 @@ float product_us(int tile, int M, int N, int K, int splits) {
   return tile_us(tile, (long long)lq_ceil_div(M, tile_times[tile].rows) * lq_ceil_div(N, tile_times[tile].cols), K, splits);
 }
 
-int best_tile(int M, int N, int K, int splits) {
-  int best = 0;
-  for (int t = 1; t < TILES; ++t)
+// A gated epilogue costs tiles of 256 rows 4 to 10 us more than the estimate says, which a short K does not outweigh (2 635 rows of 3 072
+// columns of K 320: 256 x 192 19.7, 128 x 64 14.7).
+int best_tile(int M, int N, int K, int splits, bool gated = false) {
+  int best = gated && K < 512 ? T128x128 : T256x256;
+  for (int t = best + 1; t < TILES; ++t)
     if (product_us(t, M, N, K, splits) < product_us(best, M, N, K, splits)) best = t;
   return best;
 }
 
-// From 65 rows, or 17 of a weight too narrow for the kernels that stream a wide one: in pieces (from K 1 024 on up to 32 rows), and whole
+// From 65 rows (a K of 64 is sooner done by the kernels that any K has, but for a gated product), or 17 of a weight too narrow for the
+// kernels that stream a wide one: in pieces (from K 1 024 on up to 32 rows), and whole
 // from 33 rows.  Microseconds, the simple kernel / 64 x 64 tiles whole / in pieces with their addition, 1 536 columns: 17 rows of K 512
 // 4.0 / 4.6 / 4.2, of 2 048 7.1 / 9.4 / 5.7, of 4 096 11.1 / 15.8 / 7.3, of 14 336 34.9 / 57.5 / 14.0; 24 rows 4.3 / 4.7 / 4.2, 8.2 / 9.5 / 5.8, 13.0 / 16.0 /
 // 7.4, 40.7 / 58.3 / 14.1; 40 rows 5.4 / 4.8 / 4.4, 10.8 / 9.6 / 6.0, 17.8 / 16.1 / 7.6, 58.4 / 60.5 / 14.7.
-inline bool takes_rows(int M, int N, int K, bool pieces) {
-  return K % 64 == 0 && K >= 512 && (M > 64 || (N < 8 * lq_compute_units() && (M > 32 || (M > 16 && pieces && K >= 1024))));
+inline bool takes_rows(int M, int N, int K, bool pieces, bool gated) {
+  if (K % 64 != 0) return false;
+  if (M > 64) return K >= (gated ? 64 : 128);
+  return K >= 512 && N < 8 * lq_compute_units() && (M > 32 || (M > 16 && pieces && K >= 1024));
 }
 
 // Shares of K: as many as make the product (whose time has the writing of its pieces) and the reading of the further pieces, 4
@@ -1257,11 +1265,11 @@ int tiled_splits(int M, int N, int K) {
 template <int EPI, typename TO>
 int launch_rows(const void* x, const void* w, void* out, int M, int N, int K, int lda, int ldw, int ldc, int splits,
                 long long split_stride, hipStream_t stream, int packed, bool whole_rounds = true) {
-  const int tile = best_tile(M, N, K, splits);
+  const int tile = best_tile(M, N, K, splits, is_glu(EPI));
   // Whole rounds of 256-column tiles, and the columns that are left in a launch of their own with the tile that suits them, where
   // that wins by more than the estimate is off (2 048 x 28 672: three rounds and 256 tiles of 256 x 128 instead of 3.5 rounds).
   const int tm = lq_ceil_div(M, 256), n1 = lq_ceil_div(N, 256) * tm / lq_compute_units() * lq_compute_units() / tm * 256;
-  if (whole_rounds && splits == 1 && n1 > 0 && n1 < N) {
+  if (whole_rounds && splits == 1 && K >= 512 && n1 > 0 && n1 < N) {
     const float two = product_us(T256x256, M, n1, K, 1) + product_us(best_tile(M, N - n1, K, 1), M, N - n1, K, 1);
     if (two < 0.95f * product_us(tile, M, N, K, 1)) {
       const int col2 = is_glu(EPI) ? n1 / 2 : n1;  // where the second launch's columns start in out
@@ -1294,7 +1302,7 @@ int narrow_splits(int M, int N, int K) {
 
 int mfma_splits(int M, int N, int K) {
   if (mid_rows(M, N, K)) return mid_splits(N, K);
-  return takes_rows(M, N, K, true) ? tiled_splits(M, N, K) : v3_splits(M, N, K);
+  return takes_rows(M, N, K, true, false) ? tiled_splits(M, N, K) : v3_splits(M, N, K);
 }
 
 template <int EPI, typename TO>
@@ -1314,7 +1322,7 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
     }
   }
   if (mid_rows(M, N, K) && !(splits == 1 && few_whole(M, N))) return launch_mid<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
-  if (takes_rows(M, N, K, splits > 1)) return launch_rows<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
+  if (takes_rows(M, N, K, splits > 1, is_glu(EPI))) return launch_rows<EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
   if (splits > 1) {
     if (M <= 32) return launch_skinny_v3<2, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
     return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, splits, split_stride, stream, packed);
@@ -1335,7 +1343,7 @@ int dispatch(const void* x, const void* w, void* out, int M, int N, int K, int l
     if (wide) return launch_skinny_v3<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);
     return pick_skinny<4, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, stream);
   }
-  // a K that is no multiple of 64, or a short one: slabs of 32 k, then the register-staged kernels, which take any K
+  // a K that is no multiple of 64, or of 64 alone: slabs of 32 k, then the register-staged kernels, which take any K
   const long long t128 = (long long)lq_ceil_div(M, 128) * lq_ceil_div(N, 256);
   if (K % 32 == 0 && t128 >= lq_compute_units())
     return launch_pipelined<2, 2, 2, 4, 32, 3, EPI, TO>(x, w, out, M, N, K, lda, ldw, ldc, 1, 0, stream, packed);

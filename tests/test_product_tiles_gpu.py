@@ -108,3 +108,28 @@ def test_whole_products_of_13_to_32_rows(n, k):
                 kn.linear_swiglu(x[:rows], held, gated, activation="relu")
                 gate, up = got[:rows].view(rows, n // 16, 2, 8).unbind(2)
                 assert torch.equal(gated, (gate.clamp(min=0) * up).reshape(rows, n // 2).to(bf))
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (65, 136, 128), (100, 2064, 64), (130, 1000, 320), (300, 28672, 128), (513, 4112, 192), (2049, 6160, 384), (2635, 3072, 320),
+    (1025, 8208, 448), (257, 264, 64)])
+def test_products_of_a_short_k(m, n, k):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, bf = HipKernels(), torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, w = (torch.randn(r, k, generator=gen, device="cuda").to(bf) for r in (m, n))
+    around = torch.full((m + 2, n), 7.0, device="cuda")
+    kn.linear(x, w, around[1:-1])
+    assert within(around[1:-1], x, w) and bool((around[0] == 7).all()) and bool((around[-1] == 7).all())
+    out = torch.full((m, n), float("nan"), dtype=bf, device="cuda")
+    kn.linear(x, w, out)
+    assert within(out, x, w, 2.0 ** -8)
+    if n % 16 == 0:
+        got = torch.full((m, n // 2), float("nan"), dtype=bf, device="cuda")
+        kn.linear_swiglu(x, w, got, activation="relu")
+        gate, up = (x.double() @ w.double().T).view(m, n // 16, 2, 8).unbind(2)
+        off_gate, off_up = (k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).view(m, n // 16, 2, 8).unbind(2)
+        want = gate.clamp(min=0) * up
+        bound = off_gate * (up.abs() + off_up) + off_up * gate.clamp(min=0) + 2.0 ** -8 * want.abs()
+        assert bool(((got.view(m, n // 16, 8).double() - want).abs() <= bound).all())
