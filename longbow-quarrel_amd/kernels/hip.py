@@ -158,7 +158,6 @@ def _packed(w) -> int:
 
 class HipKernels:
     name = "hip-gfx950"
-    stores_maps = True  # `qkv_norm_store` takes heads in parts (`maps`)
 
     def __init__(self) -> None:
         self.lib = load_library()

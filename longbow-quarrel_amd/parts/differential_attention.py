@@ -110,17 +110,14 @@ class DifferentialAttention(Mixer):
         proj = ctx.ws.alloc((rows, (total + 3) // 4 * 4), torch.float32)[:, :total]
         project(kn, ctx, h, self.w_in, proj)
         q = ctx.ws.alloc((rows, self.q_width), ctx.dtype)
-        # every map of every head is a head of key_dim to the rotation; the values pass
-        if getattr(kn, "stores_maps", False):
-            # straight into the cache, one launch for two (8 + 2 heads of 2 x 128: 8 rows 5.2 -> 3.5 us, 4 096 rows 35.1 -> 31.3)
-            place = dict(row_pos=ctx.row_pos, row_seq=ctx.row_seq, seq_slot=ctx.seq_slot, block_table=cache.block_table,
-                         kcache=cache.k, vcache=cache.v, block_size=cache.block_size) if cache.write else {}
-            if self.rot_dims:
-                place.update(cos_sin=step_angles(ctx, self.freqs, self.freq_table), interleaved=self.rot_interleaved,
-                             magnitude=self.rot_magnitude)
-            kn.qkv_norm_store(proj, q, self.heads, self.kv_heads, M * self.key_dim, self.value_dim, 0.0, maps=M, **place)
-        else:
-            self._by_way_of_rows(kn, proj, q, ctx, cache)
+        # every map of every head is rotated by itself; keys and values go straight into the cache, one launch for two
+        # (8 + 2 heads of 2 x 128: 8 rows 5.2 -> 3.5 us, 4 096 rows 35.1 -> 31.3)
+        place = dict(row_pos=ctx.row_pos, row_seq=ctx.row_seq, seq_slot=ctx.seq_slot, block_table=cache.block_table,
+                     kcache=cache.k, vcache=cache.v, block_size=cache.block_size) if cache.write else {}
+        if self.rot_dims:
+            place.update(cos_sin=step_angles(ctx, self.freqs, self.freq_table), interleaved=self.rot_interleaved,
+                         magnitude=self.rot_magnitude)
+        kn.qkv_norm_store(proj, q, self.heads, self.kv_heads, M * self.key_dim, self.value_dim, 0.0, maps=M, **place)
         both = ctx.ws.alloc((rows, M * self.o_width), torch.float32)
         kn.sink_attention(q, both, M * self.heads, M * self.kv_heads, self.key_dim, self.value_dim, ctx.row_pos,
                           ctx.row_seq, ctx.seq_slot, cache.block_table, cache.k, cache.v, cache.block_size, self.scale,
@@ -133,14 +130,3 @@ class DifferentialAttention(Mixer):
             out = ctx.ws.alloc((rows, self.width), torch.float32)
         project(kn, ctx, att, self.w_o, out)
         return out
-
-    def _by_way_of_rows(self, kn, proj, q, ctx: StepContext, cache: LayerCache) -> None:
-        """The same on kernels whose `qkv_norm_store` takes whole heads only: rows of keys and values, then the cache."""
-        rows, M = proj.shape[0], self.MAPS
-        k = ctx.ws.alloc((rows, self.k_width), ctx.dtype)
-        v = ctx.ws.alloc((rows, self.v_width), ctx.dtype)
-        kn.rotary_qkv(proj, q, k, v, M * self.heads, M * self.kv_heads, self.key_dim, self.value_dim, self.rot_dims,
-                      self.rot_interleaved, self.freqs, self.rot_magnitude, None, ctx.row_pos, value_width=self.v_width)
-        if cache.write:
-            kn.kv_store(k, v, self.kv_heads, M * self.key_dim, self.value_dim, ctx.row_pos, ctx.row_seq, ctx.seq_slot,
-                        cache.block_table, cache.k, cache.v, cache.block_size)

@@ -356,8 +356,8 @@ class CpuKernels:
     def qkv_norm_store(self, src, q_out, heads, kv_heads, key_dim, value_dim, eps, bias=None, q_weight=None, k_weight=None,
                        norm_qk=None, norm_v=False, v_from_k=False, row_pos=None, row_seq=None, seq_slot=None,
                        block_table=None, kcache=None, vcache=None, block_size=0, cos_sin=None, interleaved=False,
-                       magnitude=1.0):
-        rows, qw, kw = src.shape[0], heads * key_dim, kv_heads * key_dim
+                       magnitude=1.0, maps=1):
+        rows, qw, kw, part = src.shape[0], heads * key_dim, kv_heads * key_dim, key_dim // maps
         t = src.float() if bias is None else src.float() + bias
 
         def unit(v, weight, per):
@@ -368,10 +368,10 @@ class CpuKernels:
         q, k = t[:, :qw], t[:, qw : qw + kw]
         v = k if v_from_k else t[:, qw + kw :]
         if cos_sin is not None:
-            q, k = (self._turned(x, key_dim, cos_sin, interleaved, magnitude) for x in (q, k))
+            q, k = (self._turned(x, part, cos_sin, interleaved, magnitude) for x in (q, k))
         if norm_qk:
-            q = unit(q, q_weight, qw if norm_qk == "row" else key_dim)
-            k = unit(k, k_weight, kw if norm_qk == "row" else key_dim)
+            q = unit(q, q_weight, qw if norm_qk == "row" else part)
+            k = unit(k, k_weight, kw if norm_qk == "row" else part)
         if norm_v:
             v = unit(v, None, value_dim)
         q_out.copy_(q.to(q_out.dtype))
