@@ -1203,10 +1203,10 @@ int launch_mid(const void* x, const void* w, void* out, int M, int N, int K, int
 // 4 406 products (15 row counts of 65 to 4 096, 1 024 to 28 672 columns, K 512 to 14 336), each on all six tiles: times of 32-bit results
 // lie 6 to 8 % above the estimate and scatter by 7 to 9 %, gated ones 10 to 22 % above, and the tile that is named takes 0.6 % more than the best of
 // the six on average, 28 % at most.  Against one rule for each range of rows (256 x 256, 256 x 192, 128 x 128 and one covering tile up to 256 rows)
-// over 6 283 products of 17 rows and more: 0.78 of the time on average, 54 of them more than 5 % slower, 16 % at most (300 rows of 4 096 x 14 336 in
-// pieces 59 -> 66, 65 rows of 14 336 x 4 096 28.0 -> 30.6); 512 rows of 2 048 x 3 584 30.3 -> 15.9 us, 2 635 of 4 112 x 2 048 74 -> 45.  Of a short K, 65
-// rows and more: 2 814 products of K 128 to 448 0.67 of the time, 469 of K 64 (of which gated ones come here) 0.90, 48 of them all more than
-// 5 % slower, 26 % at most (1 000 rows of 8 192 x 256 12.7 -> 15.9).
+// over 6 283 products of 17 rows and more: 0.78 of the time on average, 67 of them more than 5 % slower, 16 % at most (2 048 rows of 1 024 x 14 336
+// in pieces 69 -> 80, 300 of 4 096 x 14 336 59 -> 65, 65 of 14 336 x 14 336 92 -> 102); 512 rows of 2 048 x 3 584 30.3 -> 15.9 us, 2 635 of 4 112 x 2 048 74 ->
+// 45.  Of a short K, 65 rows and more: 2 814 products of K 128 to 448 0.67 of the time, 469 of K 64 (of which gated ones come here) 0.90, 40 of them
+// all more than 5 % slower, 19 % at most (2 048 rows of 4 096 x 256 13.4 -> 15.8).
 struct TileTime {
   int rows, cols, on_unit;  // on_unit: how many workgroups a compute unit holds (their LDS)
   float fixed, per_round, per_layer, per_fill, out_fill;
