@@ -38,6 +38,25 @@ def test_gated_with_biases(rows, n, k, tail):
         assert bool((wide[:, 0] == 7).all()) and bool((wide[:, inner + tail + 1 :] == 7).all()) and bool((wide[rows] == 7).all())
 
 
+@pytest.mark.parametrize("rows,n,k,tail", [
+    (8, 2064, 1024, 128), (40, 14336, 2048, 8), (65, 2064, 512, 128), (300, 8208, 512, 8), (2047, 8208, 512, 128), (2048, 14336, 2048, 128)])
+def test_gated_with_biases_has_the_activation_kernels_bits(rows, n, k, tail):
+    """Sizes whose sums are made in one order either way: the epilogue's functions are then as exact as the activation kernel's."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, inner = HipKernels(), n // 2
+    x, w, bias = operands(rows, n, k)
+    product = torch.empty(rows, n, device="cuda")
+    kn.linear(x, w, product)
+    both = torch.cat([part.reshape(rows, inner) for part in (product + bias).view(rows, n // 16, 2, 8).unbind(2)], dim=1).contiguous()
+    want = torch.empty(rows, inner + tail, dtype=torch.bfloat16, device="cuda")
+    kn.glu(both, want, "silu", tail=tail)
+    for held in (w, kn.pack_weight(w)):
+        out = torch.empty_like(want)
+        kn.linear_unit(x, held, out, "silu", bias=bias, tail=tail)
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("activation", ["silu", "relu", "gelu_tanh", "gelu", "relu2"])
 @pytest.mark.parametrize("rows,n,k", [(1, 2048, 512), (7, 2056, 2048), (16, 10752, 576)])
 def test_plain_activations_of_few_rows(activation, rows, n, k):
