@@ -213,6 +213,8 @@ __global__ __launch_bounds__(THREADS) void moe_few_first_kernel(const bf16_t* __
 // 64 k (2 KiB), filled by two transfers of whole lines that are marked as a stream, with the slot's x beside them; a slot is waited for, read,
 // and asked for anew, so that three are always on their way.  (Fragments loaded into registers, 64 bytes from each of 16 rows,
 // three chunks ahead: 2 048 x 28 672 at 8 rows that choose 7 of 8 experts 23.6 us, this way 17.4, 6 TB/s.)
+// At most 8 rows take chunks of 128 k and keep the sums of a chunk's halves of 64 k apart to the end (twice as many sums, half as long);
+// more rows, and experts that are not in 128s, take chunks of 64.
 // Position of 16-byte chunk c of a slot's row r: c ^ r / 2.  Behind a wavefront's last chunk transfers go on, out of the buffer's range,
 // until all slots are done: a wait then always counts the same number of them; such a slot takes part in no sum.
 constexpr int SLOTS = 4, SLOT = 2048, NOWHERE = (int)0x80000000u;  // (NOWHERE: an offset beyond every buffer)
@@ -222,6 +224,8 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
                                                                  int ldw, int packed, float* __restrict__ out, int ldo, long long piece,
                                                                  int N, Experts ex, const bf16_t* __restrict__ h, int ldh,
                                                                  const float* __restrict__ passed, int n_passed) {
+  constexpr int SUMS = CHUNK / 64;
+  static_assert(SLOTS % SUMS == 0, "a slot's part of its chunk is the slot's number modulo the parts");
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];  // [KW][SLOTS][SLOT]; a wavefront's sums at its part's start
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
   const int n0 = blockIdx.x * 16, rows = min(16, N - n0);
@@ -285,7 +289,9 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   int frag[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) frag[i] = c16 * 128 + (((4 * i + g) ^ (c16 >> 1)) & 7) * 16;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[SUMS];
+#pragma unroll
+  for (int j = 0; j < SUMS; ++j) acc[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
   auto use = [&](int d) {  // (its transfers have landed)
     __builtin_amdgcn_sched_barrier(0);
     u32x4 wv[2];
@@ -295,7 +301,7 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
     __builtin_amdgcn_sched_barrier(0);
     if (there[d])
 #pragma unroll
-      for (int i = 0; i < 2; ++i) acc = mfma(xv[d][i], wv[i], acc);
+      for (int i = 0; i < 2; ++i) acc[d % SUMS] = mfma(xv[d][i], wv[i], acc[d % SUMS]);
   };
   while (there[SLOTS - 1]) {  // (slots are filled in their order: the last one asked for stands for all)
 #pragma unroll
@@ -310,8 +316,10 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   for (int d = 0; d < SLOTS; ++d) use(d);
   float* red = (float*)mine;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) red[e * 64 + lane] = acc[e];
-  // four wavefronts finish the entries of 16 columns: wavefront e those of acc[e]
+  for (int j = 0; j < SUMS; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[j * 256 + e * 64 + lane] = acc[j][e];
+  // four wavefronts finish the entries of 16 columns: wavefront e those of acc[..][e]
   const int r = 4 * g + wave, n = n0 + c16;
   const bool ends = wave < 4 && r < ex.rows && n < N;
   float add = 0.f;
@@ -324,7 +332,9 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   if (!ends) return;
   float s = 0.f;
 #pragma unroll
-  for (int w = 0; w < KW; ++w) s += ((const float*)(ring + w * (SLOTS * SLOT)))[wave * 64 + lane];
+  for (int w = 0; w < KW; ++w)
+#pragma unroll
+    for (int j = 0; j < SUMS; ++j) s += ((const float*)(ring + w * (SLOTS * SLOT)))[j * 256 + wave * 64 + lane];
   out[blockIdx.y * piece + (long long)r * ldo + n] = s + add;
 }
 
@@ -410,7 +420,7 @@ extern "C" int lq_moe_few_second(const void* act, int lda, const void* w, int ld
   LQ_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)act | (uintptr_t)w) % 16 == 0 && (!w_packed || (ldw % 64 == 0 && width % 8 == 0)),
              "moe_few: operands are not aligned");
   LQ_REQUIRE(passed == nullptr || (h != nullptr && ldh >= width && n_passed >= 1), "moe_few: identity experts come with the rows");
-  const bool long_chunks = ff % 128 == 0 && shared % 128 == 0;
+  const bool long_chunks = rows <= 8 && ff % 128 == 0 && shared % 128 == 0;
   LQ_REQUIRE((long long)ldw * 32 < (1ll << 31) && (long long)rows * lda * 2 < (1ll << 31), "moe_few: rows too far apart for 32-bit offsets");
   const auto kernel = long_chunks ? moe_few_second_kernel<128> : moe_few_second_kernel<64>;
   constexpr int lds = KW * SLOTS * SLOT;

@@ -96,6 +96,31 @@ def test_chosen_experts_alone(rows, E, top, ff, shared, width, activation, more,
         assert torch.equal(again[:, 0], out[:, 0])
 
 
+@pytest.mark.parametrize("rows,ff,places", [
+    (8, 2176, (0, 64, 2048)),     # a wavefront's chunks 0 and 16 of 128 k: the sums of their halves are apart
+    (1, 2176, (100, 40, 2148)),
+    (9, 2048, (0, 64, 1024)),     # chunks of 64 k: 0 and 16 are one wavefront's, 1 another's
+    (8, 1088, (3, 67, 1027))])
+@pytest.mark.parametrize("pack", [True, False])
+def test_sums_of_halves_and_chunks_stay_apart(rows, ff, places, pack):
+    """2^24 + 1 - 2^24 at three places of the second product's k: one where the two large ones are of one sum and the one of another,
+    nothing where a sum takes the one between them."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, width = HipKernels(), 4096
+    kn.pack_weights = pack
+    assert kn.moe_few_pieces(width) == 1 and kn.moe_few_supported(torch.bfloat16, rows, 1, ff, 0, width)
+    w_in = torch.zeros(ff, width, dtype=torch.bfloat16)
+    w_out = torch.zeros(width, ff, dtype=torch.bfloat16)
+    for k, v in zip(places, (2.0 ** 24, 1.0, -2.0 ** 24)):
+        w_in[k, 0], w_out[:, k] = 1.0, v  # (relu(1)^2 is 1)
+    x = torch.ones(rows, width, dtype=torch.bfloat16)
+    act, out = torch.empty(rows, ff, dtype=torch.bfloat16, device="cuda"), torch.empty(rows, width, device="cuda")
+    kn.moe_few(x.cuda(), kn.pack_weight(w_in.cuda()), kn.pack_weight(w_out.cuda()), torch.ones(rows, 1, device="cuda"), act, out,
+               ff, 0, "relu2")
+    assert bool((out == 1.0).all())
+
+
 def test_sizes_that_are_not_taken():
     from longbow_quarrel_amd.kernels.hip import HipKernels
 
