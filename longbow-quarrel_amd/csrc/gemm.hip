@@ -33,9 +33,9 @@ extern "C" int lq_linear_narrow_splits(int in_dtype, int M, int N, int K, int fo
   return lq_gemm_narrow_splits(M, N, K);
 }
 
-// Whether that caller is better off without pieces: at most 8 rows, whose kernel takes K in pairs of chunks, up to four pieces.
-// Microseconds in pieces with the launch that adds them up, and whole: 128 x 2 048 in two, 1 row 4.4 and 2.9, 8 rows 5.2 and 3.8; 8
-// rows of 64 x 4 096 in four 5.4 and 5.4; 288 x 8 192 in eight, 1 row 5.9 and 6.2, 8 rows 6.8 and 9.0.
+// Whether that caller is better off without pieces: at most 8 rows, whose kernels share K over the waves of a block, up to four pieces.
+// Microseconds in pieces with the launch that adds them up, and whole: 128 x 2 048 in two, 1 row 4.6 and 3.1, 8 rows 5.5 and 4.0; 8
+// rows in four of 64 x 4 096 5.7 and 5.4, of 288 x 4 096 6.3 and 5.5; 288 x 8 192 in eight, 1 row 6.5 and 6.9, 8 rows 7.7 and 8.9.
 extern "C" int lq_linear_whole(int in_dtype, int M, int N, int K, int force_generic) {
   return !force_generic && in_dtype == LQ_BF16 && K % 8 == 0 && lq_gemm_mfma_splits(M, N, K) <= 1 && lq_gemm_few_and_narrow(M, N, K) &&
          lq_gemm_narrow_splits(M, N, K) <= 4;

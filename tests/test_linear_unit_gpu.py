@@ -39,7 +39,7 @@ def test_gated_with_biases(rows, n, k, tail):
 
 
 @pytest.mark.parametrize("rows,n,k,tail", [
-    (8, 2064, 1024, 128), (40, 14336, 2048, 8), (65, 2064, 512, 128), (300, 8208, 512, 8), (2047, 8208, 512, 128), (2048, 14336, 2048, 128)])
+    (4, 2048, 1024, 8), (2, 2048, 8192, 128), (8, 2048, 4096, 8), (8, 2064, 1024, 128), (40, 14336, 2048, 8), (65, 2064, 512, 128), (300, 8208, 512, 8), (2047, 8208, 512, 128), (2048, 14336, 2048, 128)])
 def test_gated_with_biases_has_the_activation_kernels_bits(rows, n, k, tail):
     """Sizes whose sums are made in one order either way: the epilogue's functions are then as exact as the activation kernel's."""
     from longbow_quarrel_amd.kernels.hip import HipKernels

@@ -49,6 +49,45 @@ def test_into_the_stream(rows, k):
     assert ((sq.double().sum(1) - (got.double() ** 2).sum(1)).abs() <= 2048 * 2.0 ** -24 * (got.double() ** 2).sum(1)).all()
 
 
+@pytest.mark.parametrize("n,k", [(320, 4096), (1000, 4096), (1536, 5376), (2040, 2176), (2040, 2048), (2040, 8320)])
+@pytest.mark.parametrize("rows", [1, 3, 8])
+def test_streamed_products_sum_in_the_same_order(rows, n, k):
+    """The same columns, of a weight whose columns are not in eights, which goes in pairs of chunks, and of one that may be streamed."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    x, w = (torch.randn(r, k, generator=gen, device="cuda").bfloat16() for r in (rows, n + 1))
+    want, got = torch.empty(rows, n + 1, device="cuda"), torch.empty(rows, n, device="cuda")
+    kn.linear(x, w, want)
+    kn.linear(x, w[:n], got)
+    assert torch.equal(got, want[:, :n])
+
+
+@pytest.mark.parametrize("rows,k", [(4, 512), (4, 8192), (3, 14464), (8, 1920), (8, 4096)])
+def test_streamed_products_of_2048_columns_sum_in_the_same_order(rows, k):
+    """Every way out of a product of 8 columns a compute unit."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, n = HipKernels(), 2048
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    x, w = (torch.randn(r, k, generator=gen, device="cuda").bfloat16() for r in (rows, n))
+    old = torch.randn(rows, n, generator=gen, device="cuda")
+    want = torch.empty(rows, n, device="cuda")
+    kn.linear(x, w[: n - 1], want[:, : n - 1])
+    kn.linear(x, w[1:], want[:, 1:])
+    acted = torch.empty(rows, n, dtype=torch.bfloat16, device="cuda")
+    kn.activation(want, acted, "relu2")
+    for held in (w, kn.pack_weight(w)):
+        wide, narrow, unit = torch.empty_like(want), torch.empty_like(acted), torch.empty_like(acted)
+        kn.linear(x, held, wide)
+        kn.linear(x, held, narrow)
+        kn.linear_unit(x, held, unit, "relu2")
+        new, sq = old.clone(), torch.empty(rows, kn.linear_fused_parts(torch.bfloat16, rows, n, k), device="cuda")
+        kn.linear_residual(x, held, new, sq)
+        assert torch.equal(wide, want) and torch.equal(narrow, want.bfloat16()) and torch.equal(unit, acted) and torch.equal(new, old + want)
+
+
 @pytest.mark.parametrize("rows,n,k,whole", [(1, 128, 2048, True), (8, 64, 4096, True), (8, 288, 8192, False), (9, 128, 2048, False),
                                             (3, 160, 2112, False), (2, 4096, 4096, False)])
 def test_whole_or_in_pieces_added_up(rows, n, k, whole):
