@@ -123,7 +123,6 @@ extern "C" int lq_linear_unit(const void* x, const void* w, void* out, int M, in
   LQ_REQUIRE(lda >= K && ldw >= K && ldc >= (bias != nullptr ? N / 2 + tail : N), "linear_unit: a row stride is smaller than its row");
   LQ_REQUIRE(lq_gemm_mfma_accepts(x, w, LQ_BF16, K, lda, ldw), "linear_unit: operands are not aligned");
   LQ_REQUIRE(!w_packed || ldw == K, "linear_unit: a packed weight is whole");
-  LQ_REQUIRE((long long)ldw * 256 < (1ll << 31) && (long long)lda * 512 < (1ll << 31), "linear_unit: rows too far apart for 32-bit offsets");
   return lq_gemm_unit(x, w, out, M, N, K, lda, ldw, ldc, bias, tail, act, w_packed, stream);
 }
 

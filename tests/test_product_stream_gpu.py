@@ -69,3 +69,37 @@ def test_an_infinity_or_nan_stays_in_its_row_or_column(rows, n, k):
         kn.linear(x, held, out)
         assert not bool(out[0].isfinite().any()) and bool(out[:, n - 1].isnan().all())
         assert torch.equal(out[1:, : n - 1], want[1:, : n - 1])
+
+
+@pytest.mark.parametrize("rows,n,k", [(12, 4096, 1024), (3, 2048, 4096), (16, 2048, 576)])
+def test_rows_of_x_beyond_32_bit_offsets(rows, n, k):
+    """Rows 2^28 bytes apart and more: the bits of the same rows side by side, dense and packed, every way out."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, bf = HipKernels(), torch.bfloat16
+    apart = 2 ** 31 // 2 // (rows - 1) // 8 * 8
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    near, w = (torch.randn(r, k, generator=gen, device="cuda").to(bf) for r in (rows, n))
+    far = torch.empty((rows - 1) * apart + k, dtype=bf, device="cuda").as_strided((rows, k), (apart, 1))
+    far.copy_(near)
+    assert ((rows - 1) * apart + k) * 2 >= 2 ** 31
+    stream = torch.randn(rows, n, generator=gen, device="cuda")
+    gain, sums = torch.linspace(-1, 1, n, device="cuda"), torch.rand(rows, 300, generator=gen, device="cuda")
+    parts = kn.linear_fused_parts(bf, rows, n, k)
+    for held in (w, kn.pack_weight(w)):
+        got = []
+        for x in (near, far):
+            wide, gated, acted, half = (torch.empty(rows, c, dtype=d, device="cuda") for c, d in
+                                        ((n, torch.float32), (n // 2, bf), (n, bf), (n, bf)))
+            kn.linear(x, held, wide)
+            kn.linear_swiglu(x, held, gated)
+            kn.linear_unit(x, held, acted, "relu2")
+            biased = torch.empty(rows, n // 2 + 8, dtype=bf, device="cuda")
+            kn.linear_unit(x, held, biased, "silu", bias=gain, tail=8)
+            got.append([wide, gated, acted, biased])
+            if parts:
+                new, sq, scaled = stream.clone(), torch.empty(rows, parts, device="cuda"), torch.empty(rows, n, dtype=bf, device="cuda")
+                kn.linear_residual(x, held, new, sq, gain=gain, scaled=scaled)
+                kn.linear_scaled(x, sums, 1e-5, held, half)
+                got[-1] += [new, sq, scaled, half]
+        assert all(torch.equal(a, b) for a, b in zip(*got))
