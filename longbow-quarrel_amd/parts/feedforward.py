@@ -121,7 +121,8 @@ class GatedLinearUnit(FeedForward):
         kn = env.kernels
         self.fused = self.activation in ("gelu_tanh", "relu") and not self.bias and gate.dtype == env.dtype == torch.bfloat16 and \
             self.inner % 8 == 0 and getattr(kn, "linear_swiglu_supported", lambda *a: False)(gate.dtype, 2 * self.inner, self.width)
-        self.unit = self.activation == "silu" and self.bias and gate.dtype == env.dtype == torch.bfloat16 and \
+        # (a second matrix in 32 bits takes its activations so, and a product's epilogue leaves 16)
+        self.unit = self.activation == "silu" and self.bias and gate.dtype == env.dtype == tensors[self.names["down"]].dtype == torch.bfloat16 and \
             getattr(kn, "linear_unit_supported", lambda *a: False)(gate.dtype, 1, 2 * self.inner, self.width, True)
         if self.fused or self.unit:
             self.w_gate_up = product_weight(env, kn.interleave_gate_up(gate, up))

@@ -41,3 +41,37 @@ def test_against_the_formula(width, inner, rows):
     terms = act.abs() @ t["m.down"].abs().T + t["m.down.b"].abs()
     largest = act.abs().amax(1, keepdim=True) * t["m.down"].abs().amax(1)
     assert ((got - want).abs() <= (inner + 128) * 2.0 ** -24 * terms + 4 * 2.0 ** -8 * largest).all()
+
+
+def bound_part(kn, width, inner, down=torch.bfloat16):
+    from longbow_quarrel_amd.parts import BuildEnv
+    from longbow_quarrel_amd.weights import random_tensors
+
+    dev = torch.device("cuda:0")
+    part = GatedLinearUnit(width, inner, "m", bias=True)
+    tensors = random_tensors(part.tensor_specs(), 3, torch.bfloat16, 0.1, device=dev)
+    tensors = {s.name: tensors[s.name].float() if s.kind == "vector32" else tensors[s.name] for s in part.tensor_specs()}
+    tensors["m.down"] = tensors["m.down"].to(down)
+    part.bind(dict(tensors), BuildEnv(torch.bfloat16, dev, kn))
+    ws = SimpleNamespace(alloc=lambda shape, dtype, **_: torch.full(tuple(shape), float("nan"), dtype=dtype, device=dev))
+    return part, {k: v.double() for k, v in tensors.items()}, SimpleNamespace(kernels=kn, ws=ws, dtype=torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 8, 17, 100])
+def test_a_second_matrix_in_32_bits(rows):
+    """Its activations stay in 32 bits, so no epilogue rounds them."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    width, inner = 512, 1024
+    part, t, ctx = bound_part(HipKernels(), width, inner, torch.float32)
+    h = torch.randn(rows, width, generator=torch.Generator().manual_seed(inner)).bfloat16().cuda()
+    got = part.forward(h, ctx).double()
+    (g, off_g), (u, off_u) = ((h.double() @ t[f"m.{n}"].T + t[f"m.{n}.b"],
+                               (h.double().abs() @ t[f"m.{n}"].abs().T + t[f"m.{n}.b"].abs()) * (width + 1) * 2.0 ** -24) for n in ("gate", "up"))
+    silu = g * torch.sigmoid(g)
+    # an activation is off by what its sums are (silu' is below 1.1) and a few roundings; then come `inner` terms
+    off = 1.1 * off_g * (u.abs() + off_u) + silu.abs() * off_u + 8 * 2.0 ** -24 * (silu * u).abs()
+    down, bias = t["m.down"].T, t["m.down.b"]
+    terms = (silu * u).abs() @ down.abs() + bias.abs()
+    assert ((got - (silu * u) @ down - bias).abs() <= 1.01 * (off @ down.abs() + (inner + 128) * 2.0 ** -24 * terms)).all()
