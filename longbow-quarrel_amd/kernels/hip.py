@@ -521,6 +521,12 @@ class HipKernels:
         return bool(self.lib.lq_linear_unit_supported(c_int(_DTYPE_CODE[dtype]), c_int(rows), c_int(rows_out), c_int(k),
                                                       c_int(1 if biased else 0), c_int(1 if self.force_generic else 0)))
 
+    def rows_aligned(self, x: torch.Tensor) -> bool:
+        """Whether x's rows begin where the matrix-core kernels read them, at multiples of 16 bytes; `linear` alone takes others,
+        by another kernel, with a dense weight."""
+        _, _, ld = self._mat(x, "rows_aligned")
+        return x.data_ptr() % 16 == 0 and ld * x.element_size() % 16 == 0
+
     def linear_unit(self, x: torch.Tensor, w, out: torch.Tensor, activation: str, bias: Optional[torch.Tensor] = None,
                     tail: int = 0) -> None:
         """The first product of a feed-forward with its activation, bfloat16 in and out.  With `bias` (float32, an entry a row of w):

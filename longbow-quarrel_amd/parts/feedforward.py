@@ -149,6 +149,10 @@ class GatedLinearUnit(FeedForward):
             project(kn, ctx, act, self.w_down, out)
             return out
         if self.unit:
+            if not getattr(self.w_gate_up, "packed", False) and not kn.rows_aligned(h):
+                near = ctx.ws.alloc(h.shape, h.dtype)  # (a dense weight's product takes rows at any address)
+                near.copy_(h)
+                h = near
             act = ctx.ws.alloc((rows, self.inner + self.tail), self.w_down.dtype)
             kn.linear_unit(h, self.w_gate_up, act, self.activation, bias=self.b_gate_up, tail=self.tail)
         else:
@@ -194,7 +198,8 @@ class PlainFeedForward(FeedForward):
     def forward(self, h, ctx: StepContext, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         kn, rows = ctx.kernels, h.shape[0]
         if ctx.dtype == self.w_up.dtype == torch.bfloat16 and \
-                getattr(kn, "linear_unit_supported", lambda *a: False)(self.w_up.dtype, rows, self.inner, self.width, False):
+                getattr(kn, "linear_unit_supported", lambda *a: False)(self.w_up.dtype, rows, self.inner, self.width, False) and \
+                kn.rows_aligned(h):
             act = ctx.ws.alloc((rows, self.inner), ctx.dtype)
             kn.linear_unit(h, self.w_up, act, self.activation)
         else:

@@ -75,3 +75,28 @@ def test_a_second_matrix_in_32_bits(rows):
     down, bias = t["m.down"].T, t["m.down.b"]
     terms = (silu * u).abs() @ down.abs() + bias.abs()
     assert ((got - (silu * u) @ down - bias).abs() <= 1.01 * (off @ down.abs() + (inner + 128) * 2.0 ** -24 * terms)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 5, 16, 40])
+@pytest.mark.parametrize("row,first", [(513, 1), (512, 4), (516, 0)])
+def test_rows_at_any_address_with_dense_weights(rows, row, first):
+    """Rows that begin at no multiple of 16 bytes: as the same rows side by side, but for the order of sums."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+    from longbow_quarrel_amd.parts import BuildEnv
+    from longbow_quarrel_amd.parts.feedforward import PlainFeedForward
+
+    kn, width, inner = HipKernels(), 512, 2048
+    kn.pack_weights = False
+    gen = torch.Generator().manual_seed(rows + row)
+    apart = torch.randn(rows * row + 8, generator=gen).bfloat16().cuda()[first:].as_strided((rows, width), (row, 1))
+    gated, _, ctx = bound_part(kn, width, inner)
+    plain = PlainFeedForward(width, inner, "m", "relu2")
+    plain.bind({f"m.{n}": (torch.randn(*size, generator=gen) * 0.1).bfloat16().cuda() for n, size in
+                (("up", (inner, width)), ("down", (width, inner)))}, BuildEnv(torch.bfloat16, torch.device("cuda:0"), kn))
+    assert gated.unit
+    for part in (gated, plain):
+        want, got = part.forward(apart.clone(memory_format=torch.contiguous_format), ctx).double(), part.forward(apart, ctx).double()
+        # an activation whose sum lies next to the middle between two bfloat16 numbers may round to the other one, 2^-8 of it: one in
+        # hundreds, so that a result of some thousand terms with signs is off by far less than its row's norm times 2^-8
+        assert ((got - want).norm(dim=1) <= 2.0 ** -8 * want.norm(dim=1)).all()
