@@ -17,7 +17,7 @@
 // number, and a chunk of an expert that only other rows chose adds zeros.
 //
 //   v_mfma_f32_16x16x32_bf16: lane (c = l % 16, g = l / 16) gives A[c][8 g .. + 8] and B[c][the same k] and receives
-//   D[4 g + e][c].  A is x (rows beyond the last repeat it), B 16 rows of the weight.
+//   D[4 g + e][c].  A is x (rows beyond the last are whatever lies there, and nothing is kept of them), B 16 rows of the weight.
 #include "device_math.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -219,7 +219,10 @@ __global__ __launch_bounds__(THREADS) void moe_few_first_kernel(const bf16_t* __
 // until all slots are done: a wait then always counts the same number of them; such a slot takes part in no sum.
 constexpr int SLOTS = 4, SLOT = 2048, NOWHERE = (int)0x80000000u;  // (NOWHERE: an offset beyond every buffer)
 
-template <int CHUNK>
+//
+// FAR: rows of the activations or of W beyond the reach of 32-bit offsets.  Everything goes by pointers then, rows that there are not
+// by those of the last one, and a slot is waited for with all that was asked for: nothing is counted.
+template <int CHUNK, bool FAR>
 __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* __restrict__ act, int lda, const bf16_t* __restrict__ W,
                                                                  int ldw, int packed, float* __restrict__ out, int ldo, long long piece,
                                                                  int N, Experts ex, const bf16_t* __restrict__ h, int ldh,
@@ -229,15 +232,21 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];  // [KW][SLOTS][SLOT]; a wavefront's sums at its part's start
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
   const int n0 = blockIdx.x * 16, rows = min(16, N - n0);
-  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (long long)n0 * ldw), 0, rows * ldw * 2, 0x00020000);
-  const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)act, 0, ((ex.rows - 1) * lda + ex.n * ex.ff + ex.shared) * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t w_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(W + (long long)n0 * ldw), 0, FAR ? 0 : rows * ldw * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t x_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void*)act, 0, FAR ? 0 : ((ex.rows - 1) * lda + ex.n * ex.ff + ex.shared) * 2, 0x00020000);
   int w_off[2];  // this lane in a transfer: row lane / 8, the chunk that lies at position lane % 8
+  const bf16_t* w_ptr[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const int row = 8 * q + (lane >> 3), chunk = (lane & 7) ^ (row >> 1);
     w_off[q] = row >= rows ? NOWHERE : (packed ? q * 16 * ldw + (lane >> 3) * 128 : row * ldw * 2) + chunk * 16;
+    const int n = n0 + min(row, rows - 1);
+    w_ptr[q] = W + (packed ? (long long)(n >> 3) * 8 * ldw + (n & 7) * 64 : (long long)n * ldw) + chunk * 8;
   }
   const int x_off = c16 < ex.rows ? c16 * lda * 2 + g * 16 : NOWHERE;
+  const bf16_t* x_ptr = act + (long long)min(c16, ex.rows - 1) * lda + g * 8;
   unsigned long long bits = chosen_experts(ex);
 
   // this wavefront's chunks of the expert that it is at: `left` more of them, the next at k
@@ -276,6 +285,16 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   auto ask = [&](int slot) {
     const int at = next();
     there[slot] = at >= 0;
+    if constexpr (FAR) {
+      const long long from = max(at, 0);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(w_ptr[q] + from * (packed ? 8 : 1)),
+                                         (__attribute__((address_space(3))) void*)(mine + slot * SLOT + q * 1024), 16, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) xv[slot][i] = *(const u32x4*)(x_ptr + from + 32 * i);
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < 2; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (__attribute__((address_space(3))) void*)(mine + slot * SLOT + q * 1024), 16,
@@ -306,7 +325,7 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   while (there[SLOTS - 1]) {  // (slots are filled in their order: the last one asked for stands for all)
 #pragma unroll
     for (int d = 0; d < SLOTS; ++d) {
-      __builtin_amdgcn_s_waitcnt(0x0F70 | 12);  // vmcnt: four a slot, three slots behind
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (FAR ? 0 : 12));  // vmcnt: four a slot, three slots behind
       use(d);
       ask(d);
     }
@@ -366,7 +385,7 @@ int launch_first(const bf16_t* x, int ldx, const bf16_t* w, int ldw, bf16_t* act
 extern "C" int lq_moe_few_supported(int dtype, int rows, int experts, int ff, int shared, int width) {
   return dtype == LQ_BF16 && rows >= 1 && rows <= ROWS && experts >= 1 && experts <= EXPERTS && ff >= 64 && ff % 64 == 0 &&
          shared >= 0 && shared % 64 == 0 && width >= 512 && width % 64 == 0 && width <= KW * 8 * 32 &&
-         (long long)experts * ff + shared < (1ll << 26);  // (16 rows of the second matrix in 32-bit offsets)
+         2ll * experts * ff + 2ll * shared <= 0x7fffffff;
 }
 
 // act[row][e ff + c] (bfloat16) = the activation of expert e's column c for the experts that some row chose: the unit's value for
@@ -421,17 +440,18 @@ extern "C" int lq_moe_few_second(const void* act, int lda, const void* w, int ld
              "moe_few: operands are not aligned");
   LQ_REQUIRE(passed == nullptr || (h != nullptr && ldh >= width && n_passed >= 1), "moe_few: identity experts come with the rows");
   const bool long_chunks = rows <= 8 && ff % 128 == 0 && shared % 128 == 0;
-  LQ_REQUIRE((long long)ldw * 32 < (1ll << 31) && (long long)rows * lda * 2 < (1ll << 31), "moe_few: rows too far apart for 32-bit offsets");
-  const auto kernel = long_chunks ? moe_few_second_kernel<128> : moe_few_second_kernel<64>;
+  const bool far = (long long)ldw * 32 >= (1ll << 31) || (long long)rows * lda * 2 >= (1ll << 31);
+  const auto kernel = far ? (long_chunks ? moe_few_second_kernel<128, true> : moe_few_second_kernel<64, true>)
+                          : (long_chunks ? moe_few_second_kernel<128, false> : moe_few_second_kernel<64, false>);
   constexpr int lds = KW * SLOTS * SLOT;
-  static bool configured[2] = {false, false};
-  if (!configured[long_chunks]) {
+  static bool configured[2][2] = {};
+  if (!configured[far][long_chunks]) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) {
       lq_set_error("moe_few: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
       return -2;
     }
-    configured[long_chunks] = true;
+    configured[far][long_chunks] = true;
   }
   kernel<<<dim3(lq_ceil_div(width, 16), pieces), THREADS, lds, stream>>>((const bf16_t*)act, lda, (const bf16_t*)w, ldw, w_packed, out, ldo,
                                                                          piece_stride, width, Experts{route, rows, experts, ff, shared},

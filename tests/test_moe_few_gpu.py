@@ -121,6 +121,38 @@ def test_sums_of_halves_and_chunks_stay_apart(rows, ff, places, pack):
     assert bool((out == 1.0).all())
 
 
+@pytest.mark.parametrize("rows,ff,width", [(8, 128, 512), (8, 576, 2048), (12, 704, 2112)])
+@pytest.mark.parametrize("pack", [True, False])
+def test_activations_beyond_32_bit_offsets(rows, ff, width, pack):
+    """Rows of activations 2^31 bytes from first to last and more: the bits of the same ones side by side."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, E, shared = HipKernels(), 3, 64
+    kn.pack_weights = pack
+    gen = torch.Generator(device="cuda").manual_seed(rows + ff)
+    inner, apart = E * ff + shared, 2 ** 31 // 2 // (rows - 1) // 8 * 8 + 8
+    x, w_in = (torch.randn(n, width, generator=gen, device="cuda").bfloat16() for n in (rows, inner))
+    w_out = torch.randn(width, inner, generator=gen, device="cuda").bfloat16()
+    route = torch.rand(rows, E, generator=gen, device="cuda")
+    route[:, 1], route[0, 2] = -1.0, -1.0
+    outs = []
+    for act in (torch.empty(rows, inner, dtype=torch.bfloat16, device="cuda"),
+                torch.empty((rows - 1) * apart + inner, dtype=torch.bfloat16, device="cuda").as_strided((rows, inner), (apart, 1))):
+        out = torch.empty(kn.moe_few_pieces(width), rows, width, device="cuda")
+        kn.moe_few(x, kn.pack_weight(w_in), kn.pack_weight(w_out), route, act, out, ff, shared, "relu2")
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
+def test_how_many_columns_are_taken():
+    """Up to 2^30 columns of the second matrix, as offsets of its rows are 64-bit where they have to be."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    assert kn.moe_few_supported(torch.bfloat16, 8, 64, 2 ** 20, 0, 512) and kn.moe_few_supported(torch.bfloat16, 16, 16, 2 ** 26 - 64, 64, 4096)
+    assert not kn.moe_few_supported(torch.bfloat16, 8, 64, 2 ** 24, 0, 512)
+
+
 def test_sizes_that_are_not_taken():
     from longbow_quarrel_amd.kernels.hip import HipKernels
 
