@@ -155,7 +155,8 @@ __device__ __forceinline__ void piece_to_lds(const float* base, int range, int o
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)lds, 16, offset, skip, 0, 0);
 }
 
-template <typename TO, int TM, int STAGES = 2>  // 32 TM rows a block
+// 32 TM rows a block.  FAR: a tile's rows lie beyond the reach of 32-bit offsets, and its transfers go by pointers.
+template <typename TO, int TM, int STAGES = 2, bool FAR = false>
 __global__ __launch_bounds__(256, 2) void gemm_f32_pipelined_kernel(const float* __restrict__ A, int lda,
                                                                     const float* __restrict__ W, int ldw,
                                                                     TO* __restrict__ C, int ldc, int M, int N, int K,
@@ -170,15 +171,19 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pipelined_kernel(const float*
   const int r16 = lane & 15, g = lane >> 4, wm = wave >> 1, wn = wave & 1;
 
   // a wave's transfers of a stage: 8 rows each, lane l the piece at place l % 8 of row l / 8
-  int from[PER];
+  using Offset = std::conditional_t<FAR, long long, int>;
+  Offset from[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int row = (wave * PER + j) * 8 + (lane >> 3), piece = (lane & 7) ^ (row >> 1 & 7);
-    from[j] = (row < BM ? min(row, M - 1 - m0) * lda : min(row - BM, N - 1 - n0) * ldw) * 4 + piece * 16;
+    from[j] = (row < BM ? min(row, M - 1 - m0) * (Offset)lda : min(row - BM, N - 1 - n0) * (Offset)ldw) * 4 + piece * 16;
   }
   auto ask = [&](int j, int s, int k0) {  // (from stage K on nothing is in range)
     const float* base = (wave * PER + j) * 8 < BM ? A + (long long)m0 * lda : W + (long long)n0 * ldw;
-    piece_to_lds(base, k0 < K ? 0x7fffffff : 0, from[j], k0 * 4, stage[s] + (wave * PER + j) * 1024);
+    if constexpr (FAR)  // (there the last stage comes again, to where nothing reads it)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((const char*)(base + min(k0, K - STAGE_K)) + from[j]),
+                                       (__attribute__((address_space(3))) void*)(stage[s] + (wave * PER + j) * 1024), 16, 0, 0);
+    else piece_to_lds(base, k0 < K ? 0x7fffffff : 0, from[j], k0 * 4, stage[s] + (wave * PER + j) * 1024);
   };
   f32x4 total[TM][4], chunk[TM][4];
 #pragma unroll
@@ -487,7 +492,7 @@ int launch(const void* x, const void* w, void* out, int M, int N, int K, int lda
   // rows of four k each, fetched as one piece: K, the strides and the addresses must allow it
   const bool pieces = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)x % (4 * el)) == 0 &&
                       ((uintptr_t)w % (4 * el)) == 0;
-  const bool tiles = sizeof(T) == 4 && pieces && K % STAGE_K == 0 && (long long)(lda > ldw ? lda : ldw) * TILE * 4 < (1ll << 31);
+  const bool tiles = sizeof(T) == 4 && pieces && K % STAGE_K == 0, far = (long long)(lda > ldw ? lda : ldw) * TILE * 4 >= (1ll << 31);
   // Few rows of a wide weight: pipelined tiles once their 128 columns fill enough of the chip, 7 sixteenths for 17 to 32 rows (17 rows by
   // the rows' kernel / here: 12 288 x 4 096 71 / 77 us, 14 336 x 4 096 90 / 78, 28 672 x 4 096 151 / 103; 32 rows of it 180 / 105)
   // and a quarter for 33 to 64 (33 rows of 4 096 x 4 096 45 / 75, 8 192 x 4 096 86 / 76, 14 336 x 4 096 158 / 79).
@@ -516,7 +521,11 @@ int launch(const void* x, const void* w, void* out, int M, int N, int K, int lda
       for (int t = 3; t >= 1; --t)
         if (pipelined_us(t, M, tiles_n, K) < pipelined_us(tm, M, tiles_n, K)) tm = t;
       const long long blocks = (long long)lq_ceil_div(M, 32 * tm) * tiles_n;
-      const auto kernel = tm == 1   ? (blocks <= lq_compute_units() ? gemm_f32_pipelined_kernel<TO, 1, 3> : gemm_f32_pipelined_kernel<TO, 1>)
+      const auto kernel = far ? (tm == 1   ? gemm_f32_pipelined_kernel<TO, 1, 2, true>
+                                 : tm == 2 ? gemm_f32_pipelined_kernel<TO, 2, 2, true>
+                                 : tm == 3 ? gemm_f32_pipelined_kernel<TO, 3, 2, true>
+                                           : gemm_f32_pipelined_kernel<TO, 4, 2, true>)
+                          : tm == 1 ? (blocks <= lq_compute_units() ? gemm_f32_pipelined_kernel<TO, 1, 3> : gemm_f32_pipelined_kernel<TO, 1>)
                           : tm == 2 ? gemm_f32_pipelined_kernel<TO, 2>
                           : tm == 3 ? gemm_f32_pipelined_kernel<TO, 3>
                                     : gemm_f32_pipelined_kernel<TO, 4>;

@@ -31,3 +31,22 @@ def test_products_in_tiles_match_64_bit_sums_and_single_rows(rows, n, k):
     for r in (0, rows // 2, rows - 1):
         kn.linear(x[r : r + 1], w, one)
         assert torch.equal(out[r : r + 1], one), r
+
+
+@pytest.mark.parametrize("rows,n,k", [(65, 65, 32), (90, 4100, 96), (70, 16600, 288), (129, 32768, 64), (40, 33000, 64)])
+@pytest.mark.parametrize("which", ["x", "w"])
+def test_rows_beyond_32_bit_offsets(rows, n, k, which):
+    """A tile's rows 2^31 bytes apart from first to last: the bits of the same rows side by side."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, apart = HipKernels(), 2 ** 22
+    n = min(n, 300) if which == "w" else n
+    gen = torch.Generator(device="cuda").manual_seed(rows + n + k)
+    x, w = (torch.randn(r, k, generator=gen, device="cuda") for r in (rows, n))
+    near = x if which == "x" else w
+    far = torch.empty((len(near) - 1) * apart + k, device="cuda").as_strided(near.shape, (apart, 1))
+    far.copy_(near)
+    want, out = torch.empty(rows, n, device="cuda"), torch.full((rows, n), float("nan"), device="cuda")
+    kn.linear(x, w, want)
+    kn.linear(*((far, w) if which == "x" else (x, far)), out)
+    assert torch.equal(out, want)
