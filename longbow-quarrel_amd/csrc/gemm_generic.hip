@@ -390,6 +390,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_stream_kernel(const fl
     for (int h = 0; h < 2; ++h)
       xv[slot][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_off, at + h * 64, 0));
     if (++ask_slab == min(PER, slabs - ask_chunk * PER)) ask_slab = 0, ask_chunk += WAVES;
+    __builtin_amdgcn_sched_barrier(0);  // (the waits count a slot's requests, x's among them: none may change its place with another slot's)
   };
   // this wave's slabs: whole chunks, but for the last of all
   const int my_chunks = wave < chunks ? (chunks - wave + WAVES - 1) / WAVES : 0;

@@ -302,6 +302,7 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       xv[slot][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, at >= 0 ? x_off + 64 * i : NOWHERE, at >= 0 ? at * 2 : 0, 0));
+    __builtin_amdgcn_sched_barrier(0);  // (the waits count a slot's requests: none may change its place with another slot's)
   };
 #pragma unroll
   for (int d = 0; d < SLOTS; ++d) ask(d);
