@@ -25,6 +25,36 @@ def test_a_row_has_the_same_bits_in_every_launch(n, k):
         assert torch.equal(out, one[:rows]), rows
 
 
+@pytest.mark.parametrize("n,k", [(4104, 4384), (8200, 2336), (6150, 6176), (4112, 2048), (4112, 2080),  # 8 wavefronts
+                                 (4096, 4384), (2064, 8224), (4096, 4128), (1000, 12288)])              # 16
+def test_streamed_rows_over_several_rounds_of_chunks(n, k):
+    """At most 16 rows whose wavefronts take more than one chunk of 256 k each, with a part chunk or none at the end: the bits of
+    pipelined tiles, and not-a-numbers around the operands and in a row and a column that stay there."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn = HipKernels()
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    x, w = (torch.full((r + 1, k + 32), float("nan"), device="cuda") for r in (80, n))
+    x[:80, :k], w[:n, :k] = (torch.randn(r, k, generator=gen, device="cuda") for r in (80, n))
+    x, w = x[:80, :k], w[:n, :k]
+    want = torch.empty(80, n, device="cuda")
+    kn.linear(x, w, want)  # (tiles)
+    exact, terms = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # chunks of 256 k in one chain each, then the chunks: at most 256 + k / 256 roundings of 2^-24 of sum |x| |w|
+    assert ((want - exact).abs() <= (256 + k / 256) * 2.0 ** -24 * terms).all()
+    for rows in (1, 4, 16):
+        out = torch.full((rows + 1, n + 3), 7.0, device="cuda")
+        kn.linear(x[:rows], w, out[:rows, :n])
+        assert torch.equal(out[:rows, :n], want[:rows]), rows
+        assert bool((out[rows] == 7).all()) and bool((out[:, n:] == 7).all())
+    w[n - 1, k - 1], x[3, 0] = float("nan"), float("inf")
+    out = torch.empty(16, n, device="cuda")
+    kn.linear(x[:16], w, out)
+    assert bool(out[:, n - 1].isnan().all()) and not bool(out[3].isfinite().any())
+    clean = [r for r in range(16) if r != 3]
+    assert torch.equal(out[clean, : n - 1], want[clean, : n - 1])
+
+
 @pytest.mark.parametrize("n", [2048, 6144])
 def test_a_row_has_the_same_bits_in_every_tile_of_a_wide_weight(n):
     """Numbers of rows around the edges of tiles of 32, 64, 96 and 128, each of which some of these launches take."""
