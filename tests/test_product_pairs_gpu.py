@@ -64,7 +64,15 @@ def test_streamed_products_sum_in_the_same_order(rows, n, k):
     assert torch.equal(got, want[:, :n])
 
 
-@pytest.mark.parametrize("rows,k", [(4, 512), (4, 8192), (3, 14464), (8, 1920), (8, 4096)])
+def squares_of_eights(x):
+    """Sums of the squares of 8 neighbours in the order of both kernels: those of columns 4 apart with one rounding, then sums."""
+    v = x.reshape(len(x), -1, 8)
+    # (a product of two 24-bit numbers and a third number, exact in 64 bits but for the rarest of sums, rounded once)
+    first = (v[..., :4].double() ** 2 + (v[..., 4:] ** 2).double()).float()
+    return (first[..., 0] + first[..., 2]) + (first[..., 1] + first[..., 3])
+
+
+@pytest.mark.parametrize("rows,k", [(1, 2048), (2, 8192), (4, 512), (4, 8192), (3, 14464), (8, 1920), (8, 2048), (8, 4096)])
 def test_streamed_products_of_2048_columns_sum_in_the_same_order(rows, k):
     """Every way out of a product of 8 columns a compute unit."""
     from longbow_quarrel_amd.kernels.hip import HipKernels
@@ -85,6 +93,8 @@ def test_streamed_products_of_2048_columns_sum_in_the_same_order(rows, k):
         kn.linear_unit(x, held, unit, "relu2")
         new, sq = old.clone(), torch.empty(rows, kn.linear_fused_parts(torch.bfloat16, rows, n, k), device="cuda")
         kn.linear_residual(x, held, new, sq)
+        parts = squares_of_eights(new)
+        assert torch.equal(sq, parts)
         assert torch.equal(wide, want) and torch.equal(narrow, want.bfloat16()) and torch.equal(unit, acted) and torch.equal(new, old + want)
 
 
