@@ -58,6 +58,25 @@ def bound_part(kn, width, inner, down=torch.bfloat16):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width,inner", [(512, 1024), (576, 1032), (2048, 1280)])
+@pytest.mark.parametrize("rows", [1, 8, 16, 17, 100])
+def test_where_the_products_epilogue_applies_the_unit(width, inner, rows):
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    part, t, ctx = bound_part(HipKernels(), width, inner)
+    assert part.unit
+    h = torch.randn(rows, width, generator=torch.Generator().manual_seed(inner)).bfloat16().cuda()
+    got = part.forward(h, ctx).double()
+    g, u = (h.double() @ t[f"m.{n}"].T + t[f"m.{n}.b"] for n in ("gate", "up"))
+    act = (g * torch.sigmoid(g) * u).bfloat16().double()
+    want = act @ t["m.down"].T + t["m.down.b"]
+    # (the bound of the test above: sums in 32 bits, and four activations that round to their other neighbour)
+    terms = act.abs() @ t["m.down"].abs().T + t["m.down.b"].abs()
+    largest = act.abs().amax(1, keepdim=True) * t["m.down"].abs().amax(1)
+    assert ((got - want).abs() <= (inner + 128) * 2.0 ** -24 * terms + 4 * 2.0 ** -8 * largest).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 8, 17, 100])
 def test_a_second_matrix_in_32_bits(rows):
     """Its activations stay in 32 bits, so no epilogue rounds them."""

@@ -9,6 +9,12 @@ SIZES = [(8, 2560), (2048, 512), (2048, 4160), (2056, 960), (2064, 1024), (3080,
          (28688, 1216), (40960, 512), (2048, 14400), (4104, 12352), (32784, 2048)]
 
 
+def halves(values, bounds):
+    """Gate's and up's columns, interleaved in eights, each with its bound."""
+    parts = [t.reshape(len(t), -1, 2, 8).unbind(2) for t in (values, bounds)]
+    return [tuple(p[i].reshape(len(values), -1) for p in parts) for i in (0, 1)]
+
+
 @pytest.mark.parametrize("rows", [1, 3, 8, 12, 16])
 @pytest.mark.parametrize("n,k", SIZES)
 def test_every_way_out(rows, n, k):
@@ -33,6 +39,8 @@ def test_every_way_out(rows, n, k):
             gated = torch.empty(rows, n // 2, dtype=bf, device="cuda")
             kn.linear_swiglu(x, held, gated, activation="relu")
             gate, up = wide[:rows, :n].reshape(rows, n // 16, 2, 8).unbind(2)
+            (g, off_g), (u, off_u) = halves(want, bound)
+            assert ((gated - g.clamp(min=0) * u).abs() <= 1.001 * (off_g * (u.abs() + off_u) + g.abs() * off_u) + 2.0 ** -8 * (g * u).abs()).all()
             # (2 048 columns and 13 rows and more: the whole product may take another kernel, whose sums have another order)
             assert rows > 12 or n <= 2048 or torch.equal(gated, (gate.clamp(min=0) * up).reshape(rows, n // 2).to(bf))
             outs.append(gated)
@@ -51,6 +59,15 @@ def test_every_way_out(rows, n, k):
             rstd = (sums.double().sum(1, keepdim=True) / k + 1e-5).rsqrt()
             assert ((half - want * rstd).abs() <= rstd * (bound + 2.0 ** -8 * want.abs()) * 1.001).all()
             outs += [new, sq, scaled, half]
+            if n % 16 == 0:
+                both = torch.empty(rows, n // 2, dtype=bf, device="cuda")
+                kn.linear_scaled(x, sums, 1e-5, held, both, swiglu=True)
+                (g, off_g), (u, off_u) = halves(want * rstd, (bound + 2.0 ** -22 * want.abs()) * rstd)  # (the root, and the product with it)
+                silu = g * torch.sigmoid(g)
+                # (silu' is below 1.1; the exponential and the reciprocal are off by an ulp or so, the exponent by 2^-23 of |gate|)
+                off = 1.1 * off_g * (u.abs() + off_u) + silu.abs() * off_u + (4 + g.abs()) * 2.0 ** -23 * (silu * u).abs()
+                assert ((both - silu * u).abs() <= 1.01 * off + 2.0 ** -8 * (silu * u).abs() + 1e-30).all()
+                outs.append(both)
         got.append(outs)
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
