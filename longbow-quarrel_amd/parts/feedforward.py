@@ -74,7 +74,7 @@ class GatedLinearUnit(FeedForward):
     """down(act(gate(h)) * up(h)) with a choice of `activation` ("relu", "silu", "gelu_tanh").  gate and up are one
     matrix product whose 32-bit result the activation kernel reads; with "gelu_tanh" or "relu" and no bias, in a bfloat16
     run, the product's epilogue applies it to its 32-bit sums (gate and up rows interleaved when weights are bound).  With `bias` every projection has one
-    (`<name>.b`): the activation kernel, or with "silu" in a bfloat16 run the product's epilogue, adds gate's and up's; down's is one
+    (`<name>.b`): the activation kernel, or with "silu" and all in bfloat16 the product's epilogue, adds gate's and up's; down's is one
     more column of its weight, which meets a column of ones left behind the activations."""
 
     graph_safe = True
