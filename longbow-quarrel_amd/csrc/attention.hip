@@ -8,22 +8,27 @@ int lq_attention_generic(const void* q, int ldq, void* out, int ldo, int dtype, 
                          int window, hipStream_t stream);
 bool lq_attention_mfma_accepts(int dtype, int nh, int nkv, int hd, int block_size, int ldq, int ldo,
                                const void* q, const void* out, int decode);
-long long lq_attention_mfma_workspace(int rows, int nh, int nkv, int hd, int max_len);
-int lq_attention_mfma_unit_search(const int* pos, int rows, int nkv, int max_len);
 int lq_attention_mfma(const void* q, int ldq, void* out, int ldo, int rows, int batch, int nh, int nkv,
                       int hd, const int* row_pos, const int* seq_slot, const int* cu_rows,
                       const int* block_table, int bt_stride, const void* kcache, const void* vcache,
-                      float scale, int window, int decode, int max_len, float* workspace,
-                      long long workspace_floats, int* tickets, long long tickets_n, const void* k_new,
-                      const void* v_new, int ldk, int ldv, const float* cs, int uneven, int pieces,
-                      long long piece_stride, hipStream_t stream);
+                      float scale, int window, hipStream_t stream);
+// attention_decode.hip: one row a sequence
+long long lq_attention_decode_workspace(int rows, int nh, int nkv, int hd, int max_len);
+int lq_attention_unit_tries(const int* pos, int rows, int nkv, int max_len);
+int lq_attention_decode(const void* q, int ldq, void* out, int ldo, int rows, int nh, int nkv,
+                        int hd, const int* row_pos, const int* seq_slot,
+                        const int* block_table, int bt_stride, const void* kcache, const void* vcache,
+                        float scale, int window, int max_len, float* workspace,
+                        long long workspace_floats, int* tickets, long long tickets_n, const void* k_new,
+                        const void* v_new, int ldk, int ldv, const float* cs, int uneven, int pieces,
+                        long long piece_stride, hipStream_t stream);
 
 // Floats of workspace lq_attention wants for this launch (0: none).
 extern "C" long long lq_attention_workspace(int dtype, int rows, int nh, int nkv, int hd, int block_size,
                                             int decode, int max_len) {
   if (!decode || dtype != LQ_BF16) return 0;
   if (!lq_attention_mfma_accepts(dtype, nh, nkv, hd, block_size, 8, 8, nullptr, nullptr, decode)) return 0;
-  return lq_attention_mfma_workspace(rows, nh, nkv, hd, max_len);
+  return lq_attention_decode_workspace(rows, nh, nkv, hd, max_len);
 }
 
 // A decoding launch shapes its grid by the bound of the lengths rounded up to this many tokens: whoever keeps
@@ -49,7 +54,7 @@ extern "C" int lq_attention_lengths_uneven(const int* lengths, int n) {
 // they would not find it, which must not happen for positions below max_len).
 extern "C" int lq_attention_unit_search(const int* pos, int rows, int nkv, int max_len) {
   if (pos == nullptr || rows <= 0 || nkv <= 0 || max_len <= 0) return 0;
-  return lq_attention_mfma_unit_search(pos, rows, nkv, max_len);
+  return lq_attention_unit_tries(pos, rows, nkv, max_len);
 }
 
 // Whether a decoding launch can take the rotation of q and k and the cache write upon itself
@@ -88,11 +93,18 @@ extern "C" int lq_attention(const void* q, int ldq, void* out, int ldo, int dtyp
   LQ_REQUIRE(window >= 0, "attention: window %d must not be negative", window);
   LQ_REQUIRE(q && out && row_pos && row_seq && seq_slot && cu_rows && block_table && kcache && vcache,
              "attention: null pointer");
-  if (!force_generic && lq_attention_mfma_accepts(dtype, nh, nkv, hd, block_size, ldq, ldo, q, out, decode))
-    return lq_attention_mfma(q, ldq, out, ldo, rows, batch, nh, nkv, hd, row_pos, seq_slot, cu_rows,
-                             block_table, bt_stride, kcache, vcache, scale, window, decode, max_len,
-                             workspace, workspace_floats, tickets, tickets_n, k_new, v_new, ldk, ldv, cs, uneven,
-                             pieces, piece_stride, stream);
+  if (!force_generic && lq_attention_mfma_accepts(dtype, nh, nkv, hd, block_size, ldq, ldo, q, out, decode)) {
+    if (!decode) {
+      LQ_REQUIRE(pieces <= 1, "attention: pieces of q, k and v are taken by the launch that rotates them only");
+      LQ_REQUIRE(cs == nullptr, "attention: the folded rotation needs a decoding step, a head size that is a multiple of 64 and the step's keys and values");
+      return lq_attention_mfma(q, ldq, out, ldo, rows, batch, nh, nkv, hd, row_pos, seq_slot, cu_rows, block_table, bt_stride,
+                               kcache, vcache, scale, window, stream);
+    }
+    LQ_REQUIRE(rows == batch, "attention: decoding needs one row a sequence (%d rows, %d sequences)", rows, batch);
+    return lq_attention_decode(q, ldq, out, ldo, rows, nh, nkv, hd, row_pos, seq_slot, block_table, bt_stride, kcache, vcache,
+                               scale, window, max_len, workspace, workspace_floats, tickets, tickets_n, k_new, v_new, ldk, ldv, cs,
+                               uneven, pieces, piece_stride, stream);
+  }
   LQ_REQUIRE(cs == nullptr && pieces <= 1, "attention: the folded rotation was asked of a launch the matrix-core kernel does not take");
   return lq_attention_generic(q, ldq, out, ldo, dtype, rows, batch, nh, nkv, hd, row_pos, row_seq, seq_slot,
                               block_table, bt_stride, kcache, vcache, block_size, scale, window, stream);

@@ -1,0 +1,59 @@
+"""Decoding attention at the lengths where cache blocks, takes of several blocks, whole rows and shares of a row end, and with operands
+that do not lie on 16 bytes, against the plain implementation in float64."""
+import math
+
+import pytest
+import torch
+
+from test_kernels_gpu import BS, DEV, i32, kn, paged_cache, rel_err  # noqa: F401
+import plain
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 63, 64, 65, 128, 129, 192, 193, 256, 257, 384, 385, 386, 640, 1030, 2049]
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,rows", [(32, 8, 128, 3), (16, 16, 64, 16), (8, 1, 64, 1), (6, 2, 256, 4),
+                                                          (4, 1, 192, 16)])
+@pytest.mark.parametrize("window", [0, 70])
+@pytest.mark.parametrize("apart", [0, 1])
+def test_folded_rows_at_the_edges(kn, heads, kv_heads, head_dim, rows, window, apart):
+    """`apart`: how many entries the step's keys and values lie behind 16 bytes, and the workspace behind 8."""
+    gen = torch.Generator().manual_seed(heads + head_dim + rows)
+    dtype, freqs = torch.bfloat16, plain.rope_frequencies(head_dim, 500000.0)
+    for at in range(0, len(EDGES), rows):
+        lengths = (EDGES[at : at + rows] + EDGES)[:rows]
+        kc, vc, table, slots, dense = paged_cache(lengths, kv_heads, head_dim, dtype, at)
+        q, k, v = (torch.randn(rows, n * head_dim + 8, generator=gen).to(dtype) for n in (heads, kv_heads, kv_heads))
+        angle = torch.tensor([n - 1 for n in lengths], dtype=torch.float64)[:, None] * freqs
+        cs = torch.stack([torch.cos(angle), torch.sin(angle)], -1).float().to(DEV)
+        c, s = cs[:, None, :, 0].double().cpu(), cs[:, None, :, 1].double().cpu()
+
+        def turned(x, n):
+            y = x[:, : n * head_dim].double().view(rows, n, 2, head_dim // 2)
+            return torch.cat([y[:, :, 0] * c - y[:, :, 1] * s, y[:, :, 0] * s + y[:, :, 1] * c], -1).to(dtype).double()
+
+        qd, kd, vd = (torch.zeros(rows, t.shape[1] + 8, dtype=dtype, device=DEV) for t in (q, k, v))
+        qd[:, : q.shape[1]], kd[:, apart : apart + k.shape[1]], vd[:, apart : apart + v.shape[1]] = q.to(DEV), k.to(DEV), v.to(DEV)
+        out = torch.empty(rows, heads * head_dim, dtype=dtype, device=DEV)
+        need = kn.attention_workspace(dtype, rows, heads, kv_heads, head_dim, BS, True, max(lengths))
+        ws = torch.empty(need + 2, dtype=torch.float32, device=DEV)[apart:]
+        for b, n in enumerate(lengths):  # the new position's place holds nothing yet, those behind it never did
+            blk = table[slots[b], (n - 1) // BS].long()
+            kc[blk, :, (n - 1) % BS :], vc[blk, :, :, (n - 1) % BS :] = float("inf"), float("nan")
+        kn.attention(qd, out, heads, kv_heads, head_dim, i32([n - 1 for n in lengths]), i32(range(rows)), i32(slots),
+                     i32(range(rows + 1)), table, kc, vc, BS, 1.0 / math.sqrt(head_dim), window, decode=True, max_len=max(lengths),
+                     workspace=ws, k_new=kd[:, apart:], v_new=vd[:, apart:], cos_sin=cs)
+        qt, kt = turned(q, heads), turned(k, kv_heads)
+        for b, n in enumerate(lengths):
+            keys, values = (t.double().clone() for t in dense[b])
+            keys[n - 1], values[n - 1] = kt[b], v[b, : kv_heads * head_dim].double().view(kv_heads, head_dim)
+            full = torch.zeros(n, heads, head_dim, dtype=torch.float64)
+            full[n - 1] = qt[b]
+            want = plain.attention(full, keys, values, window=window, rows=[n - 1])[n - 1]
+            # (the result and the probabilities are rounded to 8 bits, 2^-9 each at most, as in the other tests of this kernel)
+            assert rel_err(out[b].view(heads, head_dim), want) < 1.2e-2, (b, n)
+            blk, off = table[slots[b], (n - 1) // BS].long(), (n - 1) % BS
+            assert torch.equal(vc[blk, :, :, off].cpu(), v[b, : kv_heads * head_dim].view(kv_heads, head_dim))
+            assert rel_err(kc[blk, :, off], kt[b]) < 4e-3
+        assert int(kn.tickets(torch.device("cuda", torch.cuda.current_device())).abs().max()) == 0
