@@ -1,20 +1,24 @@
 // Steps of single tokens of a bfloat16 run through the windowed attention of attention_sink.hip (the same masks, sinks,
 // shaped scores, maps and gates).
 //
-// A workgroup of four wavefronts takes one row of the step, up to 16 query heads of one key head and one of `splits`
-// shares of the keys: the blocks of 64 positions that the row sees, numbered from the kept first ones on, go to the
-// wavefronts of all shares in turn, so that at a few thousand keys every wavefront has one.  It asks for all of a block's
-// keys and values before it waits for any: what bounds such a step is the chain of round trips to memory, not the bytes
-// (tiles that asked for a few bytes of a key row at a time, a product between, and a second launch that merged the
-// shares: microseconds before and now, 8 rows, 16 heads: 4 key heads of 128 at 512 keys 20 -> 12, at 1 500 keys under a
-// window of 1 024 31 -> 13, with values of 256 and two maps 28 -> 16; one key head of 256 with values of 192 28 -> 21;
-// 64 rows at 500 keys 34 -> 19; 2 rows with capped scores and a table of biases 30 -> 15).  The shares of a row meet in its
-// last workgroup to finish (a ticket a row and key head; partial results pass the dies' caches as device-scope atomics),
-// which adds them up in their order; a caller who gives no tickets gets a second launch that does the same.
+// A workgroup of four wavefronts takes one row of the step, up to 16 query heads of one key head and one of up to `splits`
+// shares of the blocks of 64 positions that the row sees, numbered from the kept first ones on.  All four work on the same block (two of
+// key and value sizes up to 64): 16 keys' scores a wavefront, whose probabilities meet in LDS, and a quarter of the value
+// entries each, so that nothing is merged at a share's end.  The next block is asked for ahead of this one's products.  What bounds
+// such a step is the rate at which one compute unit draws its blocks (1.1 us for 32 KB), the chain of round trips around it and the
+// code's own way from memory (attention_decode.hip, which has the same structure for plain causal attention): so blocks are
+// dealt out evenly over as many workgroups as pay for it, and a key head's query heads over several workgroups where rows are few
+// (`shares_for`).  The shares of a row meet in its last workgroup to finish (a ticket a row and tile of heads; partial
+// results pass the dies' caches as device-scope atomics), which adds them up in their order; a caller who gives no tickets gets
+// a second launch that does the same.
+//
+// Microseconds a launch, a wavefront with a block of its own, shares of at least four blocks and 16 heads a workgroup -> this:
+// one key head of 256 with values of 192 under 16 heads, 8 rows of 216 to 716 keys 18.2 -> 11.0, one of 700 18.0 -> 9.2, one of 3 000 21.4 -> 12.9,
+// 24 of 100 11.5 -> 8.7; 16 heads of 128 over 4: 8 rows of 520 keys 11.8 -> 8.9, with two maps over values of 256 15.1 -> 11.1, 2 rows of
+// 1 000 with capped scores 13.2 -> 10.2, with a table of biases 14.6 -> 10.6; 24 rows of 120 keys, 32 heads over 8, 8.2 -> 8.0.
 //
 //   S^T[key][head] = K . Q^T by v_mfma_f32_16x16x32_bf16: lane (c = l % 16, g = l / 16) gives A[c][8 g .. + 8] and B[c][the
-//   same] and receives D[4 g + e][c].  Row i of tile j (of a run of 32 keys) is key 8 (i / 4) + 4 j + i % 4: a lane's scores
-//   of both tiles are then keys 8 g .. + 7 of its head, which O^T[d][head] += V^T . P^T takes as they are.
+//   same] and receives D[4 g + e][c]; O^T[d][head] += V^T . P^T with eight consecutive keys a lane, read back from LDS.
 // The probabilities stay 32-bit, multiplied in three bfloat16 parts that add up to them exactly (attention_sink_rows.hip).
 // Values of positions that were never written count as zero.
 #include "attention_sink.h"
@@ -24,6 +28,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int BLOCK = 64, NW = 4, MAX_SPLITS = 64;
+constexpr int NARROW = 3;  // blocks a share up to which one workgroup a compute unit is better than two
 
 // over the four lanes that share l % 16
 __device__ inline float across_max(float x) {
@@ -39,13 +44,9 @@ __device__ inline float across_sum(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-__device__ inline void publish(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ inline void publish2(float* p, float x, float y) {  // two neighbours on 8 bytes
   const unsigned long long v = (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x);
   __hip_atomic_store((unsigned long long*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline float published(const float* p) {
-  return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ inline float2 published2(const float* p) {  // two neighbours on 8 bytes
   const unsigned long long v = __hip_atomic_load((unsigned long long*)const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -53,8 +54,11 @@ __device__ inline float2 published2(const float* p) {  // two neighbours on 8 by
 }
 
 struct Shares {
-  int splits;
-  float* part;   // [row][key head's tile][split]: cols x VD results, then cols maxima and cols sums
+  int splits, narrow;    // workgroups a row and tile at most; the same without a second one on any compute unit
+  int heads, tiles;      // query heads a workgroup; how many such tiles a key head has
+  int whole;             // blocks up to which a row stays whole
+  float apart;           // what a share more costs, in blocks' time
+  float* part;   // [row][key head's tile][split]: heads x VD results, then maximum and sum of each head
   int* tickets;  // [row][key head's tile], zero between launches; or null: a second launch adds the shares up
 };
 
@@ -70,143 +74,115 @@ __device__ inline Blocks blocks_of(const SinkArgs& a, int pos) {
   b.n = b.kept + pos / BLOCK - b.wstart / BLOCK + 1;
   return b;
 }
-__device__ inline int live_shares(const Shares& sh, const Blocks& b) {  // shares with a block for some wavefront
-  return min(sh.splits, (b.n + NW - 1) / NW);
+
+// n / d and its ceiling for whole numbers below 2^20: half a unit of the numerator is more than the reciprocal's error.
+__device__ inline int quotient(int n, int d) {
+  return __builtin_amdgcn_readfirstlane((int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d)));
+}
+
+// Blocks a share of a row that has n: the rule of attention_decode.hip, with the costs of these sizes (`shares_for`).
+__device__ inline int blocks_a_share(const Shares& sh, int n) {
+  if (n <= sh.whole || sh.splits == 1) return n;
+  const int narrow = quotient(n - 1, sh.narrow) + 1, even = narrow <= NARROW ? narrow : quotient(n - 1, sh.splits) + 1;
+  return max(even, __builtin_amdgcn_readfirstlane((int)(__builtin_amdgcn_sqrtf((float)n * sh.apart) + 0.5f)));
 }
 
 // A workgroup's row and key head's tile: its query heads hbase .. hbase + cols - 1.
 struct Heads {
   int kvh, hbase, cols, share_floats;
 };
-__device__ inline Heads heads_of(const SinkArgs& a) {
-  const int group = a.nh / a.nkv, tiles = (group + 15) / 16, kvh = blockIdx.y / tiles;
-  const int hbase = kvh * group + blockIdx.y % tiles * 16;
-  return {kvh, hbase, min(16, (kvh + 1) * group - hbase), min(16, group) * (a.VD + 2)};
+__device__ inline Heads heads_of(const SinkArgs& a, const Shares& sh) {
+  const int group = a.heads_per_tile, kvh = sh.tiles == 1 ? blockIdx.y : quotient(blockIdx.y, sh.tiles);
+  const int hbase = kvh * group + (blockIdx.y - kvh * sh.tiles) * sh.heads;
+  return {kvh, hbase, min(sh.heads, (kvh + 1) * group - hbase), sh.heads * (a.VD + 2)};
 }
 
-// What a head's entries are multiplied with, from the sum of its probabilities and the logit of its gate (asked for by gate_of,
-// long before the sums are there).
-__device__ inline float gate_of(const bf16_t* gate, const SinkArgs& a, int r, int hbase, int cc, int cols) {
-  return gate != nullptr && cc < cols ? to_f32(gate[(long long)r * a.ldg + hbase + cc]) : 0.f;
+__device__ inline float gate_of(const bf16_t* gate, const SinkArgs& a, int r, int h) {
+  return gate != nullptr ? to_f32(gate[(long long)r * a.ldg + h]) : 0.f;
 }
+// What a head's entries are multiplied with, from the sum of its probabilities and the logit of its gate.
 __device__ inline float head_factor(const bf16_t* gate, float logit, float L) {
   float f = 1.0f / L;
   if (gate != nullptr) f /= 1.f + expf(-logit);
   return f;
 }
 
-// Two neighbouring entries (idx: of the tile's cols x VD, even) from their sums over the keys.
-__device__ inline float2 wide_gate_of(const SinkArgs& a, int r, int hbase, int idx) {
-  if (a.wide_gate == nullptr) return make_float2(0.f, 0.f);
-  const float* p = a.wide_gate + (long long)r * a.ldwg + hbase * a.VD + idx;
-  return make_float2(p[0], p[1]);
-}
-__device__ inline void finish2(void* out, const SinkArgs& a, int r, int hbase, int idx, float2 sum, float factor, float2 wide) {
+// Two neighbouring entries (d, even, of head h) from their sums over the keys.
+__device__ inline void finish2(void* out, const SinkArgs& a, int r, int h, int d, float2 sum, float factor) {
   float2 v = make_float2(sum.x * factor, sum.y * factor);
-  if (a.wide_gate != nullptr) v.x /= 1.f + expf(-wide.x), v.y /= 1.f + expf(-wide.y);
-  const long long at = (long long)r * a.ldo + hbase * a.VD + idx;
+  if (a.wide_gate != nullptr) {
+    const float* p = a.wide_gate + (long long)r * a.ldwg + h * a.VD + d;
+    v.x /= 1.f + expf(-p[0]), v.y /= 1.f + expf(-p[1]);
+  }
+  const long long at = (long long)r * a.ldo + h * a.VD + d;
   put_out((bf16_t*)out, at, v.x, a.out_f32);
   put_out((bf16_t*)out, at + 1, v.y, a.out_f32);
 }
 
-// The shares of a row and tile added up in their order, by a whole workgroup.
-__device__ inline void add_shares(void* out, const bf16_t* gate, float gate_logit, const SinkArgs& a, const Shares& sh, const Heads& hd, int live) {
-  __shared__ float factor[MAX_SPLITS][16], sums[MAX_SPLITS][16], whole[16];
-  const int tid = threadIdx.x, r = blockIdx.x, cols = hd.cols, VD = a.VD;
+// The shares of a row and tile added up in their order, by a whole workgroup: two neighbouring entries a thread, eight shares' asked
+// for at once (one beyond the last is the last once more, with a weight of zero).
+__device__ inline void add_shares(void* out, const bf16_t* gate, const SinkArgs& a, const Shares& sh, const Heads& hd, int live) {
+  constexpr int AT_ONCE = 8;
+  const int r = blockIdx.x, VD = a.VD;
   const float* shares = sh.part + ((long long)r * gridDim.y + blockIdx.y) * sh.splits * hd.share_floats;
-  // The results of the first eight shares (three pairs of entries a thread) are asked for together with every share's factor
-  // for every head and the heads' sums: all that a row of up to eight shares waits for is one round trip for every 1 536 entries.
-  // (Entries one by one, four of four shares together, behind the factors, 16 heads of 192 of five shares waited for seven: 8 rows
-  // of 700 keys 20.8 -> 19.2 us, 4 rows of 2 900 and 32 heads 26.4 -> 22.7; 8 rows of 32 heads of 128 over 8 14.7 -> 13.6.)
-  constexpr int PAIRS = 3, SHARES = 8;
-  const int entries = cols * VD;
-  float2 v[SHARES][PAIRS];
-  auto ask = [&](int s0, int i0) {
-#pragma unroll
-    for (int j = 0; j < SHARES; ++j)
-      if (s0 + j < live)  // (the same for the whole workgroup)
-#pragma unroll
-        for (int x = 0; x < PAIRS; ++x)
-          v[j][x] = published2(shares + (s0 + j) * hd.share_floats + min(i0 + 2 * x * NW * 64, entries - 2));
-  };
-  ask(0, 2 * tid);
-  float2 wide[PAIRS];
-  auto ask_wide = [&](int i0) {
-#pragma unroll
-    for (int x = 0; x < PAIRS; ++x) wide[x] = wide_gate_of(a, r, hd.hbase, min(i0 + 2 * x * NW * 64, entries - 2));
-  };
-  ask_wide(2 * tid);
-  for (int x = tid; x < live * cols; x += NW * 64) {
-    const int s = x / cols, cc = x - s * cols;
-    const float* p = shares + s * hd.share_floats + entries + cc;
-    factor[s][cc] = published(p), sums[s][cc] = published(p + cols);
-  }
-  __syncthreads();
-  if (tid < cols) {
+  for (int i = 2 * threadIdx.x; i < hd.cols * VD; i += 2 * NW * 64) {  // (VD is even: a pair is one head's)
+    const int c = (int)(((float)i + 0.5f) * __builtin_amdgcn_rcpf((float)VD));
+    const float logit = gate_of(gate, a, r, hd.hbase + c);
     float M = NONE, L = 0.f;
-    for (int s = 0; s < live; ++s) M = fmaxf(M, factor[s][tid]);
-    for (int s = 0; s < live; ++s) {
-      const float f = __builtin_amdgcn_exp2f(factor[s][tid] - M);
-      factor[s][tid] = f, L = fmaf(f, sums[s][tid], L);
+    float2 acc = make_float2(0.f, 0.f);
+    for (int s0 = 0; s0 < live; s0 += AT_ONCE) {
+      float2 stat[AT_ONCE], sum[AT_ONCE];
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) {
+        const float* p = shares + min(s0 + j, live - 1) * hd.share_floats;
+        stat[j] = published2(p + sh.heads * VD + 2 * c), sum[j] = published2(p + i);
+      }
+      float top = M;
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) top = fmaxf(top, stat[j].x);
+      const float keep = __builtin_amdgcn_exp2f(M - top);
+      acc.x *= keep, acc.y *= keep, L *= keep, M = top;
+#pragma unroll
+      for (int j = 0; j < AT_ONCE; ++j) {
+        const float f = s0 + j < live ? __builtin_amdgcn_exp2f(stat[j].x - M) : 0.f;
+        acc.x = fmaf(f, sum[j].x, acc.x), acc.y = fmaf(f, sum[j].y, acc.y), L = fmaf(f, stat[j].y, L);
+      }
     }
-    whole[tid] = head_factor(gate, gate_logit, L);
-  }
-  __syncthreads();
-  for (int i0 = 2 * tid; i0 < entries; i0 += 2 * PAIRS * NW * 64) {
-    float2 sum[PAIRS];
-#pragma unroll
-    for (int x = 0; x < PAIRS; ++x) sum[x] = make_float2(0.f, 0.f);
-    if (i0 > 2 * tid) ask_wide(i0);
-    for (int s0 = 0; s0 < live; s0 += SHARES) {
-      if (s0 > 0 || i0 > 2 * tid) ask(s0, i0);
-#pragma unroll
-      for (int j = 0; j < SHARES; ++j)
-        if (s0 + j < live)
-#pragma unroll
-          for (int x = 0; x < PAIRS; ++x) {
-            const float f = factor[s0 + j][min(i0 + 2 * x * NW * 64, entries - 2) / VD];  // (VD is even: a pair is one head's)
-            sum[x].x = fmaf(f, v[j][x].x, sum[x].x), sum[x].y = fmaf(f, v[j][x].y, sum[x].y);
-          }
-    }
-#pragma unroll
-    for (int x = 0; x < PAIRS; ++x) {
-      const int idx = i0 + 2 * x * NW * 64;
-      if (idx >= entries) continue;
-      finish2(out, a, r, hd.hbase, idx, sum[x], whole[idx / VD], wide[x]);
-    }
+    finish2(out, a, r, hd.hbase + c, i - c * VD, acc, head_factor(gate, logit, L));
   }
 }
 
 __global__ __launch_bounds__(NW * 64) void sink_add_shares_kernel(void* __restrict__ out, const bf16_t* __restrict__ gate,
                                                                   SinkArgs a, Shares sh) {
-  const int live = live_shares(sh, blocks_of(a, a.row_pos[blockIdx.x]));
-  const Heads hd = heads_of(a);
-  if (live > 1) add_shares(out, gate, gate_of(gate, a, blockIdx.x, hd.hbase, threadIdx.x, hd.cols), a, sh, hd, live);  // (else the row is finished)
+  const int n = blocks_of(a, a.row_pos[blockIdx.x]).n, live = quotient(n - 1, blocks_a_share(sh, n)) + 1;
+  if (live > 1) add_shares(out, gate, a, sh, heads_of(a, sh), live);  // (else the row is finished)
 }
 
-// KD and VD up to 32 KS and 16 VT: sizes in between run with zeros behind their keys and values.
+// KD and VD up to 32 KS and 16 VT: sizes in between run with zeros behind their keys and values.  GB blocks are taken together.
+template <int KS, int VT>
+struct Share {
+  static constexpr int VW = VT / NW, GB = KS + VT / 2 <= 4 ? 2 : 1;
+  u32x4 k[GB][KS];     // of the wavefront's 16 keys row lane % 16, entries 32 ks + 8 (lane / 16) ..
+  u32x4 v[GB][VW][2];  // of its tiles of value entries row lane % 16, positions 32 j + 8 (lane / 16) ..
+  float bias[GB][4];   // by distance, for scores 4 (lane / 16) + e
+};
+
 template <int KS, int VT, bool SHAPED>
-__global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink_decode_kernel(
+__global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
     const bf16_t* __restrict__ q, void* __restrict__ out, const bf16_t* __restrict__ gate,
     const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache, SinkArgs a, Shares sh) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];  // [NW][16][VD + 4]
-  __shared__ float lds_m[NW][16], lds_l[NW][16], factors[NW + 1][16];
+  using S = Share<KS, VT>;
+  __shared__ __attribute__((aligned(16))) float scores[2][16][S::GB * BLOCK + 4];  // (apart so that neighbouring heads' lie in other banks)
+  __shared__ __attribute__((aligned(16))) float tops[2][16][NW];  // (what wavefronts' probabilities were taken against)
   __shared__ int last;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
   const int r = blockIdx.x, split = blockIdx.z;
-  const Heads hd = heads_of(a);
-  const int kvh = hd.kvh, hbase = hd.hbase, cols = hd.cols, h = hbase + min(c, cols - 1);
-  const int nvh = a.nkv / a.maps, vh = kvh / a.maps, KD = a.KD, VD = a.VD, row_floats = VD + 4;
-  const long long krow = (long long)a.maps * KD;
-
   // (rows of single tokens mostly are their sequences' in order: that one's slot is asked for beside the row's sequence, not behind it)
   const int pos = a.row_pos[r], seq = a.row_seq[r], likely = a.seq_slot[r];
-  const float gate_logit = gate_of(gate, a, r, hbase, tid, cols);
-  const int* table = a.block_table + (long long)(seq == r ? likely : a.seq_slot[seq]) * a.bt_stride;
-  const Blocks seen = blocks_of(a, pos);
-  const int lo = seen.lo, wstart = seen.wstart, kept = seen.kept, blocks = seen.n, live = live_shares(sh, seen);
-  if (split >= live) return;  // the whole workgroup
-
+  const Heads hd = heads_of(a, sh);
+  const int kvh = hd.kvh, cols = hd.cols, h = hd.hbase + min(c, cols - 1);  // (columns beyond the tile's heads repeat the last one's)
+  const int KD = a.KD, VD = a.VD, maps = a.maps, vh = maps == 1 ? kvh : quotient(kvh, maps), nvh = maps == 1 ? a.nkv : quotient(a.nkv, maps);
+  // the query and what is asked of its head, before the position is known
   u32x4 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
@@ -214,143 +190,168 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
     qf[ks] = d < KD ? __builtin_bit_cast(u32x4, load_q8(q + (long long)r * a.ldq + h * KD + d)) : (u32x4){0u, 0u, 0u, 0u};
   }
   HeadShape hs;
-  if constexpr (SHAPED) hs = head_shape(a, h);
+  const float* dist = nullptr;
+  if constexpr (SHAPED) {
+    hs = head_shape(a, h);
+    dist = hs.dist, hs.dist = nullptr;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int* table = a.block_table + (long long)(seq == r ? likely : a.seq_slot[seq]) * a.bt_stride;
+  const Blocks seen = blocks_of(a, pos);
+  const int lo = seen.lo, wstart = seen.wstart, kept = seen.kept;
+  const int per = blocks_a_share(sh, seen.n), live = quotient(seen.n - 1, per) + 1;
+  if (split >= live) return;  // the whole workgroup
+  const int i0 = split * per, i1 = min(i0 + per, seen.n) - 1;
+  auto start_of = [&](int i) { return i < kept ? i * BLOCK : wstart + (i - kept) * BLOCK; };
+
+  const int krow = maps * KD * 2;  // bytes
+  const int k_at = (16 * w + c) * krow + ((kvh - vh * maps) * KD + 8 * g) * 2, v_at = ((16 * w + c) * BLOCK + 8 * g) * 2;
+  // Asks for a block, or, with the same instructions, for nothing at all (a descriptor of no bytes, every access of which is
+  // out of bounds and yields zero), as entries beyond KD and VD are.
+  auto ask = [&](int i, int blk, int u, S& s) {
+    const bool there = i <= i1;
+    const long long at = (long long)blk * nvh + vh;
+    const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)(kcache + at * BLOCK * (maps * KD)), 0, there ? BLOCK * krow : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void*)(vcache + at * BLOCK * VD), 0, there ? BLOCK * VD * 2 : 0, 0x00020000);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      s.k[u][ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(kr, 32 * ks + 8 * g < KD ? k_at + 64 * ks : 0x40000000, 0, 0));
+#pragma unroll
+    for (int x = 0; x < S::VW; ++x)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        s.v[u][x][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, v_at + x * (NW * 16 * BLOCK * 2) + 64 * j, 0, 0));
+    if constexpr (SHAPED)
+      if (dist != nullptr)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s.bias[u][e] = dist[min(max(pos - (start_of(i) + 16 * w + 4 * g + e), 0), hs.last)];
+  };
+  S cur;
+  int ahead[S::GB];
+#pragma unroll
+  for (int u = 0; u < S::GB; ++u) ahead[u] = table[start_of(min(i0 + u, i1)) / BLOCK];
+#pragma unroll
+  for (int u = 0; u < S::GB; ++u) ask(i0 + u, ahead[u], u, cur);
+  __builtin_amdgcn_sched_barrier(0);
+
   const float c2 = a.scale * LOG2E;
   float m = NONE, l = 0.f;  // the head's running maximum (in powers of two); this lane's share of its sum
-  if (a.sink && split == 0 && w == 0) {
+  if (a.sink && split == 0) {
     const SinkStart start = sink_start(a, h);
     m = start.m, l = g == 0 ? start.l : 0.f;
   }
-  f32x4 o[VT];  // o[dt][e]: value entry 16 dt + 4 g + e of head c
+  const float gate_logit = gate_of(gate, a, r, h);
+  f32x4 o[S::VW];  // o[x][e]: value entry 16 (w + NW x) + 4 g + e of head c
 #pragma unroll
-  for (int dt = 0; dt < VT; ++dt) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int x = 0; x < S::VW; ++x) o[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  for (int i = split * NW + w; i < blocks; i += live * NW) {
-    const int t0 = i < kept ? i * BLOCK : wstart + (i - kept) * BLOCK;
-    const long long blk = table[t0 / BLOCK];
-    const bf16_t* kb = kcache + (blk * nvh + vh) * BLOCK * krow + (kvh % a.maps) * KD + 8 * g;
-    const bf16_t* vb = vcache + (blk * nvh + vh) * (long long)VD * BLOCK + 8 * g;
-    u32x4 kf[4][KS], vf[VT][2];
+  // Blocks i .. i + GB - 1 of the share, as far as it reaches; `turn`: whose turn it is of the two buffers.  A wavefront takes its
+  // keys' probabilities against their own maximum; whoever reads them multiplies them up to the row's.
+  auto take = [&](int i, int turn, S& s) {
+    f32x4 st[S::GB];  // keys 16 w + 4 g + e of each block
+    float own_top = NONE;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int key = 32 * (j >> 1) + (c >> 2) * 8 + (j & 1) * 4 + (c & 3);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        kf[j][ks] = 32 * ks + 8 * g < KD ? *(const u32x4*)(kb + key * krow + 32 * ks) : (u32x4){0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int dt = 0; dt < VT; ++dt)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        vf[dt][j] = 16 * dt + c < VD ? *(const u32x4*)(vb + (16 * dt + c) * BLOCK + 32 * j) : (u32x4){0u, 0u, 0u, 0u};
-    __builtin_amdgcn_sched_barrier(0);  // (all of them before the first product)
-    f32x4 st[4];  // st[j][e]: key t0 + 32 (j / 2) + 8 g + 4 (j % 2) + e
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      st[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < S::GB; ++u) {
+      const int t0 = start_of(i + u);
+      st[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
-        st[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[j][ks]), as_bf16x8(qf[ks]), st[j], 0, 0, 0);
-    }
-    float top = NONE;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
+        st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(s.k[u][ks]), as_bf16x8(qf[ks]), st[u], 0, 0, 0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int t = t0 + 32 * (j >> 1) + 8 * g + 4 * (j & 1) + e;
-        float s;
-        if constexpr (SHAPED) s = shaped<false>(st[j][e], max(pos - t, 0), hs) * LOG2E;
-        else s = st[j][e] * c2;
-        st[j][e] = t <= pos && (t >= lo || t < a.keep_first) ? s : -INFINITY;
-        top = fmaxf(top, st[j][e]);
+        const int t = t0 + 16 * w + 4 * g + e;
+        float x;
+        if constexpr (SHAPED) {
+          x = shaped<false>(st[u][e], max(pos - t, 0), hs);
+          if (dist != nullptr) x += s.bias[u][e];
+          x *= LOG2E;
+        } else {
+          x = st[u][e] * c2;
+        }
+        st[u][e] = t <= pos && (t >= lo || t < a.keep_first) && i + u <= i1 ? x : -INFINITY;
+        own_top = fmaxf(own_top, st[u][e]);
       }
-    const float m_new = fmaxf(m, across_max(top)), alpha = __builtin_amdgcn_exp2f(m - m_new);
+      if (t0 + BLOCK - 1 > pos) {  // (0 times what lies in unwritten memory may be NaN)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const int t = t0 + 32 * j + 8 * g + 2 * x;
+            const unsigned keep = t + 1 <= pos ? 0xffffffffu : t <= pos ? 0x0000ffffu : 0u;
+#pragma unroll
+            for (int y = 0; y < S::VW; ++y) s.v[u][y][j][x] &= keep;
+          }
+      }
+    }
+    own_top = across_max(own_top);
+#pragma unroll
+    for (int u = 0; u < S::GB; ++u) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[u][e] = __builtin_amdgcn_exp2f(st[u][e] - own_top);
+      *(f32x4*)&scores[turn][c][u * BLOCK + 16 * w + 4 * g] = st[u];
+    }
+    if (g == 0) tops[turn][c][w] = own_top;
+    // (loads fly on; the other buffer's readers have passed this barrier once more than its writers)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const f32x4 tw = *(const f32x4*)&tops[turn][c][0];
+    const float m_new = fmaxf(m, fmaxf(fmaxf(tw[0], tw[1]), fmaxf(tw[2], tw[3]))), alpha = __builtin_amdgcn_exp2f(m - m_new);
     m = m_new;
-    float sum = 0.f;
+    l *= alpha;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int x = 0; x < S::VW; ++x) o[x] *= alpha;
+    const float up[2] = {__builtin_amdgcn_exp2f((g < 2 ? tw[0] : tw[1]) - m), __builtin_amdgcn_exp2f((g < 2 ? tw[2] : tw[3]) - m)};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        st[j][e] = __builtin_amdgcn_exp2f(st[j][e] - m);
-        sum += st[j][e];
-      }
-    l = l * alpha + sum;
+    for (int u = 0; u < S::GB; ++u)
 #pragma unroll
-    for (int dt = 0; dt < VT; ++dt) o[dt] *= alpha;
-    if (t0 + BLOCK - 1 > pos) {  // (0 times what lies in unwritten memory may be NaN)
+      for (int j = 0; j < 2; ++j) {
+        f32x4 pr[2];  // keys 32 j + 8 g .. + 7
+        u32x4 part[3];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+        for (int x = 0; x < 2; ++x) pr[x] = *(const f32x4*)&scores[turn][c][u * BLOCK + 32 * j + 8 * g + 4 * x] * up[j];
+        const f32x4 both = pr[0] + pr[1];
+        l += (both[0] + both[1]) + (both[2] + both[3]);
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-          const int t = t0 + 32 * j + 8 * g + 2 * x;
-          const unsigned keep = t + 1 <= pos ? 0xffffffffu : t <= pos ? 0x0000ffffu : 0u;
+          const float p0 = pr[x >> 1][2 * (x & 1)], p1 = pr[x >> 1][2 * (x & 1) + 1];
+          const float q0 = below_upper(p0), q1 = below_upper(p1);
+          part[0][x] = upper2(p0, p1), part[1][x] = upper2(q0, q1), part[2][x] = upper2(below_upper(q0), below_upper(q1));
+        }
 #pragma unroll
-          for (int dt = 0; dt < VT; ++dt) vf[dt][j][x] &= keep;
+        for (int i3 = 2; i3 >= 0; --i3)
+#pragma unroll
+          for (int x = 0; x < S::VW; ++x)
+            o[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(s.v[u][x][j]), as_bf16x8(part[i3]), o[x], 0, 0, 0);
+      }
+  };
+#pragma unroll
+  for (int u = 0; u < S::GB; ++u) ahead[u] = table[start_of(min(i0 + S::GB + u, i1)) / BLOCK];
+  for (int i = i0, odd = 0;; i += S::GB, odd ^= 1) {
+    S next;
+#pragma unroll
+    for (int u = 0; u < S::GB; ++u) {
+      ask(min(i + S::GB + u, i1 + 1), ahead[u], u, next);
+      ahead[u] = table[start_of(min(i + 2 * S::GB + u, i1)) / BLOCK];
+    }
+    take(i, odd, cur);
+    if (i + S::GB > i1) break;
+    cur = next;
+  }
+  l = across_sum(l);
+  const long long at = (long long)r * gridDim.y + blockIdx.y;
+  if (c < cols) {
+    const float factor = live == 1 ? head_factor(gate, gate_logit, l) : 0.f;
+    float* mine = sh.part + (at * sh.splits + split) * hd.share_floats;
+#pragma unroll
+    for (int x = 0; x < S::VW; ++x) {
+      const int d = 16 * (w + NW * x) + 4 * g;
+      if (d < VD)  // (VD is a multiple of 4)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          if (live == 1) finish2(out, a, r, h, d + 2 * y, make_float2(o[x][2 * y], o[x][2 * y + 1]), factor);
+          else publish2(mine + c * VD + d + 2 * y, o[x][2 * y], o[x][2 * y + 1]);
         }
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      u32x4 part[3];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const float p0 = st[2 * j + (x >> 1)][2 * (x & 1)], p1 = st[2 * j + (x >> 1)][2 * (x & 1) + 1];
-        const float q0 = below_upper(p0), q1 = below_upper(p1);
-        part[0][x] = upper2(p0, p1), part[1][x] = upper2(q0, q1), part[2][x] = upper2(below_upper(q0), below_upper(q1));
-      }
-#pragma unroll
-      for (int i3 = 2; i3 >= 0; --i3)
-#pragma unroll
-        for (int dt = 0; dt < VT; ++dt)
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf[dt][j]), as_bf16x8(part[i3]), o[dt], 0, 0, 0);
-    }
-  }
-  // the wavefronts' results meet
-  l = across_sum(l);
-#pragma unroll
-  for (int dt = 0; dt < VT; ++dt)
-    if (16 * dt + 4 * g < VD && c < cols) *(f32x4*)(lds + (w * 16 + c) * row_floats + 16 * dt + 4 * g) = o[dt];
-  if (g == 0) lds_m[w][c] = m, lds_l[w][c] = l;
-  __syncthreads();
-  const long long at = (long long)r * gridDim.y + blockIdx.y;
-  float* mine = sh.part + (at * sh.splits + split) * hd.share_floats;
-  // A head's factors once for all of its entries; then four neighbouring entries at a time.  (Every entry on its own, with its
-  // maxima, exponentials, division and gate, and the row's slot asked for behind its sequence: eight rows of 200 to 730 keys, one key head of 256,
-  // 16 heads of 192 21.4 -> 18.2 us; of 520 keys, four key heads, two maps over values of 256 17.2 -> 15.7, of 128 13.0 -> 12.3; two rows of 1 000
-  // keys, capped scores, 16.4 -> 15.0.)
-  if (tid < cols) {
-    float M = lds_m[0][tid], L = 0.f;
-#pragma unroll
-    for (int j = 1; j < NW; ++j) M = fmaxf(M, lds_m[j][tid]);
-#pragma unroll
-    for (int j = 0; j < NW; ++j) {
-      const float f = __builtin_amdgcn_exp2f(lds_m[j][tid] - M);
-      factors[j][tid] = f, L = fmaf(f, lds_l[j][tid], L);
-    }
-    if (live == 1) factors[NW][tid] = head_factor(gate, gate_logit, L);
-    else publish(mine + cols * VD + tid, M), publish(mine + cols * VD + cols + tid, L);
-  }
-  float2 wide[2];  // (of the first four entries, when they are the result)
-#pragma unroll
-  for (int x = 0; x < 2; ++x) wide[x] = live == 1 ? wide_gate_of(a, r, hbase, min(4 * tid + 2 * x, cols * VD - 2)) : make_float2(0.f, 0.f);
-  __syncthreads();
-  for (int idx = 4 * tid; idx < cols * VD; idx += 4 * NW * 64) {
-    const int cc = idx / VD, d = idx - cc * VD;  // (VD is a multiple of 4)
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < NW; ++j) {
-      const f32x4 v = *(const f32x4*)(lds + (j * 16 + cc) * row_floats + d);
-      const float f = factors[j][cc];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum[e] = fmaf(f, v[e], sum[e]);
-    }
-#pragma unroll
-    for (int x = 0; x < 2; ++x) {
-      if (live == 1)
-        finish2(out, a, r, hbase, idx + 2 * x, make_float2(sum[2 * x], sum[2 * x + 1]), factors[NW][cc],
-                idx == 4 * tid ? wide[x] : wide_gate_of(a, r, hbase, idx + 2 * x));
-      else
-        publish2(mine + idx + 2 * x, sum[2 * x], sum[2 * x + 1]);
-    }
+    if (live > 1 && w == 0 && g == 0) publish2(mine + sh.heads * VD + 2 * c, m, l);
   }
   if (live == 1 || sh.tickets == nullptr) return;
   // Once every thread's stores have completed the workgroup takes a ticket; the last one adds the shares up.
@@ -360,27 +361,15 @@ __global__ __launch_bounds__(NW * 64, 16 * KS + 8 * VT <= 128 ? 2 : 1) void sink
     last = __hip_atomic_fetch_add(sh.tickets + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == live - 1;
   __syncthreads();
   if (!last) return;
-  add_shares(out, gate, gate_logit, a, sh, hd, live);
+  add_shares(out, gate, a, sh, hd, live);
   if (tid == 0) __hip_atomic_store(sh.tickets + at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
 }
 
 template <int KS, int VT>
 int launch(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache, const SinkArgs& a,
            const Shares& sh, dim3 grid, hipStream_t stream) {
-  const int bytes = NW * 16 * (a.VD + 4) * (int)sizeof(float);
-  const bool with_shape = scores_shaped(a.shape);
-  const auto kernel = with_shape ? sink_decode_kernel<KS, VT, true> : sink_decode_kernel<KS, VT, false>;
-  static bool configured[2] = {false, false};
-  if (!configured[with_shape]) {
-    const int most = NW * 16 * (16 * VT + 4) * (int)sizeof(float);
-    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, most);
-    if (e != hipSuccess) {
-      lq_set_error("sink_attention: cannot reserve %d bytes of LDS: %s", most, hipGetErrorString(e));
-      return -2;
-    }
-    configured[with_shape] = true;
-  }
-  kernel<<<grid, NW * 64, bytes, stream>>>(q, out, gate, kcache, vcache, a, sh);
+  if (scores_shaped(a.shape)) sink_decode_kernel<KS, VT, true><<<grid, NW * 64, 0, stream>>>(q, out, gate, kcache, vcache, a, sh);
+  else sink_decode_kernel<KS, VT, false><<<grid, NW * 64, 0, stream>>>(q, out, gate, kcache, vcache, a, sh);
   LQ_CHECK_LAUNCH("sink_attention(single tokens)");
   if (sh.splits > 1 && sh.tickets == nullptr) {
     sink_add_shares_kernel<<<dim3(grid.x, grid.y), NW * 64, 0, stream>>>(out, gate, a, sh);
@@ -389,17 +378,37 @@ int launch(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache,
   return 1;
 }
 
-// Shares of a row's keys: as many as give every wavefront one block of the `max_len` bound, within two rounds of
-// workgroups.
-int splits_for(int rows, int nh, int nkv, int window, int keep_first, int chunk, int max_len) {
-  if (max_len <= 0) return 1;
+// How a launch is shared out: `splits` is 1 where no row goes in shares.
+//
+// In units of the time for 32 KB (1.1 us): a block of KD + VD entries takes (KD + VD) / 256, a share more its ticket and its results'
+// way into the last workgroup, 0.06 + 0.07 for every 512 entries.  A row of up to 3.6 units stays whole (24 rows of 100 keys of
+// 256 + 192: 9.4 -> 8.7 us), else a share has the blocks that an even deal gives it and no fewer than the root of n times
+// the quotient of the two.
+//
+// Query heads a workgroup: 16 where rows are many; half as many, and half again, while that makes no more than 128 workgroups a
+// share, down to 4 (the last workgroup of a row then adds up a quarter: 8 rows of 216 to 716 keys 17.6 us with 16 heads, 13.7 with 8, 11.2 with 4), and
+// down to 2 while it makes no more than 32 (4 rows of 700 keys 12.1 -> 10.3, one 10.7 -> 9.2; with 64 of them 11.0 -> 12.0).
+Shares shares_for(int rows, int nh, int nkv, int KD, int VD, int window, int keep_first, int chunk, int max_len) {
+  Shares sh = {};
+  const int group = nh / nkv, cus = lq_compute_units();
+  const float block = (KD + VD) / 256.f;
+  auto tiles = [&](int heads) { return (long long)rows * nkv * lq_ceil_div(group, heads); };
+  int heads = 16;
+  while (max_len > 0 && ((heads > 4 && tiles(heads / 2) <= 128) || (heads > 2 && tiles(heads / 2) <= 32))) heads /= 2;
+  sh.heads = group < heads ? group : heads;
+  sh.tiles = lq_ceil_div(group, sh.heads);
+  sh.whole = 3.6f / block > 1.f ? (int)(3.6f / block) : 1;
+  sh.apart = (0.06f + 0.07f * sh.heads * VD / 512.f) / block;
+  sh.splits = sh.narrow = 1;
+  if (max_len <= 0) return sh;
   const long long seen = window > 0 ? (long long)window + keep_first + 2 * BLOCK : max_len;
   int keys = seen < max_len ? (int)seen : max_len;
   if (chunk > 0 && chunk + BLOCK < keys) keys = chunk + BLOCK;
-  const long long tiles = (long long)rows * nkv * lq_ceil_div(nh / nkv, 16);
-  const int wanted = lq_ceil_div(lq_ceil_div(keys, BLOCK) + 1, NW), room = (int)(2 * lq_compute_units() / tiles);
-  const int most = room > MAX_SPLITS ? MAX_SPLITS : room;
-  return wanted < most ? wanted : most > 1 ? most : 1;
+  const long long room = 2 * cus / tiles(heads), alone = cus / tiles(heads);
+  const int wanted = lq_ceil_div(keys, BLOCK) + 1, most = room > MAX_SPLITS ? MAX_SPLITS : (int)room;
+  sh.splits = wanted < most ? wanted : most > 1 ? most : 1;
+  sh.narrow = alone > sh.splits ? sh.splits : alone > 1 ? (int)alone : 1;
+  return sh;
 }
 
 bool takes(int KD, int VD, int block_size, int nh, int nkv, int rows) {
@@ -412,9 +421,9 @@ bool takes(int KD, int VD, int block_size, int nh, int nkv, int rows) {
 long long lq_sink_decode_workspace(int rows, int nh, int nkv, int KD, int VD, int block_size, int window, int keep_first,
                                    int chunk, int max_len) {
   if (!takes(KD, VD, block_size, nh, nkv, rows)) return 0;
-  const int splits = splits_for(rows, nh, nkv, window, keep_first, chunk, max_len), group = nh / nkv;
-  if (splits == 1) return 0;
-  return (long long)rows * nkv * lq_ceil_div(group, 16) * splits * (group < 16 ? group : 16) * (VD + 2);
+  const Shares sh = shares_for(rows, nh, nkv, KD, VD, window, keep_first, chunk, max_len);
+  if (sh.splits == 1) return 0;
+  return (long long)rows * nkv * sh.tiles * sh.splits * sh.heads * (VD + 2);
 }
 
 int lq_sink_decode(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache, const bf16_t* vcache,
@@ -423,14 +432,16 @@ int lq_sink_decode(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t*
   if (a.ldq % 4 != 0 || (uintptr_t)q % 8 != 0 || ((uintptr_t)kcache | (uintptr_t)vcache) % 16 != 0 ||
       !takes(a.KD, a.VD, a.BS, a.nh, a.nkv, a.rows))
     return 0;
-  const int tiles = a.nkv * lq_ceil_div(a.nh / a.nkv, 16);
-  Shares sh = {1, part, (long long)a.rows * tiles <= tickets_n ? tickets : nullptr};
-  if (part != nullptr && (uintptr_t)part % 8 == 0) {  // (shares are read in pairs)
-    const long long need = lq_sink_decode_workspace(a.rows, a.nh, a.nkv, a.KD, a.VD, a.BS, a.window, a.keep_first, a.chunk, max_len);
-    if (need > 0 && need <= part_floats) sh.splits = splits_for(a.rows, a.nh, a.nkv, a.window, a.keep_first, a.chunk, max_len);
-  }
-  const dim3 grid(a.rows, tiles, sh.splits);
-#define LQ_DECODE(KS, VT) launch<KS, VT>(q, out, gate, kcache, vcache, a, sh, grid, stream)
+  Shares sh = shares_for(a.rows, a.nh, a.nkv, a.KD, a.VD, a.window, a.keep_first, a.chunk, max_len);
+  const long long need = lq_sink_decode_workspace(a.rows, a.nh, a.nkv, a.KD, a.VD, a.BS, a.window, a.keep_first, a.chunk, max_len);
+  if (part == nullptr || need <= 0 || need > part_floats || (uintptr_t)part % 8 != 0)  // (shares are read in pairs)
+    sh = shares_for(a.rows, a.nh, a.nkv, a.KD, a.VD, a.window, a.keep_first, a.chunk, 0);
+  sh.part = part;
+  sh.tickets = (long long)a.rows * a.nkv * sh.tiles <= tickets_n ? tickets : nullptr;
+  SinkArgs b = a;
+  b.heads_per_tile = a.nh / a.nkv;  // (here: query heads a key head)
+  const dim3 grid(a.rows, a.nkv * sh.tiles, sh.splits);
+#define LQ_DECODE(KS, VT) launch<KS, VT>(q, out, gate, kcache, vcache, b, sh, grid, stream)
   if (a.KD <= 64 && a.VD <= 64) return LQ_DECODE(2, 4);
   if (a.KD <= 128 && a.VD <= 128) return LQ_DECODE(4, 8);
   if (a.KD <= 128) return LQ_DECODE(4, 16);

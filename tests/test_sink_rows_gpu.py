@@ -46,6 +46,15 @@ def test_single_tokens(H, G, D, P, options, shared):
     check(H, G, D, P, [(1, n - 1) for n in LENGTHS], options, shared)
 
 
+@pytest.mark.parametrize("lengths", [[1], [64, 65], [129], [700], [192, 193, 321], [4097]])
+@pytest.mark.parametrize("H,G,D,P,options", [(16, 1, 256, 192, PLAIN), (20, 1, 64, 40, dict(sinks=True, gate=True)), (3, 1, 128, 256, PLAIN),
+                                             (8, 2, 128, 128, dict(PLAIN, cap=5.0, dist=100, wide=True)),
+                                             (24, 1, 40, 72, dict(window=300, keep_first=130))])
+def test_single_tokens_of_few_rows(H, G, D, P, options, lengths):
+    """A key head's query heads in several workgroups, down to two heads each, and shares of one block upwards."""
+    check(H, G, D, P, [(1, n - 1) for n in lengths], options, True)
+
+
 @pytest.mark.parametrize("H,G,D,P,seqs,options", CASES)
 def test_tiles_of_32_rows(H, G, D, P, seqs, options):
     check(H, G, D, P, seqs, options, False)
