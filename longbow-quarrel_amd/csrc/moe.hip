@@ -87,20 +87,29 @@ constexpr int ROUTE_PER = 16;  // outputs a lane at most in the kernels below
 // the weights are the same to the bit.
 // A thread a row -> a wavefront a row, the same bits: 8 rows, 2 of 8 experts 8.1 -> 2.9 us; 8 rows, 4 of 16 in groups
 // with a softmax 29 -> 5.6; 8 rows, 8 of 64 in groups 220 -> 7.1; 2635 rows of 16 35.7 -> 6.3; 17 rows of 1024 1414 -> 45.
+struct RouteArgs {
+  float* route;
+  int E, top, renorm;
+  const float* correction;
+  int groups, keep, softmax, mark_max;
+  float renorm_eps;
+  float* ident;
+  int n_ident;
+};
+
+// Row r, whose logits are z[0 .. E), by one wavefront; `mine`: E floats of LDS for the choice scores, where groups are marked.
 template <int PER>
-__global__ __launch_bounds__(256) void moe_route_lanes_kernel(const float* __restrict__ z, int ldz, float* __restrict__ route,
-                                                              int rows, int E, int top, int renorm,
-                                                              const float* __restrict__ correction, int groups, int keep,
-                                                              int softmax, int mark_max, float renorm_eps,
-                                                              float* __restrict__ ident, int n_ident) {
-  extern __shared__ float lds[];  // [4][E]: a row's choice scores, where groups are marked
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (r >= rows) return;  // (a wavefront shares nothing with the others: no barrier below)
+__device__ inline void route_row(const float* z, float* mine, int r, const RouteArgs& a) {
+  const int lane = threadIdx.x & 63, E = a.E, top = a.top, renorm = a.renorm, groups = a.groups, keep = a.keep, n_ident = a.n_ident;
+  const int softmax = a.softmax, mark_max = a.mark_max;
+  const float renorm_eps = a.renorm_eps;
+  const float* correction = a.correction;
+  float *route = a.route, *ident = a.ident;
   float s[PER], v[PER];   // scores; what the choice goes by
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int e = lane + 64 * j;
-    s[j] = e < E ? z[(long long)r * ldz + e] : -INFINITY;
+    s[j] = e < E ? z[e] : -INFINITY;
   }
   if (softmax) {
     float zmax = -INFINITY, sum = 0.f;
@@ -155,7 +164,6 @@ __global__ __launch_bounds__(256) void moe_route_lanes_kernel(const float* __res
   for (int j = 0; j < PER; ++j)
     if (lane + 64 * j < E) from |= 1u << j;
   if (groups > 1 && keep < groups) {
-    float* mine = lds + (threadIdx.x >> 6) * E;
 #pragma unroll
     for (int j = 0; j < PER; ++j)
       if (lane + 64 * j < E) mine[lane + 64 * j] = v[j];
@@ -211,17 +219,24 @@ __global__ __launch_bounds__(256) void moe_route_lanes_kernel(const float* __res
   }
 }
 
+template <int PER>
+__global__ __launch_bounds__(256) void moe_route_lanes_kernel(const float* __restrict__ z, int ldz, int rows, RouteArgs a) {
+  extern __shared__ float lds[];  // [4][E]
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r < rows) route_row<PER>(z + (long long)r * ldz, lds + (threadIdx.x >> 6) * a.E, r, a);  // (a wavefront shares nothing with the others)
+}
+
 // The `top` largest logits win (the lower index on a tie) and the weights are the softmax over these alone.  A wavefront a
 // row: lane l has the logits l, l + 64, ...; every round finds the largest that is left.
-__global__ __launch_bounds__(256) void moe_route_chosen_kernel(const float* __restrict__ z, int ldz, float* __restrict__ route,
-                                                               int rows, int E, int top) {
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (r >= rows) return;
-  float v[ROUTE_PER], w[ROUTE_PER];
+template <int PER>
+__device__ inline void route_row_chosen(const float* z, int r, const RouteArgs& a) {
+  const int lane = threadIdx.x & 63, E = a.E, top = a.top;
+  float* route = a.route;
+  float v[PER], w[PER];
 #pragma unroll
-  for (int j = 0; j < ROUTE_PER; ++j) {
+  for (int j = 0; j < PER; ++j) {
     const int e = lane + 64 * j;
-    v[j] = e < E ? z[(long long)r * ldz + e] : -INFINITY;
+    v[j] = e < E ? z[e] : -INFINITY;
     if (v[j] != v[j]) v[j] = -INFINITY;
     w[j] = -1.f;
   }
@@ -230,7 +245,7 @@ __global__ __launch_bounds__(256) void moe_route_chosen_kernel(const float* __re
     float best = -INFINITY;
     int at = 0x7fffffff;  // the best's index: among equals, and where nothing is a number, the lowest that is left
 #pragma unroll
-    for (int j = 0; j < ROUTE_PER; ++j) {
+    for (int j = 0; j < PER; ++j) {
       const int e = lane + 64 * j;
       if (e < E && w[j] < 0.f && (at == 0x7fffffff || v[j] > best)) best = v[j], at = e;
     }
@@ -246,15 +261,52 @@ __global__ __launch_bounds__(256) void moe_route_chosen_kernel(const float* __re
     if (share != share) share = 0.f;
     sum += share;
 #pragma unroll
-    for (int j = 0; j < ROUTE_PER; ++j)
+    for (int j = 0; j < PER; ++j)
       if (lane + 64 * j == at) w[j] = share;
   }
   const float inv = sum > 0.f ? 1.f / sum : 0.f;
 #pragma unroll
-  for (int j = 0; j < ROUTE_PER; ++j) {
+  for (int j = 0; j < PER; ++j) {
     const int e = lane + 64 * j;
     if (e < E) route[(long long)r * E + e] = w[j] < 0.f ? -1.f : w[j] * inv;
   }
+}
+
+__global__ __launch_bounds__(256) void moe_route_chosen_kernel(const float* __restrict__ z, int ldz, int rows, RouteArgs a) {
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r < rows) route_row_chosen<ROUTE_PER>(z + (long long)r * ldz, r, a);
+}
+
+// Few rows: the router's product and the choice in one launch, a workgroup a row.  Wavefront w makes logits w, w + 16, ... of the N
+// (products of bfloat16, which are exact, in 32-bit sums), the first one chooses.  What bounds it is a launch's start and one trip for
+// the operands, which the two launches that this stands for (a product of one workgroup, then a wavefront a row) both had: replayed
+// steps of 8 rows of 2 048 over 8 experts take 2.5 us a layer less.
+constexpr int ROUTER_MOST = 64, ROUTER_WAVES = 16;
+__global__ __launch_bounds__(ROUTER_WAVES * 64) void moe_router_kernel(const bf16_t* __restrict__ h, int ldh, const bf16_t* __restrict__ w, int ldw,
+                                                                       float* __restrict__ z, int ldz, int K, int N, RouteArgs a) {
+  __shared__ float logits[ROUTER_MOST], choice[ROUTER_MOST];
+  const int r = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bf16_t* x = h + (long long)r * ldh;
+  for (int n = wave; n < N; n += ROUTER_WAVES) {
+    const bf16_t* y = w + (long long)n * ldw;
+    float sum[2] = {0.f, 0.f};
+#pragma unroll 4
+    for (int k = lane * 8; k < K; k += 512) {
+      const uint4 p = *(const uint4*)(x + k), q = *(const uint4*)(y + k);
+      const unsigned u[4] = {p.x, p.y, p.z, p.w}, v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sum[0] = fmaf(__uint_as_float(u[i] << 16), __uint_as_float(v[i] << 16), sum[0]);
+        sum[1] = fmaf(__uint_as_float(u[i] & 0xffff0000u), __uint_as_float(v[i] & 0xffff0000u), sum[1]);
+      }
+    }
+    const float all = wave_sum(sum[0] + sum[1]);
+    if (lane == 0) logits[n] = all, z[(long long)r * ldz + n] = all;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  if (a.softmax == 2) route_row_chosen<1>(logits, r, a);
+  else route_row<1>(logits, choice, r, a);
 }
 
 // out[r, :] += h[r, :] * (the sum of the row's chosen identity experts' weights); weights [rows, n] (-1: not chosen)
@@ -442,9 +494,9 @@ __global__ __launch_bounds__(256) void moe_scatter_kernel(const float* __restric
 
 // `experts` counts every output of the router, the `n_ident` identity experts at its end included: route is
 // [rows, experts - n_ident], ident [rows, n_ident] (null without identity experts).
-extern "C" int lq_moe_route(const float* z, int ldz, float* route, int rows, int experts, int top, int renormalize,
-                            const float* correction, int groups, int keep, int softmax, int mark_max, float renorm_eps,
-                            float* ident, int n_ident, hipStream_t stream) {
+// what the choice's options must be, whichever launch makes it
+static int check_route(int rows, int experts, int top, int ldz, const float* correction, int groups, int keep, int softmax, float renorm_eps,
+                       const float* ident, int n_ident) {
   LQ_REQUIRE(groups >= 0 && (groups <= 1 || (groups <= 64 && experts % groups == 0 && keep >= 1 && keep <= groups)),
              "moe_route: %d experts in %d groups of which %d are kept", experts, groups, keep);
   LQ_REQUIRE(rows > 0 && experts > 0 && top >= 1 && top <= experts && ldz >= experts, "moe_route: rows %d, %d of %d experts",
@@ -453,19 +505,25 @@ extern "C" int lq_moe_route(const float* z, int ldz, float* route, int rows, int
              "moe_route: a softmax over the chosen logits takes no correction, groups or identity experts");
   LQ_REQUIRE(n_ident >= 0 && n_ident < experts && (n_ident == 0 || ident != nullptr) && renorm_eps >= 0.f,
              "moe_route: %d identity experts of %d", n_ident, experts);
+  return 0;
+}
+
+extern "C" int lq_moe_route(const float* z, int ldz, float* route, int rows, int experts, int top, int renormalize,
+                            const float* correction, int groups, int keep, int softmax, int mark_max, float renorm_eps,
+                            float* ident, int n_ident, hipStream_t stream) {
+  const int rc = check_route(rows, experts, top, ldz, correction, groups, keep, softmax, renorm_eps, ident, n_ident);
+  if (rc != 0) return rc;
   LQ_REQUIRE(z && route, "moe_route: null pointer");
+  const RouteArgs a = {route, experts, top, renormalize, correction, groups, keep, softmax, mark_max, renorm_eps, ident, n_ident};
   if (softmax == 2) {
     LQ_REQUIRE(experts <= 64 * ROUTE_PER, "moe_route: %d experts (at most %d)", experts, 64 * ROUTE_PER);
-    moe_route_chosen_kernel<<<lq_ceil_div(rows, 4), 256, 0, stream>>>(z, ldz, route, rows, experts, top);
+    moe_route_chosen_kernel<<<lq_ceil_div(rows, 4), 256, 0, stream>>>(z, ldz, rows, a);
     LQ_CHECK_LAUNCH("moe_route(softmax over the chosen)");
     return 0;
   }
   // (up to 16 outputs a lane, as above; more would not stay in registers)
   const size_t lds = groups > 1 ? 4 * (size_t)experts * sizeof(float) : 0;
-#define LQ_ROUTE(PER)                                                                                                \
-  moe_route_lanes_kernel<PER><<<lq_ceil_div(rows, 4), 256, lds, stream>>>(z, ldz, route, rows, experts, top, renormalize, \
-                                                                          correction, groups, keep, softmax, mark_max,  \
-                                                                          renorm_eps, ident, n_ident)
+#define LQ_ROUTE(PER) moe_route_lanes_kernel<PER><<<lq_ceil_div(rows, 4), 256, lds, stream>>>(z, ldz, rows, a)
   if (experts <= 64) LQ_ROUTE(1);
   else if (experts <= 256) LQ_ROUTE(4);
   else if (experts <= 64 * ROUTE_PER) LQ_ROUTE(ROUTE_PER);
@@ -474,6 +532,27 @@ extern "C" int lq_moe_route(const float* z, int ldz, float* route, int rows, int
                                                                groups, keep, softmax, mark_max, renorm_eps, ident, n_ident);
 #undef LQ_ROUTE
   LQ_CHECK_LAUNCH("moe_route");
+  return 0;
+}
+
+// Whether lq_moe_router takes the router's product [rows, K] x [N, K]^T and the choice together.  Up to 16 rows: every row's workgroup
+// reads the whole weight, which for more of them the product reads once.
+extern "C" int lq_moe_router_takes(int dtype, int rows, int K, int N) {
+  return dtype == LQ_BF16 && rows >= 1 && rows <= 16 && K >= 8 && K % 8 == 0 && N >= 1 && N <= ROUTER_MOST;
+}
+
+// z[rows, N] = h . w^T, and lq_moe_route of z's first `experts` columns.
+extern "C" int lq_moe_router(const void* h, int ldh, const void* w, int ldw, float* z, int ldz, float* route, int dtype, int rows, int K,
+                             int N, int experts, int top, int renormalize, const float* correction, int groups, int keep, int softmax,
+                             int mark_max, float renorm_eps, float* ident, int n_ident, hipStream_t stream) {
+  LQ_REQUIRE(lq_moe_router_takes(dtype, rows, K, N) && N >= experts && ldz >= N, "moe_router: %d rows of %d, %d outputs are not taken", rows, K, N);
+  const int rc = check_route(rows, experts, top, ldz, correction, groups, keep, softmax, renorm_eps, ident, n_ident);
+  if (rc != 0) return rc;
+  LQ_REQUIRE(h && w && z && route, "moe_router: null pointer");
+  LQ_REQUIRE(ldh >= K && ldw >= K && ldh % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)h | (uintptr_t)w) % 16 == 0, "moe_router: rows must lie on 16 bytes");
+  const RouteArgs a = {route, experts, top, renormalize, correction, groups, keep, softmax, mark_max, renorm_eps, ident, n_ident};
+  moe_router_kernel<<<rows, ROUTER_WAVES * 64, 0, stream>>>((const bf16_t*)h, ldh, (const bf16_t*)w, ldw, z, ldz, K, N, a);
+  LQ_CHECK_LAUNCH("moe_router");
   return 0;
 }
 

@@ -1783,20 +1783,50 @@ class HipKernels:
         without tensors; their weights (-1: not chosen) go there and `route` is [rows, experts - n]."""
         rows, experts, ldz = self._mat(logits, "moe_route: logits")
         self._f32(logits, "moe_route: logits")
-        n_ident = 0
-        if identity is not None:
-            n_ident = identity.shape[-1]
-            self._f32(identity, "moe_route: identity", rows * n_ident)
-        how = {"sigmoid": 0, "softmax": 1, "softmax_chosen": 2}.get(scoring)
-        if how is None or group_mark not in ("top2", "max"):
-            raise KernelLibraryError(f"moe_route: scoring {scoring!r}, group_mark {group_mark!r}")
-        self._f32(route, "moe_route: route", rows * (experts - n_ident))
-        if correction is not None:
-            self._f32(correction, "moe_route: correction", experts)
+        n_ident, how = self._route_options("moe_route", rows, experts, route, correction, scoring, group_mark, identity)
         self._check(self.lib.lq_moe_route(_ptr(logits), c_int(ldz), _ptr(route), c_int(rows), c_int(experts), c_int(top),
                                           c_int(1 if renormalize else 0), _ptr(correction), c_int(groups), c_int(keep),
                                           c_int(how), c_int(1 if group_mark == "max" else 0),
                                           c_float(renormalize_eps), _ptr(identity), c_int(n_ident), self.stream))
+
+    def _route_options(self, what: str, rows: int, experts: int, route, correction, scoring: str, group_mark: str, identity):
+        """-> (identity experts, the scoring's number)"""
+        n_ident = 0
+        if identity is not None:
+            n_ident = identity.shape[-1]
+            self._f32(identity, f"{what}: identity", rows * n_ident)
+        how = {"sigmoid": 0, "softmax": 1, "softmax_chosen": 2}.get(scoring)
+        if how is None or group_mark not in ("top2", "max"):
+            raise KernelLibraryError(f"{what}: scoring {scoring!r}, group_mark {group_mark!r}")
+        self._f32(route, f"{what}: route", rows * (experts - n_ident))
+        if correction is not None:
+            self._f32(correction, f"{what}: correction", experts)
+        return n_ident, how
+
+    @query
+    def moe_router_takes(self, dtype: torch.dtype, rows: int, width: int, outputs: int) -> bool:
+        """Whether `moe_router` takes a router of so many outputs over so few rows."""
+        if self.force_generic or dtype not in _DTYPE_CODE:
+            return False
+        return bool(self.lib.lq_moe_router_takes(c_int(_DTYPE_CODE[dtype]), c_int(rows), c_int(width), c_int(outputs)))
+
+    def moe_router(self, h: torch.Tensor, w: torch.Tensor, logits: torch.Tensor, experts: int, route: torch.Tensor, top: int,
+                   renormalize: bool = False, correction: Optional[torch.Tensor] = None, groups: int = 0, keep: int = 0,
+                   scoring: str = "sigmoid", group_mark: str = "top2", renormalize_eps: float = 0.0,
+                   identity: Optional[torch.Tensor] = None) -> None:
+        """`linear` of h and the router w into `logits`, and `moe_route` of its first `experts` columns, in one launch
+        (where `moe_router_takes` the sizes; rows of h and w on 16 bytes)."""
+        self._dev(h, w, logits, route, correction, identity)
+        rows, n, ldz = self._mat(logits, "moe_router: logits")
+        self._f32(logits, "moe_router: logits")
+        if h.dtype != w.dtype or h.shape[0] != rows or w.shape[0] != n or h.shape[1] != w.shape[1] or not 1 <= experts <= n:
+            raise KernelLibraryError("moe_router: h, the weight and the logits do not belong together")
+        n_ident, how = self._route_options("moe_router", rows, experts, route, correction, scoring, group_mark, identity)
+        self._check(self.lib.lq_moe_router(_ptr(h), c_int(self._rows2d(h, "h")), _ptr(w), c_int(self._rows2d(w, "w")), _ptr(logits), c_int(ldz),
+                                           _ptr(route), c_int(_code(h)), c_int(rows), c_int(h.shape[1]), c_int(n), c_int(experts), c_int(top),
+                                           c_int(1 if renormalize else 0), _ptr(correction), c_int(groups), c_int(keep),
+                                           c_int(how), c_int(1 if group_mark == "max" else 0),
+                                           c_float(renormalize_eps), _ptr(identity), c_int(n_ident), self.stream))
 
     def moe_identity(self, h: torch.Tensor, weights: torch.Tensor, out: torch.Tensor) -> None:
         """out [rows, width] (float32) += h * (the sum of the row's entries of `weights` [rows, n] that are not

@@ -90,3 +90,29 @@ def test_choice_and_weights(kn, E, top, groups, keep, ident, softmax):
             assert torch.equal(got[r] >= 0, w >= 0), (r, by_max)
             # a score: exp, an addition or a sum of E terms, a division; then a sum of `top` and a division more
             assert torch.allclose(got[r].double(), w, rtol=(E + top + 8) * 2.0 ** -24, atol=1e-30), (r, by_max)
+
+
+@pytest.mark.parametrize("rows,K,E,extra", [(1, 8, 1, 0), (3, 520, 8, 1), (8, 2048, 8, 0), (16, 4096, 17, 0), (5, 1000, 63, 1), (2, 256, 64, 0)])
+@pytest.mark.parametrize("scoring", ["sigmoid", "softmax", "softmax_chosen"])
+def test_the_product_and_the_choice_in_one_launch(kn, rows, K, E, extra, scoring):
+    """Its logits against 64 bits, and the choice that `moe_route` makes of them, bit for bit; rows apart by more than K."""
+    gen = torch.Generator(device="cuda").manual_seed(rows + K + E)
+    h, w = (torch.randn(n, K + 8, generator=gen, device="cuda").bfloat16()[:, :K] for n in (rows, E + extra))
+    assert kn.moe_router_takes(torch.bfloat16, rows, K, E + extra) and not kn.moe_router_takes(torch.float32, rows, K, E)
+    options = dict(scoring=scoring)
+    if scoring != "softmax_chosen" and E % 8 == 0:
+        options.update(correction=torch.randn(E, generator=gen, device="cuda"), groups=4, keep=2, renormalize_eps=1e-20,
+                       identity=torch.full((rows, 2), 7.0, device="cuda"))
+    R, top = E - (2 if "identity" in options else 0), min(E, 2)
+    z = torch.full((rows, E + extra + 3), 7.0, device="cuda")
+    route, want = (torch.full((rows, R), 7.0, device="cuda") for _ in range(2))
+    kn.moe_router(h, w, z[:, : E + extra], E, route, top, True, **options)
+    assert bool((z[:, E + extra :] == 7).all())
+    # K exact products of bfloat16, in any order: at most K roundings of 2^-24 of their absolute sum
+    exact, terms = h.double() @ w.double().T, h.double().abs() @ w.double().abs().T
+    assert bool(((z[:, : E + extra] - exact).abs() <= K * 2.0 ** -24 * terms).all())
+    passed = options.pop("identity", None)
+    if passed is not None:
+        options["identity"] = torch.empty_like(passed)
+    kn.moe_route(z[:, :E], want, top, True, **options)
+    assert torch.equal(route, want) and (passed is None or torch.equal(passed, options["identity"]))
