@@ -155,28 +155,41 @@ __global__ __launch_bounds__(256) void causal_conv4_kernel(const T* __restrict__
     for (int j = 0; j < TAPS; ++j) wt[e][j] = w[(long long)(c + e) * TAPS + j];
   float4 bv = make_float4(0.f, 0.f, 0.f, 0.f);
   if (bias != nullptr) bv = *(const float4*)(bias + c);
+  // A tile of several rows asks for all its inputs, those of the rows before it and the rows' sequences at once.  Two rows a thread:
+  // 2 048 rows of 4 096 channels 16.5 us (4.1 TB/s), with four 20.3, with eight 21.9 (too few wavefronts to hide the activation), and
+  // 24.7 when each of eight was asked for by itself, behind its sequence's slot.
+  constexpr bool TILE = ROWS > 1;
+  float4 in[TILE ? ROWS + TAPS - 1 : 1];
+  int seqs[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) seqs[i] = row_seq[min(first + i, rows - 1)];
+  if constexpr (TILE)
+#pragma unroll
+    for (int i = 0; i < ROWS + TAPS - 1; ++i) in[i] = load4<T>(x + (long long)min(max(first + i - (TAPS - 1), 0), rows - 1) * ldx + c);
   float4 hist[TAPS];  // hist[j]: the input TAPS - 1 - j tokens before the row; the last is the row's own
   int before = -1;    // the sequence that hist belongs to
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
     const int r = first + i;
     if (r >= rows) break;
-    const int b = row_seq[r];
-    const long long slot = (long long)seq_slot[b] * (TAPS - 1);
+    const int b = seqs[i];
     if (b != before) {  // a tile's first row, or another sequence's
       const int since = row_pos[r] - seq_start[b];  // rows of this step before this one, in its sequence
+      const long long slot = since < TAPS - 1 ? (long long)seq_slot[b] * (TAPS - 1) : 0;
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) {
         const int back = TAPS - 1 - j;
-        hist[j] = back <= since ? load4<T>(x + (long long)(r - back) * ldx + c)
-                                : *(const float4*)(state + (slot + TAPS - 1 - (back - since)) * C + c);
+        if (back > since) hist[j] = *(const float4*)(state + (slot + TAPS - 1 - (back - since)) * C + c);
+        else if constexpr (TILE) hist[j] = in[i + j];
+        else hist[j] = load4<T>(x + (long long)(r - back) * ldx + c);
       }
       before = b;
     } else {
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) hist[j] = hist[j + 1];
     }
-    hist[TAPS - 1] = load4<T>(x + (long long)r * ldx + c);
+    if constexpr (TILE) hist[TAPS - 1] = in[i + TAPS - 1];
+    else hist[TAPS - 1] = load4<T>(x + (long long)r * ldx + c);
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) {
@@ -187,6 +200,7 @@ __global__ __launch_bounds__(256) void causal_conv4_kernel(const T* __restrict__
     store4<T>(out + (long long)r * ldo + c,
               make_float4(activate(acc.x, act), activate(acc.y, act), activate(acc.z, act), activate(acc.w, act)));
     if (single) {
+      const long long slot = (long long)seq_slot[b] * (TAPS - 1);
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) *(float4*)(state + (slot + j) * C + c) = hist[j + 1];
     }
@@ -1028,6 +1042,47 @@ __global__ __launch_bounds__(256) void gated_rmsnorm4_kernel(const float* __rest
   }
 }
 
+// Many rows and groups of up to 4 LANES columns (128): LANES lanes a group and four rows a thread, all asked for together.
+// (A wavefront a row and group had at most two loads on their way a lane, and half of its lanes none where a group has 128:
+// 2 048 rows of 32 groups of 128 took 20.6 us, now 15.2.  Groups of 256 with 64 lanes took 12.9, a wavefront a row and
+// group 11.1: they stay there, and so do few rows, which a fourth of the wavefronts would not spread over the chip.)
+constexpr int GATED_ROWS = 4;
+template <typename T, int LANES>
+__global__ __launch_bounds__(256) void gated_rmsnorm_rows_kernel(const float* __restrict__ y, int ldy, const float* __restrict__ z,
+                                                                 int ldz, const float* __restrict__ w, int wlen, float eps,
+                                                                 int group, int groups, T* __restrict__ out, int ldo, int rows,
+                                                                 int gate_first, int sigmoid_gate) {
+  const int gi = blockIdx.x * (256 / LANES) + threadIdx.x / LANES, i = 4 * (threadIdx.x % LANES);
+  if (gi >= groups) return;  // (all lanes of a group)
+  const bool there = i < group;
+  const int c = gi * group + (there ? i : 0);
+  const long long r0 = (long long)blockIdx.y * GATED_ROWS;
+  float4 v[GATED_ROWS], g[GATED_ROWS];
+#pragma unroll
+  for (int j = 0; j < GATED_ROWS; ++j) {
+    const long long r = min(r0 + j, (long long)rows - 1);
+    v[j] = *(const float4*)(y + r * ldy + c), g[j] = *(const float4*)(z + r * ldz + c);
+  }
+  float4 wv = make_float4(1.f, 1.f, 1.f, 1.f);
+  if (w != nullptr) wv = *(const float4*)(w + (wlen >= groups * group ? c : (c - gi * group) % wlen));
+  auto gated = [&](float x) { return sigmoid_gate ? sigmoid_f(x) : silu_f(x); };
+#pragma unroll
+  for (int j = 0; j < GATED_ROWS; ++j) {
+    g[j].x = gated(g[j].x), g[j].y = gated(g[j].y), g[j].z = gated(g[j].z), g[j].w = gated(g[j].w);
+    if (gate_first) v[j].x *= g[j].x, v[j].y *= g[j].y, v[j].z *= g[j].z, v[j].w *= g[j].w;
+    const float ss = there ? fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, v[j].w * v[j].w))) : 0.f;
+    float sum = ss;  // (the sum of the kernel above, bit for bit)
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, LQ_WAVE);
+    const float inv = 1.f / sqrtf(sum / group + eps);
+    if (!there || r0 + j >= rows) continue;
+    float4 x = make_float4(v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv);
+    x.x *= wv.x, x.y *= wv.y, x.z *= wv.z, x.w *= wv.w;
+    if (!gate_first) x.x *= g[j].x, x.y *= g[j].y, x.z *= g[j].z, x.w *= g[j].w;
+    store4<T>(out + (r0 + j) * ldo + c, x);
+  }
+}
+
 struct MeanInputs {
   const float* x[4];
   const float* w[4];
@@ -1170,14 +1225,14 @@ static int launch_causal_conv(const T* x, int ldx, const float* w, const float* 
                      (uintptr_t)state % 16 == 0 && (uintptr_t)bias % 16 == 0;
   if (fours) {
     const bool single = rows == batch;  // (every sequence of a step brings at least one row)
-    const int per = rows >= 512 ? 8 : 1;
+    const int per = rows >= 512 ? 2 : 1;
     const dim3 grid(lq_ceil_div(C, 256), lq_ceil_div(rows, 4 * per)), block(64, 4);
 #define LQ_CONV4(TAPS, ROWS)                                                                                              \
   causal_conv4_kernel<T, TAPS, ROWS><<<grid, block, 0, stream>>>(x, ldx, w, bias, state, out, ldo, rows, C, row_seq,      \
                                                                  row_pos, seq_slot, seq_start, act, single ? 1 : 0)
 #define LQ_CONV4_TAPS(TAPS)           \
   do {                                \
-    if (per == 8) LQ_CONV4(TAPS, 8);  \
+    if (per > 1) LQ_CONV4(TAPS, 2);   \
     else LQ_CONV4(TAPS, 1);           \
   } while (0)
     if (taps == 2) LQ_CONV4_TAPS(2);
@@ -1415,6 +1470,16 @@ extern "C" int lq_gated_rmsnorm(const float* y, int ldy, const float* z, int ldz
   const bool fours = group % 4 == 0 && group <= 8192 && ldy % 4 == 0 && ldz % 4 == 0 && ldo % 4 == 0 && (w == nullptr || wlen % 4 == 0) &&
                      (uintptr_t)y % 16 == 0 && (uintptr_t)z % 16 == 0 && (uintptr_t)w % 16 == 0 &&
                      (uintptr_t)out % (4 * el) == 0 && (out_dtype == LQ_F32 || out_dtype == LQ_BF16);
+  if (fours && group <= 128 && rows >= 512 && rows <= 65535 * GATED_ROWS) {
+#define LQ_GATED_ROWS(T, LANES)                                                                                                    \
+  gated_rmsnorm_rows_kernel<T, LANES><<<dim3(lq_ceil_div(groups, 256 / LANES), lq_ceil_div(rows, GATED_ROWS)), 256, 0, stream>>>( \
+      y, ldy, z, ldz, w, wlen, eps, group, groups, (T*)out, ldo, rows, gate_first, sigmoid_gate)
+    if (out_dtype == LQ_F32) LQ_GATED_ROWS(float, 32);
+    else LQ_GATED_ROWS(bf16_t, 32);
+#undef LQ_GATED_ROWS
+    LQ_CHECK_LAUNCH("gated_rmsnorm(rows)");
+    return 0;
+  }
   for (int r0 = 0; fours && r0 < rows; r0 += 65535) {
     const int nr = rows - r0 < 65535 ? rows - r0 : 65535;
     const bool wave = group <= 512;

@@ -1,0 +1,73 @@
+"""Kernels that take many rows (512 and more) in tiles against the same kernels' paths for fewer rows: a row's sums
+are the same whatever tile it lies in, so every result is equal bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def kn():
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+    return HipKernels()
+
+
+def rnd(*shape, seed):
+    return torch.empty(shape).normal_(0, 1.0, generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+def i32(values):
+    return torch.tensor(list(values), dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("lengths", [(512,), (513, ), (1, 2, 1, 3, 505, 7, 1), (255, 256, 2, 1, 3)])
+def test_convolution_of_many_rows(kn, lengths, taps, dtype):
+    C, wide = 132, 140
+    rows, n = sum(lengths), len(lengths)
+    x = rnd(rows, wide, seed=1).to(dtype)[:, 4 : 4 + C]
+    w, b = rnd(C, taps, seed=2), rnd(C, seed=3)
+    first = rnd(n + 1, taps - 1, C, seed=4)
+    start = [0 if s % 2 else 11 for s in range(n)]  # (some go on after earlier tokens)
+    slot = [n - s for s in range(n)]
+
+    def run(state, out, lo, hi, at):  # the rows lo .. hi - 1 of every sequence that has them
+        live = [s for s in range(n) if lengths[s] > lo]
+        take = [min(hi, lengths[s]) - lo for s in live]
+        cu = [0]
+        for m in take:
+            cu.append(cu[-1] + m)
+        pick = torch.cat([torch.arange(at[s] + lo, at[s] + lo + m) for s, m in zip(live, take)]).to(DEV)
+        xs, one = (x, out) if len(pick) == rows else (x[pick], torch.zeros((len(pick), C), dtype=dtype, device=DEV))
+        kn.causal_conv(xs, w, b, state, one, i32(start[s] + lo + r for s, m in zip(live, take) for r in range(m)),
+                       i32(i for i, m in enumerate(take) for _ in range(m)), i32(slot[s] for s in live),
+                       i32(start[s] + lo for s in live), i32(start[s] + lo + m for s, m in zip(live, take)), i32(cu), len(live))
+        if one is not out:
+            out[pick] = one
+
+    at = [sum(lengths[:s]) for s in range(n)]
+    whole, parts = torch.zeros((rows, C), dtype=dtype, device=DEV), torch.zeros((rows, C), dtype=dtype, device=DEV)
+    sw, sp = first.clone(), first.clone()
+    run(sw, whole, 0, max(lengths), at)
+    for lo in range(0, max(lengths), 97):
+        run(sp, parts, lo, lo + 97, at)
+    assert torch.equal(whole, parts)
+    assert torch.equal(sw, sp)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [512, 514, 1025])
+@pytest.mark.parametrize("group,groups,wlen", [(128, 3, 384), (64, 17, 64), (4, 2, 8), (100, 9, 900), (128, 8, 0)])
+def test_gated_norms_of_many_rows(kn, group, groups, wlen, rows, dtype):
+    n = group * groups
+    y, z = rnd(rows, n + 8, seed=5)[:, 4 : 4 + n], rnd(rows, n, seed=6)
+    wt = rnd(wlen, seed=7) if wlen else None
+    y[5, 0], z[rows - 1, n - 1], y[rows - 2, 0] = float("nan"), float("-inf"), float("inf")
+    for gate, before in (("silu", True), ("silu", False), ("sigmoid", False)):
+        got, want = torch.zeros((rows, n), dtype=dtype, device=DEV), torch.zeros((rows, n), dtype=dtype, device=DEV)
+        kn.gated_rmsnorm(y, z, wt, 1e-5, group, got, gate_first=before, gate=gate)
+        for lo in range(0, rows, 300):
+            kn.gated_rmsnorm(y[lo : lo + 300], z[lo : lo + 300], wt, 1e-5, group, want[lo : lo + 300], gate_first=before, gate=gate)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(3.0), want.nan_to_num(3.0)), gate
