@@ -353,17 +353,41 @@ __device__ inline Walk walk_of(const DeltaArgs& a) {
   return {sequence_by_length(a.cu_rows, a.batch, rank), in % a.heads, in / a.heads * 16};
 }
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000);
+}
+// 16 bytes a lane of the tile `tile` (a constant) behind `at` floats of a part of the scratch
+__device__ __forceinline__ f32x4 load_frag(__amdgpu_buffer_rsrc_t from, int lane16, int at, int tile) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, lane16 + tile % 4 * FRAG * 4, (at + tile / 4 * 4 * FRAG) * 4, 0));
+}
+
+__device__ __forceinline__ f32x4& lane_of(f32x4 (&tile)[64], int lane16) { return *(f32x4*)((char*)tile + lane16); }
+
+template <bool CAREFUL>
+__device__ __forceinline__ f32x4 step4_diagonal(const f32x4& a, const f32x4& b, f32x4 c) {
+  if constexpr (CAREFUL) return step4_lower(a, b, c);
+  else return step4(a, b, c);
+}
+
 // One workgroup of eight wavefronts a (sequence, head, 16 columns of the values); wavefront w holds channels 16 w .. + 15
-// of the state.  A chunk: wavefronts 0 to 3 make 16 tokens of V - K~ S each and 4 to 7 of Q~ S; then 0 to 3 of U; then
-// all update the state and 4 to 7 add B U.  Tiles cross between wavefronts through LDS in lane order.  A chunk's
-// operands are asked for as soon as the chunk before has used theirs.
+// of the state.  A chunk: wavefronts 0 to 3 make 16 tokens of V - K~ S each and 4 to 7 of Q~ S; then 0 to 3 of U, while
+// 4 to 7 add B U of the chunk before to its results; then all update the state.  Tiles cross between wavefronts through
+// LDS in lane order.
+// What bounds a chunk is this chain: matrix instructions keep a SIMD for 1.5 us of its 2.55, the rest are the three crossings.
+// So the loads of the next chunk's operands go out between the products that free their registers, in the shadow of
+// the matrix instructions; B U, which no later chunk needs, waits until the wavefronts that make it would be idle; and the two
+// wavefronts of a SIMD share the triangles' tiles evenly.  (With the loads and B U each in a place of its own a chunk took 3.4 us.
+// A launch of 2 100 tokens, 128 workgroups, 113 us before and 85 now; 1 024 workgroups 159 and 124.  In half the
+// registers, two workgroups a compute unit, the latter took 118, but 384 workgroups, of which the longest 256
+// had a compute unit each, 87 instead of 71.)
 __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
-  __shared__ f32x4 Ss[NT][64], Ws[KT][64], Us[KT][64];
+  __shared__ f32x4 Ss[NT][64], Ws[KT][64], Us[2][KT][64];
   __shared__ int again;
   const Walk at = walk_of(a);
-  const int b = at.b, h = at.h, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int c = lane & 15, g = lane >> 4, p = at.p0 + c, mt = w & 3;
+  const int b = at.b, h = at.h, tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4, p = at.p0 + c;
   const bool second = w >= KT;  // Q~, B and the results
+  const int mt = second ? NT - 1 - w : w;  // (the two wavefronts of a SIMD have five tiles of T and B together)
   const long long r1 = a.cu_rows[b + 1];
   const int base = first_chunk(a.cu_rows, b, a.least), i0 = max(a.first - base, 0);
   const int chunks = min(chunks_of((int)(r1 - a.cu_rows[b]), a.least), a.last - base) - i0;  // from the sequence's i0th on
@@ -371,113 +395,138 @@ __global__ __launch_bounds__(512, 2) void delta_walk_kernel(DeltaArgs a) {
   const long long r0 = a.cu_rows[b] + (long long)i0 * CHUNK;
   const float* part = a.scratch + ((long long)(base + i0 - a.first) * a.heads + h) * PART;
   const long long step = (long long)a.heads * PART;
-  float* sp = a.state + (((long long)a.seq_slot[b] * a.heads + h) * a.P + min(p, a.P - 1)) * a.N;
   const bool live = p < a.P;
-  f32x4 S, rows[NT], tri[KT - 1], diag, upd[KT], V, decay;
-  auto ask_rows = [&](const float* from) {
-#pragma unroll
-    for (int nb = 0; nb < NT; ++nb)
-      rows[nb] = *(const f32x4*)(from + (second ? AT_QUERIES : AT_KEYS) + ((mt * NT + nb) * 64 + lane) * 4);
+  int lane16 = lane * 16;
+  const int row0 = SUB * mt + 4 * g, none = 0x7fffffff;  // (no buffer's offset: such a lane reads 0 and writes nothing)
+  const __amdgpu_buffer_rsrc_t state = buffer_of(a.state + ((long long)a.seq_slot[b] * a.heads + h) * a.P * a.N, a.P * a.N * 4);
+  const int n0 = 16 * w + 4 * g, at_state = live ? (p * a.N + n0) * 4 : none;
+  const int at_v = live ? (row0 * a.ldv + p) * 4 : none, at_out = live ? (row0 * a.ldo + p) * 4 : none;
+  f32x4 S, rows[NT], tri[KT - 1], diag, upd[KT], decay, Y = {0.f, 0.f, 0.f, 0.f};
+  f32x4 V = {0.f, 0.f, 0.f, 0.f};
+  // Every wavefront asks for as many tiles, whatever it needs and whether there is another chunk (a buffer of no bytes gives zeros and
+  // moves nothing): the compiler then knows how many loads are behind the one it waits for.
+  auto ask_rows = [&](int nb, int i) {
+    rows[nb] = load_frag(buffer_of(part + i * step, i < chunks ? PART * 4 : 0), lane16,
+                            (second ? AT_QUERIES : AT_KEYS) + mt * NT * FRAG, nb);
   };
-  auto ask_tri = [&](const float* from) {
+  auto ask_tri = [&](int i) {
+    const int at_tri = (second ? AT_B : AT_T) + mt * KT * FRAG, bytes = i < chunks ? PART * 4 : 0;
 #pragma unroll
-    for (int kb = 0; kb < KT - 1; ++kb)
-      if (kb < mt) tri[kb] = *(const f32x4*)(from + (second ? AT_B : AT_T) + ((mt * KT + kb) * 64 + lane) * 4);
-    diag = *(const f32x4*)(from + (second ? AT_B : AT_T) + ((mt * KT + mt) * 64 + lane) * 4);
+    for (int kb = 0; kb < KT - 1; ++kb) tri[kb] = load_frag(buffer_of(part + i * step, kb < mt ? bytes : 0), lane16, at_tri, kb);
+    diag = load_frag(buffer_of(part + i * step, bytes), lane16, at_tri + mt * FRAG, 0);
   };
-  auto ask_upd = [&](const float* from) {
+  auto ask_upd = [&](int kb, int i) {
+    upd[kb] = load_frag(buffer_of(part + i * step, i < chunks ? PART * 4 : 0), lane16, AT_UPDATE + w * KT * FRAG, kb);
+  };
+  auto ask_decay = [&](int i) {
+    const int bytes = i < chunks ? PART * 4 : 0;
+    decay = load_frag(buffer_of(part + i * step, bytes), 16 * g, AT_DECAY + 16 * w, 0);
+  };
+  // (a matrix's rows of a chunk, from its first row's first column of the head on)
+  auto ask_v = [&](int i) {
+    const long long c0 = r0 + (long long)i * CHUNK;
+    const int n = second || i >= chunks ? 0 : (int)min((long long)CHUNK, r1 - c0);
+    const __amdgpu_buffer_rsrc_t from = buffer_of(a.v + c0 * a.ldv + (long long)h * a.P, second || i >= chunks ? 0 : (CHUNK * a.ldv + a.P) * 4);
 #pragma unroll
-    for (int kb = 0; kb < KT; ++kb) upd[kb] = *(const f32x4*)(from + AT_UPDATE + ((w * KT + kb) * 64 + lane) * 4);
-    decay = *(const f32x4*)(from + AT_DECAY + 16 * w + 4 * g);
+    for (int e = 0; e < 4; ++e)
+      V[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, row0 < n - e ? at_v : none, e * a.ldv * 4, 0));
   };
-  auto ask_v = [&](long long c0) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const long long r = c0 + SUB * mt + 4 * g + e;
-      V[e] = live && r < r1 ? a.v[r * a.ldv + (long long)h * a.P + p] : 0.f;
-    }
-  };
-  // The triangular products' zeros are no matter until a token brings a NaN or an infinity (V - K~ S or U has one): then
+  // The triangular products' zeros are no matter until a token brings a NaN or an infinity (U has one): then
   // all is walked again, and none of them reaches an earlier token.  (A test of every chunk's operands ahead of those
   // products lay in the chain and took 0.5 of its 3.3 microseconds; this takes 171 for 168.6 microseconds of a whole launch
   // of 2 048 tokens.)
   if (tid == 0) again = 0;  // (barriers follow)
-  int careful = 0;
-  while (true) {
-    const float* from = part;
+  auto walk = [&](auto with_care) {
+    constexpr bool careful = decltype(with_care)::value;
     float odd = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int n = 16 * w + 4 * g + e;
-      S[e] = live && n < a.N ? sp[n] : 0.f;
-    }
-    Ss[w][lane] = S;
-    V = (f32x4){0.f, 0.f, 0.f, 0.f};
-    ask_rows(from), ask_tri(from), ask_upd(from);
-    if (!second) ask_v(r0);
+    for (int e = 0; e < 4; ++e) S[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(state, n0 < a.N - e ? at_state : none, 4 * e, 0));
+    lane_of(Ss[w], lane16) = S;
+#pragma unroll
+    for (int nb = 0; nb < NT; ++nb) ask_rows(nb, 0);
+    __builtin_amdgcn_sched_barrier(0);  // (the loop's first wait is for these: nothing that it need not wait for goes ahead of them)
+    ask_tri(0), ask_v(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kb = 0; kb < KT; ++kb) ask_upd(kb, 0);
+    ask_decay(0);
     lds_barrier();
-    for (int i = 0; i < chunks; ++i, from += step) {
-      const bool more = i + 1 < chunks;
+    auto finish = [&](int i) {  // B U on top of chunk i's results
+      f32x4 all[KT], own = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < KT - 1; ++kb) all[kb] = lane_of(Us[i & 1][kb], lane16);
+      all[KT - 1] = lane_of(Us[i & 1][mt], lane16);
+#pragma unroll
+      for (int kb = 0; kb < KT - 1; ++kb)
+        if (kb < mt) own = step4(tri[kb], all[kb], own);
+      own = step4_diagonal<careful>(diag, all[KT - 1], own);
+      const f32x4 whole = Y + own;
       const long long c0 = r0 + (long long)i * CHUNK;
+      const int n = i < 0 ? 0 : (int)min((long long)CHUNK, r1 - c0);
+      const __amdgpu_buffer_rsrc_t to = buffer_of(a.out + c0 * a.ldo + (long long)h * a.P, i < 0 ? 0 : (CHUNK * a.ldo + a.P) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(whole[e]), to, row0 < n - e ? at_out : none, e * a.ldo * 4, 0);
+    };
+#pragma unroll 1
+    for (int i = 0; i < chunks; ++i) {
+      const int u = i & 1;
+      asm volatile("" : "+v"(lane16));  // (or the loads' offsets, lane16 and a constant each, stay in registers of their own)
       f32x4 acc[4];  // (four chains of products: their roundings are smaller, and none waits for the one before it)
 #pragma unroll
       for (int x = 0; x < 4; ++x) acc[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      f32x4 from[NT];
 #pragma unroll
-      for (int nb = 0; nb < NT; ++nb) acc[nb & 3] = step4(rows[nb], Ss[nb][lane], acc[nb & 3]);
-      f32x4 Y = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-      if (more) ask_rows(from + step);
+      for (int nb = 0; nb < NT; ++nb) from[nb] = lane_of(Ss[nb], lane16);
+#pragma unroll
+      for (int nb = 0; nb < NT; ++nb) {
+        acc[nb & 3] = step4(rows[nb], from[nb], acc[nb & 3]);
+        ask_rows(nb, i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const f32x4 next = (acc[0] + acc[1]) + (acc[2] + acc[3]);
       if (!second) {
-        const f32x4 W = V - Y;
-        Ws[mt][lane] = W;
-        odd = not_finite(W, odd);
-        if (more) ask_v(c0 + CHUNK);
+        lane_of(Ws[mt], lane16) = V - next;
       }
       lds_barrier();
       if (!second) {
-        f32x4 U = {0.f, 0.f, 0.f, 0.f};
+        f32x4 all[KT], U = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < KT - 1; ++kb) all[kb] = lane_of(Ws[kb], lane16);
+        all[KT - 1] = lane_of(Ws[mt], lane16);
 #pragma unroll
         for (int kb = 0; kb < KT - 1; ++kb)
-          if (kb < mt) U = step4(tri[kb], Ws[kb][lane], U);
-        U = careful ? step4_lower(diag, Ws[mt][lane], U) : step4(diag, Ws[mt][lane], U);
-        Us[mt][lane] = U;
-        odd = not_finite(U, odd);
-        if (more) ask_tri(from + step);
+          if (kb < mt) U = step4(tri[kb], all[kb], U);
+        U = step4_diagonal<careful>(diag, all[KT - 1], U);
+        lane_of(Us[u][mt], lane16) = U;
+        odd = not_finite(U, odd);  // (a token's V - K~ S that is not finite leaves its U so too, whatever stands on T's diagonal)
+      } else {
+        finish(i - 1);
+        Y = next;
       }
+      ask_tri(second ? i : i + 1), ask_v(i + 1);
       lds_barrier();
       // (what the chunk adds is summed by itself: one rounding at the state's size a chunk, not one a product)
       f32x4 add[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int kb = 0; kb < KT; ++kb) add[kb & 1] = step4(upd[kb], Us[kb][lane], add[kb & 1]);
-      S = S * decay + (add[0] + add[1]);
-      Ss[w][lane] = S;
-      if (more) ask_upd(from + step);
-      if (second) {
-        f32x4 own = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = 0; kb < KT - 1; ++kb)
-          if (kb < mt) own = step4(tri[kb], Us[kb][lane], own);
-        own = careful ? step4_lower(diag, Us[mt][lane], own) : step4(diag, Us[mt][lane], own);
-        Y += own;
-        if (more) ask_tri(from + step);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const long long r = c0 + SUB * mt + 4 * g + e;
-          if (live && r < r1) a.out[r * a.ldo + (long long)h * a.P + p] = Y[e];
-        }
+      for (int kb = 0; kb < KT; ++kb) {
+        add[kb & 1] = step4(upd[kb], lane_of(Us[u][kb], lane16), add[kb & 1]);
+        ask_upd(kb, i + 1);
       }
+      S = S * decay + (add[0] + add[1]);
+      ask_decay(i + 1);
+      lane_of(Ss[w], lane16) = S;
       lds_barrier();
     }
-    if (careful) break;
-    if (odd != odd) again = 1;
-    lds_barrier();  // (no wait for the results' stores)
-    careful = __builtin_amdgcn_readfirstlane(again);
-    if (!careful) break;
-  }
+    if (second) finish(chunks - 1);
+    return odd;
+  };
+  const float odd = walk(std::false_type{});
+  if (odd != odd) again = 1;
+  lds_barrier();  // (no wait for the results' stores)
+  if (__builtin_amdgcn_readfirstlane(again)) walk(std::true_type{});
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int n = 16 * w + 4 * g + e;
-    if (live && n < a.N) sp[n] = S[e];
-  }
+  for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(S[e]), state, n0 < a.N - e ? at_state : none, 4 * e, 0);
 }
 
 // The walk of gated linear attention, U = V:  O = Q~ S + B V;  S <- diag(p_64) S + sum_s (f_s,64 k_s) v_s^T.  One workgroup of eight
@@ -614,6 +663,7 @@ extern "C" long long lq_delta_scan_least(int heads) { return (long long)heads * 
 // chunks, 16 heads of 128 x 128: a decay a head, 70 sequences of 64 tokens 306 / 418, of 200 845 / 1 163, 16 of 100
 // 126 / 151, eight of 512 267 / 215, one of 256 89 / 44; a decay a channel, 16 of 64 171 / 112, 70 of 200 2 037 / 1 249;
 // of 64 x 64, 16 of 128 74 / 107.
+// (Of a walk over chunks of 3.4 microseconds each; it takes 2.55 now, so that the line leaves some launches near it token by token.)
 extern "C" int lq_delta_scan_in_chunks(int rows, int batch, int heads, int Dk, int P, int max_rows, int channel_decay) {
   if (lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) == 0) return 0;
   const double size = P / 128.0 * (Dk > 64 ? Dk / 128.0 : 0.4), cols = (P + 15) / 16;

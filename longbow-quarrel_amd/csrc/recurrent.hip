@@ -1415,7 +1415,9 @@ extern "C" int lq_delta_scan(float* q, int ldq, float* k, int ldk, const float* 
   unit_heads_kernel<<<dim3((unsigned)rows, kv_heads), 64, 0, stream>>>(q, ldq, k, ldk, Dk, q_scale, unit_eps);
   LQ_CHECK_LAUNCH("delta_scan(unit vectors)");
   int below = 0x7fffffff;  // sequences of fewer rows are walked token by token
-  const long long need = scratch != nullptr ? lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) : 0;
+  // (a chunk's rows of v and out are reached by 32-bit offsets)
+  const bool near_rows = ldv < (1 << 22) && ldo < (1 << 22);
+  const long long need = scratch != nullptr && near_rows ? lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) : 0;
   if (need > 0) {
     LQ_REQUIRE(lq_delta_scan_least(heads) <= scratch_floats && ((uintptr_t)scratch & 15) == 0,
                "delta_scan: %lld floats of aligned scratch for a launch in chunks, %lld given", lq_delta_scan_least(heads),

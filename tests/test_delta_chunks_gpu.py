@@ -101,6 +101,37 @@ def test_rounds_of_chunks_make_the_same_bits(lens, chunks):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("lens", [[64], [65], [128], [129, 191, 64], [70, 320]])
+@pytest.mark.parametrize("N,P", [(128, 16), (44, 36), (4, 3)])
+def test_the_walk_over_chunks_keeps_to_its_columns(lens, N, P):
+    """Values and results that are columns of wider matrices, odd and even numbers of chunks, heads' values that end inside
+    a tile of 16 columns: the bits of dense matrices, and nothing beside them is read or written."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    gen = torch.Generator().manual_seed(N + P)
+    rand = lambda *s: torch.randn(*s, generator=gen).cuda()
+    i32 = lambda v: torch.tensor(list(v), dtype=torch.int32, device="cuda")
+    rows, batch, H = sum(lens), len(lens), 3
+    q, k, beta, a = rand(rows, H * N), rand(rows, H * N), rand(rows, H), 0.3 * rand(rows, H)
+    dt_bias, a_log, state = rand(H) - 3.0, 0.5 * rand(H) + 1.0, rand(batch, H, P, N)
+    kn = HipKernels()
+    scratch = torch.full((kn.delta_scan_workspace(rows, batch, H, N, P, max(lens)),), float("nan"), device="cuda")
+    v, got = rand(rows, H * P), []
+    for extra in (0, 5):
+        wide = torch.full((rows + 64, H * P + 2 * extra), float("nan"), device="cuda")
+        wide[:rows, extra : extra + H * P] = v
+        out, end = torch.full_like(wide, 7.0), state.clone()
+        cut = lambda m: m[:rows, extra : extra + H * P]
+        kn.delta_scan(q.clone(), k.clone(), cut(wide), beta, a, dt_bias, a_log, end, cut(out), H, H, N, P, N ** -0.5, 1e-6,
+                      i32(range(batch)), i32(sum(lens[:b]) for b in range(batch + 1)), batch, channel_decay=False,
+                      max_rows=max(lens), workspace=scratch)
+        got.append((cut(out).clone(), end))
+        cut(out).fill_(7.0)
+        assert (out == 7.0).all()
+    for dense, apart in zip(*got):
+        assert torch.isfinite(dense).all() and torch.equal(dense, apart)
+
+
 def test_scratch_is_bounded():
     from longbow_quarrel_amd.kernels.hip import HipKernels
 
