@@ -10,7 +10,7 @@
 // Microseconds for a mixture's two products and the activation, every row through all experts -> this; 8 experts of 3 584 and width
 // 2 048, two of them a row: 1 row 77 -> 21, 4 rows (7 experts chosen) 76 -> 62, 8 rows 80 -> 66, 16 rows 152 -> 76; of 7 168 and
 // width 4 096: 1 row 239 -> 70, 8 rows 248 -> 225, 16 rows 370 -> 272; of 1 792 and width 1 024: 33 -> 12, 38 -> 22, 44 -> 27.  The
-// first product streams its weights at 5.0 to 6.3 TB/s from 4 rows on, the second at 6 (at 4.0 to 4.8 when these times were taken).
+// products stream their weights at 5.7 to 6 TB/s from 4 rows on (the second at 4.0 to 4.8 when these times were taken).
 //
 // What a row's result is made of does not depend on the other rows' choices: an expert's columns are sums over the same shares
 // of K whichever block takes them, a wavefront of the second product takes chunk i of the whole matrix's k where i % 16 is its
@@ -33,15 +33,8 @@ __device__ inline f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// A weight is read once a launch.  Packed ones are marked as a stream (nt), so that the caches keep the activations, the code and
-// what the products around these read instead: 33 tokens of eight sequences of Vupelorn 40.7 -> 39.7 ms, 17 of Sofinex 24.8 -> 24.2 (the
-// first product's mark alone 41.2 and 24.7, the second's 41.0 and 24.8).  A dense row's two halves of a line are asked for further
-// apart, and marked they would come twice.
-template <bool PACKED>
-__device__ inline u32x4 load_weight(const bf16_t* p) {
-  if constexpr (PACKED) return __builtin_nontemporal_load((const u32x4*)p);
-  else return *(const u32x4*)p;
-}
+// A weight is read once a launch, in whole lines through LDS, and marked as a stream (nt), so that the caches keep the activations, the
+// code and what the products around these read instead: 33 tokens of eight sequences of Vupelorn 40.7 -> 39.7 ms, 17 of Sofinex 24.8 -> 24.2.
 
 struct Experts {
   const float* route;  // [rows][n]: an expert's weight, or -1
@@ -80,91 +73,96 @@ struct FirstArgs {
 
 // act[row][column] of every chosen expert's columns and the shared one's (others are left as they are), bfloat16; W's rows are
 // expert by expert the gate's ff and the up matrix's ff (`GATED`), or the up matrix's alone.
-// A unit is 16 columns of an expert: a tile of 16 weight rows, with a gate two.  The units are dealt out evenly over the
-// workgroups, the 16 wavefronts of which own a share of K each and keep their rows of x in registers; the weights of the tile
-// after are asked for before a tile is multiplied, across the barriers at which up to 8 tiles' partial sums meet in LDS.
-// XS: steps of 32 k that a wavefront owns at most.
-template <int XS, bool GATED, bool PACKED>
+// A unit is a tile of 16 weight rows: 16 columns of an expert, or with a gate 8, their gate rows and their up rows.  The units
+// are dealt out evenly over the workgroups, the 16 wavefronts of which own a share of K each and keep their rows of x in
+// registers.  The weights come through LDS as in the second product: a wavefront has three slots of its own, 16 rows of 64 k,
+// filled by two transfers of whole lines; a slot is waited for, read, and asked for anew, across tiles and units, so that two
+// and more are always on their way (64 KiB a compute unit).  After every two tiles the wavefronts' partial sums meet in LDS,
+// where eight of them, in turn, finish a fourth of a unit each while the rest go on: the barrier behind lies ahead of the next
+// two tiles' sums.
+// What bounds it: the memory, and the round trip to the routing table ahead of the first weight.  8 rows that choose 7 of 8 experts of
+// 3 584, width 2 048 (205 MB) 35.8 us, 5.7 TB/s; with units of 16 columns of a gated expert, 6 or 7 a workgroup instead of 12 or
+// 13, 36.4; with fragments loaded into registers, half lines of 16 rows, two tiles ahead, and all wavefronts waiting for the end of
+// every eight tiles, 40.9.
+// SLABS: 64s of k that a wavefront owns at most.
+constexpr int SLOTS1 = 3, SLOT = 2048;
+
+__device__ __forceinline__ void lds_meet() { asm volatile("s_waitcnt lgkmcnt(0)\ns_barrier" ::: "memory"); }  // (transfers go on)
+
+template <int SLABS, bool GATED>
 __global__ __launch_bounds__(THREADS) void moe_few_first_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ W,
-                                                                int ldw, bf16_t* __restrict__ act, int ldo, int K, int ks_per_wave,
-                                                                FirstArgs a) {
-  constexpr int PARTS = GATED ? 2 : 1, TILES = 8, UNITS = TILES / PARTS;  // tiles and units between two barriers
-  constexpr int GT = 8 / XS;                                             // tiles asked for together
-  extern __shared__ __attribute__((aligned(16))) float red[];            // [TILES][KW][256]
-  __shared__ float route_sh[ROWS * EXPERTS], gate_sh[ROWS];
+                                                                int ldw, int packed, bf16_t* __restrict__ act, int ldo, int K,
+                                                                int slabs_per_wave, FirstArgs a) {
+  constexpr int PARTS = GATED ? 2 : 1, COLS = 16 / PARTS, TILES = 2;  // columns a unit; units between two meetings
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];  // [KW][SLOTS1][SLOT]
+  __shared__ float red[TILES][KW][256], route_sh[ROWS * EXPERTS], gate_sh[ROWS];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
   const Experts& ex = a.ex;
 
-  const int k0 = wave * ks_per_wave * 32, k1 = min(K, k0 + ks_per_wave * 32);
+  const int s0 = wave * slabs_per_wave, slabs = max(0, min(K / 64, s0 + slabs_per_wave) - s0);
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  u32x4 xv[XS];
+  u32x4 xv[SLABS][2];
 #pragma unroll
-  for (int s = 0; s < XS; ++s) {
-    const int k = k0 + 32 * s + 8 * g;
-    xv[s] = k < k1 ? *(const u32x4*)(x + (long long)min(c16, ex.rows - 1) * ldx + k) : zero;
-  }
+  for (int s = 0; s < SLABS; ++s)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      xv[s][h] = s < slabs ? *(const u32x4*)(x + (long long)min(c16, ex.rows - 1) * ldx + (s0 + s) * 64 + 32 * h + 8 * g) : zero;
   if (tid < ex.rows * ex.n) route_sh[tid] = ex.route[tid];  // (rows * experts <= 1024 = the threads)
   if (a.shared_gate != nullptr && tid < ex.rows) gate_sh[tid] = sigmoid_f(a.shared_gate[(long long)tid * a.ld_gate]);
 
   const unsigned long long bits = chosen_experts(ex);
-  const int per = ex.ff / 16, of_experts = __popcll(bits) * per;
-  const long long units = of_experts + ex.shared / 16;
-  const int u0 = (int)(units * blockIdx.x / gridDim.x), u1 = (int)(units * (blockIdx.x + 1) / gridDim.x);
-  const int tiles = (u1 - u0) * PARTS;
+  const int per = ex.ff / COLS, of_experts = __popcll(bits) * per;
+  const long long units = of_experts + ex.shared / COLS;
+  const int u0 = (int)(units * blockIdx.x / gridDim.x), u1 = (int)(units * (blockIdx.x + 1) / gridDim.x), tiles = u1 - u0;
   if (tiles == 0) return;  // (the whole workgroup)
 
-  // a unit's first row of W (of its first part), the distance to its second part's, and its first column of act
+  // a unit's first row of W, the distance to its second eight rows, and its first column of act
   auto place = [&](int u, int& row, int& apart, int& col) {
     if (u < of_experts) {
-      const int e = nth_bit(bits, u / per), j = u % per * 16;
+      const int e = nth_bit(bits, u / per), j = u % per * COLS;
       row = e * PARTS * ex.ff + j, apart = ex.ff, col = e * ex.ff + j;
     } else {
-      const int j = (u - of_experts) * 16;
+      const int j = (u - of_experts) * COLS;
       row = ex.n * PARTS * ex.ff + j, apart = ex.shared, col = ex.n * ex.ff + j;
     }
+    if constexpr (!GATED) apart = 8;
   };
-  u32x4 wv[2][GT][XS];
-  auto ask = [&](int buf, int t0) {
+  const bf16_t* lane_at[2];  // this lane in a transfer of 8 rows: row lane / 8, the chunk that lies at position lane % 8
 #pragma unroll
-    for (int i = 0; i < GT; ++i) {
+  for (int q = 0; q < 2; ++q) {
+    const int row = lane >> 3, chunk = (lane & 7) ^ (4 * q + (row >> 1));
+    lane_at[q] = W + (packed ? row * 64 + (long long)s0 * 512 : (long long)row * ldw + s0 * 64) + chunk * 8;
+  }
+  unsigned char* mine = ring + wave * (SLOTS1 * SLOT);
+  int ask_tile = 0, ask_slab = 0;
+  long long ask_from = 0, ask_apart = 0;  // where the tile that is asked for begins, and its second eight rows behind that
+  auto ask = [&](int slot) {
+    if (ask_slab == 0) {
       int row, apart, col;
-      const int t = min(t0 + i, tiles - 1);
-      place(u0 + t / PARTS, row, apart, col);
-      const int n = row + (t % PARTS) * apart + c16;
-      const bf16_t* wp = PACKED ? W + (long long)(n >> 3) * 8 * ldw + (n & 7) * 64 + (long long)(k0 >> 6) * 512 + g * 8
-                                : W + (long long)n * ldw + k0 + g * 8;
-#pragma unroll
-      for (int s = 0; s < XS; ++s)
-        wv[buf][i][s] = k0 + 32 * s + 8 * g < k1 ? load_weight<PACKED>(wp + (PACKED ? (s >> 1) * 512 + (s & 1) * 32 : s * 32)) : zero;
+      place(u0 + ask_tile, row, apart, col);
+      ask_from = (long long)__builtin_amdgcn_readfirstlane(row) * ldw, ask_apart = (long long)apart * ldw;
     }
+    const long long from = ask_from + ask_slab * (packed ? 512 : 64);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(lane_at[q] + from + q * ask_apart),
+                                       (__attribute__((address_space(3))) void*)(mine + slot * SLOT + q * 1024), 16, 0, 2);
+    if (++ask_slab == slabs) ask_slab = 0, ++ask_tile;
   };
-  auto multiply = [&](int buf, int t0) {  // tiles t0 .. of the batch that starts at tile t0 / TILES * TILES
-#pragma unroll
-    for (int i = 0; i < GT; ++i) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < XS; ++s) acc = mfma(xv[s], wv[buf][i][s], acc);
-      float* to = red + ((t0 + i) % TILES * KW + wave) * 256 + lane;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) to[e * 64] = acc[e];
-    }
-  };
-  // a unit's values of four rows and 16 columns: the wavefronts' shares in their order, and the activation
+  // a unit's values of four rows: the wavefronts' shares in their order, and the activation
   auto finish = [&](int u, int e, int t) {
     int row, apart, col;
     place(u, row, apart, col);
-    float s[PARTS];
+    float s[2] = {0.f, 0.f};
 #pragma unroll
-    for (int p = 0; p < PARTS; ++p) {
-      s[p] = 0.f;
-#pragma unroll
-      for (int w = 0; w < KW; ++w) s[p] += red[((t + p) * KW + w) * 256 + e * 64 + lane];
-    }
+    for (int w = 0; w < KW; ++w) s[0] += red[t][w][e * 64 + lane];
+    if constexpr (GATED) s[1] = dpp_swap<0x128>(s[0]);  // (the up row's, eight lanes on)
+    if (c16 >= COLS) return;
     const int r = 4 * g + e;
     if (r >= ex.rows) return;
     float y = 0.f;
     if (u >= of_experts) {  // the shared expert
-      if constexpr (GATED) y = silu_f(s[0]) * (a.shared_gate != nullptr ? s[PARTS - 1] * gate_sh[r] : s[PARTS - 1]);
+      if constexpr (GATED) y = silu_f(s[0]) * (a.shared_gate != nullptr ? s[1] * gate_sh[r] : s[1]);
       else y = activate(s[0], ACT_RELU2);
     } else {
       const float w = route_sh[r * ex.n + col / ex.ff];
@@ -173,7 +171,7 @@ __global__ __launch_bounds__(THREADS) void moe_few_first_kernel(const bf16_t* __
           y = activate(s[0], ACT_RELU2) * w;
         } else {
           const float in = a.on_input ? w : 1.f;
-          float gate = s[0] * in, up = s[PARTS - 1] * in;
+          float gate = s[0] * in, up = s[1] * in;
           if (a.unit == UNIT_SILU) {
             y = silu_f(gate) * up;
           } else {
@@ -187,21 +185,48 @@ __global__ __launch_bounds__(THREADS) void moe_few_first_kernel(const bf16_t* __
     act[(long long)r * ldo + col + c16] = f32_to_bf16(y);
   };
 
-  ask(0, 0);
-  for (int b0 = 0; b0 < tiles; b0 += TILES) {  // a batch; TILES / GT is even, so a batch starts with buffer 0
+  int left = slabs * tiles, slot = 0;  // slots' worth of weights that are not read yet
 #pragma unroll
-    for (int i = 0; i < TILES / GT; ++i) {
-      const int t = b0 + i * GT;
-      if (t < tiles) {
-        if (t + GT < tiles) ask((i + 1) & 1, t + GT);
-        __builtin_amdgcn_sched_barrier(0);  // (the next tiles' weights are asked for ahead of these products)
-        multiply(i & 1, t);
-      }
+  for (int i = 0; i < SLOTS1; ++i)
+    if (i < left) ask(i);
+  int frag[2];  // this lane's 16 bytes of a slot's 32-k halves
+#pragma unroll
+  for (int h = 0; h < 2; ++h) frag[h] = c16 * 128 + (((4 * h + g) ^ (c16 >> 1)) & 7) * 16;
+  for (int b0 = 0; b0 < tiles; b0 += TILES) {
+    f32x4 acc[TILES];
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+      acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if (b0 + i < tiles)
+#pragma unroll
+        for (int s = 0; s < SLABS; ++s)
+          if (s < slabs) {
+            // the oldest slot's transfers have landed: the two of each slot asked for after it may still fly (what a unit's end stored
+            // since makes the wait longer, never shorter)
+            if (left >= SLOTS1) __builtin_amdgcn_s_waitcnt(0x0F70 | 2 * (SLOTS1 - 1));
+            else if (left == 2) __builtin_amdgcn_s_waitcnt(0x0F72);
+            else __builtin_amdgcn_s_waitcnt(0x0F70);
+            __builtin_amdgcn_sched_barrier(0);
+            u32x4 wv[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) wv[h] = *(const u32x4*)(mine + slot * SLOT + frag[h]);
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot has been read
+            __builtin_amdgcn_sched_barrier(0);
+            if (left > SLOTS1) ask(slot);
+            --left;
+            slot = slot == SLOTS1 - 1 ? 0 : slot + 1;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) acc[i] = mfma(xv[s][h], wv[h], acc[i]);
+          }
     }
-    __syncthreads();
-    for (int j = wave; j < 4 * UNITS; j += KW)
-      if (b0 + (j >> 2) * PARTS < tiles) finish(u0 + b0 / PARTS + (j >> 2), j & 3, (j >> 2) * PARTS);
-    __syncthreads();
+    if (b0 > 0) lds_meet();  // the sums before have been read
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) red[i][wave][e * 64 + lane] = acc[i][e];
+    lds_meet();
+    const int j = (wave - 4 * b0) & (KW - 1);
+    if (j < 4 * TILES && b0 + (j >> 2) < tiles) finish(u0 + b0 + (j >> 2), j & 3, j >> 2);
   }
 }
 
@@ -217,7 +242,7 @@ __global__ __launch_bounds__(THREADS) void moe_few_first_kernel(const bf16_t* __
 // more rows, and experts that are not in 128s, take chunks of 64.
 // Position of 16-byte chunk c of a slot's row r: c ^ r / 2.  Behind a wavefront's last chunk transfers go on, out of the buffer's range,
 // until all slots are done: a wait then always counts the same number of them; such a slot takes part in no sum.
-constexpr int SLOTS = 4, SLOT = 2048, NOWHERE = (int)0x80000000u;  // (NOWHERE: an offset beyond every buffer)
+constexpr int SLOTS = 4, NOWHERE = (int)0x80000000u;  // (NOWHERE: an offset beyond every buffer)
 
 //
 // FAR: rows of the activations or of W beyond the reach of 32-bit offsets.  Everything goes by pointers then, rows that there are not
@@ -358,13 +383,13 @@ __global__ __launch_bounds__(THREADS) void moe_few_second_kernel(const bf16_t* _
   out[blockIdx.y * piece + (long long)r * ldo + n] = s + add;
 }
 
-int steps_per_wave(int K) { return (lq_ceil_div(lq_ceil_div(K, 32), KW) + 1) / 2 * 2; }
+int slabs_per_wave(int K) { return lq_ceil_div(K / 64, KW); }
 
-template <int XS, bool GATED, bool PACKED>
-int launch_first(const bf16_t* x, int ldx, const bf16_t* w, int ldw, bf16_t* act, int ldo, int K, const FirstArgs& a, int grid,
+template <int SLABS, bool GATED>
+int launch_first(const bf16_t* x, int ldx, const bf16_t* w, int ldw, int packed, bf16_t* act, int ldo, int K, const FirstArgs& a, int grid,
                  hipStream_t stream) {
-  const auto kernel = moe_few_first_kernel<XS, GATED, PACKED>;
-  constexpr int lds = 8 * KW * 256 * (int)sizeof(float);
+  const auto kernel = moe_few_first_kernel<SLABS, GATED>;
+  constexpr int lds = KW * SLOTS1 * SLOT;
   static bool configured = false;
   if (!configured) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -374,7 +399,7 @@ int launch_first(const bf16_t* x, int ldx, const bf16_t* w, int ldw, bf16_t* act
     }
     configured = true;
   }
-  kernel<<<grid, THREADS, lds, stream>>>(x, ldx, w, ldw, act, ldo, K, steps_per_wave(K), a);
+  kernel<<<grid, THREADS, lds, stream>>>(x, ldx, w, ldw, packed, act, ldo, K, slabs_per_wave(K), a);
   LQ_CHECK_LAUNCH("moe_few(first product)");
   return 0;
 }
@@ -406,15 +431,13 @@ extern "C" int lq_moe_few_first(const void* x, int ldx, const void* w, int ldw, 
              "moe_few: operands are not aligned");
   LQ_REQUIRE(shared_gate == nullptr || (shared > 0 && unit == UNIT_SILU && ld_gate >= 1), "moe_few: the shared expert's gate");
   const FirstArgs a = {{route, rows, experts, ff, shared}, shared_gate, ld_gate, unit, on_input, limit};
-  const long long units = ((long long)experts * ff + shared) / 16;
-  const int grid = units < lq_compute_units() ? (int)units : lq_compute_units(), gated = unit != UNIT_RELU2;
-#define LQ_FIRST(XS, GATED, PACKED) \
-  launch_first<XS, GATED, PACKED>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, (bf16_t*)act, ldo, width, a, grid, stream)
-  if (steps_per_wave(width) <= 4)
-    return gated ? (w_packed ? LQ_FIRST(4, true, true) : LQ_FIRST(4, true, false))
-                 : (w_packed ? LQ_FIRST(4, false, true) : LQ_FIRST(4, false, false));
-  return gated ? (w_packed ? LQ_FIRST(8, true, true) : LQ_FIRST(8, true, false))
-               : (w_packed ? LQ_FIRST(8, false, true) : LQ_FIRST(8, false, false));
+  const int gated = unit != UNIT_RELU2;
+  const long long units = ((long long)experts * ff + shared) / (gated ? 8 : 16);
+  const int grid = units < lq_compute_units() ? (int)units : lq_compute_units();
+#define LQ_FIRST(SLABS, GATED) \
+  launch_first<SLABS, GATED>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, w_packed, (bf16_t*)act, ldo, width, a, grid, stream)
+  if (slabs_per_wave(width) <= 2) return gated ? LQ_FIRST(2, true) : LQ_FIRST(2, false);
+  return gated ? LQ_FIRST(4, true) : LQ_FIRST(4, false);
 #undef LQ_FIRST
 }
 

@@ -96,6 +96,38 @@ def test_chosen_experts_alone(rows, E, top, ff, shared, width, activation, more,
         assert torch.equal(again[:, 0], out[:, 0])
 
 
+@pytest.mark.parametrize("ff,shared,width", [(64, 0, 512), (64, 64, 1088), (2112, 0, 1024), (4160, 64, 576), (10304, 0, 2112)])
+@pytest.mark.parametrize("activation", ["silu", "relu2"])
+@pytest.mark.parametrize("apart", [0, 72])
+def test_first_product_of_any_number_of_tiles(ff, shared, width, activation, apart):
+    """Workgroups of none, one, an odd and an even number of tiles, wavefronts without a share of K, and a dense weight's rows apart."""
+    from longbow_quarrel_amd.kernels.hip import HipKernels
+
+    kn, rows, E = HipKernels(), 3, 2
+    gen = torch.Generator().manual_seed(ff + width)
+    parts, inner = 1 if activation == "relu2" else 2, E * ff + shared
+    x = torch.randn(rows, width, generator=gen).bfloat16()
+    wide = torch.full((inner * parts, width + apart), float("nan"), dtype=torch.bfloat16)
+    w_in = wide[:, :width]
+    w_in.copy_(torch.randn(inner * parts, width, generator=gen) * width ** -0.5)
+    route = torch.tensor([[0.5, -1.0], [0.25, 0.75], [-1.0, 1.0]])
+    act = torch.full((rows, inner), 7.0, dtype=torch.bfloat16, device="cuda")
+    w_out = torch.zeros(width, inner, dtype=torch.bfloat16, device="cuda")
+    out = torch.empty(1, rows, width, device="cuda")
+    kn.pack_weights = apart == 0
+    held = wide.cuda()[:, :width] if apart else kn.pack_weight(w_in.contiguous().cuda())
+    kn.moe_few(x.cuda(), held, w_out, route.cuda(), act, out, ff, shared, activation)
+    for e in range(E + (1 if shared else 0)):
+        n, at = (ff, e * ff) if e < E else (shared, E * ff)
+        y = x.double() @ w_in[at * parts : (at + n) * parts].double().T
+        w = route[:, e : e + 1].double() if e < E else torch.ones(rows, 1, dtype=torch.float64)
+        v = weighted(y[:, :n] if parts == 2 else None, y[:, (parts - 1) * n :], w, activation, False, 0.0)
+        want = torch.where(w >= 0, v, 0.0)
+        # (half a unit of 8 bits at the result; the sums' 2^-24 a term of at most 2 112 at the products' size, times the factors beside them)
+        bound = 2.0 ** -8 * want.abs() + 2112 * 2.0 ** -24 * 16.0
+        assert ((act[:, at : at + n].double().cpu() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("rows,ff,places", [
     (8, 2176, (0, 64, 2048)),     # a wavefront's chunks 0 and 16 of 128 k: the sums of their halves are apart
     (1, 2176, (100, 40, 2148)),
