@@ -245,46 +245,67 @@ __global__ __launch_bounds__(64) void attention_tiles_kernel(
   }
 }
 
-// Steps of single tokens in float32: the tile above with one row in it takes its keys in a chain of eight round trips to memory and 256
-// dependent products a chunk.  Here four wavefronts share a row and head: each makes the scores of 16 keys of a chunk, which all of
-// them read from LDS, and the dimensions dt % 4 of the result, with the next chunk's keys and values on their way.  Every score,
-// the softmax and every dimension's sum are made as above, so the bits are the same.  4 rows of 100 to 340 keys, 32 heads of 128: 48.8 -> 24.3 us.
-template <int HS>  // HS: head size / 16, a multiple of 4
+// Steps of single tokens in float32: the tile above with one row in it takes its keys in a chain of eight round trips to memory and
+// 256 dependent products a chunk.  Here four wavefronts share a row and HEADS heads of a group (4, 2 or 1, as the group's size
+// allows), which are columns of the scores' products and rows of the values': each makes the scores of 16 keys of a chunk, which
+// all of them read from LDS, with the next chunk's keys and values on their way.  HEADS workgroups of such heads each make
+// HS / HEADS of the result's 16-column tiles.  Every score, the softmax and every dimension's sum are made as above, so the bits are
+// the same.  What bounds a chunk: its chain of products, and what a compute unit draws of it (29 GB/s), keys and 1 / HEADS of the values.
+// 4 rows of 100 to 340 keys, 32 heads of 128: as tiles 48.8 us; a head a workgroup 24.3; four heads 20.9, and 16.9 with the blocks looked up
+// a chunk earlier.
+template <int HS, int HEADS>  // HS: head size / 16, a multiple of 4
 __global__ __launch_bounds__(256) void attention_single_kernel(const float* __restrict__ q, int ldq, float* __restrict__ out, int ldo, int nh,
                                                                int nkv, const int* __restrict__ row_pos, const int* __restrict__ row_seq,
                                                                const int* __restrict__ seq_slot, const int* __restrict__ block_table,
                                                                int bt_stride, const float* __restrict__ kcache,
                                                                const float* __restrict__ vcache, int BS, float scale, int window) {
-  constexpr int HD = HS * 16, MINE = HS / 4;
-  __shared__ float scores[2][64];
+  constexpr int HD = HS * 16, TILES = HS / HEADS, MINE = (TILES + 3) / 4;  // 16-column tiles of a workgroup, and of a wavefront at most
+  __shared__ float scores[2][HEADS][64];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
-  const int r = blockIdx.x, h = blockIdx.y, kvh = h / (nh / nkv);
+  const int r = blockIdx.x, h0 = blockIdx.y / HEADS * HEADS, tile0 = blockIdx.y % HEADS * TILES, kvh = h0 / (nh / nkv);
+  const int head = c % HEADS;  // this lane's column of the scores, row of the probabilities
   const int pos = row_pos[r], lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
   const int* table = block_table + (long long)seq_slot[row_seq[r]] * bt_stride;
   f32x4 qv[HS];
 #pragma unroll
-  for (int sl = 0; sl < HS; ++sl) qv[sl] = load4f(q + (long long)r * ldq + h * HD + sl * 16 + 4 * g);
-  f32x4 kn[HS], vn[4][MINE];  // the chunk that is asked for: 16 keys, and the values' dimensions 16 (w + 4 i) + c
+  for (int sl = 0; sl < HS; ++sl) qv[sl] = load4f(q + (long long)r * ldq + (h0 + head) * HD + sl * 16 + 4 * g);
+  f32x4 kn[HS], vn[4][MINE];  // the chunk that is asked for: 16 keys, and the values' dimensions 16 (tile0 + w + 4 i) + c
+  // Sixteens of keys lie in a block each: the blocks of a chunk's four are looked up a chunk before it is asked for (else
+  // their round trip lies ahead of every chunk's keys).
+  const int first = lo / 64 * 64, last = pos / BS;
+  int block[4], entry[4], at = first / BS, in = first - at * BS;  // of the chunk that is asked for next; the sixteen behind it
+  auto look = [&]() {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      block[kt] = min(at, last), entry[kt] = table[block[kt]];
+      in += 16;
+      if (in >= BS) in = 0, ++at;
+    }
+  };
   auto ask = [&](int t0) {
-    const int tk = min(t0 + 16 * w + c, pos);
-    const float* kr = kcache + (((long long)table[tk / BS] * nkv + kvh) * BS + tk % BS) * (long long)HD + 4 * g;
+    const int own_block = w == 0 ? block[0] : w == 1 ? block[1] : w == 2 ? block[2] : block[3];
+    const int own_entry = w == 0 ? entry[0] : w == 1 ? entry[1] : w == 2 ? entry[2] : entry[3];
+    const float* kr = kcache + ((long long)own_entry * nkv + kvh) * BS * (long long)HD + (min(t0 + 16 * w + c, pos) - own_block * BS) * HD + 4 * g;
 #pragma unroll
     for (int sl = 0; sl < HS; ++sl) kn[sl] = load4f(kr + sl * 16);
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      const int t = min(t0 + 16 * kt + 4 * g, pos) & ~3;
-      const float* vr = vcache + (((long long)table[t / BS] * nkv + kvh) * (long long)HD + 16 * w + c) * BS + t % BS;
+      const int t = (min(t0 + 16 * kt + 4 * g, pos) & ~3) - block[kt] * BS;
+      const float* vr = vcache + (((long long)entry[kt] * nkv + kvh) * (long long)HD + 16 * (tile0 + w)) * BS + (long long)c * BS + t;
 #pragma unroll
-      for (int i = 0; i < MINE; ++i) vn[kt][i] = load4f(vr + (long long)i * 64 * BS);
+      for (int i = 0; i < MINE; ++i)
+        vn[kt][i] = TILES % 4 == 0 || w + 4 * i < TILES ? load4f(vr + (long long)i * 64 * BS) : (f32x4){0.f, 0.f, 0.f, 0.f};  // (no tile: nothing is stored)
     }
   };
   float m = -INFINITY, l = 0.f;
-  f32x4 o[MINE];  // (all 16 rows of a tile are the one row)
+  f32x4 o[MINE];  // (row e: of head e % HEADS)
 #pragma unroll
   for (int i = 0; i < MINE; ++i) o[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
   int turn = 0;
-  ask(lo / 64 * 64);
-  for (int t0 = lo / 64 * 64; t0 <= pos; t0 += 64, turn ^= 1) {
+  look();
+  ask(first);
+  look();
+  for (int t0 = first; t0 <= pos; t0 += 64, turn ^= 1) {
     f32x4 kv[HS], vv[4][MINE], own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int sl = 0; sl < HS; ++sl) kv[sl] = kn[sl];
@@ -292,16 +313,16 @@ __global__ __launch_bounds__(256) void attention_single_kernel(const float* __re
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
       for (int i = 0; i < MINE; ++i) vv[kt][i] = vn[kt][i];
-    if (t0 + 64 <= pos) ask(t0 + 64);
+    if (t0 + 64 <= pos) ask(t0 + 64), look();
 #pragma unroll
     for (int sl = 0; sl < HS; ++sl)
 #pragma unroll
       for (int j = 0; j < 4; ++j) own = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[sl][j], qv[sl][j], own, 0, 0, 0);
-    if (c == 0) {
+    if (c < HEADS) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int t = t0 + 16 * w + 4 * g + e;
-        scores[turn][16 * w + 4 * g + e] = t >= lo && t <= pos ? own[e] * scale : -INFINITY;
+        scores[turn][c][16 * w + 4 * g + e] = t >= lo && t <= pos ? own[e] * scale : -INFINITY;
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (loads fly on; of two turns' scores the other's have been read)
@@ -309,7 +330,7 @@ __global__ __launch_bounds__(256) void attention_single_kernel(const float* __re
     float cmax = -INFINITY;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      st[kt] = *(const f32x4*)&scores[turn][16 * kt + 4 * g];
+      st[kt] = *(const f32x4*)&scores[turn][head][16 * kt + 4 * g];
 #pragma unroll
       for (int e = 0; e < 4; ++e) cmax = fmaxf(cmax, st[kt][e]);
     }
@@ -330,19 +351,29 @@ __global__ __launch_bounds__(256) void attention_single_kernel(const float* __re
     psum += __shfl_xor(psum, 32, 64);
     l = l * alpha + psum;
     m = m_new;
+    f32x4 fade;
 #pragma unroll
-    for (int i = 0; i < MINE; ++i) o[i] *= alpha;
+    for (int e = 0; e < 4; ++e) fade[e] = HEADS == 1 ? alpha : __shfl(alpha, e % HEADS, 64);
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
+    for (int i = 0; i < MINE; ++i) o[i] *= fade;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+    for (int i = 0; i < MINE; ++i)
+      if (TILES % 4 == 0 || w + 4 * i < TILES)
 #pragma unroll
-        for (int i = 0; i < MINE; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[kt][j], vv[kt][i][j], o[i], 0, 0, 0);
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[kt][j], vv[kt][i][j], o[i], 0, 0, 0);
   }
   const float inv = 1.0f / l;
+  float all_inv[HEADS];
+#pragma unroll
+  for (int e = 0; e < HEADS; ++e) all_inv[e] = HEADS == 1 ? inv : __shfl(inv, e, 64);
   if (g == 0) {
 #pragma unroll
-    for (int i = 0; i < MINE; ++i) out[(long long)r * ldo + h * HD + 16 * (w + 4 * i) + c] = o[i][0] * inv;
+    for (int i = 0; i < MINE; ++i)
+      if (TILES % 4 == 0 || w + 4 * i < TILES)
+#pragma unroll
+        for (int e = 0; e < HEADS; ++e) out[(long long)r * ldo + (h0 + e) * HD + 16 * (tile0 + w + 4 * i) + c] = o[i][e] * all_inv[e];
   }
 }
 
@@ -369,13 +400,21 @@ bool try_tiles(const void* q, int ldq, void* out, int ldo, int rows, int batch, 
   if constexpr (sizeof(T) == 4)
     if (rpt == 1 && hd % 64 == 0) {
       const dim3 grid(rows, nh);
-#define LQ_SINGLE(HS)                                                                                                          \
-  attention_single_kernel<HS><<<grid, 256, 0, stream>>>((const float*)q, ldq, (float*)out, ldo, nh, nkv, row_pos, row_seq, seq_slot, \
-                                                        block_table, bt_stride, (const float*)kcache, (const float*)vcache, BS, scale, window)
-      if (hd == 64) LQ_SINGLE(4);
-      else if (hd == 128) LQ_SINGLE(8);
-      else if (hd == 192) LQ_SINGLE(12);
-      else LQ_SINGLE(16);
+#define LQ_SINGLE(HS, HEADS)                                                                                                          \
+  attention_single_kernel<HS, HEADS><<<grid, 256, 0, stream>>>((const float*)q, ldq, (float*)out, ldo, nh, nkv, row_pos, row_seq, seq_slot, \
+                                                               block_table, bt_stride, (const float*)kcache, (const float*)vcache, BS, scale, window)
+#define LQ_SINGLE_HEADS(HS)             \
+  do {                                  \
+    if (of_a_group == 4) LQ_SINGLE(HS, 4);      \
+    else if (of_a_group == 2) LQ_SINGLE(HS, 2); \
+    else LQ_SINGLE(HS, 1);              \
+  } while (0)
+      const int group = nh / nkv, of_a_group = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);
+      if (hd == 64) LQ_SINGLE_HEADS(4);
+      else if (hd == 128) LQ_SINGLE_HEADS(8);
+      else if (hd == 192) LQ_SINGLE_HEADS(12);
+      else LQ_SINGLE_HEADS(16);
+#undef LQ_SINGLE_HEADS
 #undef LQ_SINGLE
       return true;
     }
