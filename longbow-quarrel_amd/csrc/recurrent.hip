@@ -11,6 +11,18 @@
 
 namespace {
 
+template <typename T>
+__device__ inline void store4(T* p, float4 v);
+template <>
+__device__ inline void store4<float>(float* p, float4 v) { *(float4*)p = v; }
+template <>
+__device__ inline void store4<bf16_t>(bf16_t* p, float4 v) {
+  uint2 packed;
+  packed.x = (uint32_t)f32_to_bf16(v.x).bits | ((uint32_t)f32_to_bf16(v.y).bits << 16);
+  packed.y = (uint32_t)f32_to_bf16(v.z).bits | ((uint32_t)f32_to_bf16(v.w).bits << 16);
+  *(uint2*)p = packed;
+}
+
 // ---------------------------------------------------------------- Dynamic Tanh and the scaled add
 // (x += scale * (piece 0 + piece 1 + ...);)  out = tanh(alpha x) w + b
 template <typename T>
@@ -39,6 +51,55 @@ __global__ __launch_bounds__(256) void add_scaled_kernel(float* __restrict__ x, 
   float d = delta[i];
   for (int p = 1; p < pieces; ++p) d += delta[i + p * piece_stride];
   x[i] += scale * d;
+}
+
+// The sum of `pieces` of a delta in their order, four neighbours of each; the first four are asked for together.
+__device__ inline float4 summed4(const float4* __restrict__ delta, int pieces, long long stride4, long long i) {
+  float4 d[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) d[p] = p < pieces ? delta[i + p * stride4] : make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 sum = d[0];
+#pragma unroll
+  for (int p = 1; p < 4; ++p)
+    if (p < pieces) sum.x += d[p].x, sum.y += d[p].y, sum.z += d[p].z, sum.w += d[p].w;
+  for (int p = 4; p < pieces; ++p) {
+    const float4 e = delta[i + p * stride4];
+    sum.x += e.x, sum.y += e.y, sum.z += e.z, sum.w += e.w;
+  }
+  return sum;
+}
+
+// The same two in fours (n and the width in fours, all operands on 16 bytes, out on 8): every load of a thread is asked for ahead of the
+// first use, and no 64-bit remainder lies in front of the weights'.  2 048 rows of 2 048, two pieces of a
+// delta: 20.2 us entry by entry, 13.8 so (5.3 TB/s); the add 17.1 and 13.6.
+template <typename T>
+__global__ __launch_bounds__(256) void dynamic_tanh4_kernel(float4* __restrict__ x, const float4* __restrict__ delta, int pieces,
+                                                            long long stride4, float scale, const float4* __restrict__ w,
+                                                            const float4* __restrict__ b, const float* __restrict__ alpha,
+                                                            T* __restrict__ out, unsigned n4, unsigned width4) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  float4 v = x[i];
+  const unsigned c = i % width4;
+  const float4 gain = w[c], add = b[c];
+  const float a = alpha[0];
+  if (pieces > 0) {
+    const float4 d = summed4(delta, pieces, stride4, i);
+    v.x += scale * d.x, v.y += scale * d.y, v.z += scale * d.z, v.w += scale * d.w;
+    x[i] = v;
+  }
+  store4<T>(out + 4ll * i, make_float4(tanhf(a * v.x) * gain.x + add.x, tanhf(a * v.y) * gain.y + add.y,
+                                       tanhf(a * v.z) * gain.z + add.z, tanhf(a * v.w) * gain.w + add.w));
+}
+
+__global__ __launch_bounds__(256) void add_scaled4_kernel(float4* __restrict__ x, const float4* __restrict__ delta, int pieces,
+                                                          long long stride4, float scale, unsigned n4) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  float4 v = x[i];
+  const float4 d = summed4(delta, pieces, stride4, i);
+  v.x += scale * d.x, v.y += scale * d.y, v.z += scale * d.z, v.w += scale * d.w;
+  x[i] = v;
 }
 
 // out[r, c] = act(gu[r, c] + bias[c]) * (gu[r, I + c] + bias[I + c]); behind the I results `tail` more columns, a
@@ -126,18 +187,6 @@ __device__ inline float4 load4<bf16_t>(const bf16_t* p) {
   return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
                      __uint_as_float(v.y & 0xffff0000u));
 }
-template <typename T>
-__device__ inline void store4(T* p, float4 v);
-template <>
-__device__ inline void store4<float>(float* p, float4 v) { *(float4*)p = v; }
-template <>
-__device__ inline void store4<bf16_t>(bf16_t* p, float4 v) {
-  uint2 packed;
-  packed.x = (uint32_t)f32_to_bf16(v.x).bits | ((uint32_t)f32_to_bf16(v.y).bits << 16);
-  packed.y = (uint32_t)f32_to_bf16(v.z).bits | ((uint32_t)f32_to_bf16(v.w).bits << 16);
-  *(uint2*)p = packed;
-}
-
 template <typename T, int TAPS, int ROWS>
 __global__ __launch_bounds__(256) void causal_conv4_kernel(const T* __restrict__ x, int ldx, const float* __restrict__ w,
                                                            const float* __restrict__ bias, float* __restrict__ state,
@@ -1147,6 +1196,10 @@ bool scan_launch(int N, int P, long long work, ScanLaunch& s) {
 
 }  // namespace
 
+static bool delta_in_fours(const float* delta, int pieces, long long piece_stride) {
+  return pieces == 0 || ((uintptr_t)delta % 16 == 0 && (pieces == 1 || piece_stride % 4 == 0));
+}
+
 extern "C" int lq_dynamic_tanh(float* x, const float* delta, int pieces, long long piece_stride, float scale,
                                const float* w, const float* b, const float* alpha, void* out, int out_dtype, int rows,
                                int width, hipStream_t stream) {
@@ -1155,7 +1208,16 @@ extern "C" int lq_dynamic_tanh(float* x, const float* delta, int pieces, long lo
   LQ_REQUIRE(pieces >= 0 && (pieces == 0 || delta != nullptr), "dynamic_tanh: %d pieces of a delta", pieces);
   const long long n = (long long)rows * width;
   const unsigned blocks = (unsigned)((n + 255) / 256);
-  if (out_dtype == LQ_F32)
+  if (width % 4 == 0 && n / 4 < 0x7fffffffll - 255 && (out_dtype == LQ_F32 || out_dtype == LQ_BF16) && delta_in_fours(delta, pieces, piece_stride) &&
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b) & 15) == 0 && (uintptr_t)out % (out_dtype == LQ_F32 ? 16 : 8) == 0) {
+    const unsigned n4 = (unsigned)(n / 4), fours = (n4 + 255) / 256;
+#define LQ_TANH4(T)                                                                                                                  \
+  dynamic_tanh4_kernel<T><<<fours, 256, 0, stream>>>((float4*)x, (const float4*)delta, pieces, piece_stride / 4, scale, (const float4*)w, \
+                                                     (const float4*)b, alpha, (T*)out, n4, (unsigned)(width / 4))
+    if (out_dtype == LQ_F32) LQ_TANH4(float);
+    else LQ_TANH4(bf16_t);
+#undef LQ_TANH4
+  } else if (out_dtype == LQ_F32)
     dynamic_tanh_kernel<float><<<blocks, 256, 0, stream>>>(x, delta, pieces, piece_stride, scale, w, b, alpha, (float*)out, n, width);
   else if (out_dtype == LQ_BF16)
     dynamic_tanh_kernel<bf16_t><<<blocks, 256, 0, stream>>>(x, delta, pieces, piece_stride, scale, w, b, alpha, (bf16_t*)out, n, width);
@@ -1168,7 +1230,11 @@ extern "C" int lq_dynamic_tanh(float* x, const float* delta, int pieces, long lo
 extern "C" int lq_add_scaled(float* x, const float* delta, int pieces, long long piece_stride, float scale, long long n,
                              hipStream_t stream) {
   LQ_REQUIRE(x && delta && pieces > 0 && n > 0, "add_scaled: bad arguments");
-  add_scaled_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(x, delta, pieces, piece_stride, scale, n);
+  if (n % 4 == 0 && n / 4 < 0x7fffffffll - 255 && (uintptr_t)x % 16 == 0 && delta_in_fours(delta, pieces, piece_stride))
+    add_scaled4_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, stream>>>((float4*)x, (const float4*)delta, pieces, piece_stride / 4, scale,
+                                                                            (unsigned)(n / 4));
+  else
+    add_scaled_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(x, delta, pieces, piece_stride, scale, n);
   LQ_CHECK_LAUNCH("add_scaled");
   return 0;
 }

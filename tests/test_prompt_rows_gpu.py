@@ -71,3 +71,51 @@ def test_gated_norms_of_many_rows(kn, group, groups, wlen, rows, dtype):
         for lo in range(0, rows, 300):
             kn.gated_rmsnorm(y[lo : lo + 300], z[lo : lo + 300], wt, 1e-5, group, want[lo : lo + 300], gate_first=before, gate=gate)
         assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(3.0), want.nan_to_num(3.0)), gate
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width,pieces", [(1, 4, 1), (3, 260, 0), (3, 260, 5), (70, 1028, 2), (7, 130, 2), (5, 33, 3)])
+def test_dynamic_tanh_in_fours(kn, rows, width, pieces, dtype):
+    """Widths in fours and others, against 64 bits; x off a multiple of 16 bytes gives the same as on one."""
+    x, w, b, alpha = rnd(rows, width, seed=8), rnd(width, seed=9), rnd(width, seed=10), rnd(1, seed=11)
+    delta = rnd(pieces, rows, width, seed=12) if pieces else None
+    outs = []
+    for off in (0, 1):
+        held = torch.zeros(rows * width + 1, device=DEV)[off : off + rows * width].view(rows, width)
+        held.copy_(x)
+        out = torch.zeros((rows, width), dtype=dtype, device=DEV)
+        kn.dynamic_tanh(held, w, b, alpha, out, delta=delta, delta_scale=0.5)
+        stream = x.double() + (0.5 * delta.double().sum(0) if pieces else 0.0)
+        # (a rounding of 2^-24 a term at the stream's size; the tangent's slope is 1, its own error and the weights' two roundings 4 more)
+        bound = 2.0 ** -24 * 8 * (pieces + 1) * (1.0 + stream.abs())
+        assert ((held.double() - stream).abs() <= bound).all()
+        want = torch.tanh(alpha.double() * stream) * w.double() + b.double()
+        slack = bound * (1.0 + alpha.abs().double()) * (1.0 + w.abs().double()) + 2.0 ** -21 * (want.abs() + b.abs().double())
+        assert ((out.double() - want).abs() <= slack + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)).all()
+        outs.append((held.clone(), out))
+        if pieces:
+            kn.add_scaled(held, delta, -0.5)
+            assert ((held.double() - x.double()).abs() <= 2 * bound).all()
+    for on, other in zip(*outs):
+        assert (on.double() - other.double()).abs().max() <= 2.0 ** -7 * (1.0 + on.double().abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [4, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 130])
+@pytest.mark.parametrize("pieces,extra", [(1, False), (2, True), (4, False)])
+def test_postnorm_of_every_width(kn, width, pieces, extra, dtype):
+    rows = 3
+    x, y, w, nw = rnd(rows, width, seed=13), rnd(pieces, rows, width, seed=14), rnd(width, seed=15), rnd(width, seed=16)
+    scales = [0.5, -1.0, 2.0, 1.0][:pieces]
+    more = rnd(rows, width, seed=17) if extra else None
+    h = torch.zeros((rows, width), dtype=dtype, device=DEV)
+    held = x.clone()
+    kn.postnorm_residual(held, y if pieces > 1 else y[0], scales, w, 1e-5, extra=more, next_weight=nw, next_eps=1e-3, h=h)
+    v = sum(s * y[p].double() for p, s in enumerate(scales))
+    stream = x.double() + v / (v.square().mean(1, keepdim=True) + 1e-5).sqrt() * w.double() + (more.double() if extra else 0.0)
+    # (sums of a row in a tree of at most 8 + 8 + 2 levels, and some ten roundings more, of 2^-24 at the largest entry's size)
+    bound = 2.0 ** -24 * 32 * (1.0 + stream.abs().max())
+    assert (held.double() - stream).abs().max() <= bound
+    want = stream / (stream.square().mean(1, keepdim=True) + 1e-3).sqrt() * nw.double()
+    slack = 2 * bound * (1.0 + nw.abs().double().max()) + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)
+    assert ((h.double() - want).abs() <= slack).all()
