@@ -26,10 +26,6 @@
 // 9.0, 7 010 21.7 -> 15.4, 30 000 38.9 -> 34.9 (3.5 TB/s); 8 of 530 12.2 -> 10.6, 8 of 2 070 23.7 -> 20.2, 8 of 8 020 54.7 -> 53.0 (5.0 TB/s);
 // 64 of 560 from pieces 41.6 -> 34.3 (4.3 TB/s); 16 of 128 to 7 628 by units 64 -> 57.  Head size 64: one of 120 4.8 -> 4.2, of 3 000 9.7 ->
 // 9.1; 16 of 80 to 1 516 by units from pieces 15.5 -> 13.8; 24 of 160 from pieces 7.5 -> 7.7, the one length found that lost.
-#include <map>
-#include <mutex>
-#include <tuple>
-
 #include "attention_mfma.h"
 
 namespace {
@@ -377,11 +373,13 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
   const bool own = folded && b1 == last;  // whether this share holds the row's own position
   u32x4 q[S::KS], k_own[S::KS];
   Share<HD> cur;
-  int ahead[S::GB];  // the next blocks' numbers
+  // The first blocks' numbers come by scalar loads, those of the blocks behind them 64 at a time, lane l that of block b0 + l.  (Each
+  // looked up on its own, a block ahead, the walk waited for its way through memory, and where two blocks go together for the
+  // keys that were asked for between the two lookups: one sequence of 160 keys, head size 64, 5.5 -> 5.0 us, 24 of 160 6.8 -> 6.1, 16 of 530 from
+  // pieces 11.8 -> 9.8; head size 128, a whole row a unit of 24 sequences of 3 000 keys 64.9 -> 58.6.)
+  int numbers = table[min(b0 + lane, b1)];
 #pragma unroll
-  for (int u = 0; u < S::GB; ++u) ahead[u] = table[min(b0 + u, b1)];
-#pragma unroll
-  for (int u = 0; u < S::GB; ++u) ask_block<HD>(a, kvh, ahead[u], b0 + u <= b1, wave, c16, g, u, cur);
+  for (int u = 0; u < S::GB; ++u) ask_block<HD>(a, kvh, table[min(b0 + u, b1)], b0 + u <= b1, wave, c16, g, u, cur);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (PIECES) {
     q_row.put(a, rows, wave, g);
@@ -501,15 +499,16 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
       }
     }
   };
-#pragma unroll
-  for (int u = 0; u < S::GB; ++u) ahead[u] = table[min(b0 + S::GB + u, b1)];
   for (int b = b0, odd = 0;; b += S::GB, odd ^= 1) {
     Share<HD> next;
-#pragma unroll
-    for (int u = 0; u < S::GB; ++u) {
-      ask_block<HD>(a, kvh, ahead[u], b + S::GB + u <= b1, wave, c16, g, u, next);
-      ahead[u] = table[min(b + 2 * S::GB + u, b1)];
+    const int at = (b + S::GB - b0) & 63;
+    if (at == 0) {  // (64 is a multiple of GB)
+      numbers = table[min(b + S::GB + lane, b1)];
+      asm volatile("" : "+v"(numbers));  // (waited for in here, not behind the branch)
     }
+#pragma unroll
+    for (int u = 0; u < S::GB; ++u)
+      ask_block<HD>(a, kvh, __builtin_amdgcn_readlane(numbers, at + u), b + S::GB + u <= b1, wave, c16, g, u, next);
     take(b, odd, cur);
     if (b + S::GB > b1) break;
     cur = next;

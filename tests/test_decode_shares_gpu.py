@@ -5,7 +5,7 @@ import math
 import pytest
 import torch
 
-from test_kernels_gpu import BS, DEV, i32, kn, paged_cache, rel_err  # noqa: F401
+from test_kernels_gpu import BS, DEV, i32, kn, paged_cache, rel_err, run_attention  # noqa: F401
 import plain
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +57,12 @@ def test_folded_rows_at_the_edges(kn, heads, kv_heads, head_dim, rows, window, a
             assert torch.equal(vc[blk, :, :, off].cpu(), v[b, : kv_heads * head_dim].view(kv_heads, head_dim))
             assert rel_err(kc[blk, :, off], kt[b]) < 4e-3
         assert int(kn.tickets(torch.device("cuda", torch.cuda.current_device())).abs().max()) == 0
+
+
+@pytest.mark.parametrize("kv_heads,head_dim", [(64, 64), (64, 128)])
+def test_rows_of_more_blocks_than_a_wavefront_has_lanes(kn, kv_heads, head_dim):
+    """Whole rows (as many as compute units) of 64 blocks and one or two more or less, whose numbers are read 64 at a time."""
+    lengths = [63 * BS, 64 * BS + 1, 65 * BS + 1, 129 * BS]
+    got, want = run_attention(kn, None, lengths, [1] * 4, kv_heads, kv_heads, head_dim, torch.bfloat16, 71, decode=True)
+    for b, n in enumerate(lengths):
+        assert rel_err(got[b], want[b]) < 1.2e-2, n
