@@ -63,8 +63,9 @@ struct DecodeArgs {
   int batch;
   float* part_o;     // [rows][nh][nsplit][HD], or [nkv][units][heads of the group][HD]
   float* part_ml;    // the same with 2: maximum and sum
-  int narrow_splits; // the same without a second workgroup on any compute unit
   int nsplit;        // workgroups a row and kv head
+  int narrow_splits; // the same without a second workgroup on any compute unit
+  int long_from;     // > 0: a row goes in nsplit shares from this many blocks on, else whole (many_rows)
   int units;         // > 0: workgroups a kv head, which share the sequences' keys out among themselves
   int* tickets;      // [rows][nkv], zero between launches: how many shares of the row have finished
   // with the rotation and the cache write folded in (all null otherwise): the step's
@@ -275,7 +276,7 @@ __device__ inline void turn_row(const Turn<HD>& by, u32x4 (&x)[HD / 32]) {
     }
 }
 
-// Blocks a share of a row that has n.  In units of 32 KB of keys and values (a block of head size 128, two of 64), which take a compute
+// Blocks a share of a row that has n, where rows leave at least half of the compute units free (else: many_rows).  In units of 32 KB of keys and values (a block of head size 128, two of 64), which take a compute
 // unit 1.1 us: a row of up to three stays whole (a second share costs 1.5 us: partial results out, ticket, and back).  Each share
 // more costs its ticket and its results' way into the last workgroup 0.13 us, which is worth it down to sqrt(n / 8) of them a share
 // (one sequence of 1 500 keys 10.1 us with one each, 9.1 with two; of 7 010: 15.4 with four).  Where up to three a share do without a second
@@ -284,7 +285,8 @@ __device__ inline void turn_row(const Turn<HD>& by, u32x4 (&x)[HD / 32]) {
 template <int HD>
 __device__ inline int blocks_a_share(const DecodeArgs& a, int n) {
   constexpr int UNIT = HD <= 64 ? 2 : 1;
-  if (n <= 3 * UNIT) return n;
+  if (n <= 3 * UNIT || n < a.long_from) return n;
+  if (a.long_from > 0) return ceil_quotient(n, a.nsplit);
   const int narrow = ceil_quotient(n, a.narrow_splits);
   const int even = narrow <= 3 * UNIT ? narrow : ceil_quotient(n, a.nsplit);
   const int apart = __builtin_amdgcn_readfirstlane((int)(__builtin_amdgcn_sqrtf((float)n * (HD <= 64 ? 0.2f : 0.125f)) + 0.99f));
@@ -624,15 +626,48 @@ int launch(const DecodeArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Workgroups a row and kv head for a launch whose longest sequence may hold `max_len` tokens: two for every compute unit in all.  It
-// depends on the bound rounded up to LQ_DECODE_LENGTH_BUCKET, so that launches whose bounds differ less than that add up their
-// sums in the same order.  (Up to 256 keys a row is its one workgroup's, and needs no workspace.)
-static int decode_splits(int rows, int nkv, int max_len) {
+// How rows are shared out that take more than half of the compute units with one workgroup a kv head: in `shares` from `from` blocks
+// on (0: never).  A unit draws at most 29 GB/s and holds two workgroups (three at head sizes up to 64); the memory gives all of them
+// 20 each.  Up to a row a unit that is enough, but for the units that have none: few more rows than half of them go in thirds,
+// which give every unit two, and the longest up to four fifths of them in fifths, four in turn.  With more rows than units
+// whole ones would leave some units two and most one: shares even that out where they fill a whole number of rounds of two (three)
+// nearly.  A share more costs its ticket and partial results, and a round its chain of round trips: short rows stay whole.
+// 32 heads over 8, whole -> so, microseconds; before this file's walk by all wavefronts of a block, which knew as many splits, in brackets:
+// head size 128: 17 sequences of 1 500 keys 31 -> 28 (38), of 6 000 106 -> 84 (91); 22 of 6 000 114 -> 107 (108); 33 of 1 000 41.5 ->
+// 38 (46), of 3 000 106 -> 84 (101), of 6 000 203 -> 161 (176); 40 of 3 000 108 -> 94 (107); 48 of 6 000 223 -> 206 (214).  Head size 64: 17 of 3 000
+// 34 -> 27 (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 48 of 6 000 117 -> 110 (112).
+// (Rows whole that would do in shares, or the reverse: 24 of 200 keys in two shares each 12.5, whole 9.5; 24 of 6 000 118 and 110; 52 of 3 000 in
+// sixes 127, whole 118.)
+struct ManyRows {
+  int shares, from;
+};
+static ManyRows many_rows(long long pairs, int hd) {
+  const long long cus = lq_compute_units();
+  const bool small = hd <= 64;
+  if (3 * pairs <= 2 * cus) return {3, small ? 16 : 12};
+  if (small && 4 * pairs <= 3 * cus) return {4, 32};
+  if (!small && 5 * pairs <= 4 * cus) return {5, 80};
+  if (pairs <= cus) return {1, 0};
+  if (5 * pairs <= 6 * cus) return {5, small ? 16 : 14};
+  if (!small && 3 * pairs <= 4 * cus) return {3, 14};
+  if (2 * pairs <= 3 * cus) return {4, 28};
+  return {1, 0};
+}
+
+// Workgroups a row and kv head for a launch whose longest sequence may hold `max_len` tokens: two for every compute unit in all, where rows
+// leave half of the units free.  It depends on the bound rounded up to LQ_DECODE_LENGTH_BUCKET, so that launches whose bounds
+// differ less than that add up their sums in the same order.  (Up to 256 keys a row is its one workgroup's, and needs no workspace.)
+static int decode_splits(int rows, int nkv, int hd, int max_len) {
   if (max_len <= 4 * BS) return 1;
   const long long bound = (long long)lq_ceil_div(max_len, LQ_DECODE_LENGTH_BUCKET) * LQ_DECODE_LENGTH_BUCKET;
   const int blocks = (int)(bound / BS);
-  const long long room = 2LL * lq_compute_units() / ((long long)rows * nkv);
-  return (int)(room < 1 ? 1 : room < blocks ? room : blocks);
+  const long long pairs = (long long)rows * nkv, cus = lq_compute_units();
+  if (2 * pairs > cus) {
+    const ManyRows many = many_rows(pairs, hd);
+    return blocks >= many.from ? many.shares : 1;
+  }
+  const long long room = 2 * cus / pairs;
+  return (int)(room < blocks ? room : blocks);
 }
 
 // Units a kv head for a decoding launch whose workgroups share the splits out themselves (0: the grid is
@@ -680,7 +715,7 @@ int lq_attention_unit_tries(const int* pos, int rows, int nkv, int max_len) {
 // Floats of workspace a launch needs (0 when no row has several shares): enough for either grid, the
 // window being unknown here.
 long long lq_attention_decode_workspace(int rows, int nh, int nkv, int hd, int max_len) {
-  const int nsplit = decode_splits(rows, nkv, max_len);
+  const int nsplit = decode_splits(rows, nkv, hd, max_len);
   const long long classic = nsplit <= 1 ? 0 : (long long)rows * nh * nsplit * (hd + 2);
   const long long shared = (long long)decode_units(rows, nkv, max_len, 0) * nh * (hd + 2);
   return classic > shared ? classic : shared;
@@ -732,7 +767,7 @@ int lq_attention_decode(const void* q, int ldq, void* out, int ldo, int rows, in
     LQ_REQUIRE(((uintptr_t)cs % 16) == 0, "attention: the cos/sin table must be 16-byte aligned");
   }
   LQ_REQUIRE(max_len > 0, "attention: decoding needs the longest sequence length");
-  a.nsplit = decode_splits(rows, nkv, max_len);
+  a.nsplit = decode_splits(rows, nkv, hd, max_len);
   a.units = uneven ? decode_units(rows, nkv, max_len, window) : 0;  // (by the bound in 1 024s, as everything here)
   if (a.units > 0 || a.nsplit > 1) {
     const long long need = a.units > 0 ? (long long)a.units * nh * (hd + 2) : lq_attention_decode_workspace(rows, nh, nkv, hd, max_len);
@@ -748,6 +783,7 @@ int lq_attention_decode(const void* q, int ldq, void* out, int ldo, int rows, in
   const long long pairs = (long long)rows * nkv;
   a.narrow_splits = pairs < lq_compute_units() ? (int)(lq_compute_units() / pairs) : 1;
   if (a.narrow_splits > a.nsplit) a.narrow_splits = a.nsplit;  // (no row in more shares than the grid has for it)
+  a.long_from = 2 * pairs > lq_compute_units() && a.nsplit > 1 ? many_rows(pairs, hd).from : 0;
   switch (hd) {
     case 32: return launch<32>(a, stream);
     case 64: return launch<64>(a, stream);

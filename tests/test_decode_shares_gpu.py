@@ -66,3 +66,24 @@ def test_rows_of_more_blocks_than_a_wavefront_has_lanes(kn, kv_heads, head_dim):
     got, want = run_attention(kn, None, lengths, [1] * 4, kv_heads, kv_heads, head_dim, torch.bfloat16, 71, decode=True)
     for b, n in enumerate(lengths):
         assert rel_err(got[b], want[b]) < 1.2e-2, n
+
+
+@pytest.mark.parametrize("rows,kv_heads,head_dim,start", [(17, 8, 128, 12), (21, 8, 64, 16), (3, 64, 64, 32), (3, 64, 128, 80), (33, 8, 192, 14),
+                                                          (5, 64, 128, 14), (6, 64, 128, 28), (6, 64, 64, 28), (12, 32, 256, 28)])
+@pytest.mark.parametrize("window", [0, 1000])
+def test_long_rows_of_launches_that_fill_the_chip(kn, rows, kv_heads, head_dim, start, window):
+    """Launches of half to twice as many rows and kv heads as compute units: rows of up to `start` blocks stay whole, longer ones go
+    in shares, which its last workgroup adds up, so that the units have equal parts.  Rows at that line, far beyond it and of one
+    key; twice the same, with the counters at zero after each."""
+    lengths = ([start * BS, (start - 1) * BS, (start - 1) * BS + 1, 3 * start * BS + 65, 1, start * BS + 1] * rows)[:rows]
+    if rows > 6:
+        lengths[6:] = [n if n < 200 else 200 + 7 * r for r, n in enumerate(lengths[6:])]
+    assert kn.attention_workspace(torch.bfloat16, rows, kv_heads, kv_heads, head_dim, BS, True, max(lengths)) > 0
+    outs = []
+    for _ in range(2):
+        got, want = run_attention(kn, None, lengths, [1] * rows, kv_heads, kv_heads, head_dim, torch.bfloat16, 83, window=window, decode=True)
+        for b, n in enumerate(lengths):
+            assert rel_err(got[b], want[b]) < 1.2e-2, (b, n)
+        assert int(kn.tickets(torch.device("cuda", torch.cuda.current_device())).abs().max()) == 0
+        outs.append(got)
+    assert torch.equal(*outs)

@@ -545,9 +545,8 @@ def test_decode_attention_over_several_splits(kn, head_dim, heads, kv_heads, win
 
 @pytest.mark.parametrize("rows", [24, 64])
 def test_decode_attention_of_many_rows_with_long_splits(kn, rows):
-    """24 and 64 sequences of 8 kv heads and head size 128, up to 3 000 keys: so many workgroups that a
-    split covers 512 to 3 072 positions (one split for some launches, several for others, with rows of one
-    launch ending in different splits).  Twice, with the ticket counters back at zero after each."""
+    """24 and 64 sequences of 8 kv heads and head size 128, up to 3 000 keys: so many workgroups that every row is one's (rows of
+    as many that go in several: test_decode_shares_gpu.py).  Twice, with the ticket counters at zero after each."""
     g = torch.Generator().manual_seed(rows)
     lengths = torch.randint(1, 3001, (rows,), generator=g).tolist()
     lengths[0], lengths[1], lengths[2] = 3000, 1, 1025
