@@ -656,9 +656,8 @@ static ManyRows many_rows(long long pairs, int hd) {
 
 // Workgroups a row and kv head for a launch whose longest sequence may hold `max_len` tokens: two for every compute unit in all, where rows
 // leave half of the units free.  It depends on the bound rounded up to LQ_DECODE_LENGTH_BUCKET, so that launches whose bounds
-// differ less than that add up their sums in the same order.  (Up to 256 keys a row is its one workgroup's, and needs no workspace.)
+// differ less than that add up their sums in the same order.
 static int decode_splits(int rows, int nkv, int hd, int max_len) {
-  if (max_len <= 4 * BS) return 1;
   const long long bound = (long long)lq_ceil_div(max_len, LQ_DECODE_LENGTH_BUCKET) * LQ_DECODE_LENGTH_BUCKET;
   const int blocks = (int)(bound / BS);
   const long long pairs = (long long)rows * nkv, cus = lq_compute_units();
@@ -769,6 +768,11 @@ int lq_attention_decode(const void* q, int ldq, void* out, int ldo, int rows, in
   LQ_REQUIRE(max_len > 0, "attention: decoding needs the longest sequence length");
   a.nsplit = decode_splits(rows, nkv, hd, max_len);
   a.units = uneven ? decode_units(rows, nkv, max_len, window) : 0;  // (by the bound in 1 024s, as everything here)
+  // Up to 256 keys a launch needs no workspace and no counters: where none are given, its rows stay whole.
+  if (a.units == 0 && a.nsplit > 1 && max_len <= 4 * BS &&
+      (workspace == nullptr || workspace_floats < lq_attention_decode_workspace(rows, nh, nkv, hd, max_len) || tickets == nullptr ||
+       tickets_n < (long long)rows * nkv))
+    a.nsplit = 1;
   if (a.units > 0 || a.nsplit > 1) {
     const long long need = a.units > 0 ? (long long)a.units * nh * (hd + 2) : lq_attention_decode_workspace(rows, nh, nkv, hd, max_len);
     LQ_REQUIRE(workspace != nullptr && workspace_floats >= need,

@@ -87,3 +87,25 @@ def test_long_rows_of_launches_that_fill_the_chip(kn, rows, kv_heads, head_dim, 
         assert int(kn.tickets(torch.device("cuda", torch.cuda.current_device())).abs().max()) == 0
         outs.append(got)
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("kv_heads,head_dim", [(8, 128), (2, 192), (1, 256), (8, 64)])
+@pytest.mark.parametrize("rows", [1, 3])
+def test_bits_do_not_depend_on_the_bound_within_its_bucket(kn, kv_heads, head_dim, rows):
+    """A step run directly gives its longest sequence as the bound, a captured one the bound rounded up: the same bits, whatever the
+    length; and without a workspace, which up to 256 keys a launch does not need, the same result but for the order of its sums."""
+    for n in (64, 150, 193, 230, 256, 257, 700):
+        outs = [run_attention(kn, None, [n] * rows, [1] * rows, 2 * kv_heads, kv_heads, head_dim, torch.bfloat16, 91, decode=True, max_len=bound)
+                for bound in (n, kn.decode_length_bound(n))]
+        assert torch.equal(outs[0][0], outs[1][0]), n
+        assert rel_err(*outs[0]) < 8e-3
+    lengths = [256, 200, 64][:rows]
+    kc, vc, table, slots, dense = paged_cache(lengths, kv_heads, head_dim, torch.bfloat16, 5)
+    q = torch.randn(rows, kv_heads * head_dim, generator=torch.Generator().manual_seed(7)).bfloat16().to(DEV)
+    out = torch.empty_like(q)
+    kn.attention(q, out, kv_heads, kv_heads, head_dim, i32([n - 1 for n in lengths]), i32(range(rows)), i32(slots), i32(range(rows + 1)), table,
+                 kc, vc, BS, 1.0 / math.sqrt(head_dim), decode=True, max_len=256)
+    for b, n in enumerate(lengths):
+        full = torch.zeros(n, kv_heads, head_dim, dtype=torch.float64)
+        full[n - 1] = q[b].double().cpu().view(kv_heads, head_dim)
+        assert rel_err(out[b].view(kv_heads, head_dim), plain.attention(full, *dense[b], rows=[n - 1])[n - 1]) < 1.2e-2
