@@ -42,10 +42,13 @@ __device__ inline int first_key(const SinkArgs& a, int p) {
 struct SinkStart {
   float m, l;
 };
+__device__ inline SinkStart start_at(float sink) {
+  const float m = sink * LOG2E;
+  return {fminf(fmaxf(m, NONE), FLT_MAX), m < NONE ? 0.f : fmaf(sink, 0.f, 1.f)};
+}
 __device__ inline SinkStart sink_start(const SinkArgs& a, int h) {
   if (a.sinks == nullptr) return {0.f, 1.f};
-  const float s = a.sinks[h], m = s * LOG2E;
-  return {fminf(fmaxf(m, NONE), FLT_MAX), m < NONE ? 0.f : fmaf(s, 0.f, 1.f)};
+  return start_at(a.sinks[h]);
 }
 
 // What a lane needs of its query head to shape a score.

@@ -195,6 +195,10 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
     hs = head_shape(a, h);
     dist = hs.dist, hs.dist = nullptr;
   }
+  // (Asked for here and used behind the keys on their way: behind the keys' requests they waited for all of these, one row under a window of 128
+  // with sinks 7.5 -> 6.6 us.  Without a sink's value or a gate something else is read, and not used.)
+  const float sink = *(a.sinks != nullptr ? a.sinks + h : (const float*)a.row_pos + r);
+  const bf16_t logit = *(gate != nullptr ? gate + (long long)r * a.ldg + h : q + (long long)r * a.ldq);
   __builtin_amdgcn_sched_barrier(0);
   const int* table = a.block_table + (long long)(seq == r ? likely : a.seq_slot[seq]) * a.bt_stride;
   const Blocks seen = blocks_of(a, pos);
@@ -226,21 +230,20 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) s.bias[u][e] = dist[min(max(pos - (start_of(i) + 16 * w + 4 * g + e), 0), hs.last)];
   };
+  // (the first blocks' numbers by scalar loads, those of the blocks behind them 64 at a time, lane l that of the share's l-th: attention_decode.hip;
+  // one row of 160 keys, 16 heads of 64 over 8, 7.6 -> 6.7 us)
   S cur;
-  int ahead[S::GB];
+  int numbers = table[start_of(min(i0 + lane, i1)) / BLOCK];
 #pragma unroll
-  for (int u = 0; u < S::GB; ++u) ahead[u] = table[start_of(min(i0 + u, i1)) / BLOCK];
-#pragma unroll
-  for (int u = 0; u < S::GB; ++u) ask(i0 + u, ahead[u], u, cur);
+  for (int u = 0; u < S::GB; ++u) ask(i0 + u, table[start_of(min(i0 + u, i1)) / BLOCK], u, cur);
   __builtin_amdgcn_sched_barrier(0);
 
   const float c2 = a.scale * LOG2E;
   float m = NONE, l = 0.f;  // the head's running maximum (in powers of two); this lane's share of its sum
   if (a.sink && split == 0) {
-    const SinkStart start = sink_start(a, h);
+    const SinkStart start = a.sinks != nullptr ? start_at(sink) : SinkStart{0.f, 1.f};
     m = start.m, l = g == 0 ? start.l : 0.f;
   }
-  const float gate_logit = gate_of(gate, a, r, h);
   f32x4 o[S::VW];  // o[x][e]: value entry 16 (w + NW x) + 4 g + e of head c
 #pragma unroll
   for (int x = 0; x < S::VW; ++x) o[x] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -252,6 +255,7 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
     float own_top = NONE;
 #pragma unroll
     for (int u = 0; u < S::GB; ++u) {
+      if (u > 0 && i + u > i1) break;  // (a share's odd last block goes alone: 160 keys as above 6.5 -> 6.1 us)
       const int t0 = start_of(i + u);
       st[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -268,9 +272,15 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
         } else {
           x = st[u][e] * c2;
         }
-        st[u][e] = t <= pos && (t >= lo || t < a.keep_first) && i + u <= i1 ? x : -INFINITY;
-        own_top = fmaxf(own_top, st[u][e]);
+        st[u][e] = x;
       }
+      if (t0 + BLOCK - 1 > pos || (t0 < lo && t0 + BLOCK > a.keep_first))  // (not all of its positions are seen)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = t0 + 16 * w + 4 * g + e;
+          if ((t > pos) | ((t < lo) & (t >= a.keep_first))) st[u][e] = -INFINITY;
+        }
+      own_top = fmaxf(own_top, fmaxf(fmaxf(st[u][0], st[u][1]), fmaxf(st[u][2], st[u][3])));
       if (t0 + BLOCK - 1 > pos) {  // (0 times what lies in unwritten memory may be NaN)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -286,6 +296,7 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
     own_top = across_max(own_top);
 #pragma unroll
     for (int u = 0; u < S::GB; ++u) {
+      if (u > 0 && i + u > i1) break;
 #pragma unroll
       for (int e = 0; e < 4; ++e) st[u][e] = __builtin_amdgcn_exp2f(st[u][e] - own_top);
       *(f32x4*)&scores[turn][c][u * BLOCK + 16 * w + 4 * g] = st[u];
@@ -301,7 +312,8 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
     for (int x = 0; x < S::VW; ++x) o[x] *= alpha;
     const float up[2] = {__builtin_amdgcn_exp2f((g < 2 ? tw[0] : tw[1]) - m), __builtin_amdgcn_exp2f((g < 2 ? tw[2] : tw[3]) - m)};
 #pragma unroll
-    for (int u = 0; u < S::GB; ++u)
+    for (int u = 0; u < S::GB; ++u) {
+      if (u > 0 && i + u > i1) break;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         f32x4 pr[2];  // keys 32 j + 8 g .. + 7
@@ -322,16 +334,17 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
           for (int x = 0; x < S::VW; ++x)
             o[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(s.v[u][x][j]), as_bf16x8(part[i3]), o[x], 0, 0, 0);
       }
+    }
   };
-#pragma unroll
-  for (int u = 0; u < S::GB; ++u) ahead[u] = table[start_of(min(i0 + S::GB + u, i1)) / BLOCK];
   for (int i = i0, odd = 0;; i += S::GB, odd ^= 1) {
     S next;
-#pragma unroll
-    for (int u = 0; u < S::GB; ++u) {
-      ask(min(i + S::GB + u, i1 + 1), ahead[u], u, next);
-      ahead[u] = table[start_of(min(i + 2 * S::GB + u, i1)) / BLOCK];
+    const int at = (i + S::GB - i0) & 63;
+    if (at == 0) {  // (64 is a multiple of GB)
+      numbers = table[start_of(min(i + S::GB + lane, i1)) / BLOCK];
+      asm volatile("" : "+v"(numbers));  // (waited for in here, not behind the branch)
     }
+#pragma unroll
+    for (int u = 0; u < S::GB; ++u) ask(min(i + S::GB + u, i1 + 1), __builtin_amdgcn_readlane(numbers, at + u), u, next);
     take(i, odd, cur);
     if (i + S::GB > i1) break;
     cur = next;
@@ -339,7 +352,7 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
   l = across_sum(l);
   const long long at = (long long)r * gridDim.y + blockIdx.y;
   if (c < cols) {
-    const float factor = live == 1 ? head_factor(gate, gate_logit, l) : 0.f;
+    const float factor = live == 1 ? head_factor(gate, to_f32(logit), l) : 0.f;
     float* mine = sh.part + (at * sh.splits + split) * hd.share_floats;
 #pragma unroll
     for (int x = 0; x < S::VW; ++x) {

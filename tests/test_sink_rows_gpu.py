@@ -55,6 +55,14 @@ def test_single_tokens_of_few_rows(H, G, D, P, options, lengths):
     check(H, G, D, P, [(1, n - 1) for n in lengths], options, True)
 
 
+@pytest.mark.parametrize("H,G,D,P,options", [(8, 8, 64, 64, dict(sinks=True, window=128)), (128, 64, 64, 40, dict(PLAIN, window=4200, keep_first=300)),
+                                             (64, 64, 128, 128, dict(sinks=True, gate=True)), (256, 8, 128, 256, dict(PLAIN, chunk=5000))])
+def test_single_tokens_of_more_blocks_than_a_wavefront_has_lanes(H, G, D, P, options):
+    """Whole rows (as many tiles of heads as compute units) of 64 blocks and more, whose numbers are read 64 at a time, and rows of an odd
+    number of blocks where two go together."""
+    check(H, G, D, P, [(1, n - 1) for n in (160, 63 * 64, 64 * 64 + 1, 65 * 64 + 1)], options, True)
+
+
 @pytest.mark.parametrize("H,G,D,P,seqs,options", CASES)
 def test_tiles_of_32_rows(H, G, D, P, seqs, options):
     check(H, G, D, P, seqs, options, False)
