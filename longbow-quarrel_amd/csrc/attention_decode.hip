@@ -580,12 +580,16 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
     const float* po = a.part_o + (long long)c * apart * HD + d;
     float M = -INFINITY, L = 0.f;
     float2 acc = make_float2(0.f, 0.f);
-    // eight shares, or twice eight, are asked for together; one beyond the last is the last once more, with a weight of zero
+    // eight shares, or twice eight, are asked for together, as far as there are so many (partial results come past the caches, at 13 GB/s
+    // a compute unit: 12 rows of 250 keys in two shares each, with requests for eight, 8.9 us, with two 8.5)
     auto ask = [&](int s0, float2 (&stat)[AT_ONCE], float2 (&sum)[AT_ONCE]) {
 #pragma unroll
       for (int j = 0; j < AT_ONCE; ++j) {
-        const long long at = place(min(s0 + j, shares - 1));
-        stat[j] = published2(ml + 2 * at), sum[j] = published2(po + at * HD);
+        stat[j] = make_float2(-INFINITY, 0.f), sum[j] = make_float2(0.f, 0.f);
+        if (s0 + j < shares) {  // (the same for the whole workgroup)
+          const long long at = place(s0 + j);
+          stat[j] = published2(ml + 2 * at), sum[j] = published2(po + at * HD);
+        }
       }
     };
     auto add = [&](int s0, const float2 (&stat)[AT_ONCE], const float2 (&sum)[AT_ONCE]) {

@@ -119,43 +119,63 @@ __device__ inline void finish2(void* out, const SinkArgs& a, int r, int h, int d
   put_out((bf16_t*)out, at + 1, v.y, a.out_f32);
 }
 
-// The shares of a row and tile added up in their order, by a whole workgroup: two neighbouring entries a thread, eight shares' asked
-// for at once (one beyond the last is the last once more, with a weight of zero).
+// The shares of a row and tile added up in their order, by a whole workgroup: PAIRS times two neighbouring entries a thread, and eight
+// shares of each, are asked for at once, as far as there are so many.  What bounds it is these round trips: partial results come past the
+// caches, and requests for shares that a row does not have would be as slow as any others (16 heads of 192, 24 rows of 160 keys, a pair at a time
+// and always eight shares 12.9 -> 12.0 us; of 1 000 17.4 -> 16.1; 4 heads of 128 with two maps, 33 rows of 500 keys 19.9 -> 18.3).
+template <int PAIRS>
 __device__ inline void add_shares(void* out, const bf16_t* gate, const SinkArgs& a, const Shares& sh, const Heads& hd, int live) {
   constexpr int AT_ONCE = 8;
-  const int r = blockIdx.x, VD = a.VD;
+  const int r = blockIdx.x, VD = a.VD, entries = hd.cols * VD;
   const float* shares = sh.part + ((long long)r * gridDim.y + blockIdx.y) * sh.splits * hd.share_floats;
-  for (int i = 2 * threadIdx.x; i < hd.cols * VD; i += 2 * NW * 64) {  // (VD is even: a pair is one head's)
-    const int c = (int)(((float)i + 0.5f) * __builtin_amdgcn_rcpf((float)VD));
-    const float logit = gate_of(gate, a, r, hd.hbase + c);
-    float M = NONE, L = 0.f;
-    float2 acc = make_float2(0.f, 0.f);
+  for (int i0 = 2 * threadIdx.x; i0 < entries; i0 += 2 * PAIRS * NW * 64) {  // (VD is even: a pair is one head's)
+    int c[PAIRS];
+    float logit[PAIRS], M[PAIRS], L[PAIRS];
+    float2 acc[PAIRS];
+#pragma unroll
+    for (int x = 0; x < PAIRS; ++x) {
+      c[x] = (int)(((float)min(i0 + 2 * x * NW * 64, entries - 2) + 0.5f) * __builtin_amdgcn_rcpf((float)VD));
+      logit[x] = gate_of(gate, a, r, hd.hbase + c[x]);
+      M[x] = NONE, L[x] = 0.f, acc[x] = make_float2(0.f, 0.f);
+    }
     for (int s0 = 0; s0 < live; s0 += AT_ONCE) {
-      float2 stat[AT_ONCE], sum[AT_ONCE];
+      float2 stat[PAIRS][AT_ONCE], sum[PAIRS][AT_ONCE];
 #pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) {
-        const float* p = shares + min(s0 + j, live - 1) * hd.share_floats;
-        stat[j] = published2(p + sh.heads * VD + 2 * c), sum[j] = published2(p + i);
-      }
-      float top = M;
+      for (int j = 0; j < AT_ONCE; ++j)
 #pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) top = fmaxf(top, stat[j].x);
-      const float keep = __builtin_amdgcn_exp2f(M - top);
-      acc.x *= keep, acc.y *= keep, L *= keep, M = top;
+        for (int x = 0; x < PAIRS; ++x) {
+          stat[x][j] = make_float2(NONE, 0.f), sum[x][j] = make_float2(0.f, 0.f);
+          if (s0 + j < live && (x == 0 || 2 * x * NW * 64 < entries)) {  // (the same for the whole workgroup)
+            const float* p = shares + (s0 + j) * hd.share_floats;
+            stat[x][j] = published2(p + sh.heads * VD + 2 * c[x]), sum[x][j] = published2(p + min(i0 + 2 * x * NW * 64, entries - 2));
+          }
+        }
 #pragma unroll
-      for (int j = 0; j < AT_ONCE; ++j) {
-        const float f = s0 + j < live ? __builtin_amdgcn_exp2f(stat[j].x - M) : 0.f;
-        acc.x = fmaf(f, sum[j].x, acc.x), acc.y = fmaf(f, sum[j].y, acc.y), L = fmaf(f, stat[j].y, L);
+      for (int x = 0; x < PAIRS; ++x) {
+        float top = M[x];
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; ++j) top = fmaxf(top, stat[x][j].x);
+        const float keep = __builtin_amdgcn_exp2f(M[x] - top);
+        acc[x].x *= keep, acc[x].y *= keep, L[x] *= keep, M[x] = top;
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; ++j) {
+          const float f = s0 + j < live ? __builtin_amdgcn_exp2f(stat[x][j].x - M[x]) : 0.f;
+          acc[x].x = fmaf(f, sum[x][j].x, acc[x].x), acc[x].y = fmaf(f, sum[x][j].y, acc[x].y), L[x] = fmaf(f, stat[x][j].y, L[x]);
+        }
       }
     }
-    finish2(out, a, r, hd.hbase + c, i - c * VD, acc, head_factor(gate, logit, L));
+#pragma unroll
+    for (int x = 0; x < PAIRS; ++x) {
+      const int i = i0 + 2 * x * NW * 64;
+      if (i < entries) finish2(out, a, r, hd.hbase + c[x], i - c[x] * VD, acc[x], head_factor(gate, logit[x], L[x]));
+    }
   }
 }
 
 __global__ __launch_bounds__(NW * 64) void sink_add_shares_kernel(void* __restrict__ out, const bf16_t* __restrict__ gate,
                                                                   SinkArgs a, Shares sh) {
   const int n = blocks_of(a, a.row_pos[blockIdx.x]).n, live = quotient(n - 1, blocks_a_share(sh, n)) + 1;
-  if (live > 1) add_shares(out, gate, a, sh, heads_of(a, sh), live);  // (else the row is finished)
+  if (live > 1) add_shares<2>(out, gate, a, sh, heads_of(a, sh), live);  // (else the row is finished)
 }
 
 // KD and VD up to 32 KS and 16 VT: sizes in between run with zeros behind their keys and values.  GB blocks are taken together.
@@ -374,7 +394,9 @@ __global__ __launch_bounds__(NW * 64, KS <= 4 ? 2 : 1) void sink_decode_kernel(
     last = __hip_atomic_fetch_add(sh.tickets + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == live - 1;
   __syncthreads();
   if (!last) return;
-  add_shares(out, gate, a, sh, hd, live);
+  // (few entries by the short code: a launch finds none of it in the instruction cache, and the longer one costs it 0.9 us)
+  if (hd.cols * VD <= 4 * NW * 64) add_shares<1>(out, gate, a, sh, hd, live);
+  else add_shares<VT <= 4 ? 2 : 3>(out, gate, a, sh, hd, live);
   if (tid == 0) __hip_atomic_store(sh.tickets + at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
 }
 
