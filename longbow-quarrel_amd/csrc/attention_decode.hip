@@ -630,18 +630,18 @@ int launch(const DecodeArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// How rows are shared out that take more than half of the compute units with one workgroup a kv head: in `shares` from `from` blocks
-// on (0: never).  A unit draws at most 29 GB/s and holds two workgroups (three at head sizes up to 64); the memory gives all of them
-// 20 each.  Up to a row a unit that is enough, but for the units that have none: few more rows than half of them go in thirds,
-// which give every unit two, and the longest up to four fifths of them in fifths, four in turn.  With more rows than units
-// whole ones would leave some units two and most one: shares even that out where they fill a whole number of rounds of two (three)
-// nearly.  A share more costs its ticket and partial results, and a round its chain of round trips: short rows stay whole.
-// 32 heads over 8, whole -> so, microseconds; before this file's walk by all wavefronts of a block, which knew as many splits, in brackets:
-// head size 128: 17 sequences of 1 500 keys 31 -> 28 (38), of 6 000 106 -> 84 (91); 22 of 6 000 114 -> 107 (108); 33 of 1 000 41.5 ->
-// 38 (46), of 3 000 106 -> 84 (101), of 6 000 203 -> 161 (176); 40 of 3 000 108 -> 94 (107); 48 of 6 000 223 -> 206 (214).  Head size 64: 17 of 3 000
-// 34 -> 27 (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 48 of 6 000 117 -> 110 (112).
-// (Rows whole that would do in shares, or the reverse: 24 of 200 keys in two shares each 12.5, whole 9.5; 24 of 6 000 118 and 110; 52 of 3 000 in
-// sixes 127, whole 118.)
+// How rows are shared out that take more than half of the compute units with one workgroup a kv head: in `shares` from `from` blocks on
+// (0: never).  A unit draws at most 29 GB/s and holds two workgroups (three at head sizes up to 64);
+// the memory gives all of them 20 each.  Up to a row a unit that is enough, but for the units that have none: few more rows than half
+// of them go in thirds, which give every unit two, and the longest up to four fifths of them in fifths, four in turn.  With more
+// rows than units whole ones would leave some units two and most one: shares even that out where they fill a whole number of rounds
+// of two (three) nearly.  A share more costs its ticket and partial results, and a round its chain of round trips: short rows stay whole.
+// 32 heads over 8, whole -> so, microseconds; a wavefront with a block of its own and up to 2 048 workgroups in brackets:
+// head size 128: 17 sequences of 1 500 keys 31 -> 28 (38), of 6 000 106 -> 84 (91); 22 of 6 000 114 -> 107 (108); 33 of 1 000 41.5 -> 38 (46), of
+// 3 000 106 -> 84 (101), of 6 000 203 -> 161 (176); 40 of 3 000 108 -> 94 (107); 48 of 6 000 223 -> 206 (214).  Head size 64: 17 of 3 000 34 -> 27
+// (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 48 of 6 000 117 -> 110 (112).
+// (Rows whole that would do in shares, or the reverse: 24 of 200 keys in two shares each 12.5, whole 9.5; 24 of 6 000 118 and 110; 52 of 3 000
+// in sixes 127, whole 118.)
 struct ManyRows {
   int shares, from;
 };

@@ -57,6 +57,7 @@ struct Shares {
   int splits, narrow;    // workgroups a row and tile at most; the same without a second one on any compute unit
   int heads, tiles;      // query heads a workgroup; how many such tiles a key head has
   int whole;             // blocks up to which a row stays whole
+  int long_from;         // > 0: a row goes in `splits` shares from this many blocks on, else whole (many_rows)
   float apart;           // what a share more costs, in blocks' time
   float* part;   // [row][key head's tile][split]: heads x VD results, then maximum and sum of each head
   int* tickets;  // [row][key head's tile], zero between launches; or null: a second launch adds the shares up
@@ -82,8 +83,11 @@ __device__ inline int quotient(int n, int d) {
 
 // Blocks a share of a row that has n: the rule of attention_decode.hip, with the costs of these sizes (`shares_for`).
 __device__ inline int blocks_a_share(const Shares& sh, int n) {
-  if (n <= sh.whole || sh.splits == 1) return n;
-  const int narrow = quotient(n - 1, sh.narrow) + 1, even = narrow <= NARROW ? narrow : quotient(n - 1, sh.splits) + 1;
+  if (n <= sh.whole || sh.splits == 1 || n < sh.long_from) return n;
+  if (sh.long_from > 0) return quotient(n - 1, sh.splits) + 1;
+  const int narrow = quotient(n - 1, sh.narrow) + 1;
+  const bool alone = narrow <= NARROW || 0.1f * narrow < sh.apart * (sh.splits - sh.narrow);
+  const int even = alone ? narrow : quotient(n - 1, sh.splits) + 1;
   return max(even, __builtin_amdgcn_readfirstlane((int)(__builtin_amdgcn_sqrtf((float)n * sh.apart) + 0.5f)));
 }
 
@@ -413,36 +417,74 @@ int launch(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache,
   return 1;
 }
 
+// How rows are shared out that take more than half of the compute units with one workgroup a tile of heads: in `shares` from `from` units of
+// 32 KB on (0: never); the reasons are attention_decode.hip's, the lines where this kernel has them, whose workgroups have more to
+// work out for what they draw, so that two a unit hide more of one another.  Whole -> so, microseconds, 32 heads of 128 over 8: 17 rows of 1 500 keys
+// 35 -> 27, 24 of 3 000 68 -> 60, 26 of 3 000 with capped scores 75 -> 67, 33 of 750 30.7 -> 28, of 3 000 102 -> 85, 40 of 3 000 109 -> 97, 48 of 1 500
+// 64 -> 61; 16 heads of 64 over 8: 17 of 1 500 22.6 -> 17.3, 28 of 3 000 45 -> 40, 33 of 3 000 55 -> 47.  (Shares that cost: 17 of 250 9.5 and, in
+// three, 11.2; 32 of 3 000 in two 75 for 72; 56 of 1 000 in any number.)
+struct ManyRows {
+  int shares, from;
+};
+ManyRows many_rows(long long tiles) {
+  const long long cus = lq_compute_units();
+  if (3 * tiles <= 2 * cus) return {3, 8};
+  if (4 * tiles <= 3 * cus) return {4, 12};
+  if (8 * tiles <= 7 * cus) return {2, 28};
+  if (tiles <= cus) return {1, 0};
+  if (5 * tiles <= 6 * cus) return {5, 9};
+  if (3 * tiles <= 4 * cus) return {4, 10};
+  if (2 * tiles <= 3 * cus) return {2, 8};
+  return {1, 0};
+}
+
 // How a launch is shared out: `splits` is 1 where no row goes in shares.
 //
 // In units of the time for 32 KB (1.1 us): a block of KD + VD entries takes (KD + VD) / 256, a share more its ticket and its results'
-// way into the last workgroup, 0.06 + 0.07 for every 512 entries.  A row of up to 3.6 units stays whole (24 rows of 100 keys of
-// 256 + 192: 9.4 -> 8.7 us), else a share has the blocks that an even deal gives it and no fewer than the root of n times
-// the quotient of the two.
+// way into the last workgroup, 0.06 + 0.07 for every 512 entries.  A row of up to 3.4 units and four shares' cost stays whole, else a
+// share has the blocks that an even deal gives it and no fewer than the root of n times the quotient of the two.
 //
 // Query heads a workgroup: 16 where rows are many; half as many, and half again, while that makes no more than 128 workgroups a
 // share, down to 4 (the last workgroup of a row then adds up a quarter: 8 rows of 216 to 716 keys 17.6 us with 16 heads, 13.7 with 8, 11.2 with 4), and
-// down to 2 while it makes no more than 32 (4 rows of 700 keys 12.1 -> 10.3, one 10.7 -> 9.2; with 64 of them 11.0 -> 12.0).
+// down to 2 while it makes no more than 32 (4 rows of 700 keys 12.1 -> 10.3, one 10.7 -> 9.2; with 64 of them 11.0 -> 12.0); and while rows of the
+// bound's length give a compute unit no more than 7.5 units to draw: every workgroup draws all of its row's keys (24 rows of 2 500, one key
+// head of 256 with values of 192 under 16 heads, four heads a workgroup 34.6 us, 16 24.0).
 Shares shares_for(int rows, int nh, int nkv, int KD, int VD, int window, int keep_first, int chunk, int max_len) {
   Shares sh = {};
   const int group = nh / nkv, cus = lq_compute_units();
   const float block = (KD + VD) / 256.f;
   auto tiles = [&](int heads) { return (long long)rows * nkv * lq_ceil_div(group, heads); };
+  // blocks that a row may see, within a bound of the lengths
+  auto most_blocks = [&](long long bound) {
+    const long long seen = window > 0 ? (long long)window + keep_first + 2 * BLOCK : bound;
+    long long keys = seen < bound ? seen : bound;
+    if (chunk > 0 && chunk + BLOCK < keys) keys = chunk + BLOCK;
+    return (int)((keys + BLOCK - 1) / BLOCK) + 1;
+  };
   int heads = 16;
-  while (max_len > 0 && ((heads > 4 && tiles(heads / 2) <= 128) || (heads > 2 && tiles(heads / 2) <= 32))) heads /= 2;
+  if (max_len > 0) {
+    // (by the bound in 1 024s: launches whose bounds differ less than that add up their sums in the same order)
+    const long long bound = ((long long)max_len + LQ_DECODE_LENGTH_BUCKET - 1) / LQ_DECODE_LENGTH_BUCKET * LQ_DECODE_LENGTH_BUCKET;
+    const float units = most_blocks(bound) * block / cus;
+    while (((heads > 4 && tiles(heads / 2) <= 128) || (heads > 2 && tiles(heads / 2) <= 32)) && tiles(heads / 2) * units <= 7.5f) heads /= 2;
+  }
+  const float share = 0.06f + 0.07f * (group < heads ? group : heads) * VD / 512.f;
   sh.heads = group < heads ? group : heads;
   sh.tiles = lq_ceil_div(group, sh.heads);
-  sh.whole = 3.6f / block > 1.f ? (int)(3.6f / block) : 1;
-  sh.apart = (0.06f + 0.07f * sh.heads * VD / 512.f) / block;
+  sh.whole = (int)((3.4f + 4 * share) / block) > 1 ? (int)((3.4f + 4 * share) / block) : 1;
+  sh.apart = share / block;
   sh.splits = sh.narrow = 1;
   if (max_len <= 0) return sh;
-  const long long seen = window > 0 ? (long long)window + keep_first + 2 * BLOCK : max_len;
-  int keys = seen < max_len ? (int)seen : max_len;
-  if (chunk > 0 && chunk + BLOCK < keys) keys = chunk + BLOCK;
-  const long long room = 2 * cus / tiles(heads), alone = cus / tiles(heads);
-  const int wanted = lq_ceil_div(keys, BLOCK) + 1, most = room > MAX_SPLITS ? MAX_SPLITS : (int)room;
-  sh.splits = wanted < most ? wanted : most > 1 ? most : 1;
-  sh.narrow = alone > sh.splits ? sh.splits : alone > 1 ? (int)alone : 1;
+  const long long all = tiles(heads), room = 2 * cus / all, alone = cus / all;
+  if (2 * all > cus) {
+    const ManyRows many = many_rows(all);
+    const int from = (int)(many.from / (block > 1.f ? block : 1.f));
+    if (many.shares > 1 && most_blocks(max_len) > from) sh.splits = sh.narrow = many.shares, sh.long_from = from;
+    return sh;
+  }
+  const int wanted = most_blocks(max_len), most = room > MAX_SPLITS ? MAX_SPLITS : (int)room;
+  sh.splits = wanted < most ? wanted : most;
+  sh.narrow = alone > sh.splits ? sh.splits : (int)alone;
   return sh;
 }
 

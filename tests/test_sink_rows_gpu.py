@@ -63,6 +63,15 @@ def test_single_tokens_of_more_blocks_than_a_wavefront_has_lanes(H, G, D, P, opt
     check(H, G, D, P, [(1, n - 1) for n in (160, 63 * 64, 64 * 64 + 1, 65 * 64 + 1)], options, True)
 
 
+@pytest.mark.parametrize("H,G,D,P,rows,start", [(128, 64, 64, 64, 3, 32), (128, 64, 64, 40, 5, 28), (132, 33, 128, 128, 4, 8), (264, 66, 128, 128, 4, 14),
+                                                (160, 80, 128, 256, 4, 6), (380, 95, 128, 128, 4, 28), (64, 16, 256, 192, 9, 4)])
+@pytest.mark.parametrize("options", [PLAIN, dict(sinks=True, window=700, gate=True)])
+def test_single_tokens_of_launches_that_fill_the_chip(H, G, D, P, rows, start, options):
+    """Half to twice as many rows and tiles of heads as compute units: rows of up to some `start` blocks stay whole, longer ones go in shares.  Rows
+    at that line, far beyond it and of one key."""
+    check(H, G, D, P, [(1, n - 1) for n in [start * 64, (start - 1) * 64, start * 64 + 1, 1, 2 * start * 64 + 65, 3, 70, 130, 260][:rows]], options, True)
+
+
 @pytest.mark.parametrize("H,G,D,P,seqs,options", CASES)
 def test_tiles_of_32_rows(H, G, D, P, seqs, options):
     check(H, G, D, P, seqs, options, False)
