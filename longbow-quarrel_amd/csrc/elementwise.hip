@@ -1122,10 +1122,11 @@ __global__ __launch_bounds__(256) void postnorm_residual_kernel(float* __restric
 }
 
 // The same for rows of up to 256 * 4 * KEEP entries, a multiple of four, all operands 16-byte aligned: a thread keeps
-// its entries (four neighbours at a time) in registers from the first pass on, so that a row is read once, and asks for all of them
-// ahead of the first sum; what a single token's step waits for is the passes' round trips, and many rows' too, of which a compute unit
-// holds eight.  2 635 rows of 2 048, one and two pieces: 15.4 to 23.8 us with an entry of x asked for behind the sum, 15.1 to 22.2 so (5 TB/s).
-template <typename T, int KEEP>
+// its entries (four neighbours at a time) in registers from the first pass on, so that a row is read once.  What a single token's step
+// waits for is the passes' round trips: AHEAD asks for all of a row, of up to PIECES pieces, ahead of the first sum.  Many wide rows are bound by the
+// memory and by how many of them a compute unit holds, and keep no more than they must (2 635 rows, asked ahead -> not: one piece, of 2 048
+// 15.3 us either way, of 3 072 23.2 -> 20.0, of 5 120 44 -> 31; two of 2 048 18.1, of 5 120 51 -> 38; one row, four pieces of 4 096 6.3 for 7.1).
+template <typename T, int KEEP, int PIECES, bool AHEAD>
 __global__ __launch_bounds__(256) void postnorm_residual_kept_kernel(float* __restrict__ x, NormPieces in, int n_in,
                                                                      const float* __restrict__ w, float eps,
                                                                      const float* __restrict__ extra,
@@ -1134,25 +1135,29 @@ __global__ __launch_bounds__(256) void postnorm_residual_kept_kernel(float* __re
   __shared__ float red[16];
   const long long base = (long long)blockIdx.x * width;
   const int n4 = width >> 2;
-  float4 y[KEEP][4], old[KEEP], more[KEEP], v[KEEP];
+  constexpr int ASKED = AHEAD ? KEEP : 1;
+  float4 y[ASKED][PIECES], old[ASKED], more[ASKED], v[KEEP];
+  if constexpr (AHEAD)
 #pragma unroll
-  for (int j = 0; j < KEEP; ++j) {
-    const int i = min((int)threadIdx.x + j * 256, n4 - 1);
+    for (int j = 0; j < KEEP; ++j) {
+      const int i = min((int)threadIdx.x + j * 256, n4 - 1);
 #pragma unroll
-    for (int p = 0; p < 4; ++p) y[j][p] = p < n_in ? reinterpret_cast<const float4*>(in.y[p] + base)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    old[j] = reinterpret_cast<const float4*>(x + base)[i];
-    more[j] = extra != nullptr ? reinterpret_cast<const float4*>(extra + base)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+      for (int p = 0; p < PIECES; ++p)
+        y[j][p] = PIECES < 4 || p < n_in ? reinterpret_cast<const float4*>(in.y[p] + base)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      old[j] = reinterpret_cast<const float4*>(x + base)[i];
+      more[j] = extra != nullptr ? reinterpret_cast<const float4*>(extra + base)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  auto piece = [&](int j, int p) { return AHEAD ? y[AHEAD ? j : 0][p] : reinterpret_cast<const float4*>(in.y[p] + base)[threadIdx.x + j * 256]; };
   float acc = 0.f;
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
     if (threadIdx.x + j * 256 < n4) {
-      float4 a = y[j][0];
+      float4 a = piece(j, 0);
       a.x *= in.scale[0], a.y *= in.scale[0], a.z *= in.scale[0], a.w *= in.scale[0];
 #pragma unroll
-      for (int p = 1; p < 4; ++p)
-        if (p < n_in) {
-          const float4 b = y[j][p];
+      for (int p = 1; p < PIECES; ++p)
+        if (PIECES < 4 || p < n_in) {
+          const float4 b = piece(j, p);
           a.x = fmaf(in.scale[p], b.x, a.x), a.y = fmaf(in.scale[p], b.y, a.y);
           a.z = fmaf(in.scale[p], b.z, a.z), a.w = fmaf(in.scale[p], b.w, a.w);
         }
@@ -1165,10 +1170,13 @@ __global__ __launch_bounds__(256) void postnorm_residual_kept_kernel(float* __re
   for (int j = 0; j < KEEP; ++j) {
     const int i = threadIdx.x + j * 256;
     if (i < n4) {
-      float4 a = old[j];
+      float4 a = AHEAD ? old[AHEAD ? j : 0] : reinterpret_cast<const float4*>(x + base)[i];
       const float4 ww = reinterpret_cast<const float4*>(w)[i];
       a.x += v[j].x * inv * ww.x, a.y += v[j].y * inv * ww.y, a.z += v[j].z * inv * ww.z, a.w += v[j].w * inv * ww.w;
-      if (extra != nullptr) a.x += more[j].x, a.y += more[j].y, a.z += more[j].z, a.w += more[j].w;
+      if (extra != nullptr) {
+        const float4 e = AHEAD ? more[AHEAD ? j : 0] : reinterpret_cast<const float4*>(extra + base)[i];
+        a.x += e.x, a.y += e.y, a.z += e.z, a.w += e.w;
+      }
       reinterpret_cast<float4*>(x + base)[i] = a;
       v[j] = a;
       acc2 = fmaf(a.x, a.x, acc2), acc2 = fmaf(a.y, a.y, acc2), acc2 = fmaf(a.z, a.z, acc2), acc2 = fmaf(a.w, a.w, acc2);
@@ -1404,18 +1412,30 @@ extern "C" int lq_postnorm_residual(float* x, const float* y, int pieces, long l
                  (uintptr_t)extra % 16 == 0 && (uintptr_t)next_w % 16 == 0;
   for (int p = 0; p < pieces; ++p) aligned = aligned && (uintptr_t)in.y[p] % 16 == 0;
 #define LQ_POSTNORM(KERNEL, T) KERNEL<<<rows, 256, 0, stream>>>(x, in, pieces, w, eps, extra, next_w, next_eps, (T*)h, width)
-#define LQ_POSTNORM_KEPT(T)                                                                    \
-  do {                                                                                         \
-    if (!aligned) LQ_POSTNORM(postnorm_residual_kernel<T>, T);                                 \
-    else if (width <= 1024) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 1>), T);             \
-    else if (width <= 2048) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 2>), T);             \
-    else if (width <= 4096) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 4>), T);             \
-    else LQ_POSTNORM((postnorm_residual_kept_kernel<T, 8>), T);                                \
+#define LQ_POSTNORM_AHEAD(T, KEEP)                                                                   \
+  do {                                                                                               \
+    if (pieces == 1) LQ_POSTNORM((postnorm_residual_kept_kernel<T, KEEP, 1, true>), T);              \
+    else if (pieces == 2) LQ_POSTNORM((postnorm_residual_kept_kernel<T, KEEP, 2, true>), T);         \
+    else LQ_POSTNORM((postnorm_residual_kept_kernel<T, KEEP, 4, true>), T);                          \
+  } while (0)
+#define LQ_POSTNORM_KEPT(T)                                                                          \
+  do {                                                                                               \
+    const int keep = lq_ceil_div(width, 1024);                                                       \
+    if (!aligned) LQ_POSTNORM(postnorm_residual_kernel<T>, T);                                       \
+    else if (keep == 1) LQ_POSTNORM_AHEAD(T, 1);                                                     \
+    else if (keep == 2) LQ_POSTNORM_AHEAD(T, 2);                                                     \
+    else if (rows >= 1024 && keep <= 4) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 4, 4, false>), T); \
+    else if (rows >= 1024) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 8, 4, false>), T);          \
+    else if (keep == 3) LQ_POSTNORM_AHEAD(T, 3);                                                     \
+    else if (keep == 4) LQ_POSTNORM_AHEAD(T, 4);                                                     \
+    else if (keep <= 6) LQ_POSTNORM_AHEAD(T, 6);                                                     \
+    else LQ_POSTNORM_AHEAD(T, 8);                                                                    \
   } while (0)
   if (h == nullptr || h_dtype == LQ_F32) LQ_POSTNORM_KEPT(float);
   else if (h_dtype == LQ_BF16) LQ_POSTNORM_KEPT(bf16_t);
   else LQ_REQUIRE(false, "postnorm_residual: unknown dtype %d", h_dtype);
 #undef LQ_POSTNORM_KEPT
+#undef LQ_POSTNORM_AHEAD
 #undef LQ_POSTNORM
   LQ_CHECK_LAUNCH("postnorm_residual");
   return 0;

@@ -119,3 +119,26 @@ def test_postnorm_of_every_width(kn, width, pieces, extra, dtype):
     want = stream / (stream.square().mean(1, keepdim=True) + 1e-3).sqrt() * nw.double()
     slack = 2 * bound * (1.0 + nw.abs().double().max()) + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)
     assert ((h.double() - want).abs() <= slack).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [2052, 3072, 3076, 5120, 5124, 6144, 6148, 8188])
+@pytest.mark.parametrize("pieces,extra", [(1, True), (2, False), (3, True), (4, False)])
+def test_postnorm_of_many_wide_rows(kn, width, pieces, extra, dtype):
+    """As few as ask for everything ahead of the sums and as many as do not: the same bits, and 64 bits' results within the bound above."""
+    rows = 1024
+    x, y, w, nw = rnd(rows, width, seed=13), rnd(pieces, rows, width, seed=14), rnd(width, seed=15), rnd(width, seed=16)
+    scales = [0.5, -1.0, 2.0, 1.0][:pieces]
+    more = rnd(rows, width, seed=17) if extra else None
+    outs = []
+    for n in (rows, 3):
+        held, h = x[:n].clone(), torch.zeros((n, width), dtype=dtype, device=DEV)
+        part = y[:, :n].contiguous()
+        kn.postnorm_residual(held, part if pieces > 1 else part[0], scales, w, 1e-5, extra=more[:n] if extra else None, next_weight=nw,
+                             next_eps=1e-3, h=h)
+        outs.append((held, h))
+    for a, b in zip(*outs):
+        assert torch.equal(a[:3], b)
+    v = sum(s * y[p].double() for p, s in enumerate(scales))
+    stream = x.double() + v / (v.square().mean(1, keepdim=True) + 1e-5).sqrt() * w.double() + (more.double() if extra else 0.0)
+    assert (outs[0][0].double() - stream).abs().max() <= 2.0 ** -24 * 32 * (1.0 + stream.abs().max())
