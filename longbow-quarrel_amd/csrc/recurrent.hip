@@ -1094,7 +1094,9 @@ __global__ __launch_bounds__(256) void gated_rmsnorm4_kernel(const float* __rest
 // Many rows and groups of up to 4 LANES columns (128): LANES lanes a group and four rows a thread, all asked for together.
 // (A wavefront a row and group had at most two loads on their way a lane, and half of its lanes none where a group has 128:
 // 2 048 rows of 32 groups of 128 took 20.6 us, now 15.2.  Groups of 256 with 64 lanes took 12.9, a wavefront a row and
-// group 11.1: they stay there, and so do few rows, which a fourth of the wavefronts would not spread over the chip.)
+// group 11.1: they stay there, and so do few rows and groups, which a fourth of the wavefronts would not spread over the chip, above all
+// where a workgroup's eight groups are not there: 512 rows of four 3.5 us, so 5.3; of 16 5.6 and 5.4; 2 048 of four 5.5 and 6.4, of six 8.3 and 6.4;
+// 4 096 of two 6.1 and 5.4.)
 constexpr int GATED_ROWS = 4;
 template <typename T, int LANES>
 __global__ __launch_bounds__(256) void gated_rmsnorm_rows_kernel(const float* __restrict__ y, int ldy, const float* __restrict__ z,
@@ -1538,7 +1540,7 @@ extern "C" int lq_gated_rmsnorm(const float* y, int ldy, const float* z, int ldz
   const bool fours = group % 4 == 0 && group <= 8192 && ldy % 4 == 0 && ldz % 4 == 0 && ldo % 4 == 0 && (w == nullptr || wlen % 4 == 0) &&
                      (uintptr_t)y % 16 == 0 && (uintptr_t)z % 16 == 0 && (uintptr_t)w % 16 == 0 &&
                      (uintptr_t)out % (4 * el) == 0 && (out_dtype == LQ_F32 || out_dtype == LQ_BF16);
-  if (fours && group <= 128 && rows >= 512 && rows <= 65535 * GATED_ROWS) {
+  if (fours && group <= 128 && rows >= 512 && rows <= 65535 * GATED_ROWS && (long long)rows * groups >= (groups % 8 == 0 || rows >= 4096 ? 8192 : 10240)) {
 #define LQ_GATED_ROWS(T, LANES)                                                                                                    \
   gated_rmsnorm_rows_kernel<T, LANES><<<dim3(lq_ceil_div(groups, 256 / LANES), lq_ceil_div(rows, GATED_ROWS)), 256, 0, stream>>>( \
       y, ldy, z, ldz, w, wlen, eps, group, groups, (T*)out, ldo, rows, gate_first, sigmoid_gate)

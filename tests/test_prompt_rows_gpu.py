@@ -74,6 +74,13 @@ def test_gated_norms_of_many_rows(kn, group, groups, wlen, rows, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("group,groups,wlen,rows", [(128, 1, 128, 8193), (64, 3, 64, 4099), (4, 2, 8, 5121), (100, 9, 900, 1140), (128, 16, 0, 513)])
+def test_gated_norms_of_many_rows_and_few_groups(kn, group, groups, wlen, rows, dtype):
+    """As many rows as a few groups need for four rows a thread."""
+    test_gated_norms_of_many_rows(kn, group, groups, wlen, rows, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows,width,pieces", [(1, 4, 1), (3, 260, 0), (3, 260, 5), (70, 1028, 2), (7, 130, 2), (5, 33, 3)])
 def test_dynamic_tanh_in_fours(kn, rows, width, pieces, dtype):
     """Widths in fours and others, against 64 bits; x off a multiple of 16 bytes gives the same as on one."""
