@@ -71,7 +71,8 @@ __device__ inline float4 summed4(const float4* __restrict__ delta, int pieces, l
 
 // The same two in fours (n and the width in fours, all operands on 16 bytes, out on 8): every load of a thread is asked for ahead of the
 // first use, and no 64-bit remainder lies in front of the weights'.  2 048 rows of 2 048, two pieces of a
-// delta: 20.2 us entry by entry, 13.8 so (5.3 TB/s); the add 17.1 and 13.6.
+// delta: 20.2 us entry by entry, 13.8 so (5.3 TB/s); the add 17.1 and 13.6.  Few entries, of which a thread then has four tangents in turn, go one a
+// thread (64 rows of 2 048 2.9 us, so 3.2; 512 of 1 024 3.7 and 3.6; the add 64 rows of 2 048 2.8 and 2.9, 512 of 512 2.9 and 2.7).
 template <typename T>
 __global__ __launch_bounds__(256) void dynamic_tanh4_kernel(float4* __restrict__ x, const float4* __restrict__ delta, int pieces,
                                                             long long stride4, float scale, const float4* __restrict__ w,
@@ -1210,7 +1211,7 @@ extern "C" int lq_dynamic_tanh(float* x, const float* delta, int pieces, long lo
   LQ_REQUIRE(pieces >= 0 && (pieces == 0 || delta != nullptr), "dynamic_tanh: %d pieces of a delta", pieces);
   const long long n = (long long)rows * width;
   const unsigned blocks = (unsigned)((n + 255) / 256);
-  if (width % 4 == 0 && n / 4 < 0x7fffffffll - 255 && (out_dtype == LQ_F32 || out_dtype == LQ_BF16) && delta_in_fours(delta, pieces, piece_stride) &&
+  if (n >= 1 << 19 && width % 4 == 0 && n / 4 < 0x7fffffffll - 255 && (out_dtype == LQ_F32 || out_dtype == LQ_BF16) && delta_in_fours(delta, pieces, piece_stride) &&
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b) & 15) == 0 && (uintptr_t)out % (out_dtype == LQ_F32 ? 16 : 8) == 0) {
     const unsigned n4 = (unsigned)(n / 4), fours = (n4 + 255) / 256;
 #define LQ_TANH4(T)                                                                                                                  \
@@ -1232,7 +1233,7 @@ extern "C" int lq_dynamic_tanh(float* x, const float* delta, int pieces, long lo
 extern "C" int lq_add_scaled(float* x, const float* delta, int pieces, long long piece_stride, float scale, long long n,
                              hipStream_t stream) {
   LQ_REQUIRE(x && delta && pieces > 0 && n > 0, "add_scaled: bad arguments");
-  if (n % 4 == 0 && n / 4 < 0x7fffffffll - 255 && (uintptr_t)x % 16 == 0 && delta_in_fours(delta, pieces, piece_stride))
+  if (n >= 1 << 18 && n % 4 == 0 && n / 4 < 0x7fffffffll - 255 && (uintptr_t)x % 16 == 0 && delta_in_fours(delta, pieces, piece_stride))
     add_scaled4_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, stream>>>((float4*)x, (const float4*)delta, pieces, piece_stride / 4, scale,
                                                                             (unsigned)(n / 4));
   else

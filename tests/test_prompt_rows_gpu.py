@@ -108,6 +108,13 @@ def test_dynamic_tanh_in_fours(kn, rows, width, pieces, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,width,pieces", [(131073, 4, 1), (521, 1028, 0), (521, 1028, 5), (1030, 516, 2)])
+def test_dynamic_tanh_of_many_entries(kn, rows, width, pieces, dtype):
+    """As many entries as are taken in fours."""
+    test_dynamic_tanh_in_fours(kn, rows, width, pieces, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width", [4, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 130])
 @pytest.mark.parametrize("pieces,extra", [(1, False), (2, True), (4, False)])
 def test_postnorm_of_every_width(kn, width, pieces, extra, dtype):
