@@ -535,10 +535,20 @@ extern "C" int lq_moe_route(const float* z, int ldz, float* route, int rows, int
   return 0;
 }
 
-// Whether lq_moe_router takes the router's product [rows, K] x [N, K]^T and the choice together.  Up to 16 rows: every row's workgroup
-// reads the whole weight, which for more of them the product reads once.
+// Whether lq_moe_router takes the router's product [rows, K] x [N, K]^T and the choice together.
 extern "C" int lq_moe_router_takes(int dtype, int rows, int K, int N) {
   return dtype == LQ_BF16 && rows >= 1 && rows <= 16 && K >= 8 && K % 8 == 0 && N >= 1 && N <= ROUTER_MOST;
+}
+
+// Whether that is faster than the product and the choice in a launch each.  Every row's workgroup reads the whole
+// weight, at what one compute unit draws (and for more than 16 outputs in more than one round of its wavefronts); the product reads it
+// with all of them, and from 9 rows on takes another kernel that is slower here.  Weights from memory, us, two launches -> one: 1 and 8 rows, 8 outputs of
+// 2 048 5.6 -> 4.5 and 6.8 -> 4.8, 16 of 3 072 6.9 -> 5.5 and 7.8 -> 5.9, 32 of 1 536 6.5 -> 6.1 and 7.1 -> 6.6, but 32 of 2 048 7.1 -> 8.5 and 8.1 -> 8.7, 8 of
+// 7 168 8.9 -> 10.5 and 10.9 -> 10.2, 64 of 2 048 7.9 -> 14.2; 9 and 16 rows, 16 of 7 168 16.7 -> 11.1 and 19.5 -> 11, 32 of 2 048 9.2 -> 8.6 and 10 -> 8.6, but 32 of
+// 4 096 12 -> 12.7, 64 of 1 024 8.7 -> 10.
+extern "C" int lq_moe_router_pays(int dtype, int rows, int K, int N) {
+  if (!lq_moe_router_takes(dtype, rows, K, N) || N > 32) return 0;
+  return (long long)N * K <= (rows <= 8 ? 49152 : N <= 16 ? 114688 : 65536);
 }
 
 // z[rows, N] = h . w^T, and lq_moe_route of z's first `experts` columns.

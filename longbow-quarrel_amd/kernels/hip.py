@@ -1810,6 +1810,13 @@ class HipKernels:
             return False
         return bool(self.lib.lq_moe_router_takes(c_int(_DTYPE_CODE[dtype]), c_int(rows), c_int(width), c_int(outputs)))
 
+    @query
+    def moe_router_pays(self, dtype: torch.dtype, rows: int, width: int, outputs: int) -> bool:
+        """Whether `moe_router` takes such a router and is faster than `linear` and `moe_route`."""
+        if self.force_generic or dtype not in _DTYPE_CODE:
+            return False
+        return bool(self.lib.lq_moe_router_pays(c_int(_DTYPE_CODE[dtype]), c_int(rows), c_int(width), c_int(outputs)))
+
     def moe_router(self, h: torch.Tensor, w: torch.Tensor, logits: torch.Tensor, experts: int, route: torch.Tensor, top: int,
                    renormalize: bool = False, correction: Optional[torch.Tensor] = None, groups: int = 0, keep: int = 0,
                    scoring: str = "sigmoid", group_mark: str = "top2", renormalize_eps: float = 0.0,

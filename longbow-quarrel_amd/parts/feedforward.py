@@ -380,9 +380,9 @@ class MixtureOfExperts(FeedForward):
         kn, rows, E, N = ctx.kernels, h.shape[0], self.experts, self.outputs
         nz = N + (1 if self.shared_gate else 0)
         z = ctx.ws.alloc((rows, (nz + 3) // 4 * 4), torch.float32)[:, :nz]
-        takes = getattr(kn, "moe_router_takes", None)
-        together = takes is not None and self.w_router.dtype == h.dtype == ctx.dtype and h.stride(1) == 1 \
-            and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and self.w_router.data_ptr() % 16 == 0 and takes(h.dtype, rows, self.width, nz)
+        pays = getattr(kn, "moe_router_pays", None)
+        together = pays is not None and self.w_router.dtype == h.dtype == ctx.dtype and h.stride(1) == 1 \
+            and h.stride(0) % 8 == 0 and h.data_ptr() % 16 == 0 and self.w_router.data_ptr() % 16 == 0 and pays(h.dtype, rows, self.width, nz)
         if not together:
             project(kn, ctx, h, self.w_router, z)
         route = ctx.ws.alloc((rows, E), torch.float32)  # the weight of a chosen expert, -1 for the others

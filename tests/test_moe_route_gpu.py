@@ -116,3 +116,10 @@ def test_the_product_and_the_choice_in_one_launch(kn, rows, K, E, extra, scoring
         options["identity"] = torch.empty_like(passed)
     kn.moe_route(z[:, :E], want, top, True, **options)
     assert torch.equal(route, want) and (passed is None or torch.equal(passed, options["identity"]))
+
+
+def test_large_routers_go_in_two_launches(kn):
+    """One launch reads the whole weight a row by one compute unit: it is taken for as much as that pays for."""
+    pays = lambda rows, K, N: kn.moe_router_pays(torch.bfloat16, rows, K, N)
+    assert pays(1, 2048, 8) and pays(8, 3072, 16) and pays(16, 7168, 16) and pays(9, 2048, 32)
+    assert not (pays(8, 2048, 64) or pays(1, 4096, 32) or pays(1, 7168, 8) or pays(16, 4096, 32) or pays(17, 2048, 8) or pays(16, 256, 64))
