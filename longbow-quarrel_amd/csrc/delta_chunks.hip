@@ -629,10 +629,9 @@ __global__ __launch_bounds__(512, 2) void gla_walk_kernel(DeltaArgs a) {
 
 // Float32 scratch with which a launch runs in chunks (0: token by token).  Microseconds a launch, token by token and in
 // chunks, 16 heads of 128 x 128 over 8 q/k heads, a decay every channel (the unit vectors' launch in both): 48 tokens
-// 32 / 34, 64 tokens 40 / 35, 256 tokens 124 / 49, 2 048 tokens 900 / 172 (one decay a head 651 / 169), 8 192 tokens
-// 3 560 / 715, three sequences of 257, 878 and 1 500 tokens 769 / 208, eight of 60 92 / 60, eight of 512 584 / 242.  Of
-// 2 048 tokens' 172 the preparation is 50 (21 for a workgroup by itself, a compute unit's LDS holds one), the walk 110
-// (3.3 a chunk, of which the matrix instructions of a SIMD are 1.5: half the chip is idle with 128 workgroups).
+// 32 / 34, 64 tokens 39 / 34, 256 tokens 124 / 49, 2 048 tokens 902 / 148 (one decay a head 654 / 146), eight of 64 93 / 62, eight of 512
+// 586 / 230.  Of 2 048 tokens' 148 the preparation is 50 (21 for a workgroup by itself, a compute unit's LDS holds one), the walk 85
+// (2.55 a chunk, of which the matrix instructions of a SIMD are 1.5: half the chip is idle with 128 workgroups).
 // Relative error against 64 bits at 2 048 tokens: 3.3e-7 both ways with a decay every channel, 4.9e-7 and 5.1e-7
 // with one a head; of the state at their end 3.4e-7 and 3.3e-7, 4.5e-7 both.
 constexpr int LQ_DELTA_MIN = 56;
@@ -660,10 +659,11 @@ extern "C" long long lq_delta_scan_least(int heads) { return (long long)heads * 
 // Whether a launch is faster in chunks (given scratch) than token by token, by what both take.  A chunk costs the same
 // whatever the sizes (their zeros are multiplied too) and however few tokens it has; a walk's token costs little where
 // states are small or one decay serves a head, as soon as there are workgroups for the whole chip.  Microseconds, walk /
-// chunks, 16 heads of 128 x 128: a decay a head, 70 sequences of 64 tokens 306 / 418, of 200 845 / 1 163, 16 of 100
-// 126 / 151, eight of 512 267 / 215, one of 256 89 / 44; a decay a channel, 16 of 64 171 / 112, 70 of 200 2 037 / 1 249;
-// of 64 x 64, 16 of 128 74 / 107.
-// (Of a walk over chunks of 3.4 microseconds each; it takes 2.55 now, so that the line leaves some launches near it token by token.)
+// chunks, 16 heads of 128 x 128: a decay a head, one of 64 tokens 30 / 32, of 256 89 / 44, 16 of 100 124 / 134, of 200 231 / 222, eight of
+// 512 284 / 212, 200 beside 16 of 1 87 / 64; a decay a channel, 16 of 64 173 / 117, 70 of 64 681 / 443; of 64 x 64, 200 beside 16 of 1 73 / 49,
+// with a decay a channel eight of 130 64 / 78, 16 of 512 261 / 368.  Over 1 800 launches (nine sizes, both decays, 1 to 128 sequences, alike or one beside
+// shorter ones) the way that is named takes 0.4 % more than the better of the two, and in 49 of them 5 % and more.  (Priced as when a
+// chunk of the walk took 3.4 microseconds, and with a tenth in the chunks' favour: 1.0 %, and 95.)
 extern "C" int lq_delta_scan_in_chunks(int rows, int batch, int heads, int Dk, int P, int max_rows, int channel_decay) {
   if (lq_delta_scan_workspace(rows, batch, heads, Dk, P, max_rows) == 0) return 0;
   const double size = P / 128.0 * (Dk > 64 ? Dk / 128.0 : 0.4), cols = (P + 15) / 16;
@@ -676,10 +676,10 @@ extern "C" int lq_delta_scan_in_chunks(int rows, int batch, int heads, int Dk, i
   const double rest = rows - max_rows, least = lq_delta_least_rows(rows, batch, heads, channel_decay);
   const bool alike = batch == 1 || rest >= least * (batch - 1);
   const double in_chunks = alike ? batch : 1, of_chunks = (alike ? rows : max_rows) / 64.0 + in_chunks / 2;
-  const double products = 0.0145 * cols * heads * of_chunks, chain = 3.3 * (max_rows / 64 + 1);
+  const double products = 0.0113 * cols * heads * of_chunks, chain = 2.55 * (max_rows / 64 + 1);
   double chunks = 25 + 0.085 * heads * of_chunks + (products > chain ? products : chain) + 0.15 * P / 128 * heads * in_chunks;
-  if (!alike) chunks += 20 + walk(rest, least, batch - 1);
-  return 0.9 * chunks < walk(rows, max_rows, batch);
+  if (!alike) chunks += walk(rest, least, batch - 1);
+  return chunks < walk(rows, max_rows, batch);
 }
 
 // q and k hold unit vectors already.  `scratch`: at least a chunk's floats for every head.  -> 0, or -2

@@ -37,6 +37,20 @@ def test_gated_linear_attention_goes_in_chunks_where_that_is_faster(lib, heads, 
     assert lib.lq_gla_scan_in_chunks(sum(lengths), len(lengths), heads, dk, dv, max(lengths)) == chunks
 
 
+@pytest.mark.parametrize("heads,dk,dv,lengths,channel,chunks", [
+    # microseconds measured, token by token and in chunks
+    (16, 64, 64, [200] + [1] * 16, 0, True),     # 73, 49
+    (16, 128, 128, [200] + [8] * 16, 0, True),   # 93, 70
+    (8, 64, 128, [200] + [1] * 70, 0, True),     # 80, 59
+    (16, 128, 128, [64], 0, False),              # 30, 32
+    (16, 64, 64, [130] * 8, 1, False),           # 64, 78
+    (16, 64, 64, [512] * 16, 1, False),          # 261, 368
+    (32, 128, 128, [64] + [1] * 70, 1, False),   # 329, 384
+    (16, 128, 128, [2048], 0, True)])            # 654, 146
+def test_the_delta_rule_goes_in_chunks_where_that_is_faster(lib, heads, dk, dv, lengths, channel, chunks):
+    assert lib.lq_delta_scan_in_chunks(sum(lengths), len(lengths), heads, dk, dv, max(lengths), channel) == chunks
+
+
 def test_what_gated_linear_attention_does_not_take_in_chunks(lib):
     for sizes in ((0, 1, 8, 128, 256, 0), (500, 1, 8, 129, 256, 500), (47, 1, 8, 128, 256, 47), (3000, 1, 0, 128, 256, 3000)):
         assert lib.lq_gla_scan_in_chunks(*sizes) == 0
