@@ -223,9 +223,10 @@ __global__ __launch_bounds__(256) void causal_conv4_kernel(const T* __restrict__
     const int r = first + i;
     if (r >= rows) break;
     const int b = seqs[i];
+    long long slot = TILE ? 0 : (long long)seq_slot[b] * (TAPS - 1);  // (asked for beside the row's place; a tile's rows seldom need it)
     if (b != before) {  // a tile's first row, or another sequence's
       const int since = row_pos[r] - seq_start[b];  // rows of this step before this one, in its sequence
-      const long long slot = since < TAPS - 1 ? (long long)seq_slot[b] * (TAPS - 1) : 0;
+      if (TILE && since < TAPS - 1) slot = (long long)seq_slot[b] * (TAPS - 1);
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) {
         const int back = TAPS - 1 - j;
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(256) void causal_conv4_kernel(const T* __restrict__
     store4<T>(out + (long long)r * ldo + c,
               make_float4(activate(acc.x, act), activate(acc.y, act), activate(acc.z, act), activate(acc.w, act)));
     if (single) {
-      const long long slot = (long long)seq_slot[b] * (TAPS - 1);
+      if (TILE) slot = (long long)seq_slot[b] * (TAPS - 1);
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) *(float4*)(state + (slot + j) * C + c) = hist[j + 1];
     }
