@@ -1411,6 +1411,11 @@ extern "C" int lq_postnorm_residual(float* x, const float* y, int pieces, long l
   bool aligned = width % 4 == 0 && width <= 256 * 4 * 8 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 &&
                  (uintptr_t)extra % 16 == 0 && (uintptr_t)next_w % 16 == 0;
   for (int p = 0; p < pieces; ++p) aligned = aligned && (uintptr_t)in.y[p] % 16 == 0;
+  // Rows wider than 2 048 are not asked for ahead of the sums where they are more than two a compute unit and their pieces and the stream more
+  // than 11 M entries, with which the registers of all that is asked for cost more rows in flight than a trip saves.  us, ahead and not: three
+  // pieces of 5 120, 512 rows 12.8 and 13.3, 768 16.9 and 15.7, 1 000 23.5 and 18.7; four of 8 192, 400 rows 18.8 and 20.3, 640 29.7 and 23.3; two of
+  // 4 096, 768 rows 11.5 and 12.0, 1 000 14.2 and 13.6; one of 2 560, 2 048 rows 12.6 and 13.0, of 5 120 25.7 and 23.0.
+  const bool many = rows > 512 && (long long)rows * width * (pieces + 1) >= 11000000;
 #define LQ_POSTNORM(KERNEL, T) KERNEL<<<rows, 256, 0, stream>>>(x, in, pieces, w, eps, extra, next_w, next_eps, (T*)h, width)
 #define LQ_POSTNORM_AHEAD(T, KEEP)                                                                   \
   do {                                                                                               \
@@ -1424,8 +1429,8 @@ extern "C" int lq_postnorm_residual(float* x, const float* y, int pieces, long l
     if (!aligned) LQ_POSTNORM(postnorm_residual_kernel<T>, T);                                       \
     else if (keep == 1) LQ_POSTNORM_AHEAD(T, 1);                                                     \
     else if (keep == 2) LQ_POSTNORM_AHEAD(T, 2);                                                     \
-    else if (rows >= 1024 && keep <= 4) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 4, 4, false>), T); \
-    else if (rows >= 1024) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 8, 4, false>), T);          \
+    else if (many && keep <= 4) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 4, 4, false>), T);     \
+    else if (many) LQ_POSTNORM((postnorm_residual_kept_kernel<T, 8, 4, false>), T);                  \
     else if (keep == 3) LQ_POSTNORM_AHEAD(T, 3);                                                     \
     else if (keep == 4) LQ_POSTNORM_AHEAD(T, 4);                                                     \
     else if (keep <= 6) LQ_POSTNORM_AHEAD(T, 6);                                                     \

@@ -140,7 +140,7 @@ def test_postnorm_of_every_width(kn, width, pieces, extra, dtype):
 @pytest.mark.parametrize("pieces,extra", [(1, True), (2, False), (3, True), (4, False)])
 def test_postnorm_of_many_wide_rows(kn, width, pieces, extra, dtype):
     """As few as ask for everything ahead of the sums and as many as do not: the same bits, and 64 bits' results within the bound above."""
-    rows = 1024
+    rows = max(513, 11000000 // (width * (pieces + 1)) + 1)
     x, y, w, nw = rnd(rows, width, seed=13), rnd(pieces, rows, width, seed=14), rnd(width, seed=15), rnd(width, seed=16)
     scales = [0.5, -1.0, 2.0, 1.0][:pieces]
     more = rnd(rows, width, seed=17) if extra else None
