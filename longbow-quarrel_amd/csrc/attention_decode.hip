@@ -631,30 +631,40 @@ int launch(const DecodeArgs& a, hipStream_t stream) {
 }  // namespace
 
 // How rows are shared out that take more than half of the compute units with one workgroup a kv head: in `shares` from `from` blocks on
-// (0: never).  A unit draws at most 29 GB/s and holds two workgroups (three at head sizes up to 64);
+// (0: never).  A unit draws at most 29 GB/s and holds two workgroups (three at head sizes up to 64, four of 96, one of 256);
 // the memory gives all of them 20 each.  Up to a row a unit that is enough, but for the units that have none: few more rows than half
-// of them go in thirds, which give every unit two, and the longest up to four fifths of them in fifths, four in turn.  With more
-// rows than units whole ones would leave some units two and most one: shares even that out where they fill a whole number of rounds
-// of two (three) nearly.  A share more costs its ticket and partial results, and a round its chain of round trips: short rows stay whole.
+// of them go in thirds, which give every unit two, and the longest up to four fifths of them in fifths, four in turn (heads of 96, of
+// which a unit has 24 KB on the way, from shorter ones on).  With more
+// rows than units whole ones would leave some units two and most one, and with more than twice as many some three: shares even that out where
+// they fill a whole number of rounds of two (three) nearly.  A share more costs its ticket and partial results, and a round its chain of round
+// trips: short rows stay whole.
 // 32 heads over 8, whole -> so, microseconds; a wavefront with a block of its own and up to 2 048 workgroups in brackets:
 // head size 128: 17 sequences of 1 500 keys 31 -> 28 (38), of 6 000 106 -> 84 (91); 22 of 6 000 114 -> 107 (108); 33 of 1 000 41.5 -> 38 (46), of
-// 3 000 106 -> 84 (101), of 6 000 203 -> 161 (176); 40 of 3 000 108 -> 94 (107); 48 of 6 000 223 -> 206 (214).  Head size 64: 17 of 3 000 34 -> 27
-// (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 48 of 6 000 117 -> 110 (112).
+// 3 000 106 -> 84 (101), of 6 000 203 -> 161 (176); 40 of 3 000 108 -> 94 (107); 48 of 6 000 223 -> 206 (214); 66 of 3 000 176 -> 153; 80 of 1 500
+// 108 -> 100, of 6 000 418 -> 341; 88 of 3 000 216 -> 196; 96 of 2 000 154 -> 146 (138).  Head size 64: 17 of 3 000 34 -> 27
+// (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 48 of 6 000 117 -> 110 (112); 66 of 3 000 92 -> 81; 80 of 6 000 186 -> 175; 16 heads over
+// as many, 33 of 8 000 235 -> 194 (197).  12 heads of 96: 16 of 3 000 48 -> 43; 43 of 750 36 -> 33, of 3 000 130 -> 112; 48 of 4 000 177 -> 154 (159).
+// Eight heads over 4 of 192: 75 of 750 45 -> 39; 144 of 3 000 257 -> 234.
 // (Rows whole that would do in shares, or the reverse: 24 of 200 keys in two shares each 12.5, whole 9.5; 24 of 6 000 118 and 110; 52 of 3 000
-// in sixes 127, whole 118.)
+// in sixes 127, whole 118; 104 of 1 500 in threes 125, whole 122; 128 of 3 000 in twos 279, whole 266.)
 struct ManyRows {
   int shares, from;
 };
 static ManyRows many_rows(long long pairs, int hd) {
   const long long cus = lq_compute_units();
-  const bool small = hd <= 64;
+  const bool small = hd <= 64, narrow = hd == 96;  // (less than 32 KB a block)
   if (3 * pairs <= 2 * cus) return {3, small ? 16 : 12};
-  if (small && 4 * pairs <= 3 * cus) return {4, 32};
-  if (!small && 5 * pairs <= 4 * cus) return {5, 80};
+  if ((small || narrow) && 4 * pairs <= 3 * cus) return {4, small ? 32 : 20};
+  if (!small && 5 * pairs <= 4 * cus) return {5, narrow ? 20 : 80};
   if (pairs <= cus) return {1, 0};
-  if (5 * pairs <= 6 * cus) return {5, small ? 16 : 14};
-  if (!small && 3 * pairs <= 4 * cus) return {3, 14};
+  if (5 * pairs <= 6 * cus) return {5, small ? 16 : hd > 128 ? 10 : 14};
+  if (!small && 3 * pairs <= 4 * cus) return {3, hd > 128 ? 10 : 14};
   if (2 * pairs <= 3 * cus) return {4, 28};
+  if (pairs <= 2 * cus) return {1, 0};
+  if (hd > 192) return {1, 0};
+  if (small && 5 * pairs > 12 * cus) return 2 * pairs <= 5 * cus ? ManyRows{2, 28} : ManyRows{1, 0};
+  if (2 * pairs <= 5 * cus) return {4, narrow ? 10 : 18};
+  if (hd == 128 && pairs <= 3 * cus) return {2, 14};
   return {1, 0};
 }
 

@@ -69,10 +69,12 @@ def test_rows_of_more_blocks_than_a_wavefront_has_lanes(kn, kv_heads, head_dim):
 
 
 @pytest.mark.parametrize("rows,kv_heads,head_dim,start", [(17, 8, 128, 12), (21, 8, 64, 16), (3, 64, 64, 32), (3, 64, 128, 80), (33, 8, 192, 14),
-                                                          (5, 64, 128, 14), (6, 64, 128, 28), (6, 64, 64, 28), (12, 32, 256, 28)])
+                                                          (5, 64, 128, 14), (6, 64, 128, 28), (6, 64, 64, 28), (12, 32, 256, 28),
+                                                          (3, 64, 96, 20), (5, 64, 192, 10), (9, 64, 96, 10), (9, 64, 128, 18), (9, 64, 192, 18),
+                                                          (11, 64, 128, 14), (9, 64, 64, 20), (10, 64, 64, 28)])
 @pytest.mark.parametrize("window", [0, 1000])
 def test_long_rows_of_launches_that_fill_the_chip(kn, rows, kv_heads, head_dim, start, window):
-    """Launches of half to twice as many rows and kv heads as compute units: rows of up to `start` blocks stay whole, longer ones go
+    """Launches of half to three times as many rows and kv heads as compute units: rows of up to `start` blocks stay whole, longer ones go
     in shares, which its last workgroup adds up, so that the units have equal parts.  Rows at that line, far beyond it and of one
     key; twice the same, with the counters at zero after each."""
     lengths = ([start * BS, (start - 1) * BS, (start - 1) * BS + 1, 3 * start * BS + 65, 1, start * BS + 1] * rows)[:rows]
