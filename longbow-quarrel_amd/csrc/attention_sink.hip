@@ -438,8 +438,9 @@ extern "C" long long lq_sink_attention_workspace(int dtype, int rows, int batch,
 }
 
 // `gate`: null, or [rows, nh] logits (stride ldg) in the dtype of q.  `rows == batch` means single tokens.  `part`:
-// lq_sink_attention_workspace(...) floats for `max_len`, or null; `tickets`: a counter a row and key head's 16 query
-// heads, zero, and left zero, that no launch beside this one uses (null or too few: one launch more).  `cap` to `dist_n`: how a score is shaped (see the
+// lq_sink_attention_workspace(...) floats for `max_len`, or null; `tickets`: a counter a row and tile of a key
+// head's query heads (up to 16 of them; down to two where that makes no more than 128 tiles in all), zero, and left zero, that no launch beside this one uses
+// (null or too few: one launch more).  `cap` to `dist_n`: how a score is shaped (see the
 // top of the file; 0 and null: not), `wide_gate` [rows, nh * VD] 32-bit logits (stride ldwg) or null.
 extern "C" int lq_sink_attention(const void* q, int ldq, void* out, int ldo, const void* gate, int ldg, int dtype, int rows,
                                  int batch, int nh, int nkv, int KD, int VD, const int* row_pos, const int* row_seq,

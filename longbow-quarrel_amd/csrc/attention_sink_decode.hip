@@ -422,15 +422,17 @@ int launch(const bf16_t* q, void* out, const bf16_t* gate, const bf16_t* kcache,
 // work out for what they draw, so that two a unit hide more of one another.  Whole -> so, microseconds, 32 heads of 128 over 8: 17 rows of 1 500 keys
 // 35 -> 27, 24 of 3 000 68 -> 60, 26 of 3 000 with capped scores 75 -> 67, 33 of 750 30.7 -> 28, of 3 000 102 -> 85, 40 of 3 000 109 -> 97, 48 of 1 500
 // 64 -> 61; 16 heads of 64 over 8: 17 of 1 500 22.6 -> 17.3, 28 of 3 000 45 -> 40, 33 of 3 000 55 -> 47.  (Shares that cost: 17 of 250 9.5 and, in
-// three, 11.2; 32 of 3 000 in two 75 for 72; 56 of 1 000 in any number.)
+// three, 11.2; 32 of 3 000 in two 75 for 72; 56 of 1 000 in any number.)  A row a unit is not enough where tiles of one
+// key head draw the same keys (40 heads of 64 with values of 40 over 2, 64 rows of 3 000 40 -> 33) and for sizes up to 64 (16 heads over 4, 64 of 3 000
+// 42.1 -> 40.5; 64 of 1 000 18.4, in two 18.7): `light`.
 struct ManyRows {
   int shares, from;
 };
-ManyRows many_rows(long long tiles) {
+ManyRows many_rows(long long tiles, bool light) {
   const long long cus = lq_compute_units();
   if (3 * tiles <= 2 * cus) return {3, 8};
   if (4 * tiles <= 3 * cus) return {4, 12};
-  if (8 * tiles <= 7 * cus) return {2, 28};
+  if (8 * tiles <= 7 * cus || (light && tiles <= cus)) return {2, 28};
   if (tiles <= cus) return {1, 0};
   if (5 * tiles <= 6 * cus) return {5, 9};
   if (3 * tiles <= 4 * cus) return {4, 10};
@@ -449,10 +451,16 @@ ManyRows many_rows(long long tiles) {
 // down to 2 while it makes no more than 32 (4 rows of 700 keys 12.1 -> 10.3, one 10.7 -> 9.2; with 64 of them 11.0 -> 12.0); and while rows of the
 // bound's length give a compute unit no more than 7.5 units to draw: every workgroup draws all of its row's keys (24 rows of 2 500, one key
 // head of 256 with values of 192 under 16 heads, four heads a workgroup 34.6 us, 16 24.0).
+//
+// Sizes of up to 64 take two blocks together, in 0.75 us each: a row of two such takes stays whole, or of three where there are many tiles (one to eight
+// rows, 16 heads over 8 or 4, 260 keys whole 7.6 us, in shares 6.7, 380 8.1 and 6.8, 440 9.3 and 7.1; 16 rows over 8, 320 keys 8.1 and 8.4, 440 9.8 and 8.9).
+// Their heads are split no further than to a pair of entries a thread of the last workgroup, from where on it has nothing to save (64 heads over 8 under
+// a window of 128, one to four rows, two heads a workgroup 6.5 us, eight 6.2; 32 over 4, one row of 500 7.3 and 6.2, of 3 000 11.5 and 9.1).
 Shares shares_for(int rows, int nh, int nkv, int KD, int VD, int window, int keep_first, int chunk, int max_len) {
   Shares sh = {};
   const int group = nh / nkv, cus = lq_compute_units();
   const float block = (KD + VD) / 256.f;
+  const bool small = KD <= 64 && VD <= 64;
   auto tiles = [&](int heads) { return (long long)rows * nkv * lq_ceil_div(group, heads); };
   // blocks that a row may see, within a bound of the lengths
   auto most_blocks = [&](long long bound) {
@@ -466,18 +474,21 @@ Shares shares_for(int rows, int nh, int nkv, int KD, int VD, int window, int kee
     // (by the bound in 1 024s: launches whose bounds differ less than that add up their sums in the same order)
     const long long bound = ((long long)max_len + LQ_DECODE_LENGTH_BUCKET - 1) / LQ_DECODE_LENGTH_BUCKET * LQ_DECODE_LENGTH_BUCKET;
     const float units = most_blocks(bound) * block / cus;
-    while (((heads > 4 && tiles(heads / 2) <= 128) || (heads > 2 && tiles(heads / 2) <= 32)) && tiles(heads / 2) * units <= 7.5f) heads /= 2;
+    while (((heads > 4 && tiles(heads / 2) <= 128) || (heads > 2 && tiles(heads / 2) <= 32)) && tiles(heads / 2) * units <= 7.5f &&
+           !(small && (group < heads ? group : heads) * VD <= 2 * NW * 64))
+      heads /= 2;
   }
   const float share = 0.06f + 0.07f * (group < heads ? group : heads) * VD / 512.f;
   sh.heads = group < heads ? group : heads;
   sh.tiles = lq_ceil_div(group, sh.heads);
   sh.whole = (int)((3.4f + 4 * share) / block) > 1 ? (int)((3.4f + 4 * share) / block) : 1;
+  if (small) sh.whole = tiles(heads) > 64 ? 6 : 4;
   sh.apart = share / block;
   sh.splits = sh.narrow = 1;
   if (max_len <= 0) return sh;
   const long long all = tiles(heads), room = 2 * cus / all, alone = cus / all;
   if (2 * all > cus) {
-    const ManyRows many = many_rows(all);
+    const ManyRows many = many_rows(all, sh.tiles > 1 || small);
     const int from = (int)(many.from / (block > 1.f ? block : 1.f));
     if (many.shares > 1 && most_blocks(max_len) > from) sh.splits = sh.narrow = many.shares, sh.long_from = from;
     return sh;

@@ -46,10 +46,11 @@ def test_single_tokens(H, G, D, P, options, shared):
     check(H, G, D, P, [(1, n - 1) for n in LENGTHS], options, shared)
 
 
-@pytest.mark.parametrize("lengths", [[1], [64, 65], [129], [700], [192, 193, 321], [4097]])
+@pytest.mark.parametrize("lengths", [[1], [64, 65], [129], [700], [192, 193, 321], [4097], [256, 257, 384, 385, 448, 449]])
 @pytest.mark.parametrize("H,G,D,P,options", [(16, 1, 256, 192, PLAIN), (20, 1, 64, 40, dict(sinks=True, gate=True)), (3, 1, 128, 256, PLAIN),
                                              (8, 2, 128, 128, dict(PLAIN, cap=5.0, dist=100, wide=True)),
-                                             (24, 1, 40, 72, dict(window=300, keep_first=130))])
+                                             (24, 1, 40, 72, dict(window=300, keep_first=130)), (64, 8, 64, 64, dict(sinks=True, window=128)),
+                                             (16, 8, 64, 64, PLAIN)])
 def test_single_tokens_of_few_rows(H, G, D, P, options, lengths):
     """A key head's query heads in several workgroups, down to two heads each, and shares of one block upwards."""
     check(H, G, D, P, [(1, n - 1) for n in lengths], options, True)
@@ -64,7 +65,7 @@ def test_single_tokens_of_more_blocks_than_a_wavefront_has_lanes(H, G, D, P, opt
 
 
 @pytest.mark.parametrize("H,G,D,P,rows,start", [(128, 64, 64, 64, 3, 32), (128, 64, 64, 40, 5, 28), (132, 33, 128, 128, 4, 8), (264, 66, 128, 128, 4, 14),
-                                                (160, 80, 128, 256, 4, 6), (380, 95, 128, 128, 4, 28), (64, 16, 256, 192, 9, 4)])
+                                                (160, 80, 128, 256, 4, 6), (380, 95, 128, 128, 4, 28), (64, 16, 256, 192, 9, 4), (640, 32, 64, 64, 4, 28)])
 @pytest.mark.parametrize("options", [PLAIN, dict(sinks=True, window=700, gate=True)])
 def test_single_tokens_of_launches_that_fill_the_chip(H, G, D, P, rows, start, options):
     """Half to twice as many rows and tiles of heads as compute units: rows of up to some `start` blocks stay whole, longer ones go in shares.  Rows
