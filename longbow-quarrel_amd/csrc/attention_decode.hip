@@ -25,7 +25,10 @@
 // positions, partial results four splits at a time) -> this: head size 128, one sequence of 100 keys 6.4 -> 5.4, 300 10.8 -> 6.8, 1 500 12.3 ->
 // 9.0, 7 010 21.7 -> 15.4, 30 000 38.9 -> 34.9 (3.5 TB/s); 8 of 530 12.2 -> 10.6, 8 of 2 070 23.7 -> 20.2, 8 of 8 020 54.7 -> 53.0 (5.0 TB/s);
 // 64 of 560 from pieces 41.6 -> 34.3 (4.3 TB/s); 16 of 128 to 7 628 by units 64 -> 57.  Head size 64: one of 120 4.8 -> 4.2, of 3 000 9.7 ->
-// 9.1; 16 of 80 to 1 516 by units from pieces 15.5 -> 13.8; 24 of 160 from pieces 7.5 -> 7.7, the one length found that lost.
+// 9.1; 16 of 80 to 1 516 by units from pieces 15.5 -> 13.8; 24 of 160 6.5 -> 6.1.
+// Found slower (of 1 202 launches of 1 to 96 rows): very many short rows of head size 64, of which a unit holds three (16 kv heads, 64 rows of 60 keys 6.9 -> 8.0, of
+// 130 12.9 -> 14.2), and three rows a unit of 128, which holds two (96 of 1 000 over 8 72 -> 78, of 2 000 138 -> 146) or four and a half of 96 (96 of
+// 1 000 over 12 81 -> 87).
 #include "attention_mfma.h"
 
 namespace {
