@@ -26,9 +26,8 @@
 // 9.0, 7 010 21.7 -> 15.4, 30 000 38.9 -> 34.9 (3.5 TB/s); 8 of 530 12.2 -> 10.6, 8 of 2 070 23.7 -> 20.2, 8 of 8 020 54.7 -> 53.0 (5.0 TB/s);
 // 64 of 560 from pieces 41.6 -> 34.3 (4.3 TB/s); 16 of 128 to 7 628 by units 64 -> 57.  Head size 64: one of 120 4.8 -> 4.2, of 3 000 9.7 ->
 // 9.1; 16 of 80 to 1 516 by units from pieces 15.5 -> 13.8; 24 of 160 6.5 -> 6.1.
-// Found slower (of 1 202 launches of 1 to 96 rows): very many short rows of head size 64, of which a unit holds three (16 kv heads, 64 rows of 60 keys 6.9 -> 8.0, of
-// 130 12.9 -> 14.2), and three rows a unit of 128, which holds two (96 of 1 000 over 8 72 -> 78, of 2 000 138 -> 146) or four and a half of 96 (96 of
-// 1 000 over 12 81 -> 87).
+// Found slower (of 1 202 launches of 1 to 96 rows) by more than 5 %: 16 heads of 64 over as many, 56 rows of 60 keys 6.9 -> 7.5, 96 9.1 -> 9.6; 12 of 96, 8 rows of 200 6.4 -> 7.0,
+// 16 of 1 000 17.8 -> 18.8, 56 of 4 000 177 -> 187.
 #include "attention_mfma.h"
 
 namespace {
@@ -159,10 +158,10 @@ __device__ inline int balanced_item(const DecodeArgs& a, int u, DecodeItem& it) 
 // What a wavefront holds of the cache blocks that are taken together: of each its 16 keys (row lane % 16, entries 32 kk + 8 (lane /
 // 16) ..), and of its tiles of value entries row lane % 16, positions 32 j + 8 (lane / 16) .. .  Both halves of a line are asked for
 // by instructions next to each other, which the L1 turns into one request of 128 bytes.  Head sizes up to 64 take two blocks together:
-// 32 KB on their way for a barrier, as with one block of 128.
-template <int HD>
+// 32 KB on their way for a barrier, as with one block of 128 (or one, where more workgroups a unit serve better: `launch`).
+template <int HD, int TOGETHER>
 struct Share {
-  static constexpr int KS = HD / 32, VT = HD / 16, VW = (VT + NW - 1) / NW, GB = HD <= 64 ? 2 : 1;
+  static constexpr int KS = HD / 32, VT = HD / 16, VW = (VT + NW - 1) / NW, GB = TOGETHER;
   u32x4 k[GB][KS];
   u32x4 v[GB][VW][2];
 };
@@ -170,9 +169,9 @@ struct Share {
 // Asks for a block, or, with the same instructions, for nothing at all (`there`: a descriptor of no bytes, every access of which
 // is out of bounds and yields zero): a share's last blocks need no branch, behind which the compiler would have to wait for
 // whatever may have been asked for.  Tiles of value entries beyond the head's are out of bounds too.
-template <int HD>
-__device__ inline void ask_block(const DecodeArgs& a, int kvh, int blk, bool there, int wave, int c16, int g, int u, Share<HD>& s) {
-  using S = Share<HD>;
+template <int HD, int GB>
+__device__ inline void ask_block(const DecodeArgs& a, int kvh, int blk, bool there, int wave, int c16, int g, int u, Share<HD, GB>& s) {
+  using S = Share<HD, GB>;
   const long long base = ((long long)blk * a.nkv + kvh) * (BS * HD);
   const int bytes = there ? BS * HD * 2 : 0;
   const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.kcache + base), 0, bytes, 0x00020000);
@@ -296,9 +295,10 @@ __device__ inline int blocks_a_share(const DecodeArgs& a, int n) {
   return max(even, apart);
 }
 
-template <int HD, bool PIECES>
-__global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel(DecodeArgs a) {
-  using S = Share<HD>;
+// GB: blocks taken together; HELD: workgroups that a compute unit holds at least.
+template <int HD, bool PIECES, int GB, int HELD>
+__global__ __launch_bounds__(NW * 64, HELD) void attn_decode_kernel(DecodeArgs a) {
+  using S = Share<HD, GB>;
   __shared__ __attribute__((aligned(16))) float scores[2][16][S::GB * BS + 4];  // (apart so that neighbouring heads' lie in other banks)
   __shared__ __attribute__((aligned(16))) float tops[2][16][NW];  // (what wavefronts' probabilities were taken against)
   __shared__ u32x4 rows[PIECES ? 2 * S::KS : 1][64];
@@ -377,14 +377,14 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
   const int* table = a.block_table + (long long)slot * a.bt_stride;
   const bool own = folded && b1 == last;  // whether this share holds the row's own position
   u32x4 q[S::KS], k_own[S::KS];
-  Share<HD> cur;
+  S cur;
   // The first blocks' numbers come by scalar loads, those of the blocks behind them 64 at a time, lane l that of block b0 + l.  (Each
   // looked up on its own, a block ahead, the walk waited for its way through memory, and where two blocks go together for the
   // keys that were asked for between the two lookups: one sequence of 160 keys, head size 64, 5.5 -> 5.0 us, 24 of 160 6.8 -> 6.1, 16 of 530 from
   // pieces 11.8 -> 9.8; head size 128, a whole row a unit of 24 sequences of 3 000 keys 64.9 -> 58.6.)
   int numbers = table[min(b0 + lane, b1)];
 #pragma unroll
-  for (int u = 0; u < S::GB; ++u) ask_block<HD>(a, kvh, table[min(b0 + u, b1)], b0 + u <= b1, wave, c16, g, u, cur);
+  for (int u = 0; u < S::GB; ++u) ask_block<HD, GB>(a, kvh, table[min(b0 + u, b1)], b0 + u <= b1, wave, c16, g, u, cur);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (PIECES) {
     q_row.put(a, rows, wave, g);
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
 
   // Blocks b .. b + GB - 1 of the share, as far as it reaches; `turn_of`: whose turn it is of the two buffers.  A wavefront takes its
   // keys' probabilities against their own maximum; whoever reads them multiplies them up to the row's.
-  auto take = [&](int b, int turn_of, Share<HD>& s) {
+  auto take = [&](int b, int turn_of, S& s) {
     f32x4 st[S::GB];  // keys 64 (b + u) + 16 wave + 4 g + e
     float own_top = -INFINITY;
 #pragma unroll
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
     }
   };
   for (int b = b0, odd = 0;; b += S::GB, odd ^= 1) {
-    Share<HD> next;
+    S next;
     const int at = (b + S::GB - b0) & 63;
     if (at == 0) {  // (64 is a multiple of GB)
       numbers = table[min(b + S::GB + lane, b1)];
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
     }
 #pragma unroll
     for (int u = 0; u < S::GB; ++u)
-      ask_block<HD>(a, kvh, __builtin_amdgcn_readlane(numbers, at + u), b + S::GB + u <= b1, wave, c16, g, u, next);
+      ask_block<HD, GB>(a, kvh, __builtin_amdgcn_readlane(numbers, at + u), b + S::GB + u <= b1, wave, c16, g, u, next);
     take(b, odd, cur);
     if (b + S::GB > b1) break;
     cur = next;
@@ -622,13 +622,30 @@ __global__ __launch_bounds__(NW * 64, HD <= 192 ? 2 : 1) void attn_decode_kernel
     __hip_atomic_store(&a.tickets[(long long)r * a.nkv + kvh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int HD>
+template <int HD, int GB, int HELD>
 int launch(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid = a.units > 0 ? dim3(a.nkv, a.units) : dim3(a.batch, a.nkv, a.nsplit);
-  if (a.pieces > 1) attn_decode_kernel<HD, true><<<grid, NW * 64, 0, stream>>>(a);
-  else attn_decode_kernel<HD, false><<<grid, NW * 64, 0, stream>>>(a);
+  if (a.pieces > 1) attn_decode_kernel<HD, true, GB, HELD><<<grid, NW * 64, 0, stream>>>(a);
+  else attn_decode_kernel<HD, false, GB, HELD><<<grid, NW * 64, 0, stream>>>(a);
   LQ_CHECK_LAUNCH("attention(single tokens)");
   return 0;
+}
+
+// Which kernel of a head size.  Of 64, one block at a time in a workgroup of which a unit holds four instead of two blocks in one of which it holds
+// three: where rows are one to three a unit, or nearly fill four, but for few more than one that go in shares (16 heads over as many, us: 17 rows of 130 keys
+// 7.7 -> 6.8, of 1 000 21.6 -> 19.6, of 7 000 in fives 94 either way; 20 of 7 000 in fours 105 and 109; 24 of 130 8.0 -> 7.0, of 4 000 77 -> 71; 32 of 130
+// 8.3 -> 7.5, of 4 000 92 -> 90; 48 of 60 6.5 -> 5.8; 64 of 60 8.3 -> 6.3, of 130 13.8 -> 12.1, of 4 000 either; but 16 of 4 000 46 and 56, 56 of 1 000 45.2
+// and 47.2, 80 of 1 000 59 and 65).  Of 128, in 168 registers instead of 170, so that a unit holds three, where there are three (32 over 8: 96 of
+// 1 000 80.7 -> 73.7, in two shares 77.4, of 4 000 295 -> 266 and 272; but 104 of 2 000 160 and 165; pieces have the room anyway).
+template <int HD>
+int launch(const DecodeArgs& a, hipStream_t stream) {
+  const long long pairs = (long long)a.batch * a.nkv, cus = lq_compute_units();
+  if constexpr (HD == 64)
+    if (a.units == 0 && ((pairs > cus && pairs <= 3 * cus && !(a.long_from > 0 && 4 * pairs <= 5 * cus)) || (4 * pairs >= 15 * cus && pairs <= 4 * cus)))
+      return launch<HD, 1, 4>(a, stream);
+  if constexpr (HD == 128)
+    if (a.units == 0 && a.pieces <= 1 && 2 * pairs > 5 * cus && pairs <= 3 * cus) return launch<HD, 1, 3>(a, stream);
+  return launch<HD, HD <= 64 ? 2 : 1, HD <= 192 ? 2 : 1>(a, stream);
 }
 
 }  // namespace
@@ -644,9 +661,9 @@ int launch(const DecodeArgs& a, hipStream_t stream) {
 // 32 heads over 8, whole -> so, microseconds; a wavefront with a block of its own and up to 2 048 workgroups in brackets:
 // head size 128: 17 sequences of 1 500 keys 31 -> 28 (38), of 6 000 106 -> 84 (91); 22 of 6 000 114 -> 107 (108); 33 of 1 000 41.5 -> 38 (46), of
 // 3 000 106 -> 84 (101), of 6 000 203 -> 161 (176); 40 of 3 000 108 -> 94 (107); 48 of 6 000 223 -> 206 (214); 66 of 3 000 176 -> 153; 80 of 1 500
-// 108 -> 100, of 6 000 418 -> 341; 88 of 3 000 216 -> 196; 96 of 2 000 154 -> 146 (138).  Head size 64: 17 of 3 000 34 -> 27
-// (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 48 of 6 000 117 -> 110 (112); 66 of 3 000 92 -> 81; 80 of 6 000 186 -> 175; 16 heads over
-// as many, 33 of 8 000 235 -> 194 (197).  12 heads of 96: 16 of 3 000 48 -> 43; 43 of 750 36 -> 33, of 3 000 130 -> 112; 48 of 4 000 177 -> 154 (159).
+// 108 -> 100, of 6 000 418 -> 341; 88 of 3 000 in twos 216 -> 196 (and whole, where a unit holds three, 190).  Head size 64: 17 of 3 000 34 -> 27
+// (30); 24 of 6 000 66 -> 60 (62); 33 of 6 000 105 -> 84 (90); 66 of 3 000 92 -> 81; 80 of 7 000 216 -> 203; 16 heads over
+// as many, 33 of 8 000 235 -> 194 (197).  12 heads of 96: 16 of 3 000 48 -> 43; 43 of 750 36 -> 33, of 3 000 130 -> 112; 48 of 4 000 177 -> 154 (159); 96 of 2 000 166 -> 159 (155).
 // Eight heads over 4 of 192: 75 of 750 45 -> 39; 144 of 3 000 257 -> 234.
 // (Rows whole that would do in shares, or the reverse: 24 of 200 keys in two shares each 12.5, whole 9.5; 24 of 6 000 118 and 110; 52 of 3 000
 // in sixes 127, whole 118; 104 of 1 500 in threes 125, whole 122; 128 of 3 000 in twos 279, whole 266.)
@@ -660,14 +677,14 @@ static ManyRows many_rows(long long pairs, int hd) {
   if ((small || narrow) && 4 * pairs <= 3 * cus) return {4, small ? 32 : 20};
   if (!small && 5 * pairs <= 4 * cus) return {5, narrow ? 20 : 80};
   if (pairs <= cus) return {1, 0};
-  if (5 * pairs <= 6 * cus) return {5, small ? 16 : hd > 128 ? 10 : 14};
+  if (5 * pairs <= 6 * cus) return {5, small ? 17 : hd > 128 ? 10 : 14};
   if (!small && 3 * pairs <= 4 * cus) return {3, hd > 128 ? 10 : 14};
-  if (2 * pairs <= 3 * cus) return {4, 28};
+  if (small ? 4 * pairs <= 5 * cus : 2 * pairs <= 3 * cus) return {4, 28};
   if (pairs <= 2 * cus) return {1, 0};
   if (hd > 192) return {1, 0};
-  if (small && 5 * pairs > 12 * cus) return 2 * pairs <= 5 * cus ? ManyRows{2, 28} : ManyRows{1, 0};
+  if (small && 5 * pairs > 12 * cus) return 2 * pairs <= 5 * cus ? ManyRows{4, 48} : ManyRows{1, 0};
   if (2 * pairs <= 5 * cus) return {4, narrow ? 10 : 18};
-  if (hd == 128 && pairs <= 3 * cus) return {2, 14};
+  if (narrow && pairs > 4 * cus && pairs <= 5 * cus) return {3, 14};
   return {1, 0};
 }
 

@@ -14,7 +14,7 @@ EDGES = [1, 63, 64, 65, 128, 129, 192, 193, 256, 257, 384, 385, 386, 640, 1030, 
 
 
 @pytest.mark.parametrize("heads,kv_heads,head_dim,rows", [(32, 8, 128, 3), (16, 16, 64, 16), (8, 1, 64, 1), (6, 2, 256, 4),
-                                                          (4, 1, 192, 16)])
+                                                          (4, 1, 192, 16), (64, 32, 64, 16), (48, 48, 128, 14)])
 @pytest.mark.parametrize("window", [0, 70])
 @pytest.mark.parametrize("apart", [0, 1])
 def test_folded_rows_at_the_edges(kn, heads, kv_heads, head_dim, rows, window, apart):
@@ -71,10 +71,10 @@ def test_rows_of_more_blocks_than_a_wavefront_has_lanes(kn, kv_heads, head_dim):
 @pytest.mark.parametrize("rows,kv_heads,head_dim,start", [(17, 8, 128, 12), (21, 8, 64, 16), (3, 64, 64, 32), (3, 64, 128, 80), (33, 8, 192, 14),
                                                           (5, 64, 128, 14), (6, 64, 128, 28), (6, 64, 64, 28), (12, 32, 256, 28),
                                                           (3, 64, 96, 20), (5, 64, 192, 10), (9, 64, 96, 10), (9, 64, 128, 18), (9, 64, 192, 18),
-                                                          (11, 64, 128, 14), (9, 64, 64, 20), (10, 64, 64, 28)])
+                                                          (9, 64, 64, 18), (10, 64, 64, 48), (18, 64, 96, 14), (5, 64, 64, 28)])
 @pytest.mark.parametrize("window", [0, 1000])
 def test_long_rows_of_launches_that_fill_the_chip(kn, rows, kv_heads, head_dim, start, window):
-    """Launches of half to three times as many rows and kv heads as compute units: rows of up to `start` blocks stay whole, longer ones go
+    """Launches of half to five times as many rows and kv heads as compute units: rows of up to `start` blocks stay whole, longer ones go
     in shares, which its last workgroup adds up, so that the units have equal parts.  Rows at that line, far beyond it and of one
     key; twice the same, with the counters at zero after each."""
     lengths = ([start * BS, (start - 1) * BS, (start - 1) * BS + 1, 3 * start * BS + 65, 1, start * BS + 1] * rows)[:rows]
@@ -89,6 +89,17 @@ def test_long_rows_of_launches_that_fill_the_chip(kn, rows, kv_heads, head_dim, 
         assert int(kn.tickets(torch.device("cuda", torch.cuda.current_device())).abs().max()) == 0
         outs.append(got)
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,head_dim", [(7, 64, 64, 64), (16, 128, 64, 64), (11, 64, 64, 128), (21, 64, 32, 128), (24, 32, 32, 64)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_rows_of_which_a_unit_holds_more(kn, rows, heads, kv_heads, head_dim, window):
+    """Where one block goes at a time at head size 64, and three workgroups are held of 128: rows of every edge of a block and of more blocks than
+    a wavefront has lanes."""
+    lengths = (EDGES + [64 * BS + 1, 65 * BS, 66 * BS + 1, 3, 70, 190, 500, 700])[-rows:]
+    got, want = run_attention(kn, None, lengths, [1] * rows, heads, kv_heads, head_dim, torch.bfloat16, 29, window=window, decode=True)
+    for b, n in enumerate(lengths):
+        assert rel_err(got[b], want[b]) < 1.2e-2, n
 
 
 @pytest.mark.parametrize("kv_heads,head_dim", [(8, 128), (2, 192), (1, 256), (8, 64)])
