@@ -230,9 +230,13 @@ __global__ __launch_bounds__(256) void causal_conv4_kernel(const T* __restrict__
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) {
         const int back = TAPS - 1 - j;
-        if (back > since) hist[j] = *(const float4*)(state + (slot + TAPS - 1 - (back - since)) * C + c);
-        else if constexpr (TILE) hist[j] = in[i + j];
-        else hist[j] = load4<T>(x + (long long)(r - back) * ldx + c);
+        const float* kept = state + (slot + TAPS - 1 - (back - since)) * C + c;
+        if constexpr (TILE) {
+          if (back > since) hist[j] = *(const float4*)kept;
+          else hist[j] = in[i + j];
+        } else {  // (one expression: of float32 rows it becomes a choice between two addresses, and no load waits for another)
+          hist[j] = back <= since ? load4<T>(x + (long long)(r - back) * ldx + c) : *(const float4*)kept;
+        }
       }
       before = b;
     } else {
